@@ -128,18 +128,18 @@ def _case(name, model, requests, prompt, new, ragged=0.0, gap=0, portion=512, dt
 
 def listed():
     return [
-        _case("chat, 0.5B", "qwen2.5-0.5b", 1, 61, 64),                                   # one short question answered: the smallest steps there are
-        _case("batch of 8, 7B", "qwen2.5-7b", 8, 1024, 48, ragged=0.5),                   # the headline size, a few users
-        _case("long prompt, 7B", "qwen2.5-7b", 1, 8192, 1),                               # a document read in portions of 2,048
-        _case("serving, 3B", "qwen2.5-3b", 24, 1024, 24, ragged=0.95, gap=1),             # prompts in portions of 512 beside requests that decode
-        _case("batch of 64, 1.5B", "qwen2.5-1.5b", 64, 200, 24, ragged=0.9),              # offline generation, the widest decode steps
-        _case("32 bits, 0.5B", "qwen2.5-0.5b", 4, 150, 16, ragged=0.5, dtype="float32"),  # the mode that logits are checked in
-        _case("batch of 8, Mumusun", "mumusun-medium", 8, 600, 32, ragged=0.4),           # a latent and many experts, decoding
-        _case("prompt, Podurax", "podurax-medium", 1, 2048, 8),                           # attention and state-space layers over a long prompt
-        _case("batch of 16, Tabatar", "tabatar-medium", 16, 333, 32, ragged=0.5),         # linear attention on several streams
-        _case("chat, Vavadra", "vavadra-medium", 1, 700, 48),                             # delta rule, differential attention, shared experts
-        _case("batch of 64, Narasun", "narasun-medium", 64, 65, 16, ragged=0.9),          # short questions to matrix memories
-        _case("four documents, Duletar", "duletar-medium", 4, 1500, 16, ragged=0.3),      # retention and shared latents
+        _case("chat 0.5B", "qwen2.5-0.5b", 1, 61, 64),                                   # one short question answered: the smallest steps there are
+        _case("batch of 8 7B", "qwen2.5-7b", 8, 1024, 48, ragged=0.5),                   # the headline size, a few users
+        _case("long prompt 7B", "qwen2.5-7b", 1, 8192, 1),                               # a document read in portions of 2,048
+        _case("serving 3B", "qwen2.5-3b", 24, 1024, 24, ragged=0.95, gap=1),             # prompts in portions of 512 beside requests that decode
+        _case("batch of 64 1.5B", "qwen2.5-1.5b", 64, 200, 24, ragged=0.9),              # offline generation, the widest decode steps
+        _case("32 bits 0.5B", "qwen2.5-0.5b", 4, 150, 16, ragged=0.5, dtype="float32"),  # the mode that logits are checked in
+        _case("batch of 8 Mumusun", "mumusun-medium", 8, 600, 32, ragged=0.4),           # a latent and many experts, decoding
+        _case("prompt Podurax", "podurax-medium", 1, 2048, 8),                           # attention and state-space layers over a long prompt
+        _case("batch of 16 Tabatar", "tabatar-medium", 16, 333, 32, ragged=0.5),         # linear attention on several streams
+        _case("chat Vavadra", "vavadra-medium", 1, 700, 48),                             # delta rule, differential attention, shared experts
+        _case("batch of 64 Narasun", "narasun-medium", 64, 65, 16, ragged=0.9),          # short questions to matrix memories
+        _case("four documents Duletar", "duletar-medium", 4, 1500, 16, ragged=0.3),      # retention and shared latents
     ]
 
 
