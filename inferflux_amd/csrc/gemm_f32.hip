@@ -1,83 +1,247 @@
 // True 32-bit matrix product:  C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]).
 //
-// The weight is float and every multiply-add is a float fmaf: no matrix-core instruction, no
-// reduced-precision mode.  Each output element is accumulated over k in ascending order by one
-// thread, so its value does not depend on M, on the element's place in the batch or on what
-// else runs.  This is the matrix product of the 32-bit path; the reference has no 32-bit path
+// The weight is float and every multiply-add is one of the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: float
+// products, float sums, no reduced-precision mode).  An element's sum does not depend on M, on the element's place in the
+// batch or on what else runs: K is cut into the same sixteen slices whatever M and N are, a slice is summed in one chain of
+// matrix instructions in ascending steps of 16 (instruction j of a step takes k = 4 q + j of the step's 16 for q = 0 .. 3,
+// which is how four consecutive floats per lane lie in registers), and the slices' sums are added in ascending order.  Both
+// kernels below keep that order, so rows computed alone and in a batch of thousands are the same bits.
+// This is the matrix product of the 32-bit path; the reference has no 32-bit path
 // (runtime/backends/cuda/native/transformer_forward.cu:4600-4601 instantiates half and bf16
 // only), its library call with float accumulation is runtime/backends/cuda/native/cublas_gemm.cpp:99-117.
 #include "common.h"
 
 IFX_DEFINE_LAST_ERROR()
 
-#define BM 64
-#define BN 64
-#define BK 16
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <typename TA, typename TO>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const TA* __restrict__ A, const float* __restrict__ W,
-                                                       const float* __restrict__ bias, TO* __restrict__ C,
-                                                       int M, int N, int K) {
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Ws[BK][BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16, ty = tid / 16;
+#define N_SLICES 16
+
+__device__ __forceinline__ int slice_len(int K) { return ((K + N_SLICES - 1) / N_SLICES + 15) / 16 * 16; }
+
+// Four consecutive elements k .. k + 3 of a row of K, zeros behind its end.  VEC: the row starts on 16 bytes (8 for bf16)
+// and K is a multiple of 4, so four elements are all there or all not.
+template <bool VEC, typename T>
+__device__ __forceinline__ f32x4 load4(const T* __restrict__ row, int k, int K) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (VEC && sizeof(T) == 4) {
+    if (k < K) v = *(const f32x4*)(row + k);
+  } else if constexpr (VEC) {
+    typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+    if (k < K) {
+      const bf16x4 b = *(const bf16x4*)(row + k);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = (float)b[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (k + j < K) v[j] = to_f(row[k + j]);
+  }
+  return v;
+}
+
+// ---- few rows: the weight is streamed once -----------------------------------------------------------------------------
+// A workgroup takes NT x 16 weight rows and MT x 16 rows of A; its sixteen waves take a slice of K each and meet in LDS.
+// Bound by the weight's bytes where N is large (5.6 TB/s at 151,936 x 896) and by the few workgroups where it is not (56 for
+// 896 rows: 1.2 TB/s at K = 4,864): a wave has STEPS steps of 16 k-values (STEPS x (NT + MT) loads of 16 bytes a lane) in
+// flight, and as many waves as a workgroup can hold do more than longer runs of loads in fewer (8 and 10 steps, eight waves:
+// 15.1 to 17.5 us where these take 14.5).
+template <typename TA, typename TO, int MT, int NT, int STEPS, bool VEC>
+__global__ __launch_bounds__(1024) void gemm_f32_few_kernel(const TA* __restrict__ A, const float* __restrict__ W,
+                                                           const float* __restrict__ bias, TO* __restrict__ C,
+                                                           int M, int N, int K) {
+  __shared__ float part[N_SLICES][MT * NT][256];
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int i = lane % 16, q = lane / 16;
+  const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
+  const int len = slice_len(K), k_lo = wave * len, k_hi = min(K, k_lo + len);
+  const float* wrow[NT];
+  const TA* arow[MT];
+  bool a_in[MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) wrow[n] = W + (size_t)min(n0 + 16 * n + i, N - 1) * K;      // (columns beyond N are computed and dropped)
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    a_in[m] = m0 + 16 * m + i < M;
+    arow[m] = A + (size_t)min(m0 + 16 * m + i, M - 1) * K;
+  }
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  f32x4 w[STEPS][NT], a[STEPS][MT];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const int k = k0 + 16 * s + 4 * q;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) w[s][n] = load4<VEC>(wrow[n], k, k_hi);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        a[s][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        if (a_in[m]) a[s][m] = load4<VEC>(arow[m], k, k_hi);
+      }
+    }
+  };
+  for (int k0 = k_lo; k0 < k_hi; k0 += 16 * STEPS) {
+    fetch(k0);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][m][j], w[s][n][j], acc[m][n], 0, 0, 0);
+  }
+  // lane (i, q) holds rows 4 q + r of column i
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[wave][m * NT + n][(4 * q + r) * 16 + i] = acc[m][n][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < MT * NT * 256; e += 1024) {
+    const int t = e / 256, at = e % 256, m = m0 + 16 * (t / NT) + at / 16, n = n0 + 16 * (t % NT) + at % 16;
+    if (m >= M || n >= N) continue;
+    float v = part[0][t][at];
+#pragma unroll
+    for (int s = 1; s < N_SLICES; ++s) v += part[s][t][at];
+    if (bias) v += bias[n];
+    C[(size_t)m * N + n] = from_f<TO>(v);
+  }
+}
+
+// ---- many rows: tiles of A and W through LDS -----------------------------------------------------------------------------
+// A workgroup of four waves makes (32 TM) x (32 TN) outputs, two waves by two; a step of 32 k-values goes through LDS, the next
+// one is on its way from memory meanwhile.  Bound by the matrix units: a wave reads TM + TN fragments of 16 bytes a lane for
+// 4 TM TN instructions of 32 cycles.  LDS rows of 32 floats, the eight pieces of 16 bytes of a row placed by piece ^ (row % 8):
+// the 16 lanes of a fragment's quarter then lie in different banks without padding.
+template <typename TA, typename TO, int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const TA* __restrict__ A, const float* __restrict__ W,
+                                                             const float* __restrict__ bias, TO* __restrict__ C,
+                                                             int M, int N, int K) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, BK = 32;
+  __shared__ f32x4 As[BM][BK / 4], Ws[BN][BK / 4];
+  const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+  const int i = lane % 16, q = lane / 16;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  float acc[4][4];
+  const int wm = (wave / 2) * 16 * TM, wn = (wave % 2) * 16 * TN;
+  const int len = slice_len(K);
+  const int pr = tid / 8, pp = tid % 8;                    // the row (of 32) and the piece this thread brings in
+  f32x4 acc[TM][TN], total[TM][TN], na[TM], nw[TN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int m = 0; m < TM; ++m)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    for (int n = 0; n < TN; ++n) acc[m][n] = total[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto fetch = [&](int k0, int k_hi) {
+    const int k = k0 + 4 * pp;
+#pragma unroll
+    for (int r = 0; r < TM; ++r) {
+      const int m = m0 + 32 * r + pr;
+      na[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (m < M) na[r] = load4<VEC>(A + (size_t)m * K, k, k_hi);
+    }
+#pragma unroll
+    for (int r = 0; r < TN; ++r) {
+      const int n = n0 + 32 * r + pr;
+      nw[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (n < N) nw[r] = load4<VEC>(W + (size_t)n * K, k, k_hi);
+    }
+  };
+  fetch(0, min(K, len));
+  for (int k_lo = 0, s = 0; k_lo < K; k_lo += len, ++s) {
+    const int k_hi = min(K, k_lo + len);
+    for (int k0 = k_lo; k0 < k_hi; k0 += BK) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < TM; ++r) As[32 * r + pr][pp ^ (pr % 8)] = na[r];
+#pragma unroll
+      for (int r = 0; r < TN; ++r) Ws[32 * r + pr][pp ^ (pr % 8)] = nw[r];
+      __syncthreads();
+      if (k0 + BK < k_hi) fetch(k0 + BK, k_hi);
+      else if (k_hi < K) fetch(k_hi, min(K, k_hi + len));
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (k0 + 16 * h >= k_hi) break;                    // (a slice may end in the middle of a step: its length is a multiple of 16)
+        f32x4 a[TM], w[TN];
+#pragma unroll
+        for (int m = 0; m < TM; ++m) a[m] = As[wm + 16 * m + i][(4 * h + q) ^ (i % 8)];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) w[n] = Ws[wn + 16 * n + i][(4 * h + q) ^ (i % 8)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][j], w[n][j], acc[m][n], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        total[m][n] = s == 0 ? acc[m][n] : total[m][n] + acc[m][n];
+        acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+  }
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const int col = n0 + wn + 16 * n + i;
+      if (col >= N) continue;
+      const float b = bias ? bias[col] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + 16 * m + 4 * q + r;
+        if (row < M) C[(size_t)row * N + col] = from_f<TO>(bias ? total[m][n][r] + b : total[m][n][r]);
+      }
+    }
+}
 
-  const int lr = tid / 4;        // tile row this thread loads (0..63)
-  const int lk = (tid % 4) * 4;  // first of its 4 k values
-  for (int k0 = 0; k0 < K; k0 += BK) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int k = k0 + lk + q;
-      const int m = m0 + lr, n = n0 + lr;
-      As[lk + q][lr] = (m < M && k < K) ? to_f(A[(size_t)m * K + k]) : 0.f;
-      Ws[lk + q][lr] = (n < N && k < K) ? W[(size_t)n * K + k] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      float a[4], w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float v = acc[i][j];
-      if (bias) v += bias[n];
-      C[(size_t)m * N + n] = from_f<TO>(v);
-    }
-  }
+// Which kernel: the one with the lowest estimate of its time, all of them in proportion to K.  A kernel's grid runs in rounds of
+// 256 workgroups (one for each compute unit; sixteen waves fill it, and two workgroups of the tile kernel share one).  A round
+// at K = 896 was measured at 5.6 us for 16 x 16 outputs, 7.5 for 32 x 16 and 10.3 for 32 x 32 with the slices side by side; the
+// tile kernel, which walks K in one go, takes 31 us for up to 256 tiles of 64 x 64 and 0.083 us a tile beyond that (but not
+// less than 44).  Before these kernels (one thread summing an output, tiles of 64 x 64, scalar loads) a product took 83 us at
+// 1 row and 102 at 475 of 896 x 896 (now 4.3 and 20), 449 and 559 of 896 x 4,864 (14.5 and 97), 90 and 266 of 9,728 x 896 (10.2
+// and 105), 410 at one row of 151,936 x 896 (97: 5.6 TB/s); 2,048 rows of 22,016 x 2,048 run at 103 TFLOP/s.  Errors against 64
+// bits fell to a third (5.4e-7 to 2.0e-7 at K = 896, 1.9e-6 to 6.6e-7 at 11,008): shorter chains.
+template <typename TA, typename TO, bool VEC>
+static void launch(const TA* A, const float* W, const float* bias, TO* C, int M, int N, int K, hipStream_t s) {
+  auto blocks = [&](int m, int n) { return (double)((M + m - 1) / m) * ((N + n - 1) / n); };
+  auto rounds = [&](int m, int n) { return (double)(long long)((blocks(m, n) + 255.0) / 256.0); };
+  const double t11 = 5.6 * rounds(16, 16), t21 = 7.5 * rounds(32, 16), t22 = 10.3 * rounds(32, 32);
+  const double b64 = blocks(64, 64), tiles = b64 <= 256.0 ? 31.0 : (b64 < 530.0 ? 44.0 : 0.083 * b64);
+#define FEW(MT, NT)                                                                                              \
+  hipLaunchKernelGGL((gemm_f32_few_kernel<TA, TO, MT, NT, 4, VEC>),                                              \
+                     dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K)
+  if (M <= 16 || (t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
+  else if (t21 <= t22 && t21 <= tiles) FEW(2, 1);
+  else if (t22 <= tiles) FEW(2, 2);
+  else
+    hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K);
+#undef FEW
 }
 
 extern "C" int ifx_gemm_f32(const void* A, int a_dtype, const float* W, const float* bias, void* C,
                             int c_dtype, int M, int N, int K, void* stream) {
   IFX_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
-  dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-  IFX_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d too large for one launch", M);
+  IFX_REQUIRE((M + 63) / 64 <= 65535, "gemm_f32: M=%d too large for one launch", M);
   hipStream_t s = (hipStream_t)stream;
-#define LAUNCH(TA, TO) \
-  hipLaunchKernelGGL((gemm_f32_kernel<TA, TO>), grid, dim3(256), 0, s, (const TA*)A, W, bias, (TO*)C, M, N, K)
+  const bool vec = K % 4 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)A % (a_dtype == DT_BF16 ? 8 : 16) == 0;
+#define LAUNCH(TA, TO)                                                              \
+  do {                                                                              \
+    if (vec) launch<TA, TO, true>((const TA*)A, W, bias, (TO*)C, M, N, K, s);       \
+    else launch<TA, TO, false>((const TA*)A, W, bias, (TO*)C, M, N, K, s);          \
+  } while (0)
   if (a_dtype == DT_F32 && c_dtype == DT_F32) LAUNCH(float, float);
   else if (a_dtype == DT_BF16 && c_dtype == DT_BF16) LAUNCH(bf16_t, bf16_t);
   else if (a_dtype == DT_BF16 && c_dtype == DT_F32) LAUNCH(bf16_t, float);

@@ -447,6 +447,23 @@ def test_gemm_f32_random_shapes(seed):
     assert torch.equal(alone[0], got[r]), (M, N, K, r)
 
 
+@pytest.mark.parametrize("N,K", [(1, 1), (15, 16), (17, 255), (64, 256), (65, 257), (896, 896), (9000, 272)])
+@pytest.mark.parametrize("adtype", [F32, BF16])
+def test_gemm_f32_kernels_agree_bit_for_bit(N, K, adtype):
+    """Numbers of rows on both sides of every kernel's range and of the tiles' edges, operands on and off 16 bytes: each row the
+    same bits as alone, and off the 64-bit product by no more than K roundings of the sum of the terms' sizes (2^-24 each)."""
+    g = gen(2100)
+    x = torch.randn(1030, K, generator=g).to(adtype).to(DEV)
+    w = torch.randn(N, K, generator=g).to(DEV)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    whole = ops.gemm_f32(x, w, None, F32)
+    assert ((whole - want).abs() <= (K + 2) * 2.0 ** -24 * size).all()
+    shifted = torch.empty(1030 * K + 1, dtype=adtype, device=DEV)[1:].view(1030, K).copy_(x)
+    for M in (1, 15, 16, 17, 32, 33, 64, 65, 129, 600):
+        assert torch.equal(ops.gemm_f32(x[:M].contiguous(), w, None, F32), whole[:M]), M
+    assert torch.equal(ops.gemm_f32(shifted, w, None, F32), whole)
+
+
 # ---- sampling -------------------------------------------------------------------------------
 def test_argmax_lowest_index_wins_ties():
     l = torch.zeros(3, 1500)
