@@ -91,7 +91,7 @@ enum { MODE_GATE_UP = 0, MODE_DOWN = 1, MODE_HEADS = 2 };
 
 struct GroupedArgs {
   const bf16_t* x;          // item i of group g reads K values from x + (i / x_div) * x_row + g * x_group
-  const bf16_t* w;          // [groups][NW][K]
+  const bf16_t* w;          // [groups][NW][K], or its tiled form (TILED; see ifx_tile_weights in gemm_bf16.hip, tiles of 16 rows)
   void* out;
   const int* sorted; const int* tile_expert; const int* tile_start; const int* tile_count; const int* n_tiles;   // (not MODE_HEADS)
   const float* weights;     // MODE_DOWN: [n_items]
@@ -102,11 +102,12 @@ struct GroupedArgs {
   const bf16_t* identity;   // MODE_DOWN: [T][NW], what an identity expert hands back
   int act; float limit;     // MODE_GATE_UP: the activation
   int weigh_input;          // the weight is on an expert's input: MODE_GATE_UP multiplies both sums by it, MODE_DOWN leaves it out
+  int k_tiles;              // TILED: tiles of 32 k-values to a row tile, an even number
   ColumnGate gate;          // MODE_HEADS: columns col + group * NW + n of row t (rows null: none)
 };
 
 // MT: tiles of 32 items per wave (1: the workgroup takes 64 items, 2: 128)
-template <int MODE, int MT>
+template <int MODE, int MT, bool TILED>
 __global__ __launch_bounds__(256) void grouped_kernel(GroupedArgs a) {
   constexpr int BM = 64 * MT;
   __shared__ __attribute__((aligned(16))) bf16_t ws[TN][LDP];
@@ -159,10 +160,17 @@ __global__ __launch_bounds__(256) void grouped_kernel(GroupedArgs a) {
   const bf16_t* wp[WP];
   const bf16_t* xp[XP];
   const int kc = 8 * (tid % 8);
+  // TILED: a step's 8 row tiles x 2 k-tiles are 1,024 pieces, 64 of which lie together: a wave asks for 1 KB at a time.  Piece
+  // q of them is row 16 (q / 128) + q % 16 at k = 32 (q / 64 % 2) + 8 (q / 16 % 4).
 #pragma unroll
   for (int p = 0; p < WP; ++p) {
-    const int wrow = n0 + (tid + 256 * p) / 8;
-    wp[p] = wrow < a.NW ? wbase + (size_t)wrow * a.K + kc : nullptr;
+    if (TILED) {
+      const int q = tid + 256 * p, t = n0 / 16 + q / 128;
+      wp[p] = t < a.NW / 16 ? a.w + (((size_t)group * (a.NW / 16) + t) * a.k_tiles * WAVE + q % 128) * 8 : nullptr;
+    } else {
+      const int wrow = n0 + (tid + 256 * p) / 8;
+      wp[p] = wrow < a.NW ? wbase + (size_t)wrow * a.K + kc : nullptr;
+    }
   }
 #pragma unroll
   for (int p = 0; p < XP; ++p) {
@@ -172,7 +180,8 @@ __global__ __launch_bounds__(256) void grouped_kernel(GroupedArgs a) {
   auto fetch = [&](int k0) {
     const bool in = k0 + kc < a.K;
 #pragma unroll
-    for (int p = 0; p < WP; ++p) wv[p] = (wp[p] && in) ? *(const bf16x8*)(wp[p] + k0) : zero;
+    for (int p = 0; p < WP; ++p)          // (TILED: k0 is within the whole tiles, which end in zeros)
+      wv[p] = (wp[p] && (TILED || in)) ? *(const bf16x8*)(wp[p] + (TILED ? (size_t)(k0 / 32) * WAVE * 8 : (size_t)k0)) : zero;
 #pragma unroll
     for (int p = 0; p < XP; ++p) xv[p] = (xp[p] && in) ? *(const bf16x8*)(xp[p] + k0) : zero;
   };
@@ -180,7 +189,11 @@ __global__ __launch_bounds__(256) void grouped_kernel(GroupedArgs a) {
   for (int k0 = 0; k0 < a.K; k0 += TK) {
     __syncthreads();          // everyone is done with the last step's tiles
 #pragma unroll
-    for (int p = 0; p < WP; ++p) *(bf16x8*)&ws[(tid + 256 * p) / 8][kc] = wv[p];
+    for (int p = 0; p < WP; ++p) {
+      const int q = tid + 256 * p;
+      if (TILED) *(bf16x8*)&ws[16 * (q / 128) + q % 16][32 * (q / 64 % 2) + 8 * (q / 16 % 4)] = wv[p];
+      else *(bf16x8*)&ws[q / 8][kc] = wv[p];
+    }
 #pragma unroll
     for (int p = 0; p < XP; ++p) *(bf16x8*)&xs[(tid + 256 * p) / 8][kc] = xv[p];
     __syncthreads();
@@ -283,14 +296,17 @@ static int check_common(int K, int x_row, int x_group) {
 // act [n_items][ff] (bfloat16) from x [T][K] and the paired weights w [E][2 ff][K]; item i is row i / top.
 extern "C" int ifx_moe_gate_up_grouped(const void* x, const void* w, void* act, const int* sorted, const int* tile_expert,
                                        const int* tile_start, const int* tile_count, const int* n_tiles, int max_tiles, int tile_items,
-                                       int K, int ff, int top, int n_real, int act_kind, float limit, const float* in_weights, void* stream) {
+                                       int K, int ff, int top, int n_real, int act_kind, float limit, const float* in_weights, int tiled,
+                                       void* stream) {
   IFX_REQUIRE(check_common(K, K, 0) && ff > 0 && ff % 16 == 0 && top > 0, "moe_gate_up_grouped: K=%d must be a multiple of 8, ff=%d of 16", K, ff);
   if (max_tiles <= 0) return 0;
   GroupedArgs a{(const bf16_t*)x, (const bf16_t*)w, act, sorted, tile_expert, tile_start, tile_count, n_tiles, in_weights,
-                K, 2 * ff, top, K, 0, 0, top, 0, 0, n_real, nullptr, act_kind, limit, in_weights ? 1 : 0, {}};
+                K, 2 * ff, top, K, 0, 0, top, 0, 0, n_real, nullptr, act_kind, limit, in_weights ? 1 : 0, (K + 63) / 64 * 2, {}};
   const dim3 grid(max_tiles, (2 * ff + TN - 1) / TN);
-  if (tile_items == 128) hipLaunchKernelGGL((grouped_kernel<MODE_GATE_UP, 2>), grid, dim3(256), 0, (hipStream_t)stream, a);
-  else if (tile_items == 64) hipLaunchKernelGGL((grouped_kernel<MODE_GATE_UP, 1>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  if (tile_items == 128 && tiled) hipLaunchKernelGGL((grouped_kernel<MODE_GATE_UP, 2, true>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  else if (tile_items == 64 && tiled) hipLaunchKernelGGL((grouped_kernel<MODE_GATE_UP, 1, true>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  else if (tile_items == 128) hipLaunchKernelGGL((grouped_kernel<MODE_GATE_UP, 2, false>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  else if (tile_items == 64) hipLaunchKernelGGL((grouped_kernel<MODE_GATE_UP, 1, false>), grid, dim3(256), 0, (hipStream_t)stream, a);
   else IFX_FAIL("moe_gate_up_grouped: tiles of %d items (64 or 128)", tile_items);
   IFX_LAUNCH_CHECK();
 }
@@ -299,14 +315,17 @@ extern "C" int ifx_moe_gate_up_grouped(const void* x, const void* w, void* act, 
 extern "C" int ifx_moe_down_grouped(const void* act, const void* w, float* parts, const float* weights, const int* sorted,
                                     const int* tile_expert, const int* tile_start, const int* tile_count, const int* n_tiles,
                                     int max_tiles, int tile_items, int T, int N, int ff, int top, int n_real, const void* identity,
-                                    int weigh_input, void* stream) {
+                                    int weigh_input, int tiled, void* stream) {
+  IFX_REQUIRE(!tiled || N % 16 == 0, "moe_down_grouped: tiled weights need N=%d to be a multiple of 16", N);
   IFX_REQUIRE(check_common(ff, ff, 0) && N > 0 && top > 0 && T >= 0, "moe_down_grouped: ff=%d must be a multiple of 8", ff);
   if (max_tiles <= 0 || T == 0) return 0;
   GroupedArgs a{(const bf16_t*)act, (const bf16_t*)w, parts, sorted, tile_expert, tile_start, tile_count, n_tiles, weights,
-                ff, N, 1, ff, 0, T, top, 0, 0, n_real, (const bf16_t*)identity, 0, 0.f, weigh_input, {}};
+                ff, N, 1, ff, 0, T, top, 0, 0, n_real, (const bf16_t*)identity, 0, 0.f, weigh_input, (ff + 63) / 64 * 2, {}};
   const dim3 grid(max_tiles, (N + TN - 1) / TN);
-  if (tile_items == 128) hipLaunchKernelGGL((grouped_kernel<MODE_DOWN, 2>), grid, dim3(256), 0, (hipStream_t)stream, a);
-  else if (tile_items == 64) hipLaunchKernelGGL((grouped_kernel<MODE_DOWN, 1>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  if (tile_items == 128 && tiled) hipLaunchKernelGGL((grouped_kernel<MODE_DOWN, 2, true>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  else if (tile_items == 64 && tiled) hipLaunchKernelGGL((grouped_kernel<MODE_DOWN, 1, true>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  else if (tile_items == 128) hipLaunchKernelGGL((grouped_kernel<MODE_DOWN, 2, false>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  else if (tile_items == 64) hipLaunchKernelGGL((grouped_kernel<MODE_DOWN, 1, false>), grid, dim3(256), 0, (hipStream_t)stream, a);
   else IFX_FAIL("moe_down_grouped: tiles of %d items (64 or 128)", tile_items);
   IFX_LAUNCH_CHECK();
 }
@@ -319,9 +338,9 @@ extern "C" int ifx_headwise_grouped(const void* x, const void* w, void* out, int
   IFX_REQUIRE(check_common(K, x_row, x_head) && N > 0 && H > 0 && out_head >= N, "headwise_grouped: K=%d, the rows of x (%d) and its heads (%d) must be multiples of 8", K, x_row, x_head);
   if (T <= 0) return 0;
   GroupedArgs a{(const bf16_t*)x, (const bf16_t*)w, out, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                K, N, 1, x_row, x_head, T, 1, out_head, H, H, nullptr, 0, 0.f, 0,
+                K, N, 1, x_row, x_head, T, 1, out_head, H, H, nullptr, 0, 0.f, 0, 0,
                 ColumnGate{gate, gate_ld, gate_col, gate_slices, (size_t)gate_stride}};
-  if (T > 64) hipLaunchKernelGGL((grouped_kernel<MODE_HEADS, 2>), dim3(((T + 127) / 128) * H, (N + TN - 1) / TN), dim3(256), 0, (hipStream_t)stream, a);
-  else hipLaunchKernelGGL((grouped_kernel<MODE_HEADS, 1>), dim3(((T + 63) / 64) * H, (N + TN - 1) / TN), dim3(256), 0, (hipStream_t)stream, a);
+  if (T > 64) hipLaunchKernelGGL((grouped_kernel<MODE_HEADS, 2, false>), dim3(((T + 127) / 128) * H, (N + TN - 1) / TN), dim3(256), 0, (hipStream_t)stream, a);
+  else hipLaunchKernelGGL((grouped_kernel<MODE_HEADS, 1, false>), dim3(((T + 63) / 64) * H, (N + TN - 1) / TN), dim3(256), 0, (hipStream_t)stream, a);
   IFX_LAUNCH_CHECK();
 }

@@ -74,6 +74,7 @@ def module_variants() -> Iterable[Tuple[str, Variant]]:
     yield ("hyper", ())
     yield ("rowwise", ())
     yield ("grouped_gemm", ())
+    yield ("moe_few", ())
     yield ("ceilings", ())            # measurement only: what the memory gives a kernel that just reads
     for d in MFMA_HEAD_DIMS_PREBUILT:
         for qt in TILE_QTS:
@@ -598,6 +599,30 @@ def grouped_takes(dtype: torch.dtype, K: int, ff: int) -> bool:
     return dtype == torch.bfloat16 and K % 8 == 0 and ff % 16 == 0
 
 
+class ExpertTiles:
+    """The experts' matrices [E, N, K] in the tiled form that the streaming products read (``tile_weights`` with tiles of 16
+    rows, N a multiple of 16), instead of their rows: a wave then asks for 1 KB of contiguous memory at a time."""
+
+    __slots__ = ("tiled", "shape")
+
+    def __init__(self, experts: torch.Tensor):
+        E, N, K = experts.shape
+        if experts.dtype != torch.bfloat16 or N % 16 or K % 8:
+            raise KernelError(f"ExpertTiles: {E} experts of {N} x {K} {experts.dtype} (bfloat16, rows a multiple of 16, columns of 8)")
+        self.shape = (E, N, K)
+        self.tiled = tile_weights(experts.reshape(E * N, K), None, 16)
+
+
+def _experts(w, nm: str, shape):
+    """(shape, address, whether tiled) of the experts' matrices, checked."""
+    if isinstance(w, ExpertTiles):
+        if any(want is not None and want != have for want, have in zip(shape, w.shape)):
+            raise KernelError(f"{nm}: shape {w.shape} where {shape} is expected")
+        return w.shape, w.tiled.data_ptr(), 1
+    _check(w, nm, shape, torch.bfloat16)
+    return tuple(w.shape), w.data_ptr(), 0
+
+
 def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor,
                         weights: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0,
                         weigh_input: bool = False) -> "SliceSums":
@@ -608,10 +633,10 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     the row itself (N = K then); ``act``, ``limit`` and ``weigh_input`` as for ``moe_experts``."""
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
-    _check(gate_up, "gate_up", (None, None, K), torch.bfloat16)
-    E, ff = gate_up.shape[0], gate_up.shape[1] // 2
-    _check(down, "down", (E, None, ff), torch.bfloat16)
-    N, top = down.shape[1], ids.shape[1]
+    gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
+    E, ff = gu_shape[0], gu_shape[1] // 2
+    down_shape, down_ptr, down_tiled = _experts(down, "down", (E, None, ff))
+    N, top = down_shape[1], ids.shape[1]
     _check(ids, "ids", (T, top), torch.int32)
     _check(weights, "weights", (T, top), torch.float32)
     if not grouped_takes(h.dtype, K, ff):
@@ -629,15 +654,65 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     _call(mod, "ifx_moe_sort", (P, I, I, I, P, P, P, P, P, P), ids.data_ptr(), n_items, E, tile_items, sorted_.data_ptr(), te.data_ptr(),
           ts.data_ptr(), tc.data_ptr(), nt.data_ptr(), _stream())
     a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)
-    _call(mod, "ifx_moe_gate_up_grouped", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, P),
-          h.data_ptr(), gate_up.data_ptr(), a.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(), tc.data_ptr(),
+    _call(mod, "ifx_moe_gate_up_grouped", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, P),
+          h.data_ptr(), gu_ptr, a.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(), tc.data_ptr(),
           nt.data_ptr(), max_tiles, tile_items, K, ff, top, n_real, int(act), float(limit),
-          weights.data_ptr() if weigh_input else 0, _stream())
+          weights.data_ptr() if weigh_input else 0, gu_tiled, _stream())
     parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, I, P),
-          a.data_ptr(), down.data_ptr(), parts.data_ptr(), weights.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(),
+    _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, I, I, P),
+          a.data_ptr(), down_ptr, parts.data_ptr(), weights.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(),
           tc.data_ptr(), nt.data_ptr(), max_tiles, tile_items, T, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0,
-          _stream())
+          down_tiled, _stream())
+    return SliceSums(parts, torch.bfloat16)
+
+
+MOE_FEW_MAX_ROWS = 64          # rows of a step up to which the experts' weights are streamed once for all of them ...
+MOE_FEW_MAX_EXPERTS = 256      # ... and experts (identity experts among them) the kernel that chooses takes
+
+
+def moe_few_takes(dtype: torch.dtype, T: int, K: int, ff: int, n_routed: int, top: int) -> bool:
+    """Whether ``moe_few`` takes a step of ``T`` rows (beyond, an expert has rows enough for tiles through LDS)."""
+    return grouped_takes(dtype, K, ff) and 0 < T <= MOE_FEW_MAX_ROWS and n_routed <= MOE_FEW_MAX_EXPERTS and top <= 32
+
+
+def moe_few(h: torch.Tensor, router, gate_up: torch.Tensor, down: torch.Tensor, top: int, groups: int = 1, keep_groups: int = 1,
+            group_top: int = 2, softmax: bool = False, renormalize: bool = False, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
+            choice_bias: Optional[torch.Tensor] = None, act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0,
+            weigh_input: bool = False) -> "SliceSums":
+    """``moe_route`` and ``moe_experts`` in one for up to 64 rows in bfloat16: the router's logits as a product (float32 sums
+    and output), a launch that chooses, and two that stream every chosen expert's weights once, whatever the number of rows
+    that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``).  Returns the choices' weighted outputs as ``SliceSums``
+    [top, T, N] like ``moe_experts_grouped``."""
+    _check(h, "h", (None, None), torch.bfloat16)
+    T, K = h.shape
+    gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
+    n_real, ff = gu_shape[0], gu_shape[1] // 2
+    down_shape, down_ptr, down_tiled = _experts(down, "down", (n_real, None, ff))
+    N, E = down_shape[1], n_real + int(n_identity)
+    rows = router.rows if isinstance(router, LinearWeight) else router
+    _check(rows, "router", (E, K), torch.bfloat16)
+    if not moe_few_takes(h.dtype, T, K, ff, E, top):
+        raise KernelError(f"moe_few: {T} rows (at most {MOE_FEW_MAX_ROWS}), {E} experts (at most {MOE_FEW_MAX_EXPERTS}), K={K} (a multiple of 8), ff={ff} (of 16)")
+    if n_identity and N != K:
+        raise KernelError(f"moe_few: identity experts hand back the row itself, so N={N} must equal K={K}")
+    for t, nm in ((bias, "bias"), (choice_bias, "choice_bias")):
+        if t is not None:
+            _check(t, nm, (E,), torch.float32)
+    mod, stream = load_module("moe_few"), _stream()
+    slices = mod.fn("ifx_moe_logit_slices", (I,))(K)
+    z = torch.empty((slices, T, E), dtype=torch.float32, device=h.device)
+    _call(mod, "ifx_moe_logits", (P, P, P, I, I, I, P), h.data_ptr(), rows.data_ptr(), z.data_ptr(), T, K, E, stream)
+    n_items = T * top
+    ids = torch.empty((n_items,), dtype=torch.int32, device=h.device)
+    weights = torch.empty((n_items,), dtype=torch.float32, device=h.device)
+    _call(mod, "ifx_moe_choose", (P, I, P, P, I, I, I, I, I, I, I, I, F, P, P, P), z.data_ptr(), slices, ids.data_ptr(), weights.data_ptr(),
+          T, E, top, groups, keep_groups, group_top, 1 if softmax else 0, 1 if renormalize else 0, float(scale), _ptr(bias), _ptr(choice_bias), stream)
+    a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)
+    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
+          T, E, K, ff, top, n_real, int(act), float(limit), weights.data_ptr() if weigh_input else 0, gu_tiled, stream)
+    parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
+    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P), a.data_ptr(), down_ptr, parts.data_ptr(),
+          weights.data_ptr(), ids.data_ptr(), T, E, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0, down_tiled, stream)
     return SliceSums(parts, torch.bfloat16)
 
 

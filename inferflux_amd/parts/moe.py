@@ -22,7 +22,7 @@ in float, to the sums of the gate and up products before the activation).
 
 Tensors (``<name>.``): router [experts + identity, H] (router.b [experts], correction [experts + identity]), e<j>.gate and e<j>.up [ff, H], e<j>.down [H, ff]; shared.gate,
 shared.up, shared.down, shared.sg [1, H]; no other biases.  The experts' matrices are stacked at load into [experts, ff, H]
-and [experts, H, ff].
+and [experts, H, ff] (in bfloat16 into the tiled form that the streaming products read).
 
 The router and the choice run on the device, and the experts' products read each (row, choice)'s expert from device
 memory: the launches of a step depend on its layout alone, so a decode step is captured and replayed like any other.
@@ -39,8 +39,9 @@ from .ffn import GATED_ACTIVATIONS, SwiGLU
 from .plan import ParamSpec
 
 
-# (row, choice) items of a step from which the experts' products go to the matrix cores, tiles of items of one expert
-# against that expert's weights; below, every item streams its expert's weights by itself
+# (row, choice) items of a step from which the experts' products take tiles of items of one expert against that expert's
+# weights where the products for few rows do not take them (more than 256 experts); below, every item streams its expert's
+# weights by itself
 GROUPED_MIN_ITEMS = 64
 
 
@@ -113,6 +114,9 @@ class MixtureOfExperts(FeedForward):
         if self.gate.is_cuda and ops.grouped_takes(dtype, self.hidden_size, self.ff):
             # one tensor that both products read: rows of gate and up in turns of 16
             self.gate, self.up = ops.pair_gate_up(self.gate, self.up), None
+            if self.hidden_size % 16 == 0 and ops.moe_few_takes(dtype, 1, self.hidden_size, self.ff, self.n_routed, self.top):
+                # ... and both products in tiles: nothing reads rows then
+                self.gate, self.down = ops.ExpertTiles(self.gate), ops.ExpertTiles(self.down)
 
         if self.router_bias:
             self.bias = tensors[f"{n}.router.b"].float().contiguous()        # the router is float whatever the file holds
@@ -134,10 +138,15 @@ class MixtureOfExperts(FeedForward):
 
     def forward(self, h, ctx):
         x = h if h.dtype == self.router.dtype else h.to(self.router.dtype)
+        if self.up is None and ops.moe_few_takes(x.dtype, x.shape[0], self.hidden_size, self.ff, self.n_routed, self.top):
+            return self._with_shared(ops.moe_few(x, self.router, self.gate, self.down, self.top, self.groups, self.keep_groups,
+                                                 self.group_top, self.scoring == "softmax", self.renormalize, self.route_scale,
+                                                 self.bias, self.correction, self.act, self.limit, self.n_identity,
+                                                 self.weigh_input), x, ctx)      # (partial sums, one per choice)
         ids, weights = self.route(x)
         if ctx.timer is not None:
             ctx.timer.mark("ffn.route")
-        if self.up is None and x.shape[0] * self.top >= GROUPED_MIN_ITEMS:
+        if self.up is None and (isinstance(self.gate, ops.ExpertTiles) or x.shape[0] * self.top >= GROUPED_MIN_ITEMS):
             return self._with_shared(ops.moe_experts_grouped(x, self.gate, self.down, ids, weights, self.act, self.limit,
                                                              self.n_identity, self.weigh_input), x, ctx)      # (partial sums, one per choice)
         out = self._with_shared(ops.moe_experts(x, self.gate, self.up, self.down, ids, weights, self.act, self.limit,

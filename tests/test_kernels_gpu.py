@@ -464,6 +464,60 @@ def test_gemm_f32_kernels_agree_bit_for_bit(N, K, adtype):
     assert torch.equal(ops.gemm_f32(shifted, w, None, F32), whole)
 
 
+# ---- mixtures of experts for few rows ---------------------------------------------------------
+@pytest.mark.parametrize("T", [1, 3, 16, 17, 33, 64])
+@pytest.mark.parametrize("E,identity,top,K,ff,groups,keep,group_top", [
+    (3, 0, 2, 64, 16, 1, 1, 2), (64, 0, 6, 200, 48, 8, 4, 2), (61, 4, 3, 512, 80, 1, 1, 2), (65, 0, 32, 128, 32, 5, 4, 3),
+    (256, 0, 5, 2048, 16, 32, 6, 8)])
+@pytest.mark.parametrize("form", ["tiles", "rows", "softmax", "input"])
+def test_moe_few(T, E, identity, top, K, ff, groups, keep, group_top, form):
+    """Rows on both sides of a column tile, experts on both sides of a wave, K and ff that end within a block of 64: against 64
+    bits.  The experts' outputs are sums of K or ff products of bfloat16 values in float, with one rounding to bfloat16 (2^-8)
+    between the two products.  Rows whose choice is closer than the logits' rounding are left out."""
+    g = gen(2200 + T + E)
+    N = K
+    h = torch.randn(T, K, generator=g).to(BF16)
+    router = (torch.randn(E + identity, K, generator=g) / K ** 0.5).to(BF16)
+    gate, up = ((torch.randn(E, ff, K, generator=g) / K ** 0.5).to(BF16) for _ in range(2))
+    down = (torch.randn(E, N, ff, generator=g) / ff ** 0.5).to(BF16)
+    softmax, weigh_input = form == "softmax", form == "input"
+    correction = torch.randn(E + identity, generator=g) * 0.01 if softmax else None
+    z = h.double() @ router.double().t()
+    s = z.softmax(-1) if softmax else z.sigmoid()
+    c = s + correction.double() if softmax else s
+    worth = c.view(T, groups, -1).topk(min(group_top, (E + identity) // groups), -1).values.sum(-1)
+    by_worth = worth.sort(-1, descending=True)
+    kept = torch.zeros_like(worth).scatter(1, by_worth.indices[:, :keep], 1.0).bool()
+    c = c.view(T, groups, -1).masked_fill(~kept[..., None], -9.0).view(T, -1)
+    best = c.sort(-1, descending=True)
+    ids, weights = best.indices[:, :top], s.gather(1, best.indices[:, :top])
+    clear = torch.ones(T, dtype=torch.bool) if top == E + identity else best.values[:, top - 1] - best.values[:, top] > 1e-5
+    if keep < groups:
+        clear &= by_worth.values[:, keep - 1] - by_worth.values[:, keep] > 1e-5
+    want = torch.zeros(T, N, dtype=torch.float64)
+    for t in range(T):
+        for e, w in zip(ids[t].tolist(), weights[t]):
+            if e >= E:
+                want[t] += w * h[t].double()
+                continue
+            wi, wo = (w, 1.0) if weigh_input else (1.0, w)
+            a = torch.nn.functional.silu(wi * (gate[e].double() @ h[t].double())) * (wi * (up[e].double() @ h[t].double()))
+            want[t] += wo * (down[e].double() @ a)
+    pairs, d = ops.pair_gate_up(gate.to(DEV), up.to(DEV)), down.to(DEV)
+    if form == "tiles" and N % 16 == 0:
+        pairs, d = ops.ExpertTiles(pairs), ops.ExpertTiles(d)
+    got = ops.moe_few(h.to(DEV), router.to(DEV), pairs, d, top, groups, keep, group_top, softmax=softmax,
+                      choice_bias=correction.to(DEV) if softmax else None, n_identity=identity, weigh_input=weigh_input)
+    assert got.parts.shape == (top, T, N)
+    out = got.sum(F32).cpu().double()
+    assert clear.sum() >= T // 2
+    size = want[clear].pow(2).mean().sqrt()
+    # (a rounding of at most half a unit of 8 bits, 2^-8, of each activation: no more than that of the result in the mean square
+    # over the outputs, which share the activations; 5 x for the largest)
+    assert (out - want)[clear].pow(2).mean().sqrt() < 2.0 ** -8 * size
+    assert (out - want)[clear].abs().max() < 5 * 2.0 ** -8 * max(size, want[clear].abs().max())
+
+
 # ---- sampling -------------------------------------------------------------------------------
 def test_argmax_lowest_index_wins_ties():
     l = torch.zeros(3, 1500)
