@@ -58,13 +58,30 @@ __device__ __forceinline__ float sum_over_groups(float v) {
   return v;
 }
 
+// The row factors gathered by a workgroup of several waves: each wave leaves its share of the rows' sums of squares in LDS
+// (``leave_row_sums``, before the workgroup's barrier), the first wave adds the shares in wave order (after it).
+__device__ __forceinline__ float* row_sum_shares() {
+  __shared__ __attribute__((aligned(16))) float shares[16][16];
+  return &shares[0][0];
+}
+__device__ __forceinline__ void leave_row_sums(const RowScale& s, const RowSumsEarly& early, int wave, int lane) {
+  const rs_floatx4 t = row_sums_of_wave(row_sums_of_thread(s, threadIdx.x, blockDim.x, early));
+  if (lane < 4) *(rs_floatx4*)(row_sum_shares() + 16 * wave + 4 * lane) = t;
+}
+__device__ __forceinline__ float gathered_row_factor(const RowScale& s, int col) {
+  float sum = 0.f;
+  for (int w = 0; w < (int)blockDim.x / WAVE; ++w) sum += row_sum_shares()[16 * w + col];
+  return rsqrtf(sum / s.width + s.eps);
+}
+
 // The sums of one workgroup: acc[nt][mt] = W tile (first_tile + nt) times x rows 16 mt ..., K split over
 // the workgroup's waves and added through LDS in wave order.  Returns true in the wave that holds the
 // sums (wave 0); the others are done.
-template <int MT, int NT, int U, bool TILED>
+// ``before_meeting(wave)`` is called once in every wave, after its last products are started and before the workgroup's barrier.
+template <int MT, int NT, int U, bool TILED, typename F>
 __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N,
                                                   int K, int k_tiles, int first_tile, floatx4 (&acc)[NT][MT], float* red,
-                                                  int tile_rows = 16) {
+                                                  int tile_rows, F before_meeting) {
   const int wid = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x % WAVE;
   const int col = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -119,6 +136,7 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
             acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][nt][h], xa[u][mt][h], acc[nt][mt], 0, 0, 0);
   }
 
+  before_meeting(wid);
   if (nw > 1) {
     if (wid > 0) {
 #pragma unroll
@@ -160,7 +178,13 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* _
   const int first_tile = blockIdx.x * NT, n_tiles = (N + tile_rows - 1) / tile_rows;
   const bool first_wave = threadIdx.x < WAVE;
   float rs = 1.f;
-  if (MT == 1 && scale.pieces && first_wave) rs = row_factor(scale, lane);
+  // The rows' factors: every thread of a workgroup of several waves asks for its share of the sums of squares ahead of the
+  // weights and adds it up after them, so that they cost no trip to the L2 of their own (computed by the first wave before its
+  // first weights they cost 1 us a product).
+  const bool shared_sums = MT == 1 && scale.pieces && blockDim.x > WAVE;
+  RowSumsEarly early;
+  if (shared_sums) row_sums_ask(scale, threadIdx.x, blockDim.x, early);
+  else if (MT == 1 && scale.pieces) rs = row_factor(scale, lane);
   // The lane's four sums of a tile are rows 4 g ... 4 g + 3 of it, handled as two pairs: tile_rows is even, so a
   // pair is held or not as a whole, and a pair's first column is even.
   // EPI 2: what the epilogue reads is asked for before the stream of weights, not after it
@@ -184,7 +208,10 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* _
   }
   floatx4 acc[NT][MT];
   if (xb.tiles > 0) x += (size_t)min(first_tile / xb.tiles, xb.n - 1) * M * K;
-  if (!skinny_accumulate<MT, NT, U, TILED>(x, W, M, N, K, k_tiles, first_tile, acc, red, tile_rows)) return;
+  if (!skinny_accumulate<MT, NT, U, TILED>(x, W, M, N, K, k_tiles, first_tile, acc, red, tile_rows, [&](int wave) {
+        if (shared_sums) leave_row_sums(scale, early, wave, lane);
+      })) return;
+  if (shared_sums) rs = gathered_row_factor(scale, col);
   // acc[nt][mt][r] = out[m = 16 mt + col][n = tile_rows (row tile of the weight) + 4 g + r], for 4 g + r < tile_rows
   if (EPI == 2) {
 #pragma unroll
@@ -263,9 +290,15 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
   extern __shared__ float red[];
   const int lane = threadIdx.x % WAVE, col = lane & 15, g = lane >> 4;
   float rs = 1.f;
-  if (scale.pieces && threadIdx.x < WAVE) rs = row_factor(scale, lane);
+  const bool shared_sums = scale.pieces && blockDim.x > WAVE;        // (as in skinny_gemm_kernel)
+  RowSumsEarly early;
+  if (shared_sums) row_sums_ask(scale, threadIdx.x, blockDim.x, early);
+  else if (scale.pieces) rs = row_factor(scale, lane);
   floatx4 acc[2][1];
-  if (!skinny_accumulate<1, 2, U, true>(x, W, M, N, K, k_tiles, 2 * blockIdx.x, acc, red)) return;
+  if (!skinny_accumulate<1, 2, U, true>(x, W, M, N, K, k_tiles, 2 * blockIdx.x, acc, red, 16, [&](int wave) {
+        if (shared_sums) leave_row_sums(scale, early, wave, lane);
+      })) return;
+  if (shared_sums) rs = gathered_row_factor(scale, col);
   const int m = col;
   if (m >= M) return;
   const int d = a.d, half = d / 2, per_head = d / 32;
