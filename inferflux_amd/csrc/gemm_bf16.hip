@@ -294,28 +294,44 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
   RowSumsEarly early;
   if (shared_sums) row_sums_ask(scale, threadIdx.x, blockDim.x, early);
   else if (scale.pieces) rs = row_factor(scale, lane);
+  // What the epilogue reads is asked for before the stream of weights, not after it (the first wave holds the sums).
+  const int m = col, d = a.d, half = d / 2, per_head = d / 32;
+  const int head = blockIdx.x / per_head, i0 = 16 * (blockIdx.x % per_head) + 4 * g;   // the lane's pairs: i0 + r and i0 + r + half
+  const bool is_q = head < a.nH, is_v = head >= a.nH + a.nKV;
+  // (the bias as it lies in memory, widened where it is used: a conversion here would wait for its load ahead of the weights)
+  union Bias { floatx4 f; bf16x4 h; };
+  Bias b0, b1;
+  b0.f = b1.f = floatx4{0.f, 0.f, 0.f, 0.f};
+  floatx4 cs{1.f, 1.f, 1.f, 1.f}, sn{0.f, 0.f, 0.f, 0.f};
+  int slot = -1;
+  if (threadIdx.x < WAVE && m < M) {
+    const size_t at = (size_t)head * d + i0;
+    if (a.bias && a.bias_dtype == DT_F32) {
+      b0.f = *(const floatx4*)((const float*)a.bias + at);
+      b1.f = *(const floatx4*)((const float*)a.bias + at + half);
+    } else if (a.bias) {
+      b0.h = *(const bf16x4*)((const bf16_t*)a.bias + at);
+      b1.h = *(const bf16x4*)((const bf16_t*)a.bias + at + half);
+    }
+    if (!is_v) {
+      cs = *(const floatx4*)(a.cs + (size_t)m * half + i0);
+      sn = *(const floatx4*)(a.sn + (size_t)m * half + i0);
+    }
+    if (!is_q && a.slots) slot = a.slots[m];
+  }
   floatx4 acc[2][1];
   if (!skinny_accumulate<1, 2, U, true>(x, W, M, N, K, k_tiles, 2 * blockIdx.x, acc, red, 16, [&](int wave) {
         if (shared_sums) leave_row_sums(scale, early, wave, lane);
       })) return;
   if (shared_sums) rs = gathered_row_factor(scale, col);
-  const int m = col;
   if (m >= M) return;
-  const int d = a.d, half = d / 2, per_head = d / 32;
-  const int head = blockIdx.x / per_head, i0 = 16 * (blockIdx.x % per_head) + 4 * g;   // the lane's pairs: i0 + r and i0 + r + half
   float x0[4], x1[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    x0[r] = acc[0][0][r] * rs;
-    x1[r] = acc[1][0][r] * rs;
-    if (a.bias) {
-      x0[r] += load_dyn(a.bias, a.bias_dtype, (size_t)head * d + i0 + r);
-      x1[r] += load_dyn(a.bias, a.bias_dtype, (size_t)head * d + half + i0 + r);
-    }
+    x0[r] = acc[0][0][r] * rs + (a.bias_dtype == DT_F32 ? b0.f[r] : (float)b0.h[r]);
+    x1[r] = acc[1][0][r] * rs + (a.bias_dtype == DT_F32 ? b1.f[r] : (float)b1.h[r]);
   }
-  const bool is_v = head >= a.nH + a.nKV;
   if (!is_v) {
-    const floatx4 cs = *(const floatx4*)(a.cs + (size_t)m * half + i0), sn = *(const floatx4*)(a.sn + (size_t)m * half + i0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float y0 = x0[r] * cs[r] - x1[r] * sn[r], y1 = x0[r] * sn[r] + x1[r] * cs[r];
@@ -326,13 +342,12 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
   bf16x4 lo, hi;
 #pragma unroll
   for (int r = 0; r < 4; ++r) { lo[r] = (__bf16)x0[r]; hi[r] = (__bf16)x1[r]; }
-  if (head < a.nH) {
+  if (is_q) {
     bf16_t* dst = a.q_out + ((size_t)m * a.nH + head) * d + i0;
     *(bf16x4*)dst = lo;
     *(bf16x4*)(dst + half) = hi;
     return;
   }
-  const int slot = a.slots ? a.slots[m] : -1;
   if (slot < 0) return;
   const int page = slot / a.P, off = slot % a.P;
   if (!is_v) {
@@ -424,6 +439,7 @@ extern "C" int ifx_qkv_rope(const void* x, const void* Wt, int M, int K, const v
   IFX_REQUIRE(cs && sn && q_out, "qkv_rope: needs the rotation table and an output");
   IFX_REQUIRE(!slots || (page_size > 0 && k_cache && v_cache), "qkv_rope: cache write without cache");
   IFX_REQUIRE(bias_dtype == DT_BF16 || bias_dtype == DT_F32 || !bias, "qkv_rope: unknown bias dtype %d", bias_dtype);
+  IFX_REQUIRE((uintptr_t)bias % 16 == 0, "qkv_rope: the bias must start on 16 bytes");
   if (M == 0) return 0;
   const int heads = nH + (slots ? 2 * nKV : 0), N = heads * d, groups = N / 32;
   const int nkb = (K + 63) / 64, k_tiles = ifx_tiled_cols(K) / 32;

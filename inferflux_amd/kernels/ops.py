@@ -1042,6 +1042,8 @@ def qkv_rope_append(x: torch.Tensor, weight: LinearWeight, bias: Optional[torch.
     _check(sin, "sin", (M, head_dim // 2), torch.float32)
     if bias is not None:
         _check(bias, "bias", (heads * head_dim,))
+        if bias.data_ptr() % 16:          # (a part of a larger tensor: the kernel reads four elements at a time)
+            bias = bias.clone()
     if slots is not None:
         _check(slots, "slots", (M,), torch.int32)
         _check(k_cache, "k_cache", (None, n_kv_heads, page_size, head_dim), torch.bfloat16)
