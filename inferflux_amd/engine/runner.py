@@ -41,7 +41,10 @@ class _DecodeGraph:
 
 class ModelRunner:
     GRAPH_WIDTH_MULTIPLE = 64     # block-table width (pages) a captured step is valid for, in steps of this
-    MAX_GRAPHS = 24               # captured layouts kept; the one unused longest goes first
+    # ... but for steps whose requests all hold few tokens, whose tables are as wide as these many: attention over few keys
+    # has a launch of its own shape (see kernels.attention.row_launch_shape), which a layout that allows 1,024 cannot take.
+    GRAPH_SHORT_TOKENS = (256, 512)
+    MAX_GRAPHS = 32               # captured layouts kept; the one unused longest goes first
     # A captured step is valid for one number of rows.  A batch that shrinks a request at a time would need a capture
     # (a wait for the GPU, an eager step, the capture: tens of milliseconds) for every size it passes through, so the
     # batch of a captured step is filled up to the next of these sizes with rows that stand for nobody (they write
@@ -135,10 +138,13 @@ class ModelRunner:
 
     def _decode_context(self, entries) -> StepContext:
         """The context of a step of single tokens in the layout its captured graph has: block tables as wide as the
-        next multiple of GRAPH_WIDTH_MULTIPLE pages, the batch filled up to the next of GRAPH_BATCH_SIZES."""
+        next multiple of GRAPH_WIDTH_MULTIPLE pages (or the next of GRAPH_SHORT_TOKENS), the batch filled up to the next of GRAPH_BATCH_SIZES."""
         n = len(entries)
+        longest = max((self.manager.length(e.rid) for e in entries), default=0) + 1
+        short = next((t for t in self.GRAPH_SHORT_TOKENS if longest <= t and t % self.page_size == 0), None)
+        width = min(short // self.page_size, self.GRAPH_WIDTH_MULTIPLE) if short else self.GRAPH_WIDTH_MULTIPLE
         size = next((b for b in self.GRAPH_BATCH_SIZES if b >= n), -(-n // 16) * 16)
-        return StepContext(entries, self.manager, self.dtype, self.device, width_multiple=self.GRAPH_WIDTH_MULTIPLE,
+        return StepContext(entries, self.manager, self.dtype, self.device, width_multiple=width,
                            upload=False, pad_requests=size - n, scratch_pages=self.storage.scratch_pages,
                            scratch_state_slot=self.storage.scratch_state_slot)
 

@@ -37,6 +37,8 @@ ROW_MAX_SPLITS = 512       # launch shares a row of many splits among up to 8 wa
                            # merge of one wave; over 3,100 keys 11.8 us in 49 splits of 64 against 13.7 in 25 of 128).
 ROW_WHOLE_MIN_PAIRS = 192   # (row, kv head) pairs from which a workgroup takes a pair's keys whole
 ROW_WAVE_SLOTS = 2048       # waves the chip holds at the row kernel's two per SIMD
+ROW_WHOLE_SHORT = 256       # keys (of 128 elements: twice as many of 64) up to which it does so whatever the number of pairs ...
+ROW_WHOLE_SHORT_PAIRS = 96  # ... and pairs from which it does up to twice as many
 
 
 DIRECT_MIN_WORK = 1 << 18       # rows x keys seen per row from which the tall tiles of head size 128 win
@@ -158,7 +160,7 @@ def tile_order(first_pos, last_pos, n_heads: int, window: Optional[int], splits:
     return order.reshape(-1)
 
 
-def _work_lists(ctx, ctx_kv_heads, tile_rows, n_heads, tile_splits=1, tile_chunk=0, window=None, row_waves=8):
+def _work_lists(ctx, ctx_kv_heads, tile_rows, n_heads, tile_splits=1, tile_chunk=0, window=None, row_waves=8, head_dim=128):
     """What the kernels need beyond the step's own arrays, computed once per step (and per number of
     kv heads, which decides how many waves a launch has)."""
     q_len, q_start, kv_len = ctx.h_q_len, ctx.h_q_start, ctx.h_kv_len
@@ -194,11 +196,11 @@ def _work_lists(ctx, ctx_kv_heads, tile_rows, n_heads, tile_splits=1, tile_chunk
             out[k] = packed[at:at + n]
             at += n + -n % 4          # every list starts at a multiple of 16 bytes
     if rows.size:
-        out["chunk"], out["waves"], out["max_splits"] = row_launch_shape(int(rows.size), ctx_kv_heads, ctx.kv_bound, row_waves)
+        out["chunk"], out["waves"], out["max_splits"] = row_launch_shape(int(rows.size), ctx_kv_heads, ctx.kv_bound, row_waves, head_dim)
     return out
 
 
-def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int = 8):
+def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int = 8, head_dim: int = 128):
     """(keys per split, waves per workgroup, splits) of a launch of the row kernel over ``n_rows`` rows whose requests
     hold at most ``max_kv`` keys (the bound of their block tables, not the lengths themselves: see
     StepContext.kv_bound).  ``max_waves``: what fits the kernel's LDS (``ops.row_waves_fit``).
@@ -209,9 +211,14 @@ def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int =
     3,100 keys, us whole / in splits with the merge launch: 48 rows 61 / 69, 64 rows 68 / 88, 96 rows 116 / 133, 128
     rows 129 / 178, 256 rows 250 / 361; 64 rows over 16,384 keys 328 / 358; 32 rows 57 / 48, so fewer pairs than 192
     keep the splits: their keys have to be spread over more compute units than there are pairs, which only a second
-    launch can merge (one wave per split of ``chunk`` keys, waves per workgroup 0)."""
+    launch can merge (one wave per split of ``chunk`` keys, waves per workgroup 0).
+
+    Rows of few keys take a workgroup each too: a compute unit reads 256 keys in less time than the second launch takes.
+    us whole / in splits at 64 and 300 keys: 14 : 2 heads of 64, 1 row 4.5, 6.3 / 8.1; 16 : 2 heads of 128, 8 rows 5.6,
+    10.2 / 11.2, 64 rows 6.1, 11.3 / 14.4, 19.9; 16 heads on one of 128, 8 rows (four waves fit) 5.6, 11.5 / 10.7."""
     pairs = n_rows * n_kv_heads
-    if pairs >= ROW_WHOLE_MIN_PAIRS:
+    short = ROW_WHOLE_SHORT if head_dim > 64 and pairs < ROW_WHOLE_SHORT_PAIRS else 2 * ROW_WHOLE_SHORT
+    if pairs >= ROW_WHOLE_MIN_PAIRS or max_kv <= short:
         waves = 1
         while waves * 2 <= min(max_waves, ROW_WAVE_SLOTS // pairs):
             waves *= 2
@@ -253,7 +260,7 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
                                           tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not other)
     tile_rows = ops.attention_tile_rows(d, qt)
     w = ctx.derived(("attention_work_lists", n_kv, tile_rows, nH, splits, chunk, window, d),
-                    lambda: _work_lists(ctx, n_kv, tile_rows, nH, splits, chunk, window, ops.row_waves_fit(nH, n_kv, d, ops.ROW_MAX_WAVES)))
+                    lambda: _work_lists(ctx, n_kv, tile_rows, nH, splits, chunk, window, ops.row_waves_fit(nH, n_kv, d, ops.ROW_MAX_WAVES), d))
     out = torch.empty((T, nH * d), dtype=q.dtype, device=q.device)
     more = dict(keep_first=keep_first, sink=sink, gate=gate, sinks=sinks, block=block) if extras else {}
     if w["n_tiles"]:
