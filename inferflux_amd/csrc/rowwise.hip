@@ -152,6 +152,63 @@ __global__ __launch_bounds__(256) void gated_add_kernel(const void* __restrict__
   }
 }
 
+// The same in bfloat16 for widths of multiples of 4 (and K of 8): a workgroup takes 1,024 columns of a row and asks for everything
+// it needs at once, the partial sums eight at a time (2,048 columns, one row, four slices: 9.8 us above).
+__global__ __launch_bounds__(256) void gated_add4_kernel(const void* __restrict__ base, int base_f32, int n_slices, size_t slice_stride,
+                                                         const void* __restrict__ extra, int extra_f32, int extra_slices, size_t extra_stride,
+                                                         const bf16_t* __restrict__ h, const bf16_t* __restrict__ w, int K,
+                                                         bf16_t* __restrict__ out, int N) {
+  typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+  union Raw { float4 f; bf16x4 h; };
+  __shared__ float red[16];
+  const size_t t = blockIdx.x;
+  const int c = 4 * (blockIdx.y * 256 + threadIdx.x);
+  constexpr int AT_ONCE = 8;
+  Raw b[AT_ONCE], e[AT_ONCE];
+  auto ask = [&](const void* p, int f32, int slices, size_t stride, int k0, Raw* r) {
+    if (c >= N) return;
+    if (!f32) {
+      if (k0 == 0) r[0].h = *(const bf16x4*)((const bf16_t*)p + t * N + c);
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u)
+      if (k0 + u < slices) r[u].f = *(const float4*)((const float*)p + (size_t)(k0 + u) * stride + t * N + c);
+  };
+  auto add = [&](int f32, int slices, int k0, const Raw* r, float* v) {
+    if (!f32) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (float)r[0].h[i];
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u)
+      if (k0 + u < slices) { v[0] += r[u].f.x; v[1] += r[u].f.y; v[2] += r[u].f.z; v[3] += r[u].f.w; }
+  };
+  ask(base, base_f32, n_slices, slice_stride, 0, b);
+  ask(extra, extra_f32, extra_slices, extra_stride, 0, e);
+  float gate = 1.0f;
+  if (w) {
+    float z = 0.f;
+    for (int k = 8 * threadIdx.x; k < K; k += 8 * 256) {
+      const row_bf16x8 x8 = *(const row_bf16x8*)(h + t * K + k), w8 = *(const row_bf16x8*)(w + k);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) z = fmaf((float)x8[i], (float)w8[i], z);
+    }
+    gate = 1.0f / (1.0f + expf(-block_sum(z, red)));
+  }
+  float bv[4] = {0.f, 0.f, 0.f, 0.f}, ev[4] = {0.f, 0.f, 0.f, 0.f};
+  add(base_f32, n_slices, 0, b, bv);
+  add(extra_f32, extra_slices, 0, e, ev);
+  for (int k0 = AT_ONCE; k0 < n_slices; k0 += AT_ONCE) { ask(base, base_f32, n_slices, slice_stride, k0, b); add(base_f32, n_slices, k0, b, bv); }
+  for (int k0 = AT_ONCE; k0 < extra_slices; k0 += AT_ONCE) { ask(extra, extra_f32, extra_slices, extra_stride, k0, e); add(extra_f32, extra_slices, k0, e, ev); }
+  if (c >= N) return;
+  bf16x4 y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = (__bf16)fmaf(gate, ev[i], bv[i]);
+  *(bf16x4*)(out + t * N + c) = y;
+}
+
 extern "C" int ifx_gated_add(const void* base, int base_f32, int n_slices, long long slice_stride, const void* extra, int extra_f32,
                              int extra_slices, long long extra_stride, const void* h, const void* w, int K, void* out, int dtype,
                              int T, int N, void* stream) {
@@ -159,7 +216,13 @@ extern "C" int ifx_gated_add(const void* base, int base_f32, int n_slices, long 
   IFX_REQUIRE((n_slices == 1 || base_f32) && (extra_slices == 1 || extra_f32), "gated_add: partial sums are float");
   if (T == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == DT_BF16)
+  // (operands on 16 bytes, for loads of four and eight elements)
+  const bool fours = dtype == DT_BF16 && N % 4 == 0 && K % 8 == 0 && slice_stride % 4 == 0 && extra_stride % 4 == 0 && N <= 4 * 256 * 65535ll &&
+                     ((uintptr_t)base | (uintptr_t)extra | (uintptr_t)h | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
+  if (fours)
+    hipLaunchKernelGGL(gated_add4_kernel, dim3(T, (N + 1023) / 1024), dim3(256), 0, s, base, base_f32, n_slices, (size_t)slice_stride, extra,
+                       extra_f32, extra_slices, (size_t)extra_stride, (const bf16_t*)h, (const bf16_t*)w, K, (bf16_t*)out, N);
+  else if (dtype == DT_BF16)
     hipLaunchKernelGGL(gated_add_kernel<bf16_t>, dim3(T), dim3(256), 0, s, base, base_f32, n_slices, (size_t)slice_stride, extra, extra_f32,
                        extra_slices, (size_t)extra_stride, (const bf16_t*)h, (const bf16_t*)w, K, (bf16_t*)out, N);
   else if (dtype == DT_F32)
