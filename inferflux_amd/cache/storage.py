@@ -15,6 +15,7 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
+from ..kernels import ops
 from ..parts.base import LayerCache, MixerBinding
 from .manager import CacheManager, GroupSpec
 
@@ -76,6 +77,7 @@ class CacheStorage:
             st = m.state_spec()
             if st is not None:
                 self._states[i] = torch.zeros((max_requests + 1, *st.shape), dtype=_STATE_DTYPES[st.dtype], device=device)
+        self._slot_table = ops.slot_table(list(self._states.values())) if self._states and torch.device(device).type == "cuda" else None
         if self._states:
             self.manager.on_add = self.reset_state       # every admission path starts a request with zero state
         self._bindings: List[MixerBinding] = []
@@ -94,6 +96,9 @@ class CacheStorage:
 
     def reset_state(self, slot: int) -> None:
         """Zero every mixer's state of one slot: a request that starts sees no history."""
+        if self._slot_table is not None:
+            ops.zero_slot(self._slot_table, slot, self.scratch_state_slot + 1)
+            return
         for t in self._states.values():
             t[slot].zero_()
 

@@ -48,7 +48,7 @@ struct StreamOut {
 };
 
 // A product whose weight's row tiles come in blocks that read inputs of their own: row tile t meets x + min(t / tiles, n - 1) * M * K
-// (x holds n inputs [M, K] end to end; tiles 0: one input for all).
+// (x holds n inputs [M, K] end to end; tiles 0: one input for all, whose rows are n elements apart, n 0: K).
 struct XBlocks { int tiles, n; };
 
 // Sum over the four lanes col, col + 16, col + 32, col + 48, the same in all four.
@@ -81,7 +81,7 @@ __device__ __forceinline__ float gathered_row_factor(const RowScale& s, int col)
 template <int MT, int NT, int U, bool TILED, typename F>
 __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N,
                                                   int K, int k_tiles, int first_tile, floatx4 (&acc)[NT][MT], float* red,
-                                                  int tile_rows, F before_meeting) {
+                                                  int tile_rows, int ldx, F before_meeting) {
   const int wid = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x % WAVE;
   const int col = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -100,7 +100,7 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     xok[mt] = 16 * mt + col < M;
-    xrow[mt] = x + (size_t)(xok[mt] ? 16 * mt + col : 0) * K;
+    xrow[mt] = x + (size_t)(xok[mt] ? 16 * mt + col : 0) * ldx;
   }
 
   const int nkb = (K + 63) / 64;
@@ -162,7 +162,7 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
 
 // EPI 0: out[m, n] = acc.  EPI 1: the rows of W alternate gate, up, gate, up ...; a lane holds two
 // such pairs of one output row and writes silu(gate) * up to out[m, n / 2] (out is [M, N / 2]).
-// EPI 2 (up to 16 rows, N a multiple of 4): see StreamOut; ``out`` is not used.  EPI 4: out[m, n] = max(acc, 0)^2.
+// EPI 2 (up to 16 rows, N a multiple of 4): see StreamOut; ``out`` is not used.  EPI 4: out[m, n] = max(acc, 0)^2.  EPI 5: gelu(acc).
 // ``order`` (tiled copies only): tile t of the copy holds the weight's rows 16 order[t] ...; null: in order.
 // ``scale`` (up to 16 rows): the results of row m are multiplied by the row's factor first.
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
@@ -208,7 +208,7 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* _
   }
   floatx4 acc[NT][MT];
   if (xb.tiles > 0) x += (size_t)min(first_tile / xb.tiles, xb.n - 1) * M * K;
-  if (!skinny_accumulate<MT, NT, U, TILED>(x, W, M, N, K, k_tiles, first_tile, acc, red, tile_rows, [&](int wave) {
+  if (!skinny_accumulate<MT, NT, U, TILED>(x, W, M, N, K, k_tiles, first_tile, acc, red, tile_rows, xb.tiles == 0 && xb.n > 0 ? xb.n : K, [&](int wave) {
         if (shared_sums) leave_row_sums(scale, early, wave, lane);
       })) return;
   if (shared_sums) rs = gathered_row_factor(scale, col);
@@ -247,12 +247,12 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* _
     for (int mt = 0; mt < MT; ++mt) {
       const int m = 16 * mt + col;
       if (m >= M) continue;
-      if (EPI == 0 || EPI == 4) {
+      if (EPI == 0 || EPI == 4 || EPI == 5) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int n = n0 + 4 * g + r;
           const float v = acc[nt][mt][r] * rs;
-          if (4 * g + r < tile_rows && n < N) out[(size_t)m * N + n] = from_f<TO>(EPI == 4 ? plain_act(v, ACT_RELU_SQUARED) : v);
+          if (4 * g + r < tile_rows && n < N) out[(size_t)m * N + n] = from_f<TO>(EPI == 4 ? plain_act(v, ACT_RELU_SQUARED) : EPI == 5 ? act_gelu_tanh(v) : v);
         }
       } else {
 #pragma unroll
@@ -320,7 +320,7 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
     if (!is_q && a.slots) slot = a.slots[m];
   }
   floatx4 acc[2][1];
-  if (!skinny_accumulate<1, 2, U, true>(x, W, M, N, K, k_tiles, 2 * blockIdx.x, acc, red, 16, [&](int wave) {
+  if (!skinny_accumulate<1, 2, U, true>(x, W, M, N, K, k_tiles, 2 * blockIdx.x, acc, red, 16, K, [&](int wave) {
         if (shared_sums) leave_row_sums(scale, early, wave, lane);
       })) return;
   if (shared_sums) rs = gathered_row_factor(scale, col);
@@ -378,6 +378,8 @@ static int launch(const void* x, const void* W, void* out, int out_dtype, int M,
     else IFX_FAIL("skinny_gemm: the stream epilogue takes at most 16 rows");
   } else if (epi == 4) {
     GO(bf16_t, 4);
+  } else if (epi == 5) {
+    GO(bf16_t, 5);
   } else if (out_dtype == DT_BF16 && epi == 0) GO(bf16_t, 0);
   else if (out_dtype == DT_BF16 && epi == 3) GO(bf16_t, 3);
   else if (out_dtype == DT_BF16) GO(bf16_t, 1);
@@ -464,8 +466,9 @@ extern "C" int ifx_qkv_rope(const void* x, const void* Wt, int M, int K, const v
 // epi 2: the product is added to ``stream`` [M, N] (float, in place), rows_out [M, N] = bf16(stream * norm_w) and
 //        pieces_out [ceil(N / 16)][16] = sums of squares of the stream in runs of 16, for the norm that follows
 //        (M <= 16, N a multiple of 4, norm_w [N] bfloat16, or float with norm_f32); ``out`` is not used.
-// epi 4: out = max(product, 0)^2, in bfloat16.
-// block_tiles, n_blocks: row tiles in blocks that read inputs of their own (see XBlocks; block_tiles 0: one input).
+// epi 4: out = max(product, 0)^2, epi 5: out = gelu(product) (the tanh form), in bfloat16.
+// block_tiles, n_blocks: row tiles in blocks that read inputs of their own (see XBlocks; block_tiles 0: one input, its rows
+//        n_blocks elements apart, a multiple of 8, 0: K).
 // tiled 1 or 16: W is the tiled form written by ifx_tile_weights, with the row-tile order it was given (or null);
 //        8 to 14 (even): that form with so many rows to a tile (no order).
 // scale_pieces [n_scale_pieces][16] (or null), scale_width, scale_eps: a factor per row of x (M <= 16), see RowScale.
@@ -478,7 +481,7 @@ extern "C" int ifx_skinny_gemm(const void* x, const void* W, void* out, int out_
   const int tile_rows = tiled >= 8 ? tiled : 16;
   IFX_REQUIRE((tiled && tile_rows == 16) || !order, "skinny_gemm: a tile order goes with a tiled copy of 16-row tiles");
   IFX_REQUIRE(epi == 0 || !order, "skinny_gemm: only the plain epilogue takes a tile order");
-  IFX_REQUIRE(epi == 0 || ((epi == 1 || epi == 3) && N % 2 == 0) || (epi == 2 && N % 4 == 0) || (epi == 4 && out_dtype == DT_BF16), "skinny_gemm: epilogue %d with N=%d", epi, N);
+  IFX_REQUIRE(epi == 0 || ((epi == 1 || epi == 3) && N % 2 == 0) || (epi == 2 && N % 4 == 0) || ((epi == 4 || epi == 5) && out_dtype == DT_BF16), "skinny_gemm: epilogue %d with N=%d", epi, N);
   IFX_REQUIRE(epi != 2 || (M <= 16 && stream_io && norm_w && rows_out && pieces_out),
               "skinny_gemm: the stream epilogue takes at most 16 rows (M=%d) and needs the stream, the norm's weight and two outputs", M);
   IFX_REQUIRE(!scale_pieces || (M <= 16 && n_scale_pieces > 0 && scale_width > 0.f),
@@ -532,6 +535,7 @@ extern "C" int ifx_skinny_gemm(const void* x, const void* W, void* out, int out_
   const int k_tiles = ifx_tiled_cols(K) / 32;
   const RowScale scale{scale_pieces, n_scale_pieces, scale_width, scale_eps};
   const StreamOut so{stream_io, norm_w, norm_f32, (bf16_t*)rows_out, pieces_out, stream_mult};
+  IFX_REQUIRE(block_tiles != 0 || n_blocks == 0 || (n_blocks >= K && n_blocks % 8 == 0), "skinny_gemm: rows of x %d apart (a multiple of 8 from K=%d on)", n_blocks, K);
   IFX_REQUIRE(block_tiles == 0 || (block_tiles > 0 && n_blocks > 0 && epi == 0 && !order && (block_tiles % 2 == 0 || nt == 1)),
               "skinny_gemm: blocks of %d tiles with inputs of their own go with the plain epilogue (and an even number of tiles, or one a wave)", block_tiles);
   const XBlocks xb{block_tiles, n_blocks};

@@ -464,6 +464,42 @@ def test_gemm_f32_kernels_agree_bit_for_bit(N, K, adtype):
     assert torch.equal(ops.gemm_f32(shifted, w, None, F32), whole)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 64])
+@pytest.mark.parametrize("N,K,wide,first", [(24, 8, 16, 8), (130, 128, 136, 0), (1024, 64, 3200, 3136)])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_skinny_columns_and_gelu(M, N, K, wide, first, tiled):
+    """Columns of wider rows as they lie and as a copy: the same bits; gelu as the epilogue: the float sums' gelu, rounded once
+    (2^-8 of the value; the sums are off by K roundings of 2^-24)."""
+    g = gen(2300 + M)
+    rows = torch.randn(M, wide, generator=g).to(BF16).to(DEV)
+    x = rows[:, first:first + K]
+    w = ops.prepare_linear((torch.randn(N, K, generator=g) / K ** 0.5).to(BF16).to(DEV))
+    if not tiled:
+        w = ops.LinearWeight(w.rows)
+    args = dict(tiled=w.tiled, tile_rows=w.tile_rows)
+    plain = ops.skinny_gemm(x.contiguous(), w.rows, F32, **args)
+    assert M == 1 or ops.columns_on_16_bytes(x)
+    assert torch.equal(ops.skinny_gemm(x, w.rows, F32, **args), plain)
+    assert torch.equal(ops.linear(x, w, F32), ops.linear(x.contiguous(), w, F32))
+    got = ops.skinny_gemm(x, w.rows, plain_act=ops.ACT_GELU_TANH, **args).double()
+    want = torch.nn.functional.gelu(x.double() @ w.rows.double().t(), approximate="tanh")
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
+def test_zero_slot():
+    """One slot of tensors of several types and sizes, on and off 16 bytes to a slot: zeros there, everything else as it was."""
+    shapes = [((5, 3, 7), F32), ((5, 16, 64, 128), F32), ((5, 9), BF16), ((5, 4), torch.int32), ((5, 1), BF16)]
+    for slot in (0, 2, 4):
+        ts = [torch.ones(s, dtype=d, device=DEV) for s, d in shapes]
+        ops.zero_slot(ops.slot_table(ts), slot, 5)
+        for t in ts:
+            want = torch.ones_like(t)
+            want[slot] = 0
+            assert torch.equal(t, want)
+    with pytest.raises(ops.KernelError):
+        ops.zero_slot(ops.slot_table(ts), 5, 5)
+
+
 # ---- mixtures of experts for few rows ---------------------------------------------------------
 @pytest.mark.parametrize("T", [1, 3, 16, 17, 33, 64])
 @pytest.mark.parametrize("E,identity,top,K,ff,groups,keep,group_top", [
