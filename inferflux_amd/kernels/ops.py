@@ -604,10 +604,8 @@ def moe_experts(h: torch.Tensor, gate: torch.Tensor, up: Optional[torch.Tensor],
     return out
 
 
-def grouped_tile_items(n_items: int, n_experts: int) -> int:
-    """Items of one expert to a workgroup of the grouped product: 128 where the experts get that many on average (every
-    weight tile fetched then serves twice the items), else 64 (steps of few rows, whose tiles are mostly empty)."""
-    return 128 if n_items >= 128 * n_experts else 64
+GROUPED_TILE_ITEMS = 128          # items of one expert to a workgroup of the grouped product (TM in csrc/grouped_gemm.hip)
+GROUPED_MAX_VALUES = 2 ** 30 - 8192          # values of the rows that the product's offsets of 32 bits reach
 
 
 def grouped_takes(dtype: torch.dtype, K: int, ff: int) -> bool:
@@ -662,22 +660,27 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
         raise KernelError(f"moe_experts_grouped: identity experts hand back the row itself, so N={N} must equal K={K}")
     n_items = T * top
     n_real, E = E, E + int(n_identity)
-    tile_items = grouped_tile_items(n_items, E)
-    max_tiles = -(-n_items // tile_items) + E          # every expert may end on a tile that is not full
+    parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
+    portion = GROUPED_MAX_VALUES // K
+    if T > portion:
+        for r in range(0, T, portion):
+            parts[:, r:r + portion] = moe_experts_grouped(h[r:r + portion], gate_up, down, ids[r:r + portion], weights[r:r + portion], act,
+                                                          limit, n_identity, weigh_input).parts
+        return SliceSums(parts, torch.bfloat16)
+    max_tiles = -(-n_items // GROUPED_TILE_ITEMS) + E          # every expert may end on a tile that is not full
     lists = torch.empty((n_items + 3 * max_tiles + 1,), dtype=torch.int32, device=h.device)
     sorted_, te, ts, tc, nt = (lists[:n_items], lists[n_items:n_items + max_tiles], lists[n_items + max_tiles:n_items + 2 * max_tiles],
                                lists[n_items + 2 * max_tiles:n_items + 3 * max_tiles], lists[n_items + 3 * max_tiles:])
-    _call(mod, "ifx_moe_sort", (P, I, I, I, P, P, P, P, P, P), ids.data_ptr(), n_items, E, tile_items, sorted_.data_ptr(), te.data_ptr(),
+    _call(mod, "ifx_moe_sort", (P, I, I, P, P, P, P, P, P), ids.data_ptr(), n_items, E, sorted_.data_ptr(), te.data_ptr(),
           ts.data_ptr(), tc.data_ptr(), nt.data_ptr(), _stream())
-    a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)
+    a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)          # (in the order of ``sorted_``)
     _call(mod, "ifx_moe_gate_up_grouped", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, P),
           h.data_ptr(), gu_ptr, a.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(), tc.data_ptr(),
-          nt.data_ptr(), max_tiles, tile_items, K, ff, top, n_real, int(act), float(limit),
+          nt.data_ptr(), max_tiles, T, K, ff, top, n_real, int(act), float(limit),
           weights.data_ptr() if weigh_input else 0, gu_tiled, _stream())
-    parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, I, I, P),
+    _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, P),
           a.data_ptr(), down_ptr, parts.data_ptr(), weights.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(),
-          tc.data_ptr(), nt.data_ptr(), max_tiles, tile_items, T, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0,
+          tc.data_ptr(), nt.data_ptr(), max_tiles, T, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0,
           down_tiled, _stream())
     return SliceSums(parts, torch.bfloat16)
 

@@ -554,6 +554,47 @@ def test_moe_few(T, E, identity, top, K, ff, groups, keep, group_top, form):
     assert (out - want)[clear].abs().max() < 5 * 2.0 ** -8 * max(size, want[clear].abs().max())
 
 
+@pytest.mark.parametrize("E,identity,top,T,K,N,ff", [
+    (1, 0, 1, 1, 8, 3, 16), (2, 0, 2, 64, 72, 40, 48), (3, 0, 1, 129, 64, 130, 16), (2, 0, 1, 256, 200, 7, 80), (5, 3, 3, 301, 200, 200, 176),
+    (130, 2, 2, 500, 128, 128, 64), (6, 0, 2, 1500, 512, 528, 304)])
+@pytest.mark.parametrize("form", ["tiles", "rows", "input", "portions"])
+def test_moe_experts_grouped_tiles(monkeypatch, E, identity, top, T, K, N, ff, form):
+    """Experts with no item, one, a tile full to the last and one more, some with most of them; weight rows and k-values that
+    end within a tile and a step; experts on both sides of a wave; rows in portions where offsets would not reach: against 64
+    bits.  Each activation is rounded to bfloat16 once (by at most 2^-9 of itself) and sums are in float: together within
+    2^-8 of the sum of the terms' magnitudes, output by output."""
+    g = gen(2300 + T + E)
+    h = torch.randn(T, K, generator=g).to(BF16)
+    gate, up = ((torch.randn(E, ff, K, generator=g) / K ** 0.5).to(BF16) for _ in range(2))
+    down = (torch.randn(E, N, ff, generator=g) / ff ** 0.5).to(BF16)
+    p = torch.arange(1, E + identity + 1).double() ** -1.5          # (a few experts take most of the rows)
+    p = torch.where(torch.arange(E + identity) == 1, p * (0.0 if E + identity > top else 1.0), p)
+    ids = torch.multinomial(p.expand(T, -1), top, generator=g)
+    weights = torch.rand(T, top, generator=g)
+    want, size = torch.zeros(T, N, dtype=torch.float64), torch.zeros(T, N, dtype=torch.float64)
+    for e in range(E + identity):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        x, w = h[t].double(), weights[t, j].double()[:, None]
+        if e >= E:
+            want.index_add_(0, t, w * x)
+            size.index_add_(0, t, w * x.abs())
+            continue
+        wi, wo = (w, 1.0) if form == "input" else (1.0, w)
+        a = torch.nn.functional.silu(wi * (x @ gate[e].double().t())) * (wi * (x @ up[e].double().t()))
+        want.index_add_(0, t, wo * (a @ down[e].double().t()))
+        size.index_add_(0, t, wo * (a.abs() @ down[e].double().abs().t()))
+    pairs, d = ops.pair_gate_up(gate.to(DEV), up.to(DEV)), down.to(DEV)
+    if form == "tiles":
+        pairs = ops.ExpertTiles(pairs)
+        d = ops.ExpertTiles(d) if N % 16 == 0 else d
+    if form == "portions":
+        monkeypatch.setattr(ops, "GROUPED_MAX_VALUES", 100 * K)
+    got = ops.moe_experts_grouped(h.to(DEV), pairs, d, ids.int().to(DEV), weights.to(DEV), n_identity=identity, weigh_input=form == "input")
+    assert got.parts.shape == (top, T, N)
+    out = got.sum(F32).cpu().double()
+    assert ((out - want).abs() <= 2.0 ** -8 * size).all()
+
+
 # ---- sampling -------------------------------------------------------------------------------
 def test_argmax_lowest_index_wins_ties():
     l = torch.zeros(3, 1500)
