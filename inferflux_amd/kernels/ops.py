@@ -75,6 +75,7 @@ def module_variants() -> Iterable[Tuple[str, Variant]]:
     yield ("rowwise", ())
     yield ("grouped_gemm", ())
     yield ("moe_few", ())
+    yield ("gemm_tiles", ())
     yield ("ceilings", ())            # measurement only: what the memory gives a kernel that just reads
     for d in MFMA_HEAD_DIMS_PREBUILT:
         for qt in TILE_QTS:
@@ -1366,11 +1367,38 @@ def _small_m_kernel(M: int, N: int, K: int, has_tiled: bool = False) -> Optional
     return None
 
 
+def pairs_tiles_take(M: int, N: int, K: int) -> bool:
+    """Whether the product for many rows with the activation as its epilogue takes gate/up pairs [N, K] in bfloat16.  Measured
+    against the library's product and a launch for the activation (weights of 5,632 x 1,024 to 37,888 x 3,584, 128 to 16,384
+    rows; csrc/gemm_tiles.hip has figures).  The library's own time goes up in steps where its tiles need another round, and
+    so does this one's, at other sizes: single sizes differ by 0.9 to 1.4 x either way, the means do not.  Up to 2,048 k-values the activation's two
+    trips to memory weigh as much as a fifth of the product: 1.08 x as fast in the mean over 385 to 16,384 rows, at up to 1,600 also
+    from 129 rows on (1.05 x); with fewer rows of deeper weights the library's tiles for few rows are better (11,264 x 2,048 at 300 rows: 28 us
+    for 31).  Deep weights (37,888 x 3,584): 1.02 to 1.15 x at 1,600 to 3,500 rows (2,048: 551 us for 481), but 0.8 to 1.1 x at fewer (512: 145
+    for 165 to 188) and 0.87 to 0.95 x at more (8,192: 1,790 for 1,900), where the library comes closer to the matrix cores' rate."""
+    if N % 4 or K % 8:
+        return False
+    if K <= 2048:
+        return M > (128 if K <= 1600 else 384)
+    return 1600 <= M <= 3500
+
+
+def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, tile: int = -1) -> torch.Tensor:
+    """``linear_swiglu`` of many rows in bfloat16 as one launch ([N, K] ``pairs``, N a multiple of 4 and K of 8, both on 16 bytes);
+    ``tile``: one of the kernel's tiles instead of its choice."""
+    _check(pairs, "weight_pairs", (None, None), torch.bfloat16)
+    N, K = pairs.shape
+    _check(x, "x", (None, K), torch.bfloat16)
+    out = torch.empty((x.shape[0], N // 2), dtype=torch.bfloat16, device=x.device)
+    _call(load_module("gemm_tiles"), "ifx_gemm_pairs", (P, P, P, I, I, I, I, F, I, P), x.data_ptr(), pairs.data_ptr(), out.data_ptr(),
+          x.shape[0], N, K, int(act), float(limit), int(tile), _stream())
+    return out
+
+
 def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: float = 0.0) -> torch.Tensor:
-    """act(x Wg^T) * (x Wu^T) (``act``: ACT_SILU, ACT_GELU_TANH, or ACT_CLAMPED_SWISH with its ``limit``, which is applied by
-    a kernel of its own after the product whatever the number of rows) where ``weight_pairs`` [2I, K] (a tensor or a
-    ``LinearWeight``) alternates the rows of Wg and Wu.  For few rows the activation is the product's epilogue; otherwise a second kernel
-    applies it."""
+    """act(x Wg^T) * (x Wu^T) (``act``: ACT_SILU, ACT_GELU_TANH, or ACT_CLAMPED_SWISH with its ``limit``) where ``weight_pairs``
+    [2I, K] (a tensor or a ``LinearWeight``) alternates the rows of Wg and Wu.  For few rows (not with ACT_CLAMPED_SWISH) and
+    for many (``pairs_tiles_take``) the activation is the product's epilogue; otherwise a second kernel applies it."""
     M, K = x.shape
     if isinstance(x, ScaledRows) and not takes_scaled_rows(M, weight_pairs):
         raise KernelError(f"linear_swiglu: scaled rows are not taken for {M} rows and this weight")
@@ -1378,6 +1406,11 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
                               else (weight_pairs, None, 16))
     if isinstance(weight_pairs, LinearWeight) and weight_pairs.order is not None:
         raise KernelError("linear_swiglu: a tile order is not supported for gate/up pairs")
+    if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.shape[1] == rows.shape[1] \
+            and pairs_tiles_take(M, rows.shape[0], K):
+        whole = x.contiguous()
+        if whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
+            return swiglu_tiles(whole, rows, act, limit)
     if act == ACT_CLAMPED_SWISH:
         return swiglu(linear(x, weight_pairs), interleaved=True, act=act, limit=limit)
     if rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16:

@@ -595,6 +595,37 @@ def test_moe_experts_grouped_tiles(monkeypatch, E, identity, top, T, K, N, ff, f
     assert ((out - want).abs() <= 2.0 ** -8 * size).all()
 
 
+# ---- gate/up of many rows with the activation as the product's epilogue ------------------------
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, -1])
+@pytest.mark.parametrize("M,N,K,act", [(1, 4, 8, "silu"), (129, 132, 64, "silu"), (192, 320, 72, "gelu"), (257, 516, 200, "clamped"),
+                                       (1700, 644, 896, "silu")])
+def test_swiglu_tiles(tile, M, N, K, act):
+    """Rows, weight rows and k-values on both sides of the tiles' edges, every tile and the kernel's own choice: against 64 bits.  Sums in
+    float (K 2^-24 of the terms' magnitudes at most, here far less) and one rounding of the result (2^-9 of it); the activation
+    has a slope of at most 1.2, which carries the sums' error over."""
+    g = gen(2400 + M)
+    x = torch.randn(M, K, generator=g).to(BF16)
+    w = (2.0 * torch.randn(N, K, generator=g) / K ** 0.5).to(BF16)
+    z = x.double() @ w.double().t()
+    gate, up = z[:, ::2], z[:, 1::2]
+    limit = 1.5 if act == "clamped" else 0.0
+    if act == "clamped":
+        gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+        want, kind = gate * torch.sigmoid(1.702 * gate) * (up + 1.0), ops.ACT_CLAMPED_SWISH
+    elif act == "gelu":
+        want, kind = torch.nn.functional.gelu(gate, approximate="tanh") * up, ops.ACT_GELU_TANH
+    else:
+        want, kind = torch.nn.functional.silu(gate) * up, ops.ACT_SILU
+    got = ops.swiglu_tiles(x.to(DEV), w.to(DEV), kind, limit, tile).cpu().double()
+    size = (x.double().abs() @ w.double().abs().t()).reshape(M, N // 2, 2).amax(-1)
+    sums = 1.2 * K ** 0.5 * 2.0 ** -24 * size * (gate.abs() + up.abs() + 2.0)
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + sums + 1e-6).all()
+    if tile == -1 and ops.pairs_tiles_take(M, N, K):          # the front door, with rows that are not contiguous
+        wide = torch.zeros(M, K + 8, dtype=BF16)
+        wide[:, :K] = x
+        assert torch.equal(ops.linear_swiglu(wide.to(DEV)[:, :K], w.to(DEV), kind, limit).cpu().double(), got)
+
+
 # ---- sampling -------------------------------------------------------------------------------
 def test_argmax_lowest_index_wins_ties():
     l = torch.zeros(3, 1500)
