@@ -1,10 +1,15 @@
 // Plain attention over the paged cache: any head size up to 640, float or bf16 storage, float
-// math.  One wave per (query row, query head): each lane scores one key of a 64-key tile, the
-// wave takes the tile's maximum and sum, then every lane accumulates its output elements over
-// the tile's keys in ascending order.  Tiles are aligned to absolute key positions (multiples of
+// math.  Four waves per (query row, query head): wave w takes every fourth tile of 64 keys, from tile w on; each lane scores
+// one key of a tile, the wave takes the tile's maximum and sum, then every lane accumulates its output elements over
+// the tile's keys in ascending order.  At the end the four running maxima, sums and outputs are joined, in the waves'
+// order.  Tiles are aligned to absolute key positions (multiples of
 // 64), so the sequence of operations for a (position, head) is the same however the request was
 // cut into steps: results are bit-equal across cuttings.  This is the attention of the 32-bit
 // path and the reference beside the matrix-core kernels.
+//
+// What bounds a step of few rows is the chain of a tile's trips to memory, shuffles and dependent additions, about 4 us, which
+// one wave went through tile by tile (four rows of 14 heads and 150 keys 16.8 us, 2,000 keys 149; now 8.6 and 50;
+// 64 rows of 500 keys 57 and 36).  Steps of many rows are bound by the loads themselves: 500 rows of a prompt 112 us, now 102.
 //
 // Formula (runtime/backends/cuda/kernels/flash_attention.cu:71-72 GQA map, 86 causal limit, 144
 // scale after the dot product, 152-173 online softmax): head h reads kv head h / (nH / nKV);
@@ -64,17 +69,15 @@ struct AttnArgs {
   const float* sinks;
   int chunk;
   float lambda, out_scale, norm_eps;
+  int row0;                 // the launch's first row
 };
 
 template <typename T, int MAPS>
 __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(AttnArgs a) {
-  __shared__ float q_s[WAVES_PER_BLOCK][MAX_D];
+  __shared__ float q_s[MAX_D];
+  __shared__ float joined[MAPS][WAVES_PER_BLOCK][MAX_D + 2];      // each wave's outputs, maximum and sum
   const int wid = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const long long item = (long long)blockIdx.x * WAVES_PER_BLOCK + wid;
-  // All lanes of a wave share `item`, so the whole wave leaves together; no block-wide
-  // barrier follows.
-  if (item >= (long long)a.T * a.nH) return;
-  const int row = (int)(item / a.nH), head = (int)(item % a.nH);
+  const int row = a.row0 + (int)(blockIdx.x / a.nH), head = (int)(blockIdx.x % a.nH);
   const int d = a.d, dv = a.dv, P = a.page_size;
   const int kvh = head / (a.nH / a.nKV);
   const int pos = a.positions[row];
@@ -85,13 +88,11 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
 
   const int kd = MAPS * d;      // elements of a query's and a key's row
   const T* qrow = (const T*)a.q + ((size_t)row * a.nH + head) * kd;
-  for (int e = lane; e < kd; e += WAVE) q_s[wid][e] = to_f(qrow[e]);
-  // q_s[wid] is written and read by this wave only.
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_s_waitcnt(0);
+  for (int e = threadIdx.x; e < kd; e += WAVE * WAVES_PER_BLOCK) q_s[e] = to_f(qrow[e]);
+  __syncthreads();
 
-  // (the sink is a key of score sink_score whose value is zero: it starts the running maximum and sum)
-  const bool sunk = a.has_sink || a.sinks;
+  // (the sink is a key of score sink_score whose value is zero: it starts the first wave's running maximum and sum)
+  const bool sunk = (a.has_sink || a.sinks) && wid == 0;
   const float sink_score = a.sinks ? a.sinks[head] : a.sink_score;
   float m[MAPS], l[MAPS], acc[MAPS][DC];
 #pragma unroll
@@ -109,6 +110,7 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
       t0 = (lo / WAVE) * WAVE - WAVE;
       continue;
     }
+    if (t0 / WAVE % WAVES_PER_BLOCK != wid) continue;
     const int j = t0 + lane;
     const bool valid = (j >= lo || j < keep) && j <= pos;
     int page = 0, off = 0;
@@ -121,7 +123,7 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
 #pragma unroll
       for (int w = 0; w < MAPS; ++w) {
         const T* kr = Kc + (((size_t)page * a.nKV + kvh) * P + off) * kd + w * d;
-        const float* qv = q_s[wid] + w * d;
+        const float* qv = q_s + w * d;
         float dot = 0.f;
         if (d % 8 == 0) {        // the key's row in 16-byte pieces; the same additions in the same order
           for (int e = 0; e < d; e += 8) {
@@ -195,6 +197,39 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
       }
     }
   }
+  // the four waves' parts joined (a wave without a tile has a sum of 0 and no maximum): every element by one lane, in the order
+  // of the waves
+#pragma unroll
+  for (int w = 0; w < MAPS; ++w) {
+#pragma unroll
+    for (int c = 0; c < DC; ++c)
+      if (lane + c * WAVE < dv) joined[w][wid][lane + c * WAVE] = acc[w][c];
+    if (lane == 0) { joined[w][wid][MAX_D] = m[w]; joined[w][wid][MAX_D + 1] = l[w]; }
+  }
+  __syncthreads();
+  if (wid > 0) return;
+#pragma unroll
+  for (int w = 0; w < MAPS; ++w) {
+    float most = m[w], f[WAVES_PER_BLOCK];
+#pragma unroll
+    for (int k = 1; k < WAVES_PER_BLOCK; ++k) most = fmaxf(most, joined[w][k][MAX_D]);
+    l[w] = 0.f;
+#pragma unroll
+    for (int k = 0; k < WAVES_PER_BLOCK; ++k) {
+      const float n = joined[w][k][MAX_D + 1];
+      f[k] = n > 0.f ? expf(joined[w][k][MAX_D] - most) : 0.f;
+      l[w] = fmaf(n, f[k], l[w]);
+    }
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      const int e = lane + c * WAVE;
+      if (e >= dv) break;
+      float v = acc[w][c] * f[0];
+#pragma unroll
+      for (int k = 1; k < WAVES_PER_BLOCK; ++k) v = fmaf(joined[w][k][e], f[k], v);
+      acc[w][c] = v;
+    }
+  }
   T* orow = (T*)a.out + ((size_t)row * a.nH + head) * dv;
   const float inv = (l[0] > 0.f ? 1.f / l[0] : 0.f) * (a.gate ? a.gate[(size_t)row * a.nH + head] : 1.f);
   if (MAPS == 1) {
@@ -235,14 +270,16 @@ extern "C" int ifx_attn_plain(const void* q, const void* k_cache, const void* v_
   IFX_REQUIRE(dv > 0 && dv <= MAX_D, "attn_plain: value head_dim %d outside 1..%d", dv, MAX_D);
   IFX_REQUIRE(page_size > 0 && max_blocks > 0 && window >= 0, "attn_plain: bad page_size/max_blocks/window");
   if (T == 0) return 0;
-  AttnArgs a{q, k_cache, v_cache, out, row_req, positions, block_table, max_blocks, T, nH, nKV, d, dv, page_size, window, scale, keep_first, has_sink, sink_score, gate, sinks, chunk, lambda, out_scale, norm_eps};
-  const long long items = (long long)T * nH;
-  const unsigned blocks = (unsigned)((items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK);
+  AttnArgs a{q, k_cache, v_cache, out, row_req, positions, block_table, max_blocks, T, nH, nKV, d, dv, page_size, window, scale, keep_first, has_sink, sink_score, gate, sinks, chunk, lambda, out_scale, norm_eps, 0};
+  IFX_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "attn_plain: unknown dtype %d", dtype);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == DT_F32 && maps == 1) hipLaunchKernelGGL((attn_plain_kernel<float, 1>), dim3(blocks), dim3(WAVE * WAVES_PER_BLOCK), 0, s, a);
-  else if (dtype == DT_BF16 && maps == 1) hipLaunchKernelGGL((attn_plain_kernel<bf16_t, 1>), dim3(blocks), dim3(WAVE * WAVES_PER_BLOCK), 0, s, a);
-  else if (dtype == DT_F32) hipLaunchKernelGGL((attn_plain_kernel<float, 2>), dim3(blocks), dim3(WAVE * WAVES_PER_BLOCK), 0, s, a);
-  else if (dtype == DT_BF16) hipLaunchKernelGGL((attn_plain_kernel<bf16_t, 2>), dim3(blocks), dim3(WAVE * WAVES_PER_BLOCK), 0, s, a);
-  else IFX_FAIL("attn_plain: unknown dtype %d", dtype);
+  const int rows = max(1, (1 << 23) / nH);          // rows of a launch: a grid holds fewer than 2^32 threads
+  for (; a.row0 < T; a.row0 += min(rows, T - a.row0)) {
+    const dim3 blocks((unsigned)min(rows, T - a.row0) * (unsigned)nH), threads(WAVE * WAVES_PER_BLOCK);
+    if (dtype == DT_F32 && maps == 1) hipLaunchKernelGGL((attn_plain_kernel<float, 1>), blocks, threads, 0, s, a);
+    else if (dtype == DT_BF16 && maps == 1) hipLaunchKernelGGL((attn_plain_kernel<bf16_t, 1>), blocks, threads, 0, s, a);
+    else if (dtype == DT_F32) hipLaunchKernelGGL((attn_plain_kernel<float, 2>), blocks, threads, 0, s, a);
+    else hipLaunchKernelGGL((attn_plain_kernel<bf16_t, 2>), blocks, threads, 0, s, a);
+  }
   IFX_LAUNCH_CHECK();
 }

@@ -398,6 +398,20 @@ def test_attention_plain(dtype, case):
     assert torch.allclose(out, want, **t), float((out - want).abs().max())
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("past", [0, 62, 63, 64, 254, 255, 256, 257, 1100])
+@pytest.mark.parametrize("window", [None, 3, 65, 130])
+def test_attention_plain_tiles_of_four_waves(dtype, past, window):
+    """A wave takes every fourth tile of 64 keys: contexts that end on both sides of a tile and of a round of four, and windows
+    that leave waves without a tile; the same row gives the same bits whatever rows are beside it."""
+    (q, kc, vc, row_req, positions, table), want, _ = paged_case(1750 + past, [3, 1], [past, past // 2], 4, 2, 32, 16, dtype, window, sharp=-2)
+    out = ops.attention_plain(q, kc, vc, row_req, positions, table, window, 1.0 / math.sqrt(32))
+    t = dict(rtol=1e-4, atol=1e-5) if dtype == F32 else dict(rtol=1e-2, atol=1e-2)
+    assert torch.allclose(out.cpu().double(), want, **t), float((out.cpu().double() - want).abs().max())
+    alone = ops.attention_plain(q[2:3].contiguous(), kc, vc, row_req[2:3].contiguous(), positions[2:3].contiguous(), table, window, 1.0 / math.sqrt(32))
+    assert torch.equal(out[2:3], alone)
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_attention_plain_random_cases(seed):
     """The plain attention kernel (the 32-bit path's, and the reference beside the matrix-core ones) at shapes drawn at
