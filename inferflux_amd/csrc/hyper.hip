@@ -204,6 +204,99 @@ __global__ __launch_bounds__(512) void hc_vec_kernel(HcArgs a) {
   }
 }
 
+// The same again where a thread's 4 columns are all it has (rows of up to 2,048): everything a row reads, the norm's weight
+// among it, is asked for before anything is used, the mixing weights come through the scalar cache instead of LDS and a
+// barrier, and the reading stays in registers.  What bounds a launch of few rows is its chain of trips to memory (one now, three
+// before) and the 64 KB a row reads and writes through one CU: 16 rows of 4 streams of 2,048 took 7.0 us, now
+// 6.3.  The
+// same additions in the same order as above.
+template <int S_MAX, typename TW>
+__global__ __launch_bounds__(512) void hc_row_kernel(HcArgs a) {
+  typedef __attribute__((__vector_size__(4 * sizeof(TW)))) TW weight4;
+  __shared__ float red[16];
+  const int S = a.S, H = a.H, c = threadIdx.x * 4;
+  const size_t t = blockIdx.x;
+  const bool in = c < H, y_bf16 = a.n_slices == 1 && a.y_dtype == DT_BF16;
+  const float* src = a.src + (a.broadcast ? t * H : t * S * H);
+  float4 x[S_MAX], y = make_float4(0.f, 0.f, 0.f, 0.f);
+  hc_bf16x4 y_halves = {};
+  weight4 nw = {};
+#pragma unroll
+  for (int s = 0; s < S_MAX; ++s) x[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (in) {
+#pragma unroll
+    for (int s = 0; s < S_MAX; ++s)
+      if (s < S) x[s] = *(const float4*)(src + (a.broadcast ? 0 : (size_t)s * H) + c);
+    if (a.norm_w) nw = *(const weight4*)((const TW*)a.norm_w + c);
+    if (a.y && y_bf16) y_halves = *(const hc_bf16x4*)((const bf16_t*)a.y + t * H + c);
+    else if (a.y) y = *(const float4*)((const float*)a.y + t * H + c);
+  }
+  if (a.y) {
+    if (y_bf16) y = make_float4((float)y_halves[0], (float)y_halves[1], (float)y_halves[2], (float)y_halves[3]);
+    if (in)
+      for (int k = 1; k < a.n_slices; ++k) {
+        const float4 v = *(const float4*)((const float*)a.y + t * H + c + (size_t)k * a.slice_stride);
+        y.x += v.x; y.y += v.y; y.z += v.z; y.w += v.w;
+      }
+    y.x *= a.y_scale; y.y *= a.y_scale; y.z *= a.y_scale; y.w *= a.y_scale;
+    float4 n[S_MAX];
+#pragma unroll
+    for (int to = 0; to < S_MAX; ++to) {
+      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int s = 0; s < S_MAX; ++s)
+        if (s < S && to < S) {
+          const float m = a.mix[s * S + to];
+          v.x = fmaf(m, x[s].x, v.x); v.y = fmaf(m, x[s].y, v.y); v.z = fmaf(m, x[s].z, v.z); v.w = fmaf(m, x[s].w, v.w);
+        }
+      const float o = a.outw[to < S ? to : 0];
+      n[to] = make_float4(fmaf(o, y.x, v.x), fmaf(o, y.y, v.y), fmaf(o, y.z, v.z), fmaf(o, y.w, v.w));
+    }
+#pragma unroll
+    for (int s = 0; s < S_MAX; ++s) x[s] = n[s];
+  }
+  float4 u = make_float4(0.f, 0.f, 0.f, 0.f);
+  float ss = 0.f;
+  if (a.inw) {
+#pragma unroll
+    for (int s = 0; s < S_MAX; ++s)
+      if (s < S) {
+        const float w = a.inw[s];
+        u.x = fmaf(w, x[s].x, u.x); u.y = fmaf(w, x[s].y, u.y); u.z = fmaf(w, x[s].z, u.z); u.w = fmaf(w, x[s].w, u.w);
+      }
+    ss = fmaf(u.x, u.x, ss); ss = fmaf(u.y, u.y, ss); ss = fmaf(u.z, u.z, ss); ss = fmaf(u.w, u.w, ss);
+  }
+  if (a.dst && (a.y || a.broadcast) && in) {
+#pragma unroll
+    for (int s = 0; s < S_MAX; ++s)
+      if (s < S) *(float4*)(a.dst + (t * S + s) * H + c) = x[s];
+  }
+  if (!a.inw) return;
+  if (!a.norm_w) {
+    if (in) *(float4*)((float*)a.out + t * H + c) = u;
+    return;
+  }
+  const float inv = rsqrtf(block_sum(ss, red) / (float)H + a.eps);
+  if (!in) return;
+  const float v[4] = {u.x * inv * (float)nw[0], u.y * inv * (float)nw[1], u.z * inv * (float)nw[2], u.w * inv * (float)nw[3]};
+  if (a.out_dtype == DT_F32) {
+    *(float4*)((float*)a.out + t * H + c) = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+    hc_bf16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (__bf16)v[e];
+    *(hc_bf16x4*)((bf16_t*)a.out + t * H + c) = o;
+  }
+}
+
+template <typename TW>
+static void launch_rows(const HcArgs& a, int T, int threads, hipStream_t s) {
+  if (a.S <= 1) hipLaunchKernelGGL((hc_row_kernel<1, TW>), dim3(T), dim3(threads), 0, s, a);
+  else if (a.S <= 2) hipLaunchKernelGGL((hc_row_kernel<2, TW>), dim3(T), dim3(threads), 0, s, a);
+  else if (a.S <= 4) hipLaunchKernelGGL((hc_row_kernel<4, TW>), dim3(T), dim3(threads), 0, s, a);
+  else hipLaunchKernelGGL((hc_row_kernel<8, TW>), dim3(T), dim3(threads), 0, s, a);
+}
+
 extern "C" int ifx_hyper_step(const float* src, int broadcast, float* dst, const void* y, int y_dtype, int n_slices,
                               long long slice_stride, float y_scale, const float* mix, const float* outw, const float* inw,
                               const void* norm_w, int norm_dtype, float eps, void* out, int out_dtype, int T, int S, int H,
@@ -225,6 +318,11 @@ extern "C" int ifx_hyper_step(const float* src, int broadcast, float* dst, const
   if (vec) {
     // (a thread per 4 columns up to 512 threads: a step of few rows has one trip to memory instead of several in a row)
     const int threads = min(512, ((H / 4 + WAVE - 1) / WAVE) * WAVE);
+    if (H <= 2048 && ((size_t)norm_w & (norm_dtype == DT_BF16 ? 7 : 15)) == 0) {
+      if (norm_w && norm_dtype == DT_BF16) launch_rows<__bf16>(a, T, threads, s);
+      else launch_rows<float>(a, T, threads, s);
+      IFX_LAUNCH_CHECK();
+    }
     if (S <= 1) hipLaunchKernelGGL(hc_vec_kernel<1>, dim3(T), dim3(threads), lds, s, a);
     else if (S <= 2) hipLaunchKernelGGL(hc_vec_kernel<2>, dim3(T), dim3(threads), lds, s, a);
     else if (S <= 4) hipLaunchKernelGGL(hc_vec_kernel<4>, dim3(T), dim3(threads), lds, s, a);

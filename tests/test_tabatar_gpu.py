@@ -379,6 +379,14 @@ def test_hyper_connections_read_and_update_all_streams_at_once(dtype, S, T, H):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("S", [1, 3, 4, 8])
+@pytest.mark.parametrize("T,H", [(2, 4), (16, 2044), (3, 2048), (3, 2052)])
+def test_hyper_connections_at_the_widths_a_thread_holds(dtype, S, T, H):
+    """Rows whose four columns to a thread are all there are, and the next width."""
+    test_hyper_connections_read_and_update_all_streams_at_once(dtype, S, T, H)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("M", [1, 7, 16, 40, 300])
 @pytest.mark.parametrize("K,ff", [(64, 96), (256, 384), (100, 50)])
 def test_feed_forward_without_a_gate(dtype, M, K, ff):
