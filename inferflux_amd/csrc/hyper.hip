@@ -206,10 +206,9 @@ __global__ __launch_bounds__(512) void hc_vec_kernel(HcArgs a) {
 
 // The same again where a thread's 4 columns are all it has (rows of up to 2,048): everything a row reads, the norm's weight
 // among it, is asked for before anything is used, the mixing weights come through the scalar cache instead of LDS and a
-// barrier, and the reading stays in registers.  What bounds a launch of few rows is its chain of trips to memory (one now, three
-// before) and the 64 KB a row reads and writes through one CU: 16 rows of 4 streams of 2,048 took 7.0 us, now
-// 6.3.  The
-// same additions in the same order as above.
+// barrier, and the reading stays in registers.  What bounds a launch of few rows is its chain of trips to memory (one now,
+// three before) and the 64 KB a row reads and writes through one CU: 16 rows of 4 streams of 2,048 took 7.0 us, now 6.3.
+// The same additions in the same order as above.
 template <int S_MAX, typename TW>
 __global__ __launch_bounds__(512) void hc_row_kernel(HcArgs a) {
   typedef __attribute__((__vector_size__(4 * sizeof(TW)))) TW weight4;
