@@ -1375,8 +1375,10 @@ def pairs_tiles_take(M: int, N: int, K: int) -> bool:
     trips to memory weigh as much as a fifth of the product: 1.08 x as fast in the mean over 385 to 16,384 rows, at up to 1,600 also
     from 129 rows on (1.05 x); with fewer rows of deeper weights the library's tiles for few rows are better (11,264 x 2,048 at 300 rows: 28 us
     for 31).  Deep weights (37,888 x 3,584): 1.02 to 1.15 x at 1,600 to 3,500 rows (2,048: 551 us for 481), but 0.8 to 1.1 x at fewer (512: 145
-    for 165 to 188) and 0.87 to 0.95 x at more (8,192: 1,790 for 1,900), where the library comes closer to the matrix cores' rate."""
-    if N % 4 or K % 8:
+    for 165 to 188) and 0.87 to 0.95 x at more (8,192: 1,790 for 1,900), where the library comes closer to the matrix cores' rate.  Where the caller
+    has the library time its kernels (``enable_library_gemm_tuning``), its choice is the faster one (2,048 tokens through the 7B shape 25.8 ms
+    for 27.9; with its default choice 28.7 for 26.9)."""
+    if N % 4 or K % 8 or torch.cuda.tunable.is_enabled():
         return False
     if K <= 2048:
         return M > (128 if K <= 1600 else 384)

@@ -640,6 +640,21 @@ def test_swiglu_tiles(tile, M, N, K, act):
         assert torch.equal(ops.linear_swiglu(wide.to(DEV)[:, :K], w.to(DEV), kind, limit).cpu().double(), got)
 
 
+def test_many_row_pairs_go_to_the_library_where_it_times_its_kernels(monkeypatch):
+    """The route of gate/up of many rows by sizes, and with the library's tuning on; on either the same function."""
+    assert ops.pairs_tiles_take(1600, 37888, 3584) and ops.pairs_tiles_take(3500, 37888, 3584)
+    assert not ops.pairs_tiles_take(1599, 37888, 3584) and not ops.pairs_tiles_take(3501, 37888, 3584)
+    assert ops.pairs_tiles_take(385, 512, 2048) and not ops.pairs_tiles_take(384, 512, 2048)
+    assert ops.pairs_tiles_take(129, 512, 1600) and not ops.pairs_tiles_take(128, 512, 1600)
+    assert not ops.pairs_tiles_take(2000, 510, 512) and not ops.pairs_tiles_take(2000, 512, 516)
+    x, w = torch.randn(200, 64, generator=gen(2450)).to(BF16).to(DEV), torch.randn(512, 64, generator=gen(2451)).to(BF16).to(DEV)
+    ours = ops.linear_swiglu(x, w).double()
+    monkeypatch.setattr(torch.cuda.tunable, "is_enabled", lambda: True)
+    assert not ops.pairs_tiles_take(200, 512, 64)
+    theirs = ops.linear_swiglu(x, w).double()          # (gate and up rounded to bfloat16 in between: 2^-9 of each, twice, and of the result)
+    assert ((ours - theirs).abs() <= 2.0 ** -6 * ours.abs() + 2.0 ** -6).all()
+
+
 # ---- sampling -------------------------------------------------------------------------------
 def test_argmax_lowest_index_wins_ties():
     l = torch.zeros(3, 1500)
