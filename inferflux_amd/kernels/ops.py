@@ -1367,6 +1367,9 @@ def _small_m_kernel(M: int, N: int, K: int, has_tiled: bool = False) -> Optional
     return None
 
 
+PAIRS_MAX_K = 1 << 20          # k-values that the product's offsets of 32 bits reach (csrc/gemm_tiles.hip)
+
+
 def pairs_tiles_take(M: int, N: int, K: int) -> bool:
     """Whether the product for many rows with the activation as its epilogue takes gate/up pairs [N, K] in bfloat16.  Measured
     against the library's product and a launch for the activation (weights of 5,632 x 1,024 to 37,888 x 3,584, 128 to 16,384
@@ -1378,7 +1381,7 @@ def pairs_tiles_take(M: int, N: int, K: int) -> bool:
     for 165 to 188) and 0.87 to 0.95 x at more (8,192: 1,790 for 1,900), where the library comes closer to the matrix cores' rate.  Where the caller
     has the library time its kernels (``enable_library_gemm_tuning``), its choice is the faster one (2,048 tokens through the 7B shape 25.8 ms
     for 27.9; with its default choice 28.7 for 26.9)."""
-    if N % 4 or K % 8 or torch.cuda.tunable.is_enabled():
+    if N % 4 or K % 8 or K > PAIRS_MAX_K or torch.cuda.tunable.is_enabled():
         return False
     if K <= 2048:
         return M > (128 if K <= 1600 else 384)

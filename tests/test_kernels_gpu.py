@@ -647,6 +647,7 @@ def test_many_row_pairs_go_to_the_library_where_it_times_its_kernels(monkeypatch
     assert ops.pairs_tiles_take(385, 512, 2048) and not ops.pairs_tiles_take(384, 512, 2048)
     assert ops.pairs_tiles_take(129, 512, 1600) and not ops.pairs_tiles_take(128, 512, 1600)
     assert not ops.pairs_tiles_take(2000, 510, 512) and not ops.pairs_tiles_take(2000, 512, 516)
+    assert ops.pairs_tiles_take(2000, 4, 1 << 20) and not ops.pairs_tiles_take(2000, 4, (1 << 20) + 8)
     x, w = torch.randn(200, 64, generator=gen(2450)).to(BF16).to(DEV), torch.randn(512, 64, generator=gen(2451)).to(BF16).to(DEV)
     ours = ops.linear_swiglu(x, w).double()
     monkeypatch.setattr(torch.cuda.tunable, "is_enabled", lambda: True)
