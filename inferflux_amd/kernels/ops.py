@@ -1231,7 +1231,8 @@ def staged_gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
 def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, keep_slices: bool = False):
     """x [M, K] times ``weight`` [N, K] transposed (a tensor or a ``LinearWeight``), chosen by the weight's
     type and by M.  With ``keep_slices`` the result may be ``SliceSums`` (the caller hands it to ``add_rmsnorm`` or
-    ``rope_append``, or calls its ``sum()``).
+    ``rope_append``, or calls its ``sum()``).  ``x`` is contiguous, or in bfloat16 columns of wider rows on 16 bytes
+    (``columns_on_16_bytes``).
 
     A float32 weight takes the true 32-bit kernel whatever the activation's type.  A bfloat16
     weight with bfloat16 activations takes the weight-streaming kernel for up to 64 rows and the
@@ -1245,18 +1246,21 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
         raise KernelError(f"linear: scaled rows are not taken for {x.shape[0]} rows and this weight")
     if isinstance(weight, LinearWeight):
         weight, tiled, order, tile_rows = weight.rows, weight.tiled, weight.order, weight.tile_rows
+    columns = columns_on_16_bytes(x)      # (the product for few rows reads them where they lie, every other one takes a copy)
     if weight.dtype == torch.float32:
-        return gemm_f32(x, weight, None, out_dtype or x.dtype)
+        return gemm_f32(x.contiguous() if columns else x, weight, None, out_dtype or x.dtype)
     if weight.dtype != torch.bfloat16 or x.dtype != torch.bfloat16:
         raise KernelError(f"linear: weight {weight.dtype} with activation {x.dtype} is not supported")
+    if not columns:
+        _check(x if not isinstance(x, ScaledRows) else x.rows, "x", (None, weight.shape[1]))
     _check(weight, "weight", (None, None))
     out_dtype = out_dtype or torch.bfloat16
     M, K = x.shape
+    if K != weight.shape[1]:
+        raise KernelError(f"x: shape {tuple(x.shape)}, expected {(None, weight.shape[1])}")
     kind = _small_m_kernel(M, weight.shape[0], K, tiled is not None)
-    if not isinstance(x, ScaledRows) and not x.is_contiguous() and x.shape[1] == weight.shape[1] and not (kind == "skinny" and columns_on_16_bytes(x)):
-        x = x.contiguous()            # (columns of wider rows: the product for few rows reads them where they lie)
-    if not columns_on_16_bytes(x):
-        _check(x if not isinstance(x, ScaledRows) else x.rows, "x", (None, weight.shape[1]))
+    if columns and kind != "skinny":
+        x = x.contiguous()
     if kind == "skinny":
         return skinny_gemm(x, weight, out_dtype, tiled=tiled, order=order, tile_rows=tile_rows)
     if kind == "wide":

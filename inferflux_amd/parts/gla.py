@@ -84,8 +84,8 @@ class GatedLinearAttention(Mixer):
         HD, HV, r = self.n_heads * self.head_dim, self.n_heads * self.v_head_dim, self.decay_rank
         rows = ops.linear(h, self.w_in)                                 # [T, q | k | v | g | a1]
         a1 = rows[:, 2 * HD + 2 * HV:] if rows.shape[0] else rows.new_empty((0, r))
-        if a1.dtype != torch.bfloat16:
-            a1 = a1.contiguous()              # (in bfloat16 the product for few rows reads the columns where they lie)
+        if not ops.columns_on_16_bytes(a1):
+            a1 = a1.contiguous()              # (``linear`` takes columns in bfloat16 on 16 bytes)
         z = ops.linear(a1, self.w_a2, out_dtype=torch.float32)         # the decays' logits are never rounded
         if t is not None:
             t.mark("mixer.project")

@@ -500,6 +500,20 @@ def test_skinny_columns_and_gelu(M, N, K, wide, first, tiled):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
 
 
+@pytest.mark.parametrize("M", [2, 7, 40, 300])
+@pytest.mark.parametrize("wdtype", [F32, BF16])
+def test_linear_takes_columns_of_wider_rows_and_no_other_strides(M, wdtype):
+    """Columns on 16 bytes give what their copy gives, whatever the weight's type; rows that are not columns on 16 bytes are refused."""
+    g = gen(2350 + M)
+    rows = torch.randn(M, 136, generator=g).to(BF16).to(DEV)
+    w = (torch.randn(48, 64, generator=g) / 8).to(wdtype).to(DEV)
+    for weight in (w, ops.prepare_linear(w)):
+        assert torch.equal(ops.linear(rows[:, 72:], weight, F32), ops.linear(rows[:, 72:].contiguous(), weight, F32))
+        for x in (rows[:, 3:67], torch.randn(64, M, generator=g).to(BF16).to(DEV).t(), rows[:, ::2][:, :64], rows[0, :64]):
+            with pytest.raises(ops.KernelError):
+                ops.linear(x, weight, F32)
+
+
 def test_zero_slot():
     """One slot of tensors of several types and sizes, on and off 16 bytes to a slot: zeros there, everything else as it was."""
     shapes = [((5, 3, 7), F32), ((5, 16, 64, 128), F32), ((5, 9), BF16), ((5, 4), torch.int32), ((5, 1), BF16)]

@@ -465,6 +465,25 @@ def test_whole_prompts(name, dtype, folders):
     runner.manager.check()
 
 
+@pytest.mark.parametrize("stored", [".mix.a2", ".mix."])
+@pytest.mark.parametrize("name", ["A", "C", "E"])
+def test_decays_whose_outer_matrix_is_stored_in_32_bits(name, stored, folders, tmp_path):
+    """A tensor that the file holds in 32 bits stays so in bfloat16 mode: the decays' outer matrix alone, and every matrix of the
+    mixers, beside bfloat16 rows of the inner product that are cut out of wider ones (on 16 bytes in C and E)."""
+    from safetensors.torch import load_file, save_file
+    folder, vocab = folders[name, "bfloat16"], tm.CONFIGS[name]["vocab"]
+    tensors = {n: t.float() if (n.endswith(stored) if stored == ".mix.a2" else stored in n) else t.bfloat16()
+               for n, t in load_file(os.path.join(folder, "model.safetensors")).items()}
+    assert any(t.dtype == torch.float32 for n, t in tensors.items() if n.endswith(".mix.a2"))
+    save_file(tensors, str(tmp_path / "model.safetensors"))
+    (tmp_path / "config.json").write_text(open(os.path.join(folder, "config.json")).read())
+    runner = load_runner(str(tmp_path), torch.bfloat16, num_pages=32, max_requests=2)
+    for seed, n in ((1, 1), (2, 7), (3, 300)):
+        ids = ids_of(seed, n, vocab)
+        assert off(run_whole(runner, "w", ids), plain(folder, ids), "bfloat16") < 1, n
+    runner.manager.check()
+
+
 @pytest.mark.parametrize("name", ["A", "B", "C", "D"])
 def test_stream_after_every_layer(name, folders):
     folder = folders[name, "float32"]
