@@ -92,7 +92,7 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
   __syncthreads();
 
   // (the sink is a key of score sink_score whose value is zero: it starts the first wave's running maximum and sum)
-  const bool sunk = (a.has_sink || a.sinks) && wid == 0;
+  const bool has_sink = a.has_sink || a.sinks, sunk = has_sink && wid == 0;
   const float sink_score = a.sinks ? a.sinks[head] : a.sink_score;
   float m[MAPS], l[MAPS], acc[MAPS][DC];
 #pragma unroll
@@ -105,7 +105,8 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
 
   const T* Kc = (const T*)a.k_cache;
   const T* Vc = (const T*)a.v_cache;
-  for (int t0 = keep > 0 ? 0 : (lo / WAVE) * WAVE; t0 <= pos; t0 += WAVE) {
+  const int t_first = keep > 0 ? 0 : (lo / WAVE) * WAVE;
+  for (int t0 = t_first; t0 <= pos; t0 += WAVE) {
     if (t0 >= keep && t0 + WAVE <= lo) {     // between the kept first keys and the window: on to the window's first tile
       t0 = (lo / WAVE) * WAVE - WAVE;
       continue;
@@ -140,9 +141,12 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
     }
 #pragma unroll
     for (int w = 0; w < MAPS; ++w) {
-      const float m_new = fmaxf(m[w], wave_max(s[w]));  // finite: the tile holds a visible key
-      p[w] = valid ? expf(s[w] - m_new) : 0.f;
-      const float alpha = expf(m[w] - m_new);  // 0 on the first tile (m = -inf)
+      const float m_new = fmaxf(m[w], wave_max(s[w]));  // finite unless every score overflows: the tile holds a visible key
+      // (a tile of scores of minus infinity counts for nothing beside a sink or behind the row's first tile, whichever wave
+      // meets it first)
+      const float from = m_new == -INFINITY && (t0 != t_first || (has_sink && sink_score > -INFINITY)) ? 0.f : m_new;
+      p[w] = valid ? expf(s[w] - from) : 0.f;
+      const float alpha = expf(m[w] - from);  // 0 on the first tile (m = -inf)
       l[w] = l[w] * alpha + wave_sum(p[w]);
 #pragma unroll
       for (int c = 0; c < DC; ++c) acc[w][c] *= alpha;

@@ -412,6 +412,35 @@ def test_attention_plain_tiles_of_four_waves(dtype, past, window):
     assert torch.equal(out[2:3], alone)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("low,window,sink", [((64, 128), None, None), ((128, 256), None, None), ((0, 64), None, 0.5), ((0, 300), None, -1.0),
+                                             ((192, 256), 130, None), ((64, 320), None, None), ((128, 192), 150, 0.0)])
+def test_attention_plain_tiles_whose_scores_are_all_minus_infinity(dtype, low, window, sink):
+    """Keys whose scores overflow to minus infinity, tiles of 64 of them: they weigh nothing, as if a mask had shut them out, whichever
+    wave meets such a tile first."""
+    d, past, P = 16, 290, 16
+    n, pages = past + 1, -(-(past + 1) // P)
+    g = gen(1790)
+    q = torch.full((1, 2, d), 2.0 ** 80)
+    k, v = torch.randn(n, 1, d, generator=g) * 2.0 ** -80, torch.randn(n, 1, d, generator=g).to(dtype).float()
+    k[low[0]:low[1]] = -2.0 ** 80
+    k = k.to(dtype).float()
+    seen = [j for j in range(n) if not low[0] <= j < low[1] and (window is None or j > past - window)]
+    s = (q.double()[0] @ k.double()[seen, 0].t()) * 0.25
+    e = torch.cat([s, torch.full((2, 1), sink, dtype=torch.float64)], 1) if sink is not None else s
+    want = (e.softmax(1)[:, :len(seen)] @ v.double()[seen, 0]) if seen else torch.zeros(2, d, dtype=torch.float64)
+    pad = torch.zeros(pages * P, 1, d)
+    pad[:n] = k
+    kc = pad.view(pages, P, 1, d).transpose(1, 2).contiguous().to(dtype).to(DEV)
+    pad[:n] = v
+    vc = pad.view(pages, P, 1, d).permute(0, 2, 3, 1).contiguous().to(dtype).to(DEV)
+    i32 = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    got = ops.attention_plain(q.to(dtype).to(DEV), kc, vc, i32(0), i32(past), torch.arange(pages, dtype=torch.int32, device=DEV)[None],
+                              window, 0.25, sink=sink).cpu().double().view(2, d)
+    t = dict(rtol=1e-4, atol=1e-5) if dtype == F32 else dict(rtol=1e-2, atol=1e-2)
+    assert torch.allclose(got, want, **t), float((got - want).abs().max())
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_attention_plain_random_cases(seed):
     """The plain attention kernel (the 32-bit path's, and the reference beside the matrix-core ones) at shapes drawn at
