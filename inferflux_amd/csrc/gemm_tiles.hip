@@ -90,6 +90,7 @@ static int choose_tile(int M, int N, int K) {
 // x, w: on 16 bytes.  tile: one of the kinds above, or -1 for the one that choose_tile takes
 extern "C" int ifx_gemm_pairs(const void* x, const void* w, void* out, int M, int N, int K, int act, float limit, int tile, void* stream) {
   IFX_REQUIRE(M >= 0 && N > 0 && N % 4 == 0 && K > 0 && K % 8 == 0 && K <= 1 << 20, "gemm_pairs: N=%d must be a multiple of 4, K=%d of 8", N, K);
+  IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f), "gated activation: unknown kind %d (limit %g)", act, (double)limit);
   IFX_REQUIRE(((size_t)x | (size_t)w) % 16 == 0, "gemm_pairs: x and the weight must lie on 16 bytes");
   if (M == 0) return 0;
   const PairsArgs a{(const bf16_t*)x, (const bf16_t*)w, (bf16_t*)out, M, N, K, act, limit};

@@ -683,6 +683,17 @@ def test_swiglu_tiles(tile, M, N, K, act):
         assert torch.equal(ops.linear_swiglu(wide.to(DEV)[:, :K], w.to(DEV), kind, limit).cpu().double(), got)
 
 
+@pytest.mark.parametrize("act,limit", [("ACT_RELU_SQUARED", 0.0), (None, 0.0), ("ACT_CLAMPED_SWISH", 0.0), ("ACT_CLAMPED_SWISH", -1.0)])
+def test_gated_activations_that_do_not_exist_are_refused_on_every_route(monkeypatch, act, limit):
+    """An activation without a gate, an unknown one, a clamp without a limit: by the product with its epilogue as by the library's
+    product and the activation's own launch."""
+    x, w = torch.randn(500, 64, generator=gen(2460)).to(BF16).to(DEV), torch.randn(1024, 64, generator=gen(2461)).to(BF16).to(DEV)
+    for takes in (True, False):
+        monkeypatch.setattr(ops, "pairs_tiles_take", lambda *a: takes)
+        with pytest.raises(ops.KernelError):
+            ops.linear_swiglu(x, w, getattr(ops, act) if act else 7, limit)
+
+
 def test_many_row_pairs_go_to_the_library_where_it_times_its_kernels(monkeypatch):
     """The route of gate/up of many rows by sizes, and with the library's tuning on; on either the same function."""
     assert ops.pairs_tiles_take(1600, 37888, 3584) and ops.pairs_tiles_take(3500, 37888, 3584)
