@@ -1406,7 +1406,7 @@ def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limi
 
 def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: float = 0.0) -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) (``act``: ACT_SILU, ACT_GELU_TANH, or ACT_CLAMPED_SWISH with its ``limit``) where ``weight_pairs``
-    [2I, K] (a tensor or a ``LinearWeight``) alternates the rows of Wg and Wu.  For few rows (not with ACT_CLAMPED_SWISH) and
+    [2I, K] (a tensor or a ``LinearWeight``) alternates the rows of Wg and Wu; ``x`` as for ``linear``.  For few rows (not with ACT_CLAMPED_SWISH) and
     for many (``pairs_tiles_take``) the activation is the product's epilogue; otherwise a second kernel applies it."""
     M, K = x.shape
     if isinstance(x, ScaledRows) and not takes_scaled_rows(M, weight_pairs):
@@ -1415,7 +1415,10 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
                               else (weight_pairs, None, 16))
     if isinstance(weight_pairs, LinearWeight) and weight_pairs.order is not None:
         raise KernelError("linear_swiglu: a tile order is not supported for gate/up pairs")
-    if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.shape[1] == rows.shape[1] \
+    columns = columns_on_16_bytes(x)          # (as for ``linear``)
+    if not columns and not isinstance(x, ScaledRows):
+        _check(x, "x", (None, rows.shape[1]))
+    if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and K == rows.shape[1] \
             and pairs_tiles_take(M, rows.shape[0], K):
         whole = x.contiguous()
         if whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
@@ -1426,6 +1429,8 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
         kind = _small_m_kernel(M, rows.shape[0], K, tiled is not None)
         if kind == "skinny":
             return skinny_gemm(x, rows, torch.bfloat16, swiglu_pairs=True, tiled=tiled, tile_rows=tile_rows, act=act)
+        if columns:
+            x = x.contiguous()
         if kind == "wide":
             return wide_gemm(x, weight_pairs, torch.bfloat16, swiglu_pairs=True, act=act)
         if kind == "staged":
@@ -2099,7 +2104,8 @@ def hyper_step(src: torch.Tensor, n_streams: int, y=None, mix: Optional[torch.Te
 
 def linear_act(x, weight, act: int) -> torch.Tensor:
     """act(x W^T) for a feed-forward without a gate (``act``: ACT_SILU, ACT_GELU_TANH or ACT_RELU_SQUARED, formed in float on the product's
-    output; in steps of few rows the square of relu and gelu are the product's epilogue: 16 rows of 8,448 x 2,048 12 us and a launch of 5 less)."""
+    output; in steps of few rows the square of relu and gelu are the product's epilogue: 16 rows of 8,448 x 2,048 12 us and a launch of 5 less);
+    ``x`` as for ``linear``."""
     if act in _PLAIN_EPILOGUE and isinstance(weight, LinearWeight) and weight.rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 \
             and weight.order is None and _small_m_kernel(x.shape[0], *weight.rows.shape, weight.tiled is not None) == "skinny" \
             and (not isinstance(x, ScaledRows) or takes_scaled_rows(x.shape[0], weight)):

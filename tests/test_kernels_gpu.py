@@ -541,6 +541,13 @@ def test_linear_takes_columns_of_wider_rows_and_no_other_strides(M, wdtype):
         for x in (rows[:, 3:67], torch.randn(64, M, generator=g).to(BF16).to(DEV).t(), rows[:, ::2][:, :64], rows[0, :64]):
             with pytest.raises(ops.KernelError):
                 ops.linear(x, weight, F32)
+    if wdtype == BF16:
+        for f in (lambda x, w: ops.linear_swiglu(x, w), lambda x, w: ops.linear_act(x, w, ops.ACT_GELU_TANH)):
+            for weight in (w, ops.prepare_linear(w)):
+                assert torch.equal(f(rows[:, 72:], weight), f(rows[:, 72:].contiguous(), weight))
+                for x in (rows[:, 3:67], torch.randn(64, M, generator=g).to(BF16).to(DEV).t(), rows[:, ::2][:, :64]):
+                    with pytest.raises(ops.KernelError):
+                        f(x, weight)
 
 
 def test_zero_slot():
