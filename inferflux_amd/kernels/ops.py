@@ -8,6 +8,7 @@ missing library or a refused size raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Dict, Iterable, Optional, Tuple
 
 import torch
@@ -1371,25 +1372,17 @@ def _small_m_kernel(M: int, N: int, K: int, has_tiled: bool = False) -> Optional
     return None
 
 
-PAIRS_MAX_K = 1 << 20          # k-values that the product's offsets of 32 bits reach (csrc/gemm_tiles.hip)
+@functools.lru_cache(maxsize=4096)
+def _pairs_tiles_win(M: int, N: int, K: int) -> bool:
+    return load_module("gemm_tiles").fn("ifx_gemm_pairs_wins", (I, I, I))(M, N, K) != 0
 
 
 def pairs_tiles_take(M: int, N: int, K: int) -> bool:
-    """Whether the product for many rows with the activation as its epilogue takes gate/up pairs [N, K] in bfloat16.  Measured
-    against the library's product and a launch for the activation (weights of 5,632 x 1,024 to 37,888 x 3,584, 128 to 16,384
-    rows; csrc/gemm_tiles.hip has figures).  The library's own time goes up in steps where its tiles need another round, and
-    so does this one's, at other sizes: single sizes differ by 0.9 to 1.4 x either way, the means do not.  Up to 2,048 k-values the activation's two
-    trips to memory weigh as much as a fifth of the product: 1.08 x as fast in the mean over 385 to 16,384 rows, at up to 1,600 also
-    from 129 rows on (1.05 x); with fewer rows of deeper weights the library's tiles for few rows are better (11,264 x 2,048 at 300 rows: 28 us
-    for 31).  Deep weights (37,888 x 3,584): 1.02 to 1.15 x at 1,600 to 3,500 rows (2,048: 551 us for 481), but 0.8 to 1.1 x at fewer (512: 145
-    for 165 to 188) and 0.87 to 0.95 x at more (8,192: 1,790 for 1,900), where the library comes closer to the matrix cores' rate.  Where the caller
-    has the library time its kernels (``enable_library_gemm_tuning``), its choice is the faster one (2,048 tokens through the 7B shape 25.8 ms
-    for 27.9; with its default choice 28.7 for 26.9)."""
-    if N % 4 or K % 8 or K > PAIRS_MAX_K or torch.cuda.tunable.is_enabled():
-        return False
-    if K <= 2048:
-        return M > (128 if K <= 1600 else 384)
-    return 1600 <= M <= 3500
+    """Whether the product for many rows with the activation as its epilogue takes gate/up pairs [N, K] in bfloat16: where it is
+    estimated to be the faster way by a fifth or more, from the rounds of tiles that either way needs (ifx_gemm_pairs_wins in
+    csrc/gemm_tiles.hip, with the measurements).  Where the caller has the library time its kernels
+    (``enable_library_gemm_tuning``), its choice is the faster one."""
+    return N % 4 == 0 and K % 8 == 0 and not torch.cuda.tunable.is_enabled() and _pairs_tiles_win(M, N, K)
 
 
 def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, tile: int = -1) -> torch.Tensor:

@@ -703,16 +703,17 @@ def test_gated_activations_that_do_not_exist_are_refused_on_every_route(monkeypa
 
 def test_many_row_pairs_go_to_the_library_where_it_times_its_kernels(monkeypatch):
     """The route of gate/up of many rows by sizes, and with the library's tuning on; on either the same function."""
-    assert ops.pairs_tiles_take(1600, 37888, 3584) and ops.pairs_tiles_take(3500, 37888, 3584)
-    assert not ops.pairs_tiles_take(1599, 37888, 3584) and not ops.pairs_tiles_take(3501, 37888, 3584)
-    assert ops.pairs_tiles_take(385, 512, 2048) and not ops.pairs_tiles_take(384, 512, 2048)
-    assert ops.pairs_tiles_take(129, 512, 1600) and not ops.pairs_tiles_take(128, 512, 1600)
+    for M, N, K in ((129, 2816, 64), (2048, 8192, 512), (512, 9728, 896), (2048, 5632, 1024), (16384, 16384, 256)):
+        assert ops.pairs_tiles_take(M, N, K), (M, N, K)
+    # few rows; sizes where the library's rounds are full or its tiles smaller; deeper weights than the estimates were fitted to
+    for M, N, K in ((128, 2816, 64), (129, 5632, 1024), (6144, 8192, 1024), (1800, 17920, 1536), (2048, 37888, 3584), (2048, 16384, 2048)):
+        assert not ops.pairs_tiles_take(M, N, K), (M, N, K)
     assert not ops.pairs_tiles_take(2000, 510, 512) and not ops.pairs_tiles_take(2000, 512, 516)
-    assert ops.pairs_tiles_take(2000, 4, 1 << 20) and not ops.pairs_tiles_take(2000, 4, (1 << 20) + 8)
+    assert not ops.pairs_tiles_take(2000, 8192, 1 << 20)
     x, w = torch.randn(200, 64, generator=gen(2450)).to(BF16).to(DEV), torch.randn(512, 64, generator=gen(2451)).to(BF16).to(DEV)
     ours = ops.linear_swiglu(x, w).double()
     monkeypatch.setattr(torch.cuda.tunable, "is_enabled", lambda: True)
-    assert not ops.pairs_tiles_take(200, 512, 64)
+    assert not ops.pairs_tiles_take(2048, 8192, 512) and not ops.pairs_tiles_take(200, 512, 64)
     theirs = ops.linear_swiglu(x, w).double()          # (gate and up rounded to bfloat16 in between: 2^-9 of each, twice, and of the result)
     assert ((ours - theirs).abs() <= 2.0 ** -6 * ours.abs() + 2.0 ** -6).all()
 
