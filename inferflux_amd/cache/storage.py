@@ -90,6 +90,11 @@ class CacheStorage:
         return self._bindings[entry]
 
     @property
+    def caches(self):
+        """Every layer's cache, once."""
+        return self._caches.values()
+
+    @property
     def has_state(self) -> bool:
         """Whether any mixer keeps per-request state besides keys and values (a step over it cannot be run twice)."""
         return bool(self._states)

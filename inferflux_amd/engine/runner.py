@@ -21,6 +21,7 @@ import torch
 from ..cache.manager import OutOfPages
 from ..cache.storage import CacheStorage
 from ..kernels import ops
+from ..kernels.attention import decode_kinds, table_tokens
 from .context import StepContext, StepEntry
 from .model import Model
 
@@ -41,12 +42,11 @@ class _DecodeGraph:
 
 class ModelRunner:
     GRAPH_WIDTH_MULTIPLE = 64     # block-table width (pages) a captured step is valid for, in steps of this
-    # ... but for steps whose requests all hold few tokens, whose tables are as wide as these many: attention over few keys
-    # has a launch of its own shape (see kernels.attention.row_launch_shape), which a layout that allows 1,024 cannot take.
-    GRAPH_SHORT_TOKENS = (256, 512)
+    # ... but for steps whose requests all hold few tokens, which may have launches of their own (kernels.attention.table_tokens):
+    # one layout more for each batch size, two where a model's attention differs from layer to layer
     MAX_GRAPHS = 32               # captured layouts kept; the one unused longest goes first
     # A captured step is valid for one number of rows.  A batch that shrinks a request at a time would need a capture
-    # (a wait for the GPU, an eager step, the capture: tens of milliseconds) for every size it passes through, so the
+    # (a wait for the GPU, an eager step, the capture: 3.5 to 12 ms) for every size it passes through, so the
     # batch of a captured step is filled up to the next of these sizes with rows that stand for nobody (they write
     # to a scratch page and their logits are dropped).  The sizes follow the products' kernels (up to 16 rows one
     # kernel, 17-64 another) and cost nothing there: a weight-streaming product reads the same bytes for 5 rows and 8.
@@ -63,6 +63,7 @@ class ModelRunner:
         self.storage = CacheStorage(model.plan.schedule, model.schedule_mixers(), page_size, num_pages,
                                     max_requests, model.dtype, model.device)
         self.manager = self.storage.manager
+        self._decode_kinds = decode_kinds(self.storage.caches)
         self.page_size = page_size
         self.vocab_size = model.plan.vocab_size
         self.max_position = model.plan.max_position
@@ -138,12 +139,11 @@ class ModelRunner:
 
     def _decode_context(self, entries) -> StepContext:
         """The context of a step of single tokens in the layout its captured graph has: block tables as wide as the
-        next multiple of GRAPH_WIDTH_MULTIPLE pages (or the next of GRAPH_SHORT_TOKENS), the batch filled up to the next of GRAPH_BATCH_SIZES."""
+        next multiple of GRAPH_WIDTH_MULTIPLE pages (or as few as ``table_tokens`` says), the batch filled up to the next of GRAPH_BATCH_SIZES."""
         n = len(entries)
-        longest = max((self.manager.length(e.rid) for e in entries), default=0) + 1
-        short = next((t for t in self.GRAPH_SHORT_TOKENS if longest <= t and t % self.page_size == 0), None)
-        width = min(short // self.page_size, self.GRAPH_WIDTH_MULTIPLE) if short else self.GRAPH_WIDTH_MULTIPLE
         size = next((b for b in self.GRAPH_BATCH_SIZES if b >= n), -(-n // 16) * 16)
+        longest = max((self.manager.length(e.rid) for e in entries), default=0) + 1
+        width = table_tokens(longest, size, self._decode_kinds, self.GRAPH_WIDTH_MULTIPLE * self.page_size) // self.page_size
         return StepContext(entries, self.manager, self.dtype, self.device, width_multiple=width,
                            upload=False, pad_requests=size - n, scratch_pages=self.storage.scratch_pages,
                            scratch_state_slot=self.storage.scratch_state_slot)

@@ -3,6 +3,7 @@ choice must satisfy for the kernel to be right."""
 import random
 
 import numpy as np
+import torch
 
 from inferflux_amd.kernels.attention import TILE_MAX_SPLITS, choose_tiling, tile_order
 
@@ -148,6 +149,43 @@ def test_library_products_are_cut_only_where_slices_fill_the_chip_and_stay_long(
             for K in (2048, 4096, 10000, 65536):
                 S = f(M, N, K)
                 assert S in (1, 2, 4, 8) and K % S == 0 and (S == 1 or (K // S >= 2048 and (K // S) % 8 == 0))
+
+
+def test_rows_of_few_keys_are_taken_whole():
+    """Whatever the number of pairs: up to 256 keys of heads wider than 64 elements, up to 512 of heads of 64 and from 96 pairs on."""
+    from inferflux_amd.kernels.attention import row_launch_shape
+    whole = lambda *a: row_launch_shape(*a)[1] > 0
+    for rows, kv_heads in ((1, 1), (1, 2), (24, 2), (95, 1)):
+        assert whole(rows, kv_heads, 256, 8, 128) and not whole(rows, kv_heads, 257, 8, 128)
+        assert whole(rows, kv_heads, 512, 8, 64) and not whole(rows, kv_heads, 513, 8, 64)
+    for rows, kv_heads in ((96, 1), (48, 2), (191, 1)):
+        for d in (64, 128):
+            assert whole(rows, kv_heads, 512, 8, d) and not whole(rows, kv_heads, 513, 8, d)
+    assert whole(192, 1, 513, 8, 128) and whole(96, 2, 100000, 8, 64)
+
+
+def test_captured_steps_have_short_tables_where_that_changes_a_launch():
+    from inferflux_amd.cache.storage import LayerCache
+    from inferflux_amd.kernels.attention import decode_kinds, row_launch_shape, table_tokens
+    cache = lambda n_kv, d, dv, page=16, dtype=torch.bfloat16: LayerCache(torch.empty(1, n_kv, page, d, dtype=dtype),
+                                                                        torch.empty(1, n_kv, dv, page, dtype=dtype), 0, page)
+    few, small, latent = cache(4, 128, 128), cache(2, 64, 64), cache(1, 576, 512)
+    assert decode_kinds([few, few, latent, small]) == ((1, 0), (2, 64), (4, 128))
+    assert decode_kinds([cache(2, 64, 64, dtype=torch.float32), cache(2, 80, 96), cache(2, 128, 128, page=512)]) == ()
+    bounds = lambda caches, rows, most=1024: [table_tokens(n, rows, decode_kinds(caches), most) for n in (1, 255, 256, 257, 511, 512, 513, 1024, 1025)]
+    assert bounds([few], 8) == [256] * 3 + [1024] * 6                     # 32 pairs
+    assert bounds([few], 32) == [512] * 6 + [1024] * 3                    # 128 pairs
+    assert bounds([few], 48) == [1024] * 9                                # 192 pairs: whole at any length
+    assert bounds([small], 1) == [512] * 6 + [1024] * 3
+    assert bounds([latent], 64) == [256] * 3 + [1024] * 6
+    assert bounds([few, small], 1) == [256] * 3 + [512] * 3 + [1024] * 3  # layers that differ: two more
+    assert bounds([], 1) == [1024] * 9                                    # (the plain kernel's launches do not depend on it)
+    assert bounds([few], 1, most=32) == [32] * 9
+    for rows in (1, 2, 8, 16, 24, 32, 48, 64):                            # no layout whose launch is that of the wide one
+        for n_kv, d in ((1, 128), (2, 64), (2, 128), (4, 128), (8, 128)):
+            for n in (1, 256, 300, 512, 600):
+                t = table_tokens(n, rows, decode_kinds([cache(n_kv, d, d)]), 1024)
+                assert t == 1024 or (row_launch_shape(rows, n_kv, t, 8, d)[1] > 0 and row_launch_shape(rows, n_kv, 1024, 8, d)[1] == 0)
 
 
 def test_row_launch_shape():

@@ -474,6 +474,56 @@ def test_replayed_decode_graphs_equal_eager_steps(name, dtype, sharp_folders):
 
 
 @pytest.mark.parametrize("name", ["A", "C"])
+def test_replayed_decode_graphs_with_rows_in_splits(name, sharp_folders, monkeypatch):
+    """The same where no row is taken whole: every decode step through splits of the keys and the launch that merges them."""
+    from inferflux_amd.kernels import attention, ops
+    used = []
+    real = ops.attention_rows
+    monkeypatch.setattr(ops, "attention_rows", lambda *a: (used.append(a[-2]), real(*a))[1])
+    monkeypatch.setattr(attention, "ROW_WHOLE_SHORT", 0)
+    test_replayed_decode_graphs_equal_eager_steps(name, "bfloat16", sharp_folders)
+    assert used and all(w == 0 for w in used)
+
+
+@pytest.mark.parametrize("d,short", [(64, 512), (128, 256)])
+def test_decode_steps_across_the_short_tables_ends(d, short, tmp_path, monkeypatch):
+    """Replayed decode steps at the usual table widths as requests grow past 256 and 512 tokens: short tables, whose rows a workgroup
+    takes whole, up to where that ends (512 tokens for heads of 64, 256 for wider ones), tables of 1,024 and splits from there on; the
+    plain model's logits throughout."""
+    from conftest import sharpen
+    from inferflux_amd.config import config_from_dict
+    from inferflux_amd.kernels import ops
+    from inferflux_amd.weights import write_random_model
+    cfg = dict(TINY["A"], head_dim=d, num_attention_heads=2, num_key_value_heads=1, max_position_embeddings=1200)
+    write_random_model(str(tmp_path / "m"), config_from_dict(cfg), seed=120, dtype=torch.bfloat16)
+    sharpen(str(tmp_path / "m"), str(tmp_path / "s"), 220, 2.0)
+    used, real = [], ops.attention_rows
+    monkeypatch.setattr(ops, "attention_rows", lambda *a: (used.append(a[-2]), real(*a))[1])
+    runner = load_runner(str(tmp_path / "s"), torch.bfloat16, num_pages=128, max_requests=2)
+    seqs = {"a": seeded_ids(460, 530, cfg["vocab_size"]), "b": seeded_ids(461, 60, cfg["vocab_size"])}
+    want = {r: plain_logits(str(tmp_path / "s"), ids) for r, ids in seqs.items()}
+    at = {"a": 250, "b": 20}
+    for r in seqs:
+        runner.add_request(r)
+        runner.step([StepEntry(r, seqs[r][:at[r]], [])])
+    got, places = {"a": [], "b": []}, {"a": [], "b": []}
+    for k in range(32):
+        if k == 16:
+            runner.step([StepEntry("a", seqs["a"][at["a"]:505], [])])
+            at["a"] = 505
+        used.clear()
+        logits = runner.step([StepEntry(r, [seqs[r][at[r]]], [0]) for r in seqs]).float().cpu()
+        assert all((w > 0) == (at["a"] < short) for w in used), at          # (used: what an eager or captured step launched)
+        for i, r in enumerate(seqs):
+            got[r].append(logits[i].clone()); places[r].append(at[r])
+            at[r] += 1
+    assert at["a"] > 513 and {key[3] for key in runner._graphs} == {(short // 16,), (64,)} and runner.graph_replays == 32 - 2
+    for r in seqs:
+        assert rel_err(torch.stack(got[r]), want[r][places[r]]) < tol("bfloat16", "A"), r
+    runner.manager.check()
+
+
+@pytest.mark.parametrize("name", ["A", "C"])
 def test_decode_rows_taken_whole_by_one_workgroup_in_the_engine(name, sharp_folders, monkeypatch):
     """The row kernel that takes a (row, kv head) pair whole in one workgroup, inside the engine: forced for every
     step of single tokens (it is chosen from 192 pairs on, which tiny models reach only with 64 requests: the second
