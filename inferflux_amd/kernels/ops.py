@@ -1436,7 +1436,7 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                     positions: torch.Tensor, block_table: torch.Tensor, window: Optional[int],
                     scale: float, keep_first: int = 0, sink: Optional[float] = None,
                     gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, chunk: Optional[int] = None,
-                    differential: Optional[Tuple[float, float, float]] = None) -> torch.Tensor:
+                    differential: Optional[Tuple[float, float, float]] = None, row_waves: int = 0) -> torch.Tensor:
     """Causal (optionally windowed) attention of q [T, nH, d] over the paged cache (K [pages, nKV, page, d],
     V [pages, nKV, dv, page]; dv may differ from d); returns [T, nH*dv].  ``keep_first``: a windowed query also sees
     the first so many positions of its request; ``sink``: the score of a key without value that is added to the
@@ -1444,7 +1444,8 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     [T, nH]: a factor on every head's output; ``chunk``: a query sees only keys of its own block of that many positions,
     counted from the sequence's start.  ``differential`` (lambda, out_scale, eps): q and the keys hold two vectors of
     d / 2 elements per head, each pair a softmax map of its own over the same values; a head's output is map 1 minus
-    lambda times map 2, divided by its root mean square (eps inside the root), times out_scale."""
+    lambda times map 2, divided by its root mean square (eps inside the root), times out_scale.  ``row_waves``: waves to a row and
+    head, 1 or 4 (0 lets the kernel choose; the same bits either way)."""
     _check(q, "q", (None, None, None))
     T, nH, d = q.shape
     maps = 2 if differential is not None else 1
@@ -1463,11 +1464,11 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if gate is not None:
         _check(gate, "gate", (T, nH), torch.float32)
     out = torch.empty((T, nH * dv), dtype=q.dtype, device=q.device)
-    _call(load_module("attn_plain"), "ifx_attn_plain", (P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, P, P, I, I, F, F, F, P),
+    _call(load_module("attn_plain"), "ifx_attn_plain", (P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, P, P, I, I, F, F, F, I, P),
           q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _dt(q), row_req.data_ptr(),
           positions.data_ptr(), block_table.data_ptr(), block_table.shape[1], T, nH, nKV, d // maps, dv, page_size,
           int(window or 0), float(scale), int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), _ptr(gate),
-          _ptr(sinks), int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), _stream())
+          _ptr(sinks), int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), int(row_waves), _stream())
     return out
 
 

@@ -413,6 +413,26 @@ def test_attention_plain_tiles_of_four_waves(dtype, past, window):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("past", [0, 63, 64, 127, 128, 200, 255, 256, 330, 700])
+@pytest.mark.parametrize("form", ["plain", "window", "first", "sink", "differential", "block"])
+def test_attention_plain_one_wave_and_four_give_the_same_bits(dtype, past, form):
+    """A row and head by one wave or by four, whose choice hangs on what else is in the step: rows with tiles in one part, in some
+    and in all, with and without a sink that starts the first."""
+    nH, nKV, d, dv, P, T = 6, 3, 24, 40, 16, 5
+    g = gen(1780 + past)
+    n, pages = past + T, -(-(past + T) // P)
+    q, kc, vc = (torch.randn(*s, generator=g).to(dtype).to(DEV) for s in ((T, nH, d), (pages, nKV, P, d), (pages, nKV, dv, P)))
+    more = {"plain": {}, "window": dict(window=70), "first": dict(window=130, keep_first=5, sink=0.3, gate=torch.rand(T, nH, generator=g).to(DEV)),
+            "sink": dict(window=40, sinks=torch.randn(nH, generator=g).to(DEV)), "differential": dict(differential=(0.4, 0.6, 1e-5)),
+            "block": dict(chunk=100)}[form]
+    window = more.pop("window", None)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    args = (q, kc, vc, i32([0] * T), i32(list(range(past, past + T))), torch.randperm(pages, generator=g).to(torch.int32)[None].to(DEV), window, 0.3)
+    one, four = (ops.attention_plain(*args, **more, row_waves=w) for w in (1, 4))
+    assert torch.equal(one, four)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("low,window,sink", [((64, 128), None, None), ((128, 256), None, None), ((0, 64), None, 0.5), ((0, 300), None, -1.0),
                                              ((192, 256), 130, None), ((64, 320), None, None), ((128, 192), 150, 0.0)])
 def test_attention_plain_tiles_whose_scores_are_all_minus_infinity(dtype, low, window, sink):
@@ -435,10 +455,11 @@ def test_attention_plain_tiles_whose_scores_are_all_minus_infinity(dtype, low, w
     pad[:n] = v
     vc = pad.view(pages, P, 1, d).permute(0, 2, 3, 1).contiguous().to(dtype).to(DEV)
     i32 = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)
-    got = ops.attention_plain(q.to(dtype).to(DEV), kc, vc, i32(0), i32(past), torch.arange(pages, dtype=torch.int32, device=DEV)[None],
-                              window, 0.25, sink=sink).cpu().double().view(2, d)
     t = dict(rtol=1e-4, atol=1e-5) if dtype == F32 else dict(rtol=1e-2, atol=1e-2)
-    assert torch.allclose(got, want, **t), float((got - want).abs().max())
+    for waves in (1, 4):
+        got = ops.attention_plain(q.to(dtype).to(DEV), kc, vc, i32(0), i32(past), torch.arange(pages, dtype=torch.int32, device=DEV)[None],
+                                  window, 0.25, sink=sink, row_waves=waves).cpu().double().view(2, d)
+        assert torch.allclose(got, want, **t), (waves, float((got - want).abs().max()))
 
 
 @pytest.mark.parametrize("seed", range(24))
