@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void add_layernorm4_kernel(float* __restrict__
   float x[NV][4];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int i = 4 * (threadIdx.x + 256 * v);
+    const int i = 4 * (threadIdx.x + blockDim.x * v);
     if (i >= H) continue;
     d0[v] = *(const typename Four<TD>::type*)(d + i);
     was[v] = *(const float4*)(s + i);
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void add_layernorm4_kernel(float* __restrict__
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     x[v][0] = x[v][1] = x[v][2] = x[v][3] = 0.f;
-    if (4 * (int)(threadIdx.x + 256 * v) < H) widen(d0[v], x[v]);
+    if (4 * (int)(threadIdx.x + blockDim.x * v) < H) widen(d0[v], x[v]);
   }
   for (int k0 = 1; k0 < n_slices; k0 += AT_ONCE) {          // partial sums, added in slice order
     typename Four<TD>::type p[AT_ONCE][NV];
@@ -145,14 +145,14 @@ __global__ __launch_bounds__(256) void add_layernorm4_kernel(float* __restrict__
     for (int u = 0; u < AT_ONCE; ++u)
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        const int i = 4 * (threadIdx.x + 256 * v);
+        const int i = 4 * (threadIdx.x + blockDim.x * v);
         if (k0 + u < n_slices && i < H) p[u][v] = *(const typename Four<TD>::type*)(d + (size_t)(k0 + u) * slice_stride + i);
       }
 #pragma unroll
     for (int u = 0; u < AT_ONCE; ++u)
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        if (k0 + u >= n_slices || 4 * (int)(threadIdx.x + 256 * v) >= H) continue;
+        if (k0 + u >= n_slices || 4 * (int)(threadIdx.x + blockDim.x * v) >= H) continue;
         float f[4];
         widen(p[u][v], f);
 #pragma unroll
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void add_layernorm4_kernel(float* __restrict__
   float sq = 0.f;
 #pragma unroll
   for (int v = 0; v < NV; ++v)
-    if (4 * (int)(threadIdx.x + 256 * v) < H)
+    if (4 * (int)(threadIdx.x + blockDim.x * v) < H)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         x[v][e] -= mean;
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void add_layernorm4_kernel(float* __restrict__
   const float rstd = 1.0f / sqrtf(block_sum(sq, red) / (float)H + eps);
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int i = 4 * (threadIdx.x + 256 * v);
+    const int i = 4 * (threadIdx.x + blockDim.x * v);
     if (i >= H) continue;
     float y[4], w[4];
     widen(was[v], y);
@@ -250,7 +250,8 @@ extern "C" int ifx_add_layernorm(float* stream_rows, const void* delta, int delt
   const size_t lds = (size_t)H * sizeof(float);
   // (operands on 16 bytes and slices a multiple of 4 apart, for loads of four elements)
   const bool fours = H % 4 == 0 && H <= 4096 && slice_stride % 4 == 0 && ((uintptr_t)stream_rows | (uintptr_t)delta | (uintptr_t)weight | (uintptr_t)cast_out) % 16 == 0;
-#define ALN4(TD, TC, TW, NV) hipLaunchKernelGGL((add_layernorm4_kernel<TD, TC, TW, NV>), dim3(T), dim3(256), 0, s, stream_rows, (const TD*)delta, \
+  const int threads4 = min(256, (H / 4 + WAVE - 1) / WAVE * WAVE);      // (a run of four columns to a thread: narrow rows fill fewer)
+#define ALN4(TD, TC, TW, NV) hipLaunchKernelGGL((add_layernorm4_kernel<TD, TC, TW, NV>), dim3(T), dim3(threads4), 0, s, stream_rows, (const TD*)delta, \
                                                 n_slices, (size_t)slice_stride, (const TW*)weight, (TC*)cast_out, H, eps)
 #define ALN_ROWS(TD, TC)                                                \
   do {                                                                  \

@@ -152,8 +152,13 @@ __global__ __launch_bounds__(256) void gated_add_kernel(const void* __restrict__
   }
 }
 
-// The same in bfloat16 for widths of multiples of 4 (and K of 8): a workgroup takes 1,024 columns of a row and asks for everything
-// it needs at once, the partial sums eight at a time (2,048 columns, one row, four slices: 9.8 us above).
+// The same in bfloat16 for widths of multiples of 4 (and K of 8).  Few rows: a workgroup takes 1,024 columns of a row and asks for
+// everything it needs at once, the partial sums eight at a time.  MANY rows, where the memory is what bounds it: a workgroup
+// takes a row, so that its gate is formed once, of as many threads as the row has columns for, two partial sums at a time, so that
+// more of them fit a compute unit.  us above, of few rows, of many (base of so many slices, with a gate): 2,048 columns, 64
+// rows, 4 slices 6.9, 3.6, 4.2; 1,024 rows 13.4, 8.2, 7.9; 2,048 rows 18.8, 18.3, 15.2; 5,120 columns, 2,048 rows, 2 slices 27.8, 35.6,
+// 22.8; 256 columns, 64 rows, 4 slices 3.6, 3.7, 3.5, 4,096 rows 7.1, 8.9, 5.0; 1,024 columns, 1,024 rows, 1 slice 5.2, 3.7, 4.4.
+template <bool MANY>
 __global__ __launch_bounds__(256) void gated_add4_kernel(const void* __restrict__ base, int base_f32, int n_slices, size_t slice_stride,
                                                          const void* __restrict__ extra, int extra_f32, int extra_slices, size_t extra_stride,
                                                          const bf16_t* __restrict__ h, const bf16_t* __restrict__ w, int K,
@@ -162,8 +167,8 @@ __global__ __launch_bounds__(256) void gated_add4_kernel(const void* __restrict_
   union Raw { float4 f; bf16x4 h; };
   __shared__ float red[16];
   const size_t t = blockIdx.x;
-  const int c = 4 * (blockIdx.y * 256 + threadIdx.x);
-  constexpr int AT_ONCE = 8;
+  int c = 4 * ((MANY ? 0 : blockIdx.y * 256) + threadIdx.x);
+  constexpr int AT_ONCE = MANY ? 2 : 8;
   Raw b[AT_ONCE], e[AT_ONCE];
   auto ask = [&](const void* p, int f32, int slices, size_t stride, int k0, Raw* r) {
     if (c >= N) return;
@@ -190,23 +195,30 @@ __global__ __launch_bounds__(256) void gated_add4_kernel(const void* __restrict_
   float gate = 1.0f;
   if (w) {
     float z = 0.f;
-    for (int k = 8 * threadIdx.x; k < K; k += 8 * 256) {
+    for (int k = 8 * threadIdx.x; k < K; k += 8 * (MANY ? blockDim.x : 256)) {
       const row_bf16x8 x8 = *(const row_bf16x8*)(h + t * K + k), w8 = *(const row_bf16x8*)(w + k);
 #pragma unroll
       for (int i = 0; i < 8; ++i) z = fmaf((float)x8[i], (float)w8[i], z);
     }
     gate = 1.0f / (1.0f + expf(-block_sum(z, red)));
   }
-  float bv[4] = {0.f, 0.f, 0.f, 0.f}, ev[4] = {0.f, 0.f, 0.f, 0.f};
-  add(base_f32, n_slices, 0, b, bv);
-  add(extra_f32, extra_slices, 0, e, ev);
-  for (int k0 = AT_ONCE; k0 < n_slices; k0 += AT_ONCE) { ask(base, base_f32, n_slices, slice_stride, k0, b); add(base_f32, n_slices, k0, b, bv); }
-  for (int k0 = AT_ONCE; k0 < extra_slices; k0 += AT_ONCE) { ask(extra, extra_f32, extra_slices, extra_stride, k0, e); add(extra_f32, extra_slices, k0, e, ev); }
-  if (c >= N) return;
-  bf16x4 y;
+  for (;;) {
+    float bv[4] = {0.f, 0.f, 0.f, 0.f}, ev[4] = {0.f, 0.f, 0.f, 0.f};
+    add(base_f32, n_slices, 0, b, bv);
+    add(extra_f32, extra_slices, 0, e, ev);
+    for (int k0 = AT_ONCE; k0 < n_slices; k0 += AT_ONCE) { ask(base, base_f32, n_slices, slice_stride, k0, b); add(base_f32, n_slices, k0, b, bv); }
+    for (int k0 = AT_ONCE; k0 < extra_slices; k0 += AT_ONCE) { ask(extra, extra_f32, extra_slices, extra_stride, k0, e); add(extra_f32, extra_slices, k0, e, ev); }
+    if (c >= N) return;
+    bf16x4 y;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) y[i] = (__bf16)fmaf(gate, ev[i], bv[i]);
-  *(bf16x4*)(out + t * N + c) = y;
+    for (int i = 0; i < 4; ++i) y[i] = (__bf16)fmaf(gate, ev[i], bv[i]);
+    *(bf16x4*)(out + t * N + c) = y;
+    if (!MANY) return;
+    c += 4 * blockDim.x;
+    if (c >= N) return;
+    ask(base, base_f32, n_slices, slice_stride, 0, b);
+    ask(extra, extra_f32, extra_slices, extra_stride, 0, e);
+  }
 }
 
 extern "C" int ifx_gated_add(const void* base, int base_f32, int n_slices, long long slice_stride, const void* extra, int extra_f32,
@@ -219,9 +231,12 @@ extern "C" int ifx_gated_add(const void* base, int base_f32, int n_slices, long 
   // (operands on 16 bytes, for loads of four and eight elements)
   const bool fours = dtype == DT_BF16 && N % 4 == 0 && K % 8 == 0 && slice_stride % 4 == 0 && extra_stride % 4 == 0 && N <= 4 * 256 * 65535ll &&
                      ((uintptr_t)base | (uintptr_t)extra | (uintptr_t)h | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
-  if (fours)
-    hipLaunchKernelGGL(gated_add4_kernel, dim3(T, (N + 1023) / 1024), dim3(256), 0, s, base, base_f32, n_slices, (size_t)slice_stride, extra,
-                       extra_f32, extra_slices, (size_t)extra_stride, (const bf16_t*)h, (const bf16_t*)w, K, (bf16_t*)out, N);
+#define FOURS(MANY, GRID, THREADS)                                                                                                    \
+  hipLaunchKernelGGL(gated_add4_kernel<MANY>, GRID, dim3(THREADS), 0, s, base, base_f32, n_slices, (size_t)slice_stride, extra, extra_f32, \
+                     extra_slices, (size_t)extra_stride, (const bf16_t*)h, (const bf16_t*)w, K, (bf16_t*)out, N)
+  if (fours && (T > 1024 || N <= 256 || (long long)T * N > 1 << 20)) FOURS(true, dim3(T), min(256, (N / 4 + WAVE - 1) / WAVE * WAVE));
+  else if (fours) FOURS(false, dim3(T, (N + 1023) / 1024), 256);
+#undef FOURS
   else if (dtype == DT_BF16)
     hipLaunchKernelGGL(gated_add_kernel<bf16_t>, dim3(T), dim3(256), 0, s, base, base_f32, n_slices, (size_t)slice_stride, extra, extra_f32,
                        extra_slices, (size_t)extra_stride, (const bf16_t*)h, (const bf16_t*)w, K, (bf16_t*)out, N);

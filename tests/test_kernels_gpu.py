@@ -571,6 +571,50 @@ def test_linear_takes_columns_of_wider_rows_and_no_other_strides(M, wdtype):
                         f(x, weight)
 
 
+@pytest.mark.parametrize("H", [4, 252, 256, 260, 768, 1020, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("slices", [1, 2, 8, 9, 20])
+@pytest.mark.parametrize("wdtype", [F32, BF16])
+def test_add_layernorm_widths_and_slices(H, slices, wdtype):
+    """Widths on both sides of every number of threads and of runs of four columns a thread holds, and of the general kernel's; partial
+    sums in one round of loads and several.  Float sums over H and the slices: relative errors of at most (slices + 12) 2^-24 of the
+    terms' sizes; 1e-5 of the largest value holds with room."""
+    g = gen(2500 + H)
+    T = 3
+    x, w = torch.randn(T, H, generator=g), (1.0 + 0.3 * torch.randn(H, generator=g)).to(wdtype)
+    parts = torch.randn(slices, T, H, generator=g) + 0.5
+    for delta in [parts if slices > 1 else parts[0]] + ([parts[0].to(BF16)] if slices == 1 else []):
+        d = delta.double().sum(0) if slices > 1 else delta.double()
+        d = d - d.mean(1, keepdim=True)
+        want = x.double() + d * torch.rsqrt(d.pow(2).mean(1, keepdim=True) + 1e-5) * w.double()
+        for cast in (F32, BF16, None):
+            stream = x.to(DEV)
+            arg = ops.SliceSums(delta.to(DEV), BF16) if slices > 1 else delta.to(DEV)
+            got = ops.add_layernorm(stream, arg, w.to(DEV), 1e-5, cast)
+            assert (stream.cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
+            assert cast is None or torch.equal(got, stream.to(cast))
+
+
+@pytest.mark.parametrize("T,N", [(2, 4), (3, 252), (3, 260), (3, 1024), (3, 1028), (2, 2052), (2, 5120), (1025, 4), (1030, 260), (1025, 1028), (520, 2052), (410, 2560)])
+@pytest.mark.parametrize("slices", [1, 2, 3, 8, 9, 20])
+@pytest.mark.parametrize("gated", [True, False])
+def test_gated_add_widths_and_slices(T, N, slices, gated):
+    """Few rows (1,024 columns to a workgroup, several of them, partial sums in one round of eight and more) and many (a row to a workgroup,
+    two at a time), slices on either operand: one rounding to bfloat16 (2^-8 of the value) over float sums."""
+    g = gen(2600 + N)
+    h, w = torch.randn(T, N, generator=g).to(BF16), (torch.randn(N, generator=g) / N ** 0.5).to(BF16)
+    one = torch.randn(T, N, generator=g).to(BF16)
+    parts = torch.randn(slices, T, N, generator=g) if slices > 1 else None
+    gate = torch.sigmoid(h.double() @ w.double())[:, None] if gated else 1.0
+    dev = lambda t: t.to(DEV)
+    s = ops.SliceSums(dev(parts), BF16) if slices > 1 else dev(one)
+    total = parts.double().sum(0) if slices > 1 else one.double()
+    size = parts.double().abs().sum(0) if slices > 1 else one.double().abs()
+    for base, extra, b, e in ((s, dev(one), total, one.double()), (dev(one), s, one.double(), total)):
+        got = ops.gated_add(base, extra, dev(h), dev(w) if gated else None).cpu().double()
+        want = b + gate * e
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (size + one.double().abs())).all()
+
+
 def test_zero_slot():
     """One slot of tensors of several types and sizes, on and off 16 bytes to a slot: zeros there, everything else as it was."""
     shapes = [((5, 3, 7), F32), ((5, 16, 64, 128), F32), ((5, 9), BF16), ((5, 4), torch.int32), ((5, 1), BF16)]
