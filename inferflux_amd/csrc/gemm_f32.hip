@@ -222,9 +222,11 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
 #define FEW(MT, NT)                                                                                              \
   hipLaunchKernelGGL((gemm_f32_few_kernel<TA, TO, MT, NT, 4, VEC>),                                              \
                      dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K)
-  if (M <= 16 || (t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
-  else if (t21 <= t22 && t21 <= tiles) FEW(2, 1);
-  else if (t22 <= tiles) FEW(2, 2);
+  // (a grid has at most 65,535 rows: millions of rows by a handful of columns are the tile kernel's, whose limit the caller checks)
+  const bool in16 = (M + 15) / 16 <= 65535, in32 = (M + 31) / 32 <= 65535;
+  if (M <= 16 || (in16 && t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
+  else if (in32 && t21 <= t22 && t21 <= tiles) FEW(2, 1);
+  else if (in32 && t22 <= tiles) FEW(2, 2);
   else
     hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K);
 #undef FEW

@@ -528,6 +528,21 @@ def test_gemm_f32_kernels_agree_bit_for_bit(N, K, adtype):
     assert torch.equal(ops.gemm_f32(shifted, w, None, F32), whole)
 
 
+@pytest.mark.parametrize("M", [1_048_560, 1_048_561, 2_097_120, 2_097_121, 2_200_000, 4_194_240])
+def test_gemm_f32_of_millions_of_rows(M):
+    """Rows on both sides of what a grid of 16 or 32 of them to a workgroup holds, and the most that a product takes; one more is refused."""
+    g = gen(2150)
+    w = torch.randn(3, 4, generator=g).to(DEV)
+    x = torch.randn(M, 4, device=DEV)
+    got = ops.gemm_f32(x, w, None, F32)
+    assert (got.double() - x.double() @ w.double().t()).abs().max() < 1e-5
+    ends = torch.cat([x[:5], x[-5:]])
+    assert torch.equal(ops.gemm_f32(ends, w, None, F32), torch.cat([got[:5], got[-5:]]))
+    if M == 4_194_240:
+        with pytest.raises(ops.KernelError):
+            ops.gemm_f32(torch.empty(M + 1, 4, device=DEV), w, None, F32)
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 64])
 @pytest.mark.parametrize("N,K,wide,first", [(24, 8, 16, 8), (130, 128, 136, 0), (1024, 64, 3200, 3136)])
 @pytest.mark.parametrize("tiled", [False, True])
