@@ -696,26 +696,18 @@ def moe_few_takes(dtype: torch.dtype, T: int, K: int, ff: int, n_routed: int, to
     return grouped_takes(dtype, K, ff) and 0 < T <= MOE_FEW_MAX_ROWS and n_routed <= MOE_FEW_MAX_EXPERTS and top <= 32
 
 
-def moe_few(h: torch.Tensor, router, gate_up: torch.Tensor, down: torch.Tensor, top: int, groups: int = 1, keep_groups: int = 1,
-            group_top: int = 2, softmax: bool = False, renormalize: bool = False, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
-            choice_bias: Optional[torch.Tensor] = None, act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0,
-            weigh_input: bool = False) -> "SliceSums":
-    """``moe_route`` and ``moe_experts`` in one for up to 64 rows in bfloat16: the router's logits as a product (float32 sums
-    and output), a launch that chooses, and two that stream every chosen expert's weights once, whatever the number of rows
-    that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``).  Returns the choices' weighted outputs as ``SliceSums``
-    [top, T, N] like ``moe_experts_grouped``."""
+def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_groups: int = 1, group_top: int = 2, softmax: bool = False,
+                   renormalize: bool = False, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
+                   choice_bias: Optional[torch.Tensor] = None):
+    """``moe_route`` for up to 64 rows in bfloat16: the router's logits as a product (float32 sums and output) and a launch that
+    chooses.  Returns (ids int32 [T, top], weights float32 [T, top])."""
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
-    gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
-    n_real, ff = gu_shape[0], gu_shape[1] // 2
-    down_shape, down_ptr, down_tiled = _experts(down, "down", (n_real, None, ff))
-    N, E = down_shape[1], n_real + int(n_identity)
     rows = router.rows if isinstance(router, LinearWeight) else router
-    _check(rows, "router", (E, K), torch.bfloat16)
-    if not moe_few_takes(h.dtype, T, K, ff, E, top):
-        raise KernelError(f"moe_few: {T} rows (at most {MOE_FEW_MAX_ROWS}), {E} experts (at most {MOE_FEW_MAX_EXPERTS}), K={K} (a multiple of 8), ff={ff} (of 16)")
-    if n_identity and N != K:
-        raise KernelError(f"moe_few: identity experts hand back the row itself, so N={N} must equal K={K}")
+    _check(rows, "router", (None, K), torch.bfloat16)
+    E = rows.shape[0]
+    if not 0 < T <= MOE_FEW_MAX_ROWS or E > MOE_FEW_MAX_EXPERTS or K % 8 or top > 32:
+        raise KernelError(f"moe_few: {T} rows (at most {MOE_FEW_MAX_ROWS}), {E} experts (at most {MOE_FEW_MAX_EXPERTS}), K={K} (a multiple of 8), top {top} (at most 32)")
     for t, nm in ((bias, "bias"), (choice_bias, "choice_bias")):
         if t is not None:
             _check(t, nm, (E,), torch.float32)
@@ -723,18 +715,50 @@ def moe_few(h: torch.Tensor, router, gate_up: torch.Tensor, down: torch.Tensor, 
     slices = mod.fn("ifx_moe_logit_slices", (I,))(K)
     z = torch.empty((slices, T, E), dtype=torch.float32, device=h.device)
     _call(mod, "ifx_moe_logits", (P, P, P, I, I, I, P), h.data_ptr(), rows.data_ptr(), z.data_ptr(), T, K, E, stream)
-    n_items = T * top
-    ids = torch.empty((n_items,), dtype=torch.int32, device=h.device)
-    weights = torch.empty((n_items,), dtype=torch.float32, device=h.device)
+    ids = torch.empty((T, top), dtype=torch.int32, device=h.device)
+    weights = torch.empty((T, top), dtype=torch.float32, device=h.device)
     _call(mod, "ifx_moe_choose", (P, I, P, P, I, I, I, I, I, I, I, I, F, P, P, P), z.data_ptr(), slices, ids.data_ptr(), weights.data_ptr(),
           T, E, top, groups, keep_groups, group_top, 1 if softmax else 0, 1 if renormalize else 0, float(scale), _ptr(bias), _ptr(choice_bias), stream)
-    a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)
+    return ids, weights
+
+
+def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, act: int = ACT_SILU,
+                    limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False) -> "SliceSums":
+    """``moe_experts`` for up to 64 rows in bfloat16: two launches that stream every chosen expert's weights once, whatever the
+    number of rows that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``; a row's ``ids`` differ from
+    each other).  Returns the choices' weighted outputs as ``SliceSums`` [top, T, N] like ``moe_experts_grouped``."""
+    _check(h, "h", (None, None), torch.bfloat16)
+    T, K = h.shape
+    gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
+    n_real, ff = gu_shape[0], gu_shape[1] // 2
+    down_shape, down_ptr, down_tiled = _experts(down, "down", (n_real, None, ff))
+    N, E, top = down_shape[1], n_real + int(n_identity), ids.shape[1]
+    _check(ids, "ids", (T, top), torch.int32)
+    _check(weights, "weights", (T, top), torch.float32)
+    if not moe_few_takes(h.dtype, T, K, ff, E, top):
+        raise KernelError(f"moe_few: {T} rows (at most {MOE_FEW_MAX_ROWS}), {E} experts (at most {MOE_FEW_MAX_EXPERTS}), K={K} (a multiple of 8), ff={ff} (of 16)")
+    if n_identity and N != K:
+        raise KernelError(f"moe_few: identity experts hand back the row itself, so N={N} must equal K={K}")
+    mod, stream = load_module("moe_few"), _stream()
+    a = torch.empty((T * top, ff), dtype=torch.bfloat16, device=h.device)
     _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
           T, E, K, ff, top, n_real, int(act), float(limit), weights.data_ptr() if weigh_input else 0, gu_tiled, stream)
     parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
     _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P), a.data_ptr(), down_ptr, parts.data_ptr(),
           weights.data_ptr(), ids.data_ptr(), T, E, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0, down_tiled, stream)
     return SliceSums(parts, torch.bfloat16)
+
+
+def moe_few(h: torch.Tensor, router, gate_up: torch.Tensor, down: torch.Tensor, top: int, groups: int = 1, keep_groups: int = 1,
+            group_top: int = 2, softmax: bool = False, renormalize: bool = False, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
+            choice_bias: Optional[torch.Tensor] = None, act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0,
+            weigh_input: bool = False) -> "SliceSums":
+    """``moe_few_choose`` and ``moe_few_experts``, one after the other."""
+    E = router.shape[0] if isinstance(router, torch.Tensor) else router.rows.shape[0]
+    if E != gate_up.shape[0] + int(n_identity):
+        raise KernelError(f"router: {E} experts where {gate_up.shape[0]} + {n_identity} are expected")
+    ids, weights = moe_few_choose(h, router, top, groups, keep_groups, group_top, softmax, renormalize, scale, bias, choice_bias)
+    return moe_few_experts(h, gate_up, down, ids, weights, act, limit, n_identity, weigh_input)
 
 
 # ----------------------------------------------------------------------------------------

@@ -125,9 +125,10 @@ class MixtureOfExperts(FeedForward):
         if self.shared_gate:
             self.shared_gate_w = tensors[f"{n}.shared.sg"].to(dtype).reshape(-1).contiguous()
 
-    def route(self, h):
-        return ops.moe_route(h, self.router, self.top, self.groups, self.keep_groups, self.group_top,
-                             self.scoring == "softmax", self.renormalize, self.route_scale, self.bias, self.correction)
+    def route(self, h, few: bool = False):
+        return (ops.moe_few_choose if few else ops.moe_route)(
+            h, self.router, self.top, self.groups, self.keep_groups, self.group_top, self.scoring == "softmax", self.renormalize,
+            self.route_scale, self.bias, self.correction)
 
     def _with_shared(self, out, x, ctx):
         """The chosen experts' sum plus the shared expert's output (times its gate of one number per row)."""
@@ -138,14 +139,13 @@ class MixtureOfExperts(FeedForward):
 
     def forward(self, h, ctx):
         x = h if h.dtype == self.router.dtype else h.to(self.router.dtype)
-        if self.up is None and ops.moe_few_takes(x.dtype, x.shape[0], self.hidden_size, self.ff, self.n_routed, self.top):
-            return self._with_shared(ops.moe_few(x, self.router, self.gate, self.down, self.top, self.groups, self.keep_groups,
-                                                 self.group_top, self.scoring == "softmax", self.renormalize, self.route_scale,
-                                                 self.bias, self.correction, self.act, self.limit, self.n_identity,
-                                                 self.weigh_input), x, ctx)      # (partial sums, one per choice)
-        ids, weights = self.route(x)
+        few = self.up is None and ops.moe_few_takes(x.dtype, x.shape[0], self.hidden_size, self.ff, self.n_routed, self.top)
+        ids, weights = self.route(x, few)
         if ctx.timer is not None:
             ctx.timer.mark("ffn.route")
+        if few:
+            return self._with_shared(ops.moe_few_experts(x, self.gate, self.down, ids, weights, self.act, self.limit, self.n_identity,
+                                                         self.weigh_input), x, ctx)      # (partial sums, one per choice)
         if self.up is None and (isinstance(self.gate, ops.ExpertTiles) or x.shape[0] * self.top >= GROUPED_MIN_ITEMS):
             return self._with_shared(ops.moe_experts_grouped(x, self.gate, self.down, ids, weights, self.act, self.limit,
                                                              self.n_identity, self.weigh_input), x, ctx)      # (partial sums, one per choice)

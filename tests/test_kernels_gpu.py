@@ -698,6 +698,22 @@ def test_moe_few(T, E, identity, top, K, ff, groups, keep, group_top, form):
     assert (out - want)[clear].abs().max() < 5 * 2.0 ** -8 * max(size, want[clear].abs().max())
 
 
+@pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
+def test_a_mixture_books_its_router_whatever_the_rows(T):
+    """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
+    from inferflux_amd.parts.moe import MixtureOfExperts
+    g = gen(2250)
+    m = MixtureOfExperts("m", 64, 6, 2, 32)
+    m.load({n: (torch.randn(s.shape, generator=g) / s.shape[-1] ** 0.5).to(BF16).to(DEV) for n, s in m.param_specs().items()})
+
+    class Ctx:
+        timer = type("Timer", (), {"marks": [], "mark": lambda self, name: self.marks.append(name)})()
+    ctx = Ctx()
+    ctx.timer.marks = []
+    m.forward(torch.randn(T, 64, generator=g).to(BF16).to(DEV), ctx)
+    assert ctx.timer.marks == ["ffn.route"]
+
+
 @pytest.mark.parametrize("E,identity,top,T,K,N,ff", [
     (1, 0, 1, 1, 8, 3, 16), (2, 0, 2, 64, 72, 40, 48), (3, 0, 1, 129, 64, 130, 16), (2, 0, 1, 256, 200, 7, 80), (5, 3, 3, 301, 200, 200, 176),
     (130, 2, 2, 500, 128, 128, 64), (6, 0, 2, 1500, 512, 528, 304)])
