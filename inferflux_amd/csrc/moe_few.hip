@@ -13,7 +13,8 @@
 // The products are bound by the chosen experts' bytes.  A workgroup takes an expert and NT x 16 of its weight rows and finds the
 // expert's items itself, from the step's few ids (no ordered list, no launch that makes one); its waves split K, meet in LDS in
 // wave order, and a wave has U x 64 k-values of the rows in flight.  The items are the columns of the matrix instruction (MT x 16
-// at a time), so an item's sums depend on its own row alone.  The weights lie in tiles (1 KB of contiguous memory to a wave's
+// at a time), so an item's sums depend on its own row and on how K is dealt to the waves: by twos of 64 k-values, or in gate/up of
+// up to 16 rows by threes, so there the bits of a row may differ from those in a step of more rows.  The weights lie in tiles (1 KB of contiguous memory to a wave's
 // load): from plain rows the same kernels take 1.1 to 1.3 times as long.
 //
 // Experts of 2,048 x 1,408 (us for a whole mixture: router, choice, both products; against a wave per output element that reads

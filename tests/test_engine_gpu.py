@@ -535,6 +535,7 @@ def test_decode_rows_taken_whole_by_one_workgroup_in_the_engine(name, sharp_fold
     real = ops.attention_rows
     monkeypatch.setattr(ops, "attention_rows", lambda *a: (used.append(a[-2]), real(*a))[1])
     monkeypatch.setattr(attention, "ROW_WHOLE_MIN_PAIRS", 1)
+    monkeypatch.setattr(attention, "ROW_WHOLE_SHORT", 0)        # (rows of so few keys are taken whole without it)
     runner = load_runner(folder, torch.bfloat16, num_pages=64, max_requests=4)
     seqs = {r: seeded_ids(440 + i, n, V) for i, (r, n) in enumerate({"a": 130, "b": 47, "c": 200}.items())}
     heads = {"a": 90, "b": 7, "c": 161}
