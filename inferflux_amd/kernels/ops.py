@@ -1104,7 +1104,8 @@ def qkv_rope_append(x: torch.Tensor, weight: LinearWeight, bias: Optional[torch.
 def columns_on_16_bytes(x) -> bool:
     """Whether ``x`` is a bfloat16 matrix on the GPU whose rows are columns of wider rows, each run of eight on 16 bytes: what
     ``skinny_gemm`` reads where it lies."""
-    return (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and not x.is_contiguous()
+    # (asked on every launch: whole rows leave at once)
+    return (type(x) is torch.Tensor and not x.is_contiguous() and x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2
             and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0)
 
 
@@ -1278,11 +1279,11 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
         raise KernelError(f"linear: weight {weight.dtype} with activation {x.dtype} is not supported")
     if not columns:
         _check(x if not isinstance(x, ScaledRows) else x.rows, "x", (None, weight.shape[1]))
+    elif x.shape[1] != weight.shape[1]:
+        raise KernelError(f"x: shape {tuple(x.shape)}, expected {(None, weight.shape[1])}")
     _check(weight, "weight", (None, None))
     out_dtype = out_dtype or torch.bfloat16
     M, K = x.shape
-    if K != weight.shape[1]:
-        raise KernelError(f"x: shape {tuple(x.shape)}, expected {(None, weight.shape[1])}")
     kind = _small_m_kernel(M, weight.shape[0], K, tiled is not None)
     if columns and kind != "skinny":
         x = x.contiguous()
@@ -1406,7 +1407,7 @@ def pairs_tiles_take(M: int, N: int, K: int) -> bool:
     estimated to be the faster way by a fifth or more, from the rounds of tiles that either way needs (ifx_gemm_pairs_wins in
     csrc/gemm_tiles.hip, with the measurements).  Where the caller has the library time its kernels
     (``enable_library_gemm_tuning``), its choice is the faster one."""
-    return N % 4 == 0 and K % 8 == 0 and not torch.cuda.tunable.is_enabled() and _pairs_tiles_win(M, N, K)
+    return N % 4 == 0 and K % 8 == 0 and _pairs_tiles_win(M, N, K) and not torch.cuda.tunable.is_enabled()
 
 
 def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, tile: int = -1) -> torch.Tensor:
@@ -1433,11 +1434,9 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
     if isinstance(weight_pairs, LinearWeight) and weight_pairs.order is not None:
         raise KernelError("linear_swiglu: a tile order is not supported for gate/up pairs")
     columns = columns_on_16_bytes(x)          # (as for ``linear``)
-    if not columns and not isinstance(x, ScaledRows):
-        _check(x, "x", (None, rows.shape[1]))
     if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and K == rows.shape[1] \
             and pairs_tiles_take(M, rows.shape[0], K):
-        whole = x.contiguous()
+        whole = x.contiguous() if columns else x
         if whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
             return swiglu_tiles(whole, rows, act, limit)
     if act == ACT_CLAMPED_SWISH:
