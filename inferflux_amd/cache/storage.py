@@ -64,6 +64,7 @@ class CacheStorage:
         # ... and one state slot more than the manager hands out, for the same rows: what they leave there is read by nobody.
         self.scratch_state_slot = max_requests
         self._caches: Dict[int, LayerCache] = {}
+        self._query_heads: Dict[int, int] = {}
         self._states: Dict[int, torch.Tensor] = {}
         for i, e in enumerate(schedule):
             m = mixers[i]
@@ -74,6 +75,7 @@ class CacheStorage:
                 k = torch.zeros((n + 1, spec.n_kv_heads, page_size, spec.k_dim), dtype=dtype, device=device)
                 v = torch.zeros((n + 1, spec.n_kv_heads, spec.v_dim, page_size), dtype=dtype, device=device)
                 self._caches[i] = LayerCache(k, v, g, page_size)
+                self._query_heads[i] = m.query_heads
             st = m.state_spec()
             if st is not None:
                 self._states[i] = torch.zeros((max_requests + 1, *st.shape), dtype=_STATE_DTYPES[st.dtype], device=device)
@@ -91,8 +93,8 @@ class CacheStorage:
 
     @property
     def caches(self):
-        """Every layer's cache, once."""
-        return self._caches.values()
+        """Every layer's cache, once, with the number of query heads that the layer reads it with."""
+        return [(c, self._query_heads[i]) for i, c in self._caches.items()]
 
     @property
     def has_state(self) -> bool:

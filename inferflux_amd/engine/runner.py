@@ -143,7 +143,7 @@ class ModelRunner:
         n = len(entries)
         size = next((b for b in self.GRAPH_BATCH_SIZES if b >= n), -(-n // 16) * 16)
         longest = max((self.manager.length(e.rid) for e in entries), default=0) + 1
-        width = table_tokens(longest, size, self._decode_kinds, self.GRAPH_WIDTH_MULTIPLE * self.page_size) // self.page_size
+        width = table_tokens(longest, size, self._decode_kinds, self.GRAPH_WIDTH_MULTIPLE * self.page_size, self.page_size) // self.page_size
         return StepContext(entries, self.manager, self.dtype, self.device, width_multiple=width,
                            upload=False, pad_requests=size - n, scratch_pages=self.storage.scratch_pages,
                            scratch_state_slot=self.storage.scratch_state_slot)

@@ -196,31 +196,33 @@ def _work_lists(ctx, ctx_kv_heads, tile_rows, n_heads, tile_splits=1, tile_chunk
             out[k] = packed[at:at + n]
             at += n + -n % 4          # every list starts at a multiple of 16 bytes
     if rows.size:
-        out["chunk"], out["waves"], out["max_splits"] = row_launch_shape(int(rows.size), ctx_kv_heads, ctx.kv_bound, row_waves, head_dim)
+        out["chunk"], out["waves"], out["max_splits"] = row_launch_shape(int(rows.size), ctx_kv_heads, ctx.kv_bound, row_waves, head_dim,
+                                                                               n_heads // ctx_kv_heads)
     return out
 
 
-def whole_row_keys(pairs: int, head_dim: int) -> int:
-    """Keys up to which rows are taken whole by a launch of ``pairs`` (row, kv head) pairs that would split longer ones."""
-    return ROW_WHOLE_SHORT if head_dim > 64 and pairs < ROW_WHOLE_SHORT_PAIRS else 2 * ROW_WHOLE_SHORT
+def whole_row_keys(pairs: int, head_dim: int, heads_per_kv: int = 16) -> int:
+    """Keys up to which rows are taken whole by a launch of ``pairs`` (row, kv head) pairs that would split longer ones.  A workgroup
+    goes through a pair's keys once for every 16 of its query heads (32 heads on one of 128, 8 rows, us whole / in splits at 128 and 256
+    keys 11.7, 16.2 / 13.8, 13.7; 64 heads on one at 64 and 128 keys 16.2, 20.5 / 19.5, 20.0)."""
+    short = ROW_WHOLE_SHORT if head_dim > 64 and pairs < ROW_WHOLE_SHORT_PAIRS else 2 * ROW_WHOLE_SHORT
+    return short // max(1, -(-heads_per_kv // 16))
 
 
 def decode_kinds(caches):
-    """What ``table_tokens`` has to know of a model's ``caches`` (LayerCaches): the distinct (kv heads, head size) of those that
-    the row kernel reads, head size 0 for attention through a latent."""
+    """What ``table_tokens`` has to know of a model's ``caches`` (LayerCaches, each with its number of query heads): the distinct (kv
+    heads, head size, query heads per kv head) of those that the row kernel reads, head size 0 for attention through a latent."""
     kinds = set()
-    for c in caches:
+    for c, n_heads in caches:
         n_kv, page_size, d = c.k.shape[1:]
-        if ROW_WHOLE_SHORT % page_size:
-            continue
         if ops.mfma_attention_supported(c.k.dtype, d, page_size) and c.v.shape[2] == d:
-            kinds.add((n_kv, d))
+            kinds.add((n_kv, d, n_heads // n_kv))
         elif ops.wide_attention_supported(c.k.dtype, n_kv, d, c.v.shape[2], page_size):
-            kinds.add((1, 0))
+            kinds.add((1, 0, 0))
     return tuple(sorted(kinds))
 
 
-def table_tokens(longest: int, n_rows: int, kinds, most: int) -> int:
+def table_tokens(longest: int, n_rows: int, kinds, most: int, page_size: int) -> int:
     """Tokens that the block tables of a captured step of ``n_rows`` single tokens have room for where its requests hold at most
     ``longest``: ``most``, or fewer where a launch over one of the caches (``decode_kinds``) then has a shape that its shorter bound
     allows.  Rows that a workgroup takes whole: us a step at 130 to 255 / 256 to 511 tokens with tables of 1,024 tokens and of as few
@@ -229,15 +231,15 @@ def table_tokens(longest: int, n_rows: int, kinds, most: int) -> int:
     3.5 to 12 ms, which these steps pay back within 30 to 130 tokens of all requests together; a bound that brings no other
     launch gets none (512 tokens where only 256 are taken whole: 1 % at best)."""
     bounds = [most]
-    for n_kv, d in kinds:
+    for n_kv, d, per_kv in kinds:
         if d == 0:
             bounds.append(ROW_WHOLE_SHORT)
         elif n_rows * n_kv < ROW_WHOLE_MIN_PAIRS:
-            bounds.append(whole_row_keys(n_rows * n_kv, d))
-    return min(b for b in bounds if b >= longest or b == most)
+            bounds.append(whole_row_keys(n_rows * n_kv, d, per_kv))
+    return min(b for b in bounds if (b >= longest and b % page_size == 0) or b == most)
 
 
-def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int = 8, head_dim: int = 128):
+def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int = 8, head_dim: int = 128, heads_per_kv: int = 16):
     """(keys per split, waves per workgroup, splits) of a launch of the row kernel over ``n_rows`` rows whose requests
     hold at most ``max_kv`` keys (the bound of their block tables, not the lengths themselves: see
     StepContext.kv_bound).  ``max_waves``: what fits the kernel's LDS (``ops.row_waves_fit``).
@@ -254,7 +256,7 @@ def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int =
     us whole / in splits at 64 and 300 keys: 14 : 2 heads of 64, 1 row 4.5, 6.3 / 8.1; 16 : 2 heads of 128, 8 rows 5.6,
     10.2 / 11.2, 64 rows 6.1, 11.3 / 14.4, 19.9; 16 heads on one of 128, 8 rows (four waves fit) 5.6, 11.5 / 10.7."""
     pairs = n_rows * n_kv_heads
-    if pairs >= ROW_WHOLE_MIN_PAIRS or max_kv <= whole_row_keys(pairs, head_dim):
+    if pairs >= ROW_WHOLE_MIN_PAIRS or max_kv <= whole_row_keys(pairs, head_dim, heads_per_kv):
         waves = 1
         while waves * 2 <= min(max_waves, ROW_WAVE_SLOTS // pairs):
             waves *= 2

@@ -131,6 +131,10 @@ class PagedAttention(Mixer):
             return 0
         return self.n_heads * self.v_head_dim if self.gate_elementwise else self.n_heads
 
+    @property
+    def query_heads(self) -> int:
+        return self.n_heads * (2 if self.differential is not None else 1)      # (each of two maps a head of its own)
+
     def cache_spec(self) -> CacheSpec:
         window = self.window
         if self.chunk is not None:             # a block's query never reads further back than the block is long

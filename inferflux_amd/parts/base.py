@@ -158,6 +158,11 @@ class Mixer(Part):
     def state_spec(self) -> Optional[StateSpec]:
         return None
 
+    @property
+    def query_heads(self) -> int:
+        """Query heads that read the mixer's cache (launches are shaped by their number)."""
+        return getattr(self, "n_heads", 1)
+
     def forward(self, h: torch.Tensor, ctx, binding: MixerBinding) -> torch.Tensor:
         raise NotImplementedError
 

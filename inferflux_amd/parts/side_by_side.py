@@ -34,6 +34,10 @@ class SideBySideMixers(Mixer):
     def cache_spec(self):
         return next((s for s in (m.cache_spec() for m in self.mixers) if s is not None), None)
 
+    @property
+    def query_heads(self):
+        return next((m.query_heads for m in self.mixers if m.cache_spec() is not None), 1)
+
     def state_spec(self):
         return next((s for s in (m.state_spec() for m in self.mixers) if s is not None), None)
 

@@ -162,30 +162,36 @@ def test_rows_of_few_keys_are_taken_whole():
         for d in (64, 128):
             assert whole(rows, kv_heads, 512, 8, d) and not whole(rows, kv_heads, 513, 8, d)
     assert whole(192, 1, 513, 8, 128) and whole(96, 2, 100000, 8, 64)
+    assert whole(8, 1, 256, 4, 128, 16) and whole(8, 1, 128, 4, 128, 17) and not whole(8, 1, 129, 4, 128, 32)      # 16 query heads at a time
+    assert whole(8, 1, 64, 4, 128, 64) and not whole(8, 1, 65, 4, 128, 64) and whole(8, 1, 256, 8, 64, 32) and not whole(8, 1, 257, 8, 64, 32)
 
 
 def test_captured_steps_have_short_tables_where_that_changes_a_launch():
     from inferflux_amd.cache.storage import LayerCache
     from inferflux_amd.kernels.attention import decode_kinds, row_launch_shape, table_tokens
-    cache = lambda n_kv, d, dv, page=16, dtype=torch.bfloat16: LayerCache(torch.empty(1, n_kv, page, d, dtype=dtype),
-                                                                        torch.empty(1, n_kv, dv, page, dtype=dtype), 0, page)
-    few, small, latent = cache(4, 128, 128), cache(2, 64, 64), cache(1, 576, 512)
-    assert decode_kinds([few, few, latent, small]) == ((1, 0), (2, 64), (4, 128))
-    assert decode_kinds([cache(2, 64, 64, dtype=torch.float32), cache(2, 80, 96), cache(2, 128, 128, page=512)]) == ()
-    bounds = lambda caches, rows, most=1024: [table_tokens(n, rows, decode_kinds(caches), most) for n in (1, 255, 256, 257, 511, 512, 513, 1024, 1025)]
-    assert bounds([few], 8) == [256] * 3 + [1024] * 6                     # 32 pairs
+    cache = lambda n_heads, n_kv, d, dv, page=16, dtype=torch.bfloat16: (LayerCache(torch.empty(1, n_kv, page, d, dtype=dtype),
+                                                                                  torch.empty(1, n_kv, dv, page, dtype=dtype), 0, page), n_heads)
+    few, small, latent, shared = cache(28, 4, 128, 128), cache(14, 2, 64, 64), cache(16, 1, 576, 512), cache(32, 1, 128, 128)
+    assert decode_kinds([few, few, latent, small]) == ((1, 0, 0), (2, 64, 7), (4, 128, 7))
+    assert decode_kinds([cache(4, 2, 64, 64, dtype=torch.float32), cache(4, 2, 80, 96)]) == ()
+    bounds = lambda caches, rows, most=1024, page=16: [table_tokens(n, rows, decode_kinds(caches), most, page)
+                                                        for n in (1, 128, 129, 256, 257, 512, 513, 1024, 1025)]
+    assert bounds([few], 8) == [256] * 4 + [1024] * 5                     # 32 pairs
     assert bounds([few], 32) == [512] * 6 + [1024] * 3                    # 128 pairs
     assert bounds([few], 48) == [1024] * 9                                # 192 pairs: whole at any length
     assert bounds([small], 1) == [512] * 6 + [1024] * 3
-    assert bounds([latent], 64) == [256] * 3 + [1024] * 6
-    assert bounds([few, small], 1) == [256] * 3 + [512] * 3 + [1024] * 3  # layers that differ: two more
+    assert bounds([latent], 64) == [256] * 4 + [1024] * 5
+    assert bounds([shared], 8) == [128] * 2 + [1024] * 7                  # (two groups of 16 query heads to a kv head)
+    assert bounds([few, small], 1) == [256] * 4 + [512] * 2 + [1024] * 3  # layers that differ: two more
     assert bounds([], 1) == [1024] * 9                                    # (the plain kernel's launches do not depend on it)
     assert bounds([few], 1, most=32) == [32] * 9
+    assert bounds([few], 1, most=64 * 512, page=512) == [64 * 512] * 9    # (a page holds more)
     for rows in (1, 2, 8, 16, 24, 32, 48, 64):                            # no layout whose launch is that of the wide one
-        for n_kv, d in ((1, 128), (2, 64), (2, 128), (4, 128), (8, 128)):
-            for n in (1, 256, 300, 512, 600):
-                t = table_tokens(n, rows, decode_kinds([cache(n_kv, d, d)]), 1024)
-                assert t == 1024 or (row_launch_shape(rows, n_kv, t, 8, d)[1] > 0 and row_launch_shape(rows, n_kv, 1024, 8, d)[1] == 0)
+        for heads, n_kv, d in ((1, 1, 128), (4, 2, 64), (14, 2, 128), (20, 4, 128), (64, 8, 128), (40, 1, 64)):
+            for n in (1, 100, 256, 300, 512, 600):
+                t = table_tokens(n, rows, decode_kinds([cache(heads, n_kv, d, d)]), 1024, 16)
+                shape = lambda bound: row_launch_shape(rows, n_kv, bound, 8, d, heads // n_kv)[1] > 0
+                assert t == 1024 or (n <= t and shape(t) and not shape(1024))
 
 
 def test_row_launch_shape():
