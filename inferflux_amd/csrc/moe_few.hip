@@ -266,12 +266,11 @@ struct FewArgs {
 
 template <bool DOWN, bool TILED, int MT, int NT, int U>
 __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
-  extern __shared__ float red[];      // [waves - 1][NT * MT][64 lanes][4]
-  __shared__ int list[MAX_ROWS];
+  extern __shared__ float red[];      // [waves - 1][NT * MT][64 lanes][4], then the list
   const int wave = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x % WAVE, col = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (16 * NT), n_items = a.T * a.top;
-  // The expert's items in rising order (a row chooses an expert at most once: at most T of them).  Every wave finds all of
-  // them and writes the same list.
+  int* list = (int*)(red + (size_t)(nw - 1) * NT * MT * WAVE * 4);      // (room for all items: a row may name an expert twice)
+  // The expert's items in rising order.  Every wave finds all of them and writes the same list.
   const int group = a.by_item ? a.ids[blockIdx.y] : (int)blockIdx.y;
   int count = 0, first = n_items;
   for (int i0 = 0; i0 < n_items; i0 += WAVE) {
@@ -397,7 +396,7 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
 template <bool DOWN, int MT, int NT, int U>
 static int launch_few(const FewArgs& a, int n_groups, int waves, hipStream_t s) {
   const dim3 grid((a.N + 16 * NT - 1) / (16 * NT), a.by_item ? a.T * a.top : n_groups);
-  const size_t lds = (size_t)(waves - 1) * NT * MT * WAVE * 4 * sizeof(float);
+  const size_t lds = (size_t)(waves - 1) * NT * MT * WAVE * 4 * sizeof(float) + (size_t)a.T * a.top * sizeof(int);
   if (a.k_tiles > 0) hipLaunchKernelGGL((moe_few_kernel<DOWN, true, MT, NT, U>), grid, dim3(waves * WAVE), lds, s, a);
   else hipLaunchKernelGGL((moe_few_kernel<DOWN, false, MT, NT, U>), grid, dim3(waves * WAVE), lds, s, a);
   IFX_LAUNCH_CHECK();

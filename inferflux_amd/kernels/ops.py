@@ -725,8 +725,7 @@ def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_grou
 def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, act: int = ACT_SILU,
                     limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False) -> "SliceSums":
     """``moe_experts`` for up to 64 rows in bfloat16: two launches that stream every chosen expert's weights once, whatever the
-    number of rows that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``; a row's ``ids`` differ from
-    each other).  Returns the choices' weighted outputs as ``SliceSums`` [top, T, N] like ``moe_experts_grouped``."""
+    number of rows that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``).  Returns the choices' weighted outputs as ``SliceSums`` [top, T, N] like ``moe_experts_grouped``."""
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
     gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))

@@ -698,6 +698,30 @@ def test_moe_few(T, E, identity, top, K, ff, groups, keep, group_top, form):
     assert (out - want)[clear].abs().max() < 5 * 2.0 ** -8 * max(size, want[clear].abs().max())
 
 
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("T,top,E", [(1, 2, 1), (1, 32, 4), (17, 8, 3), (40, 3, 2), (64, 2, 1), (64, 32, 9), (64, 32, 256)])
+def test_moe_few_experts_of_rows_that_name_an_expert_twice(T, top, E, tiled):
+    """An expert with up to all of the 2,048 items that a step can have: every choice counts, as for the product for many rows.  One
+    rounding to bfloat16 of the activations (half a unit of 2^-8) between float sums."""
+    g = gen(2260 + T + E)
+    K, ff, N = 72, 48, 80
+    h = torch.randn(T, K, generator=g).to(BF16)
+    gate, up = ((torch.randn(E, ff, K, generator=g) / K ** 0.5).to(BF16) for _ in range(2))
+    down = (torch.randn(E, N, ff, generator=g) / ff ** 0.5).to(BF16)
+    ids = torch.randint(0, E, (T, top), generator=g, dtype=torch.int32)
+    weights = torch.rand(T, top, generator=g)
+    x = h.double()
+    a = torch.stack([torch.nn.functional.silu(x @ gate[e].double().t()) * (x @ up[e].double().t()) for e in range(E)])      # [E, T, ff]
+    every = torch.stack([a[e] @ down[e].double().t() for e in range(E)])                                                    # [E, T, N]
+    want = weights.double().t()[..., None] * every[ids.t().long(), torch.arange(T)[None]]                                   # [top, T, N]
+    pairs, d = ops.pair_gate_up(gate.to(DEV), up.to(DEV)), down.to(DEV)
+    if tiled:
+        pairs, d = ops.ExpertTiles(pairs), ops.ExpertTiles(d)
+    got = ops.moe_few_experts(h.to(DEV), pairs, d, ids.to(DEV), weights.to(DEV)).parts.cpu().double()
+    assert (got - want).pow(2).mean().sqrt() < 2.0 ** -8 * want.pow(2).mean().sqrt()
+    assert (got - want).abs().max() < 5 * 2.0 ** -8 * want.abs().max()
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
