@@ -1,44 +1,170 @@
-// out[M][N / 2] = act(x Wg^T) * (x Wu^T) for many rows, on the matrix cores (bfloat16 in and out, float sums), W [N][K] with
-// the rows of Wg and Wu in turn: a lane holds a gate and its up, and the activation is the product's epilogue, from the sums
-// as they are.  The library's product followed by a launch for the activation writes the N columns and reads them back (2,048
-// rows of 37,888 columns: 233 MB, 40 us of 545) and rounds them to bfloat16 in between.
+// Products of many rows with the activation as their epilogue, on the matrix cores (bfloat16 in and out, float sums), from the sums
+// as they are:
+//   OUT_PAIRS   out[M][N / 2] = act(x Wg^T) * (x Wu^T), W [N][K] with the rows of Wg and Wu in turn: a lane holds a gate and its up
+//   OUT_ACT     out[M][N] = act(x W^T)
+// The library's product followed by a launch for the activation writes the N columns and reads them back (2,048 rows of
+// 37,888 columns: 233 MB, 40 us of 552) and rounds them to bfloat16 in between.
 //
-// The inner loop is product_tiles.h; what is chosen here is the tile, and whether the library's product and the activation's
-// launch would be faster.  Large tiles read less of LDS for their products but there are few of them, and the last of the
-// rounds that they take on 256 CUs may be nearly empty; so choose_tile() takes the tile whose rounds are estimated to take least,
-// from what a round of each was measured to take (see `kinds`; estimates are off by 7 % in the mean square, the choice is
-// within 4 % of the best tile at nine sizes of ten).
-// (256 x 192, 256 x 128 and 384 x 128 with one workgroup to a CU were never the fastest by more than 2 %; 256 x 256 by four
-// waves of 128 x 128, which read a third less of LDS, took 700 us where eight waves take 475: one wave to a SIMD does not
-// hide the loop's own latencies.)
-//
-// The library runs a round of its 256 x 256 tiles in 0.75 to 0.8 of the time of one here (K 1,536 to 8,192: 1,300 to 1,480 TFLOP/s
-// where its rounds are full, 1,000 to 1,200 here), so what this product has to win is the activation's two trips to memory and
-// the launch, which weigh less the deeper the weight.  By K (ten weights of 1,024 to 32,768 rows, 300 to 16,384 rows of x; a replayed
-// graph, geometric mean and worst of library and activation / this): 64 1.66 x and 1.11; 256 1.52, 1.04; 512 1.40, 0.99; 640 1.21, 0.87;
-// 768 1.15, 0.82; 1,024 1.10, 0.78; 1,280 1.01, 0.71; 1,792 to 8,192 0.97, 0.65.  Beyond about 1,500 k-values the library is faster by a
-// fifth where the kernel it chooses fits the size and slower by as much where it does not (2,048 rows: N 20,480, K 3,584 354 : 283 us;
-// 37,888 x 3,584 563 : 510; 35,840 x 3,072 406 : 430; 40,960 x 2,560 368 : 418; 49,152 x 3,584 563 : 655), and no property of the
-// size tells which.  So the product is taken up to PAIRS_MAX_K k-values, where the estimate of the library's time (its rounds of
-// 256 x 256, 256 x 128 or 128 x 128, whichever least, off by 10 % in the mean) is at least 1.2 times this one's.  Of 2,300 sizes of
-// up to 1,536 k-values that rule takes 1,124: mean 1.41 x, worst 0.95 x, ten below 1; of other sizes, drawn at random, 768: mean
-// 1.80 x, worst 0.88 x (at launches of 6 us, where the launch that it saves weighs more than the 0.7 us).
+// The inner loop is wave_tiles.h, and for small tiles, of which two workgroups to a CU hide each other's ends, product_tiles.h.
+// What is chosen here is the tile.  A large tile reads less of LDS and of the caches for its products, but there are few of
+// them, and the last of the rounds that they take on 256 CUs may be nearly empty (600 rows of 22,016 x 2,048: 258 tiles of
+// 256 x 256 take 89 us, 232 of 384 x 160 49 us).  So choose_tile() takes the tile whose rounds are estimated to take least, from
+// what rounds of each were measured to take (see `kinds`: 170 sizes, off by 4 to 8 % in the mean square; the choice is 1 % off
+// the best tile in the mean; 384 x 128, 256 x 160 and 128 x 256 were the best of all by 1 % in the mean, and left out).
+// 2,048 rows of 37,888 x 3,584: 422 us (1,320 TFLOP/s; tiles of 256 x 256 by eight waves took 481, the library and the
+// activation 552); 600 of 22,016 x 2,048 49 (93; 72); 4,500 of 17,920 x 1,536 200 (255; 239).  Which sizes come here is a rule
+// of ops.py (many_tiles_take, pairs_tiles_take), with both sides measured.
 #include "product_tiles.h"
+#include "wave_tiles.h"
 
 IFX_DEFINE_LAST_ERROR()
 
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 
-struct PairsArgs {
+enum { OUT_PAIRS = 0, OUT_ACT = 1 };
+
+struct TilesArgs {
   const bf16_t* x;          // [M][K]
   const bf16_t* w;          // [N][K]
-  bf16_t* out;              // [M][N / 2]
+  bf16_t* out;              // OUT_PAIRS: [M][N / 2]; OUT_ACT: [M][N]
   int M, N, K, act;
   float limit;
 };
 
+#define GROUP 4          // tiles of x that meet a tile of W one after the other
+
+// act(g) up and act(v) for the epilogues, where a lane has 256 of them and the matrix cores wait: sigmoid from the hardware's
+// exponential and reciprocal (1 ulp each; the results are rounded to 8 bits), the tanh form of gelu as v sigmoid(2 u)
+__device__ __forceinline__ float quick_sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
+__device__ __forceinline__ float quick_gelu(float v) { return v * quick_sigmoid(1.5957691216057308f * (v + 0.044715f * v * v * v)); }
+template <int ACT> __device__ __forceinline__ float quick_gated(float g, float up, float limit) {
+  if (ACT == ACT_GELU_TANH) return quick_gelu(g) * up;
+  if (ACT == ACT_SILU) return g * quick_sigmoid(g) * up;
+  g = fminf(g, limit), up = fminf(fmaxf(up, -limit), limit);
+  return g * quick_sigmoid(1.702f * g) * (up + 1.0f);
+}
+template <int ACT> __device__ __forceinline__ float quick_act(float v) {
+  if (ACT == ACT_RELU_SQUARED) { const float r = fmaxf(v, 0.f); return r * r; }
+  return ACT == ACT_GELU_TANH ? quick_gelu(v) : v * quick_sigmoid(v);
+}
+
+template <int FN, int FM, int OUT>
+struct TilesOut {
+  static constexpr int CHUNK = OUT == OUT_ACT && FN > 8 ? FN / 2 : FN;          // fragments that are turned in LDS at a time
+  static constexpr int ROW = 16 * CHUNK * (OUT == OUT_PAIRS ? 1 : 2);      // bytes of a row of them
+  static constexpr int PITCH = ROW + 16, WAVE_BYTES = 16 * PITCH;
+  static constexpr int LDS = WaveTiles<FN, FM>::LDS + 4 * WAVE_BYTES;
+};
+
+template <int FN, int FM, int OUT, int ACT>
+__device__ __forceinline__ void tiles_out(const WaveTiles<FN, FM>& p, const TilesArgs& a, unsigned char* lds, tile_floatx4 (&acc)[FN][FM], int m, int n) {
+  typedef TilesOut<FN, FM, OUT> O;
+  // this wave's results: a buffer from its first row on; stores beyond it, or with TILE_NO_ROW for an offset, are dropped
+  const int columns = OUT == OUT_PAIRS ? a.N / 2 : a.N, first = OUT == OUT_PAIRS ? n / 2 : n;
+  const int rows = a.M - m;
+  const unsigned long long at0 = (unsigned long long)a.out + (size_t)m * columns * 2;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at0), hi = __builtin_amdgcn_readfirstlane((unsigned)(at0 >> 32));
+  const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc((void*)((unsigned long long)hi << 32 | lo), 0,
+                                                                        __builtin_amdgcn_readfirstlane(max(0, min(16 * FM, rows)) * columns * 2), 0x00020000);
+  // 16 rows of the wave's results at a time, turned in LDS so that they go out in whole lines
+  unsigned char* st = lds + WaveTiles<FN, FM>::LDS + p.wid * O::WAVE_BYTES;
+  const bool whole = columns % 8 == 0;
+#pragma unroll
+  for (int b = 0; b < FM; ++b)
+#pragma unroll
+    for (int c0 = 0; c0 < FN; c0 += O::CHUNK) {
+#pragma unroll
+      for (int c = 0; c < O::CHUNK; ++c) {
+        asm volatile("" : "+a"(acc[c0 + c][b]));          // (not before: the registers beside the sums are taken)
+        const tile_floatx4 v = acc[c0 + c][b];
+        if (OUT == OUT_PAIRS) {
+          bf16x2 y;
+          y[0] = (__bf16)quick_gated<ACT>(v[0], v[1], a.limit);
+          y[1] = (__bf16)quick_gated<ACT>(v[2], v[3], a.limit);
+          *(bf16x2*)(st + p.col * O::PITCH + c * 16 + p.g * 4) = y;
+        } else {
+          bf16x4 y;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) y[r] = (__bf16)quick_act<ACT>(v[r]);
+          *(bf16x4*)(st + p.col * O::PITCH + c * 32 + p.g * 8) = y;
+        }
+      }
+      constexpr int PIECES = O::ROW / 16;
+      const int from = first + c0 * (OUT == OUT_PAIRS ? 8 : 16), step = 16 * b * columns * 2;
+      if (whole) {
+#pragma unroll
+        for (int j0 = 0; j0 < 16 * PIECES; j0 += 64) {
+          const int j = j0 + p.lane, r = j / PIECES, at = 8 * (j % PIECES);
+          const bool in = j < 16 * PIECES && r < rows - 16 * b && from + at < columns;
+          const tile_uintx4 v = *(const tile_uintx4*)(st + min(r, 15) * O::PITCH + 2 * at);
+          __builtin_amdgcn_raw_buffer_store_b128(v, out, in ? (r * columns + from + at) * 2 : TILE_NO_ROW, step, 0);
+        }
+      } else {            // (an even number of columns)
+#pragma unroll 1
+        for (int j = p.lane; j < 64 * PIECES; j += 64) {
+          const int r = j / (4 * PIECES), at = 2 * (j % (4 * PIECES));
+          const bool in = r < rows - 16 * b && from + at < columns;
+          const unsigned v = *(const unsigned*)(st + r * O::PITCH + 2 * at);
+          __builtin_amdgcn_raw_buffer_store_b32(v, out, in ? (r * columns + from + at) * 2 : TILE_NO_ROW, step, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// One workgroup to a CU, one tile after the other.  Workgroup b runs on XCD b % 8, which takes a contiguous range of the tiles.
+template <int FN, int FM, int OUT>
+__global__ __launch_bounds__(256, 1) void tiles_kernel(TilesArgs a) {
+  typedef WaveTiles<FN, FM> P;
+  typedef TilesOut<FN, FM, OUT> O;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[O::LDS];
+  static_assert(O::LDS <= 160 * 1024, "LDS");
+  const int nt = (a.N + P::BN - 1) / P::BN, mt = (a.M + P::BM - 1) / P::BM, total = nt * mt;
+  const int per = (total + 7) / 8, end = min(total, (int)(blockIdx.x % 8 + 1) * per), stride = gridDim.x / 8;
+  int id = blockIdx.x % 8 * per + blockIdx.x / 8;
+  if (id >= end) return;
+  P p;
+  p.init(lds);
+  int n0, m0, share, sharers;
+  auto find = [&](int t) {          // groups of GROUP tiles of x by all of W's
+    auto div = [](int v, int by) { return __builtin_amdgcn_readfirstlane(v / by); };        // (by vector instructions: back to scalars)
+    const int turn = div(t, GROUP * nt), in = t - turn * GROUP * nt;
+    sharers = min(GROUP, mt - turn * GROUP);
+    const int tn = div(in, sharers);
+    share = in - tn * sharers;
+    m0 = (turn * GROUP + share) * P::BM, n0 = tn * P::BN;
+  };
+  auto rows_of_w = [&]() { return tile_buffer(a.w + (size_t)n0 * a.K, (unsigned)min(P::BN, a.N - n0) * (unsigned)a.K * 2u); };
+  auto begin = [&]() {
+    const int count = min(P::BM, a.M - m0);
+    const tile_uintx4 x = tile_buffer(a.x + (size_t)m0 * a.K, (unsigned)count * (unsigned)a.K * 2u);
+    p.begin(rows_of_w(), x, a.K, a.K * 2, [&](int i) { return i < count ? i * a.K * 2 : TILE_NO_ROW; });
+    p.touch_rows(share, sharers, a.K * 2);
+  };
+  find(id);
+  begin();
+  while (true) {
+    const int n = n0 + p.wn(), m = m0 + p.wm();
+    id += stride;
+    const bool more = id < end;
+    if (more) find(id);
+    p.next = rows_of_w();
+    if (!more) p.next[2] = 0;          // (nothing to touch)
+    tile_floatx4 acc[FN][FM];
+    p.run(lds, a.K, acc);
+    if (more) begin();
+    switch (a.act) {
+      case ACT_GELU_TANH: tiles_out<FN, FM, OUT, ACT_GELU_TANH>(p, a, lds, acc, m, n); break;
+      case ACT_SILU: tiles_out<FN, FM, OUT, ACT_SILU>(p, a, lds, acc, m, n); break;
+      default: tiles_out<FN, FM, OUT, OUT == OUT_PAIRS ? ACT_CLAMPED_SWISH : ACT_RELU_SQUARED>(p, a, lds, acc, m, n); break;
+    }
+    if (!more) break;
+  }
+}
+
 template <int BN, int BM, int WN, int WM, int PER_CU>
-__global__ __launch_bounds__(64 * (BN / WN) * (BM / WM), 2 * PER_CU) void pairs_kernel(PairsArgs a) {
+__global__ __launch_bounds__(64 * (BN / WN) * (BM / WM), 2 * PER_CU) void pairs_kernel(TilesArgs a) {
   typedef ProductTiles<BN, BM, WN, WM, false> P;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[P::LDS];
   int tn, tm;
@@ -66,61 +192,104 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM), 2 * PER_CU) void pairs_
   }
 }
 
-enum { TILE_256_256, TILE_320_192, TILE_192_128, TILE_128_128, TILE_KINDS };
+enum { TILE_256_256, TILE_320_192, TILE_192_128, TILE_128_128, TILE_384_160, TILE_256_192, TILE_192_256, TILE_256_128, TILE_KINDS };
 
-template <int BN, int BM, int WN, int WM, int PER_CU>
-static void launch_pairs(const PairsArgs& a, hipStream_t s) {
-  const int blocks = ((a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) + 7) / 8 * 8;
-  hipLaunchKernelGGL((pairs_kernel<BN, BM, WN, WM, PER_CU>), dim3(blocks), dim3(64 * (BN / WN) * (BM / WM)), 0, s, a);
-}
+// us of a launch with tiles of a kind: workgroups to a CU; a launch, a full round of the chip (and each 1,000 k-values of it), the
+// last round (and each 1,000 k-values, and those times the share of CUs that have a tile: fewer of them find memory faster, and
+// the chip's power goes further).  For two workgroups to a CU the last round is one of one to a CU at most, others count as full.
+static const struct { int bn, bm, per_cu; double launch, base, per_k, last_base, last_per_k, last_fill; } kinds[TILE_KINDS] = {
+    {256, 256, 1, 3.57, 4.82, 22.45, 5.39, 16.26, 4.72}, {320, 192, 1, 8.36, 4.73, 21.04, 0.00, 15.94, 4.44},
+    {192, 128, 2, 3.35, 5.58, 20.42, 3.56, 13.15, 0.00}, {128, 128, 2, 2.73, 3.67, 15.50, 2.81, 10.34, 0.00},
+    {384, 160, 1, 3.37, 4.38, 21.80, 5.06, 15.61, 5.41}, {256, 192, 1, 2.25, 3.52, 17.31, 4.71, 13.05, 4.33},
+    {192, 256, 1, 3.76, 3.73, 17.02, 3.83, 12.74, 3.63}, {256, 128, 1, 1.16, 1.98, 14.46, 4.24, 12.07, 3.06}};
 
-// us of a launch with tiles of a kind: full rounds of 256 CUs (with `per_cu` workgroups each) and the last one
 static double tiles_us(int kind, int M, int N, int K) {
-  static const struct { int bn, bm, per_cu; double base, per_k, one_base, one_per_k; } kinds[TILE_KINDS] = {
-      {256, 256, 1, 13.7, 0.0206, 0, 0}, {320, 192, 1, 13.0, 0.0190, 0, 0},
-      {192, 128, 2, 7.6, 0.0189, 5.6, 0.0112}, {128, 128, 2, 5.4, 0.0147, 3.7, 0.0089}};      // (one_: with one workgroup to a CU only)
   const auto& k = kinds[kind];
-  const long long tiles = (long long)((N + k.bn - 1) / k.bn) * ((M + k.bm - 1) / k.bm), round = 256 * k.per_cu, rest = tiles % round;
-  const double full = k.base + k.per_k * K;
-  return 2.0 + (double)(tiles / round) * full + (rest == 0 ? 0.0 : k.per_cu == 2 && rest <= 256 ? k.one_base + k.one_per_k * K : full);
+  const long long tiles = (long long)((N + k.bn - 1) / k.bn) * ((M + k.bm - 1) / k.bm), per = (tiles + 7) / 8, round = 32 * k.per_cu;      // (of an XCD)
+  const long long rest = per % round;
+  const double kk = K / 1000.0, full = k.base + k.per_k * kk;
+  const double last = rest == 0 ? 0.0 : k.per_cu == 2 && rest > 32 ? full : k.last_base + kk * (k.last_per_k + k.last_fill * (double)rest / 32);
+  return k.launch + (double)(per / round) * full + last;
 }
 
-static int choose_tile(int M, int N, int K) {
+static bool eight_waves(int kind) { return kind == TILE_192_128 || kind == TILE_128_128; }
+
+static int choose_tile(int M, int N, int K, int out) {
   int best = 0;
   for (int i = 1; i < TILE_KINDS; ++i)
-    if (tiles_us(i, M, N, K) < tiles_us(best, M, N, K)) best = i;
+    if (!(out == OUT_ACT && eight_waves(i)) && tiles_us(i, M, N, K) < tiles_us(best, M, N, K)) best = i;
   return best;
 }
 
-// us of the library's product and the activation's launch
+// us of the library's product and the activation's launch (its rounds of 256 x 256, 256 x 128 or 128 x 128, whichever least;
+// off by 10 % in the mean up to 1,536 k-values)
 static double library_us(int M, int N, int K) {
   auto rounds = [&](int bn, int bm) { return (double)(((long long)((N + bn - 1) / bn) * ((M + bm - 1) / bm) + 255) / 256); };
   const double product = K * fmin(0.0151 * rounds(256, 256), fmin(0.00984 * rounds(256, 128), 0.0059 * rounds(128, 128)));
   return 7.5 + 1.24e-6 * (double)M * (double)N + product;
 }
 
+// Shallow weights: whether ifx_gemm_tiles with OUT_PAIRS is the faster way by a fifth, by what tiles by eight waves take.  Of 2,300 sizes
+// of up to 1,536 k-values the rule takes 1,124: mean 1.41 x, worst 0.95 x, ten below 1; of other sizes, drawn at random, 768: mean 1.80 x,
+// worst 0.88 x (at launches of 6 us, where the launch that it saves weighs more than the 0.7 us).
 #define PAIRS_MAX_K 1536
-#define PAIRS_MIN_ROWS 129      // fewer rows were not measured (up to 128 are mostly the streaming products')
+#define TILES_MIN_ROWS 129      // fewer rows were not measured (up to 128 are mostly the streaming products')
 
-// whether ifx_gemm_pairs is the faster way for M rows (see above)
-extern "C" int ifx_gemm_pairs_wins(int M, int N, int K) {
-  return M >= PAIRS_MIN_ROWS && K <= PAIRS_MAX_K && library_us(M, N, K) >= 1.2 * tiles_us(choose_tile(M, N, K), M, N, K);
+static double eight_waves_us(int M, int N, int K) {
+  static const struct { int bn, bm, per_cu; double base, per_k, one_base, one_per_k; } tiles[4] = {
+      {256, 256, 1, 13.7, 0.0206, 0, 0}, {320, 192, 1, 13.0, 0.0190, 0, 0},
+      {192, 128, 2, 7.6, 0.0189, 5.6, 0.0112}, {128, 128, 2, 5.4, 0.0147, 3.7, 0.0089}};      // (one_: with one workgroup to a CU only)
+  double least = 1e30;
+  for (const auto& k : tiles) {
+    const long long n = (long long)((N + k.bn - 1) / k.bn) * ((M + k.bm - 1) / k.bm), round = 256 * k.per_cu, rest = n % round;
+    const double full = k.base + k.per_k * K;
+    least = fmin(least, 2.0 + (double)(n / round) * full + (rest == 0 ? 0.0 : k.per_cu == 2 && rest <= 256 ? k.one_base + k.one_per_k * K : full));
+  }
+  return least;
 }
 
-// x, w: on 16 bytes.  tile: one of the kinds above, or -1 for the one that choose_tile takes
-extern "C" int ifx_gemm_pairs(const void* x, const void* w, void* out, int M, int N, int K, int act, float limit, int tile, void* stream) {
-  IFX_REQUIRE(M >= 0 && N > 0 && N % 4 == 0 && K > 0 && K % 8 == 0 && K <= 1 << 20, "gemm_pairs: N=%d must be a multiple of 4, K=%d of 8", N, K);
-  IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f), "gated activation: unknown kind %d (limit %g)", act, (double)limit);
-  IFX_REQUIRE(((size_t)x | (size_t)w) % 16 == 0, "gemm_pairs: x and the weight must lie on 16 bytes");
+extern "C" int ifx_gemm_pairs_wins(int M, int N, int K) {
+  return M >= TILES_MIN_ROWS && K <= PAIRS_MAX_K && library_us(M, N, K) >= 1.2 * eight_waves_us(M, N, K);
+}
+
+template <int FN, int FM>
+static void launch_waves(const TilesArgs& a, int out, hipStream_t s) {
+  typedef WaveTiles<FN, FM> P;
+  const int tiles = ((a.N + P::BN - 1) / P::BN) * ((a.M + P::BM - 1) / P::BM), blocks = tiles < 256 ? (tiles + 7) / 8 * 8 : 256;
+  if (out == OUT_PAIRS) hipLaunchKernelGGL((tiles_kernel<FN, FM, OUT_PAIRS>), dim3(blocks), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((tiles_kernel<FN, FM, OUT_ACT>), dim3(blocks), dim3(256), 0, s, a);
+}
+
+template <int BN, int BM, int WN, int WM, int PER_CU>
+static void launch_pairs(const TilesArgs& a, hipStream_t s) {
+  const int blocks = ((a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) + 7) / 8 * 8;
+  hipLaunchKernelGGL((pairs_kernel<BN, BM, WN, WM, PER_CU>), dim3(blocks), dim3(64 * (BN / WN) * (BM / WM)), 0, s, a);
+}
+
+// x, w, with OUT_ACT the result: on 16 bytes.  tile: one of the kinds above, or -1 for the one that choose_tile takes
+extern "C" int ifx_gemm_tiles(const void* x, const void* w, void* result, int M, int N, int K, int out, int act, float limit, int tile, void* stream) {
+  IFX_REQUIRE(out == OUT_PAIRS || out == OUT_ACT, "gemm_tiles: result %d", out);
+  IFX_REQUIRE(M >= 0 && N > 0 && N % (out == OUT_PAIRS ? 4 : 2) == 0 && K > 0 && K % 8 == 0 && K <= 1 << 20 && N <= 1 << 22,
+              "gemm_tiles: N=%d must be a multiple of %d, K=%d of 8", N, out == OUT_PAIRS ? 4 : 2, K);
+  if (out == OUT_PAIRS)
+    IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f), "gated activation: unknown kind %d (limit %g)", act, (double)limit);
+  else
+    IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || act == ACT_RELU_SQUARED, "activation: unknown kind %d", act);
+  IFX_REQUIRE(((size_t)x | (size_t)w | (size_t)result) % 16 == 0, "gemm_tiles: x, the weight and the result must lie on 16 bytes");
   if (M == 0) return 0;
-  const PairsArgs a{(const bf16_t*)x, (const bf16_t*)w, (bf16_t*)out, M, N, K, act, limit};
+  const TilesArgs a{(const bf16_t*)x, (const bf16_t*)w, (bf16_t*)result, M, N, K, act, limit};
   hipStream_t s = (hipStream_t)stream;
-  switch (tile < 0 ? choose_tile(M, N, K) : tile) {
-    case TILE_256_256: launch_pairs<256, 256, 128, 64, 1>(a, s); break;
-    case TILE_320_192: launch_pairs<320, 192, 80, 96, 1>(a, s); break;
+  const int kind = tile < 0 ? choose_tile(M, N, K, out) : tile;
+  IFX_REQUIRE(kind < TILE_KINDS && !(out == OUT_ACT && eight_waves(kind)), "gemm_tiles: tile %d", tile);
+  switch (kind) {
+    case TILE_256_256: launch_waves<8, 8>(a, out, s); break;
+    case TILE_320_192: launch_waves<10, 6>(a, out, s); break;
     case TILE_192_128: launch_pairs<192, 128, 48, 64, 2>(a, s); break;
     case TILE_128_128: launch_pairs<128, 128, 32, 64, 2>(a, s); break;
-    default: IFX_FAIL("gemm_pairs: tile %d", tile);
+    case TILE_384_160: launch_waves<12, 5>(a, out, s); break;
+    case TILE_256_192: launch_waves<8, 6>(a, out, s); break;
+    case TILE_192_256: launch_waves<6, 8>(a, out, s); break;
+    case TILE_256_128: launch_waves<8, 4>(a, out, s); break;
   }
   IFX_LAUNCH_CHECK();
 }

@@ -29,6 +29,7 @@ ROPE_NONE, ROPE_SPLIT_HALF, ROPE_CONSECUTIVE = 0, 1, 2
 ACT_SILU, ACT_GELU_TANH = 0, 1          # gated activations of a feed-forward: act(gate) * up
 ACT_CLAMPED_SWISH = 2                   # ... and min(gate, L) sigmoid(1.702 min(gate, L)) (clamp(up, -L, L) + 1), which takes its limit L
 ACT_RELU_SQUARED = 3                    # max(x, 0)^2, for a feed-forward without a gate
+PLAIN_ACTS = (ACT_SILU, ACT_GELU_TANH, ACT_RELU_SQUARED)
 _PLAIN_EPILOGUE = {ACT_RELU_SQUARED: 4, ACT_GELU_TANH: 5}     # the activations without a gate that the product for few rows has as an epilogue
 _GATED_EPILOGUE = {ACT_SILU: 1, ACT_GELU_TANH: 3}    # ... as the epilogue number of the streaming products
 
@@ -1402,11 +1403,30 @@ def _pairs_tiles_win(M: int, N: int, K: int) -> bool:
 
 
 def pairs_tiles_take(M: int, N: int, K: int) -> bool:
-    """Whether the product for many rows with the activation as its epilogue takes gate/up pairs [N, K] in bfloat16: where it is
-    estimated to be the faster way by a fifth or more, from the rounds of tiles that either way needs (ifx_gemm_pairs_wins in
-    csrc/gemm_tiles.hip, with the measurements).  Where the caller has the library time its kernels
-    (``enable_library_gemm_tuning``), its choice is the faster one."""
+    """Whether the product for many rows with the activation as its epilogue takes gate/up pairs [N, K] of shallow weights (up to 1,536
+    k-values) in bfloat16 whatever their number of tiles: where tiles by eight waves are estimated to be the faster way by a fifth or
+    more, from the rounds that either way needs (ifx_gemm_pairs_wins in csrc/gemm_tiles.hip).  Where the caller has the library
+    time its kernels (``enable_library_gemm_tuning``), its choice is the faster one at such sizes; larger ones: ``many_tiles_take``."""
     return N % 4 == 0 and K % 8 == 0 and _pairs_tiles_win(M, N, K) and not torch.cuda.tunable.is_enabled()
+
+
+MANY_TILES_MIN_ROWS = 129          # (up to 128 rows are mostly the streaming products')
+# k-values up to which ...: the least M N / 65,536 (tiles of 256 x 256) from which ..., of gate/up pairs and of products without a gate
+MANY_TILES = ((800, 16, 32), (1536, 32, 48), (2560, 96, 96), (4096, 128, 128))
+
+
+def many_tiles_take(M: int, N: int, K: int, gated: bool = True) -> bool:
+    """Whether the product for many rows with the activation as its epilogue takes a bfloat16 weight [N, K] because its tiles fill the
+    chip.  600 sizes drawn over 129 to 8,192 rows, 2,048 to 61,000 weight rows, 64 to 8,192 k-values, the library's product and
+    the activation's launch in the time of this one, geometric mean and worst:
+        K      up to 800: 16 to 64 tiles 1.46 x and 1.05, more 1.99 and 1.35     800 to 1,536: 32 to 64 1.15 and 1.03, more 1.40 and 1.10
+        K 1,536 to 2,560: 64 to 128 1.05 and 0.96, more 1.21 and 1.06          2,560 to 4,096: 32 to 64 0.85, more 1.20 and 1.00
+        K 4,096 to 8,192: 128 to 256 1.06 and 0.76, more 1.11 and 0.94 (there the library keeps the product), and 0.4 to 0.9 below these lines
+    (without a gate, whose activation's launch the library pays less for: 0.97 to 1.31 below 64 tiles up to 800, 1.02 there up to 1,536).
+    Where the library has timed its kernels the lines are the same (42 sizes beyond them: 1.33 and 0.97)."""
+    if M < MANY_TILES_MIN_ROWS or K < 64 or K % 8 or N % (16 if gated else 8):
+        return False
+    return any(K <= deepest and M * N >= 65536 * (pairs if gated else plain) for deepest, pairs, plain in MANY_TILES)
 
 
 def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, tile: int = -1) -> torch.Tensor:
@@ -1416,15 +1436,30 @@ def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limi
     N, K = pairs.shape
     _check(x, "x", (None, K), torch.bfloat16)
     out = torch.empty((x.shape[0], N // 2), dtype=torch.bfloat16, device=x.device)
-    _call(load_module("gemm_tiles"), "ifx_gemm_pairs", (P, P, P, I, I, I, I, F, I, P), x.data_ptr(), pairs.data_ptr(), out.data_ptr(),
-          x.shape[0], N, K, int(act), float(limit), int(tile), _stream())
+    _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x.data_ptr(), pairs.data_ptr(), out.data_ptr(),
+          x.shape[0], N, K, 0, int(act), float(limit), int(tile), _stream())
     return out
+
+
+def act_tiles(x: torch.Tensor, weight: torch.Tensor, act: int, tile: int = -1) -> torch.Tensor:
+    """``linear_act`` of many rows in bfloat16 as one launch ([N, K] ``weight``, N even and K a multiple of 8, both on 16 bytes);
+    ``tile`` as for ``swiglu_tiles``, one by four waves."""
+    _check(weight, "weight", (None, None), torch.bfloat16)
+    N, K = weight.shape
+    _check(x, "x", (None, K), torch.bfloat16)
+    out = torch.empty((x.shape[0], N), dtype=torch.bfloat16, device=x.device)
+    _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x.data_ptr(), weight.data_ptr(), out.data_ptr(),
+          x.shape[0], N, K, 1, int(act), 0.0, int(tile), _stream())
+    return out
+
+
+_TILES_ARGS = (P, P, P, I, I, I, I, I, F, I, P)
 
 
 def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: float = 0.0) -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) (``act``: ACT_SILU, ACT_GELU_TANH, or ACT_CLAMPED_SWISH with its ``limit``) where ``weight_pairs``
     [2I, K] (a tensor or a ``LinearWeight``) alternates the rows of Wg and Wu; ``x`` as for ``linear``.  For few rows (not with ACT_CLAMPED_SWISH) and
-    for many (``pairs_tiles_take``) the activation is the product's epilogue; otherwise a second kernel applies it."""
+    for many (``pairs_tiles_take``, ``many_tiles_take``) the activation is the product's epilogue; otherwise a second kernel applies it."""
     M, K = x.shape
     if isinstance(x, ScaledRows) and not takes_scaled_rows(M, weight_pairs):
         raise KernelError(f"linear_swiglu: scaled rows are not taken for {M} rows and this weight")
@@ -1434,7 +1469,7 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
         raise KernelError("linear_swiglu: a tile order is not supported for gate/up pairs")
     columns = columns_on_16_bytes(x)          # (as for ``linear``)
     if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and K == rows.shape[1] \
-            and pairs_tiles_take(M, rows.shape[0], K):
+            and (pairs_tiles_take(M, rows.shape[0], K) or many_tiles_take(M, rows.shape[0], K)):
         whole = x.contiguous() if columns else x
         if whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
             return swiglu_tiles(whole, rows, act, limit)
@@ -2120,12 +2155,19 @@ def hyper_step(src: torch.Tensor, n_streams: int, y=None, mix: Optional[torch.Te
 
 def linear_act(x, weight, act: int) -> torch.Tensor:
     """act(x W^T) for a feed-forward without a gate (``act``: ACT_SILU, ACT_GELU_TANH or ACT_RELU_SQUARED, formed in float on the product's
-    output; in steps of few rows the square of relu and gelu are the product's epilogue: 16 rows of 8,448 x 2,048 12 us and a launch of 5 less);
+    output; in steps of few rows the square of relu and gelu are the product's epilogue: 16 rows of 8,448 x 2,048 12 us and a launch of 5 less,
+    in those of many rows any of them: ``many_tiles_take``);
     ``x`` as for ``linear``."""
     if act in _PLAIN_EPILOGUE and isinstance(weight, LinearWeight) and weight.rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 \
             and weight.order is None and _small_m_kernel(x.shape[0], *weight.rows.shape, weight.tiled is not None) == "skinny" \
             and (not isinstance(x, ScaledRows) or takes_scaled_rows(x.shape[0], weight)):
         return skinny_gemm(x, weight.rows, tiled=weight.tiled, tile_rows=weight.tile_rows, plain_act=act)
+    rows = weight.rows if isinstance(weight, LinearWeight) else weight
+    if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and rows.dim() == 2 and x.dim() == 2 \
+            and x.shape[1] == rows.shape[1] and act in PLAIN_ACTS and many_tiles_take(x.shape[0], *rows.shape, gated=False):
+        whole = x.contiguous() if columns_on_16_bytes(x) else x          # (as for ``linear``)
+        if whole.is_contiguous() and whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
+            return act_tiles(whole, rows, act)
     return activation(linear(x, weight, keep_slices=True), act)
 
 

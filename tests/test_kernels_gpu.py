@@ -838,6 +838,47 @@ def test_many_row_pairs_go_to_the_library_where_it_times_its_kernels(monkeypatch
     assert ((ours - theirs).abs() <= 2.0 ** -6 * ours.abs() + 2.0 ** -6).all()
 
 
+@pytest.mark.parametrize("tile", [0, 1, 4, 5, 6, 7, -1])
+@pytest.mark.parametrize("M,N,K,act", [(1, 16, 8, "silu"), (2, 34, 64, "relu2"), (193, 388, 72, "gelu"), (257, 520, 136, "silu"),
+                                       (650, 776, 192, "gelu"), (129, 4110, 320, "relu2")])
+def test_product_tiles_with_an_activation(tile, M, N, K, act):
+    """The tiles by four waves without a gate: edges of every tile, one step of 64 k-values, two, an odd number and a last one that is not
+    full, rows on 16 bytes and not, more tiles than workgroups: as test_swiglu_tiles, with the slope of relu squared (twice the value)."""
+    g = gen(2470 + M)
+    x = torch.randn(M, K, generator=g).to(BF16)
+    w = (2.0 * torch.randn(N, K, generator=g) / K ** 0.5).to(BF16)
+    z = x.double() @ w.double().t()
+    kind = {"silu": ops.ACT_SILU, "gelu": ops.ACT_GELU_TANH, "relu2": ops.ACT_RELU_SQUARED}[act]
+    want = {"silu": torch.nn.functional.silu(z), "gelu": torch.nn.functional.gelu(z, approximate="tanh"), "relu2": z.clamp(min=0) ** 2}[act]
+    got = ops.act_tiles(x.to(DEV), w.to(DEV), kind, tile).cpu().double()
+    sums = 1.2 * K ** 0.5 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) * (2.0 * z.abs() + 1.0)
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + sums + 1e-6).all()
+
+
+@pytest.mark.parametrize("tile", [4, 5, 6, 7])
+@pytest.mark.parametrize("M,N,K,act", [(1, 4, 8, "silu"), (129, 132, 64, "silu"), (321, 776, 136, "gelu"), (257, 516, 200, "clamped"), (700, 12304, 192, "silu")])
+def test_swiglu_tiles_by_four_waves(tile, M, N, K, act):
+    test_swiglu_tiles(tile, M, N, K, act)
+
+
+def test_many_row_products_go_where_their_tiles_fill_the_chip():
+    for M, N, K in ((600, 22016, 2048), (2048, 37888, 3584), (129, 8192, 64), (4096, 8448, 2048)):
+        assert ops.many_tiles_take(M, N, K) and ops.many_tiles_take(4 * M, N, K, gated=False), (M, N, K)
+    for M, N, K in ((128, 37888, 512), (2048, 37888, 4104), (200, 22016, 2048), (600, 5632, 2048), (2048, 8200, 516), (2048, 8196, 512)):
+        assert not ops.many_tiles_take(M, N, K) and not ops.many_tiles_take(M, N, K, gated=False), (M, N, K)
+    g = gen(2480)
+    x, w = torch.randn(600, 80, generator=g).to(BF16).to(DEV), torch.randn(4096, 72, generator=g).to(BF16).to(DEV)
+    assert ops.many_tiles_take(600, 4096, 72, gated=False) and ops.columns_on_16_bytes(x[:, :72])
+    want = ops.activation(ops.linear(x[:, :72].contiguous(), w), ops.ACT_GELU_TANH).double()
+    for rows in (x[:, :72], x[:, :72].contiguous()):
+        got = ops.linear_act(rows, w, ops.ACT_GELU_TANH).double()          # (the product rounded in between there: 2^-9 of it and of the result)
+        assert ((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -6).all()
+    with pytest.raises(ops.KernelError):
+        ops.linear_act(x[:, 1:73], w, ops.ACT_GELU_TANH)                   # (not on 16 bytes: refused as by linear)
+    with pytest.raises(ops.KernelError):
+        ops.linear_act(x[:, :72], w, ops.ACT_CLAMPED_SWISH)
+
+
 # ---- sampling -------------------------------------------------------------------------------
 def test_argmax_lowest_index_wins_ties():
     l = torch.zeros(3, 1500)
