@@ -64,13 +64,13 @@ __device__ __forceinline__ float* row_sum_shares() {
   __shared__ __attribute__((aligned(16))) float shares[16][16];
   return &shares[0][0];
 }
-__device__ __forceinline__ void leave_row_sums(const RowScale& s, const RowSumsEarly& early, int wave, int lane) {
-  const rs_floatx4 t = row_sums_of_wave(row_sums_of_thread(s, threadIdx.x, blockDim.x, early));
+__device__ __forceinline__ void leave_row_sums(const RowScale& s, const RowSumsEarly& early, int wave, int lane, int waves) {
+  const rs_floatx4 t = row_sums_of_wave(row_sums_of_thread(s, threadIdx.x, waves * WAVE, early));
   if (lane < 4) *(rs_floatx4*)(row_sum_shares() + 16 * wave + 4 * lane) = t;
 }
-__device__ __forceinline__ float gathered_row_factor(const RowScale& s, int col) {
+__device__ __forceinline__ float gathered_row_factor(const RowScale& s, int col, int waves) {
   float sum = 0.f;
-  for (int w = 0; w < (int)blockDim.x / WAVE; ++w) sum += row_sum_shares()[16 * w + col];
+  for (int w = 0; w < waves; ++w) sum += row_sum_shares()[16 * w + col];
   return rsqrtf(sum / s.width + s.eps);
 }
 
@@ -78,22 +78,48 @@ __device__ __forceinline__ float gathered_row_factor(const RowScale& s, int col)
 // the workgroup's waves and added through LDS in wave order.  Returns true in the wave that holds the
 // sums (wave 0); the others are done.
 // ``before_meeting(wave)`` is called once in every wave, after its last products are started and before the workgroup's barrier.
-template <int MT, int NT, int U, bool TILED, typename F>
-__device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N,
+// EIGHT (one tile of 8 rows, up to 8 rows of x): a product of 16 x 16 takes two k-tiles at once, the second one's 8 rows of W
+// standing below the first one's and its 8 rows of x beside the first one's; of the four quarters of the sums two are those of the
+// tile and are added up, the other two (a k-tile's W with the other's x) are left.  A load then has work for all 64 lanes, where
+// one k-tile's 8 rows have it for 32, and a wave asks for its share of K in half the loads, of W and of x.
+// HALVES (tiles of 16 rows): rows first_row ... + 7 of W tile first_tile and, below them, those of first_tile + 1.
+template <int MT, int NT, int U, bool TILED, bool EIGHT, bool HALVES = false, typename F>
+__device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int n_tiles,
                                                   int K, int k_tiles, int first_tile, floatx4 (&acc)[NT][MT], float* red,
-                                                  int tile_rows, int ldx, F before_meeting) {
-  const int wid = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x % WAVE;
+                                                  int tile_rows, int ldx, int nw, F before_meeting, int first_row = 0) {
+  const int wid = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int col = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  const bf16_t* wrow[NT];  // rows (tiles) past N are read again, never stored
+  if constexpr (EIGHT) {
+    const int sub = col >> 3, row = col & 7;
+    const bf16_t* wt = W + ((size_t)first_tile * k_tiles * 32 + (4 * sub + g) * 8 + row) * 8;
+    const bool held = row < M;
+    const bf16_t* xr = x + (size_t)(held ? row : 0) * ldx + 32 * sub + 8 * g;
+    const int nkb = (K + 63) / 64, k_left = K - 32 * sub - 8 * g;
+    for (int kb0 = wid * U; kb0 < nkb; kb0 += nw * U) {
+      bf16x8 wa[U], xa[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int kb = kb0 + u;
+        wa[u] = kb < nkb ? __builtin_nontemporal_load((const bf16x8*)(wt + (size_t)kb * 512)) : zero8();
+        xa[u] = kb < nkb && held && kb * 64 < k_left ? *(const bf16x8*)(xr + kb * 64) : zero8();
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u], xa[u], acc[0][0], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[0][0][r] += __shfl_xor(acc[0][0][r], 40);        // (lanes of columns and rows of less than 8 hold the tile's)
+  } else {
+  size_t wrow[NT];         // where the lane's row begins in W: tiles past the last are read again, never stored (TILED: whole ones; else rows past N)
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
-    wrow[nt] = TILED ? W + ((size_t)min(first_tile + nt, (N - 1) / tile_rows) * k_tiles * 4 * tile_rows + tile_rows * g + col) * 8
-                     : W + (size_t)min(16 * (first_tile + nt) + col, N - 1) * K;
+    wrow[nt] = HALVES ? ((size_t)(first_tile + (col >> 3)) * k_tiles * 64 + 16 * g + first_row + (col & 7)) * 8
+               : TILED ? ((size_t)min(first_tile + nt, n_tiles - 1) * k_tiles * 4 * tile_rows + tile_rows * g + col) * 8
+                     : (size_t)min(16 * (first_tile + nt) + col, N - 1) * K;
   const bool row_held = !TILED || col < tile_rows;   // a tile of the copy holds tile_rows rows: the other lanes' rows are zeros
   const bf16_t* xrow[MT];
   bool xok[MT];
@@ -103,7 +129,10 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
     xrow[mt] = x + (size_t)(xok[mt] ? 16 * mt + col : 0) * ldx;
   }
 
-  const int nkb = (K + 63) / 64;
+  const int nkb = (K + 63) / 64, k_tile = 32 * tile_rows;     // (elements of the copy to a k-tile)
+  if (TILED)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) wrow[nt] += wid * U * 2 * k_tile;
   for (int kb0 = wid * U; kb0 < nkb; kb0 += nw * U) {
     bf16x8 wa[U][NT][2], xa[U][MT][2];
 #pragma unroll
@@ -112,13 +141,13 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
       for (int h = 0; h < 2; ++h) {
         // the lane's 8 k-values of step h of block kb0 + u, and where its piece of W lies
         const int k = TILED ? (kb0 + u) * 64 + 32 * h + 8 * g : (kb0 + u) * 64 + 16 * g + 8 * h;
-        const size_t w_off = TILED ? (size_t)(2 * (kb0 + u) + h) * 4 * tile_rows * 8 : (size_t)k;
+        const int w_off = TILED ? (2 * u + h) * k_tile : k;
         const bool blk = kb0 + u < nkb && row_held, kok = kb0 + u < nkb && k < K;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           // Tiles are read once, in whole lines: a streaming load keeps them from pushing x out of the L2.
           // (Rows are read in half lines by two loads; there the hint costs more than it gives.)
-          const bf16x8* wp = (const bf16x8*)(wrow[nt] + w_off);
+          const bf16x8* wp = (const bf16x8*)(W + wrow[nt] + w_off);
           wa[u][nt][h] = TILED ? (blk ? __builtin_nontemporal_load(wp) : zero8()) : (kok ? *wp : zero8());
         }
 #pragma unroll
@@ -134,6 +163,10 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
             acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][nt][h], xa[u][mt][h], acc[nt][mt], 0, 0, 0);
+    if (TILED)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) wrow[nt] += nw * U * 2 * k_tile;
+  }
   }
 
   before_meeting(wid);
@@ -147,15 +180,26 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
     }
     __syncthreads();
     if (wid > 0) return false;
-    for (int w = 1; w < nw; ++w)
+    constexpr int AT_ONCE = NT * MT == 1 ? 4 : 1;        // waves' shares asked for before the first is added (the order is the waves')
+    for (int w0 = 1; w0 < nw; w0 += AT_ONCE) {
+      floatx4 o[AT_ONCE][NT][MT];
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+      for (int i = 0; i < AT_ONCE; ++i)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const floatx4 o = *(const floatx4*)(red + ((size_t)((w - 1) * NT * MT + nt * MT + mt) * WAVE + lane) * 4);
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[nt][mt][r] += o[r];
-        }
+          for (int mt = 0; mt < MT; ++mt)
+            o[i][nt][mt] = *(const floatx4*)(red + ((size_t)((min(w0 + i, nw - 1) - 1) * NT * MT + nt * MT + mt) * WAVE + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i)
+        if (w0 + i < nw)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[nt][mt][r] += o[i][nt][mt][r];
+    }
   }
   return true;
 }
@@ -169,27 +213,34 @@ typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 typedef __attribute__((__vector_size__(2 * sizeof(float)))) float floatx2;
 
-template <int MT, int NT, int U, typename TO, int EPI, bool TILED>
-__global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, TO* __restrict__ out,
-                                   int M, int N, int K, int k_tiles, const int* __restrict__ order, RowScale scale,
-                                   StreamOut so, int tile_rows, XBlocks xb) {
+// (Four waves to a SIMD at most: where the registers allow a fifth, workgroups of eight waves over tall weights lose a tenth, 8 rows of
+// 37,888 x 3,584 47.0 us instead of 42.3, and nothing measured gains.)
+template <int MT, int NT, int U, typename TO, int EPI, bool TILED, bool EIGHT>
+__global__ __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, int tile_rows, int n_tiles, int waves,
+                                   int block_tiles, int n_blocks, const float* __restrict__ pieces, int n_pieces, TO* __restrict__ out,
+                                   const int* __restrict__ order, float scale_width, float scale_eps, StreamOut so) {
+  const RowScale scale{pieces, n_pieces, scale_width, scale_eps};
+  const XBlocks xb{block_tiles, n_blocks};
+  const int k_tiles = (K + 63) / 64 * 2;
   extern __shared__ float red[];  // [(waves - 1)][NT * MT][64 lanes][4]
   const int lane = threadIdx.x % WAVE, col = lane & 15, g = lane >> 4;
-  const int first_tile = blockIdx.x * NT, n_tiles = (N + tile_rows - 1) / tile_rows;
+  const int first_tile = blockIdx.x * NT;
   const bool first_wave = threadIdx.x < WAVE;
   float rs = 1.f;
   // The rows' factors: every thread of a workgroup of several waves asks for its share of the sums of squares ahead of the
   // weights and adds it up after them, so that they cost no trip to the L2 of their own (computed by the first wave before its
   // first weights they cost 1 us a product).
-  const bool shared_sums = MT == 1 && scale.pieces && blockDim.x > WAVE;
+  const bool shared_sums = MT == 1 && scale.pieces && waves > 1;
   RowSumsEarly early;
-  if (shared_sums) row_sums_ask(scale, threadIdx.x, blockDim.x, early);
+  if (shared_sums) row_sums_ask(scale, threadIdx.x, waves * WAVE, early);
   else if (MT == 1 && scale.pieces) rs = row_factor(scale, lane);
   // The lane's four sums of a tile are rows 4 g ... 4 g + 3 of it, handled as two pairs: tile_rows is even, so a
   // pair is held or not as a whole, and a pair's first column is even.
   // EPI 2: what the epilogue reads is asked for before the stream of weights, not after it
+  // (the norm's weight as it lies in memory, widened where it is used: a conversion here would wait for its load ahead of the weights)
+  union Two { floatx2 f; bf16x2 h; };
   floatx2 was[NT][2];
-  floatx2 nw[NT][2];
+  Two nw[NT][2];
   if (EPI == 2 && first_wave) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -198,20 +249,17 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* _
         const int n = tile_rows * (first_tile + nt) + 4 * g + 2 * q;
         const bool ok = 4 * g + 2 * q < tile_rows && n < N && col < M;
         was[nt][q] = ok ? *(const floatx2*)(so.stream + (size_t)col * N + n) : floatx2{0.f, 0.f};
-        nw[nt][q] = floatx2{0.f, 0.f};
-        if (ok && so.norm_f32) nw[nt][q] = *(const floatx2*)((const float*)so.norm_w + n);
-        else if (ok) {
-          const bf16x2 w2 = *(const bf16x2*)((const bf16_t*)so.norm_w + n);
-          nw[nt][q] = floatx2{(float)w2[0], (float)w2[1]};
-        }
+        nw[nt][q].f = floatx2{0.f, 0.f};
+        if (ok && so.norm_f32) nw[nt][q].f = *(const floatx2*)((const float*)so.norm_w + n);
+        else if (ok) nw[nt][q].h = *(const bf16x2*)((const bf16_t*)so.norm_w + n);
       }
   }
   floatx4 acc[NT][MT];
   if (xb.tiles > 0) x += (size_t)min(first_tile / xb.tiles, xb.n - 1) * M * K;
-  if (!skinny_accumulate<MT, NT, U, TILED>(x, W, M, N, K, k_tiles, first_tile, acc, red, tile_rows, xb.tiles == 0 && xb.n > 0 ? xb.n : K, [&](int wave) {
-        if (shared_sums) leave_row_sums(scale, early, wave, lane);
+  if (!skinny_accumulate<MT, NT, U, TILED, EIGHT>(x, W, M, N, n_tiles, K, k_tiles, first_tile, acc, red, tile_rows, xb.tiles == 0 && xb.n > 0 ? xb.n : K, waves, [&](int wave) {
+        if (shared_sums) leave_row_sums(scale, early, wave, lane, waves);
       })) return;
-  if (shared_sums) rs = gathered_row_factor(scale, col);
+  if (shared_sums) rs = gathered_row_factor(scale, col, waves);
   // acc[nt][mt][r] = out[m = 16 mt + col][n = tile_rows (row tile of the weight) + 4 g + r], for 4 g + r < tile_rows
   if (EPI == 2) {
 #pragma unroll
@@ -227,7 +275,7 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* _
 #pragma unroll
           for (int r = 0; r < 2; ++r) {
             v[r] = was[nt][q][r] + acc[nt][0][2 * q + r] * rs * so.mult;
-            y[r] = (__bf16)(v[r] * nw[nt][q][r]);
+            y[r] = (__bf16)(v[r] * (so.norm_f32 ? nw[nt][q].f[r] : (float)nw[nt][q].h[r]));
             sq += v[r] * v[r];
           }
           *(floatx2*)(so.stream + (size_t)col * N + n) = v;
@@ -281,23 +329,27 @@ struct QkvArgs {
   bf16_t* q_out;          // [M, nH * d]
   bf16_t* k_cache;        // [pages, nKV, P, d]
   bf16_t* v_cache;        // [pages, nKV, d, P]
-  int nH, nKV, d, P;
+  int P;
 };
 
-template <int U>
-__global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, int k_tiles,
-                                QkvArgs a, RowScale scale) {
+// HALVES: a workgroup takes 8 of the 16 rotation pairs of two tiles; lanes of g < 2 hold first elements, the others second ones.
+template <int U, bool HALVES>
+__global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, int waves, int nH, int nKV, int d,
+                                const float* __restrict__ pieces, int n_pieces, float scale_width, float scale_eps, QkvArgs a) {
+  const RowScale scale{pieces, n_pieces, scale_width, scale_eps};
+  const int k_tiles = (K + 63) / 64 * 2;
   extern __shared__ float red[];
   const int lane = threadIdx.x % WAVE, col = lane & 15, g = lane >> 4;
   float rs = 1.f;
-  const bool shared_sums = scale.pieces && blockDim.x > WAVE;        // (as in skinny_gemm_kernel)
+  const bool shared_sums = scale.pieces && waves > 1;        // (as in skinny_gemm_kernel)
   RowSumsEarly early;
-  if (shared_sums) row_sums_ask(scale, threadIdx.x, blockDim.x, early);
+  if (shared_sums) row_sums_ask(scale, threadIdx.x, waves * WAVE, early);
   else if (scale.pieces) rs = row_factor(scale, lane);
   // What the epilogue reads is asked for before the stream of weights, not after it (the first wave holds the sums).
-  const int m = col, d = a.d, half = d / 2, per_head = d / 32;
-  const int head = blockIdx.x / per_head, i0 = 16 * (blockIdx.x % per_head) + 4 * g;   // the lane's pairs: i0 + r and i0 + r + half
-  const bool is_q = head < a.nH, is_v = head >= a.nH + a.nKV;
+  const int m = col, half = d / 2, per_head = d / 32;
+  const int pair_tile = HALVES ? blockIdx.x / 2 : blockIdx.x, first_row = HALVES ? blockIdx.x % 2 * 8 : 0;
+  const int head = pair_tile / per_head, i0 = 16 * (pair_tile % per_head) + first_row + (HALVES ? 4 * (g & 1) : 4 * g);   // the lane's pairs: i0 + r and i0 + r + half
+  const bool is_q = head < nH, is_v = head >= nH + nKV;
   // (the bias as it lies in memory, widened where it is used: a conversion here would wait for its load ahead of the weights)
   union Bias { floatx4 f; bf16x4 h; };
   Bias b0, b1;
@@ -319,18 +371,20 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
     }
     if (!is_q && a.slots) slot = a.slots[m];
   }
-  floatx4 acc[2][1];
-  if (!skinny_accumulate<1, 2, U, true>(x, W, M, N, K, k_tiles, 2 * blockIdx.x, acc, red, 16, K, [&](int wave) {
-        if (shared_sums) leave_row_sums(scale, early, wave, lane);
-      })) return;
-  if (shared_sums) rs = gathered_row_factor(scale, col);
-  if (m >= M) return;
+  constexpr int NT = HALVES ? 1 : 2;
+  floatx4 acc[NT][1];
+  if (!skinny_accumulate<1, NT, U, true, false, HALVES>(x, W, M, N, N / 16, K, k_tiles, 2 * pair_tile, acc, red, 16, K, waves, [&](int wave) {
+        if (shared_sums) leave_row_sums(scale, early, wave, lane, waves);
+      }, first_row)) return;
+  if (shared_sums) rs = gathered_row_factor(scale, col, waves);
   float x0[4], x1[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
+    const float second = HALVES ? __shfl_xor(acc[0][0][r], 32) : acc[NT - 1][0][r];
     x0[r] = acc[0][0][r] * rs + (a.bias_dtype == DT_F32 ? b0.f[r] : (float)b0.h[r]);
-    x1[r] = acc[1][0][r] * rs + (a.bias_dtype == DT_F32 ? b1.f[r] : (float)b1.h[r]);
+    x1[r] = second * rs + (a.bias_dtype == DT_F32 ? b1.f[r] : (float)b1.h[r]);
   }
+  if (m >= M || (HALVES && g >= 2)) return;
   if (!is_v) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -343,7 +397,7 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
 #pragma unroll
   for (int r = 0; r < 4; ++r) { lo[r] = (__bf16)x0[r]; hi[r] = (__bf16)x1[r]; }
   if (is_q) {
-    bf16_t* dst = a.q_out + ((size_t)m * a.nH + head) * d + i0;
+    bf16_t* dst = a.q_out + ((size_t)m * nH + head) * d + i0;
     *(bf16x4*)dst = lo;
     *(bf16x4*)(dst + half) = hi;
     return;
@@ -351,11 +405,11 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
   if (slot < 0) return;
   const int page = slot / a.P, off = slot % a.P;
   if (!is_v) {
-    bf16_t* dst = a.k_cache + (((size_t)page * a.nKV + (head - a.nH)) * a.P + off) * d + i0;
+    bf16_t* dst = a.k_cache + (((size_t)page * nKV + (head - nH)) * a.P + off) * d + i0;
     *(bf16x4*)dst = lo;
     *(bf16x4*)(dst + half) = hi;
   } else {
-    bf16_t* dst = a.v_cache + (((size_t)page * a.nKV + (head - a.nH - a.nKV)) * d + i0) * a.P + off;
+    bf16_t* dst = a.v_cache + (((size_t)page * nKV + (head - nH - nKV)) * d + i0) * a.P + off;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       dst[(size_t)r * a.P] = lo[r];
@@ -364,15 +418,15 @@ __global__ void qkv_rope_kernel(const bf16_t* __restrict__ x, const bf16_t* __re
   }
 }
 
-template <int MT, int NT, int U, bool TILED>
-static int launch(const void* x, const void* W, void* out, int out_dtype, int M, int N, int K, int k_tiles, int waves, int epi,
+template <int MT, int NT, int U, bool TILED, bool EIGHT = false>
+static int launch(const void* x, const void* W, void* out, int out_dtype, int M, int N, int K, int waves, int epi,
                   const int* order, const RowScale& scale, const StreamOut& so, int tile_rows, XBlocks xb, hipStream_t s) {
-  const int groups = ((N + tile_rows - 1) / tile_rows + NT - 1) / NT;
+  const int n_tiles = (N + tile_rows - 1) / tile_rows, groups = (n_tiles + NT - 1) / NT;
   const size_t lds = (size_t)(waves - 1) * NT * MT * WAVE * 4 * sizeof(float);
   IFX_REQUIRE(lds <= 64 * 1024, "skinny_gemm: %d waves of %dx%d tiles need %zu bytes of LDS", waves, NT, MT, lds);
 #define GO(TO_, EPI_)                                                                                              \
-  hipLaunchKernelGGL((skinny_gemm_kernel<MT, NT, U, TO_, EPI_, TILED>), dim3(groups), dim3(waves * WAVE), lds, s,  \
-                     (const bf16_t*)x, (const bf16_t*)W, (TO_*)out, M, N, K, k_tiles, order, scale, so, tile_rows, xb)
+  hipLaunchKernelGGL((skinny_gemm_kernel<MT, NT, U, TO_, EPI_, TILED, EIGHT>), dim3(groups), dim3(waves * WAVE), lds, s,  \
+                     (const bf16_t*)x, (const bf16_t*)W, M, N, K, tile_rows, n_tiles, waves, xb.tiles, xb.n, scale.pieces, scale.n, (TO_*)out, order, scale.width, scale.eps, so)
   if (epi == 2) {
     if constexpr (MT == 1) GO(float, 2);
     else IFX_FAIL("skinny_gemm: the stream epilogue takes at most 16 rows");
@@ -443,21 +497,28 @@ extern "C" int ifx_qkv_rope(const void* x, const void* Wt, int M, int K, const v
   IFX_REQUIRE(bias_dtype == DT_BF16 || bias_dtype == DT_F32 || !bias, "qkv_rope: unknown bias dtype %d", bias_dtype);
   IFX_REQUIRE((uintptr_t)bias % 16 == 0, "qkv_rope: the bias must start on 16 bytes");
   if (M == 0) return 0;
-  const int heads = nH + (slots ? 2 * nKV : 0), N = heads * d, groups = N / 32;
-  const int nkb = (K + 63) / 64, k_tiles = ifx_tiled_cols(K) / 32;
-  if (unroll == 0) unroll = 2;
+  const int heads = nH + (slots ? 2 * nKV : 0), N = heads * d;
+  // Half a pair of tiles to a workgroup where that still leaves every compute unit one at most (us at 1 and 8 rows:
+  // 1,152 x 896 4.1, 4.4 -> 3.5, 3.7; 2,048 x 1,536 5.0, 5.5 -> 4.4, 4.9; 2,560 x 2,048 6.1, 6.7 -> 5.0, 5.6; 4,608 x 3,584, two to
+  // some units, 11.1-11.6 in 288 workgroups and 9.0-9.7 in 144).
+  const bool halves = N / 16 <= UNITS;
+  const int groups = halves ? N / 16 : N / 32;
+  const int nkb = (K + 63) / 64;
+  if (unroll == 0) unroll = halves ? 4 : 2;
   if (waves == 0) {
     waves = 1;
     while (waves < 16 && groups * waves < 1024) waves *= 2;
     while (waves > 1 && nkb < waves * 2) waves /= 2;
   }
   IFX_REQUIRE(waves >= 1 && waves <= 16 && (unroll == 2 || unroll == 4), "qkv_rope: waves=%d unroll=%d", waves, unroll);
-  const size_t lds = (size_t)(waves - 1) * 2 * WAVE * 4 * sizeof(float);
-  QkvArgs a{bias, bias_dtype, slots, cs, sn, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, nH, slots ? nKV : 0, d, page_size};
-  const RowScale scale{scale_pieces, n_scale_pieces, scale_width, scale_eps};
+  const size_t lds = (size_t)(waves - 1) * (halves ? 1 : 2) * WAVE * 4 * sizeof(float);
+  QkvArgs a{bias, bias_dtype, slots, cs, sn, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, page_size};
   hipStream_t s = (hipStream_t)stream;
-  if (unroll == 2) hipLaunchKernelGGL(qkv_rope_kernel<2>, dim3(groups), dim3(waves * WAVE), lds, s, (const bf16_t*)x, (const bf16_t*)Wt, M, N, K, k_tiles, a, scale);
-  else hipLaunchKernelGGL(qkv_rope_kernel<4>, dim3(groups), dim3(waves * WAVE), lds, s, (const bf16_t*)x, (const bf16_t*)Wt, M, N, K, k_tiles, a, scale);
+#define GO(U_, H_) hipLaunchKernelGGL((qkv_rope_kernel<U_, H_>), dim3(groups), dim3(waves * WAVE), lds, s, (const bf16_t*)x, (const bf16_t*)Wt, M, N, K, waves, nH, slots ? nKV : 0, d, scale_pieces, n_scale_pieces, scale_width, scale_eps, a)
+  if (halves) { if (unroll == 2) GO(2, true); else GO(4, true); }
+  else if (unroll == 2) GO(2, false);
+  else GO(4, false);
+#undef GO
   IFX_LAUNCH_CHECK();
 }
 
@@ -494,7 +555,22 @@ extern "C" int ifx_skinny_gemm(const void* x, const void* W, void* out, int out_
   const int nkb = (K + 63) / 64;
   // Choices measured on the 7B shapes at 1-16 rows: two row tiles per wave pay off only for very tall
   // weights; deeper unrolling than 4 blocks spills; about 1500-2500 waves fill the chip.
-  if (tiled && mt == 1) {
+  const bool eight = tiled && tile_rows == 8 && M <= 8 && nt <= 1 && (unroll == 0 || unroll == 4 || unroll == 8);
+  if (eight) {
+    // K in one trip of eight blocks of 64 a wave, or of four where it is short, as far as the chip takes it: measured (us; the way of
+    // taller tiles, which shares nothing between the k-tiles, at 1 and 8 rows; then this one by waves x blocks)
+    // (0.5 of each more was the norm's weight, widened ahead of the weights of the product and so waited for; see skinny_gemm_kernel)
+    //   896 x 896      4.6, 4.9    4 x 4 3.9, 4.2   2 x 8 4.1, 4.4        2,048 x 2,048   5.7, 5.9    4 x 8 4.6, 4.8   8 x 4 5.0, 5.1
+    //   896 x 4,864    7.1, 7.6    10 x 8 5.2, 6.6   5 x 8 5.6, 6.3       2,048 x 5,632   9.8, 9.5    12 x 8 6.5, 7.5   6 x 8 6.7, 7.2
+    //   1,536 x 8,960  12.3, 12.2  10 x 8 7.3, 9.6   6 x 8 8.0, 9.3       2,048 x 11,008  15.8, 14.4   10 x 8 10.1, 11.3   6 x 8 10.1, 11.0
+    nt = 1;
+    if (unroll == 0) unroll = nkb <= 16 ? 4 : 8;
+    if (waves == 0) {
+      const int trips = nkb > (M > 4 ? 48 : 96) ? 2 : 1, most = trips == 1 ? 16 : M > 4 ? 6 : 10;
+      waves = (nkb + unroll * trips - 1) / (unroll * trips);
+      if (waves > most) waves = most;
+    }
+  } else if (tiled && mt == 1) {
     // Measured on the tiled copy (shapes of the 0.5B to 72B models, 1-16 rows).  Two row tiles per wave halve the
     // reads of x; they win where they leave 128 workgroups or more and do not make the fullest compute unit fuller
     // (every workgroup of a launch is resident at once, so what counts is how many tiles the unit with the most gets:
@@ -539,10 +615,14 @@ extern "C" int ifx_skinny_gemm(const void* x, const void* W, void* out, int out_
   IFX_REQUIRE(block_tiles == 0 || (block_tiles > 0 && n_blocks > 0 && epi == 0 && !order && (block_tiles % 2 == 0 || nt == 1)),
               "skinny_gemm: blocks of %d tiles with inputs of their own go with the plain epilogue (and an even number of tiles, or one a wave)", block_tiles);
   const XBlocks xb{block_tiles, n_blocks};
+  if (eight) {
+    if (unroll == 4) return launch<1, 1, 4, true, true>(x, W, out, out_dtype, M, N, K, waves, epi, order, scale, so, tile_rows, xb, s);
+    return launch<1, 1, 8, true, true>(x, W, out, out_dtype, M, N, K, waves, epi, order, scale, so, tile_rows, xb, s);
+  }
 #define CASE(MT_, NT_, U_)                                                                                             \
   if (mt == MT_ && nt == NT_ && unroll == U_)                                                                          \
-    return tiled ? launch<MT_, NT_, U_, true>(x, W, out, out_dtype, M, N, K, k_tiles, waves, epi, order, scale, so, tile_rows, xb, s)  \
-                 : launch<MT_, NT_, U_, false>(x, W, out, out_dtype, M, N, K, k_tiles, waves, epi, order, scale, so, 16, xb, s)
+    return tiled ? launch<MT_, NT_, U_, true>(x, W, out, out_dtype, M, N, K, waves, epi, order, scale, so, tile_rows, xb, s)  \
+                 : launch<MT_, NT_, U_, false>(x, W, out, out_dtype, M, N, K, waves, epi, order, scale, so, 16, xb, s)
   // (the combinations left out need more than the 128 registers a workgroup of 16 waves leaves a lane)
   CASE(1, 1, 4); CASE(1, 2, 4); CASE(1, 1, 2); CASE(1, 2, 2);
   CASE(2, 1, 4); CASE(2, 2, 2); CASE(2, 1, 2);

@@ -1361,6 +1361,39 @@ def test_skinny_gemm_from_the_tiled_copy_equals_from_rows(M, N, K, tile_rows):
         assert torch.allclose(pairs, torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2], rtol=1e-4, atol=1e-3 * math.sqrt(K))
 
 
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N,K,waves,unroll", [(8, 8, 0, 0), (14, 72, 2, 8), (896, 896, 0, 0), (1030, 1160, 3, 4), (2048, 2816, 0, 0), (24, 11016, 0, 0), (24, 9000, 16, 8)])
+def test_eight_row_tiles_of_up_to_eight_rows(M, N, K, waves, unroll):
+    """Two k-tiles to a product of the matrix cores: k-values on both sides of a tile, a block and a wave's share, rows of W that fill no
+    tile, with every epilogue; against 64 bits.  Sums in float: 2^-24 of the terms' magnitudes, times the root of their number."""
+    g = gen(2490 + M)
+    x, w = torch.randn(M, K, generator=g).to(BF16), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16)
+    z, sums = x.double() @ w.double().t(), K ** 0.5 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-7
+    tiled = ops.tile_weights(w.to(DEV), tile_rows=8)
+    args = dict(waves=waves, unroll=unroll, tiled=tiled, tile_rows=8)
+    got = ops.skinny_gemm(x.to(DEV), w.to(DEV), F32, **args).cpu().double()
+    assert ((got - z).abs() <= sums).all(), float(((got - z).abs() / sums).max())
+    got = ops.skinny_gemm(x.to(DEV), w.to(DEV), F32, swiglu_pairs=True, **args).cpu().double()
+    gate, up = z[:, ::2], z[:, 1::2]
+    slope = 1.1 * (gate.abs() + up.abs() + 1.0)
+    assert ((got - torch.nn.functional.silu(gate) * up).abs() <= slope * torch.maximum(sums[:, ::2], sums[:, 1::2]) + 2.0 ** -21 * (gate * up).abs()).all()
+    got = ops.skinny_gemm(x.to(DEV), w.to(DEV), BF16, plain_act=ops.ACT_RELU_SQUARED, **args).cpu().double()
+    want = z.clamp(min=0) ** 2
+    assert ((got - want).abs() <= 2.0 ** -8 * want + 3.0 * z.abs() * sums + sums).all()
+    if N % 4 == 0:
+        lw = ops.LinearWeight(w.to(DEV), tiled, None, 8)
+        stream, nw = torch.randn(M, N, generator=g), (1 + 0.1 * torch.randn(N, generator=g))
+        for norm in (nw, nw.to(BF16)):
+            s = stream.to(DEV)
+            out = ops.linear_into_stream(x.to(DEV), lw, s, norm.to(DEV), 1e-5)
+            total = stream.double() + z
+            assert ((s.cpu().double() - total).abs() <= sums + 2.0 ** -22 * total.abs()).all()
+            factor = torch.rsqrt(out.pieces.sum(0)[:M].cpu().double() / N + 1e-5)
+            rows = out.rows.cpu().double() * factor[:, None]
+            want = pm.rms_norm(total, norm.double(), 1e-5)
+            assert ((rows - want).abs() <= 2.0 ** -8 * want.abs() + 4.0 * sums * factor[:, None] + 1e-6).all()
+
+
 def test_tiled_copies_of_other_tile_heights():
     """A tile of p rows is stored as 4 runs of p 16-byte pieces per 32 k-values; p is chosen below 16 where 16-row
     tiles would leave compute units without a tile; what is not a height, or a height with an order, is refused."""
