@@ -31,8 +31,11 @@ CSRC = os.path.normpath(CSRC)
 from .device import ARCH
 # -packed-fp32-ops is switched off for device code: some packed float forms have given wrong
 # results on this hardware.  The host pass of hipcc does not know the feature and says so.
+# Kernel arguments that come first and are no structs arrive in scalar registers with the launch (up to 14 of four bytes) instead of
+# by a load of their own, which every small launch waits for before its first real one: 0.25 to 0.3 us of 3.5 to 5 in a graph
+# of launches of 56 to 256 workgroups that read 32 to 64 KB of weights each.
 FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",
-         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-result"]
+         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-result"]
 
 HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC"]
 # INFERFLUX_HOST_SANITIZE=1 builds the host-only modules (the cache's bookkeeping) with the address and
