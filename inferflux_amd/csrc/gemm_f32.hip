@@ -117,6 +117,58 @@ __global__ __launch_bounds__(1024) void gemm_f32_few_kernel(const TA* __restrict
   }
 }
 
+// ---- up to 8 rows: SP slices of K to a wave ------------------------------------------------------------------------------
+// With up to 16 / SP rows of A the matrix instruction's 16 x 16 outputs hold as many rows of W for SP slices at once: lane i's
+// row of W and of A is i % B of slice SP wave + i / B (B = 16 / SP), and of the B x B blocks of outputs those on the diagonal are
+// a slice's (the others, one slice's rows of A by another's of W, are left).  So a workgroup takes B weight rows instead of 16,
+// every load still has work for all lanes, and the order of an element's sum is the one of the other kernels.  Taken where 16
+// weight rows to a workgroup leave compute units without one (us at 4 rows, 16 rows : 8 rows : 4 rows to a workgroup)
+//   896 x 896 4.5 : 3.5 : 3.1     896 x 4,864 17.2 : 10.5 : 8.8     1,024 x 2,816 11.6 : 7.2 : 6.6    1,536 x 1,536 7.6 : 5.5 : 6.1
+//   2,048 x 11,008 38.0 : 23.1 : 27.3     2,560 x 2,048 8.6 : 8.8 : 9.1      4,096 x 4,096 16.7 : 17.5 : 20.3
+// or where their last round is far from full and A is little to read (6,144 x 2,048 15.0 : 13.6, 9,728 x 896 11.1 : 10.4; but
+// 11,264 x 2,048 22.7 : 25.6).  More than four steps in flight a wave (5, 10, 20) gain at K = 4,864 only (8.0 at 20) and lose elsewhere.
+template <typename TA, typename TO, int SP, int STEPS, bool VEC>
+__global__ __launch_bounds__(64 * N_SLICES / SP) void gemm_f32_narrow_kernel(const TA* __restrict__ A, const float* __restrict__ W,
+                                                                             const float* __restrict__ bias, TO* __restrict__ C,
+                                                                             int M, int N, int K) {
+  constexpr int B = 16 / SP;
+  __shared__ float part[N_SLICES][B * B];
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int i = lane % 16, q = lane / 16, r = i % B, slice = SP * wave + i / B;
+  const int n0 = blockIdx.x * B;
+  const int len = slice_len(K), k_lo = slice * len, k_hi = min(K, k_lo + len);
+  const float* wrow = W + (size_t)min(n0 + r, N - 1) * K;      // (columns beyond N are computed and dropped)
+  const TA* arow = A + (size_t)min(r, M - 1) * K;
+  const int a_hi = r < M ? k_hi : 0;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < len; k0 += 16 * STEPS) {
+    f32x4 w[STEPS], a[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const int k = k_lo + k0 + 16 * s + 4 * q;
+      w[s] = load4<VEC>(wrow, k, k_hi);
+      a[s] = load4<VEC>(arow, k, a_hi);
+    }
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][j], w[s][j], acc, 0, 0, 0);
+  }
+  // lane (i, q) holds rows 4 q + j of column i
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if ((4 * q + j) / B == i / B) part[slice][(4 * q + j) % B * B + r] = acc[j];
+  __syncthreads();
+  const int e = threadIdx.x, m = e / B, n = n0 + e % B;
+  if (e < B * B && m < M && n < N) {
+    float v = part[0][e];
+#pragma unroll
+    for (int s = 1; s < N_SLICES; ++s) v += part[s][e];
+    if (bias) v += bias[n];
+    C[(size_t)m * N + n] = from_f<TO>(v);
+  }
+}
+
 // ---- many rows: tiles of A and W through LDS -----------------------------------------------------------------------------
 // A workgroup of four waves makes (32 TM) x (32 TN) outputs, two waves by two; a step of 32 k-values goes through LDS, the next
 // one is on its way from memory meanwhile.  Bound by the matrix units: a wave reads TM + TN fragments of 16 bytes a lane for
@@ -224,12 +276,19 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
                      dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K)
   // (a grid has at most 65,535 rows: millions of rows by a handful of columns are the tile kernel's, whose limit the caller checks)
   const bool in16 = (M + 15) / 16 <= 65535, in32 = (M + 31) / 32 <= 65535;
-  if (M <= 16 || (in16 && t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
+#define NARROW(SP, STEPS)                                                                                        \
+  hipLaunchKernelGGL((gemm_f32_narrow_kernel<TA, TO, SP, STEPS, VEC>), dim3((N + 16 / SP - 1) / (16 / SP)),      \
+                     dim3(64 * N_SLICES / SP), 0, s, A, W, bias, C, M, N, K)
+  const double b16 = blocks(16, 16), full16 = 256.0 * rounds(16, 16);
+  if (M <= 4 && N <= 1024) NARROW(4, 4);
+  else if ((M <= 8 && N <= 2048) || (M <= 4 && b16 > 256.0 && b16 < 0.85 * full16)) NARROW(2, 4);
+  else if (M <= 16 || (in16 && t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
   else if (in32 && t21 <= t22 && t21 <= tiles) FEW(2, 1);
   else if (in32 && t22 <= tiles) FEW(2, 2);
   else
     hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K);
 #undef FEW
+#undef NARROW
 }
 
 extern "C" int ifx_gemm_f32(const void* A, int a_dtype, const float* W, const float* bias, void* C,

@@ -528,6 +528,17 @@ def test_gemm_f32_kernels_agree_bit_for_bit(N, K, adtype):
     assert torch.equal(ops.gemm_f32(shifted, w, None, F32), whole)
 
 
+@pytest.mark.parametrize("N,K", [(3, 5), (130, 36), (1024, 260), (1030, 896), (2048, 1160), (6160, 64)])
+@pytest.mark.parametrize("adtype", [F32, BF16])
+def test_gemm_f32_of_up_to_8_rows_is_a_part_of_many(N, K, adtype):
+    """Several slices of K to a wave (up to 4 and up to 8 rows, weights of few rows, a last round that is not full): the bits of a product of many."""
+    g = gen(2510 + N)
+    x, w = torch.randn(300, K, generator=g).to(adtype).to(DEV), torch.randn(N, K, generator=g).to(DEV)
+    whole = ops.gemm_f32(x, w, None, F32)
+    for M in (1, 3, 4, 5, 8, 9):
+        assert torch.equal(ops.gemm_f32(x[:M].contiguous(), w, None, F32), whole[:M]), M
+
+
 @pytest.mark.parametrize("M", [1_048_560, 1_048_561, 2_097_120, 2_097_121, 2_200_000, 4_194_240])
 def test_gemm_f32_of_millions_of_rows(M):
     """Rows on both sides of what a grid of 16 or 32 of them to a workgroup holds, and the most that a product takes; one more is refused."""
