@@ -62,6 +62,7 @@ def module_variants() -> Iterable[Tuple[str, Variant]]:
     yield ("sampling", ())
     yield ("gemm_bf16", ())
     yield ("gemm_wide", ())
+    yield ("gemm_ring", ())
     yield ("layernorm", ())
     yield ("latent", ())
     yield ("moe", ())
@@ -1155,12 +1156,16 @@ def wide_gemm(x, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, 
     """bfloat16 x [M <= 128, K] times ``weight`` transposed from its tiled copy, x shared through LDS by the waves
     of a workgroup: the product for 17-64 rows, for 65-128 rows of weights with few rows, and for 9-16 rows of large
     tall weights.  ``waves`` (4-16 per workgroup, 8 beyond 64 rows; one tile of weight rows each) and ``slices`` of K
-    (added in a fixed order): 0 lets the kernel choose.  With ``keep_slices`` a product of several slices comes back as
+    (added in a fixed order): 0 lets the kernel choose, and with both 0 the ring of slots is taken where it is faster (``ring_takes``).  With ``keep_slices`` a product of several slices comes back as
     ``SliceSums``.  ``x`` may be ``ScaledRows`` (up to 16 rows)."""
     x, scale = _scale_args(x)
     _check(x, "x", (None, None), torch.bfloat16)
     M, K = x.shape
     N = weight.rows.shape[0]
+    # (more than 16 rows carry no factor)
+    if waves == 0 and slices == 0 and weight.tiled is not None and ring_takes(M, N, K, weight.tile_rows, swiglu_pairs) and K % 8 == 0 \
+            and x.data_ptr() % 16 == 0 and not (swiglu_pairs and (N % 2 or weight.order is not None)):
+        return ring_gemm(x, weight, out_dtype, swiglu_pairs=swiglu_pairs, keep_slices=keep_slices, act=act)
     if weight.tiled is None or weight.rows.shape[1] != K or weight.rows.dtype != torch.bfloat16:
         raise KernelError(f"wide_gemm: needs the tiled copy of a bfloat16 [N, {K}] weight")
     if M > WIDE_MAX_M or K % 8:
@@ -1179,6 +1184,62 @@ def wide_gemm(x, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, 
           x.data_ptr(), weight.tiled.data_ptr(), _ptr(out), _DT[out_dtype], _ptr(part), M, N, K, n_waves, n_slices,
           _GATED_EPILOGUE[act] if swiglu_pairs else 0, _ptr(weight.order), weight.tile_rows, *scale, 0, 0, _stream())
     return SliceSums(part, out_dtype) if keep else out
+
+
+def ring_gemm(x: torch.Tensor, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, row_tiles: int = 0, slices: int = 0,
+              swiglu_pairs: bool = False, keep_slices: bool = False, act: int = ACT_SILU):
+    """bfloat16 x [M <= 64, K] times ``weight`` transposed from its tiled copy, both through a ring of slots in LDS.  ``row_tiles`` (1 to 8)
+    of the weight to a workgroup and ``slices`` of K: 0 chooses (``ring_plan``); ``keep_slices`` and
+    the epilogue as for ``wide_gemm``."""
+    _check(x, "x", (None, None), torch.bfloat16)
+    M, K = x.shape
+    N = weight.rows.shape[0]
+    if weight.tiled is None or weight.rows.shape[1] != K or weight.rows.dtype != torch.bfloat16 or K % 8:
+        raise KernelError(f"ring_gemm: needs the tiled copy of a bfloat16 [N, {K}] weight")
+    if swiglu_pairs and (N % 2 or weight.order is not None):
+        raise KernelError("ring_gemm: gate/up pairs need an even number of weight rows in their natural order")
+    if _tiled_size(N, K, weight.tile_rows) != weight.tiled.numel():
+        raise KernelError(f"ring_gemm: the copy is not that of a [{N}, {K}] weight in tiles of {weight.tile_rows} rows")
+    row_tiles, steps = ring_plan(M, N, K, weight.tile_rows, swiglu_pairs, row_tiles, slices)
+    n_slices = -(-(-(-K // 128)) // steps)
+    part = torch.empty((n_slices, M, N), dtype=torch.float32, device=x.device) if n_slices > 1 else None
+    out = None if n_slices > 1 else torch.empty((M, N // 2 if swiglu_pairs else N), dtype=out_dtype, device=x.device)
+    _call(load_module("gemm_ring"), "ifx_ring_gemm", (P, P, P, I, P, I, I, I, I, I, I, I, P, I, P),
+          x.data_ptr(), weight.tiled.data_ptr(), _ptr(out), _DT[out_dtype], _ptr(part), M, N, K, row_tiles, n_slices, steps,
+          _GATED_EPILOGUE[act] if swiglu_pairs else 0, _ptr(weight.order), weight.tile_rows, _stream())
+    if n_slices == 1:
+        return out
+    sums = SliceSums(part, out_dtype)
+    return sums if keep_slices else sums.sum()
+
+
+RING_DEEP_STEPS = 48          # steps of 128 k-values from which a slice's own traffic, not its start, sets the row tiles to a workgroup
+
+
+def ring_plan(M: int, N: int, K: int, tile_rows: int, one_slice: bool, row_tiles: int = 0, slices: int = 0) -> Tuple[int, int]:
+    """(row tiles to a workgroup, steps of 128 k-values to a slice): about one workgroup to each of the 256 compute units.  Weights that
+    are cut into slices of K take two row tiles where K is short (896 x 4,864 at 64 rows 7.3 us, 8.0 with eight) and, where it is
+    deep, four up to 32 rows and eight beyond, whose x is read half as often (1,536 x 8,960 12.3 : 11.8, 3,584 x 18,944 30.1 :
+    28.3, but at 17 rows 8.9 : 9.6 and 24.1 : 25.3)."""
+    n_tiles, steps = -(-N // tile_rows), -(-K // 128)
+    if row_tiles <= 0:
+        row_tiles = -(-n_tiles // COMPUTE_UNITS) if one_slice else 2 if steps < RING_DEEP_STEPS else 4 if M <= 32 else 8
+        row_tiles = min(8, row_tiles)
+    if one_slice:
+        slices = 1
+    elif slices <= 0:
+        slices = max(1, min(COMPUTE_UNITS // -(-n_tiles // row_tiles), steps // 2))
+    return row_tiles, -(-steps // min(slices, steps))
+
+
+def ring_takes(M: int, N: int, K: int, tile_rows: int, one_slice: bool) -> bool:
+    """Whether 17 to 64 rows go to ``ring_gemm`` instead of ``wide_gemm``: where a row of workgroups holds the weight's row tiles, up to
+    six to a workgroup for gate/up and one a compute unit for weights that are cut into slices (us at 17 / 32 / 64 rows, wide : ring)
+        gate/up 9,728 x 896 9.4 : 6.8, 9.7 : 7.2, 10.7 : 8.6      17,920 x 1,536 14.4 : 13.4, 14.9 : 13.4, 16.9 : 14.7
+                22,016 x 2,048 22.2 : 19.1, 22.2 : 19.3, 22.1 : 20.0, but 37,888 x 3,584 45.1 : 46.8, 44.1 : 47.5, 50.8 : 54.2
+        896 x 4,864 6.6 : 5.7, 6.7 : 5.6, 9.0 : 7.3     1,536 x 8,960 10.5 : 8.9, 10.3 : 9.2, 13.6 : 11.8    1,024 x 1,024 4.3 : 3.7, 4.5 : 3.8, 5.6 : 4.4
+        3,584 x 18,944 25.5 : 24.1, 25.6 : 24.5, 31.0 : 28.3     2,560 x 2,048 5.3 : 5.2, 5.8 : 5.6, 7.6 : 7.1, but 4,608 x 3,584 8.5 : 8.8, 9.1 : 9.2, 11.2 : 11.1."""
+    return 17 <= M <= SKINNY_MAX_M and -(-N // tile_rows) <= (6 if one_slice else 1) * COMPUTE_UNITS and K < 1 << 20
 
 
 def streams_weight(n_rows: int, weight) -> bool:

@@ -1539,6 +1539,44 @@ def test_fused_qkv_random_shapes(seed):
     assert torch.all(vc.cpu().permute(0, 3, 1, 2).reshape(pages * P_, -1)[~written] == 0), case
 
 
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 50, 64])
+@pytest.mark.parametrize("N,K,tile_rows,row_tiles,slices", [(50, 64, 16, 1, 1), (130, 200, 8, 2, 0), (577, 1000, 10, 4, 3), (3, 8, 16, 8, 1), (300, 2104, 14, 8, 16),
+                                                            (900, 640, 16, 5, 1), (1024, 1160, 8, 0, 0), (96, 8968, 16, 3, 2), (700, 264, 12, 6, 1), (112, 520, 16, 7, 5)])
+def test_ring_gemm(M, N, K, tile_rows, row_tiles, slices):
+    """Every number of row tiles to a workgroup; rows of x and W that fill no tile; one step, fewer and more than the ring's slots, slices
+    whose last one is short, a K that ends within a step and a k-tile: against 64 bits.  Sums in float: 2^-24 of the terms'
+    magnitudes, times the root of their number; gate/up and a tile order as well."""
+    g = gen(2500 + M + N)
+    x, w = torch.randn(M, K, generator=g).to(BF16), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16)
+    z, sums = x.double() @ w.double().t(), K ** 0.5 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-7
+    lw = ops.prepare_linear(w.to(DEV), tile_rows=tile_rows)
+    got = ops.ring_gemm(x.to(DEV), lw, F32, row_tiles, slices).cpu().double()
+    assert ((got - z).abs() <= sums).all(), float(((got - z).abs() / sums).max())
+    kept = ops.ring_gemm(x.to(DEV), lw, BF16, row_tiles, slices, keep_slices=True)
+    kept = kept.sum(F32).cpu().double() if isinstance(kept, ops.SliceSums) else kept.cpu().double()
+    assert ((kept - z).abs() <= sums + 2.0 ** -8 * z.abs()).all()
+    if N % 2 == 0:
+        for act, f in ((ops.ACT_SILU, torch.nn.functional.silu), (ops.ACT_GELU_TANH, lambda v: torch.nn.functional.gelu(v, approximate="tanh"))):
+            got = ops.ring_gemm(x.to(DEV), lw, BF16, row_tiles, swiglu_pairs=True, act=act).cpu().double()
+            gate, up = z[:, ::2], z[:, 1::2]
+            want = f(gate) * up
+            assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1.2 * (gate.abs() + up.abs() + 1.0) * torch.maximum(sums[:, ::2], sums[:, 1::2])).all()
+    if tile_rows == 16 and N % 16 == 0:
+        order = torch.randperm(N // 16, generator=g).to(torch.int32)
+        shuffled = ops.prepare_linear(w.to(DEV), order.to(DEV))
+        assert torch.equal(ops.ring_gemm(x.to(DEV), shuffled, F32, row_tiles, slices), ops.ring_gemm(x.to(DEV), lw, F32, row_tiles, slices))
+
+
+def test_17_to_64_rows_go_to_the_ring_where_their_tiles_make_one_row_of_workgroups():
+    assert ops.ring_takes(17, 9728, 896, 16, True) and ops.ring_takes(64, 24576, 2048, 16, True) and ops.ring_takes(33, 2048, 11008, 8, False)
+    assert not ops.ring_takes(16, 9728, 896, 16, True) and not ops.ring_takes(65, 1024, 1024, 8, False)
+    assert not ops.ring_takes(64, 37888, 3584, 16, True) and not ops.ring_takes(64, 4608, 3584, 16, False)
+    for M, N, K, p, one in ((64, 17920, 1536, 16, True), (17, 1536, 8960, 8, False), (64, 1536, 8960, 8, False), (40, 896, 4864, 8, False), (20, 64, 64, 16, False)):
+        tiles, steps = ops.ring_plan(M, N, K, p, one)
+        groups, all_steps = -(-(-(-N // p)) // tiles), -(-K // 128)
+        assert 1 <= tiles <= 8 and 1 <= steps <= all_steps and (steps == all_steps if one else groups * -(-all_steps // steps) <= 256)
+
+
 @pytest.mark.parametrize("M", [9, 17, 32, 33, 50, 64, 65, 81, 100, 128])
 @pytest.mark.parametrize("N,K", [(50, 64), (130, 200), (577, 1000), (4608, 3584), (200, 2104), (4100, 136),
                                  (9000, 264)])                     # tall enough for workgroups of fewer than 8 waves at 33-64 rows
