@@ -8,7 +8,10 @@
 //                          weights whose rows alternate 16 of Wg with 16 of Wu
 //   ifx_moe_few_down       parts[choice][row][:] = weight[item] * Wd[e] act[item] in float; the kernel that adds the result to
 //                          the stream sums the choices in order
-// Identity experts (ids from `n_real` on) and weights on the experts' inputs are those of grouped_gemm.hip.
+// Identity experts (ids from `n_real` on) and weights on the experts' inputs are those of grouped_gemm.hip.  A shared expert, which
+// every row takes with weight 1, runs in the same launches: its rows are workgroups of their own ahead of the experts', its output
+// one more part.  As two products, an activation's launch and the launch that added it, one row of 2,048 values to a shared
+// expert of 1,408 took 19.5 us beside its experts, now 7.5.
 //
 // The products are bound by the chosen experts' bytes.  A workgroup takes an expert and NT x 16 of its weight rows and finds the
 // expert's items itself, from the step's few ids (no ordered list, no launch that makes one); its waves split K, meet in LDS in
@@ -262,27 +265,41 @@ struct FewArgs {
   float limit;
   int weigh_input;          // the weight is on an expert's input: gate/up multiplies its sums by it, down leaves it out
   int k_tiles;              // tiled: tiles of 32 k-values to a row tile, an even number; 0: plain rows
+  // the shared expert: the first shared_y rows of workgroups (0: there is none), all T rows its items
+  int shared_y, shared_k, shared_n, shared_k_tiles;
+  const bf16_t* shared_x;   // [T][shared_k]
+  const bf16_t* shared_w;   // [shared_n][shared_k], in the experts' form
+  void* shared_out;         // gate/up: [T][shared_n / 2]; down: [T][N]
+  float shared_limit;
 };
 
 template <bool DOWN, bool TILED, int MT, int NT, int U>
 __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
   extern __shared__ float red[];      // [waves - 1][NT * MT][64 lanes][4], then the list
   const int wave = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x % WAVE, col = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (16 * NT), n_items = a.T * a.top;
+  const bool shared = (int)blockIdx.y < a.shared_y;
+  const int n0 = (shared ? blockIdx.y * gridDim.x + blockIdx.x : blockIdx.x) * (16 * NT), n_items = a.T * a.top, y = blockIdx.y - a.shared_y;
+  const int K = shared ? a.shared_k : a.K, N = shared ? a.shared_n : a.N, k_tiles = shared ? a.shared_k_tiles : a.k_tiles;
   int* list = (int*)(red + (size_t)(nw - 1) * NT * MT * WAVE * 4);      // (room for all items: a row may name an expert twice)
   // The expert's items in rising order.  Every wave finds all of them and writes the same list.
-  const int group = a.by_item ? a.ids[blockIdx.y] : (int)blockIdx.y;
-  int count = 0, first = n_items;
-  for (int i0 = 0; i0 < n_items; i0 += WAVE) {
-    const int i = i0 + lane;
-    const unsigned long long has = __ballot(i < n_items && a.ids[min(i, n_items - 1)] == group);
-    if (has & (1ull << lane)) list[count + __popcll(has & ((1ull << lane) - 1))] = i;
-    if (has && first == n_items) first = i0 + __ffsll(has) - 1;
-    count += __popcll(has);
+  int group = 0, count = 0;
+  if (shared) {
+    if (n0 >= N) return;
+    count = a.T;
+  } else {
+    group = a.by_item ? a.ids[y] : y;
+    int first = n_items;
+    for (int i0 = 0; i0 < n_items; i0 += WAVE) {
+      const int i = i0 + lane;
+      const unsigned long long has = __ballot(i < n_items && a.ids[min(i, n_items - 1)] == group);
+      if (has & (1ull << lane)) list[count + __popcll(has & ((1ull << lane) - 1))] = i;
+      if (has && first == n_items) first = i0 + __ffsll(has) - 1;
+      count += __popcll(has);
+    }
+    if (count == 0 || (a.by_item && first != y)) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
-  if (count == 0 || (a.by_item && first != (int)blockIdx.y)) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  if (group >= a.n_real) {             // an identity expert (the whole workgroup)
+  if (!shared && group >= a.n_real) {             // an identity expert (the whole workgroup)
     if (DOWN)
       for (int i = threadIdx.x; i < count * 16 * NT; i += blockDim.x) {
         const int m = list[i / (16 * NT)], n = n0 + i % (16 * NT);
@@ -291,25 +308,27 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
       }
     return;
   }
+  const bf16_t *w = shared ? a.shared_w : a.w, *x = shared ? a.shared_x : a.x;
   const bf16_t* wrow[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)      // (rows past N are read again, never stored)
-    wrow[nt] = TILED ? a.w + ((size_t)(group * (a.N / 16) + min(n0 / 16 + nt, a.N / 16 - 1)) * a.k_tiles * WAVE + lane) * 8
-                     : a.w + ((size_t)group * a.N + min(n0 + 16 * nt + col, a.N - 1)) * a.K;
+    wrow[nt] = TILED ? w + ((size_t)(group * (N / 16) + min(n0 / 16 + nt, N / 16 - 1)) * k_tiles * WAVE + lane) * 8
+                     : w + ((size_t)group * N + min(n0 + 16 * nt + col, N - 1)) * K;
   for (int start = 0; start < count; start += 16 * MT) {      // (more items than columns: the rows are streamed again, from the L2)
   int item[MT];
   const bf16_t* xrow[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    item[mt] = start + 16 * mt + col < count ? list[start + 16 * mt + col] : -1;
-    xrow[mt] = a.x + (size_t)(item[mt] < 0 ? 0 : item[mt] / a.x_div) * a.K;
+    const int at = start + 16 * mt + col;
+    item[mt] = at < count ? (shared ? at : list[at]) : -1;
+    xrow[mt] = x + (size_t)(item[mt] < 0 ? 0 : shared ? item[mt] : item[mt] / a.x_div) * K;
   }
   floatx4 acc[NT][MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int nkb = (a.K + 63) / 64;
+  const int nkb = (K + 63) / 64;
   for (int kb0 = wave * U; kb0 < nkb; kb0 += nw * U) {
     bf16x8 wv[U][NT][2], xv[U][MT][2];
 #pragma unroll
@@ -318,7 +337,7 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
       for (int h = 0; h < 2; ++h) {
         // plain rows: a lane's two pieces are 32 contiguous bytes, four lanes cover a line; tiles: a wave's piece is 1 KB of contiguous memory
         const int k = (kb0 + u) * 64 + 16 * g + 8 * h;
-        const bool in = TILED ? kb0 + u < nkb : k < a.K;
+        const bool in = TILED ? kb0 + u < nkb : k < K;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           const bf16x8* p = (const bf16x8*)(wrow[nt] + (TILED ? (size_t)(2 * (kb0 + u) + h) * WAVE * 8 : (size_t)k));
@@ -331,7 +350,7 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
       for (int h = 0; h < 2; ++h) {
         const int k = TILED ? (kb0 + u) * 64 + 32 * h + 8 * g : (kb0 + u) * 64 + 16 * g + 8 * h;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) xv[u][mt][h] = (k < a.K && item[mt] >= 0) ? *(const bf16x8*)(xrow[mt] + k) : zero8();
+        for (int mt = 0; mt < MT; ++mt) xv[u][mt][h] = (k < K && item[mt] >= 0) ? *(const bf16x8*)(xrow[mt] + k) : zero8();
       }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -353,12 +372,12 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
           *(floatx4*)(red + ((size_t)((wave - 1) * NT * MT + nt * MT + mt) * WAVE + lane) * 4) = acc[nt][mt];
     __syncthreads();
     if (wave > 0) continue;
-    for (int w = 1; w < nw; ++w)
+    for (int v = 1; v < nw; ++v)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const floatx4 o = *(const floatx4*)(red + ((size_t)((w - 1) * NT * MT + nt * MT + mt) * WAVE + lane) * 4);
+          const floatx4 o = *(const floatx4*)(red + ((size_t)((v - 1) * NT * MT + nt * MT + mt) * WAVE + lane) * 4);
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc[nt][mt][r] += o[r];
         }
@@ -369,23 +388,23 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
     const int m = item[mt];
     if (m < 0) continue;
     if constexpr (!DOWN) {             // NT = 2: 16 rows of Wg and the same 16 of Wu
-      const float wi = a.weigh_input ? a.weights[m] : 1.f;
+      const float wi = a.weigh_input && !shared ? a.weights[m] : 1.f, limit = shared ? a.shared_limit : a.limit;
       bf16x4 y;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) y[r] = (__bf16)gated_act(wi * acc[0][mt][r], wi * acc[1][mt][r], a.act, a.limit);
-      *(bf16x4*)((bf16_t*)a.out + (size_t)m * (a.N / 2) + n0 / 2 + 4 * g) = y;
+      for (int r = 0; r < 4; ++r) y[r] = (__bf16)gated_act(wi * acc[0][mt][r], wi * acc[1][mt][r], a.act, limit);
+      *(bf16x4*)((bf16_t*)(shared ? a.shared_out : a.out) + (size_t)m * (N / 2) + n0 / 2 + 4 * g) = y;
     } else {
-      const float wgt = a.weigh_input ? 1.f : a.weights[m];
-      float* o = (float*)a.out + ((size_t)(m % a.top) * a.T + m / a.top) * a.N;
+      const float wgt = a.weigh_input || shared ? 1.f : a.weights[m];
+      float* o = shared ? (float*)a.shared_out + (size_t)m * N : (float*)a.out + ((size_t)(m % a.top) * a.T + m / a.top) * N;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const int n = n0 + 16 * nt + 4 * g;
-        if (n + 3 < a.N && a.N % 4 == 0) {
+        if (n + 3 < N && N % 4 == 0) {
           *(floatx4*)(o + n) = floatx4{wgt * acc[nt][mt][0], wgt * acc[nt][mt][1], wgt * acc[nt][mt][2], wgt * acc[nt][mt][3]};
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (n + r < a.N) o[n + r] = wgt * acc[nt][mt][r];
+            if (n + r < N) o[n + r] = wgt * acc[nt][mt][r];
         }
       }
     }
@@ -394,8 +413,10 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
 }
 
 template <bool DOWN, int MT, int NT, int U>
-static int launch_few(const FewArgs& a, int n_groups, int waves, hipStream_t s) {
-  const dim3 grid((a.N + 16 * NT - 1) / (16 * NT), a.by_item ? a.T * a.top : n_groups);
+static int launch_few(FewArgs a, int n_groups, int waves, hipStream_t s) {
+  const int columns = (a.N + 16 * NT - 1) / (16 * NT);
+  if (a.shared_w) a.shared_y = ((a.shared_n + 16 * NT - 1) / (16 * NT) + columns - 1) / columns;
+  const dim3 grid(columns, a.shared_y + (a.by_item ? a.T * a.top : n_groups));
   const size_t lds = (size_t)(waves - 1) * NT * MT * WAVE * 4 * sizeof(float) + (size_t)a.T * a.top * sizeof(int);
   if (a.k_tiles > 0) hipLaunchKernelGGL((moe_few_kernel<DOWN, true, MT, NT, U>), grid, dim3(waves * WAVE), lds, s, a);
   else hipLaunchKernelGGL((moe_few_kernel<DOWN, false, MT, NT, U>), grid, dim3(waves * WAVE), lds, s, a);
@@ -410,25 +431,33 @@ static int few_waves(int K) {
   return waves;
 }
 
-// E: the experts and the identity experts that ids name; T rows, at most MAX_ROWS.
+// E: the experts and the identity experts that ids name; T rows, at most MAX_ROWS.  shared_w (or null): a shared expert of
+// shared_ff inner values, in the experts' form, its activations to shared_act [T][shared_ff].
 extern "C" int ifx_moe_few_gate_up(const void* x, const void* w, void* act, const int* ids, int T, int E, int K, int ff, int top, int n_real,
-                                   int act_kind, float limit, const float* in_weights, int tiled, void* stream) {
+                                   int act_kind, float limit, const float* in_weights, int tiled, const void* shared_w, void* shared_act,
+                                   int shared_ff, float shared_limit, void* stream) {
   IFX_REQUIRE(K > 0 && K % 8 == 0 && ff > 0 && ff % 16 == 0, "moe_few_gate_up: K=%d must be a multiple of 8, ff=%d of 16", K, ff);
   IFX_REQUIRE(T > 0 && T <= MAX_ROWS && top > 0 && top <= MAX_TOP && E > 0 && E <= MAX_E, "moe_few_gate_up: %d rows (at most %d) of %d of %d experts", T, MAX_ROWS, top, E);
+  IFX_REQUIRE(!shared_w || (shared_act && shared_ff > 0 && shared_ff % 16 == 0 && shared_ff <= 1 << 20), "moe_few_gate_up: a shared expert of %d (a multiple of 16)", shared_ff);
+  const int k_tiles = tiled ? (K + 63) / 64 * 2 : 0;
   FewArgs a{(const bf16_t*)x, (const bf16_t*)w, act, ids, in_weights, nullptr, K, 2 * ff, top, T, top, n_real, act_kind,
-            T * top < E ? 1 : 0, limit, in_weights ? 1 : 0, tiled ? (K + 63) / 64 * 2 : 0};
+            T * top < E ? 1 : 0, limit, in_weights ? 1 : 0, k_tiles, 0, K, 2 * shared_ff, k_tiles, (const bf16_t*)x, (const bf16_t*)shared_w, shared_act, shared_limit};
   const int waves = few_waves(K);
   if (T <= 16) return launch_few<false, 1, 2, 3>(a, E, waves, (hipStream_t)stream);
   return launch_few<false, 2, 2, 2>(a, E, waves, (hipStream_t)stream);
 }
 
+// parts [top][T][N], and with a shared expert [top + 1][T][N], its output the last.
 extern "C" int ifx_moe_few_down(const void* act, const void* w, float* parts, const float* weights, const int* ids, int T, int E, int N,
-                                int ff, int top, int n_real, const void* identity, int weigh_input, int tiled, void* stream) {
+                                int ff, int top, int n_real, const void* identity, int weigh_input, int tiled, const void* shared_act,
+                                const void* shared_w, int shared_ff, void* stream) {
   IFX_REQUIRE(ff > 0 && ff % 8 == 0 && N > 0 && (!tiled || N % 16 == 0), "moe_few_down: ff=%d must be a multiple of 8, N=%d of 16 if tiled", ff, N);
   IFX_REQUIRE(T > 0 && T <= MAX_ROWS && top > 0 && top <= MAX_TOP && E > 0 && E <= MAX_E, "moe_few_down: %d rows (at most %d) of %d of %d experts", T, MAX_ROWS, top, E);
+  IFX_REQUIRE(!shared_w || (shared_act && shared_ff > 0 && shared_ff % 8 == 0 && shared_ff <= 1 << 20), "moe_few_down: a shared expert of %d (a multiple of 8)", shared_ff);
   FewArgs a{(const bf16_t*)act, (const bf16_t*)w, parts, ids, weights, (const bf16_t*)identity, ff, N, 1, T, top, n_real, 0,
-            T * top < E ? 1 : 0, 0.f, weigh_input, tiled ? (ff + 63) / 64 * 2 : 0};
-  const int waves = few_waves(ff);
+            T * top < E ? 1 : 0, 0.f, weigh_input, tiled ? (ff + 63) / 64 * 2 : 0, 0, shared_ff, N, tiled ? (shared_ff + 63) / 64 * 2 : 0,
+            (const bf16_t*)shared_act, (const bf16_t*)shared_w, parts + (size_t)top * T * N, 0.f};
+  const int waves = few_waves(shared_w && shared_ff > ff ? shared_ff : ff);
   hipStream_t s = (hipStream_t)stream;
   // (two row tiles to a wave halve its reads of the items; up to 64 items one is better: twice the workgroups)
   if (T <= 16) return T * top <= 64 ? launch_few<true, 1, 1, 2>(a, E, waves, s) : launch_few<true, 1, 2, 2>(a, E, waves, s);

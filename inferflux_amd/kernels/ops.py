@@ -725,9 +725,11 @@ def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_grou
 
 
 def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, act: int = ACT_SILU,
-                    limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False) -> "SliceSums":
+                    limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False, shared=None, shared_limit: float = 0.0) -> "SliceSums":
     """``moe_experts`` for up to 64 rows in bfloat16: two launches that stream every chosen expert's weights once, whatever the
-    number of rows that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``).  Returns the choices' weighted outputs as ``SliceSums`` [top, T, N] like ``moe_experts_grouped``."""
+    number of rows that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``).  Returns the choices' weighted outputs as ``SliceSums`` [top, T, N] like ``moe_experts_grouped``.
+    ``shared``: (gate_up, down) of an expert that every row takes, [1, 2 shared_ff, K] and [1, N, shared_ff] in the experts' form
+    (with its own ``shared_limit``): its output is the last of [top + 1, T, N]."""
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
     gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
@@ -741,12 +743,22 @@ def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, 
     if n_identity and N != K:
         raise KernelError(f"moe_few: identity experts hand back the row itself, so N={N} must equal K={K}")
     mod, stream = load_module("moe_few"), _stream()
-    a = torch.empty((T * top, ff), dtype=torch.bfloat16, device=h.device)
-    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
-          T, E, K, ff, top, n_real, int(act), float(limit), weights.data_ptr() if weigh_input else 0, gu_tiled, stream)
-    parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P), a.data_ptr(), down_ptr, parts.data_ptr(),
-          weights.data_ptr(), ids.data_ptr(), T, E, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0, down_tiled, stream)
+    shared_ff = shared_gu = shared_down = 0
+    if shared is not None:
+        shape, shared_gu, gu_form = _experts(shared[0], "shared gate_up", (1, None, K))
+        shared_ff = shape[1] // 2
+        _, shared_down, down_form = _experts(shared[1], "shared down", (1, N, shared_ff))
+        if shape[1] % 32 or (gu_form, down_form) != (gu_tiled, down_tiled):
+            raise KernelError(f"moe_few: a shared expert of {shape[1]} gate and up rows (a multiple of 32), in the experts' form")
+    a = torch.empty((T * (top * ff + shared_ff),), dtype=torch.bfloat16, device=h.device)
+    shared_a = a.data_ptr() + 2 * T * top * ff
+    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P, P, I, F, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
+          T, E, K, ff, top, n_real, int(act), float(limit), weights.data_ptr() if weigh_input else 0, gu_tiled,
+          shared_gu, shared_a, shared_ff, float(shared_limit), stream)
+    parts = torch.empty((top + (1 if shared is not None else 0), T, N), dtype=torch.float32, device=h.device)
+    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, P), a.data_ptr(), down_ptr, parts.data_ptr(),
+          weights.data_ptr(), ids.data_ptr(), T, E, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0, down_tiled,
+          shared_a, shared_down, shared_ff, stream)
     return SliceSums(parts, torch.bfloat16)
 
 

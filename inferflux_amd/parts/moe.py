@@ -77,7 +77,7 @@ class MixtureOfExperts(FeedForward):
         self.router = self.gate = self.up = self.down = None
         self.router_bias, self.bias = bool(router_bias), None
         self.shared_gate, self.shared_gate_w = bool(shared_gate), None
-        self.shared = None
+        self.shared = self.shared_few = None
         if shared_ff:
             n = f"{name}.shared"
             self.shared = SwiGLU(n, hidden_size, int(shared_ff), init_std, activation,
@@ -117,13 +117,25 @@ class MixtureOfExperts(FeedForward):
             if self.hidden_size % 16 == 0 and ops.moe_few_takes(dtype, 1, self.hidden_size, self.ff, self.n_routed, self.top):
                 # ... and both products in tiles: nothing reads rows then
                 self.gate, self.down = ops.ExpertTiles(self.gate), ops.ExpertTiles(self.down)
-
+                self._prepare_shared_for_few(tensors, dtype)
         if self.router_bias:
             self.bias = tensors[f"{n}.router.b"].float().contiguous()        # the router is float whatever the file holds
         if self.choice_bias:
             self.correction = tensors[f"{n}.correction"].float().contiguous()
         if self.shared_gate:
             self.shared_gate_w = tensors[f"{n}.shared.sg"].to(dtype).reshape(-1).contiguous()
+
+    def _prepare_shared_for_few(self, tensors, dtype) -> None:
+        """The shared expert in the experts' form too, for steps of few rows, whose experts' launches take it along (where the
+        card has room for one more expert, as for ``prepare_linear``'s copies)."""
+        if self.shared is None or self.shared.intermediate_size % 16 or not ops.decode_weight_copy:
+            return
+        if any(name not in tensors for name in self.shared.names.values()):        # (a caller that loads it by itself)
+            return
+        gate, up, down = (tensors[self.shared.names[k]] for k in ("gate", "up", "down"))
+        if {gate.dtype, up.dtype, down.dtype} != {dtype} or torch.cuda.mem_get_info(gate.device)[0] < 3 * 2 * gate.nbytes + ops.DECODE_COPY_RESERVE_BYTES:
+            return
+        self.shared_few = (ops.ExpertTiles(ops.pair_gate_up(gate[None].contiguous(), up[None].contiguous())), ops.ExpertTiles(down[None].contiguous()))
 
     def route(self, h, few: bool = False):
         return (ops.moe_few_choose if few else ops.moe_route)(
@@ -143,6 +155,13 @@ class MixtureOfExperts(FeedForward):
         ids, weights = self.route(x, few)
         if ctx.timer is not None:
             ctx.timer.mark("ffn.route")
+        if few and self.shared_few is not None:
+            sums = ops.moe_few_experts(x, self.gate, self.down, ids, weights, self.act, self.limit, self.n_identity, self.weigh_input,
+                                       self.shared_few, self.shared.limit)
+            if not self.shared_gate:
+                return sums                 # (the shared expert's output is one more partial sum)
+            base, extra = ops.SliceSums(sums.parts[:-1], sums.dtype), ops.SliceSums(sums.parts[-1:], sums.dtype)
+            return ops.gated_add(base, extra, x, self.shared_gate_w)
         if few:
             return self._with_shared(ops.moe_few_experts(x, self.gate, self.down, ids, weights, self.act, self.limit, self.n_identity,
                                                          self.weigh_input), x, ctx)      # (partial sums, one per choice)

@@ -733,6 +733,37 @@ def test_moe_few_experts_of_rows_that_name_an_expert_twice(T, top, E, tiled):
     assert (got - want).abs().max() < 5 * 2.0 ** -8 * want.abs().max()
 
 
+@pytest.mark.parametrize("T,top,E,K,ff,shared_ff", [(1, 1, 3, 64, 16, 16), (1, 2, 4, 72, 48, 208), (16, 3, 5, 128, 96, 32), (17, 2, 40, 512, 64, 528), (33, 2, 3, 200, 32, 48),
+                                                    (64, 1, 2, 264, 80, 1040)])
+@pytest.mark.parametrize("form", ["tiles", "rows", "input", "clamped"])
+def test_moe_few_with_a_shared_expert(T, top, E, K, ff, shared_ff, form):
+    """A shared expert narrower and wider than the experts, by up to several rows of their workgroups, its rows on both sides of one and
+    two column tiles: the experts' parts as without it up to how K is dealt to the waves, its own part against 64 bits.  One
+    rounding to bfloat16 (2^-8) between the products."""
+    g = gen(2280 + T + shared_ff)
+    N = K // 16 * 16 if form != "rows" else K
+    h = torch.randn(T, K, generator=g).to(BF16)
+    mats = lambda n, f: [(torch.randn(n, f, K, generator=g) / K ** 0.5).to(BF16) for _ in range(2)] + [(torch.randn(n, N, f, generator=g) / f ** 0.5).to(BF16)]
+    (gate, up, down), (sg, su, sd) = mats(E, ff), mats(1, shared_ff)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    weights = torch.rand(T, top, generator=g).to(DEV)
+    form_of = (lambda w: w) if form == "rows" else ops.ExpertTiles
+    few = [(form_of(ops.pair_gate_up(a.to(DEV), b.to(DEV))), form_of(c.to(DEV))) for a, b, c in ((gate, up, down), (sg, su, sd))]
+    act = ops.ACT_CLAMPED_SWISH if form == "clamped" else ops.ACT_SILU
+    limits = (1.0, 0.75) if form == "clamped" else (0.0, 0.0)
+    args = (h.to(DEV), *few[0], ids, weights, act, limits[0], 0, form == "input")
+    got = ops.moe_few_experts(*args, shared=few[1], shared_limit=limits[1]).parts.cpu().double()
+    alone = ops.moe_few_experts(*args).parts.cpu().double()
+    assert got.shape == (top + 1, T, N)
+    z, u = h.double() @ sg[0].double().t(), h.double() @ su[0].double().t()
+    if form == "clamped":
+        z, u = z.clamp(max=limits[1]), u.clamp(-limits[1], limits[1]) + 1.0
+    want = (z * torch.sigmoid((1.702 if form == "clamped" else 1.0) * z) * u) @ sd[0].double().t()
+    for a, b in ((got[-1], want), (got[:-1], alone)):
+        assert (a - b).pow(2).mean().sqrt() < 2.0 ** -8 * b.pow(2).mean().sqrt()
+        assert (a - b).abs().max() < 5 * 2.0 ** -8 * b.abs().max()
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
