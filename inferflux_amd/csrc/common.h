@@ -99,6 +99,7 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 #define ACT_GELU_TANH 1
 #define ACT_CLAMPED_SWISH 2
 #define ACT_RELU_SQUARED 3       // (without a gate: max(x, 0)^2)
+#define ACT_NONE 4               // (the product as it is)
 __device__ __forceinline__ float act_silu(float g) { return g / (1.0f + expf(-g)); }
 __device__ __forceinline__ float act_gelu_tanh(float g) {
   return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));

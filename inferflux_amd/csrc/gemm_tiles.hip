@@ -14,6 +14,12 @@
 // 2,048 rows of 37,888 x 3,584: 422 us (1,320 TFLOP/s; tiles of 256 x 256 by eight waves took 481, the library and the
 // activation 552); 600 of 22,016 x 2,048 49 (93; 72); 4,500 of 17,920 x 1,536 200 (255; 239).  Which sizes come here is a rule
 // of ops.py (many_tiles_take, pairs_tiles_take), with both sides measured.
+//
+// The plain product of deep weights, too, for callers that add partial sums (down):
+//   OUT_SUMS    parts[slice][M][N] = x W^T over a slice of K, in float
+// The library's has no kernel that fits some of these sizes (6,144 rows of 3,584 x 18,944, where 336 tiles of 256 x 256 are 1.3 rounds:
+// 1,061 us, 786 TFLOP/s) and its batched product over slices none that fits others (520 rows 115 us, 1,034 of 2,048 x 11,008 62).
+// Slices of tiles fill the rounds: 650, 69 and 45 us.  Which sizes, tiles and slices: ifx_gemm_tiles_sums_plan.
 #include "product_tiles.h"
 #include "wave_tiles.h"
 
@@ -22,14 +28,15 @@ IFX_DEFINE_LAST_ERROR()
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 
-enum { OUT_PAIRS = 0, OUT_ACT = 1 };
+enum { OUT_PAIRS = 0, OUT_ACT = 1, OUT_SUMS = 2 };
 
 struct TilesArgs {
   const bf16_t* x;          // [M][K]
   const bf16_t* w;          // [N][K]
-  bf16_t* out;              // OUT_PAIRS: [M][N / 2]; OUT_ACT: [M][N]
+  void* out;                // OUT_PAIRS: bf16 [M][N / 2]; OUT_ACT: bf16 [M][N]; OUT_SUMS: float [slices][M][N]
   int M, N, K, act;
   float limit;
+  int slices, slice_k;      // K in so many slices of slice_k values (a multiple of 64; the last what is left)
 };
 
 #define GROUP 4          // tiles of x that meet a tile of W one after the other
@@ -45,15 +52,17 @@ template <int ACT> __device__ __forceinline__ float quick_gated(float g, float u
   return g * quick_sigmoid(1.702f * g) * (up + 1.0f);
 }
 template <int ACT> __device__ __forceinline__ float quick_act(float v) {
+  if (ACT == ACT_NONE) return v;
   if (ACT == ACT_RELU_SQUARED) { const float r = fmaxf(v, 0.f); return r * r; }
   return ACT == ACT_GELU_TANH ? quick_gelu(v) : v * quick_sigmoid(v);
 }
 
 template <int FN, int FM, int OUT>
 struct TilesOut {
+  static constexpr bool TURNED = OUT != OUT_SUMS;          // (a lane's four sums in float are a whole store)
   static constexpr int CHUNK = OUT == OUT_ACT && FN > 8 ? FN / 2 : FN;          // fragments that are turned in LDS at a time
   static constexpr int ROW = 16 * CHUNK * (OUT == OUT_PAIRS ? 1 : 2);      // bytes of a row of them
-  static constexpr int PITCH = ROW + 16, WAVE_BYTES = 16 * PITCH;
+  static constexpr int PITCH = ROW + 16, WAVE_BYTES = TURNED ? 16 * PITCH : 0;
   static constexpr int LDS = WaveTiles<FN, FM>::LDS + 4 * WAVE_BYTES;
 };
 
@@ -113,6 +122,28 @@ __device__ __forceinline__ void tiles_out(const WaveTiles<FN, FM>& p, const Tile
     }
 }
 
+// The sums of a slice of K as they are; stores beyond the rows and columns are dropped.
+template <int FN, int FM>
+__device__ __forceinline__ void tiles_sums(const WaveTiles<FN, FM>& p, const TilesArgs& a, tile_floatx4 (&acc)[FN][FM], int slice, int m, int n) {
+  const int rows = a.M - m;
+  const unsigned long long at0 = (unsigned long long)a.out + ((size_t)slice * a.M + min(m, a.M)) * a.N * 4;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at0), hi = __builtin_amdgcn_readfirstlane((unsigned)(at0 >> 32));
+  const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc((void*)((unsigned long long)hi << 32 | lo), 0,
+                                                                        __builtin_amdgcn_readfirstlane(max(0, min(16 * FM, rows)) * a.N * 4), 0x00020000);
+#pragma unroll
+  for (int b = 0; b < FM; ++b) {
+#pragma unroll
+    for (int c = 0; c < FN; ++c) {
+      asm volatile("" : "+a"(acc[c][b]));
+      const int at = n + 16 * c + 4 * p.g;
+      const bool in = p.col < rows - 16 * b && at < a.N;
+      const tile_floatx4 v = acc[c][b];
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(tile_uintx4, v), out, in ? (p.col * a.N + at) * 4 : TILE_NO_ROW, 16 * b * a.N * 4, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // One workgroup to a CU, one tile after the other.  Workgroup b runs on XCD b % 8, which takes a contiguous range of the tiles.
 template <int FN, int FM, int OUT>
 __global__ __launch_bounds__(256, 1) void tiles_kernel(TilesArgs a) {
@@ -120,43 +151,53 @@ __global__ __launch_bounds__(256, 1) void tiles_kernel(TilesArgs a) {
   typedef TilesOut<FN, FM, OUT> O;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[O::LDS];
   static_assert(O::LDS <= 160 * 1024, "LDS");
-  const int nt = (a.N + P::BN - 1) / P::BN, mt = (a.M + P::BM - 1) / P::BM, total = nt * mt;
+  const int nt = (a.N + P::BN - 1) / P::BN, mt = (a.M + P::BM - 1) / P::BM, total = nt * mt * a.slices;
   const int per = (total + 7) / 8, end = min(total, (int)(blockIdx.x % 8 + 1) * per), stride = gridDim.x / 8;
   int id = blockIdx.x % 8 * per + blockIdx.x / 8;
   if (id >= end) return;
   P p;
   p.init(lds);
-  int n0, m0, share, sharers;
+  int n0, m0, share, sharers, slice = 0, K = a.K;
   auto find = [&](int t) {          // groups of GROUP tiles of x by all of W's
     auto div = [](int v, int by) { return __builtin_amdgcn_readfirstlane(v / by); };        // (by vector instructions: back to scalars)
+    if (OUT == OUT_SUMS) {
+      slice = div(t, nt * mt), t -= slice * nt * mt;
+      K = min(a.slice_k, a.K - slice * a.slice_k);
+    }
     const int turn = div(t, GROUP * nt), in = t - turn * GROUP * nt;
     sharers = min(GROUP, mt - turn * GROUP);
     const int tn = div(in, sharers);
     share = in - tn * sharers;
     m0 = (turn * GROUP + share) * P::BM, n0 = tn * P::BN;
   };
-  auto rows_of_w = [&]() { return tile_buffer(a.w + (size_t)n0 * a.K, (unsigned)min(P::BN, a.N - n0) * (unsigned)a.K * 2u); };
+  auto rows_of_w = [&]() {
+    const int k0 = slice * a.slice_k;
+    return tile_buffer(a.w + (size_t)n0 * a.K + k0, ((unsigned)min(P::BN, a.N - n0) * (unsigned)a.K - (unsigned)k0) * 2u);
+  };
   auto begin = [&]() {
     const int count = min(P::BM, a.M - m0);
-    const tile_uintx4 x = tile_buffer(a.x + (size_t)m0 * a.K, (unsigned)count * (unsigned)a.K * 2u);
-    p.begin(rows_of_w(), x, a.K, a.K * 2, [&](int i) { return i < count ? i * a.K * 2 : TILE_NO_ROW; });
+    const int k0 = slice * a.slice_k;
+    const tile_uintx4 x = tile_buffer(a.x + (size_t)m0 * a.K + k0, ((unsigned)count * (unsigned)a.K - (unsigned)k0) * 2u);
+    p.begin(rows_of_w(), x, K, a.K * 2, [&](int i) { return i < count ? i * a.K * 2 : TILE_NO_ROW; });
     p.touch_rows(share, sharers, a.K * 2);
   };
   find(id);
   begin();
   while (true) {
-    const int n = n0 + p.wn(), m = m0 + p.wm();
+    const int n = n0 + p.wn(), m = m0 + p.wm(), this_slice = slice, this_k = K;
     id += stride;
     const bool more = id < end;
     if (more) find(id);
     p.next = rows_of_w();
     if (!more) p.next[2] = 0;          // (nothing to touch)
     tile_floatx4 acc[FN][FM];
-    p.run(lds, a.K, acc);
+    p.run(lds, this_k, acc);
     if (more) begin();
-    switch (a.act) {
+    if constexpr (OUT == OUT_SUMS) tiles_sums<FN, FM>(p, a, acc, this_slice, m, n);
+    else switch (a.act) {
       case ACT_GELU_TANH: tiles_out<FN, FM, OUT, ACT_GELU_TANH>(p, a, lds, acc, m, n); break;
       case ACT_SILU: tiles_out<FN, FM, OUT, ACT_SILU>(p, a, lds, acc, m, n); break;
+      case ACT_NONE: if constexpr (OUT == OUT_ACT) tiles_out<FN, FM, OUT, ACT_NONE>(p, a, lds, acc, m, n); break;
       default: tiles_out<FN, FM, OUT, OUT == OUT_PAIRS ? ACT_CLAMPED_SWISH : ACT_RELU_SQUARED>(p, a, lds, acc, m, n); break;
     }
     if (!more) break;
@@ -179,7 +220,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM), 2 * PER_CU) void pairs_
   for (int b = 0; b < P::FM; ++b) {
     const int m = m0 + P::wm() + 16 * b + lane % 16;
     if (m >= a.M) continue;
-    bf16_t* out = a.out + (size_t)m * (a.N / 2);
+    bf16_t* out = (bf16_t*)a.out + (size_t)m * (a.N / 2);
 #pragma unroll
     for (int c = 0; c < P::FN; ++c) {
       const int n = n0 + P::wn() + 16 * c + 4 * g;
@@ -252,12 +293,61 @@ extern "C" int ifx_gemm_pairs_wins(int M, int N, int K) {
   return M >= TILES_MIN_ROWS && K <= PAIRS_MAX_K && library_us(M, N, K) >= 1.2 * eight_waves_us(M, N, K);
 }
 
+// us of the partial sums of a slice of slice_k values, the coefficients as for `kinds` but of this product (380 sizes of 896 to 20,000
+// k-values in 1 to 8 slices: off by 5 to 7 % in the mean square) and, for every slice after the first, of what the reader of the sums pays
+static double sums_us(int kind, int M, int N, int slices, int slice_k) {
+  static const double sums[TILE_KINDS][6] = {
+      {1.71, 9.86, 22.96, 10.23, 15.63, 6.15}, {3.43, 8.36, 21.49, 8.44, 15.09, 4.84}, {}, {}, {2.80, 7.93, 22.05, 9.30, 15.29, 4.32},
+      {2.78, 6.62, 18.46, 7.16, 11.93, 5.03}, {1.58, 6.75, 18.74, 7.87, 11.78, 5.63}, {1.86, 4.34, 15.21, 5.42, 10.92, 3.72}};
+  const double* c = sums[kind];
+  const long long tiles = (long long)((N + kinds[kind].bn - 1) / kinds[kind].bn) * ((M + kinds[kind].bm - 1) / kinds[kind].bm) * slices;
+  const long long per = (tiles + 7) / 8, rest = per % 32;
+  const double kk = slice_k / 1000.0;
+  const double last = rest == 0 ? 0.0 : c[3] + kk * (c[4] + c[5] * (double)rest / 32);
+  return c[0] + (double)(per / 32) * (c[1] + c[2] * kk) + last + (slices > 1 ? 0.5 + 1.2e-6 * (double)M * (double)N * (slices - 1) : 0.0);
+}
+
+#define SUMS_MIN_ROWS 257
+#define SUMS_MIN_N 896          // (lower weights were not measured)
+#define SUMS_MIN_K 8192
+#define SUMS_MAX_SLICES 8
+#define SUMS_MAX_BYTES (512ll << 20)      // of partial sums
+
+// Whether the product of M rows with a weight [N, K], whose reader adds partial sums, is faster here than by the library, by which
+// tile and in how many slices: slices << 8 | tile (1 slice: the plain product in bfloat16), 0: it is not.  The library's time over
+// this one's, with the norm that adds the sums (100 sizes drawn over 129 to 8,192 rows, 896 to 8,192 weight rows, 8,192 to 20,000
+// k-values and 40 of four models' down; geometric mean and worst), by the number of tiles of 256 x 256:
+//   up to 128 tiles (the library takes slices of K): 257 to 600 rows 1.30 and 0.88, more 1.20 and 0.90, up to 256 rows 1.14 and 0.68; where
+//   the library's slices fill a round to 85 % or more 1.1 and, as 2,048 rows of 3,584 x 18,944 behind other products, 0.96.  (And the batched
+//   product costs the host 15 us more: 24 arriving requests at the 3B shape 244.8 -> 234.8 ms from 257 rows on, 239.8 from 800.)
+//   129 to 256 tiles, which are one round of the library's: 0.94     more, whose last round is at most 85 % full on the whole: 1.22 and
+//   0.81, fuller ones 0.97            weights of 4,096 to 8,192 k-values, of multiples of 512 rows: 0.94
+// `library_slices`: the slices that the library would take.
+extern "C" int ifx_gemm_tiles_sums_plan(int M, int N, int K, int library_slices) {
+  if (M < SUMS_MIN_ROWS || N < SUMS_MIN_N || K < SUMS_MIN_K || K > 1 << 20 || N > 1 << 20 || N % 8 || K % 8) return 0;
+  const long long tiles = (long long)((N + 255) / 256) * ((M + 255) / 256), library = tiles * library_slices;
+  if ((tiles > 128 && tiles <= 256) || library >= 0.85 * 256 * ((library + 255) / 256)) return 0;
+  int best = 0;
+  double least = 0;
+  for (int s = 1; s <= SUMS_MAX_SLICES; ++s) {
+    const int slice_k = ((K + s - 1) / s + 63) / 64 * 64;
+    if ((K + slice_k - 1) / slice_k != s || (s > 1 && (long long)s * M * N * 4 > SUMS_MAX_BYTES)) continue;
+    for (int kind = 0; kind < TILE_KINDS; ++kind) {
+      if (eight_waves(kind)) continue;
+      const double us = sums_us(kind, M, N, s, slice_k);
+      if (best == 0 || us < least) best = s << 8 | kind, least = us;
+    }
+  }
+  return best;
+}
+
 template <int FN, int FM>
 static void launch_waves(const TilesArgs& a, int out, hipStream_t s) {
   typedef WaveTiles<FN, FM> P;
-  const int tiles = ((a.N + P::BN - 1) / P::BN) * ((a.M + P::BM - 1) / P::BM), blocks = tiles < 256 ? (tiles + 7) / 8 * 8 : 256;
+  const int tiles = ((a.N + P::BN - 1) / P::BN) * ((a.M + P::BM - 1) / P::BM) * a.slices, blocks = tiles < 256 ? (tiles + 7) / 8 * 8 : 256;
   if (out == OUT_PAIRS) hipLaunchKernelGGL((tiles_kernel<FN, FM, OUT_PAIRS>), dim3(blocks), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((tiles_kernel<FN, FM, OUT_ACT>), dim3(blocks), dim3(256), 0, s, a);
+  else if (out == OUT_ACT) hipLaunchKernelGGL((tiles_kernel<FN, FM, OUT_ACT>), dim3(blocks), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((tiles_kernel<FN, FM, OUT_SUMS>), dim3(blocks), dim3(256), 0, s, a);
 }
 
 template <int BN, int BM, int WN, int WM, int PER_CU>
@@ -266,21 +356,7 @@ static void launch_pairs(const TilesArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((pairs_kernel<BN, BM, WN, WM, PER_CU>), dim3(blocks), dim3(64 * (BN / WN) * (BM / WM)), 0, s, a);
 }
 
-// x, w, with OUT_ACT the result: on 16 bytes.  tile: one of the kinds above, or -1 for the one that choose_tile takes
-extern "C" int ifx_gemm_tiles(const void* x, const void* w, void* result, int M, int N, int K, int out, int act, float limit, int tile, void* stream) {
-  IFX_REQUIRE(out == OUT_PAIRS || out == OUT_ACT, "gemm_tiles: result %d", out);
-  IFX_REQUIRE(M >= 0 && N > 0 && N % (out == OUT_PAIRS ? 4 : 2) == 0 && K > 0 && K % 8 == 0 && K <= 1 << 20 && N <= 1 << 22,
-              "gemm_tiles: N=%d must be a multiple of %d, K=%d of 8", N, out == OUT_PAIRS ? 4 : 2, K);
-  if (out == OUT_PAIRS)
-    IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f), "gated activation: unknown kind %d (limit %g)", act, (double)limit);
-  else
-    IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || act == ACT_RELU_SQUARED, "activation: unknown kind %d", act);
-  IFX_REQUIRE(((size_t)x | (size_t)w | (size_t)result) % 16 == 0, "gemm_tiles: x, the weight and the result must lie on 16 bytes");
-  if (M == 0) return 0;
-  const TilesArgs a{(const bf16_t*)x, (const bf16_t*)w, (bf16_t*)result, M, N, K, act, limit};
-  hipStream_t s = (hipStream_t)stream;
-  const int kind = tile < 0 ? choose_tile(M, N, K, out) : tile;
-  IFX_REQUIRE(kind < TILE_KINDS && !(out == OUT_ACT && eight_waves(kind)), "gemm_tiles: tile %d", tile);
+static void launch_kind(const TilesArgs& a, int kind, int out, hipStream_t s) {
   switch (kind) {
     case TILE_256_256: launch_waves<8, 8>(a, out, s); break;
     case TILE_320_192: launch_waves<10, 6>(a, out, s); break;
@@ -291,5 +367,36 @@ extern "C" int ifx_gemm_tiles(const void* x, const void* w, void* result, int M,
     case TILE_192_256: launch_waves<6, 8>(a, out, s); break;
     case TILE_256_128: launch_waves<8, 4>(a, out, s); break;
   }
+}
+
+// x, w, with OUT_ACT the result: on 16 bytes.  tile: one of the kinds above, or -1 for the one that choose_tile takes.
+// OUT_ACT also takes ACT_NONE: the plain product.
+extern "C" int ifx_gemm_tiles(const void* x, const void* w, void* result, int M, int N, int K, int out, int act, float limit, int tile, void* stream) {
+  IFX_REQUIRE(out == OUT_PAIRS || out == OUT_ACT, "gemm_tiles: result %d", out);
+  IFX_REQUIRE(M >= 0 && N > 0 && N % (out == OUT_PAIRS ? 4 : 2) == 0 && K > 0 && K % 8 == 0 && K <= 1 << 20 && N <= 1 << 22,
+              "gemm_tiles: N=%d must be a multiple of %d, K=%d of 8", N, out == OUT_PAIRS ? 4 : 2, K);
+  if (out == OUT_PAIRS)
+    IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f), "gated activation: unknown kind %d (limit %g)", act, (double)limit);
+  else
+    IFX_REQUIRE(act == ACT_SILU || act == ACT_GELU_TANH || act == ACT_RELU_SQUARED || act == ACT_NONE, "activation: unknown kind %d", act);
+  IFX_REQUIRE(((size_t)x | (size_t)w | (size_t)result) % 16 == 0, "gemm_tiles: x, the weight and the result must lie on 16 bytes");
+  if (M == 0) return 0;
+  const TilesArgs a{(const bf16_t*)x, (const bf16_t*)w, result, M, N, K, act, limit, 1, K};
+  const int kind = tile < 0 ? choose_tile(M, N, K, out) : tile;
+  IFX_REQUIRE(kind < TILE_KINDS && !(out == OUT_ACT && eight_waves(kind)), "gemm_tiles: tile %d", tile);
+  launch_kind(a, kind, out, (hipStream_t)stream);
+  IFX_LAUNCH_CHECK();
+}
+
+// parts [slices][M][N] in float: x times w transposed over slices of slice_k values of K (a multiple of 64); x, w, parts on 16 bytes
+extern "C" int ifx_gemm_tiles_sums(const void* x, const void* w, float* parts, int M, int N, int K, int slices, int slice_k, int tile, void* stream) {
+  IFX_REQUIRE(M >= 0 && N > 0 && N % 4 == 0 && K > 0 && K % 8 == 0 && K <= 1 << 20 && N <= 1 << 20, "gemm_tiles_sums: N=%d must be a multiple of 4, K=%d of 8", N, K);
+  IFX_REQUIRE(slices > 0 && slice_k > 0 && slice_k % 64 == 0 && (long long)slices * slice_k >= K && (long long)(slices - 1) * slice_k < K,
+              "gemm_tiles_sums: %d slices of %d values of K=%d", slices, slice_k, K);
+  IFX_REQUIRE(((size_t)x | (size_t)w | (size_t)parts) % 16 == 0, "gemm_tiles_sums: x, the weight and the result must lie on 16 bytes");
+  IFX_REQUIRE(tile >= 0 && tile < TILE_KINDS && !eight_waves(tile), "gemm_tiles_sums: tile %d", tile);
+  if (M == 0) return 0;
+  const TilesArgs a{(const bf16_t*)x, (const bf16_t*)w, parts, M, N, K, ACT_NONE, 0.f, slices, slice_k};
+  launch_kind(a, tile, OUT_SUMS, (hipStream_t)stream);
   IFX_LAUNCH_CHECK();
 }

@@ -29,6 +29,7 @@ ROPE_NONE, ROPE_SPLIT_HALF, ROPE_CONSECUTIVE = 0, 1, 2
 ACT_SILU, ACT_GELU_TANH = 0, 1          # gated activations of a feed-forward: act(gate) * up
 ACT_CLAMPED_SWISH = 2                   # ... and min(gate, L) sigmoid(1.702 min(gate, L)) (clamp(up, -L, L) + 1), which takes its limit L
 ACT_RELU_SQUARED = 3                    # max(x, 0)^2, for a feed-forward without a gate
+ACT_NONE = 4                            # the product as it is (of the products of many rows)
 PLAIN_ACTS = (ACT_SILU, ACT_GELU_TANH, ACT_RELU_SQUARED)
 _PLAIN_EPILOGUE = {ACT_RELU_SQUARED: 4, ACT_GELU_TANH: 5}     # the activations without a gate that the product for few rows has as an epilogue
 _GATED_EPILOGUE = {ACT_SILU: 1, ACT_GELU_TANH: 3}    # ... as the epilogue number of the streaming products
@@ -1368,6 +1369,11 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
         return staged_gemm(x, weight, out_dtype)
     if out_dtype == torch.float32:
         return torch.mm(x, weight.t(), out_dtype=torch.float32)
+    if keep_slices and not torch.cuda.tunable.is_enabled():          # (where the library has timed its kernels its choice is the better one)
+        plan = _tiles_sums_plan(M, weight.shape[0], K)
+        if plan and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0:
+            slices, tile = plan >> 8, plan & 255
+            return sums_tiles(x, weight, slices, -(-(-(-K // slices)) // 64) * 64, tile) if slices > 1 else act_tiles(x, weight, ACT_NONE, tile)
     if keep_slices:
         S = library_k_slices(M, weight.shape[0], K)
         if S > 1 and not torch.cuda.is_current_stream_capturing():
@@ -1376,6 +1382,12 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
             ws = weight.view(weight.shape[0], S, K // S).permute(1, 2, 0)
             return SliceSums(torch.bmm(xs, ws, out_dtype=torch.float32), out_dtype)
     return torch.matmul(x, weight.t())
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles_sums_plan(M: int, N: int, K: int) -> int:
+    """slices << 8 | tile of a product by slices of tiles whose partial sums the caller adds (1: the plain product), 0: the library's."""
+    return load_module("gemm_tiles").fn("ifx_gemm_tiles_sums_plan", (I, I, I, I))(M, N, K, library_k_slices(M, N, K))
 
 
 LIBRARY_SLICE_MIN_K = 2048      # k-values a slice of a library product keeps at least
@@ -1524,6 +1536,18 @@ def act_tiles(x: torch.Tensor, weight: torch.Tensor, act: int, tile: int = -1) -
     _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x.data_ptr(), weight.data_ptr(), out.data_ptr(),
           x.shape[0], N, K, 1, int(act), 0.0, int(tile), _stream())
     return out
+
+
+def sums_tiles(x: torch.Tensor, weight: torch.Tensor, slices: int, slice_k: int, tile: int) -> "SliceSums":
+    """bfloat16 x [M, K] times ``weight`` [N, K] transposed as ``SliceSums`` over ``slices`` of ``slice_k`` values of K (a multiple of
+    64), N a multiple of 4, K of 8, both on 16 bytes; ``tile``: one of the kernel's tiles by four waves."""
+    _check(weight, "weight", (None, None), torch.bfloat16)
+    N, K = weight.shape
+    _check(x, "x", (None, K), torch.bfloat16)
+    parts = torch.empty((slices, x.shape[0], N), dtype=torch.float32, device=x.device)
+    _call(load_module("gemm_tiles"), "ifx_gemm_tiles_sums", (P, P, P, I, I, I, I, I, I, P), x.data_ptr(), weight.data_ptr(), parts.data_ptr(),
+          x.shape[0], N, K, int(slices), int(slice_k), int(tile), _stream())
+    return SliceSums(parts, torch.bfloat16)
 
 
 _TILES_ARGS = (P, P, P, I, I, I, I, I, F, I, P)

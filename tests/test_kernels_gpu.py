@@ -764,6 +764,45 @@ def test_moe_few_with_a_shared_expert(T, top, E, K, ff, shared_ff, form):
         assert (a - b).abs().max() < 5 * 2.0 ** -8 * b.abs().max()
 
 
+@pytest.mark.parametrize("M,N,K,slices,slice_k", [(1, 4, 8, 1, 64), (129, 260, 64, 1, 64), (257, 100, 136, 3, 64), (300, 516, 1000, 2, 512), (513, 388, 2056, 3, 704),
+                                                  (700, 2052, 328, 1, 384), (130, 8, 4104, 8, 576), (2100, 772, 1032, 4, 320)])
+def test_tiles_products_as_partial_sums_and_plain(M, N, K, slices, slice_k):
+    """Rows, weight rows and k-values that end within a tile, a fragment and a step, slices whose last one is a piece of a step, more tiles
+    than workgroups: against 64 bits.  Sums of K products of bfloat16 in float: rounding errors of 2^-24 each, at most K of them, far
+    fewer in the mean square; the plain product is rounded to bfloat16 (2^-9) besides.  What lies beyond the result stays as it was."""
+    g = gen(2300 + M + N)
+    x, w = torch.randn(M, K, generator=g).to(BF16).to(DEV), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16).to(DEV)
+    parts = [x[:, s * slice_k:(s + 1) * slice_k].double() @ w[:, s * slice_k:(s + 1) * slice_k].double().t() for s in range(slices)]
+    for tile in (0, 1, 4, 5, 6, 7):
+        got = ops.sums_tiles(x, w, slices, slice_k, tile)
+        for a, b in zip(got.parts, parts):
+            assert (a.double() - b).abs().max() < K ** 0.5 * 2.0 ** -22
+        assert torch.equal(got.parts, ops.sums_tiles(x, w, slices, slice_k, 5).parts)          # (an element does not depend on its tile)
+        plain = ops.act_tiles(x, w, ops.ACT_NONE, tile).double()
+        assert ((plain - sum(parts)).abs() <= 2.0 ** -8 * sum(parts).abs() + K ** 0.5 * 2.0 ** -22).all()
+    with pytest.raises(ops.KernelError):
+        ops.sums_tiles(x, w, slices + 1, slice_k, 0)
+    with pytest.raises(ops.KernelError):
+        ops.sums_tiles(x, w, slices, slice_k, 2)
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(256, 1024, 8192, 0), (257, 896, 8192, 8), (300, 888, 8192, 0), (1000, 2048, 8200, 4), (1025, 904, 9000, 7), (6144, 3584, 8192, 1),
+                                          (2048, 3584, 18944, 0), (4500, 3584, 8192, 0), (1030, 2052, 8192, 0), (1030, 2048, 8184, 0)])
+def test_deep_products_of_many_rows_take_slices_of_tiles(M, N, K, slices):
+    """The sizes on both sides of the rule's lines, through ``linear``, against 64 bits (partial sums in float, or one rounding to
+    bfloat16, 2^-9)."""
+    assert ops._tiles_sums_plan(M, N, K) >> 8 == slices
+    g = gen(2330)
+    x, w = torch.randn(M, K, generator=g).to(BF16).to(DEV), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16).to(DEV)
+    got = ops.linear(x, w, keep_slices=True)
+    if slices > 1:
+        assert isinstance(got, ops.SliceSums) and got.parts.shape == (slices, M, N)
+    out = (got.sum(F32) if isinstance(got, ops.SliceSums) else got).double()
+    rows = torch.randperm(M, generator=g)[:64].to(DEV)
+    want = x[rows].double() @ w.double().t()
+    assert ((out[rows] - want).abs() <= 2.0 ** -8 * want.abs() + K ** 0.5 * 2.0 ** -22).all()
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
