@@ -41,6 +41,25 @@ __device__ __forceinline__ f32x4 load4(const T* __restrict__ row, int k, int K) 
   return v;
 }
 
+// ---- the results ---------------------------------------------------------------------------------------------------------
+// Either the sums as they are, C [M][N], or, with an activation, weight rows of gate and up in turn and C [M][N / 2] = act(gate) * up:
+// neighbouring lanes hold neighbouring columns, the even one stores for both.  Called by all lanes of a wave that hold a sum (an even
+// number of them); `in`: whether this lane's is within C.  The formula is that of the kernel that would read the sums back
+// (swiglu, 4.9 us a launch of few rows), so the bits are the same.
+struct Gated {
+  int act;                  // -1: none
+  float limit;
+};
+template <typename TO>
+__device__ __forceinline__ void put(TO* __restrict__ C, int m, int n, int N, float v, bool in, const Gated& g) {
+  if (g.act < 0) {
+    if (in) C[(size_t)m * N + n] = from_f<TO>(v);
+    return;
+  }
+  const float up = __shfl_down(v, 1);
+  if (in && n % 2 == 0) C[(size_t)m * (N / 2) + n / 2] = from_f<TO>(gated_act(v, up, g.act, g.limit));
+}
+
 // ---- few rows: the weight is streamed once -----------------------------------------------------------------------------
 // A workgroup takes NT x 16 weight rows and MT x 16 rows of A; its sixteen waves take a slice of K each and meet in LDS.
 // Bound by the weight's bytes where N is large (5.6 TB/s at 151,936 x 896) and by the few workgroups where it is not (56 for
@@ -50,7 +69,7 @@ __device__ __forceinline__ f32x4 load4(const T* __restrict__ row, int k, int K) 
 template <typename TA, typename TO, int MT, int NT, int STEPS, bool VEC>
 __global__ __launch_bounds__(1024) void gemm_f32_few_kernel(const TA* __restrict__ A, const float* __restrict__ W,
                                                            const float* __restrict__ bias, TO* __restrict__ C,
-                                                           int M, int N, int K) {
+                                                           int M, int N, int K, Gated gated) {
   __shared__ float part[N_SLICES][MT * NT][256];
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const int i = lane % 16, q = lane / 16;
@@ -108,12 +127,11 @@ __global__ __launch_bounds__(1024) void gemm_f32_few_kernel(const TA* __restrict
   __syncthreads();
   for (int e = threadIdx.x; e < MT * NT * 256; e += 1024) {
     const int t = e / 256, at = e % 256, m = m0 + 16 * (t / NT) + at / 16, n = n0 + 16 * (t % NT) + at % 16;
-    if (m >= M || n >= N) continue;
     float v = part[0][t][at];
 #pragma unroll
     for (int s = 1; s < N_SLICES; ++s) v += part[s][t][at];
-    if (bias) v += bias[n];
-    C[(size_t)m * N + n] = from_f<TO>(v);
+    if (bias && n < N) v += bias[n];
+    put(C, m, n, N, v, m < M && n < N, gated);
   }
 }
 
@@ -130,7 +148,7 @@ __global__ __launch_bounds__(1024) void gemm_f32_few_kernel(const TA* __restrict
 template <typename TA, typename TO, int SP, int STEPS, bool VEC>
 __global__ __launch_bounds__(64 * N_SLICES / SP) void gemm_f32_narrow_kernel(const TA* __restrict__ A, const float* __restrict__ W,
                                                                              const float* __restrict__ bias, TO* __restrict__ C,
-                                                                             int M, int N, int K) {
+                                                                             int M, int N, int K, Gated gated) {
   constexpr int B = 16 / SP;
   __shared__ float part[N_SLICES][B * B];
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
@@ -160,12 +178,12 @@ __global__ __launch_bounds__(64 * N_SLICES / SP) void gemm_f32_narrow_kernel(con
     if ((4 * q + j) / B == i / B) part[slice][(4 * q + j) % B * B + r] = acc[j];
   __syncthreads();
   const int e = threadIdx.x, m = e / B, n = n0 + e % B;
-  if (e < B * B && m < M && n < N) {
+  if (e < B * B) {
     float v = part[0][e];
 #pragma unroll
     for (int s = 1; s < N_SLICES; ++s) v += part[s][e];
-    if (bias) v += bias[n];
-    C[(size_t)m * N + n] = from_f<TO>(v);
+    if (bias && n < N) v += bias[n];
+    put(C, m, n, N, v, m < M && n < N, gated);
   }
 }
 
@@ -177,7 +195,7 @@ __global__ __launch_bounds__(64 * N_SLICES / SP) void gemm_f32_narrow_kernel(con
 template <typename TA, typename TO, int TM, int TN, bool VEC>
 __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const TA* __restrict__ A, const float* __restrict__ W,
                                                              const float* __restrict__ bias, TO* __restrict__ C,
-                                                             int M, int N, int K) {
+                                                             int M, int N, int K, Gated gated) {
   constexpr int BM = 32 * TM, BN = 32 * TN, BK = 32;
   __shared__ f32x4 As[BM][BK / 4], Ws[BN][BK / 4];
   const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
@@ -247,12 +265,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const TA* __restric
 #pragma unroll
     for (int n = 0; n < TN; ++n) {
       const int col = n0 + wn + 16 * n + i;
-      if (col >= N) continue;
-      const float b = bias ? bias[col] : 0.f;
+      const float b = bias && col < N ? bias[col] : 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm + 16 * m + 4 * q + r;
-        if (row < M) C[(size_t)row * N + col] = from_f<TO>(bias ? total[m][n][r] + b : total[m][n][r]);
+        put(C, row, col, N, bias ? total[m][n][r] + b : total[m][n][r], row < M && col < N, gated);
       }
     }
 }
@@ -266,19 +283,19 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const TA* __restric
 // and 105), 410 at one row of 151,936 x 896 (97: 5.6 TB/s); 2,048 rows of 22,016 x 2,048 run at 103 TFLOP/s.  Errors against 64
 // bits fell to a third (5.4e-7 to 2.0e-7 at K = 896, 1.9e-6 to 6.6e-7 at 11,008): shorter chains.
 template <typename TA, typename TO, bool VEC>
-static void launch(const TA* A, const float* W, const float* bias, TO* C, int M, int N, int K, hipStream_t s) {
+static void launch(const TA* A, const float* W, const float* bias, TO* C, int M, int N, int K, Gated gated, hipStream_t s) {
   auto blocks = [&](int m, int n) { return (double)((M + m - 1) / m) * ((N + n - 1) / n); };
   auto rounds = [&](int m, int n) { return (double)(long long)((blocks(m, n) + 255.0) / 256.0); };
   const double t11 = 5.6 * rounds(16, 16), t21 = 7.5 * rounds(32, 16), t22 = 10.3 * rounds(32, 32);
   const double b64 = blocks(64, 64), tiles = b64 <= 256.0 ? 31.0 : (b64 < 530.0 ? 44.0 : 0.083 * b64);
 #define FEW(MT, NT)                                                                                              \
   hipLaunchKernelGGL((gemm_f32_few_kernel<TA, TO, MT, NT, 4, VEC>),                                              \
-                     dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K)
+                     dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K, gated)
   // (a grid has at most 65,535 rows: millions of rows by a handful of columns are the tile kernel's, whose limit the caller checks)
   const bool in16 = (M + 15) / 16 <= 65535, in32 = (M + 31) / 32 <= 65535;
 #define NARROW(SP, STEPS)                                                                                        \
   hipLaunchKernelGGL((gemm_f32_narrow_kernel<TA, TO, SP, STEPS, VEC>), dim3((N + 16 / SP - 1) / (16 / SP)),      \
-                     dim3(64 * N_SLICES / SP), 0, s, A, W, bias, C, M, N, K)
+                     dim3(64 * N_SLICES / SP), 0, s, A, W, bias, C, M, N, K, gated)
   const double b16 = blocks(16, 16), full16 = 256.0 * rounds(16, 16);
   if (M <= 4 && N <= 1024) NARROW(4, 4);
   else if ((M <= 8 && N <= 2048) || (M <= 4 && b16 > 256.0 && b16 < 0.85 * full16)) NARROW(2, 4);
@@ -286,22 +303,27 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
   else if (in32 && t21 <= t22 && t21 <= tiles) FEW(2, 1);
   else if (in32 && t22 <= tiles) FEW(2, 2);
   else
-    hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K);
+    hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K, gated);
 #undef FEW
 #undef NARROW
 }
 
+// act: -1, or the activation of gate and up rows in turn (N even, no bias, C [M][N / 2] of A's type)
 extern "C" int ifx_gemm_f32(const void* A, int a_dtype, const float* W, const float* bias, void* C,
-                            int c_dtype, int M, int N, int K, void* stream) {
+                            int c_dtype, int M, int N, int K, int act, float limit, void* stream) {
   IFX_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
+  IFX_REQUIRE(act < 0 || (N % 2 == 0 && !bias && a_dtype == DT_F32 && c_dtype == DT_F32 &&
+                          (act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f))),
+              "gemm_f32: gated activation %d (limit %g) of %d columns", act, (double)limit, N);
+  const Gated gated{act, limit};
   if (M == 0) return 0;
   IFX_REQUIRE((M + 63) / 64 <= 65535, "gemm_f32: M=%d too large for one launch", M);
   hipStream_t s = (hipStream_t)stream;
   const bool vec = K % 4 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)A % (a_dtype == DT_BF16 ? 8 : 16) == 0;
 #define LAUNCH(TA, TO)                                                              \
   do {                                                                              \
-    if (vec) launch<TA, TO, true>((const TA*)A, W, bias, (TO*)C, M, N, K, s);       \
-    else launch<TA, TO, false>((const TA*)A, W, bias, (TO*)C, M, N, K, s);          \
+    if (vec) launch<TA, TO, true>((const TA*)A, W, bias, (TO*)C, M, N, K, gated, s);       \
+    else launch<TA, TO, false>((const TA*)A, W, bias, (TO*)C, M, N, K, gated, s);          \
   } while (0)
   if (a_dtype == DT_F32 && c_dtype == DT_F32) LAUNCH(float, float);
   else if (a_dtype == DT_BF16 && c_dtype == DT_BF16) LAUNCH(bf16_t, bf16_t);

@@ -777,8 +777,9 @@ def moe_few(h: torch.Tensor, router, gate_up: torch.Tensor, down: torch.Tensor, 
 
 # ----------------------------------------------------------------------------------------
 def gemm_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-             out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """x [M, K] (float32 or bfloat16) times float32 ``weight`` [N, K] transposed, true 32-bit math."""
+             out_dtype: Optional[torch.dtype] = None, gated: Optional[int] = None, limit: float = 0.0) -> torch.Tensor:
+    """x [M, K] (float32 or bfloat16) times float32 ``weight`` [N, K] transposed, true 32-bit math.  ``gated`` (float32 x, no bias): the
+    activation of weight rows of gate and up in turn, the result [M, N / 2] (``limit``: ACT_CLAMPED_SWISH's)."""
     _check(x, "x", (None, None))
     M, K = x.shape
     _check(weight, "weight", (None, K), torch.float32)
@@ -786,9 +787,9 @@ def gemm_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     if bias is not None:
         _check(bias, "bias", (N,), torch.float32)
     out_dtype = out_dtype or x.dtype
-    out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    _call(load_module("gemm_f32"), "ifx_gemm_f32", (P, I, P, P, P, I, I, I, I, P),
-          x.data_ptr(), _dt(x), weight.data_ptr(), _ptr(bias), out.data_ptr(), _DT[out_dtype], M, N, K, _stream())
+    out = torch.empty((M, N if gated is None else N // 2), dtype=out_dtype, device=x.device)
+    _call(load_module("gemm_f32"), "ifx_gemm_f32", (P, I, P, P, P, I, I, I, I, I, F, P), x.data_ptr(), _dt(x), weight.data_ptr(), _ptr(bias),
+          out.data_ptr(), _DT[out_dtype], M, N, K, -1 if gated is None else int(gated), float(limit), _stream())
     return out
 
 
@@ -1570,6 +1571,8 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
         whole = x.contiguous() if columns else x
         if whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
             return swiglu_tiles(whole, rows, act, limit)
+    if rows.dtype == torch.float32 and x.dtype == torch.float32 and not isinstance(x, ScaledRows):
+        return gemm_f32(x.contiguous() if columns else x, rows, gated=act, limit=limit)
     if act == ACT_CLAMPED_SWISH:
         return swiglu(linear(x, weight_pairs), interleaved=True, act=act, limit=limit)
     if rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16:
