@@ -433,6 +433,24 @@ def test_attention_plain_one_wave_and_four_give_the_same_bits(dtype, past, form)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("d,dv,P,rows", [(8, 8, 8, 3), (64, 64, 16, 4), (56, 64, 24, 129), (64, 65, 16, 5), (40, 128, 8, 64), (64, 128, 16, 65)])
+@pytest.mark.parametrize("form", ["plain", "window", "differential"])
+def test_attention_plain_whole_tiles_at_once_give_the_same_bits(dtype, d, dv, P, rows, form):
+    """Keys and values asked for at once (up to 64 and 128 elements, up to 512 and 256 rows and heads) against a wave to a row and head,
+    which asks for them one after the other: windows that begin within eight keys of a page, first keys, two maps."""
+    nH, nKV, past = 4, 2, 171
+    g = gen(1785 + d + dv)
+    pages = -(-(past + rows) // P)
+    q, kc, vc = (torch.randn(*s, generator=g).to(dtype).to(DEV) for s in ((rows, nH, d), (pages, nKV, P, d), (pages, nKV, dv, P)))
+    more = {"plain": {}, "window": dict(keep_first=11, sink=0.3), "differential": dict(differential=(0.4, 0.6, 1e-5))}[form]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    args = (q, kc, vc, i32([0] * rows), i32(list(range(past, past + rows))), torch.randperm(pages, generator=g).to(torch.int32)[None].to(DEV),
+            77 if form == "window" else None, 0.3)
+    one, four = (ops.attention_plain(*args, **more, row_waves=w) for w in (1, 4))
+    assert torch.equal(one, four)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("low,window,sink", [((64, 128), None, None), ((128, 256), None, None), ((0, 64), None, 0.5), ((0, 300), None, -1.0),
                                              ((192, 256), 130, None), ((64, 320), None, None), ((128, 192), 150, 0.0)])
 def test_attention_plain_tiles_whose_scores_are_all_minus_infinity(dtype, low, window, sink):
