@@ -12,7 +12,7 @@
 // Rows of x lie in a slot as in product_tiles.h (two halves of 64 k-values, piece p of row r at p ^ (r & 7) ^ (r >> 3 & 1)), row tiles
 // of W as they are stored (a k-tile is a wave's fragment in the order of its lanes; of tiles of fewer than 16 rows the lanes of the
 // other rows load zeros).  With four tiles of x (33-64 rows) a wave multiplies one of them with all row tiles; with two (17-32
-// rows) two waves share one, half of the step's k-tiles each, and add their sums through LDS.
+// rows) two waves share one, half of the step's k-tiles each, with one (9-16 rows) all four, a k-tile each, and add their sums through LDS.
 //
 // With more than one slice of K the slices write float partial sums, added in slice order by whoever reads them.
 #include "product_tiles.h"
@@ -35,7 +35,7 @@ struct RingArgs {
 template <int NTW, int MT>
 struct Ring {
   static constexpr int STAGE = (NTW + MT) * 4096, LOADS = NTW + MT;      // bytes of a step; direct loads of a wave and a step
-  static constexpr int SLOTS = 160 * 1024 / STAGE < 5 ? 160 * 1024 / STAGE : 5;
+  static constexpr int MOST = MT == 1 ? 8 : 5, SLOTS = 160 * 1024 / STAGE < MOST ? 160 * 1024 / STAGE : MOST;
   static_assert(SLOTS >= 3 && (SLOTS - 2) * LOADS < 64, "ring");
 };
 
@@ -102,8 +102,8 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(RingArgs a) {
     for (int i = 0; i < MT; ++i)
       ring_load(x, last && at * 128 + xk[i] >= a.K ? TILE_NO_ROW : xo[i], at * 256, to + NTW * 4096 + (wid * MT + i) * 1024);
   };
-  constexpr int KT0_STEP = MT == 4 ? 4 : 2;          // k-tiles of a step to a wave
-  const int m_tile = MT == 4 ? wid : wid % 2, kt0 = MT == 4 ? 0 : wid / 2 * 2;
+  constexpr int KT0_STEP = MT;          // k-tiles of a step to a wave
+  const int m_tile = wid % MT, kt0 = wid / MT * MT;
   tile_floatx4 acc[NTW];
 #pragma unroll
   for (int j = 0; j < NTW; ++j) acc[j] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
@@ -130,15 +130,17 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(RingArgs a) {
     slot = slot == R::SLOTS - 1 ? 0 : slot + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");          // (the loads beyond the end; all have read the last step)
-  if (MT == 2) {
+  if (MT < 4) {
     tile_floatx4* shares = (tile_floatx4*)lds;
-    if (wid >= 2)
+    if (wid >= MT)
 #pragma unroll
-      for (int j = 0; j < NTW; ++j) shares[((wid - 2) * NTW + j) * 64 + lane] = acc[j];
+      for (int j = 0; j < NTW; ++j) shares[((wid - MT) * NTW + j) * 64 + lane] = acc[j];
     __syncthreads();
-    if (wid >= 2) return;
+    if (wid >= MT) return;
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) acc[j] += shares[(wid * NTW + j) * 64 + lane];
+    for (int k = 0; k < 4 / MT - 1; ++k)
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) acc[j] += shares[((k * MT + wid) * NTW + j) * 64 + lane];
   }
   // acc[j][r] = out[m = 16 m_tile + col][n = tile_rows (row tile of the weight) + 4 g + r], for 4 g + r < tile_rows
   const int m = 16 * m_tile + col, held = min(4, a.tile_rows - 4 * g);      // (held: even, may be <= 0)
@@ -162,7 +164,10 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(RingArgs a) {
         for (int r = 0; r < 4; ++r)
           if (r < held && n0 + r < a.N) dst[r] = acc[j][r];
       }
-    } else if (EPI == 0) {
+    } else if (EPI == 0 || EPI >= 4) {
+      if (EPI >= 4)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j][r] = plain_act(acc[j][r], EPI == 4 ? ACT_RELU_SQUARED : ACT_GELU_TANH);
       TO* dst = (TO*)a.out + (size_t)m * a.N + n0;
       if (whole) {
         store4(dst, acc[j]);
@@ -190,6 +195,8 @@ static int launch_ring(const RingArgs& a, int out_dtype, int slices, int epi, hi
 #define GO(TO_, EPI_) hipLaunchKernelGGL((ring_gemm_kernel<NTW, MT, TO_, EPI_>), grid, dim3(256), 0, s, a)
   if (epi == 1) GO(bf16_t, 1);
   else if (epi == 3) GO(bf16_t, 3);
+  else if (epi == 4 && MT == 1) GO(bf16_t, (MT == 1 ? 4 : 0));
+  else if (epi == 5 && MT == 1) GO(bf16_t, (MT == 1 ? 5 : 0));
   else if (out_dtype == DT_BF16) GO(bf16_t, 0);
   else GO(float, 0);
 #undef GO
@@ -206,7 +213,7 @@ extern "C" int ifx_ring_gemm(const void* x, const void* w, void* out, int out_dt
   IFX_REQUIRE(row_tiles >= 1 && row_tiles <= 8 && slices >= 1 && steps >= 1, "ring_gemm: %d row tiles, %d slices of %d steps", row_tiles, slices, steps);
   const int all = (K + 127) / 128;
   IFX_REQUIRE((all + steps - 1) / steps == slices, "ring_gemm: %d steps do not cut into %d slices of %d", all, slices, steps);
-  IFX_REQUIRE(epi == 0 || ((epi == 1 || epi == 3) && N % 2 == 0 && !order && slices == 1 && out_dtype == DT_BF16), "ring_gemm: epilogue %d with N=%d, %d slices", epi, N, slices);
+  IFX_REQUIRE(epi == 0 || ((epi == 4 || epi == 5) && M <= 16 && !order && slices == 1 && out_dtype == DT_BF16) || ((epi == 1 || epi == 3) && N % 2 == 0 && !order && slices == 1 && out_dtype == DT_BF16), "ring_gemm: epilogue %d with N=%d, %d slices", epi, N, slices);
   IFX_REQUIRE(slices == 1 ? out != nullptr : part != nullptr, "ring_gemm: no result");
   IFX_REQUIRE(out_dtype == DT_BF16 || out_dtype == DT_F32, "ring_gemm: unknown out dtype %d", out_dtype);
   IFX_REQUIRE((size_t)x % 16 == 0, "ring_gemm: x must lie on 16 bytes");
@@ -214,7 +221,7 @@ extern "C" int ifx_ring_gemm(const void* x, const void* w, void* out, int out_dt
   if (M == 0) return 0;
   const RingArgs a{(const bf16_t*)x, (const bf16_t*)w, out, part, M, N, K, (N + tile_rows - 1) / tile_rows, tile_rows, steps, order};
   hipStream_t s = (hipStream_t)stream;
-#define CASE(NTW_) case NTW_: return M <= 32 ? launch_ring<NTW_, 2>(a, out_dtype, slices, epi, s) : launch_ring<NTW_, 4>(a, out_dtype, slices, epi, s)
+#define CASE(NTW_) case NTW_: return M <= 16 ? launch_ring<NTW_, 1>(a, out_dtype, slices, epi, s) : M <= 32 ? launch_ring<NTW_, 2>(a, out_dtype, slices, epi, s) : launch_ring<NTW_, 4>(a, out_dtype, slices, epi, s)
   switch (row_tiles) {
     CASE(1); CASE(2); CASE(3); CASE(4); CASE(5); CASE(6); CASE(7); CASE(8);
   }

@@ -1201,10 +1201,12 @@ def wide_gemm(x, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, 
 
 
 def ring_gemm(x: torch.Tensor, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, row_tiles: int = 0, slices: int = 0,
-              swiglu_pairs: bool = False, keep_slices: bool = False, act: int = ACT_SILU):
+              swiglu_pairs: bool = False, keep_slices: bool = False, act: int = ACT_SILU, plain_act: Optional[int] = None):
     """bfloat16 x [M <= 64, K] times ``weight`` transposed from its tiled copy, both through a ring of slots in LDS.  ``row_tiles`` (1 to 8)
-    of the weight to a workgroup and ``slices`` of K: 0 chooses (``ring_plan``); ``keep_slices`` and
-    the epilogue as for ``wide_gemm``."""
+    of the weight to a workgroup and ``slices`` of K: 0 chooses (``ring_plan``); ``keep_slices`` and the gated epilogue as for
+    ``wide_gemm``, ``plain_act`` (up to 16 rows) as for ``skinny_gemm``."""
+    if plain_act is not None and (plain_act not in _PLAIN_EPILOGUE or swiglu_pairs or weight.order is not None or out_dtype != torch.bfloat16 or x.shape[0] > 16):
+        raise KernelError(f"ring_gemm: activation {plain_act} is no epilogue of this product")
     _check(x, "x", (None, None), torch.bfloat16)
     M, K = x.shape
     N = weight.rows.shape[0]
@@ -1214,13 +1216,14 @@ def ring_gemm(x: torch.Tensor, weight: LinearWeight, out_dtype: torch.dtype = to
         raise KernelError("ring_gemm: gate/up pairs need an even number of weight rows in their natural order")
     if _tiled_size(N, K, weight.tile_rows) != weight.tiled.numel():
         raise KernelError(f"ring_gemm: the copy is not that of a [{N}, {K}] weight in tiles of {weight.tile_rows} rows")
-    row_tiles, steps = ring_plan(M, N, K, weight.tile_rows, swiglu_pairs, row_tiles, slices)
+    row_tiles, steps = ring_plan(M, N, K, weight.tile_rows, swiglu_pairs or plain_act is not None or slices == 1, row_tiles, slices)
     n_slices = -(-(-(-K // 128)) // steps)
     part = torch.empty((n_slices, M, N), dtype=torch.float32, device=x.device) if n_slices > 1 else None
     out = None if n_slices > 1 else torch.empty((M, N // 2 if swiglu_pairs else N), dtype=out_dtype, device=x.device)
     _call(load_module("gemm_ring"), "ifx_ring_gemm", (P, P, P, I, P, I, I, I, I, I, I, I, P, I, P),
           x.data_ptr(), weight.tiled.data_ptr(), _ptr(out), _DT[out_dtype], _ptr(part), M, N, K, row_tiles, n_slices, steps,
-          _GATED_EPILOGUE[act] if swiglu_pairs else 0, _ptr(weight.order), weight.tile_rows, _stream())
+          _GATED_EPILOGUE[act] if swiglu_pairs else (_PLAIN_EPILOGUE[plain_act] if plain_act is not None else 0), _ptr(weight.order),
+          weight.tile_rows, _stream())
     if n_slices == 1:
         return out
     sums = SliceSums(part, out_dtype)
@@ -1254,6 +1257,31 @@ def ring_takes(M: int, N: int, K: int, tile_rows: int, one_slice: bool) -> bool:
         896 x 4,864 6.6 : 5.7, 6.7 : 5.6, 9.0 : 7.3     1,536 x 8,960 10.5 : 8.9, 10.3 : 9.2, 13.6 : 11.8    1,024 x 1,024 4.3 : 3.7, 4.5 : 3.8, 5.6 : 4.4
         3,584 x 18,944 25.5 : 24.1, 25.6 : 24.5, 31.0 : 28.3     2,560 x 2,048 5.3 : 5.2, 5.8 : 5.6, 7.6 : 7.1, but 4,608 x 3,584 8.5 : 8.8, 9.1 : 9.2, 11.2 : 11.1."""
     return 17 <= M <= SKINNY_MAX_M and -(-N // tile_rows) <= (6 if one_slice else 1) * COMPUTE_UNITS and K < 1 << 20
+
+
+RING_FEW_MIN_ROWS = 9            # (up to 8 rows x is little to read beside W)
+RING_FEW_MIN_SLICED_K = 4096
+
+
+def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
+    """Whether 9 to 16 rows that would go to the product whose waves each read x from the L2 go to ``ring_gemm``, whose workgroups read it
+    once: 1 in one slice of K, 2 in slices whose sum the caller takes, 0 not (us at 9 and 16 rows, that product : this one)
+        one slice, weights of 2,049 to 12,288 rows and up to 4,096 k-values: 8,448 x 2,048 10.0, 12.9 : 9.1, 9.4     6,272 x 2,048 8.2, 9.4 : 7.5, 7.7
+            11,264 x 2,048 12.2, 12.4 : 11.1, 10.7     9,728 x 896 6.8, 7.1 : 6.6, 6.8     4,224 x 1,024 5.6, 5.9 : 5.5, 5.5     3,136 x 1,024 4.4, 4.8 :
+            4.2, 4.3, but 17,920 x 1,536 11.9, 13.9 : 12.9, 12.6, 22,016 x 2,048 16.8, 17.5 : 18.1, 17.7, 2,048 x 8,448 12.9, 14.4 : 13.6, 13.4
+        slices, a row tile for a compute unit at most and 4,096 k-values or more: 2,048 x 8,448 12.9, 14.4 : 10.0, 10.0     1,024 x 4,224 7.2, 8.6 : 5.5, 5.6
+            2,048 x 5,632 9.7, 10.9 : 8.1, 8.2     1,536 x 8,960 12.3, 13.7 : 8.8, 8.9     3,584 x 18,944 26.2, 32.8 : 24.5, 24.2, but 2,048 x 2,048 5.4, 5.8 :
+            5.3, 5.4 and a sum for the reader to form."""
+    if not isinstance(weight, LinearWeight) or isinstance(x, ScaledRows) or weight.tiled is None or weight.rows.dtype != torch.bfloat16 \
+            or x.dtype != torch.bfloat16 or not x.is_contiguous() or x.data_ptr() % 16:
+        return 0
+    (M, K), N = x.shape, weight.rows.shape[0]
+    if not RING_FEW_MIN_ROWS <= M <= 16 or K % 8 or K != weight.rows.shape[1] or _small_m_kernel(M, N, K, True) != "skinny":
+        return 0
+    tiles = -(-N // weight.tile_rows)
+    if keep_slices and tiles <= COMPUTE_UNITS and RING_FEW_MIN_SLICED_K <= K < 1 << 20:
+        return 2
+    return 1 if 2048 < N and tiles <= 3 * COMPUTE_UNITS and K <= RING_FEW_MIN_SLICED_K else 0
 
 
 def streams_weight(n_rows: int, weight) -> bool:
@@ -1363,6 +1391,9 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
     if columns and kind != "skinny":
         x = x.contiguous()
     if kind == "skinny":
+        ring = ring_takes_few(x, LinearWeight(weight, tiled, order, tile_rows), keep_slices and out_dtype == torch.bfloat16)
+        if ring:
+            return ring_gemm(x, LinearWeight(weight, tiled, order, tile_rows), out_dtype, slices=0 if ring == 2 else 1, keep_slices=True)
         return skinny_gemm(x, weight, out_dtype, tiled=tiled, order=order, tile_rows=tile_rows)
     if kind == "wide":
         return wide_gemm(x, LinearWeight(weight, tiled, order, tile_rows), out_dtype, keep_slices=keep_slices)
@@ -1578,6 +1609,8 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
     if rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16:
         kind = _small_m_kernel(M, rows.shape[0], K, tiled is not None)
         if kind == "skinny":
+            if ring_takes_few(x, weight_pairs) and rows.shape[0] % 2 == 0:
+                return ring_gemm(x, weight_pairs, swiglu_pairs=True, act=act)
             return skinny_gemm(x, rows, torch.bfloat16, swiglu_pairs=True, tiled=tiled, tile_rows=tile_rows, act=act)
         if columns:
             x = x.contiguous()
@@ -2261,6 +2294,8 @@ def linear_act(x, weight, act: int) -> torch.Tensor:
     if act in _PLAIN_EPILOGUE and isinstance(weight, LinearWeight) and weight.rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 \
             and weight.order is None and _small_m_kernel(x.shape[0], *weight.rows.shape, weight.tiled is not None) == "skinny" \
             and (not isinstance(x, ScaledRows) or takes_scaled_rows(x.shape[0], weight)):
+        if ring_takes_few(x, weight):
+            return ring_gemm(x, weight, plain_act=act)
         return skinny_gemm(x, weight.rows, tiled=weight.tiled, tile_rows=weight.tile_rows, plain_act=act)
     rows = weight.rows if isinstance(weight, LinearWeight) else weight
     if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and rows.dim() == 2 and x.dim() == 2 \

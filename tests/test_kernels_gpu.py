@@ -1667,6 +1667,33 @@ def test_ring_gemm(M, N, K, tile_rows, row_tiles, slices):
         assert torch.equal(ops.ring_gemm(x.to(DEV), shuffled, F32, row_tiles, slices), ops.ring_gemm(x.to(DEV), lw, F32, row_tiles, slices))
 
 
+@pytest.mark.parametrize("M", [9, 16])
+@pytest.mark.parametrize("N,K,route", [(2050, 72, 1), (2080, 1032, 1), (6272, 136, 1), (12288, 264, 1), (12290, 72, 0), (2048, 264, 0), (40, 4096, 2), (2048, 4104, 2),
+                                       (264, 12296, 2), (4096, 4096, 2), (4098, 4096, 1), (4098, 4104, 0)])
+def test_9_to_16_rows_go_to_the_ring(M, N, K, route):
+    """The weights on both sides of the rule's lines, through ``linear`` (with partial sums taken and not), gate/up and the activations
+    without a gate, against 64 bits: sums of K products of bfloat16 in float, rounded to bfloat16 (2^-9) but for partial sums."""
+    g = gen(2350 + N)
+    x, w = torch.randn(M, K, generator=g).to(BF16).to(DEV), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16).to(DEV)
+    lw = ops.prepare_linear(w)
+    assert ops.ring_takes_few(x, lw, True) == route
+    assert ops.ring_takes_few(x[:8], lw, True) == 0 and ops.ring_takes_few(torch.cat([x, x])[:17], lw, True) == 0
+    want = x.double() @ w.double().t()
+    sums = K ** 0.5 * 2.0 ** -22
+    got = ops.linear(x, lw, keep_slices=True)
+    assert isinstance(got, ops.SliceSums) == (route == 2)
+    if route == 2:
+        assert (got.sum(F32).double() - want).abs().max() < sums
+    assert ((ops.linear(x, lw).double() - want).abs() <= 2.0 ** -8 * want.abs() + sums).all()
+    assert (ops.linear(x, lw, out_dtype=F32).double() - want).abs().max() < sums
+    gate, up = want[:, 0::2], want[:, 1::2]
+    for act, f in ((ops.ACT_SILU, torch.nn.functional.silu), (ops.ACT_GELU_TANH, lambda v: torch.nn.functional.gelu(v, approximate="tanh"))):
+        pairs = f(gate) * up
+        assert ((ops.linear_swiglu(x, lw, act).double() - pairs).abs() <= 2.0 ** -8 * pairs.abs() + 8 * sums * (1 + up.abs())).all()
+    for act, f in ((ops.ACT_RELU_SQUARED, lambda v: v.clamp(min=0) ** 2), (ops.ACT_GELU_TANH, lambda v: torch.nn.functional.gelu(v, approximate="tanh"))):
+        assert ((ops.linear_act(x, lw, act).double() - f(want)).abs() <= 2.0 ** -8 * f(want).abs() + 8 * sums * (1 + want.abs())).all()
+
+
 def test_17_to_64_rows_go_to_the_ring_where_their_tiles_make_one_row_of_workgroups():
     assert ops.ring_takes(17, 9728, 896, 16, True) and ops.ring_takes(64, 24576, 2048, 16, True) and ops.ring_takes(33, 2048, 11008, 8, False)
     assert not ops.ring_takes(16, 9728, 896, 16, True) and not ops.ring_takes(65, 1024, 1024, 8, False)
