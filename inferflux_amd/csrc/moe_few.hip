@@ -8,6 +8,8 @@
 //                          weights whose rows alternate 16 of Wg with 16 of Wu
 //   ifx_moe_few_down       parts[choice][row][:] = weight[item] * Wd[e] act[item] in float; the kernel that adds the result to
 //                          the stream sums the choices in order
+// Rows may come up to a norm's factor (row_scale.h, up to 16 rows): the logits' product forms it beside its own loads, multiplies
+// the logits by it and leaves it for the experts' products, which multiply their sums by it; the norm's own launch is saved.
 // Identity experts (ids from `n_real` on) and weights on the experts' inputs are those of grouped_gemm.hip.  A shared expert, which
 // every row takes with weight 1, runs in the same launches: its rows are workgroups of their own ahead of the experts', its output
 // one more part.  As two products, an activation's launch and the launch that added it, one row of 2,048 values to a shared
@@ -25,6 +27,7 @@
 // 64 experts of which a row takes 6, at 1 / 8 / 16 / 64 rows 30 / 102 / 150 / 180 (53 / 142 / 230 / 264; the chosen experts'
 // bytes at 6.5 TB/s: 16 / 93 / 141 / 170); 32 experts, 4 to a row, 23 / 66 / 86 / 99 (32 / 97 / 125 / 153; 11 / 53 / 77 / 85).
 #include "common.h"
+#include "row_scale.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -50,12 +53,14 @@ __device__ __forceinline__ bf16x8 zero8() {
 // here (the kernel that chooses reads the slices side by side).
 #define LOGIT_SLICES 16
 __global__ __launch_bounds__(256) void moe_logits_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, float* __restrict__ z,
-                                                         int T, int K, int E, int slice_blocks) {
+                                                         int T, int K, int E, int slice_blocks, RowScale scale, float* __restrict__ factor) {
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, col = lane & 15, g = lane >> 4;
   const int e0 = 16 * blockIdx.x, m = 16 * wave + col;
   const bf16_t* wrow = w + (size_t)min(e0 + col, E - 1) * K;
   const bf16_t* xrow = x + (size_t)min(m, T - 1) * K;
   floatx4 acc{0.f, 0.f, 0.f, 0.f};
+  // (its loads go out ahead of the first of W, which are waited for together)
+  const float f = scale.pieces ? row_factor(scale, lane) : 1.f;
   const int kb_end = min((K + 63) / 64, (int)(blockIdx.y + 1) * slice_blocks);
   for (int kb0 = blockIdx.y * slice_blocks; kb0 < kb_end; kb0 += 2) {
     bf16x8 wv[4], xv[4];
@@ -71,7 +76,8 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const bf16_t* __restric
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r)
-    if (m < T && e0 + 4 * g + r < E) z[((size_t)blockIdx.y * T + m) * E + e0 + 4 * g + r] = acc[r];
+    if (m < T && e0 + 4 * g + r < E) z[((size_t)blockIdx.y * T + m) * E + e0 + 4 * g + r] = acc[r] * f;
+  if (scale.pieces && blockIdx.x == 0 && blockIdx.y == 0 && lane < T) factor[lane] = f;
 }
 
 static int logit_slice_blocks(int K) {                  // blocks of 64 k-values to a slice
@@ -80,10 +86,12 @@ static int logit_slice_blocks(int K) {                  // blocks of 64 k-values
 }
 extern "C" int ifx_moe_logit_slices(int K) { return ((K + 63) / 64 + logit_slice_blocks(K) - 1) / logit_slice_blocks(K); }
 
-extern "C" int ifx_moe_logits(const void* x, const void* w, float* z, int T, int K, int E, void* stream) {
+extern "C" int ifx_moe_logits(const void* x, const void* w, float* z, int T, int K, int E, const float* pieces, int n_pieces,
+                              float width, float eps, float* factor, void* stream) {
+  IFX_REQUIRE(!pieces || (T <= 16 && n_pieces > 0 && width > 0.f && factor), "moe_logits: bad row factors (%d rows, %d pieces, width %g)", T, n_pieces, (double)width);
   IFX_REQUIRE(T > 0 && T <= MAX_ROWS && E > 0 && K > 0 && K % 8 == 0, "moe_logits: %d rows (at most %d), %d experts, K=%d (a multiple of 8)", T, MAX_ROWS, E, K);
   hipLaunchKernelGGL(moe_logits_kernel, dim3((E + 15) / 16, ifx_moe_logit_slices(K)), dim3((T + 15) / 16 * WAVE), 0, (hipStream_t)stream,
-                     (const bf16_t*)x, (const bf16_t*)w, z, T, K, E, logit_slice_blocks(K));
+                     (const bf16_t*)x, (const bf16_t*)w, z, T, K, E, logit_slice_blocks(K), RowScale{pieces, n_pieces, width, eps}, factor);
   IFX_LAUNCH_CHECK();
 }
 
@@ -271,6 +279,7 @@ struct FewArgs {
   const bf16_t* shared_w;   // [shared_n][shared_k], in the experts' form
   void* shared_out;         // gate/up: [T][shared_n / 2]; down: [T][N]
   float shared_limit;
+  const float* factor;      // [T] a factor on the rows (gate/up: x; down: identity), or null
 };
 
 template <bool DOWN, bool TILED, int MT, int NT, int U>
@@ -304,7 +313,7 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
       for (int i = threadIdx.x; i < count * 16 * NT; i += blockDim.x) {
         const int m = list[i / (16 * NT)], n = n0 + i % (16 * NT);
         if (n < a.N)
-          ((float*)a.out)[((size_t)(m % a.top) * a.T + m / a.top) * a.N + n] = a.weights[m] * (float)a.identity[(size_t)(m / a.top) * a.N + n];
+          ((float*)a.out)[((size_t)(m % a.top) * a.T + m / a.top) * a.N + n] = a.weights[m] * (a.factor ? a.factor[m / a.top] : 1.f) * (float)a.identity[(size_t)(m / a.top) * a.N + n];
       }
     return;
   }
@@ -388,7 +397,7 @@ __global__ __launch_bounds__(256) void moe_few_kernel(FewArgs a) {
     const int m = item[mt];
     if (m < 0) continue;
     if constexpr (!DOWN) {             // NT = 2: 16 rows of Wg and the same 16 of Wu
-      const float wi = a.weigh_input && !shared ? a.weights[m] : 1.f, limit = shared ? a.shared_limit : a.limit;
+      const float wi = (a.weigh_input && !shared ? a.weights[m] : 1.f) * (a.factor ? a.factor[shared ? m : m / a.top] : 1.f), limit = shared ? a.shared_limit : a.limit;
       bf16x4 y;
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[r] = (__bf16)gated_act(wi * acc[0][mt][r], wi * acc[1][mt][r], a.act, limit);
@@ -435,13 +444,13 @@ static int few_waves(int K) {
 // shared_ff inner values, in the experts' form, its activations to shared_act [T][shared_ff].
 extern "C" int ifx_moe_few_gate_up(const void* x, const void* w, void* act, const int* ids, int T, int E, int K, int ff, int top, int n_real,
                                    int act_kind, float limit, const float* in_weights, int tiled, const void* shared_w, void* shared_act,
-                                   int shared_ff, float shared_limit, void* stream) {
+                                   int shared_ff, float shared_limit, const float* factor, void* stream) {
   IFX_REQUIRE(K > 0 && K % 8 == 0 && ff > 0 && ff % 16 == 0, "moe_few_gate_up: K=%d must be a multiple of 8, ff=%d of 16", K, ff);
   IFX_REQUIRE(T > 0 && T <= MAX_ROWS && top > 0 && top <= MAX_TOP && E > 0 && E <= MAX_E, "moe_few_gate_up: %d rows (at most %d) of %d of %d experts", T, MAX_ROWS, top, E);
   IFX_REQUIRE(!shared_w || (shared_act && shared_ff > 0 && shared_ff % 16 == 0 && shared_ff <= 1 << 20), "moe_few_gate_up: a shared expert of %d (a multiple of 16)", shared_ff);
   const int k_tiles = tiled ? (K + 63) / 64 * 2 : 0;
   FewArgs a{(const bf16_t*)x, (const bf16_t*)w, act, ids, in_weights, nullptr, K, 2 * ff, top, T, top, n_real, act_kind,
-            T * top < E ? 1 : 0, limit, in_weights ? 1 : 0, k_tiles, 0, K, 2 * shared_ff, k_tiles, (const bf16_t*)x, (const bf16_t*)shared_w, shared_act, shared_limit};
+            T * top < E ? 1 : 0, limit, in_weights ? 1 : 0, k_tiles, 0, K, 2 * shared_ff, k_tiles, (const bf16_t*)x, (const bf16_t*)shared_w, shared_act, shared_limit, factor};
   const int waves = few_waves(K);
   if (T <= 16) return launch_few<false, 1, 2, 3>(a, E, waves, (hipStream_t)stream);
   return launch_few<false, 2, 2, 2>(a, E, waves, (hipStream_t)stream);
@@ -450,13 +459,13 @@ extern "C" int ifx_moe_few_gate_up(const void* x, const void* w, void* act, cons
 // parts [top][T][N], and with a shared expert [top + 1][T][N], its output the last.
 extern "C" int ifx_moe_few_down(const void* act, const void* w, float* parts, const float* weights, const int* ids, int T, int E, int N,
                                 int ff, int top, int n_real, const void* identity, int weigh_input, int tiled, const void* shared_act,
-                                const void* shared_w, int shared_ff, void* stream) {
+                                const void* shared_w, int shared_ff, const float* factor, void* stream) {
   IFX_REQUIRE(ff > 0 && ff % 8 == 0 && N > 0 && (!tiled || N % 16 == 0), "moe_few_down: ff=%d must be a multiple of 8, N=%d of 16 if tiled", ff, N);
   IFX_REQUIRE(T > 0 && T <= MAX_ROWS && top > 0 && top <= MAX_TOP && E > 0 && E <= MAX_E, "moe_few_down: %d rows (at most %d) of %d of %d experts", T, MAX_ROWS, top, E);
   IFX_REQUIRE(!shared_w || (shared_act && shared_ff > 0 && shared_ff % 8 == 0 && shared_ff <= 1 << 20), "moe_few_down: a shared expert of %d (a multiple of 8)", shared_ff);
   FewArgs a{(const bf16_t*)act, (const bf16_t*)w, parts, ids, weights, (const bf16_t*)identity, ff, N, 1, T, top, n_real, 0,
             T * top < E ? 1 : 0, 0.f, weigh_input, tiled ? (ff + 63) / 64 * 2 : 0, 0, shared_ff, N, tiled ? (shared_ff + 63) / 64 * 2 : 0,
-            (const bf16_t*)shared_act, (const bf16_t*)shared_w, parts + (size_t)top * T * N, 0.f};
+            (const bf16_t*)shared_act, (const bf16_t*)shared_w, parts + (size_t)top * T * N, 0.f, factor};
   const int waves = few_waves(shared_w && shared_ff > ff ? shared_ff : ff);
   hipStream_t s = (hipStream_t)stream;
   // (two row tiles to a wave halve its reads of the items; up to 64 items one is better: twice the workgroups)

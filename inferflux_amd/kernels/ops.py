@@ -701,9 +701,15 @@ def moe_few_takes(dtype: torch.dtype, T: int, K: int, ff: int, n_routed: int, to
 
 def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_groups: int = 1, group_top: int = 2, softmax: bool = False,
                    renormalize: bool = False, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
-                   choice_bias: Optional[torch.Tensor] = None):
+                   choice_bias: Optional[torch.Tensor] = None, factor: Optional[torch.Tensor] = None):
     """``moe_route`` for up to 64 rows in bfloat16: the router's logits as a product (float32 sums and output) and a launch that
-    chooses.  Returns (ids int32 [T, top], weights float32 [T, top])."""
+    chooses.  Returns (ids int32 [T, top], weights float32 [T, top]).  ``h`` may be ``ScaledRows``, whose factors are then written to
+    ``factor`` [T] (float32)."""
+    h, scale_args = _scale_args(h)
+    if (factor is None) != (scale_args[0] == 0):
+        raise KernelError("moe_few: scaled rows and a place for their factors go together")
+    if factor is not None:
+        _check(factor, "factor", (h.shape[0],), torch.float32)
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
     rows = router.rows if isinstance(router, LinearWeight) else router
@@ -717,7 +723,8 @@ def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_grou
     mod, stream = load_module("moe_few"), _stream()
     slices = mod.fn("ifx_moe_logit_slices", (I,))(K)
     z = torch.empty((slices, T, E), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_logits", (P, P, P, I, I, I, P), h.data_ptr(), rows.data_ptr(), z.data_ptr(), T, K, E, stream)
+    _call(mod, "ifx_moe_logits", (P, P, P, I, I, I, P, I, F, F, P, P), h.data_ptr(), rows.data_ptr(), z.data_ptr(), T, K, E, *scale_args,
+          _ptr(factor), stream)
     ids = torch.empty((T, top), dtype=torch.int32, device=h.device)
     weights = torch.empty((T, top), dtype=torch.float32, device=h.device)
     _call(mod, "ifx_moe_choose", (P, I, P, P, I, I, I, I, I, I, I, I, F, P, P, P), z.data_ptr(), slices, ids.data_ptr(), weights.data_ptr(),
@@ -726,11 +733,14 @@ def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_grou
 
 
 def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, act: int = ACT_SILU,
-                    limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False, shared=None, shared_limit: float = 0.0) -> "SliceSums":
+                    limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False, shared=None, shared_limit: float = 0.0,
+                    factor: Optional[torch.Tensor] = None) -> "SliceSums":
     """``moe_experts`` for up to 64 rows in bfloat16: two launches that stream every chosen expert's weights once, whatever the
     number of rows that chose it (``gate_up`` from ``pair_gate_up``; both as tensors or ``ExpertTiles``).  Returns the choices' weighted outputs as ``SliceSums`` [top, T, N] like ``moe_experts_grouped``.
     ``shared``: (gate_up, down) of an expert that every row takes, [1, 2 shared_ff, K] and [1, N, shared_ff] in the experts' form
-    (with its own ``shared_limit``): its output is the last of [top + 1, T, N]."""
+    (with its own ``shared_limit``): its output is the last of [top + 1, T, N].  ``factor`` [T] (float32): h's rows are to be multiplied by it."""
+    if factor is not None:
+        _check(factor, "factor", (h.shape[0],), torch.float32)
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
     gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
@@ -753,13 +763,13 @@ def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, 
             raise KernelError(f"moe_few: a shared expert of {shape[1]} gate and up rows (a multiple of 32), in the experts' form")
     a = torch.empty((T * (top * ff + shared_ff),), dtype=torch.bfloat16, device=h.device)
     shared_a = a.data_ptr() + 2 * T * top * ff
-    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P, P, I, F, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
+    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P, P, I, F, P, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
           T, E, K, ff, top, n_real, int(act), float(limit), weights.data_ptr() if weigh_input else 0, gu_tiled,
-          shared_gu, shared_a, shared_ff, float(shared_limit), stream)
+          shared_gu, shared_a, shared_ff, float(shared_limit), _ptr(factor), stream)
     parts = torch.empty((top + (1 if shared is not None else 0), T, N), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, P), a.data_ptr(), down_ptr, parts.data_ptr(),
+    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, P, P), a.data_ptr(), down_ptr, parts.data_ptr(),
           weights.data_ptr(), ids.data_ptr(), T, E, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0, down_tiled,
-          shared_a, shared_down, shared_ff, stream)
+          shared_a, shared_down, shared_ff, _ptr(factor), stream)
     return SliceSums(parts, torch.bfloat16)
 
 

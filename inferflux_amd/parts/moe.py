@@ -137,10 +137,18 @@ class MixtureOfExperts(FeedForward):
             return
         self.shared_few = (ops.ExpertTiles(ops.pair_gate_up(gate[None].contiguous(), up[None].contiguous())), ops.ExpertTiles(down[None].contiguous()))
 
-    def route(self, h, few: bool = False):
-        return (ops.moe_few_choose if few else ops.moe_route)(
-            h, self.router, self.top, self.groups, self.keep_groups, self.group_top, self.scoring == "softmax", self.renormalize,
-            self.route_scale, self.bias, self.correction)
+    def route(self, h, few: bool = False, factor=None):
+        args = (h, self.router, self.top, self.groups, self.keep_groups, self.group_top, self.scoring == "softmax", self.renormalize,
+                self.route_scale, self.bias, self.correction)
+        return ops.moe_few_choose(*args, factor) if few else ops.moe_route(*args)
+
+    def _takes_few(self, dtype, n_rows: int) -> bool:
+        return self.up is None and ops.moe_few_takes(dtype, n_rows, self.hidden_size, self.ff, self.n_routed, self.top)
+
+    def accepts_scaled_rows(self, n_rows: int) -> bool:
+        """Where one launch forms the rows' factors and all that read the rows follow it."""
+        return (self.up is None and n_rows <= 16 and self.router.dtype == torch.bfloat16 and self._takes_few(torch.bfloat16, n_rows)
+                and (self.shared is None or (self.shared_few is not None and not self.shared_gate)))
 
     def _with_shared(self, out, x, ctx):
         """The chosen experts' sum plus the shared expert's output (times its gate of one number per row)."""
@@ -151,20 +159,24 @@ class MixtureOfExperts(FeedForward):
 
     def forward(self, h, ctx):
         x = h if h.dtype == self.router.dtype else h.to(self.router.dtype)
-        few = self.up is None and ops.moe_few_takes(x.dtype, x.shape[0], self.hidden_size, self.ff, self.n_routed, self.top)
-        ids, weights = self.route(x, few)
+        few = self._takes_few(x.dtype, x.shape[0])
+        factor = None
+        if isinstance(x, ops.ScaledRows):
+            factor = torch.empty((x.shape[0],), dtype=torch.float32, device=x.rows.device)
+        ids, weights = self.route(x, few, factor)
+        x = x if factor is None else x.rows
         if ctx.timer is not None:
             ctx.timer.mark("ffn.route")
         if few and self.shared_few is not None:
             sums = ops.moe_few_experts(x, self.gate, self.down, ids, weights, self.act, self.limit, self.n_identity, self.weigh_input,
-                                       self.shared_few, self.shared.limit)
+                                       self.shared_few, self.shared.limit, factor)
             if not self.shared_gate:
                 return sums                 # (the shared expert's output is one more partial sum)
             base, extra = ops.SliceSums(sums.parts[:-1], sums.dtype), ops.SliceSums(sums.parts[-1:], sums.dtype)
             return ops.gated_add(base, extra, x, self.shared_gate_w)
         if few:
             return self._with_shared(ops.moe_few_experts(x, self.gate, self.down, ids, weights, self.act, self.limit, self.n_identity,
-                                                         self.weigh_input), x, ctx)      # (partial sums, one per choice)
+                                                         self.weigh_input, factor=factor), x, ctx)      # (partial sums, one per choice)
         if self.up is None and (isinstance(self.gate, ops.ExpertTiles) or x.shape[0] * self.top >= GROUPED_MIN_ITEMS):
             return self._with_shared(ops.moe_experts_grouped(x, self.gate, self.down, ids, weights, self.act, self.limit,
                                                              self.n_identity, self.weigh_input), x, ctx)      # (partial sums, one per choice)

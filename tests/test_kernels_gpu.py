@@ -833,6 +833,41 @@ def test_gemm_f32_with_a_gated_activation_gives_the_bits_of_both_launches(M, N, 
         ops.gemm_f32(x, w, torch.zeros(N, device=DEV), gated=act, limit=limit)
 
 
+@pytest.mark.parametrize("T,E,identity,top,K,ff,shared_ff,n_pieces", [(1, 4, 0, 2, 64, 16, 0, 1), (3, 6, 2, 3, 128, 48, 32, 7), (16, 70, 0, 2, 256, 32, 0, 16), (16, 5, 3, 4, 2048, 32, 64, 300)])
+@pytest.mark.parametrize("form", ["sigmoid", "softmax", "input"])
+def test_moe_few_takes_rows_up_to_a_factor(T, E, identity, top, K, ff, shared_ff, n_pieces, form):
+    """Rows whose norm's factors are powers of two, given as sums of squares in pieces, and the same rows multiplied by them: every
+    product and sum is the same up to that power, so the bits are the same."""
+    g = gen(2360 + T)
+    power = torch.randint(-2, 3, (T,), generator=g)
+    pieces = torch.zeros(n_pieces, 16)
+    pieces[torch.randint(0, n_pieces, (T,), generator=g), torch.arange(T)] = K * 4.0 ** -power.float()
+    rows = torch.randn(T, K, generator=g).to(BF16)
+    scaled = ops.ScaledRows(rows.to(DEV), pieces.to(DEV), K, 0.0)
+    whole = (rows.float() * 2.0 ** power[:, None].float()).to(BF16).to(DEV)
+    router = (torch.randn(E + identity, K, generator=g) / K ** 0.5).to(BF16).to(DEV)
+    mats = lambda n, f: [(torch.randn(n, f, K, generator=g) / K ** 0.5).to(BF16).to(DEV) for _ in range(2)] + [(torch.randn(n, K, f, generator=g) / f ** 0.5).to(BF16).to(DEV)]
+    gate, up, down = mats(E, ff)
+    args = (ops.ExpertTiles(ops.pair_gate_up(gate, up)), ops.ExpertTiles(down))
+    shared = None
+    if shared_ff:
+        sg, su, sd = mats(1, shared_ff)
+        shared = (ops.ExpertTiles(ops.pair_gate_up(sg, su)), ops.ExpertTiles(sd))
+    outs = []
+    for h in (scaled, whole):
+        factor = torch.empty(T, device=DEV) if h is scaled else None
+        ids, weights = ops.moe_few_choose(h, router, top, softmax=form == "softmax", factor=factor)
+        x = h.rows if factor is not None else h
+        parts = ops.moe_few_experts(x, *args, ids, weights, n_identity=identity, weigh_input=form == "input", shared=shared, factor=factor).parts
+        outs.append((ids, weights, parts))
+        if factor is not None:
+            assert torch.equal(factor.cpu(), 2.0 ** power.float())
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    with pytest.raises(ops.KernelError):
+        ops.moe_few_choose(scaled, router, top)
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
