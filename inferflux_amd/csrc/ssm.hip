@@ -131,6 +131,36 @@ __global__ __launch_bounds__(256) void conv_state_kernel(ConvArgs a) {
   }
 }
 
+// Both at once for steps of single tokens: a thread walks a request's rows for one channel with the last inputs in registers and leaves
+// them in the state (the two launches read the same few values, 4.6 us each; the same additions in the same order).
+template <typename T>
+__global__ __launch_bounds__(256) void conv_step_kernel(ConvArgs a) {
+  const int c = blockIdx.x * 256 + threadIdx.x, r = blockIdx.y, keep = a.taps - 1;
+  if (c >= a.C) return;
+  const int n = a.q_len[r], t0 = a.q_start[r];
+  float* st = a.state + (size_t)a.slots[r] * a.state_stride + (size_t)c * keep;
+  float v[MAX_TAPS], w[MAX_TAPS];
+#pragma unroll
+  for (int k = 0; k < MAX_TAPS; ++k) {
+    w[k] = k < a.taps ? load_dyn(a.w, a.w_dtype, (size_t)c * a.taps + k) : 0.f;
+    v[k] = k < keep ? st[k] : 0.f;
+  }
+  const float b = a.b ? load_dyn(a.b, a.w_dtype, c) : 0.f;
+  for (int t = t0; t < t0 + n; ++t) {
+    const float x = to_f(((const T*)a.x)[(size_t)t * a.ld + c]);
+    float acc = b;
+#pragma unroll
+    for (int k = 0; k < MAX_TAPS; ++k)
+      if (k < a.taps) acc = fmaf(w[k], k < keep ? v[k] : x, acc);
+#pragma unroll
+    for (int k = 0; k < MAX_TAPS - 1; ++k) v[k] = k + 1 < keep ? v[k + 1] : x;
+    ((T*)a.out)[(size_t)t * a.C + c] = from_f<T>(act_silu(acc));
+  }
+#pragma unroll
+  for (int k = 0; k < MAX_TAPS - 1; ++k)
+    if (k < keep) st[k] = v[k];
+}
+
 extern "C" int ifx_causal_conv(const void* x, int dtype, int ld, const void* w, const void* b, int w_dtype, float* state,
                                long long state_stride, const int* row_req, const int* q_start, const int* q_len,
                                const int* slots, void* out, int T, int R, int C, int taps, void* stream) {
@@ -142,6 +172,11 @@ extern "C" int ifx_causal_conv(const void* x, int dtype, int ld, const void* w, 
   ConvArgs a{x, ld, w, b, w_dtype, state, (size_t)state_stride, row_req, q_start, q_len, slots, out, T, R, C, taps};
   hipStream_t s = (hipStream_t)stream;
   const unsigned cb = (unsigned)((C + 255) / 256);
+  if (T <= R && (dtype == DT_F32 || dtype == DT_BF16)) {
+    if (dtype == DT_F32) hipLaunchKernelGGL(conv_step_kernel<float>, dim3(cb, R), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(conv_step_kernel<bf16_t>, dim3(cb, R), dim3(256), 0, s, a);
+    IFX_LAUNCH_CHECK();
+  }
   if (dtype == DT_F32) {
     hipLaunchKernelGGL(conv_silu_kernel<float>, dim3(cb, T), dim3(256), 0, s, a);
     if (taps > 1) hipLaunchKernelGGL(conv_state_kernel<float>, dim3(cb, R), dim3(256), 0, s, a);

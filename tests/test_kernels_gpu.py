@@ -868,6 +868,25 @@ def test_moe_few_takes_rows_up_to_a_factor(T, E, identity, top, K, ff, shared_ff
         ops.moe_few_choose(scaled, router, top)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("R,channels,taps,bias", [(1, 8, 4, True), (3, 300, 2, False), (5, 256, 1, True), (16, 1032, 3, True), (2, 40, 16, False)])
+def test_causal_conv_of_single_tokens_gives_the_bits_of_whole_requests(dtype, R, channels, taps, bias):
+    """Every request's rows at once (two launches) and token by token (one): the same outputs and the same state."""
+    g = gen(2380 + channels)
+    n, ld = taps + 3, channels + 8
+    x = torch.randn(R, n, ld, generator=g).to(dtype).to(DEV)
+    w, b = torch.randn(channels, taps, generator=g).to(dtype).to(DEV), torch.randn(channels, generator=g).to(dtype).to(DEV) if bias else None
+    start = torch.randn(R + 1, channels * (taps - 1) + 4, generator=g).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    slots = i32(list(range(R, 0, -1)))
+    one, whole = start.clone(), start.clone()
+    want = ops.causal_conv_silu(x.reshape(R * n, ld), channels, w, b, whole, i32([r for r in range(R) for _ in range(n)]), i32([r * n for r in range(R)]), i32([n] * R), slots)
+    for t in range(n):
+        got = ops.causal_conv_silu(x[:, t].contiguous(), channels, w, b, one, i32(list(range(R))), i32(list(range(R))), i32([1] * R), slots)
+        assert torch.equal(got, want.view(R, n, channels)[:, t])
+    assert torch.equal(one, whole)
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
