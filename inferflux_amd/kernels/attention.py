@@ -279,6 +279,10 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
     T, nH, d = q.shape
     table = ctx.block_table(cache.group)
     keep_first = int(keep_first or 0) if window else 0
+    if keep_first and ctx.h_q_len.max() >= TILE_MIN and ctx.h_kv_len.max() <= window:
+        # prompts that the window holds whole see their first keys anyway, and without them the kernel that loads straight into LDS
+        # takes them (2,048 rows of 16 heads of 128 82 us, then 51; steps of single rows are captured for later lengths, too)
+        keep_first = 0
     other = keep_first > 0 or sink is not None or gate is not None or bool(block)      # (a sink score per head some kernels do take)
     extras = other or sinks is not None
     if not ops.mfma_attention_supported(q.dtype, d, cache.page_size) or cache.v.shape[2] != d:
@@ -295,7 +299,7 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
     qt, splits, chunk = 1, 1, 0
     if tiled.any():
         qt, splits, chunk = choose_tiling(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, lambda t: ops.attention_tile_rows(d, t),
-                                          tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not other)
+                                          tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not keep_first and not block)
     tile_rows = ops.attention_tile_rows(d, qt)
     w = ctx.derived(("attention_work_lists", n_kv, tile_rows, nH, splits, chunk, window, d),
                     lambda: _work_lists(ctx, n_kv, tile_rows, nH, splits, chunk, window, ops.row_waves_fit(nH, n_kv, d, ops.ROW_MAX_WAVES), d))

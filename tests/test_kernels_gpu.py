@@ -887,6 +887,29 @@ def test_causal_conv_of_single_tokens_gives_the_bits_of_whole_requests(dtype, R,
     assert torch.equal(one, whole)
 
 
+@pytest.mark.parametrize("T,past,chunk", [(16, 0, 0), (129, 60, 0), (300, 700, 0), (200, 900, 448)])
+@pytest.mark.parametrize("form", ["sink", "gate", "both", "sinks and gate"])
+def test_direct_tiles_with_a_sink_and_a_gate(T, past, chunk, form):
+    """The prompts' kernel that loads straight into LDS, whole and in splits of the keys, against the plain kernel in 32 bits on the same
+    values: rounding of the weights and of the result to bfloat16 (2^-8 each)."""
+    nH, nKV, d, P = 4, 2, 128, 16
+    g = gen(2390 + T)
+    n, pages = past + T, -(-(past + T) // P)
+    q, kc, vc = (torch.randn(*s, generator=g).to(BF16).to(DEV) for s in ((T, nH, d), (pages, nKV, P, d), (pages, nKV, d, P)))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    table, pos = torch.randperm(pages, generator=g).to(torch.int32)[None].to(DEV), i32(list(range(past, n)))
+    more = {"sink": dict(sink=0.7), "gate": dict(gate=torch.rand(T, nH, generator=g).to(DEV)), "both": dict(sink=-0.2, gate=torch.rand(T, nH, generator=g).to(DEV)),
+            "sinks and gate": dict(sinks=torch.randn(nH, generator=g).to(DEV), gate=torch.rand(T, nH, generator=g).to(DEV))}[form]
+    rows = ops.attention_tile_rows(d, 2)
+    q0 = list(range(0, T, rows))
+    splits = dict(chunk=chunk, max_splits=-(-n // chunk), rows=i32(list(range(T))), row_req=i32([0] * T), positions=pos) if chunk else {}
+    out = torch.full((T, nH * d), 9.0, dtype=BF16, device=DEV)
+    ops.attention_tiles(q, kc, vc, out, i32([0] * len(q0)), i32(q0), i32([0]), i32([T]), i32([n]), table, None, 0.1, 2, **splits, **more)
+    want = ops.attention_plain(q.float(), kc.float(), vc.float(), i32([0] * T), pos, table, None, 0.1, **more).view(T, -1)
+    assert (out.float() - want).pow(2).mean().sqrt() < 2.0 ** -8 * want.pow(2).mean().sqrt()
+    assert (out.float() - want).abs().max() < 6 * 2.0 ** -8 * want.abs().max()
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
