@@ -310,6 +310,9 @@ static double sums_us(int kind, int M, int N, int slices, int slice_k) {
 #define SUMS_MIN_ROWS 257
 #define SUMS_MIN_N 896          // (lower weights were not measured)
 #define SUMS_MIN_K 8192
+#define SMALL_MIN_ROWS 129
+#define SMALL_MIN_K 896
+#define SMALL_MOST 4.0e9        // M N K
 #define SUMS_MAX_SLICES 8
 #define SUMS_MAX_BYTES (512ll << 20)      // of partial sums
 
@@ -322,11 +325,18 @@ static double sums_us(int kind, int M, int N, int slices, int slice_k) {
 //   product costs the host 15 us more: 24 arriving requests at the 3B shape 244.8 -> 234.8 ms from 257 rows on, 239.8 from 800.)
 //   129 to 256 tiles, which are one round of the library's: 0.94     more, whose last round is at most 85 % full on the whole: 1.22 and
 //   0.81, fuller ones 0.97            weights of 4,096 to 8,192 k-values, of multiples of 512 rows: 0.94
+// Small products come here for the host's sake: the library's choice of a kernel and launch take it 26 us a call (the batched product
+// 40), this one's 8, and steps that mix portions with decoding are run launch by launch, so that 530 rows of 2,560 x 2,048, 14.2 us
+// there and 16.0 here, cost the longer of the two.  24 arriving requests at the 3B shape: 235.4 -> 228.0 ms.
 // `library_slices`: the slices that the library would take.
 extern "C" int ifx_gemm_tiles_sums_plan(int M, int N, int K, int library_slices) {
-  if (M < SUMS_MIN_ROWS || N < SUMS_MIN_N || K < SUMS_MIN_K || K > 1 << 20 || N > 1 << 20 || N % 8 || K % 8) return 0;
-  const long long tiles = (long long)((N + 255) / 256) * ((M + 255) / 256), library = tiles * library_slices;
-  if ((tiles > 128 && tiles <= 256) || library >= 0.85 * 256 * ((library + 255) / 256)) return 0;
+  if (N < SUMS_MIN_N || K > 1 << 20 || N > 1 << 20 || N % 8 || K % 8) return 0;
+  const bool small = M >= SMALL_MIN_ROWS && K >= SMALL_MIN_K && (double)M * N * K <= SMALL_MOST;
+  if (!small) {
+    if (M < SUMS_MIN_ROWS || K < SUMS_MIN_K) return 0;
+    const long long tiles = (long long)((N + 255) / 256) * ((M + 255) / 256), library = tiles * library_slices;
+    if ((tiles > 128 && tiles <= 256) || library >= 0.85 * 256 * ((library + 255) / 256)) return 0;
+  }
   int best = 0;
   double least = 0;
   for (int s = 1; s <= SUMS_MAX_SLICES; ++s) {

@@ -804,7 +804,8 @@ def test_tiles_products_as_partial_sums_and_plain(M, N, K, slices, slice_k):
         ops.sums_tiles(x, w, slices, slice_k, 2)
 
 
-@pytest.mark.parametrize("M,N,K,slices", [(256, 1024, 8192, 0), (257, 896, 8192, 8), (300, 888, 8192, 0), (1000, 2048, 8200, 4), (1025, 904, 9000, 7), (6144, 3584, 8192, 1),
+@pytest.mark.parametrize("M,N,K,slices", [(128, 1024, 8192, 0), (129, 896, 896, 7), (256, 1024, 8192, 8), (530, 2560, 2048, 4), (1034, 2048, 2048, 0), (530, 2560, 888, 0),
+                                          (256, 2048, 8192, 0), (257, 896, 8192, 8), (300, 888, 8192, 0), (1000, 2048, 8200, 4), (1025, 904, 9000, 7), (6144, 3584, 8192, 1),
                                           (2048, 3584, 18944, 0), (4500, 3584, 8192, 0), (1030, 2052, 8192, 0), (1030, 2048, 8184, 0)])
 def test_deep_products_of_many_rows_take_slices_of_tiles(M, N, K, slices):
     """The sizes on both sides of the rule's lines, through ``linear``, against 64 bits (partial sums in float, or one rounding to
