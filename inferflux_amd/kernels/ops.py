@@ -1187,8 +1187,10 @@ def wide_gemm(x, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, 
     M, K = x.shape
     N = weight.rows.shape[0]
     # (more than 16 rows carry no factor)
-    if waves == 0 and slices == 0 and weight.tiled is not None and ring_takes(M, N, K, weight.tile_rows, swiglu_pairs) and K % 8 == 0 \
-            and x.data_ptr() % 16 == 0 and not (swiglu_pairs and (N % 2 or weight.order is not None)):
+    ring = waves == 0 and slices == 0 and weight.tiled is not None and K % 8 == 0 and x.data_ptr() % 16 == 0
+    if ring and not swiglu_pairs and _ring_in_one_slice(M, N, K, weight.tile_rows, keep_slices):
+        return ring_gemm(x, weight, out_dtype, slices=1)
+    if ring and ring_takes(M, N, K, weight.tile_rows, swiglu_pairs) and not (swiglu_pairs and (N % 2 or weight.order is not None)):
         return ring_gemm(x, weight, out_dtype, swiglu_pairs=swiglu_pairs, keep_slices=keep_slices, act=act)
     if weight.tiled is None or weight.rows.shape[1] != K or weight.rows.dtype != torch.bfloat16:
         raise KernelError(f"wide_gemm: needs the tiled copy of a bfloat16 [N, {K}] weight")
@@ -1267,6 +1269,18 @@ def ring_takes(M: int, N: int, K: int, tile_rows: int, one_slice: bool) -> bool:
         896 x 4,864 6.6 : 5.7, 6.7 : 5.6, 9.0 : 7.3     1,536 x 8,960 10.5 : 8.9, 10.3 : 9.2, 13.6 : 11.8    1,024 x 1,024 4.3 : 3.7, 4.5 : 3.8, 5.6 : 4.4
         3,584 x 18,944 25.5 : 24.1, 25.6 : 24.5, 31.0 : 28.3     2,560 x 2,048 5.3 : 5.2, 5.8 : 5.6, 7.6 : 7.1, but 4,608 x 3,584 8.5 : 8.8, 9.1 : 9.2, 11.2 : 11.1."""
     return 17 <= M <= SKINNY_MAX_M and -(-N // tile_rows) <= (6 if one_slice else 1) * COMPUTE_UNITS and K < 1 << 20
+
+
+def _ring_in_one_slice(M: int, N: int, K: int, tile_rows: int, keep_slices: bool) -> bool:
+    """Whether ``wide_gemm`` hands 17 to 64 rows times a weight that it would cut into slices of K to ``ring_gemm`` uncut: up to 4,096 k-values
+    where nobody adds slices on the way, up to 2,048 where the reader does (us at 17 / 32 / 64 rows: slices and their sum, slices alone, uncut)
+        6,208 x 2,048 10.9, 8.2, 7.3 / 11.9, 8.5, 7.9 / 15.2, 10.6, 10.6     12,288 x 2,048 16.7, 14.3, 10.8 / 17.1, 14.4, 11.1 / 21.2, 17.1, 13.5
+        4,608 x 3,584 12.4, 8.7, 9.9 / 13.3, 9.2, 11.2 / 17.2, 11.3, 15.3     3,104 x 1,024 6.7, 4.7, 4.7 / 6.9, 4.9, 5.0 / 8.4, 6.2, 6.4
+        4,352 x 2,048 10.5, 7.4, 7.0 / 11.6, 7.9, 7.6 / 14.7, 9.9, 10.3     4,096 x 4,096 10.8, 8.2, 9.6 / 10.9, 8.8, 9.9 / 13.7, 11.3, 13.9."""
+    tiles = -(-N // tile_rows)
+    if not 17 <= M <= SKINNY_MAX_M or K % 8 or N <= 2048 or tiles > 6 * COMPUTE_UNITS:
+        return False
+    return tiles > COMPUTE_UNITS and K <= 2048 if keep_slices else K <= 4096
 
 
 RING_FEW_MIN_ROWS = 9            # (up to 8 rows x is little to read beside W)

@@ -911,6 +911,21 @@ def test_direct_tiles_with_a_sink_and_a_gate(T, past, chunk, form):
     assert (out.float() - want).abs().max() < 6 * 2.0 ** -8 * want.abs().max()
 
 
+@pytest.mark.parametrize("M,N,K,one", [(17, 2064, 4096, (0, 1)), (64, 4112, 2048, (1, 1)), (32, 4112, 2056, (0, 1)), (40, 2064, 4104, (0, 0)), (33, 24592, 72, (0, 0)),
+                                       (64, 24576, 72, (1, 1)), (20, 4096, 1000, (0, 1))])
+def test_17_to_64_rows_of_plain_products_in_one_slice(M, N, K, one):
+    """The weights on both sides of the rule's lines, with the slices taken by the reader and not, against 64 bits (as test_ring_gemm)."""
+    g = gen(2395 + N)
+    x, w = torch.randn(M, K, generator=g).to(BF16).to(DEV), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16).to(DEV)
+    lw = ops.prepare_linear(w)
+    assert tuple(int(ops._ring_in_one_slice(M, N, K, lw.tile_rows, keep)) for keep in (True, False)) == one
+    want, sums = x.double() @ w.double().t(), K ** 0.5 * 2.0 ** -22
+    kept = ops.linear(x, lw, keep_slices=True)
+    kept = kept.sum(F32) if isinstance(kept, ops.SliceSums) else kept
+    assert ((kept.double() - want).abs() <= 2.0 ** -8 * want.abs() + sums).all()
+    assert (ops.linear(x, lw, out_dtype=F32).double() - want).abs().max() < sums
+
+
 @pytest.mark.parametrize("T", [1, 16, 64, 65, 200])
 def test_a_mixture_books_its_router_whatever_the_rows(T):
     """The phase "ffn.route" of the per-phase timing, on both sides of the rows that the products for few rows take."""
