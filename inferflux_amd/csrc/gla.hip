@@ -72,9 +72,13 @@ __device__ __forceinline__ float log_sigmoid(float x) {      // -softplus(-x), w
 // (a thread's registers hold DP numbers of S: the more of them, the fewer threads a workgroup may have)
 #define GLA_MAX_THREADS(DP) ((DP) <= 32 ? 1024 : ((DP) <= 64 ? 512 : 256))
 
-template <typename T, typename TO, int DP, int MODE, int COLS>
-__global__ __launch_bounds__(GLA_MAX_THREADS(DP)) void gla_kernel(GlaArgs a) {
-  extern __shared__ float lds[];
+// WHOLE: the parts' channels are all of a head's (parts * DP = d), so nothing is asked of a channel before it is read, and what a thread
+// reads of a token from LDS goes in pieces of 16 bytes (4,000 rows of 16 heads of 64 x 128 in chunks: 151 and 222 us -> 98 and 195 for the two
+// walks, a third of it the values, which lay in 32 registers; time mixing of 64 requests' prompts 148 -> 93).  With up to 512 threads: it wants 140
+// registers, and with 128 of them (1,024 threads) steps of single tokens take 12.4 us for 10.8.
+template <typename T, typename TO, int DP, int MODE, int COLS, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? 512 : GLA_MAX_THREADS(DP)) void gla_kernel(GlaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   const int d = a.d, dv = a.dv, parts = a.parts, H = a.H;
   float* lq = lds;                       // [STAGE][d]
   float* lk = lq + STAGE * d;            // [STAGE][d]
@@ -116,6 +120,15 @@ __global__ __launch_bounds__(GLA_MAX_THREADS(DP)) void gla_kernel(GlaArgs a) {
   const T* rq = (const T*)a.q; const T* rk = (const T*)a.k; const T* rv = (const T*)a.v; const T* rg = (const T*)a.g;
   const int wid = tid / WAVE, lane = tid % WAVE, nw = (blockDim.x + WAVE - 1) / WAVE;
   float loga_sum = 0.f;
+  auto put_back = [&]() {
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+      if (j0 + c < dv) {
+#pragma unroll
+        for (int i = 0; i < DP; i += 4)
+          *(float4*)(sp + (size_t)c * parts * DP + i) = make_float4(S[c][i], S[c][i + 1], S[c][i + 2], S[c][i + 3]);
+      }
+  };
   for (int s0 = 0; s0 < n; s0 += STAGE) {
     const int ns = min(STAGE, n - s0);
     // the stage's q, k and decays: one (token, channel) a thread and trip, neighbouring threads on neighbouring channels
@@ -131,12 +144,22 @@ __global__ __launch_bounds__(GLA_MAX_THREADS(DP)) void gla_kernel(GlaArgs a) {
       lk[it] = kq;
       lq[it] = qq * a.q_scale;
     }
-    float vv[COLS][STAGE];
+    // (a wave's first token's gate and norm weights, up to two of each a lane, come with the stage's own loads)
+    float g_early[2], w_early[2];
+    if (MODE != 1) {
 #pragma unroll
-    for (int c = 0; c < COLS; ++c)
-#pragma unroll
-      for (int tt = 0; tt < STAGE; ++tt)
-        vv[c][tt] = (j0 + c < dv && tt < ns) ? to_f(rv[(size_t)(t0 + s0 + tt) * a.ld + head * dv + j0 + c]) : 0.f;
+      for (int c = 0; c < 2; ++c) {
+        const int e = lane + c * WAVE;
+        const bool in = wid < ns && e < dv;
+        g_early[c] = in ? to_f(rg[(size_t)(t0 + s0 + wid) * a.ld + head * dv + e]) : 0.f;
+        w_early[c] = in ? load_dyn(a.norm_w, a.norm_dtype, TIME_MIX ? head * dv + e : e) : 0.f;
+      }
+    }
+    // the values lie where the outputs will: a column's value is read by the lanes that form its output before one of them writes it
+    for (int it = tid; it < ns * dv; it += blockDim.x) {
+      const int tt = it / dv, c = it - tt * dv;
+      lo[it] = to_f(rv[(size_t)(t0 + s0 + tt) * a.ld + head * dv + c]);
+    }
     __syncthreads();
     if (MODE == 1 && tid < d)
       for (int tt = 0; tt < ns; ++tt) loga_sum += lg[tt * d + tid];
@@ -149,35 +172,50 @@ __global__ __launch_bounds__(GLA_MAX_THREADS(DP)) void gla_kernel(GlaArgs a) {
       }
       __syncthreads();
     }
+#pragma unroll 1
     for (int tt = 0; tt < ns; ++tt) {
       const float* aa = la + tt * d + p * DP;
       const float* kk = lk + tt * d + p * DP;
       const float* qv = lq + tt * d + p * DP;
-      float acc[COLS];
+      float acc[COLS], vt[COLS];
 #pragma unroll
-      for (int c = 0; c < COLS; ++c) acc[c] = 0.f;
+      for (int c = 0; c < COLS; ++c) {
+        acc[c] = 0.f;
+        vt[c] = j0 + c < dv ? lo[tt * dv + j0 + c] : 0.f;
+      }
+      auto channel = [&](int i, float al, float kv, float qq) {
 #pragma unroll
-      for (int i = 0; i < DP; ++i) {
-        if (p * DP + i < d) {              // (uniform over the lanes that share p; DP divides into d for the usual sizes)
-          const float al = aa[i], kv = kk[i], qq = MODE != 1 ? qv[i] : 0.f;
-#pragma unroll
-          for (int c = 0; c < COLS; ++c) {
-            if (TIME_MIX && MODE != 1) acc[c] = fmaf(S[c][i], qq, acc[c]);        // (the read-out comes before the write)
-            S[c][i] = fmaf(al, S[c][i], kv * vv[c][tt]);
-            if (!TIME_MIX && MODE != 1) acc[c] = fmaf(S[c][i], qq, acc[c]);
-          }
+        for (int c = 0; c < COLS; ++c) {
+          if (TIME_MIX && MODE != 1) acc[c] = fmaf(S[c][i], qq, acc[c]);        // (the read-out comes before the write)
+          S[c][i] = fmaf(al, S[c][i], kv * vt[c]);
+          if (!TIME_MIX && MODE != 1) acc[c] = fmaf(S[c][i], qq, acc[c]);
         }
+      };
+      if constexpr (WHOLE) {
+#pragma unroll
+        for (int i = 0; i < DP; i += 4) {
+          const float4 al = *(const float4*)(aa + i), kv = *(const float4*)(kk + i), qq = MODE != 1 ? *(const float4*)(qv + i) : float4{0.f, 0.f, 0.f, 0.f};
+          channel(i, al.x, kv.x, qq.x);
+          channel(i + 1, al.y, kv.y, qq.y);
+          channel(i + 2, al.z, kv.z, qq.z);
+          channel(i + 3, al.w, kv.w, qq.w);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < DP; ++i)
+          if (p * DP + i < d) channel(i, aa[i], kk[i], MODE != 1 ? qv[i] : 0.f);              // (uniform over the lanes that share p)
       }
       if (MODE != 1) {
 #pragma unroll
         for (int c = 0; c < COLS; ++c) {
           float r = acc[c];
           for (int o = 1; o < parts; o <<= 1) r += __shfl_xor(r, o, WAVE);
-          if (TIME_MIX) r = fmaf(lb[tt], vv[c][tt], r);
+          if (TIME_MIX) r = fmaf(lb[tt], vt[c], r);
           if (j0 + c < dv && p == 0) lo[tt * dv + j0 + c] = r;
         }
       }
     }
+    if (MODE == 0 && s0 + STAGE >= n) put_back();          // (on its way while the outputs are formed)
     __syncthreads();
     if (MODE != 1) {
       // a wave per token: the head's norm over dv, its weight, the gate
@@ -186,24 +224,18 @@ __global__ __launch_bounds__(GLA_MAX_THREADS(DP)) void gla_kernel(GlaArgs a) {
         float ss = 0.f;
         for (int c = lane; c < dv; c += WAVE) ss = fmaf(lo[tt * dv + c], lo[tt * dv + c], ss);
         const float inv = rsqrtf(wave_sum(ss) / (float)dv + a.eps);
-        for (int c = lane; c < dv; c += WAVE) {
-          const float g = to_f(rg[t * a.ld + head * dv + c]);
-          ((TO*)a.out)[t * (size_t)(H * dv) + head * dv + c] =
-              from_f<TO>(lo[tt * dv + c] * inv * load_dyn(a.norm_w, a.norm_dtype, TIME_MIX ? head * dv + c : c) * act_silu(g));
+        int u = 0;
+        for (int c = lane; c < dv; c += WAVE, ++u) {
+          const bool early = tt == wid && u < 2;
+          const float g = early ? (u == 0 ? g_early[0] : g_early[1]) : to_f(rg[t * a.ld + head * dv + c]);
+          const float w = early ? (u == 0 ? w_early[0] : w_early[1]) : load_dyn(a.norm_w, a.norm_dtype, TIME_MIX ? head * dv + c : c);
+          ((TO*)a.out)[t * (size_t)(H * dv) + head * dv + c] = from_f<TO>(lo[tt * dv + c] * inv * w * act_silu(g));
         }
       }
     }
     __syncthreads();                       // (the next stage's loads overwrite what this stage read)
   }
-  if (MODE != 2) {
-#pragma unroll
-    for (int c = 0; c < COLS; ++c)
-      if (j0 + c < dv) {
-#pragma unroll
-        for (int i = 0; i < DP; i += 4)
-          *(float4*)(sp + (size_t)c * parts * DP + i) = make_float4(S[c][i], S[c][i + 1], S[c][i + 2], S[c][i + 3]);
-      }
-  }
+  if (MODE == 1) put_back();
   if (MODE == 1 && tid < d) a.chunk_loga[(size_t)unit * H * d + head * d + tid] = loga_sum;
 }
 
@@ -249,7 +281,13 @@ __global__ __launch_bounds__(256) void gla_combine_kernel(CombineArgs a) {
 
 template <typename T, typename TO, int DP, int MODE, int COLS>
 static void launch_gla_mode(const GlaArgs& a, int units, int threads, size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL((gla_kernel<T, TO, DP, MODE, COLS>), dim3(units, a.H), dim3(threads), lds, s, a);
+  if constexpr (DP <= 32) {
+    if (a.parts * DP == a.d && threads <= 512) {
+      hipLaunchKernelGGL((gla_kernel<T, TO, DP, MODE, COLS, true>), dim3(units, a.H), dim3(threads), lds, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((gla_kernel<T, TO, DP, MODE, COLS, false>), dim3(units, a.H), dim3(threads), lds, s, a);
 }
 
 // A launch of MODE with ``cols`` columns of S a thread (1, 2 or 4; what DP allows is checked by the caller).
