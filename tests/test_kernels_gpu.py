@@ -823,9 +823,10 @@ def test_deep_products_of_many_rows_take_slices_of_tiles(M, N, K, slices):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 2, 4), (4, 1022, 36), (4, 4098, 64), (8, 2046, 100), (16, 34, 7), (40, 130, 64), (300, 514, 72), (700, 1026, 48)])
-@pytest.mark.parametrize("act,limit", [(ops.ACT_SILU, 0.0), (ops.ACT_GELU_TANH, 0.0), (ops.ACT_CLAMPED_SWISH, 0.75)])
+@pytest.mark.parametrize("act,limit", [("ACT_SILU", 0.0), ("ACT_GELU_TANH", 0.0), ("ACT_CLAMPED_SWISH", 0.75)])
 def test_gemm_f32_with_a_gated_activation_gives_the_bits_of_both_launches(M, N, K, act, limit):
     """Every one of the 32-bit kernels, columns that end within its workgroups, K off 16 bytes."""
+    act = getattr(ops, act)
     g = gen(2340 + M)
     x, w = torch.randn(M, K, generator=g).to(DEV), (torch.randn(N, K, generator=g) / K ** 0.5).to(DEV)
     want = ops.swiglu(ops.gemm_f32(x, w), interleaved=True, act=act, limit=limit)
