@@ -374,6 +374,31 @@ def test_matrix_memory_over_steps_with_state_in_slots(dtype, H, d, dv):
             assert rel_err(torch.cat(got[r]), T64(want[r])) < (3e-5 if dtype == "float32" else 2e-2), (r, chunked)
 
 
+@pytest.mark.parametrize("H,d,dv", [(2, 16, 1), (3, 10, 63), (4, 64, 128), (2, 64, 255), (2, 64, 256), (3, 128, 128), (1, 512, 31), (1, 512, 63), (2, 8, 40)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float32 to bfloat16"])
+def test_single_tokens_of_the_memory_against_the_walk(dtype, H, d, dv):
+    """Heads on both sides of what a workgroup takes with 16 and 32 channels a thread: single tokens of four requests, twice, against the
+    walk, which the same tokens take beside a request of two.  Sums of at most 512 products in another order: 2e-5 of the result."""
+    dt, out_dt = DT[dtype.split()[0]], DT[dtype.split()[-1]]
+    ib, fb, norm_w = rnd(8, H).float(), (rnd(9, H) * 2 + 3).float(), (1.0 + 0.3 * rnd(10, H * dv)).float()
+    rows, cols, gates, gate_cols = _memory_inputs(5, 6, H, d, dv, dt)
+    outs, states = [], []
+    for beside in (False, True):
+        state = torch.randn(6, ops.matrix_memory_state_floats(H, d, dv), generator=torch.Generator().manual_seed(3)).to(DEV) * 0.5
+        if d & (d - 1):         # (the padded channels hold zeros)
+            dpad = 1 << (d - 1).bit_length()
+            off = state.shape[1] - H * (dv + 1) * dpad
+            state[:, off:].view(6, -1, dpad)[:, :, d:] = 0
+        for turn in range(2):
+            r, g = (rows, gates) if beside else (rows[:4], gates[:4])
+            lens, slots = ([1, 1, 1, 1, 2], [3, 0, 5, 1, 4]) if beside else ([1, 1, 1, 1], [3, 0, 5, 1])
+            out = _memory_call(r, cols, g, gate_cols, ib, fb, 9.0, norm_w, 1e-5, H, d, dv, state, lens, slots, out_dt, False, True)
+        outs.append(out[:4].double())
+        states.append(state[[3, 0, 5, 1, 2]].cpu().double())
+    assert rel_err(outs[0], outs[1]) < (2e-5 if out_dt == torch.float32 else 2.0 ** -8)
+    assert rel_err(states[0], states[1]) < 2e-6
+
+
 @pytest.mark.parametrize("H,d,dv", [(4, 64, 128), (2, 24, 40), (1, 256, 320)])
 def test_chunks_on_the_matrix_cores_round_nothing_of_the_recurrence(H, d, dv):
     """From the same bfloat16 rows, with a float output, the chunks give what the 32-bit walk gives: the state, the weights
