@@ -60,7 +60,7 @@ template <int ACT> __device__ __forceinline__ float quick_act(float v) {
 template <int FN, int FM, int OUT>
 struct TilesOut {
   static constexpr bool TURNED = OUT != OUT_SUMS;          // (a lane's four sums in float are a whole store)
-  static constexpr int CHUNK = OUT == OUT_ACT && FN > 8 ? FN / 2 : FN;          // fragments that are turned in LDS at a time
+  static constexpr int CHUNK = OUT == OUT_ACT && (FN > 8 || WaveTiles<FN, FM>::SLOTS > 2) ? FN / 2 : FN;          // fragments that are turned in LDS at a time
   static constexpr int ROW = 16 * CHUNK * (OUT == OUT_PAIRS ? 1 : 2);      // bytes of a row of them
   static constexpr int PITCH = ROW + 16, WAVE_BYTES = TURNED ? 16 * PITCH : 0;
   static constexpr int LDS = WaveTiles<FN, FM>::LDS + 4 * WAVE_BYTES;

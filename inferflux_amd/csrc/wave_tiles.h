@@ -1,7 +1,7 @@
 // The inner loop of a product of many rows by four large waves (bfloat16 in, float sums): C[n][m] = sum_k W[n][k] X[m][k] for
 // a tile of 32 FN weight rows and 32 FM rows of x; each of the workgroup's four waves, one to a SIMD, holds a quarter of the sums.
 //
-// Steps of 64 k-values of both operands are staged in LDS by loads that go there directly, two slots in turn, and each step
+// Steps of 64 k-values of both operands are staged in LDS by loads that go there directly, two slots in turn (three of tiles of 256 x 128), and each step
 // is taken in two halves: while one half's fragments are multiplied, the next half's are read.  A step of 256 x 256 is 2,048
 // cycles of matrix instructions to a SIMD, and the rest has to stay out of their way:
 //   LDS   a wave of 128 x 128 reads 32 KB a step, a third less than two of 128 x 64 (which fill LDS as long as the matrix
@@ -16,6 +16,8 @@
 //         touching it too costs more than it gives (1.05 x).
 //   ends  a workgroup takes one tile after the other and asks for a tile's first two steps before it writes the one before
 //         it out (12 us a tile without that and with exact division and expf in the activation, now 5).
+// Tiles of 256 x 128 are half the arithmetic for three quarters of the bytes and wait for loads one step ahead; their three slots reach two
+// (260 rows of 37,888 x 3,584 125 -> 107 us, 530 of 2,048 x 11,008 in six slices 34.3 -> 32.3, 300 of 17,920 x 1,536 24.1 -> 22.9).
 // Rows of 32 k-values in five slots, which reach twice as far ahead, took 1.05 x the time: half lines cost more requests.
 //
 // A row is 128 bytes in LDS, 8 pieces of 16; piece p of row r lies at p ^ (r & 7) ^ (r >> 3 & 1), so that the 16 rows a
@@ -30,7 +32,8 @@ template <int FN, int FM>
 struct WaveTiles {
   static constexpr int BN = 32 * FN, BM = 32 * FM, WN = 16 * FN, WM = 16 * FM, THREADS = 256;
   static constexpr int ROW = 128, W_BYTES = BN * ROW, STAGE = (BN + BM) * ROW;
-  static constexpr int TOUCHED = 2 * STAGE, LDS = 2 * STAGE + 1024;      // (the touches' values: 256 bytes a wave)
+  static constexpr int SLOTS = 3 * STAGE + 1024 <= 148 * 1024 ? 3 : 2;
+  static constexpr int TOUCHED = SLOTS * STAGE, LDS = SLOTS * STAGE + 1024;      // (the touches' values: 256 bytes a wave)
   static constexpr int READS = FN + FM, LOADS = FN + FM, PRODUCTS = FN * FM, AHEAD = 2;
   static_assert(FN * FM <= 64, "a wave's sums are 256 registers at most");
 
@@ -80,7 +83,7 @@ struct WaveTiles {
     }
     const int steps = (K + 63) / 64;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int s = 0; s < SLOTS; ++s) {
       if (s == steps - 1 && K % 64 != 0) cut(K);
       if (s < steps) {
 #pragma unroll
@@ -145,25 +148,52 @@ struct WaveTiles {
     for (int a = 0; a < FN; ++a)
 #pragma unroll
       for (int b = 0; b < FM; ++b) acc[a][b] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
-    if (steps > 1) tile_meet<LOADS>();          // (whatever was issued after begin() leaves the first step's loads the oldest)
+    if (steps >= SLOTS) tile_meet<(SLOTS - 1) * LOADS>();          // (whatever was issued after begin() leaves the first step's loads the oldest)
     else tile_meet<0>();
 #pragma unroll
     for (int i = 0; i < READS; ++i) read(i, 0, 0);
     int s = 0;
-    for (; s + 2 < steps; s += 2) {
-      half(0, 0, false, 0, 0);
-      meet(s > 0);
-      if (uneven && s + 2 == steps - 1) cut(K);
-      half(1, 1, true, s + 2, 0);
-      half(0, 1, false, 0, 0);
-      meet(true);
-      if (uneven && s + 3 == steps - 1) cut(K);
-      half(1, 0, true, min(s + 3, steps - 1), 1);        // (beyond the end: the last step again, into a slot that nothing reads)
-    }
-    for (; s < steps; ++s) {
-      half(0, s & 1, false, 0, 0);
-      meet(false);
-      half(1, s & 1 ^ 1, false, 0, 0);
+    if constexpr (SLOTS == 3) {
+      // step s lies in slot s % 3; the loads of step s + 2, and a touch behind them, may still be on their way where step s + 1 is met
+      auto meet3 = [&](int newer) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);        // lgkmcnt(0)
+        if (newer == 2 && touches) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LOADS + 1) : "memory");
+        else if (newer >= 1) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");
+      };
+      int at = 0;
+      for (; s + 3 < steps; ++s) {
+        const int then = at == 2 ? 0 : at + 1;
+        half(0, at, false, 0, 0);
+        meet3(s > 0 ? 2 : 1);
+        if (uneven && s + 3 == steps - 1) cut(K);
+        half(1, then, true, s + 3, at);
+        at = then;
+      }
+      for (; s < steps; ++s) {
+        const int then = at == 2 ? 0 : at + 1;
+        half(0, at, false, 0, 0);
+        meet3(0);
+        half(1, then, false, 0, 0);
+        at = then;
+      }
+    } else {
+      for (; s + 2 < steps; s += 2) {
+        half(0, 0, false, 0, 0);
+        meet(s > 0);
+        if (uneven && s + 2 == steps - 1) cut(K);
+        half(1, 1, true, s + 2, 0);
+        half(0, 1, false, 0, 0);
+        meet(true);
+        if (uneven && s + 3 == steps - 1) cut(K);
+        half(1, 0, true, min(s + 3, steps - 1), 1);        // (beyond the end: the last step again, into a slot that nothing reads)
+      }
+      for (; s < steps; ++s) {
+        half(0, s & 1, false, 0, 0);
+        meet(false);
+        half(1, s & 1 ^ 1, false, 0, 0);
+      }
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");          // (the last products' sums are there)
     meet(false);
