@@ -14,7 +14,7 @@
 //         more steps ahead by loads whose values nobody reads, which brings them as far as the L2: 2,480 cycles.  The workgroups that
 //         meet the same rows of W share the touches; the last steps touch the next tile's first ones.  x comes from the caches;
 //         touching it too costs more than it gives (1.05 x).
-//   ends  a workgroup takes one tile after the other and asks for a tile's first two steps before it writes the one before
+//   ends  a workgroup takes one tile after the other and asks for a tile's first steps before it writes the one before
 //         it out (12 us a tile without that and with exact division and expf in the activation, now 5).
 // Tiles of 256 x 128 are half the arithmetic for three quarters of the bytes and wait for loads one step ahead; their three slots reach two
 // (260 rows of 37,888 x 3,584 125 -> 107 us, 530 of 2,048 x 11,008 in six slices 34.3 -> 32.3, 300 of 17,920 x 1,536 24.1 -> 22.9).
@@ -66,7 +66,7 @@ struct WaveTiles {
     base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
   }
 
-  // Asks for a tile's first two steps (K a multiple of 8).  wb, xb: buffers that start at the tile's first row of W and
+  // Asks for a tile's first steps, a slot each (K a multiple of 8).  wb, xb: buffers that start at the tile's first row of W and
   // x, at the first of the K values; row m of x starts at byte x_offset(m), row n of W at n * w_row.
   template <class XOffset>
   __device__ __forceinline__ void begin(const tile_uintx4& wb, const tile_uintx4& xb, int K, int w_row, XOffset x_offset) {
