@@ -19,11 +19,13 @@
 //   ifx_headwise_grouped      out[t][h][:N] = W[h] x[t][h], tiles of TM rows of one head; optionally times sigmoid of a column
 //                      of a wider projected row, one per output element
 //
-// The experts' products stand on product_tiles.h, an item's result whatever shares its tile.  The heads' product, whose
+// The experts' products stand on product_tiles.h and wave_tiles.h (which of them: grouped_wave_items in ops.py), an item's result whatever shares its tile.  The heads' product, whose
 // matrices are small (K of a hundred), is heads_kernel below.
 #include "common.h"
 #include "column_gate.h"
 #include "product_tiles.h"
+#include "wave_tiles.h"
+#include "tile_acts.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -32,7 +34,9 @@ typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
-#define TM 128         // items to a tile
+#define TM 128         // items to a tile of the eight-wave kernel
+#define WAVE_ITEMS 192 // ... of the kernel by four large waves
+#define EXPERTS_GROUP 4          // tiles of items that meet a tile of W one after the other
 #define MAX_EXPERTS 1024
 
 
@@ -41,8 +45,8 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // count) and their number.  One workgroup.  The order of an expert's items among themselves is not fixed; no result
 // depends on it.  A wave adds the experts' counts up and cuts the tiles (one thread did), and
 // a thread asks for eight ids at a time: 22,800 items took 33 us with a trip for each.
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ ids, int n_items, int E, int* __restrict__ sorted,
-                                                        int* __restrict__ tile_expert, int* __restrict__ tile_start,
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ ids, int n_items, int E, int n_real, int tile_items,
+                                                        int* __restrict__ sorted, int* __restrict__ tile_expert, int* __restrict__ tile_start,
                                                         int* __restrict__ tile_count, int* __restrict__ n_tiles) {
   constexpr int AT_ONCE = 8;          // ids that a thread asks for at a time: the launch is a chain of trips to memory
   __shared__ int cnt[MAX_EXPERTS];
@@ -62,7 +66,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
   if (tid < WAVE) {          // sums over the experts before, of items and of tiles, an expert to a lane
     int at = 0, n = 0;
     for (int e0 = 0; e0 < E; e0 += WAVE) {
-      const int e = e0 + tid, c = e < E ? cnt[e] : 0, t = (c + TM - 1) / TM;
+      const int e = e0 + tid, c = e < E ? cnt[e] : 0, t = (c + tile_items - 1) / tile_items;
       int items = c, tiles = t;
 #pragma unroll
       for (int d = 1; d < WAVE; d *= 2) {
@@ -74,9 +78,10 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
         offs[e] = start;
         for (int k = 0; k < t; ++k) {
           tile_expert[first + k] = e;
-          tile_start[first + k] = start + k * TM;
-          tile_count[first + k] = min(TM, c - k * TM);
+          tile_start[first + k] = start + k * tile_items;
+          tile_count[first + k] = min(tile_items, c - k * tile_items);
         }
+        if (e == n_real - 1) n_tiles[1] = first + t;
       }
       at += __shfl(items, WAVE - 1);
       n += __shfl(tiles, WAVE - 1);
@@ -94,10 +99,12 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
   }
 }
 
-extern "C" int ifx_moe_sort(const int* ids, int n_items, int E, int* sorted, int* tile_expert, int* tile_start,
+// n_tiles [2]: all tiles, and those of the n_real experts with weights, which come first
+extern "C" int ifx_moe_sort(const int* ids, int n_items, int E, int n_real, int tile_items, int* sorted, int* tile_expert, int* tile_start,
                             int* tile_count, int* n_tiles, void* stream) {
   IFX_REQUIRE(n_items >= 0 && E > 0 && E <= MAX_EXPERTS, "moe_sort: %d items, %d experts (at most %d)", n_items, E, MAX_EXPERTS);
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, n_items, E, sorted, tile_expert,
+  IFX_REQUIRE(n_real > 0 && n_real <= E && tile_items >= 1, "moe_sort: %d of %d experts, %d items to a tile", n_real, E, tile_items);
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, n_items, E, n_real, tile_items, sorted, tile_expert,
                      tile_start, tile_count, n_tiles);
   IFX_LAUNCH_CHECK();
 }
@@ -126,27 +133,27 @@ struct ExpertsArgs {
 // before, with the pieces through registers into LDS and rows of 64 k-values padded, now 362 + 241 (730 TFLOP/s with the tiles
 // that are not full).  One size of tile for all: tiles of 64 items were 0.91 of the time where experts have 88 items and
 // matrices are small (37 for 41 us), 1.03 to 1.2 of it everywhere else.
-#define BN 128
-typedef ProductTiles<BN, TM, 32, 64, false> RowTiles;
+constexpr int TILE_BN = 128;
+typedef ProductTiles<TILE_BN, TM, 32, 64, false> RowTiles;
 template <int MODE, bool TILED>
 __global__ __launch_bounds__(RowTiles::THREADS, 4) void experts_kernel(ExpertsArgs a) {
-  typedef ProductTiles<BN, TM, 32, 64, TILED> P;
+  typedef ProductTiles<TILE_BN, TM, 32, 64, TILED> P;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[P::LDS];
   const int tid = threadIdx.x;
   int tn, tm;
-  if (!product_tile((a.NW + BN - 1) / BN, *a.n_tiles, 2, &tn, &tm)) return;
-  const int e = a.tile_expert[tm], start = a.tile_start[tm], count = min(a.tile_count[tm], TM), n0 = tn * BN;
+  if (!product_tile((a.NW + TILE_BN - 1) / TILE_BN, *a.n_tiles, 2, &tn, &tm)) return;
+  const int e = a.tile_expert[tm], start = a.tile_start[tm], count = min(a.tile_count[tm], TM), n0 = tn * TILE_BN;
   const int* items = a.sorted + start;
   if (e >= a.n_real) {        // an identity expert's tile
     if (MODE == MODE_DOWN)
-      for (int i = tid; i < count * BN; i += P::THREADS) {
-        const int m = items[i / BN], n = n0 + i % BN;
+      for (int i = tid; i < count * TILE_BN; i += P::THREADS) {
+        const int m = items[i / TILE_BN], n = n0 + i % TILE_BN;
         if (n < a.NW)
           ((float*)a.out)[((size_t)(m % a.top) * a.T + m / a.top) * a.NW + n] = a.weights[m] * (float)a.identity[(size_t)(m / a.top) * a.NW + n];
       }
     return;
   }
-  const int rows = min(BN, a.NW - n0);
+  const int rows = min(TILE_BN, a.NW - n0);
   const size_t row_values = TILED ? (size_t)((a.K + 63) / 64 * 64) : (size_t)a.K;
   const tile_uintx4 w = tile_buffer(a.w + ((size_t)e * a.NW + n0) * row_values, (unsigned)(rows * row_values) * 2u);
   const tile_uintx4 x = MODE == MODE_GATE_UP ? tile_buffer(a.x, (unsigned)a.T * (unsigned)a.K * 2u)
@@ -191,11 +198,158 @@ __global__ __launch_bounds__(RowTiles::THREADS, 4) void experts_kernel(ExpertsAr
   }
 }
 
+// The same products by four large waves, one workgroup to a CU that takes one tile of 192 items by 256 weight rows after the other
+// (wave_tiles.h; weights in tiles, whose lines are touched ahead by each workgroup for itself).  The next tile's place in the lists and its
+// items are asked for before a tile's steps, its first steps before the results go out.  What is left of the matrix rate is the tiles that are
+// not full and the last round of the chip: 20,400 items of 32 experts (2,048 wide, 1,408 inner) both products and the order of the items
+// 537 -> 477 us (740 TFLOP/s), 65,536 items 1,414 -> 1,219 (930).  Tiles of 128 items (three slots) were
+// 1.0 to 1.2 x the eight waves' time; with tiles of 256 the sums, the fragments and the rows' addresses fill the registers, and the compiler
+// moves sums about between the products in assembly, whose results it does not wait for: wrong sums.  So whoever changes this kernel looks
+// for such moves (v_accvgpr_read within 14 instructions of the product that writes it) in its assembly.
+template <int MODE, int FN, int FM>
+struct ExpertWaves {
+  typedef WaveTiles<FN, FM, true> P;
+  static constexpr int PITCH = 16 * FN + 16, WAVE_BYTES = MODE == MODE_GATE_UP ? 16 * PITCH : 0, LDS = P::LDS + 4 * WAVE_BYTES;
+};
+
+// 16 rows of a wave's activations at a time, turned in LDS so that they go out in whole lines; stores beyond the rows and columns are dropped
+template <int FN, int FM, int ACT>
+__device__ __forceinline__ void waves_gate_up_out(const WaveTiles<FN, FM, true>& p, const ExpertsArgs& a, unsigned char* lds, tile_floatx4 (&acc)[FN][FM],
+                                                  const float (&weight)[FM], int start, int count, int n0) {
+  typedef ExpertWaves<MODE_GATE_UP, FN, FM> O;
+  const int ff = a.NW / 2, m = p.wm(), rows = count - m, first = (n0 + p.wn()) / 2;
+  const unsigned long long at0 = (unsigned long long)a.out + (size_t)(start + m) * ff * 2;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at0), hi = __builtin_amdgcn_readfirstlane((unsigned)(at0 >> 32));
+  const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc((void*)((unsigned long long)hi << 32 | lo), 0,
+                                                                        __builtin_amdgcn_readfirstlane(max(0, min(16 * FM, rows)) * ff * 2), 0x00020000);
+  unsigned char* st = lds + WaveTiles<FN, FM, true>::LDS + p.wid * O::WAVE_BYTES;
+#pragma unroll
+  for (int b = 0; b < FM; ++b) {
+    const float w = weight[b];
+#pragma unroll
+    for (int c = 0; c < FN; c += 2) {
+      asm volatile("" : "+a"(acc[c][b]), "+a"(acc[c + 1][b]));          // (not before: the registers beside the sums are taken)
+      const tile_floatx4 gt = acc[c][b], up = acc[c + 1][b];
+      bf16x4 y;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = (__bf16)tile_gated<ACT>(w * gt[r], w * up[r], a.limit);
+      *(bf16x4*)(st + p.col * O::PITCH + c * 16 + p.g * 8) = y;
+    }
+    constexpr int PIECES = FN;          // of 16 bytes to a row
+#pragma unroll
+    for (int j0 = 0; j0 < 16 * PIECES; j0 += 64) {
+      const int j = j0 + p.lane, r = j / PIECES, at = 8 * (j % PIECES);
+      const bool in = r < rows - 16 * b && first + at < ff;
+      const tile_uintx4 v = *(const tile_uintx4*)(st + r * O::PITCH + 2 * at);
+      __builtin_amdgcn_raw_buffer_store_b128(v, out, in ? ((16 * b + r) * ff + first + at) * 2 : TILE_NO_ROW, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+template <int MODE, int FN, int FM>
+__global__ __launch_bounds__(256, 1) void experts_waves_kernel(ExpertsArgs a) {
+  typedef ExpertWaves<MODE, FN, FM> O;
+  typedef typename O::P P;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[O::LDS];
+  static_assert(O::LDS <= 160 * 1024 && FN % 4 == 0, "LDS");
+  const int nt = (a.NW + P::BN - 1) / P::BN, mt = a.n_tiles[1], total = nt * mt;
+  if (MODE == MODE_DOWN)          // identity experts' tiles
+    for (int tm = mt + blockIdx.x; tm < a.n_tiles[0]; tm += gridDim.x) {
+      const int* items = a.sorted + a.tile_start[tm];
+      const int count = a.tile_count[tm];
+      for (int i = 0; i < count; ++i) {
+        const int m = items[i], t = m / a.top;
+        const float w = a.weights[m];
+        float* out = (float*)a.out + ((size_t)(m - t * a.top) * a.T + t) * a.NW;
+        for (int n = threadIdx.x; n < a.NW; n += P::THREADS) out[n] = w * (float)a.identity[(size_t)t * a.NW + n];
+      }
+    }
+  const int per = (total + 7) / 8, end = min(total, (int)(blockIdx.x % 8 + 1) * per), stride = gridDim.x / 8;
+  int id = blockIdx.x % 8 * per + blockIdx.x / 8;
+  if (id >= end) return;
+  const size_t row_values = (size_t)((a.K + 63) / 64 * 64);
+  P p;
+  p.init(lds);
+  int e, start, count, n0, rows[FM];          // the tile, and where this lane's rows of x start
+  auto scalar = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  auto find = [&](int t) {          // groups of EXPERTS_GROUP tiles of x by all of W's
+    const int turn = scalar(t / (EXPERTS_GROUP * nt)), in = t - turn * EXPERTS_GROUP * nt, gm = min(EXPERTS_GROUP, mt - turn * EXPERTS_GROUP);
+    const int tn = scalar(in / gm), tm = turn * EXPERTS_GROUP + in - tn * gm;
+    e = scalar(a.tile_expert[tm]), start = scalar(a.tile_start[tm]), count = scalar(a.tile_count[tm]), n0 = tn * P::BN;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int row = (p.wid * FM + i) * 8 + p.lane / 8;
+      rows[i] = row >= count ? -1 : MODE == MODE_GATE_UP ? a.sorted[start + row] : row;
+    }
+  };
+  auto rows_of_w = [&]() {
+    return tile_buffer(a.w + ((size_t)e * a.NW + n0) * row_values, (unsigned)(min(P::BN, a.NW - n0) * row_values) * 2u);
+  };
+  auto begin = [&]() {
+    const tile_uintx4 x = MODE == MODE_GATE_UP ? tile_buffer(a.x, (unsigned)a.T * (unsigned)a.K * 2u)
+                                               : tile_buffer(a.x + (size_t)start * a.K, (unsigned)count * (unsigned)a.K * 2u);
+    p.begin(rows_of_w(), x, a.K, 0, [&](int, int i) { return rows[i] < 0 ? TILE_NO_ROW : (MODE == MODE_GATE_UP ? rows[i] / a.top : rows[i]) * a.K * 2; });
+    p.touch_tiles(a.K);
+  };
+  find(id);
+  begin();
+  while (true) {
+    const int this_start = start, this_count = count, this_n0 = n0;
+    int item[FM];
+    float weight[FM];
+#pragma unroll
+    for (int b = 0; b < FM; ++b) {
+      const int i = p.wm() + 16 * b + p.col;
+      item[b] = i < count && (MODE == MODE_DOWN || a.weigh_input) ? a.sorted[start + i] : -1;
+    }
+#pragma unroll
+    for (int b = 0; b < FM; ++b) weight[b] = item[b] >= 0 && (MODE == MODE_GATE_UP || !a.weigh_input) ? a.weights[item[b]] : 1.f;
+    id += stride;
+    const bool more = id < end;
+    if (more) find(id);
+    p.next = rows_of_w(), p.next_steps = more ? (a.K + 63) / 64 : 0;
+    if (!more) p.next[2] = 0;          // (nothing to touch)
+    tile_floatx4 acc[FN][FM];
+    p.run(lds, a.K, acc);
+    if (more) begin();
+    if constexpr (MODE == MODE_GATE_UP) {
+      switch (a.act) {
+        case ACT_GELU_TANH: waves_gate_up_out<FN, FM, ACT_GELU_TANH>(p, a, lds, acc, weight, this_start, this_count, this_n0); break;
+        case ACT_SILU: waves_gate_up_out<FN, FM, ACT_SILU>(p, a, lds, acc, weight, this_start, this_count, this_n0); break;
+        default: waves_gate_up_out<FN, FM, ACT_CLAMPED_SWISH>(p, a, lds, acc, weight, this_start, this_count, this_n0); break;
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < FM; ++b) {
+        const int t = item[b] / a.top;
+        float* out = (float*)a.out + ((size_t)(item[b] - t * a.top) * a.T + t) * a.NW;
+#pragma unroll
+        for (int c = 0; c < FN; ++c) {
+          asm volatile("" : "+a"(acc[c][b]));
+          const int n = this_n0 + p.wn() + 16 * c + 4 * p.g;
+          const tile_floatx4 v = acc[c][b];
+          if (item[b] >= 0 && n < a.NW) *(floatx4*)(out + n) = floatx4{weight[b] * v[0], weight[b] * v[1], weight[b] * v[2], weight[b] * v[3]};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (!more) break;
+  }
+}
+
 template <int MODE>
 static void launch_experts(const ExpertsArgs& a, int max_tiles, int tiled, hipStream_t s) {
-  const dim3 blocks((max_tiles * ((a.NW + BN - 1) / BN) + 7) / 8 * 8), threads(RowTiles::THREADS);
+  const dim3 blocks((max_tiles * ((a.NW + TILE_BN - 1) / TILE_BN) + 7) / 8 * 8), threads(RowTiles::THREADS);
   if (tiled) hipLaunchKernelGGL((experts_kernel<MODE, true>), blocks, threads, 0, s, a);
   else hipLaunchKernelGGL((experts_kernel<MODE, false>), blocks, threads, 0, s, a);
+}
+
+template <int MODE>
+static void launch_experts_waves(const ExpertsArgs& a, int max_tiles, hipStream_t s) {
+  const long long most = (long long)max_tiles * ((a.NW + 255) / 256);
+  const dim3 blocks(most < 256 ? (int)(most + 7) / 8 * 8 : 256);
+  hipLaunchKernelGGL((experts_waves_kernel<MODE, 8, WAVE_ITEMS / 32>), blocks, dim3(256), 0, s, a);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -333,13 +487,15 @@ __global__ __launch_bounds__(256, 2) void heads_kernel(HeadsArgs a) {
 extern "C" int ifx_moe_gate_up_grouped(const void* x, const void* w, void* act, const int* sorted, const int* tile_expert,
                                        const int* tile_start, const int* tile_count, const int* n_tiles, int max_tiles,
                                        int T, int K, int ff, int top, int n_real, int act_kind, float limit, const float* in_weights,
-                                       int tiled, void* stream) {
+                                       int tiled, int wave_items, void* stream) {
   IFX_REQUIRE(K > 0 && K % 8 == 0 && ff > 0 && ff % 16 == 0 && top > 0 && T >= 0, "moe_gate_up_grouped: K=%d must be a multiple of 8, ff=%d of 16", K, ff);
   IFX_REQUIRE((long long)T * K < (1ll << 30) - 4096, "moe_gate_up_grouped: %d rows of %d values are 2 GB or more", T, K);
   if (max_tiles <= 0 || T == 0) return 0;
   const ExpertsArgs a{(const bf16_t*)x, (const bf16_t*)w, act, sorted, tile_expert, tile_start, tile_count, n_tiles, in_weights,
                       nullptr, T, top, K, 2 * ff, n_real, act_kind, limit, in_weights ? 1 : 0};
-  launch_experts<MODE_GATE_UP>(a, max_tiles, tiled, (hipStream_t)stream);
+  IFX_REQUIRE(wave_items == 0 || (tiled && wave_items == WAVE_ITEMS), "moe_gate_up_grouped: tiles of %d items", wave_items);
+  if (wave_items) launch_experts_waves<MODE_GATE_UP>(a, max_tiles, (hipStream_t)stream);
+  else launch_experts<MODE_GATE_UP>(a, max_tiles, tiled, (hipStream_t)stream);
   IFX_LAUNCH_CHECK();
 }
 
@@ -347,13 +503,15 @@ extern "C" int ifx_moe_gate_up_grouped(const void* x, const void* w, void* act, 
 extern "C" int ifx_moe_down_grouped(const void* act, const void* w, float* parts, const float* weights, const int* sorted,
                                     const int* tile_expert, const int* tile_start, const int* tile_count, const int* n_tiles,
                                     int max_tiles, int T, int N, int ff, int top, int n_real, const void* identity,
-                                    int weigh_input, int tiled, void* stream) {
+                                    int weigh_input, int tiled, int wave_items, void* stream) {
   IFX_REQUIRE(!tiled || N % 16 == 0, "moe_down_grouped: tiled weights need N=%d to be a multiple of 16", N);
   IFX_REQUIRE(ff > 0 && ff % 8 == 0 && N > 0 && top > 0 && T >= 0, "moe_down_grouped: ff=%d must be a multiple of 8", ff);
   if (max_tiles <= 0 || T == 0) return 0;
   const ExpertsArgs a{(const bf16_t*)act, (const bf16_t*)w, parts, sorted, tile_expert, tile_start, tile_count, n_tiles, weights,
                       (const bf16_t*)identity, T, top, ff, N, n_real, 0, 0.f, weigh_input};
-  launch_experts<MODE_DOWN>(a, max_tiles, tiled, (hipStream_t)stream);
+  IFX_REQUIRE(wave_items == 0 || (tiled && wave_items == WAVE_ITEMS), "moe_down_grouped: tiles of %d items", wave_items);
+  if (wave_items) launch_experts_waves<MODE_DOWN>(a, max_tiles, (hipStream_t)stream);
+  else launch_experts<MODE_DOWN>(a, max_tiles, tiled, (hipStream_t)stream);
   IFX_LAUNCH_CHECK();
 }
 

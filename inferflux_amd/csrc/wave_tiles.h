@@ -21,17 +21,18 @@
 // Rows of 32 k-values in five slots, which reach twice as far ahead, took 1.05 x the time: half lines cost more requests.
 //
 // A row is 128 bytes in LDS, 8 pieces of 16; piece p of row r lies at p ^ (r & 7) ^ (r >> 3 & 1), so that the 16 rows a
-// fragment takes a piece of meet every bank evenly.
+// fragment takes a piece of meet every bank evenly.  With TILED W comes as the tiles of ifx_tile_weights (16 rows x 32 k-values, 1 KB), which
+// lie in LDS as they are: a fragment each, in the order of a wave's lanes.
 //
 // Sums run over k in ascending order, 32 k-values to an instruction, whatever the tile: an element of C does not depend on
 // the tile's size or what shares it.
 #pragma once
 #include "product_tiles.h"
 
-template <int FN, int FM>
+template <int FN, int FM, bool TILED = false>
 struct WaveTiles {
   static constexpr int BN = 32 * FN, BM = 32 * FM, WN = 16 * FN, WM = 16 * FM, THREADS = 256;
-  static constexpr int ROW = 128, W_BYTES = BN * ROW, STAGE = (BN + BM) * ROW;
+  static constexpr int ROW = 128, W_STEP = TILED ? 2048 : ROW, W_BYTES = BN * ROW, STAGE = (BN + BM) * ROW;
   static constexpr int SLOTS = 3 * STAGE + 1024 <= 148 * 1024 ? 3 : 2;
   static constexpr int TOUCHED = SLOTS * STAGE, LDS = SLOTS * STAGE + 1024;      // (the touches' values: 256 bytes a wave)
   static constexpr int READS = FN + FM, LOADS = FN + FM, PRODUCTS = FN * FM, AHEAD = 2;
@@ -68,18 +69,19 @@ struct WaveTiles {
   }
 
   // Asks for a tile's first steps, a slot each (K a multiple of 8).  wb, xb: buffers that start at the tile's first row of W and
-  // x, at the first of the K values; row m of x starts at byte x_offset(m), row n of W at n * w_row.
+  // x, at the first of the K values; row m of x starts at byte x_offset(m, i), where i is the
+  // number of m among the rows that this lane loads, row n of W at n * w_row.
   template <class XOffset>
   __device__ __forceinline__ void begin(const tile_uintx4& wb, const tile_uintx4& xb, int K, int w_row, XOffset x_offset) {
     w = wb, x = xb;
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
       const int row = (wid * FN + i) * 8 + lane / 8;
-      wo[i] = row * w_row + 16 * (lane % 8 ^ place(row));
+      wo[i] = TILED ? tiles_at(wid * FN + i, K) + 16 * lane : row * w_row + 16 * (lane % 8 ^ place(row));
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int row = (wid * FM + i) * 8 + lane / 8, at = x_offset(row);
+      const int row = (wid * FM + i) * 8 + lane / 8, at = x_offset(row, i);
       xo[i] = at == TILE_NO_ROW ? at : at + 16 * (lane % 8 ^ place(row));
     }
     const int steps = (K + 63) / 64;
@@ -98,6 +100,12 @@ struct WaveTiles {
     touches = set < (BN + 63) / 64;
     touch = set * 64 + lane < BN ? (set * 64 + lane) * w_row : TILE_NO_ROW;
   }
+  // ... of tiles, all of them by this workgroup: a step's lines of 8 rows, 128 bytes each, lie one after the other
+  __device__ __forceinline__ void touch_tiles(int K) {
+    const int line = 64 * wid + lane;
+    touches = 64 * wid < BN;
+    touch = line < BN ? tiles_at(line / 8, K) + 128 * (line % 8) : TILE_NO_ROW;
+  }
 
   // acc = the tile's sums.  All of the workgroup's waves are done with the slots when it returns.
   __device__ __forceinline__ void run(const unsigned char* lds, int K, tile_floatx4 (&acc)[FN][FM]) {
@@ -107,7 +115,7 @@ struct WaveTiles {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int at = col * ROW + ((4 * h + g) ^ place(col)) * 16;
-      wr[h] = wn() * ROW + at;
+      wr[h] = wn() * ROW + (TILED ? 1024 * h + 16 * lane : at);
       xr[h] = W_BYTES + wm() * ROW + at;
     }
     tile_bf16x8 wf[2][FN], xf[2][FM];
@@ -133,8 +141,8 @@ struct WaveTiles {
         for (; l < LOADS; ++l) issue(l, s, to);
         if (touches) {
           const int t = s + AHEAD;
-          if (t < steps) load_one(w, touch, t * ROW, base + TOUCHED + wid * 256);
-          else load_one(next, touch, max(0, min(t - steps, next_steps - 1)) * ROW, base + TOUCHED + wid * 256);      // (within the next one's K, which may be a step long)
+          if (t < steps) load_one(w, touch, t * W_STEP, base + TOUCHED + wid * 256);
+          else load_one(next, touch, max(0, min(t - steps, next_steps - 1)) * W_STEP, base + TOUCHED + wid * 256);      // (within the next one's K, which may be a step long)
         }
       }
     };
@@ -201,17 +209,20 @@ struct WaveTiles {
   }
 
  private:
+  // where the j-th 1 KB of a step of tiles lies: tile j % 2 along k of row tile j / 2
+  static __device__ __forceinline__ int tiles_at(int j, int K) { return j / 2 * ((K + 63) / 64 * 2048) + j % 2 * 1024; }
   __device__ __forceinline__ void issue(int i, int s, int slot) {
     const unsigned to = base + slot * STAGE;
-    if (i < FN) load(w, wo[i], s * ROW, to + (wid * FN + i) * 1024);
+    if (i < FN) load(w, wo[i], s * W_STEP, to + (wid * FN + i) * 1024);
     else load(x, xo[i - FN], s * ROW, to + W_BYTES + (wid * FM + i - FN) * 1024);
   }
   // pieces beyond K in the last step arrive as zeros
   __device__ __forceinline__ void cut(int K) {
     const int k0 = (K - 1) / 64 * 64;
+    if (!TILED)          // (tiles are padded with zeros)
 #pragma unroll
-    for (int i = 0; i < FN; ++i)
-      if (k0 + 8 * (lane % 8 ^ place((wid * FN + i) * 8 + lane / 8)) >= K) wo[i] = TILE_NO_ROW;
+      for (int i = 0; i < FN; ++i)
+        if (k0 + 8 * (lane % 8 ^ place((wid * FN + i) * 8 + lane / 8)) >= K) wo[i] = TILE_NO_ROW;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
       if (k0 + 8 * (lane % 8 ^ place((wid * FM + i) * 8 + lane / 8)) >= K) xo[i] = TILE_NO_ROW;

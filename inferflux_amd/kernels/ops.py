@@ -616,6 +616,22 @@ GROUPED_TILE_ITEMS = 128          # items of one expert to a workgroup of the gr
 GROUPED_MAX_VALUES = 2 ** 30 - 8192          # values of the rows that the product's offsets of 32 bits reach
 
 
+GROUPED_WAVE_ITEMS = 192          # ... of the product by four large waves,
+GROUPED_WAVE_MIN_ITEMS = 225      # which takes experts of so many items on average
+GROUPED_WAVE_MIN_ROUNDS = 2.6     # where its tiles take the chip so many times
+
+
+def grouped_wave_items(n_items: int, n_experts: int, pair_rows: int) -> int:
+    """Items to a tile of the product by four large waves where experts with ``pair_rows`` rows of gate and up take it, else 0.  Its tiles of
+    256 x 192 are faster by a sixth where all are full, but an expert's last one is half empty on average and so is the last round of the
+    chip (90 draws of 14 to 64 experts, 1,024 or 2,048 wide, 704 or 1,408 inner, both products and the order of the items, its time over
+    that of tiles of 128 x 128 by eight waves: beyond both lines 0.83 to 0.98, 0.89 in the mean; 100 to 225 items 0.95 to 1.37, fewer
+    1.13 to 1.54; fewer rounds 0.85 to 1.28.  20,400 items of 32 experts, 2,048 wide and 1,408 inner: 537 -> 477 us)."""
+    tiles = n_items / GROUPED_WAVE_ITEMS + n_experts / 2
+    fits = n_items >= GROUPED_WAVE_MIN_ITEMS * n_experts and tiles * -(-pair_rows // 256) >= GROUPED_WAVE_MIN_ROUNDS * COMPUTE_UNITS
+    return GROUPED_WAVE_ITEMS if fits else 0
+
+
 def grouped_takes(dtype: torch.dtype, K: int, ff: int) -> bool:
     """Whether the grouped matrix-core product takes experts of these sizes."""
     return dtype == torch.bfloat16 and K % 8 == 0 and ff % 16 == 0
@@ -647,12 +663,13 @@ def _experts(w, nm: str, shape):
 
 def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor,
                         weights: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0,
-                        weigh_input: bool = False) -> "SliceSums":
+                        weigh_input: bool = False, wave_items: int = -1) -> "SliceSums":
     """The same sum for steps of many rows, on the matrix cores: the (row, choice) items are ordered by expert on the
     device and every expert's weights meet tiles of its items (bfloat16; ``gate_up`` from ``pair_gate_up``).  Returns the
     choices' weighted outputs as ``SliceSums`` [top, T, N] (float32), which the kernel that adds them to the stream sums
     in the order of the choices.  ``n_identity``: ids from E up to E + n_identity name identity experts, whose output is
-    the row itself (N = K then); ``act``, ``limit`` and ``weigh_input`` as for ``moe_experts``."""
+    the row itself (N = K then); ``act``, ``limit`` and ``weigh_input`` as for ``moe_experts``.  ``wave_items`` (both weights as
+    ``ExpertTiles``): tiles of so many items by four large waves (128 or 192), 0 those by eight, -1 chooses (``grouped_wave_items``)."""
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
     gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
@@ -673,23 +690,26 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     if T > portion:
         for r in range(0, T, portion):
             parts[:, r:r + portion] = moe_experts_grouped(h[r:r + portion], gate_up, down, ids[r:r + portion], weights[r:r + portion], act,
-                                                          limit, n_identity, weigh_input).parts
+                                                          limit, n_identity, weigh_input, wave_items).parts
         return SliceSums(parts, torch.bfloat16)
-    max_tiles = -(-n_items // GROUPED_TILE_ITEMS) + E          # every expert may end on a tile that is not full
-    lists = torch.empty((n_items + 3 * max_tiles + 1,), dtype=torch.int32, device=h.device)
+    if wave_items < 0:
+        wave_items = grouped_wave_items(n_items, n_real, 2 * ff) if gu_tiled and down_tiled else 0
+    tile_items = wave_items or GROUPED_TILE_ITEMS
+    max_tiles = -(-n_items // tile_items) + E          # every expert may end on a tile that is not full
+    lists = torch.empty((n_items + 3 * max_tiles + 2,), dtype=torch.int32, device=h.device)
     sorted_, te, ts, tc, nt = (lists[:n_items], lists[n_items:n_items + max_tiles], lists[n_items + max_tiles:n_items + 2 * max_tiles],
                                lists[n_items + 2 * max_tiles:n_items + 3 * max_tiles], lists[n_items + 3 * max_tiles:])
-    _call(mod, "ifx_moe_sort", (P, I, I, P, P, P, P, P, P), ids.data_ptr(), n_items, E, sorted_.data_ptr(), te.data_ptr(),
+    _call(mod, "ifx_moe_sort", (P, I, I, I, I, P, P, P, P, P, P), ids.data_ptr(), n_items, E, n_real, tile_items, sorted_.data_ptr(), te.data_ptr(),
           ts.data_ptr(), tc.data_ptr(), nt.data_ptr(), _stream())
     a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)          # (in the order of ``sorted_``)
-    _call(mod, "ifx_moe_gate_up_grouped", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, P),
+    _call(mod, "ifx_moe_gate_up_grouped", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, I, P),
           h.data_ptr(), gu_ptr, a.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(), tc.data_ptr(),
           nt.data_ptr(), max_tiles, T, K, ff, top, n_real, int(act), float(limit),
-          weights.data_ptr() if weigh_input else 0, gu_tiled, _stream())
-    _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, P),
+          weights.data_ptr() if weigh_input else 0, gu_tiled, wave_items, _stream())
+    _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, I, P),
           a.data_ptr(), down_ptr, parts.data_ptr(), weights.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(),
           tc.data_ptr(), nt.data_ptr(), max_tiles, T, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0,
-          down_tiled, _stream())
+          down_tiled, wave_items, _stream())
     return SliceSums(parts, torch.bfloat16)
 
 
