@@ -20,6 +20,8 @@ from typing import Callable, Dict, Hashable, List, Sequence
 import numpy as np
 import torch
 
+from ..kernels.ops import upload
+
 
 @dataclasses.dataclass
 class StepEntry:
@@ -136,14 +138,14 @@ class StepContext:
 
     def bind(self, slab: torch.Tensor = None, pinned: torch.Tensor = None) -> None:
         """Put the step's arrays on the device: into ``slab`` through ``pinned`` when given (an
-        asynchronous copy on the current stream), else into a new tensor."""
+        asynchronous copy on the current stream), else into a new tensor (which the host does not wait for either)."""
         if pinned is not None:
             host = pinned.numpy()
         else:
             host = np.zeros(self.slab_size, dtype=np.int32)
         self.write_host(host)
         if slab is None:
-            slab = torch.from_numpy(host).to(self.device)
+            slab = upload(host, self.device)
         elif pinned is not None:
             slab.copy_(pinned, non_blocking=True)
         else:
@@ -205,4 +207,4 @@ class StepContext:
         return self._derived.get(key)
 
     def upload(self, array: np.ndarray) -> torch.Tensor:
-        return torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
+        return upload(np.ascontiguousarray(array), self.device)

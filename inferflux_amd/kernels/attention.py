@@ -279,7 +279,7 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
     T, nH, d = q.shape
     table = ctx.block_table(cache.group)
     keep_first = int(keep_first or 0) if window else 0
-    if keep_first and ctx.h_q_len.max() >= TILE_MIN and ctx.h_kv_len.max() <= window:
+    if keep_first and ctx.derived(("attention_window_whole", window), lambda: ctx.h_q_len.max() >= TILE_MIN and ctx.h_kv_len.max() <= window):
         # prompts that the window holds whole see their first keys anyway, and without them the kernel that loads straight into LDS
         # takes them (2,048 rows of 16 heads of 128 82 us, then 51; steps of single rows are captured for later lengths, too)
         keep_first = 0
@@ -294,16 +294,21 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
         return ops.attention_plain(q, cache.k, cache.v, ctx.row_req, ctx.positions, table, window, scale, keep_first, sink, gate,
                                    sinks=sinks, chunk=block)
     n_kv = cache.k.shape[1]
-    # Two query tiles per wave (128 rows per workgroup) read every key and value from LDS half as often.
-    tiled = ctx.h_q_len >= TILE_MIN
-    qt, splits, chunk = 1, 1, 0
-    if tiled.any():
-        qt, splits, chunk = choose_tiling(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, lambda t: ops.attention_tile_rows(d, t),
-                                          tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not keep_first and not block)
-    tile_rows = ops.attention_tile_rows(d, qt)
-    w = ctx.derived(("attention_work_lists", n_kv, tile_rows, nH, splits, chunk, window, d),
-                    lambda: _work_lists(ctx, n_kv, tile_rows, nH, splits, chunk, window, ops.row_waves_fit(nH, n_kv, d, ops.ROW_MAX_WAVES), d))
-    out = torch.empty((T, nH * d), dtype=q.dtype, device=q.device)
+
+    def plan():
+        # Two query tiles per wave (128 rows per workgroup) read every key and value from LDS half as often.
+        tiled = ctx.h_q_len >= TILE_MIN
+        qt, splits, chunk = 1, 1, 0
+        if tiled.any():
+            qt, splits, chunk = choose_tiling(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, lambda t: ops.attention_tile_rows(d, t),
+                                              tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not keep_first and not block)
+        tile_rows = ops.attention_tile_rows(d, qt)
+        return qt, ctx.derived(("attention_work_lists", n_kv, tile_rows, nH, splits, chunk, window, d),
+                               lambda: _work_lists(ctx, n_kv, tile_rows, nH, splits, chunk, window, ops.row_waves_fit(nH, n_kv, d, ops.ROW_MAX_WAVES), d))
+
+    # (once a step for all layers of a kind)
+    qt, w = ctx.derived(("attention_plan", n_kv, nH, d, window, keep_first, block), plan)
+    out = ops.empty((T, nH * d), q.dtype, q)
     more = dict(keep_first=keep_first, sink=sink, gate=gate, sinks=sinks, block=block) if extras else {}
     if w["n_tiles"]:
         ops.attention_tiles(q, cache.k, cache.v, out, w["tile_req"], w["tile_q0"], ctx.q_start, ctx.q_len, ctx.kv_len,

@@ -45,6 +45,9 @@ HOST_SANITIZE = os.environ.get("INFERFLUX_HOST_SANITIZE", "") == "1"
 if HOST_SANITIZE:
     HOST_FLAGS = ["-O1", "-g", "-fno-omit-frame-pointer", "-fsanitize=address,undefined", "-std=c++17", "-shared", "-fPIC"]
 
+# Host modules that are Python extensions over torch's tensors: they are built against this interpreter and this torch, which their hash covers.
+EXTENSIONS = ("host_calls",)
+
 Variant = Tuple[Tuple[str, int], ...]
 
 
@@ -74,6 +77,24 @@ def _cxx() -> str:
     return _hipcc()          # hipcc compiles plain C++ too
 
 
+def _extension_flags() -> Tuple[str, ...]:
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
+    lib = os.path.join(root, "lib")
+    return ("-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in include),
+            f"-L{lib}", f"-Wl,-rpath,{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip")
+
+
+def _host_flags(name: str) -> Sequence[str]:
+    return _extension_flags() if name in EXTENSIONS else HOST_FLAGS
+
+
 def _sources(name: str) -> Tuple[str, ...]:
     """The files a module is built from: its source, the header of the same name (its public entry points) where it
     has one, and every header of this folder that the source includes."""
@@ -95,7 +116,10 @@ def _digest(name: str, variant: Variant) -> str:
     for fn in _sources(name):
         with open(os.path.join(CSRC, fn), "rb") as f:
             h.update(f.read())
-    h.update(" ".join(HOST_FLAGS if host else FLAGS).encode())
+    h.update(" ".join(_host_flags(name) if host else FLAGS).encode())
+    if name in EXTENSIONS:
+        import torch
+        h.update(f"{sys.version_info[:2]} {torch.__version__}".encode())
     h.update(repr(variant).encode())
     return h.hexdigest()[:12]
 
@@ -125,7 +149,7 @@ def _fallback_dir(create: bool = False) -> Optional[str]:
 def _stem(name: str, variant: Variant) -> str:
     """A library's file name up to its hash (a sanitized host build has a name of its own, so that it and the
     ordinary build do not take each other for stale)."""
-    san = "-hostsan" if HOST_SANITIZE and _is_host_module(name) else ""
+    san = "-hostsan" if HOST_SANITIZE and _is_host_module(name) and name not in EXTENSIONS else ""
     return f"{name}{san}{_variant_tag(variant)}"
 
 
@@ -173,7 +197,8 @@ def compile_module(name: str, variant: Variant = (), force: bool = False) -> str
                 return out
             tmp = f"{out}.{os.getpid()}.tmp"
             defines = [f"-D{k}={v}" for k, v in variant]
-            cmd = [_cxx(), *HOST_FLAGS, *defines, src, "-o", tmp] if host else [_hipcc(), *FLAGS, *defines, src, "-o", tmp]
+            # (an extension's libraries come after its source)
+            cmd = [_cxx(), src, *_host_flags(name), *defines, "-o", tmp] if host else [_hipcc(), *FLAGS, *defines, src, "-o", tmp]
             label = f"{name}{_variant_tag(variant)}"
             _progress(f"compiling {label} for {'the host' if host else ARCH} ...")
             t0 = time.time()
@@ -197,11 +222,23 @@ def compile_module(name: str, variant: Variant = (), force: bool = False) -> str
             fcntl.flock(lock, fcntl.LOCK_UN)
 
 
+def load_extension(name: str):
+    """The Python extension ``name``, built first where it is not."""
+    import importlib.util
+    from importlib.machinery import ExtensionFileLoader
+    path = compile_module(name)
+    spec = importlib.util.spec_from_file_location(name, path, loader=ExtensionFileLoader(name, path))
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
 class KernelModule:
     """A loaded library; functions are looked up by name, with their argument types set once."""
 
     def __init__(self, name: str, variant: Variant, path: str):
         self.name, self.variant, self.path = name, variant, path
+        self.entries: Dict[str, object] = {}        # what the native calls keep of each function (see host_calls.cpp)
         self.lib = ctypes.CDLL(path)
         self.lib.ifx_last_error.restype = ctypes.c_char_p
         self._fns: Dict[str, ctypes._CFuncPtr] = {}

@@ -15,7 +15,7 @@ import torch
 
 from .. import log
 from .device import ARCH, COMPUTE_UNITS, N_XCD
-from .library import KernelModule, Variant, load_module
+from .library import KernelModule, Variant, load_extension, load_module
 
 P = ctypes.c_void_p
 I = ctypes.c_int
@@ -57,6 +57,7 @@ class KernelError(RuntimeError):
 
 def module_variants() -> Iterable[Tuple[str, Variant]]:
     yield ("cache_manager", ())       # host code: the cache's bookkeeping
+    yield ("host_calls", ())          # host code: checks, results and calls of every launch
     yield ("core", ())
     yield ("gemm_f32", ())
     yield ("attn_plain", ())
@@ -105,8 +106,7 @@ def _dt(t: torch.Tensor) -> int:
         raise KernelError(f"unsupported element type {t.dtype} (float32 or bfloat16)") from None
 
 
-def _check(t: torch.Tensor, name: str, shape=None, dtype=None) -> None:
-    # on every launch: written for the case that nothing is wrong
+def _check_in_python(t: torch.Tensor, name: str, shape=None, dtype=None) -> None:
     if not (isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous()):
         if not isinstance(t, torch.Tensor):
             raise KernelError(f"{name}: not a tensor")
@@ -127,25 +127,41 @@ def _check(t: torch.Tensor, name: str, shape=None, dtype=None) -> None:
             raise KernelError(f"{name}: shape {tuple(ts)}, expected {tuple(shape)}")
 
 
-def _ptr(t: Optional[torch.Tensor]) -> int:
-    return 0 if t is None else t.data_ptr()
+def upload(array, device) -> torch.Tensor:
+    """The numpy ``array`` on ``device``, by a copy on the current stream that the host does not wait for: from pinned memory of its own,
+    which torch's allocator hands out again only after the copy (from ordinary memory ``to`` waits for everything launched before it)."""
+    if torch.device(device).type != "cuda":
+        return torch.from_numpy(array).to(device)
+    pageable = torch.from_numpy(array)
+    pinned = torch.empty(pageable.shape, dtype=pageable.dtype, pin_memory=True)
+    pinned.copy_(pageable)
+    return pinned.to(device, non_blocking=True)
 
 
-def _stream() -> int:
-    # torch's current stream as a raw handle; the accessor that skips building a Stream object is used
-    # where this torch has it (it is called once per launch)
-    if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
-    return torch.cuda.current_stream().cuda_stream
-
-
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-
-
-def _call(mod: KernelModule, fname: str, argtypes, *args) -> None:
-    rc = mod.fn(fname, argtypes)(*args)
+def _call_by_ctypes(mod: KernelModule, fname: str, argtypes, *args) -> None:
+    rc = mod.fn(fname, argtypes)(*(a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args))
     if rc != 0:
-        raise KernelError(f"{fname}: {mod.last_error()} (code {rc})")
+        _call_failed(mod, fname, rc)
+
+
+def _call_failed(mod: KernelModule, fname: str, rc: int) -> None:
+    raise KernelError(f"{fname}: {mod.last_error()} (code {rc})")
+
+
+_WORDS = {P: "p", I: "i", LL: "l", F: "f"}
+
+
+def _entry(mod: KernelModule, fname: str, argtypes):
+    """What the native call keeps of a function: its address and argument types, or None where one of them is no plain word."""
+    f = mod.fn(fname, argtypes)
+    types = "".join(_WORDS.get(t) or ("a" if issubclass(t, ctypes._Pointer) else "?") for t in argtypes)
+    found = mod.entries[fname] = _native.entry(ctypes.cast(f, P).value, types)
+    return found
+
+
+_native = load_extension("host_calls")
+_native.connect(_check_in_python, _call_by_ctypes, _call_failed, _entry)
+_check, _call, empty, _stream = _native.check, _native.call, _native.empty, _native.stream      # (see csrc/host_calls.cpp)
 
 
 # ----------------------------------------------------------------------------------------
@@ -154,9 +170,9 @@ def embedding(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0) -> tor
     _check(ids, "ids", (None,), torch.int32)
     _check(table, "table", (None, None))
     T, H = ids.shape[0], table.shape[1]
-    out = torch.empty((T, H), dtype=torch.float32, device=table.device)
+    out = empty((T, H), torch.float32, table)
     _call(load_module("core"), "ifx_embedding", (P, P, I, P, I, I, F, P),
-          ids.data_ptr(), table.data_ptr(), _dt(table), out.data_ptr(), T, H, float(scale), _stream())
+          ids, table, _dt(table), out, T, H, float(scale), _stream())
     return out
 
 
@@ -169,12 +185,12 @@ def embedding_scaled(ids: torch.Tensor, table: torch.Tensor, norm_weight: torch.
     _check(norm_weight, "norm_weight", (H,))
     if T > 16:
         raise KernelError(f"embedding_scaled: {T} rows (at most 16)")
-    out = torch.empty((T, H), dtype=torch.float32, device=table.device)
-    rows = torch.empty((T, H), dtype=torch.bfloat16, device=table.device)
-    pieces = torch.empty((-(-H // 4096), 16), dtype=torch.float32, device=table.device)
+    out = empty((T, H), torch.float32, table)
+    rows = empty((T, H), torch.bfloat16, table)
+    pieces = empty((-(-H // 4096), 16), torch.float32, table)
     _call(load_module("core"), "ifx_embedding_norm", (P, P, I, P, I, P, P, P, I, I, F, P),
-          ids.data_ptr(), table.data_ptr(), _dt(table), norm_weight.data_ptr(), _dt(norm_weight), out.data_ptr(), rows.data_ptr(),
-          pieces.data_ptr(), T, H, float(scale), _stream())
+          ids, table, _dt(table), norm_weight, _dt(norm_weight), out, rows,
+          pieces, T, H, float(scale), _stream())
     return out, ScaledRows(rows, pieces, H, eps, norm_weight)
 
 
@@ -207,10 +223,10 @@ def add_rmsnorm(residual: torch.Tensor, delta: Optional[torch.Tensor], weight: t
     if rows is not None:
         _check(rows, "rows", (None,), torch.int32)
         n = rows.shape[0]
-    out = torch.empty((n, H), dtype=out_dtype, device=residual.device)
+    out = empty((n, H), out_dtype, residual)
     _call(load_module("core"), "ifx_add_rmsnorm", (P, P, I, P, I, P, I, P, I, I, F, I, I, LL, F, P),
-          residual.data_ptr(), _ptr(delta), _dt(delta) if delta is not None else 0, weight.data_ptr(),
-          _dt(weight), out.data_ptr(), _DT[out_dtype], _ptr(rows), n, H, float(eps),
+          residual, delta, _dt(delta) if delta is not None else 0, weight,
+          _dt(weight), out, _DT[out_dtype], rows, n, H, float(eps),
           1 if (delta is not None and rows is None) else 0, n_slices, T * H, float(delta_scale), _stream())
     return out
 
@@ -248,9 +264,9 @@ def _add_terms_rmsnorm(residual, delta: "DeltaSum", weight, eps, out_dtype, rows
     if rows is not None:
         _check(rows, "rows", (None,), torch.int32)
         n = rows.shape[0]
-    out = torch.empty((n, H), dtype=out_dtype, device=residual.device)
+    out = empty((n, H), out_dtype, residual)
     _call(load_module("deltas"), "ifx_add_terms_rmsnorm", (P, *_TERM_TYPES, P, I, P, I, P, I, I, F, I, P),
-          residual.data_ptr(), *_term_args(delta, T, H), weight.data_ptr(), _dt(weight), out.data_ptr(), _DT[out_dtype], _ptr(rows), n, H,
+          residual, *_term_args(delta, T, H), weight, _dt(weight), out, _DT[out_dtype], rows, n, H,
           float(eps), 0 if rows is not None else 1, _stream())
     return out
 
@@ -261,18 +277,18 @@ def join_stream(residual: torch.Tensor, delta, other: torch.Tensor, dtype: torch
     _check(residual, "residual", (None, None), torch.float32)
     T, H = residual.shape
     _check(other, "other", (T, H), torch.float32)
-    out = torch.empty((T, 2 * H), dtype=dtype, device=residual.device)
+    out = empty((T, 2 * H), dtype, residual)
     delta = DeltaSum.of(delta).in_pieces(MAX_DELTA_PIECES)
     _call(load_module("deltas"), "ifx_join_stream", (P, *_TERM_TYPES, P, P, I, I, I, P),
-          residual.data_ptr(), *_term_args(delta, T, H), other.data_ptr(), out.data_ptr(), _DT[dtype], T, H, _stream())
+          residual, *_term_args(delta, T, H), other, out, _DT[dtype], T, H, _stream())
     return out
 
 
 def query_temperature(positions: torch.Tensor, coef: float, every: int) -> torch.Tensor:
     """float32 [T]: 1 + coef ln(floor((p + 1) / every) + 1) of int32 ``positions`` [T]."""
     _check(positions, "positions", (None,), torch.int32)
-    out = torch.empty(positions.shape, dtype=torch.float32, device=positions.device)
-    _call(load_module("core"), "ifx_query_temperature", (P, P, I, F, I, P), positions.data_ptr(), out.data_ptr(), positions.shape[0],
+    out = empty(positions.shape, torch.float32, positions)
+    _call(load_module("core"), "ifx_query_temperature", (P, P, I, F, I, P), positions, out, positions.shape[0],
           float(coef), int(every), _stream())
     return out
 
@@ -290,7 +306,7 @@ def zero_slot(table: torch.Tensor, slot: int, n_slots: int) -> None:
     _check(table, "table", (None, 2), torch.int64)
     if not 0 <= slot < n_slots:
         raise KernelError(f"zero_slot: slot {slot} of {n_slots}")
-    _call(load_module("core"), "ifx_zero_slot", (P, I, LL, P), table.data_ptr(), table.shape[0], int(slot), _stream())
+    _call(load_module("core"), "ifx_zero_slot", (P, I, LL, P), table, table.shape[0], int(slot), _stream())
 
 
 def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, magnitude: float = 1.0):
@@ -298,10 +314,10 @@ def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, magnitude: float
     _check(positions, "positions", (None,), torch.int32)
     _check(inv_freq, "inv_freq", (None,), torch.float32)
     T, n = positions.shape[0], inv_freq.shape[0]
-    cs = torch.empty((T, n), dtype=torch.float32, device=positions.device)
-    sn = torch.empty((T, n), dtype=torch.float32, device=positions.device)
+    cs = empty((T, n), torch.float32, positions)
+    sn = empty((T, n), torch.float32, positions)
     _call(load_module("core"), "ifx_rope_table", (P, P, P, P, I, I, F, P),
-          positions.data_ptr(), inv_freq.data_ptr(), cs.data_ptr(), sn.data_ptr(), T, n, float(magnitude), _stream())
+          positions, inv_freq, cs, sn, T, n, float(magnitude), _stream())
     return cs, sn
 
 
@@ -364,15 +380,15 @@ def rope_append(qkv: torch.Tensor, bias: Optional[torch.Tensor], slots: Optional
         _check(kn, "k norm weight", (head_dim,), qn.dtype)
     if q_mult is not None:
         _check(q_mult, "q_mult", (T,), torch.float32)
-    q = torch.empty((T, n_heads, head_dim), dtype=dtype, device=qkv.device)
+    q = empty((T, n_heads, head_dim), dtype, qkv)
     _call(load_module("core"), "ifx_rope_append",
           (P, I, P, I, P, P, P, I, I, I, I, I, I, I, P, P, P, I, LL, I, I, P, I, F, P, F, P, P, P, I, F, I, P, P),
-          qkv.data_ptr(), _DT[dtype], _ptr(bias), _dt(bias) if bias is not None else 0, _ptr(slots),
-          _ptr(cos) if rope_style != ROPE_NONE else 0, _ptr(sin) if rope_style != ROPE_NONE else 0, rope_style,
-          rotary_dim, T, n_heads, n_kv_heads, head_dim, page_size, q.data_ptr(), _ptr(k_cache), _ptr(v_cache),
-          n_slices, T * width, dv, gate_cols, _ptr(gate_out), 1 if unit_norm_eps is not None else 0,
-          float(unit_norm_eps or 0.0), _ptr(v_first), float(v_mix), _ptr(v_out), _ptr(qn), _ptr(kn),
-          _dt(qn) if qn is not None else 0, float(pre_eps) if qn is not None else 0.0, int(extra_cols), _ptr(q_mult), _stream())
+          qkv, _DT[dtype], bias, _dt(bias) if bias is not None else 0, slots,
+          cos if rope_style != ROPE_NONE else None, sin if rope_style != ROPE_NONE else None, rope_style,
+          rotary_dim, T, n_heads, n_kv_heads, head_dim, page_size, q, k_cache, v_cache,
+          n_slices, T * width, dv, gate_cols, gate_out, 1 if unit_norm_eps is not None else 0,
+          float(unit_norm_eps or 0.0), v_first, float(v_mix), v_out, qn, kn,
+          _dt(qn) if qn is not None else 0, float(pre_eps) if qn is not None else 0.0, int(extra_cols), q_mult, _stream())
     return q
 
 
@@ -384,9 +400,9 @@ def swiglu(gate_up: torch.Tensor, interleaved: bool = False, act: int = ACT_SILU
     T, two_i = gate_up.shape
     if two_i % 2:
         raise KernelError("swiglu: odd width")
-    out = torch.empty((T, two_i // 2), dtype=gate_up.dtype, device=gate_up.device)
+    out = empty((T, two_i // 2), gate_up.dtype, gate_up)
     _call(load_module("core"), "ifx_swiglu", (P, P, I, I, I, I, I, F, P),
-          gate_up.data_ptr(), out.data_ptr(), _dt(gate_up), T, two_i // 2, 1 if interleaved else 0, int(act), float(limit), _stream())
+          gate_up, out, _dt(gate_up), T, two_i // 2, 1 if interleaved else 0, int(act), float(limit), _stream())
     return out
 
 
@@ -418,10 +434,10 @@ def layernorm(x: torch.Tensor, delta, weight: torch.Tensor, eps: float, out_dtyp
     if rows is not None:
         _check(rows, "rows", (None,), torch.int32)
         n = rows.shape[0]
-    out = torch.empty((n, H), dtype=out_dtype, device=x.device)
+    out = empty((n, H), out_dtype, x)
     _call(load_module("layernorm"), "ifx_layernorm", (P, I, P, I, I, LL, P, I, P, I, P, I, I, F, P),
-          x.data_ptr(), _dt(x), dp, dd, n_slices, stride, weight.data_ptr(), _dt(weight), out.data_ptr(), _DT[out_dtype],
-          _ptr(rows), n, H, float(eps), _stream())
+          x, _dt(x), dp, dd, n_slices, stride, weight, _dt(weight), out, _DT[out_dtype],
+          rows, n, H, float(eps), _stream())
     return out
 
 
@@ -434,9 +450,9 @@ def add_layernorm(stream: torch.Tensor, delta, weight: torch.Tensor, eps: float,
     T, H = stream.shape
     _check(weight, "weight", (H,))
     dp, dd, n_slices, stride = _delta_args(delta, (T, H), "delta")
-    cast = torch.empty((T, H), dtype=cast_dtype, device=stream.device) if cast_dtype not in (None, torch.float32) else None
+    cast = empty((T, H), cast_dtype, stream) if cast_dtype not in (None, torch.float32) else None
     _call(load_module("layernorm"), "ifx_add_layernorm", (P, P, I, I, LL, P, I, P, I, I, I, F, P),
-          stream.data_ptr(), dp, dd, n_slices, stride, weight.data_ptr(), _dt(weight), _ptr(cast),
+          stream, dp, dd, n_slices, stride, weight, _dt(weight), cast,
           _DT[cast_dtype] if cast is not None else 0, T, H, float(eps), _stream())
     return stream if cast_dtype == torch.float32 else cast
 
@@ -444,8 +460,8 @@ def add_layernorm(stream: torch.Tensor, delta, weight: torch.Tensor, eps: float,
 def cast_rows(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """The float32 rows ``x`` rounded to ``dtype`` (bfloat16)."""
     _check(x, "x", None, torch.float32)
-    out = torch.empty(x.shape, dtype=dtype, device=x.device)
-    _call(load_module("layernorm"), "ifx_cast_rows", (P, P, I, LL, P), x.data_ptr(), out.data_ptr(), _DT[dtype], x.numel(), _stream())
+    out = empty(x.shape, dtype, x)
+    _call(load_module("layernorm"), "ifx_cast_rows", (P, P, I, LL, P), x, out, _DT[dtype], x.numel(), _stream())
     return out
 
 
@@ -480,11 +496,11 @@ def latent_finish(y, q_norm: Optional[torch.Tensor], kv_norm: Optional[torch.Ten
         _check(v_cache, "v_cache", (k_cache.shape[0], 1, None, page_size), dtype)
         if v_cache.shape[2] not in (kv_rank, kv_rank + rot_dim):
             raise KernelError(f"latent_finish: values of {v_cache.shape[2]} rows (the latent's {kv_rank}, or {kv_rank + rot_dim} with the key part)")
-    cq = torch.empty((T, q_rank), dtype=dtype, device=any_norm.device) if q_rank else None
+    cq = empty((T, q_rank), dtype, any_norm) if q_rank else None
     _call(load_module("latent"), "ifx_latent_finish", (P, I, I, LL, P, P, I, P, P, I, P, P, P, P, I, I, I, I, I, I, F, I, I, P),
-          yp, yd, n_slices, stride, _ptr(q_norm), _ptr(kv_norm), _dt(any_norm), _ptr(cos) if rot_dims else 0,
-          _ptr(sin) if rot_dims else 0, rot_dims, _ptr(slots), _ptr(cq), _ptr(k_cache) if slots is not None else 0,
-          _ptr(v_cache) if slots is not None else 0, _DT[dtype], T, q_rank, kv_rank, rot_dim, page_size, float(eps),
+          yp, yd, n_slices, stride, q_norm, kv_norm, _dt(any_norm), cos if rot_dims else None,
+          sin if rot_dims else None, rot_dims, slots, cq, k_cache if slots is not None else None,
+          v_cache if slots is not None else None, _DT[dtype], T, q_rank, kv_rank, rot_dim, page_size, float(eps),
           v_cache.shape[2] if slots is not None else kv_rank, width, _stream())
     return cq
 
@@ -510,7 +526,7 @@ def headwise(x: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, t
     if rot_dims:
         _check(cos, "cos", (T, rot_dims // 2), torch.float32)
         _check(sin, "sin", (T, rot_dims // 2), torch.float32)
-    out = torch.empty((T, n_heads, N + tail), dtype=x.dtype, device=x.device)
+    out = empty((T, n_heads, N + tail), x.dtype, x)
     gate_args = (0, 0, 0, 0, 0)
     if gate is not None:
         rows, col = gate
@@ -527,13 +543,13 @@ def headwise(x: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, t
     if x.dtype == torch.bfloat16 and T >= HEADWISE_GROUPED_MIN_ROWS and K % 8 == 0 and x_head % 8 == 0 and x.shape[1] % 8 == 0:
         # many rows: the products on the matrix cores, and of the other kernel only the tails
         _call(load_module("grouped_gemm"), "ifx_headwise_grouped", (P, P, P, I, I, I, I, I, I, I, P, I, I, I, LL, P),
-              x.data_ptr(), weight.data_ptr(), out.data_ptr(), T, n_heads, K, N, x.shape[1], x_head, N + tail, *gate_args, _stream())
+              x, weight, out, T, n_heads, K, N, x.shape[1], x_head, N + tail, *gate_args, _stream())
         if not tail:
             return out
         tail_only = 1
     _call(load_module("latent"), "ifx_headwise", (P, P, P, I, I, I, I, I, I, I, I, P, P, I, I, P, I, I, I, LL, P),
-          x.data_ptr(), weight.data_ptr(), out.data_ptr(), _dt(x), T, n_heads, K, N, x.shape[1], x_head, tail,
-          _ptr(cos) if rot_dims else 0, _ptr(sin) if rot_dims else 0, rot_dims, tail_only, *gate_args, _stream())
+          x, weight, out, _dt(x), T, n_heads, K, N, x.shape[1], x_head, tail,
+          cos if rot_dims else None, sin if rot_dims else None, rot_dims, tail_only, *gate_args, _stream())
     return out
 
 
@@ -557,15 +573,15 @@ def moe_route(h: torch.Tensor, router, top: int, groups: int = 1, keep_groups: i
     E = rows.shape[0]
     # (in 32-bit the kernel forms them whatever the rows: a row's sums then never depend on what shares its step)
     z = linear(h, router, out_dtype=torch.float32) if (T > ROUTE_FUSED_MAX_ROWS and h.dtype == torch.bfloat16) else None
-    ids = torch.empty((T, top), dtype=torch.int32, device=h.device)
-    weights = torch.empty((T, top), dtype=torch.float32, device=h.device)
+    ids = empty((T, top), torch.int32, h)
+    weights = empty((T, top), torch.float32, h)
     if bias is not None:
         _check(bias, "bias", (E,), torch.float32)
     if choice_bias is not None:
         _check(choice_bias, "choice_bias", (E,), torch.float32)
     _call(load_module("moe"), "ifx_moe_route", (P, P, I, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, P),
-          h.data_ptr(), rows.data_ptr(), _dt(h), _ptr(z), ids.data_ptr(), weights.data_ptr(), T, K, E, top, groups, keep_groups,
-          group_top, 1 if softmax else 0, 1 if renormalize else 0, float(scale), _ptr(bias), _ptr(choice_bias), _stream())
+          h, rows, _dt(h), z, ids, weights, T, K, E, top, groups, keep_groups,
+          group_top, 1 if softmax else 0, 1 if renormalize else 0, float(scale), bias, choice_bias, _stream())
     return ids, weights
 
 
@@ -602,13 +618,13 @@ def moe_experts(h: torch.Tensor, gate: torch.Tensor, up: Optional[torch.Tensor],
     if n_identity and N != K:
         raise KernelError(f"moe_experts: identity experts hand back the row itself, so N={N} must equal K={K}")
     mod = load_module("moe")
-    a = torch.empty((T, top, ff), dtype=h.dtype, device=h.device)
+    a = empty((T, top, ff), h.dtype, h)
     _call(mod, "ifx_moe_gate_up", (P, P, P, P, P, I, I, I, I, I, I, I, I, F, P, P),
-          h.data_ptr(), gate.data_ptr(), _ptr(up), ids.data_ptr(), a.data_ptr(), _dt(h), T, K, ff, top, 1 if paired else 0, E,
-          int(act), float(limit), weights.data_ptr() if weigh_input else 0, _stream())
-    out = torch.empty((T, N), dtype=h.dtype, device=h.device)
+          h, gate, up, ids, a, _dt(h), T, K, ff, top, 1 if paired else 0, E,
+          int(act), float(limit), weights if weigh_input else None, _stream())
+    out = empty((T, N), h.dtype, h)
     _call(mod, "ifx_moe_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, P),
-          a.data_ptr(), down.data_ptr(), ids.data_ptr(), weights.data_ptr(), out.data_ptr(), _dt(h), T, N, ff, top, E, h.data_ptr(), 1 if weigh_input else 0, _stream())
+          a, down, ids, weights, out, _dt(h), T, N, ff, top, E, h, 1 if weigh_input else 0, _stream())
     return out
 
 
@@ -685,7 +701,7 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
         raise KernelError(f"moe_experts_grouped: identity experts hand back the row itself, so N={N} must equal K={K}")
     n_items = T * top
     n_real, E = E, E + int(n_identity)
-    parts = torch.empty((top, T, N), dtype=torch.float32, device=h.device)
+    parts = empty((top, T, N), torch.float32, h)
     portion = GROUPED_MAX_VALUES // K
     if T > portion:
         for r in range(0, T, portion):
@@ -696,19 +712,19 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
         wave_items = grouped_wave_items(n_items, n_real, 2 * ff) if gu_tiled and down_tiled else 0
     tile_items = wave_items or GROUPED_TILE_ITEMS
     max_tiles = -(-n_items // tile_items) + E          # every expert may end on a tile that is not full
-    lists = torch.empty((n_items + 3 * max_tiles + 2,), dtype=torch.int32, device=h.device)
+    lists = empty((n_items + 3 * max_tiles + 2,), torch.int32, h)
     sorted_, te, ts, tc, nt = (lists[:n_items], lists[n_items:n_items + max_tiles], lists[n_items + max_tiles:n_items + 2 * max_tiles],
                                lists[n_items + 2 * max_tiles:n_items + 3 * max_tiles], lists[n_items + 3 * max_tiles:])
-    _call(mod, "ifx_moe_sort", (P, I, I, I, I, P, P, P, P, P, P), ids.data_ptr(), n_items, E, n_real, tile_items, sorted_.data_ptr(), te.data_ptr(),
-          ts.data_ptr(), tc.data_ptr(), nt.data_ptr(), _stream())
-    a = torch.empty((n_items, ff), dtype=torch.bfloat16, device=h.device)          # (in the order of ``sorted_``)
+    _call(mod, "ifx_moe_sort", (P, I, I, I, I, P, P, P, P, P, P), ids, n_items, E, n_real, tile_items, sorted_, te,
+          ts, tc, nt, _stream())
+    a = empty((n_items, ff), torch.bfloat16, h)          # (in the order of ``sorted_``)
     _call(mod, "ifx_moe_gate_up_grouped", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, I, P),
-          h.data_ptr(), gu_ptr, a.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(), tc.data_ptr(),
-          nt.data_ptr(), max_tiles, T, K, ff, top, n_real, int(act), float(limit),
-          weights.data_ptr() if weigh_input else 0, gu_tiled, wave_items, _stream())
+          h, gu_ptr, a, sorted_, te, ts, tc,
+          nt, max_tiles, T, K, ff, top, n_real, int(act), float(limit),
+          weights if weigh_input else None, gu_tiled, wave_items, _stream())
     _call(mod, "ifx_moe_down_grouped", (P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, I, P),
-          a.data_ptr(), down_ptr, parts.data_ptr(), weights.data_ptr(), sorted_.data_ptr(), te.data_ptr(), ts.data_ptr(),
-          tc.data_ptr(), nt.data_ptr(), max_tiles, T, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0,
+          a, down_ptr, parts, weights, sorted_, te, ts,
+          tc, nt, max_tiles, T, N, ff, top, n_real, h, 1 if weigh_input else 0,
           down_tiled, wave_items, _stream())
     return SliceSums(parts, torch.bfloat16)
 
@@ -745,13 +761,13 @@ def moe_few_choose(h: torch.Tensor, router, top: int, groups: int = 1, keep_grou
             _check(t, nm, (E,), torch.float32)
     mod, stream = load_module("moe_few"), _stream()
     slices = mod.fn("ifx_moe_logit_slices", (I,))(K)
-    z = torch.empty((slices, T, E), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_logits", (P, P, P, I, I, I, P, I, F, F, P, P), h.data_ptr(), rows.data_ptr(), z.data_ptr(), T, K, E, *scale_args,
-          _ptr(factor), stream)
-    ids = torch.empty((T, top), dtype=torch.int32, device=h.device)
-    weights = torch.empty((T, top), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_choose", (P, I, P, P, I, I, I, I, I, I, I, I, F, P, P, P), z.data_ptr(), slices, ids.data_ptr(), weights.data_ptr(),
-          T, E, top, groups, keep_groups, group_top, 1 if softmax else 0, 1 if renormalize else 0, float(scale), _ptr(bias), _ptr(choice_bias), stream)
+    z = empty((slices, T, E), torch.float32, h)
+    _call(mod, "ifx_moe_logits", (P, P, P, I, I, I, P, I, F, F, P, P), h, rows, z, T, K, E, *scale_args,
+          factor, stream)
+    ids = empty((T, top), torch.int32, h)
+    weights = empty((T, top), torch.float32, h)
+    _call(mod, "ifx_moe_choose", (P, I, P, P, I, I, I, I, I, I, I, I, F, P, P, P), z, slices, ids, weights,
+          T, E, top, groups, keep_groups, group_top, 1 if softmax else 0, 1 if renormalize else 0, float(scale), bias, choice_bias, stream)
     return ids, weights
 
 
@@ -784,15 +800,15 @@ def moe_few_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, 
         _, shared_down, down_form = _experts(shared[1], "shared down", (1, N, shared_ff))
         if shape[1] % 32 or (gu_form, down_form) != (gu_tiled, down_tiled):
             raise KernelError(f"moe_few: a shared expert of {shape[1]} gate and up rows (a multiple of 32), in the experts' form")
-    a = torch.empty((T * (top * ff + shared_ff),), dtype=torch.bfloat16, device=h.device)
+    a = empty((T * (top * ff + shared_ff),), torch.bfloat16, h)
     shared_a = a.data_ptr() + 2 * T * top * ff
-    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P, P, I, F, P, P), h.data_ptr(), gu_ptr, a.data_ptr(), ids.data_ptr(),
-          T, E, K, ff, top, n_real, int(act), float(limit), weights.data_ptr() if weigh_input else 0, gu_tiled,
-          shared_gu, shared_a, shared_ff, float(shared_limit), _ptr(factor), stream)
-    parts = torch.empty((top + (1 if shared is not None else 0), T, N), dtype=torch.float32, device=h.device)
-    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, P, P), a.data_ptr(), down_ptr, parts.data_ptr(),
-          weights.data_ptr(), ids.data_ptr(), T, E, N, ff, top, n_real, h.data_ptr(), 1 if weigh_input else 0, down_tiled,
-          shared_a, shared_down, shared_ff, _ptr(factor), stream)
+    _call(mod, "ifx_moe_few_gate_up", (P, P, P, P, I, I, I, I, I, I, I, F, P, I, P, P, I, F, P, P), h, gu_ptr, a, ids,
+          T, E, K, ff, top, n_real, int(act), float(limit), weights if weigh_input else None, gu_tiled,
+          shared_gu, shared_a, shared_ff, float(shared_limit), factor, stream)
+    parts = empty((top + (1 if shared is not None else 0), T, N), torch.float32, h)
+    _call(mod, "ifx_moe_few_down", (P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, P, P), a, down_ptr, parts,
+          weights, ids, T, E, N, ff, top, n_real, h, 1 if weigh_input else 0, down_tiled,
+          shared_a, shared_down, shared_ff, factor, stream)
     return SliceSums(parts, torch.bfloat16)
 
 
@@ -820,9 +836,9 @@ def gemm_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     if bias is not None:
         _check(bias, "bias", (N,), torch.float32)
     out_dtype = out_dtype or x.dtype
-    out = torch.empty((M, N if gated is None else N // 2), dtype=out_dtype, device=x.device)
-    _call(load_module("gemm_f32"), "ifx_gemm_f32", (P, I, P, P, P, I, I, I, I, I, F, P), x.data_ptr(), _dt(x), weight.data_ptr(), _ptr(bias),
-          out.data_ptr(), _DT[out_dtype], M, N, K, -1 if gated is None else int(gated), float(limit), _stream())
+    out = empty((M, N if gated is None else N // 2), out_dtype, x)
+    _call(load_module("gemm_f32"), "ifx_gemm_f32", (P, I, P, P, P, I, I, I, I, I, F, P), x, _dt(x), weight, bias,
+          out, _DT[out_dtype], M, N, K, -1 if gated is None else int(gated), float(limit), _stream())
     return out
 
 
@@ -872,8 +888,8 @@ def tile_weights(weight: torch.Tensor, order: Optional[torch.Tensor] = None, til
         _check(order, "order", (n_tiles,), torch.int32)
         if sorted(order.tolist()) != list(range(n_tiles)):
             raise KernelError("tile_weights: order is not a permutation of the weight's row tiles")
-    out = torch.empty((_tiled_size(N, K, tile_rows),), dtype=torch.bfloat16, device=weight.device)
-    _call(mod, "ifx_tile_weights", (P, P, I, I, P, I, P), weight.data_ptr(), out.data_ptr(), N, K, _ptr(order), tile_rows, _stream())
+    out = empty((_tiled_size(N, K, tile_rows),), torch.bfloat16, weight)
+    _call(mod, "ifx_tile_weights", (P, P, I, I, P, I, P), weight, out, N, K, order, tile_rows, _stream())
     return out
 
 
@@ -1053,7 +1069,7 @@ class SliceSums:
         S, M, N = self.parts.shape
         out = torch.empty((M, N), dtype=dtype or self.dtype, device=self.parts.device)
         _call(load_module("gemm_wide"), "ifx_sum_slices", (P, P, I, I, LL, P),
-              self.parts.data_ptr(), out.data_ptr(), _DT[out.dtype], S, M * N, _stream())
+              self.parts, out, _DT[out.dtype], S, M * N, _stream())
         return out
 
 
@@ -1101,14 +1117,14 @@ def linear_into_stream(x: torch.Tensor, weight: LinearWeight, stream: torch.Tens
         raise KernelError(f"linear_into_stream: not for {M} rows times a {tuple(weight.rows.shape)} weight")
     _check(stream, "stream", (M, N), torch.float32)
     _check(norm_weight, "norm_weight", (N,))
-    rows = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    rows = empty((M, N), torch.bfloat16, x)
     tile_rows = 16 if weight.tiled is None else weight.tile_rows
-    pieces = torch.empty((-(-N // tile_rows), 16), dtype=torch.float32, device=x.device)    # one piece per row tile
+    pieces = empty((-(-N // tile_rows), 16), torch.float32, x)    # one piece per row tile
     w = weight.rows if weight.tiled is None else weight.tiled
     _call(load_module("gemm_bf16"), "ifx_skinny_gemm", _SKINNY_ARGS,
-          x.data_ptr(), w.data_ptr(), 0, DT_F32, M, N, K, 0, 0, 0, 2, 0 if weight.tiled is None else tile_rows, 0,
-          0, 0, 0.0, 0.0, stream.data_ptr(), norm_weight.data_ptr(), 1 if norm_weight.dtype == torch.float32 else 0, rows.data_ptr(),
-          pieces.data_ptr(), float(mult), 0, 0, _stream())
+          x, w, 0, DT_F32, M, N, K, 0, 0, 0, 2, 0 if weight.tiled is None else tile_rows, 0,
+          0, 0, 0.0, 0.0, stream, norm_weight, 1 if norm_weight.dtype == torch.float32 else 0, rows,
+          pieces, float(mult), 0, 0, _stream())
     return ScaledRows(rows, pieces, N, eps, norm_weight)
 
 
@@ -1150,11 +1166,11 @@ def qkv_rope_append(x: torch.Tensor, weight: LinearWeight, bias: Optional[torch.
         _check(slots, "slots", (M,), torch.int32)
         _check(k_cache, "k_cache", (None, n_kv_heads, page_size, head_dim), torch.bfloat16)
         _check(v_cache, "v_cache", (k_cache.shape[0], n_kv_heads, head_dim, page_size), torch.bfloat16)
-    q = torch.empty((M, n_heads, head_dim), dtype=torch.bfloat16, device=x.device)
+    q = empty((M, n_heads, head_dim), torch.bfloat16, x)
     _call(load_module("gemm_bf16"), "ifx_qkv_rope", (P, P, I, I, P, I, P, P, P, I, I, I, I, P, P, P, I, I, P, I, F, F, P),
-          x.data_ptr(), weight.tiled.data_ptr(), M, K, _ptr(bias), _dt(bias) if bias is not None else 0, _ptr(slots),
-          cos.data_ptr(), sin.data_ptr(), n_heads, n_kv_heads, head_dim, page_size, q.data_ptr(), _ptr(k_cache),
-          _ptr(v_cache), waves, unroll, *scale, _stream())
+          x, weight.tiled, M, K, bias, _dt(bias) if bias is not None else 0, slots,
+          cos, sin, n_heads, n_kv_heads, head_dim, page_size, q, k_cache,
+          v_cache, waves, unroll, *scale, _stream())
     return q
 
 
@@ -1197,12 +1213,12 @@ def skinny_gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
         raise KernelError(f"skinny_gemm: M={M} must be <= {SKINNY_MAX_M} and K={K} a multiple of 8")
     if swiglu_pairs and N % 2:
         raise KernelError("skinny_gemm: gate/up pairs need an even number of weight rows")
-    out = torch.empty((M, N // 2 if swiglu_pairs else N), dtype=out_dtype, device=x.device)
+    out = empty((M, N // 2 if swiglu_pairs else N), out_dtype, x)
     if order is not None and (tiled is None or swiglu_pairs):
         raise KernelError("skinny_gemm: a tile order goes with a tiled copy and a plain product")
     _call(load_module("gemm_bf16"), "ifx_skinny_gemm", _SKINNY_ARGS,
-          x.data_ptr(), (weight if tiled is None else tiled).data_ptr(), out.data_ptr(), _DT[out_dtype], M, N, K, nt, waves,
-          unroll, epilogue, 0 if tiled is None else tile_rows, _ptr(order), *scale, 0, 0, 0, 0, 0,
+          x, (weight if tiled is None else tiled), out, _DT[out_dtype], M, N, K, nt, waves,
+          unroll, epilogue, 0 if tiled is None else tile_rows, order, *scale, 0, 0, 0, 0, 0,
           1.0, 0, apart, _stream())
     return out
 
@@ -1233,15 +1249,21 @@ def wide_gemm(x, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, 
     mod = load_module("gemm_wide")
     if _tiled_size(N, K, weight.tile_rows) != weight.tiled.numel():
         raise KernelError(f"wide_gemm: the copy is not that of a [{N}, {K}] weight in tiles of {weight.tile_rows} rows")
-    plan = mod.fn("ifx_wide_gemm_plan", (I, I, I, I, I, I, I))(M, N, K, waves, slices, 1 if swiglu_pairs else 0, weight.tile_rows)
+    plan = _wide_plan(M, N, K, waves, slices, 1 if swiglu_pairs else 0, weight.tile_rows)
     n_waves, n_slices = plan // 256, plan % 256
-    part = torch.empty((n_slices, M, N), dtype=torch.float32, device=x.device) if n_slices > 1 else None
+    part = empty((n_slices, M, N), torch.float32, x) if n_slices > 1 else None
     keep = keep_slices and n_slices > 1
-    out = None if keep else torch.empty((M, N // 2 if swiglu_pairs else N), dtype=out_dtype, device=x.device)
+    out = None if keep else empty((M, N // 2 if swiglu_pairs else N), out_dtype, x)
     _call(mod, "ifx_wide_gemm", (P, P, P, I, P, I, I, I, I, I, I, P, I, P, I, F, F, I, I, P),
-          x.data_ptr(), weight.tiled.data_ptr(), _ptr(out), _DT[out_dtype], _ptr(part), M, N, K, n_waves, n_slices,
-          _GATED_EPILOGUE[act] if swiglu_pairs else 0, _ptr(weight.order), weight.tile_rows, *scale, 0, 0, _stream())
+          x, weight.tiled, out, _DT[out_dtype], part, M, N, K, n_waves, n_slices,
+          _GATED_EPILOGUE[act] if swiglu_pairs else 0, weight.order, weight.tile_rows, *scale, 0, 0, _stream())
     return SliceSums(part, out_dtype) if keep else out
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_plan(M: int, N: int, K: int, waves: int, slices: int, pairs: int, tile_rows: int) -> int:
+    """waves * 256 + slices of the product that shares x through LDS."""
+    return load_module("gemm_wide").fn("ifx_wide_gemm_plan", (I, I, I, I, I, I, I))(M, N, K, waves, slices, pairs, tile_rows)
 
 
 def ring_gemm(x: torch.Tensor, weight: LinearWeight, out_dtype: torch.dtype = torch.bfloat16, row_tiles: int = 0, slices: int = 0,
@@ -1262,11 +1284,11 @@ def ring_gemm(x: torch.Tensor, weight: LinearWeight, out_dtype: torch.dtype = to
         raise KernelError(f"ring_gemm: the copy is not that of a [{N}, {K}] weight in tiles of {weight.tile_rows} rows")
     row_tiles, steps = ring_plan(M, N, K, weight.tile_rows, swiglu_pairs or plain_act is not None or slices == 1, row_tiles, slices)
     n_slices = -(-(-(-K // 128)) // steps)
-    part = torch.empty((n_slices, M, N), dtype=torch.float32, device=x.device) if n_slices > 1 else None
-    out = None if n_slices > 1 else torch.empty((M, N // 2 if swiglu_pairs else N), dtype=out_dtype, device=x.device)
+    part = empty((n_slices, M, N), torch.float32, x) if n_slices > 1 else None
+    out = None if n_slices > 1 else empty((M, N // 2 if swiglu_pairs else N), out_dtype, x)
     _call(load_module("gemm_ring"), "ifx_ring_gemm", (P, P, P, I, P, I, I, I, I, I, I, I, P, I, P),
-          x.data_ptr(), weight.tiled.data_ptr(), _ptr(out), _DT[out_dtype], _ptr(part), M, N, K, row_tiles, n_slices, steps,
-          _GATED_EPILOGUE[act] if swiglu_pairs else (_PLAIN_EPILOGUE[plain_act] if plain_act is not None else 0), _ptr(weight.order),
+          x, weight.tiled, out, _DT[out_dtype], part, M, N, K, row_tiles, n_slices, steps,
+          _GATED_EPILOGUE[act] if swiglu_pairs else (_PLAIN_EPILOGUE[plain_act] if plain_act is not None else 0), weight.order,
           weight.tile_rows, _stream())
     if n_slices == 1:
         return out
@@ -1277,6 +1299,7 @@ def ring_gemm(x: torch.Tensor, weight: LinearWeight, out_dtype: torch.dtype = to
 RING_DEEP_STEPS = 48          # steps of 128 k-values from which a slice's own traffic, not its start, sets the row tiles to a workgroup
 
 
+@functools.lru_cache(maxsize=4096)
 def ring_plan(M: int, N: int, K: int, tile_rows: int, one_slice: bool, row_tiles: int = 0, slices: int = 0) -> Tuple[int, int]:
     """(row tiles to a workgroup, steps of 128 k-values to a slice): about one workgroup to each of the 256 compute units.  Weights that
     are cut into slices of K take two row tiles where K is short (896 x 4,864 at 64 rows 7.3 us, 8.0 with eight) and, where it is
@@ -1293,6 +1316,7 @@ def ring_plan(M: int, N: int, K: int, tile_rows: int, one_slice: bool, row_tiles
     return row_tiles, -(-steps // min(slices, steps))
 
 
+@functools.lru_cache(maxsize=4096)
 def ring_takes(M: int, N: int, K: int, tile_rows: int, one_slice: bool) -> bool:
     """Whether 17 to 64 rows go to ``ring_gemm`` instead of ``wide_gemm``: where a row of workgroups holds the weight's row tiles, up to
     six to a workgroup for gate/up and one a compute unit for weights that are cut into slices (us at 17 / 32 / 64 rows, wide : ring)
@@ -1303,6 +1327,7 @@ def ring_takes(M: int, N: int, K: int, tile_rows: int, one_slice: bool) -> bool:
     return 17 <= M <= SKINNY_MAX_M and -(-N // tile_rows) <= (6 if one_slice else 1) * COMPUTE_UNITS and K < 1 << 20
 
 
+@functools.lru_cache(maxsize=4096)
 def _ring_in_one_slice(M: int, N: int, K: int, tile_rows: int, keep_slices: bool) -> bool:
     """Whether ``wide_gemm`` hands 17 to 64 rows times a weight that it would cut into slices of K to ``ring_gemm`` uncut: up to 4,096 k-values
     where nobody adds slices on the way, up to 2,048 where the reader does (us at 17 / 32 / 64 rows: slices and their sum, slices alone, uncut)
@@ -1376,17 +1401,17 @@ def linear_blocks(x: torch.Tensor, weight: "LinearWeight", block_rows: int, out_
         raise KernelError(f"linear_blocks: not for {n} inputs of {M} rows times a {tuple(weight.rows.shape)} weight in blocks of {block_rows}")
     tiles = block_rows // 16
     if kind == "skinny":
-        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-        _call(load_module("gemm_bf16"), "ifx_skinny_gemm", _SKINNY_ARGS, x.data_ptr(), weight.tiled.data_ptr(), out.data_ptr(), _DT[out_dtype],
+        out = empty((M, N), out_dtype, x)
+        _call(load_module("gemm_bf16"), "ifx_skinny_gemm", _SKINNY_ARGS, x, weight.tiled, out, _DT[out_dtype],
               M, N, K, 0 if tiles % 2 == 0 else 1, 0, 0, 0, 16, 0, 0, 0, 0.0, 0.0, 0, 0, 0, 0, 0, 1.0, tiles, n, _stream())
         return out
     mod = load_module("gemm_wide")
-    plan = mod.fn("ifx_wide_gemm_plan", (I, I, I, I, I, I, I))(M, N, K, 8, 0, 0, 16)
+    plan = _wide_plan(M, N, K, 8, 0, 0, 16)
     n_slices = plan % 256
-    part = torch.empty((n_slices, M, N), dtype=torch.float32, device=x.device) if n_slices > 1 else None
-    out = torch.empty((M, N), dtype=out_dtype, device=x.device)
+    part = empty((n_slices, M, N), torch.float32, x) if n_slices > 1 else None
+    out = empty((M, N), out_dtype, x)
     _call(mod, "ifx_wide_gemm", (P, P, P, I, P, I, I, I, I, I, I, P, I, P, I, F, F, I, I, P),
-          x.data_ptr(), weight.tiled.data_ptr(), out.data_ptr(), _DT[out_dtype], _ptr(part), M, N, K, 8, n_slices, 0, 0, 16, 0, 0, 0.0, 0.0,
+          x, weight.tiled, out, _DT[out_dtype], part, M, N, K, 8, n_slices, 0, 0, 16, 0, 0, 0.0, 0.0,
           tiles, n, _stream())
     return out
 
@@ -1405,10 +1430,10 @@ def staged_gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
         raise KernelError("staged_gemm: gate/up pairs need an even number of weight rows")
     mod = load_module("gemm_bf16")
     n_slices = 1 if swiglu_pairs else mod.fn("ifx_staged_gemm_slices", (I, I, I, I))(M, N, K, slices)
-    part = torch.empty((n_slices, M, N), dtype=torch.float32, device=x.device) if n_slices > 1 else None
-    out = torch.empty((M, N // 2 if swiglu_pairs else N), dtype=out_dtype, device=x.device)
+    part = empty((n_slices, M, N), torch.float32, x) if n_slices > 1 else None
+    out = empty((M, N // 2 if swiglu_pairs else N), out_dtype, x)
     _call(mod, "ifx_staged_gemm", (P, P, P, I, P, I, I, I, I, I, I, P),
-          x.data_ptr(), weight.data_ptr(), out.data_ptr(), _DT[out_dtype], _ptr(part), M, N, K, slices, unroll,
+          x, weight, out, _DT[out_dtype], part, M, N, K, slices, unroll,
           _GATED_EPILOGUE[act] if swiglu_pairs else 0, _stream())
     return out
 
@@ -1485,6 +1510,7 @@ LIBRARY_SLICE_MIN_K = 2048      # k-values a slice of a library product keeps at
 LIBRARY_MAX_SLICES = 8
 
 
+@functools.lru_cache(maxsize=4096)
 def library_k_slices(M: int, N: int, K: int) -> int:
     """Into how many slices of K a product that goes to the library is cut when the caller adds partial sums anyway.
     A product of many rows with a deep, narrow weight (down: 3,584 x 18,944) has few output tiles (the library's are
@@ -1615,8 +1641,8 @@ def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limi
     _check(pairs, "weight_pairs", (None, None), torch.bfloat16)
     N, K = pairs.shape
     _check(x, "x", (None, K), torch.bfloat16)
-    out = torch.empty((x.shape[0], N // 2), dtype=torch.bfloat16, device=x.device)
-    _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x.data_ptr(), pairs.data_ptr(), out.data_ptr(),
+    out = empty((x.shape[0], N // 2), torch.bfloat16, x)
+    _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x, pairs, out,
           x.shape[0], N, K, 0, int(act), float(limit), int(tile), _stream())
     return out
 
@@ -1627,8 +1653,8 @@ def act_tiles(x: torch.Tensor, weight: torch.Tensor, act: int, tile: int = -1) -
     _check(weight, "weight", (None, None), torch.bfloat16)
     N, K = weight.shape
     _check(x, "x", (None, K), torch.bfloat16)
-    out = torch.empty((x.shape[0], N), dtype=torch.bfloat16, device=x.device)
-    _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x.data_ptr(), weight.data_ptr(), out.data_ptr(),
+    out = empty((x.shape[0], N), torch.bfloat16, x)
+    _call(load_module("gemm_tiles"), "ifx_gemm_tiles", _TILES_ARGS, x, weight, out,
           x.shape[0], N, K, 1, int(act), 0.0, int(tile), _stream())
     return out
 
@@ -1639,8 +1665,8 @@ def sums_tiles(x: torch.Tensor, weight: torch.Tensor, slices: int, slice_k: int,
     _check(weight, "weight", (None, None), torch.bfloat16)
     N, K = weight.shape
     _check(x, "x", (None, K), torch.bfloat16)
-    parts = torch.empty((slices, x.shape[0], N), dtype=torch.float32, device=x.device)
-    _call(load_module("gemm_tiles"), "ifx_gemm_tiles_sums", (P, P, P, I, I, I, I, I, I, P), x.data_ptr(), weight.data_ptr(), parts.data_ptr(),
+    parts = empty((slices, x.shape[0], N), torch.float32, x)
+    _call(load_module("gemm_tiles"), "ifx_gemm_tiles_sums", (P, P, P, I, I, I, I, I, I, P), x, weight, parts,
           x.shape[0], N, K, int(slices), int(slice_k), int(tile), _stream())
     return SliceSums(parts, torch.bfloat16)
 
@@ -1716,12 +1742,12 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     _check(block_table, "block_table", (None, None), torch.int32)
     if gate is not None:
         _check(gate, "gate", (T, nH), torch.float32)
-    out = torch.empty((T, nH * dv), dtype=q.dtype, device=q.device)
+    out = empty((T, nH * dv), q.dtype, q)
     _call(load_module("attn_plain"), "ifx_attn_plain", (P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, P, P, I, I, F, F, F, I, P),
-          q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _dt(q), row_req.data_ptr(),
-          positions.data_ptr(), block_table.data_ptr(), block_table.shape[1], T, nH, nKV, d // maps, dv, page_size,
-          int(window or 0), float(scale), int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), _ptr(gate),
-          _ptr(sinks), int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), int(row_waves), _stream())
+          q, k_cache, v_cache, out, _dt(q), row_req,
+          positions, block_table, block_table.shape[1], T, nH, nKV, d // maps, dv, page_size,
+          int(window or 0), float(scale), int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), gate,
+          sinks, int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), int(row_waves), _stream())
     return out
 
 
@@ -1799,12 +1825,12 @@ def delta_rule(u: torch.Tensor, rows: torch.Tensor, cols: Tuple[int, int, int], 
     ch, ks, cols = delta_layout(d, dv, single_tokens)
     if state_offset + H * dv * ch * ks > state.shape[1]:
         raise KernelError("delta_rule: the state rows are too short")
-    out = torch.empty((T, H * dv), dtype=u.dtype, device=u.device)
-    o_raw = torch.empty((T, H * dv), dtype=torch.float32, device=u.device)
+    out = empty((T, H * dv), u.dtype, u)
+    o_raw = empty((T, H * dv), torch.float32, u)
     _call(load_module("delta"), "ifx_delta_rule", (P, I, P, I, I, I, I, I, P, P, P, I, F, P, LL, LL, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P),
-          u.data_ptr(), ldu, rows.data_ptr(), ldr, col_g, col_b, col_a, _dt(u), A_log.data_ptr(), dt_bias.data_ptr(),
-          norm_w.data_ptr(), _dt(norm_w), float(eps), state.data_ptr(), state.shape[1], int(state_offset), q_start.data_ptr(),
-          q_len.data_ptr(), slots.data_ptr(), out.data_ptr(), o_raw.data_ptr(), T, R, H, G, d, dv, ch, ks, cols, _stream())
+          u, ldu, rows, ldr, col_g, col_b, col_a, _dt(u), A_log, dt_bias,
+          norm_w, _dt(norm_w), float(eps), state, state.shape[1], int(state_offset), q_start,
+          q_len, slots, out, o_raw, T, R, H, G, d, dv, ch, ks, cols, _stream())
     return out
 
 
@@ -1815,8 +1841,8 @@ def diff_expand(q: torch.Tensor) -> torch.Tensor:
     T, H, two_d = q.shape
     if two_d % 2:
         raise KernelError("diff_expand: a row of two maps has an even number of elements")
-    out = torch.empty((T, 2 * H, two_d), dtype=q.dtype, device=q.device)
-    _call(load_module("rowwise"), "ifx_diff_expand", (P, P, I, LL, I, P), q.data_ptr(), out.data_ptr(), _dt(q), T * H, two_d // 2, _stream())
+    out = empty((T, 2 * H, two_d), q.dtype, q)
+    _call(load_module("rowwise"), "ifx_diff_expand", (P, P, I, LL, I, P), q, out, _dt(q), T * H, two_d // 2, _stream())
     return out
 
 
@@ -1825,8 +1851,8 @@ def diff_combine(a: torch.Tensor, n_heads: int, dv: int, lam: float, out_scale: 
     mean square over dv (eps inside the root), times out_scale."""
     _check(a, "a", (None, 2 * n_heads * dv))
     T = a.shape[0]
-    out = torch.empty((T, n_heads * dv), dtype=a.dtype, device=a.device)
-    _call(load_module("rowwise"), "ifx_diff_combine", (P, P, I, LL, I, F, F, F, P), a.data_ptr(), out.data_ptr(), _dt(a), T * n_heads, dv,
+    out = empty((T, n_heads * dv), a.dtype, a)
+    _call(load_module("rowwise"), "ifx_diff_combine", (P, P, I, LL, I, F, F, F, P), a, out, _dt(a), T * n_heads, dv,
           float(lam), float(out_scale), float(eps), _stream())
     return out
 
@@ -1839,7 +1865,7 @@ def stream_add(stream: torch.Tensor, rows: Optional[torch.Tensor] = None, vec: O
         _check(rows, "rows", (T, H), torch.float32)
     if vec is not None:
         _check(vec, "vec", (H,))
-    _call(load_module("rowwise"), "ifx_stream_add", (P, P, P, I, I, I, P), stream.data_ptr(), _ptr(rows), _ptr(vec),
+    _call(load_module("rowwise"), "ifx_stream_add", (P, P, P, I, I, I, P), stream, rows, vec,
           _dt(vec) if vec is not None else 0, T, H, _stream())
     return stream
 
@@ -1863,10 +1889,10 @@ def causal_conv_silu(x: torch.Tensor, channels: int, weight: torch.Tensor, bias:
     R = q_start.shape[0]
     for t, nm in ((q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
         _check(t, nm, (R,), torch.int32)
-    out = torch.empty((T, channels), dtype=x.dtype, device=x.device)
+    out = empty((T, channels), x.dtype, x)
     _call(load_module("ssm"), "ifx_causal_conv", (P, I, I, P, P, I, P, LL, P, P, P, P, P, I, I, I, I, P),
-          x.data_ptr(), _dt(x), ld, weight.data_ptr(), _ptr(bias), _dt(weight), state.data_ptr(), state.shape[1],
-          row_req.data_ptr(), q_start.data_ptr(), q_len.data_ptr(), slots.data_ptr(), out.data_ptr(), T, R, channels, taps, _stream())
+          x, _dt(x), ld, weight, bias, _dt(weight), state, state.shape[1],
+          row_req, q_start, q_len, slots, out, T, R, channels, taps, _stream())
     return out
 
 
@@ -1896,22 +1922,22 @@ def selective_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor,
     R = q_start.shape[0]
     for t, nm in ((q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
         _check(t, nm, (R,), torch.int32)
-    out = torch.empty((T, C), dtype=u.dtype, device=u.device)
+    out = empty((T, C), u.dtype, u)
     n_chunks, max_chunk, lists = 0, 0, (0, 0, 0, 0, 0, 0)
     if chunks is not None:
         n_chunks, max_chunk = chunks["req"].shape[0], int(chunks["rows"])
         for nm in ("req", "t0", "len"):
             _check(chunks[nm], f"chunks.{nm}", (n_chunks,), torch.int32)
         _check(chunks["req_chunk0"], "chunks.req_chunk0", (R + 1,), torch.int32)
-        chunk_state = torch.empty((n_chunks, C, N), dtype=torch.float32, device=u.device)
-        chunk_dt = torch.empty((n_chunks, C), dtype=torch.float32, device=u.device)
+        chunk_state = empty((n_chunks, C, N), torch.float32, u)
+        chunk_dt = empty((n_chunks, C), torch.float32, u)
         lists = (chunks["req"].data_ptr(), chunks["t0"].data_ptr(), chunks["len"].data_ptr(), chunks["req_chunk0"].data_ptr(),
                  chunk_state.data_ptr(), chunk_dt.data_ptr())
     _call(load_module("ssm"), "ifx_selective_scan",
           (P, I, P, P, P, P, I, P, I, P, I, P, LL, LL, P, P, P, P, I, I, I, I, I, I, P, P, P, P, P, P, P),
-          u.data_ptr(), _dt(u), dt_raw.data_ptr(), dt_bias.data_ptr(), A.data_ptr(), bc.data_ptr(), bc.shape[1], D.data_ptr(),
-          _dt(D), z.data_ptr(), z.stride(0) if T else C, state.data_ptr(), state.shape[1], int(state_offset), q_start.data_ptr(),
-          q_len.data_ptr(), slots.data_ptr(), out.data_ptr(), T, R, C, N, n_chunks, max_chunk, *lists, _stream())
+          u, _dt(u), dt_raw, dt_bias, A, bc, bc.shape[1], D,
+          _dt(D), z, z.stride(0) if T else C, state, state.shape[1], int(state_offset), q_start,
+          q_len, slots, out, T, R, C, N, n_chunks, max_chunk, *lists, _stream())
     return out
 
 
@@ -1926,7 +1952,7 @@ def scan_chunks(q_start, q_len, chunk: int, device) -> Dict[str, object]:
         first.append(len(req))
     n = len(req)
     pad = lambda v: v + [0] * (-len(v) % 4)
-    packed = torch.from_numpy(np.asarray(pad(req) + pad(t0) + pad(ln) + first, dtype=np.int32)).to(device)
+    packed = upload(np.asarray(pad(req) + pad(t0) + pad(ln) + first, dtype=np.int32), device)
     w = n + -n % 4
     return {"req": packed[:n], "t0": packed[w:w + n], "len": packed[2 * w:2 * w + n], "req_chunk0": packed[3 * w:3 * w + len(first)],
             "rows": int(chunk)}       # (the most rows a chunk has: the kernels keep a chunk's B and C in LDS)
@@ -1994,13 +2020,13 @@ def gla_scan(rows: torch.Tensor, cols: Tuple[int, int, int, int], z: torch.Tenso
     dp, parts = gla_layout(d, dv)
     if state_offset + n_heads * dv * parts * dp > state.shape[1]:
         raise KernelError("gla_scan: the state rows are too short")
-    out = torch.empty((T, HV), dtype=rows.dtype, device=rows.device)
+    out = empty((T, HV), rows.dtype, rows)
     base, size = rows.data_ptr(), rows.element_size()
     n_chunks, lists, _keep = _chunk_lists(chunks, R, HV * parts * dp, HD, rows.device)
     _call(load_module("gla"), "ifx_gla_scan", _GLA_ARGS,
-          base + q_col * size, base + k_col * size, base + v_col * size, base + g_col * size, _dt(rows), _dt(out), ld, z.data_ptr(),
-          _ptr(z_bias), 1.0 / float(tau), float(q_scale), float(eps), norm_weight.data_ptr(), _dt(norm_weight), 0, state.data_ptr(),
-          state.shape[1], int(state_offset), q_start.data_ptr(), q_len.data_ptr(), slots.data_ptr(), out.data_ptr(), T, R, n_heads, d, dv,
+          base + q_col * size, base + k_col * size, base + v_col * size, base + g_col * size, _dt(rows), _dt(out), ld, z,
+          z_bias, 1.0 / float(tau), float(q_scale), float(eps), norm_weight, _dt(norm_weight), 0, state,
+          state.shape[1], int(state_offset), q_start, q_len, slots, out, T, R, n_heads, d, dv,
           dp, parts, n_chunks, *lists, _stream())
     return out
 
@@ -2043,10 +2069,10 @@ def shifted_mixes(h: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, state_
     R = q_start.shape[0]
     for t, nm in ((q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
         _check(t, nm, (R,), torch.int32)
-    out = torch.empty((mu.shape[0], T, H), dtype=h.dtype, device=h.device)
+    out = empty((mu.shape[0], T, H), h.dtype, h)
     _call(load_module("time_mix"), "ifx_shifted_mixes", (P, I, P, P, LL, LL, P, P, P, P, P, I, I, I, P),
-          h.data_ptr(), _dt(h), mu.data_ptr(), state.data_ptr(), state.shape[1], int(state_offset), row_req.data_ptr(), q_start.data_ptr(),
-          q_len.data_ptr(), slots.data_ptr(), out.data_ptr(), T, H, mu.shape[0], _stream())
+          h, _dt(h), mu, state, state.shape[1], int(state_offset), row_req, q_start,
+          q_len, slots, out, T, H, mu.shape[0], _stream())
     return out
 
 
@@ -2056,8 +2082,8 @@ def lowrank_tanh(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     r, C = w.shape
     T = a.shape[0]
     lda = _check_rows(a, "a", T, r, torch.float32)
-    z = torch.empty((T, C), dtype=torch.float32, device=w.device)
-    _call(load_module("time_mix"), "ifx_lowrank_tanh", (P, I, P, I, P, I, I, I, P), a.data_ptr(), lda, w.data_ptr(), _dt(w), z.data_ptr(), T, r, C,
+    z = empty((T, C), torch.float32, w)
+    _call(load_module("time_mix"), "ifx_lowrank_tanh", (P, I, P, I, P, I, I, I, P), a, lda, w, _dt(w), z, T, r, C,
           _stream())
     return z
 
@@ -2084,12 +2110,12 @@ def time_mix_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     dp, parts = gla_layout(d, d)
     if state_offset + HD * parts * dp > state.shape[1]:
         raise KernelError("time_mix_scan: the state rows are too short")
-    out = torch.empty((T, HD), dtype=out_dtype, device=r.device)
+    out = empty((T, HD), out_dtype, r)
     n_chunks, lists, _keep = _chunk_lists(chunks, R, HD * parts * dp, HD, r.device)
     _call(load_module("gla", TIME_MIX), "ifx_gla_scan", _GLA_ARGS,
-          r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), _dt(r), _DT[out_dtype], lds[0], z.data_ptr(), w0.data_ptr(), 1.0, 1.0,
-          float(eps), norm_weight.data_ptr(), _dt(norm_weight), u.data_ptr(), state.data_ptr(), state.shape[1], int(state_offset),
-          q_start.data_ptr(), q_len.data_ptr(), slots.data_ptr(), out.data_ptr(), T, R, n_heads, d, d, dp, parts, n_chunks, *lists, _stream())
+          r, k, v, g, _dt(r), _DT[out_dtype], lds[0], z, w0, 1.0, 1.0,
+          float(eps), norm_weight, _dt(norm_weight), u, state, state.shape[1], int(state_offset),
+          q_start, q_len, slots, out, T, R, n_heads, d, d, dp, parts, n_chunks, *lists, _stream())
     return out
 
 
@@ -2170,8 +2196,8 @@ def matrix_memory(rows: torch.Tensor, cols: Tuple[int, int, int, int], gates: to
     s_off = _memory_max_floats(n_heads)
     if s_off + n_heads * (dv + 1) * ch * ks > state.shape[1]:
         raise KernelError("matrix_memory: the state rows are too short")
-    out = torch.empty((T, HV), dtype=out_dtype, device=rows.device)
-    scratch = torch.empty((T * n_heads * (dv + 2) + R * n_heads,), dtype=torch.float32, device=rows.device)
+    out = empty((T, HV), out_dtype, rows)
+    scratch = empty((T * n_heads * (dv + 2) + R * n_heads,), torch.float32, rows)
     o_raw = scratch.data_ptr()
     nq = o_raw + 4 * T * n_heads * dv
     floor = nq + 4 * T * n_heads
@@ -2185,15 +2211,15 @@ def matrix_memory(rows: torch.Tensor, cols: Tuple[int, int, int, int], gates: to
         for nm in ("req", "t0", "len"):
             _check(chunks[nm], f"chunks.{nm}", (n_chunks,), torch.int32)
         _check(chunks["req_chunk0"], "chunks.req_chunk0", (R + 1,), torch.int32)
-        gates_scratch = torch.empty((3 * n_heads * T + 2 * n_heads * n_chunks,), dtype=torch.float32, device=rows.device)
-        chunk_state = torch.empty((n_chunks, n_heads * (dv + 1) * ch * ks), dtype=torch.float32, device=rows.device)
+        gates_scratch = empty((3 * n_heads * T + 2 * n_heads * n_chunks,), torch.float32, rows)
+        chunk_state = empty((n_chunks, n_heads * (dv + 1) * ch * ks), torch.float32, rows)
         lists = (chunks["req"].data_ptr(), chunks["t0"].data_ptr(), chunks["len"].data_ptr(), chunks["req_chunk0"].data_ptr(),
                  gates_scratch.data_ptr(), gates_scratch.data_ptr() + 12 * n_heads * T, chunk_state.data_ptr())
     _call(load_module("matrix_memory"), "ifx_matrix_memory",
           (P, I, I, I, I, I, I, P, I, I, I, P, P, F, F, P, F, P, LL, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, P, P, P, P, P, P),
-          rows.data_ptr(), _dt(rows), ld, q_col, k_col, v_col, g_col, gates.data_ptr(), ldg, i_col, f_col, i_bias.data_ptr(),
-          f_bias.data_ptr(), float(cap), float(d) ** -0.5, norm_weight.data_ptr(), float(eps), state.data_ptr(), state.shape[1], s_off,
-          q_start.data_ptr(), q_len.data_ptr(), slots.data_ptr(), row_req.data_ptr(), o_raw, nq, floor, m_end, out.data_ptr(), _DT[out_dtype],
+          rows, _dt(rows), ld, q_col, k_col, v_col, g_col, gates, ldg, i_col, f_col, i_bias,
+          f_bias, float(cap), float(d) ** -0.5, norm_weight, float(eps), state, state.shape[1], s_off,
+          q_start, q_len, slots, row_req, o_raw, nq, floor, m_end, out, _DT[out_dtype],
           T, R, n_heads, d, dv, ch, ks, wg_cols, n_chunks, *lists, _stream())
     return out
 
@@ -2272,7 +2298,7 @@ def retention(rows: torch.Tensor, cols: Tuple[int, int, int, int], cos: torch.Te
     _check(state, "state", (None, n_heads * dv * ch * ks), torch.float32)
     if single_tokens and T != R:
         raise KernelError(f"retention: {T} rows of {R} requests are no step of single tokens")
-    out = torch.empty((T, HV), dtype=out_dtype, device=rows.device)
+    out = empty((T, HV), out_dtype, rows)
     n_chunks, lists, o_raw = 0, (0,) * 5, None
     if chunks is not None:
         if not retention_takes_chunks(rows.dtype, d, dv) or chunks["rows"] != RETENTION_CHUNK:
@@ -2282,18 +2308,18 @@ def retention(rows: torch.Tensor, cols: Tuple[int, int, int, int], cos: torch.Te
         for nm in ("t0", "len"):
             _check(chunks[nm], f"chunks.{nm}", (n_chunks,), torch.int32)
         _check(chunks["req_chunk0"], "chunks.req_chunk0", (R + 1,), torch.int32)
-        turned = torch.empty((4, T * HD), dtype=torch.bfloat16, device=rows.device)
-        chunk_state = torch.empty((n_chunks, n_heads * dv * ch * ks), dtype=torch.float32, device=rows.device)
+        turned = empty((4, T * HD), torch.bfloat16, rows)
+        chunk_state = empty((n_chunks, n_heads * dv * ch * ks), torch.float32, rows)
         lists = (chunks["t0"].data_ptr(), chunks["len"].data_ptr(), chunks["req_chunk0"].data_ptr(), turned.data_ptr(), chunk_state.data_ptr())
     if single_tokens and chunks is None:
         wg_cols = retention_step_columns(T, n_heads, d, dv)
     if (chunks is None and (not single_tokens or wg_cols < dv)) or (chunks is not None and dv > 128):
-        o_raw = torch.empty((T, HV), dtype=torch.float32, device=rows.device)
+        o_raw = empty((T, HV), torch.float32, rows)
     _call(load_module("retention"), "ifx_retention",
           (P, I, I, I, I, I, I, P, P, I, P, P, F, F, P, LL, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, I, P, P, P, P, P, P),
-          rows.data_ptr(), _dt(rows), ld, q_col, k_col, v_col, g_col, _ptr(cos) if rot_dims else 0, _ptr(sin) if rot_dims else 0, rot_dims // 2,
-          decay.data_ptr(), log2_decay.data_ptr(), float(d) ** -0.5, float(eps), state.data_ptr(), state.shape[1], q_start.data_ptr(),
-          q_len.data_ptr(), slots.data_ptr(), _ptr(o_raw), out.data_ptr(), _DT[out_dtype], T, R, n_heads, d, dv, ch, ks, wg_cols,
+          rows, _dt(rows), ld, q_col, k_col, v_col, g_col, cos if rot_dims else None, sin if rot_dims else None, rot_dims // 2,
+          decay, log2_decay, float(d) ** -0.5, float(eps), state, state.shape[1], q_start,
+          q_len, slots, o_raw, out, _DT[out_dtype], T, R, n_heads, d, dv, ch, ks, wg_cols,
           1 if single_tokens else 0, n_chunks, *lists, _stream())
     return out
 
@@ -2334,17 +2360,17 @@ def hyper_step(src: torch.Tensor, n_streams: int, y=None, mix: Optional[torch.Te
         else:
             _check(y, "y", (T, H))
             y_ptr, y_dt = y.data_ptr(), _dt(y)
-    dst = torch.empty((T, S, H), dtype=torch.float32, device=src.device) if single else src
+    dst = empty((T, S, H), torch.float32, src) if single else src
     rows = None
     if in_weights is not None:
         if norm_weight is not None:
             _check(norm_weight, "norm_weight", (H,))
             rows = torch.empty((T, H), dtype=out_dtype or torch.float32, device=src.device)
         else:
-            rows = torch.empty((T, H), dtype=torch.float32, device=src.device)
+            rows = empty((T, H), torch.float32, src)
     _call(load_module("hyper"), "ifx_hyper_step", (P, I, P, P, I, I, LL, F, P, P, P, P, I, F, P, I, I, I, I, P),
-          src.data_ptr(), 1 if single else 0, dst.data_ptr(), y_ptr, y_dt, n_slices, stride, float(y_scale), _ptr(mix), _ptr(out_weights),
-          _ptr(in_weights), _ptr(norm_weight), _dt(norm_weight) if norm_weight is not None else 0, float(eps), _ptr(rows),
+          src, 1 if single else 0, dst, y_ptr, y_dt, n_slices, stride, float(y_scale), mix, out_weights,
+          in_weights, norm_weight, _dt(norm_weight) if norm_weight is not None else 0, float(eps), rows,
           _DT[rows.dtype] if rows is not None else 0, T, S, H, _stream())
     return dst, rows
 
@@ -2379,12 +2405,12 @@ def activation(x, act: int) -> torch.Tensor:
         if n % 4:
             return activation(x.sum(x.dtype), act)
         out = torch.empty(parts.shape[1:], dtype=x.dtype, device=parts.device)
-        _call(load_module("rowwise"), "ifx_activation_slices", (P, I, LL, P, I, LL, I, P), parts.data_ptr(), parts.shape[0], n,
-              out.data_ptr(), _DT[x.dtype], n, int(act), _stream())
+        _call(load_module("rowwise"), "ifx_activation_slices", (P, I, LL, P, I, LL, I, P), parts, parts.shape[0], n,
+              out, _DT[x.dtype], n, int(act), _stream())
         return out
     _check(x, "x")
     out = torch.empty_like(x)
-    _call(load_module("rowwise"), "ifx_activation", (P, P, I, LL, I, P), x.data_ptr(), out.data_ptr(), _dt(x), x.numel(), int(act), _stream())
+    _call(load_module("rowwise"), "ifx_activation", (P, P, I, LL, I, P), x, out, _dt(x), x.numel(), int(act), _stream())
     return out
 
 
@@ -2404,7 +2430,7 @@ def sigmoid_gate(x: torch.Tensor, rows, g_col: int) -> torch.Tensor:
         raise KernelError(f"sigmoid_gate: columns {g_col}..{g_col + C} lie outside rows of {ld}")
     out = torch.empty_like(x)
     _call(load_module("rowwise"), "ifx_sigmoid_gate", (P, P, I, I, I, LL, P, I, I, I, P),
-          x.data_ptr(), ptr, ld, int(g_col), n_slices, stride, out.data_ptr(), _dt(x), T, C, _stream())
+          x, ptr, ld, int(g_col), n_slices, stride, out, _dt(x), T, C, _stream())
     return out
 
 
@@ -2428,16 +2454,16 @@ def gated_add(base, extra, h: torch.Tensor, gate_weight: Optional[torch.Tensor])
     ep, ef, en, es, N2 = operand(extra, "extra")
     if N != N2:
         raise KernelError(f"gated_add: base is {N} wide, extra {N2}")
-    out = torch.empty((T, N), dtype=h.dtype, device=h.device)
+    out = empty((T, N), h.dtype, h)
     _call(load_module("rowwise"), "ifx_gated_add", (P, I, I, LL, P, I, I, LL, P, P, I, P, I, I, I, P),
-          bp, bf, bn, bs, ep, ef, en, es, h.data_ptr(), _ptr(gate_weight), K, out.data_ptr(), _dt(h), T, N, _stream())
+          bp, bf, bn, bs, ep, ef, en, es, h, gate_weight, K, out, _dt(h), T, N, _stream())
     return out
 
 
 def scale_softcap(logits: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> torch.Tensor:
     """In place on float32 ``logits``: x <- x * scale, then (cap > 0) x <- cap * tanh(x / cap)."""
     _check(logits, "logits", None, torch.float32)
-    _call(load_module("rowwise"), "ifx_scale_softcap", (P, LL, F, F, P), logits.data_ptr(), logits.numel(), float(scale), float(cap or 0.0), _stream())
+    _call(load_module("rowwise"), "ifx_scale_softcap", (P, LL, F, F, P), logits, logits.numel(), float(scale), float(cap or 0.0), _stream())
     return logits
 
 
@@ -2483,14 +2509,14 @@ def attention_wide(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     _check(row_req, "row_req", (T,), torch.int32)
     _check(positions, "positions", (T,), torch.int32)
     _check(block_table, "block_table", (None, None), torch.int32)
-    out = torch.empty((T, nH * dv), dtype=torch.bfloat16, device=q.device)
-    part_o = torch.empty((T, nH, max_splits, dv), dtype=torch.float32, device=q.device)
-    part_ml = torch.empty((T, nH, max_splits, 2), dtype=torch.float32, device=q.device)
+    out = empty((T, nH * dv), torch.bfloat16, q)
+    part_o = empty((T, nH, max_splits, dv), torch.float32, q)
+    part_ml = empty((T, nH, max_splits, 2), torch.float32, q)
     _call(load_module("attn_wide", (("K_DIM", d), ("V_DIM", dv))), "ifx_attn_wide",
           (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, P, P),
-          q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), 0, row_req.data_ptr(), positions.data_ptr(),
-          block_table.data_ptr(), block_table.shape[1], T, nH, d, dv, page_size, int(window or 0), int(chunk), int(max_splits),
-          float(scale), part_o.data_ptr(), part_ml.data_ptr(), _ptr(sinks), _stream())
+          q, k_cache, v_cache, out, 0, row_req, positions,
+          block_table, block_table.shape[1], T, nH, d, dv, page_size, int(window or 0), int(chunk), int(max_splits),
+          float(scale), part_o, part_ml, sinks, _stream())
     return out
 
 
@@ -2519,7 +2545,7 @@ def _attn_extras(T, nH, keep_first, sink, gate, sinks=None, block=None):
         _check(gate, "gate", (T, nH), torch.float32)
     if sinks is not None:
         _check(sinks, "sinks", (nH,), torch.float32)
-    return int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), _ptr(gate), _ptr(sinks), int(block or 0)
+    return int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), gate, sinks, int(block or 0)
 
 
 ROW_MAX_WAVES = 8
@@ -2561,14 +2587,14 @@ def attention_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
                           f"up to {row_waves_fit(nH, nKV, d, ROW_MAX_WAVES)} at these head counts)")
     part_o = part_ml = None
     if waves == 0:
-        part_o = torch.empty((n_rows, nH, max_splits, d), dtype=torch.float32, device=q.device)
-        part_ml = torch.empty((n_rows, nH, max_splits, 2), dtype=torch.float32, device=q.device)
+        part_o = empty((n_rows, nH, max_splits, d), torch.float32, q)
+        part_ml = empty((n_rows, nH, max_splits, 2), torch.float32, q)
     if req_is_row and block_table.shape[0] < T:
         raise KernelError("attention_rows: req_is_row needs a block-table row for every row of the step")
     _call(mod, "ifx_attn_rows", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, I, I, I, I, F, P, P, I, P),
-          q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _ptr(rows), row_req.data_ptr(),
-          positions.data_ptr(), block_table.data_ptr(), block_table.shape[1], n_rows, nH, nKV, d, page_size,
-          int(window or 0), chunk, max_splits, float(scale), _ptr(part_o), _ptr(part_ml), waves, 1 if req_is_row else 0,
+          q, k_cache, v_cache, out, rows, row_req,
+          positions, block_table, block_table.shape[1], n_rows, nH, nKV, d, page_size,
+          int(window or 0), chunk, max_splits, float(scale), part_o, part_ml, waves, 1 if req_is_row else 0,
           *_attn_extras(T, nH, keep_first, sink, gate, sinks, block), _stream())
 
 
@@ -2619,18 +2645,17 @@ def attention_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         _check(rows, "rows", (n_rows,), torch.int32)
         _check(row_req, "row_req", (T,), torch.int32)
         _check(positions, "positions", (T,), torch.int32)
-        part_o = torch.empty((T, nH, max_splits, d), dtype=torch.float32, device=q.device)
-        part_ml = torch.empty((T, nH, max_splits, 2), dtype=torch.float32, device=q.device)
+        part_o = empty((T, nH, max_splits, d), torch.float32, q)
+        part_ml = empty((T, nH, max_splits, 2), torch.float32, q)
     per_xcd = 0
     if order is not None:
         _check(order, "order", (None,), torch.int32)
         if order.shape[0] % N_XCD:
             raise KernelError(f"attention_tiles: the order has a place for each of {N_XCD} XCDs' workgroups")
         per_xcd = order.shape[0] // N_XCD
-    args = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), tile_req.data_ptr(), tile_q0.data_ptr(),
-            n_tiles, q_start.data_ptr(), q_len.data_ptr(), kv_len.data_ptr(), block_table.data_ptr(),
+    args = (q, k_cache, v_cache, out, tile_req, tile_q0, n_tiles, q_start, q_len, kv_len, block_table,
             block_table.shape[1], nH, nKV, d, page_size, int(window or 0), float(scale), int(chunk), int(max_splits),
-            _ptr(part_o), _ptr(part_ml), _ptr(rows), n_rows, _ptr(row_req), _ptr(positions), _ptr(order), per_xcd, N_XCD)
+            part_o, part_ml, rows, n_rows, row_req, positions, order, per_xcd, N_XCD)
     types = (P, P, P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, F, I, I, P, P, P, I, P, P, P, I, I)
     if entry == "ifx_attn_tiles":
         _call(mod, entry, types + (I, I, F, P, P, I, P), *args, *_attn_extras(T, nH, keep_first, sink, gate, sinks, block), _stream())
@@ -2643,11 +2668,11 @@ def argmax(logits: torch.Tensor) -> torch.Tensor:
     """Lowest index of the maximum of each row of float32 ``logits`` [R, V]; int32 [R]."""
     _check(logits, "logits", (None, None), torch.float32)
     R, V = logits.shape
-    out = torch.empty((R,), dtype=torch.int32, device=logits.device)
-    pv = torch.empty((R, 32), dtype=torch.float32, device=logits.device)
-    pi = torch.empty((R, 32), dtype=torch.int32, device=logits.device)
-    _call(load_module("sampling"), "ifx_argmax", (P, I, I, P, P, P, P), logits.data_ptr(), R, V, out.data_ptr(),
-          pv.data_ptr(), pi.data_ptr(), _stream())
+    out = empty((R,), torch.int32, logits)
+    pv = empty((R, 32), torch.float32, logits)
+    pi = empty((R, 32), torch.int32, logits)
+    _call(load_module("sampling"), "ifx_argmax", (P, I, I, P, P, P, P), logits, R, V, out,
+          pv, pi, _stream())
     return out
 
 
@@ -2661,8 +2686,8 @@ def apply_penalties(logits: torch.Tensor, rows: torch.Tensor, ids: torch.Tensor,
     for t, nm in ((rep, "rep"), (freq, "freq"), (pres, "pres")):
         _check(t, nm, (R,), torch.float32)
     _call(load_module("sampling"), "ifx_apply_penalties", (P, I, P, P, P, I, P, P, P, P),
-          logits.data_ptr(), V, rows.data_ptr(), ids.data_ptr(), counts.data_ptr(), n, rep.data_ptr(),
-          freq.data_ptr(), pres.data_ptr(), _stream())
+          logits, V, rows, ids, counts, n, rep,
+          freq, pres, _stream())
 
 
 def add_logit_bias(logits: torch.Tensor, rows: torch.Tensor, ids: torch.Tensor, bias: torch.Tensor) -> None:
@@ -2672,7 +2697,7 @@ def add_logit_bias(logits: torch.Tensor, rows: torch.Tensor, ids: torch.Tensor, 
     _check(ids, "ids", (n,), torch.int32)
     _check(bias, "bias", (n,), torch.float32)
     _call(load_module("sampling"), "ifx_add_logit_bias", (P, I, P, P, P, I, P),
-          logits.data_ptr(), logits.shape[1], rows.data_ptr(), ids.data_ptr(), bias.data_ptr(), n, _stream())
+          logits, logits.shape[1], rows, ids, bias, n, _stream())
 
 
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
@@ -2698,14 +2723,14 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
         _check(draws, "draws", (R, 4), torch.int32)
     mod = load_module("sampling")
     weights = torch.empty_like(logits)
-    out = torch.empty((R,), dtype=torch.int32, device=logits.device)
+    out = empty((R,), torch.int32, logits)
     # large vocabularies are drawn by several workgroups a row, which hand each other their results in scratch memory
     n_scratch = mod.fn("ifx_sample_scratch_blocks", (I, I, I))(R, V, 1 if any_filters else 0)
-    scratch = torch.empty((n_scratch * 256,), dtype=torch.uint8, device=logits.device) if n_scratch else None
+    scratch = empty((n_scratch * 256,), torch.uint8, logits) if n_scratch else None
     _call(mod, "ifx_sample", (P, P, P, P, P, P, P, P, P, I, I, P, I, I, P),
-          logits.data_ptr(), weights.data_ptr(), temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(),
-          min_p.data_ptr(), uniform.data_ptr() if uniform is not None else None,
-          draws.data_ptr() if draws is not None else None, out.data_ptr(), R, V, _ptr(scratch), 1 if any_greedy else 0,
+          logits, weights, temperature, top_k, top_p,
+          min_p, uniform,
+          draws, out, R, V, scratch, 1 if any_greedy else 0,
           1 if any_filters else 0, _stream())
     return out
 
@@ -2716,11 +2741,11 @@ def logprobs(logits: torch.Tensor, chosen: torch.Tensor, top_n: int):
     _check(logits, "logits", (None, None), torch.float32)
     R, V = logits.shape
     _check(chosen, "chosen", (R,), torch.int32)
-    lp = torch.empty((R,), dtype=torch.float32, device=logits.device)
-    top_ids = torch.empty((R, top_n), dtype=torch.int32, device=logits.device)
-    top_lp = torch.empty((R, top_n), dtype=torch.float32, device=logits.device)
+    lp = empty((R,), torch.float32, logits)
+    top_ids = empty((R, top_n), torch.int32, logits)
+    top_lp = empty((R, top_n), torch.float32, logits)
     _call(load_module("sampling"), "ifx_logprobs", (P, P, I, I, I, P, P, P, P),
-          logits.data_ptr(), chosen.data_ptr(), R, V, top_n, lp.data_ptr(), top_ids.data_ptr(), top_lp.data_ptr(), _stream())
+          logits, chosen, R, V, top_n, lp, top_ids, top_lp, _stream())
     return lp, top_ids, top_lp
 
 
@@ -2735,7 +2760,7 @@ def stream_read(region: torch.Tensor, waves: int, streaming: bool) -> None:
     if sink is None:
         sink = _SINKS[region.device.index] = torch.zeros(1, dtype=torch.float32, device=region.device)
     _call(load_module("ceilings"), "ifx_stream_read", (P, LL, I, I, P, P),
-          region.data_ptr(), region.numel() * region.element_size(), waves, int(streaming), sink.data_ptr(), _stream())
+          region, region.numel() * region.element_size(), waves, int(streaming), sink, _stream())
 
 
 def stream_copy(src: torch.Tensor, dst: torch.Tensor, waves: int, streaming: bool) -> None:
@@ -2745,4 +2770,4 @@ def stream_copy(src: torch.Tensor, dst: torch.Tensor, waves: int, streaming: boo
     n = src.numel() * src.element_size()
     if n != dst.numel() * dst.element_size():
         raise KernelError(f"stream_copy: {n} bytes into {dst.numel() * dst.element_size()}")
-    _call(load_module("ceilings"), "ifx_stream_copy", (P, P, LL, I, I, P), src.data_ptr(), dst.data_ptr(), n, waves, int(streaming), _stream())
+    _call(load_module("ceilings"), "ifx_stream_copy", (P, P, LL, I, I, P), src, dst, n, waves, int(streaming), _stream())

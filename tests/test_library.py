@@ -3,6 +3,7 @@ import os
 import stat
 
 import pytest
+import torch
 
 from inferflux_amd.kernels import library
 
@@ -40,3 +41,124 @@ def test_barriers_in_assembly_stand_behind_a_wait_for_what_was_read_from_lds():
                 before = "\n".join(lines[max(0, i - 5):i])
                 assert "lgkmcnt(0)" in line.split("//")[0] or "__builtin_amdgcn_s_waitcnt(0xc07f)" in before, f"{name}:{i + 1}"
     assert found >= 4
+
+
+class _Function:
+    """A function of ``types`` (p, a, i, l, f) in a module of its own that keeps what it is called with and returns ``rc``."""
+
+    def __init__(self, types, rc=0):
+        import ctypes
+
+        from inferflux_amd.kernels import ops
+        words = {"p": ops.P, "a": ops.P, "i": ops.I, "l": ops.LL, "f": ops.F}
+        self.got, self.name, self.entries = None, "fake", {}
+        self.argtypes = tuple(ctypes.POINTER(ops.I) if c == "a" else words[c] for c in types)
+
+        def record(*args):
+            self.got = args
+            return rc
+        self.keep = ctypes.CFUNCTYPE(ctypes.c_int, *(words[c] for c in types))(record)
+
+    def fn(self, fname, argtypes):
+        return self.keep
+
+    def last_error(self):
+        return "an error of its own"
+
+
+@pytest.mark.parametrize("types", ["", "p", "f", "pppppp", "ppppppp", "ffffffff", "pifpifpifl", "iiiiiiiiiifffffffflp",
+                                   "pppppppppppiiiiiiiifiippppiiiippiif", "i" * 38, "l" * 38 + "f" * 8])
+def test_native_calls_pass_what_ctypes_passes(types):
+    import ctypes
+    import random
+    import struct
+
+    from inferflux_amd.kernels import ops
+    rng, t = random.Random(len(types)), torch.arange(6, dtype=torch.int32)
+    f = _Function(types)
+    args, want = [], []
+    for c in types:
+        if c == "p":
+            v = rng.choice([None, 0, t, 0x7fff12345678, (1 << 64) - 16])
+            args.append(v)
+            want.append((v.data_ptr() if v is t else v) or None)
+        elif c == "f":
+            args.append(rng.choice([1, 0.1, -3.5e30, float("inf"), 2 ** -149]))
+            want.append(struct.unpack("f", struct.pack("f", float(args[-1])))[0])
+        else:
+            args.append(rng.choice([0, -1, True, 2 ** 31 - 1, -2 ** 31] + ([2 ** 40 + 3] if c == "l" else [])))
+            want.append(int(args[-1]))
+    ops._call(f, "fake", f.argtypes, *args)
+    assert "fake" in f.entries and f.entries["fake"] is not None
+    assert list(f.got) == want
+    f.got = None
+    ops._call(f, "fake", f.argtypes, *args)              # (by what was kept of the first call)
+    assert list(f.got) == want
+    assert ctypes.sizeof(ctypes.c_void_p) == 8
+
+
+def test_native_calls_leave_the_rest_to_ctypes():
+    import ctypes
+
+    import numpy as np
+
+    from inferflux_amd.kernels import ops
+    f = _Function("iaf")
+    ints = (ctypes.c_int * 3)(4, 5, 6)
+    ops._call(f, "fake", f.argtypes, 1, ints, 2.0)       # (the address of an array)
+    assert f.got[1] == ctypes.addressof(ints) and f.got[0::2] == (1, 2.0)
+    f = _Function("i" * 39)                              # more than the native call has places for
+    ops._call(f, "fake", f.argtypes, *range(39))
+    assert f.entries["fake"] is None and f.got == tuple(range(39))
+    f = _Function("if")
+    for wrong in ((1,), (1, 2.0, "three"), ("one", 2.0), (1, "two"), (np.int64(1), None)):
+        with pytest.raises((TypeError, ctypes.ArgumentError)):
+            g = _Function("if")
+            g.keep.argtypes = list(g.argtypes)
+            ops._call(g, "fake", g.argtypes, *wrong)
+            assert len(wrong) <= 2 or g.got == (1, 2.0)  # (ctypes takes further arguments)
+            raise TypeError
+    f = _Function("p", rc=-7)
+    with pytest.raises(ops.KernelError, match=r"fake: an error of its own \(code -7\)"):
+        ops._call(f, "fake", f.argtypes, None)
+
+
+def test_native_checks_raise_what_the_python_check_raises():
+    from inferflux_amd.kernels import ops
+    x = torch.zeros(2, 3)
+    for args in ((3, "x"), (x, "x"), (x, "x", (2, 3)), (x, "x", None, torch.float32), (x.t(), "x", (3, 2), torch.float64), (None, "x", (None,))):
+        with pytest.raises(ops.KernelError) as a:
+            ops._check_in_python(*args)
+        with pytest.raises(ops.KernelError) as b:
+            ops._check(*args)
+        assert str(a.value) == str(b.value)
+    with pytest.raises(ops.KernelError):
+        ops._check(x, "x", dtype=torch.float32)          # (keywords, too)
+    y = ops.empty((2, 0, 5), torch.bfloat16, x)
+    assert y.shape == (2, 0, 5) and y.dtype == torch.bfloat16 and y.device == x.device and y.is_contiguous()
+    for wrong in (((2,), torch.int32), ([2], torch.int32, x), ((2,), "int32", x), ((2,), torch.int32, None), ((2.5,), torch.int32, x), ((-1,), torch.int32, x)):
+        with pytest.raises((TypeError, RuntimeError)):
+            ops.empty(*wrong)
+
+
+@pytest.mark.gpu
+def test_native_checks_on_the_gpu():
+    from inferflux_amd.kernels import ops
+    x = torch.zeros(4, 6, device="cuda")
+    tensors = (x, x.t(), x[:, :3], x[1:3], x.bfloat16(), x[0], x[0, 0], torch.empty(0, 6, device="cuda"), torch.nn.Parameter(x))
+    shapes = (None, (4, 6), (None, 6), (4, None), (None, None), (6,), (), (2, 6), [4, 6], (4, 6, 1), x.shape, (0, None))
+    for t in tensors:
+        for shape in shapes:
+            for dtype in (None, torch.float32, torch.bfloat16):
+                def outcome(f):
+                    try:
+                        f(t, "t", shape, dtype)
+                    except ops.KernelError as e:
+                        return str(e)
+                assert outcome(ops._check) == outcome(ops._check_in_python), (t.shape, shape, dtype)
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert ops._stream() == side.cuda_stream != 0
+    a = ops.upload(__import__("numpy").arange(1000, dtype="int32"), x.device)
+    assert torch.equal(a.cpu(), torch.arange(1000, dtype=torch.int32))
