@@ -80,6 +80,7 @@ def module_variants() -> Iterable[Tuple[str, Variant]]:
     yield ("rowwise", ())
     yield ("grouped_gemm", ())
     yield ("moe_few", ())
+    yield ("moe_f32", ())
     yield ("gemm_tiles", ())
     yield ("ceilings", ())            # measurement only: what the memory gives a kernel that just reads
     for d in MFMA_HEAD_DIMS_PREBUILT:
@@ -727,6 +728,50 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
           tc, nt, max_tiles, T, N, ff, top, n_real, h, 1 if weigh_input else 0,
           down_tiled, wave_items, _stream())
     return SliceSums(parts, torch.bfloat16)
+
+
+MOE_F32_TILE_ITEMS = 64          # items of one expert to a workgroup of the 32-bit tiles
+MOE_F32_FEW_ITEMS = 3.25         # (row, choice) items for each expert up to which each streams its expert's weights for itself (see csrc/moe_f32.hip)
+MOE_F32_PORTION = 16384          # rows of a launch at most (a grid has up to 65,535 tiles)
+
+
+def moe_experts_f32(h: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
+                    act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False,
+                    few: Optional[bool] = None) -> "SliceSums":
+    """``moe_experts`` in 32 bits on the matrix cores (``gate`` / ``up`` [E, ff, K], ``down`` [E, N, ff], float32): the choices' weighted
+    outputs as ``SliceSums`` [top, T, N].  An element's sum has one order whatever the number of rows; ``few``: each item streams its
+    expert's weights for itself, or items are ordered by expert and meet them in tiles (None chooses)."""
+    _check(h, "h", (None, None), torch.float32)
+    T, K = h.shape
+    _check(gate, "gate", (None, None, K), torch.float32)
+    n_real, ff = gate.shape[0], gate.shape[1]
+    _check(up, "up", (n_real, ff, K), torch.float32)
+    _check(down, "down", (n_real, None, ff), torch.float32)
+    N, top, E = down.shape[1], ids.shape[1], n_real + int(n_identity)
+    _check(ids, "ids", (T, top), torch.int32)
+    _check(weights, "weights", (T, top), torch.float32)
+    if n_identity and N != K:
+        raise KernelError(f"moe_experts_f32: identity experts hand back the row itself, so N={N} must equal K={K}")
+    parts = empty((top, T, N), torch.float32, h)
+    portion = max(1, min(MOE_F32_PORTION, (65535 - E) * MOE_F32_TILE_ITEMS // top))
+    if T > portion:
+        for r in range(0, T, portion):
+            parts[:, r:r + portion] = moe_experts_f32(h[r:r + portion], gate, up, down, ids[r:r + portion].contiguous(), weights[r:r + portion].contiguous(),
+                                                      act, limit, n_identity, weigh_input, few).parts
+        return SliceSums(parts, torch.float32)
+    n_items = T * top
+    if few is None:
+        few = n_items <= MOE_F32_FEW_ITEMS * n_real
+    lists, max_tiles = (None, None, None, None, None), 0
+    if not few:
+        max_tiles = -(-n_items // MOE_F32_TILE_ITEMS) + E          # every expert may end on a tile that is not full
+        ints = empty((n_items + 3 * max_tiles + 2,), torch.int32, h)
+        lists = (ints[:n_items], *(ints[n_items + i * max_tiles:n_items + (i + 1) * max_tiles] for i in range(3)), ints[n_items + 3 * max_tiles:])
+        _call(load_module("grouped_gemm"), "ifx_moe_sort", (P, I, I, I, I, P, P, P, P, P, P), ids, n_items, E, n_real, MOE_F32_TILE_ITEMS, *lists, _stream())
+    a = empty((n_items, ff), torch.float32, h)
+    _call(load_module("moe_f32"), "ifx_moe_f32", (P,) * 13 + (I,) * 9 + (F, I, P), h, gate, up, down, ids, weights, a, parts, *lists, max_tiles,
+          T, K, ff, N, top, n_real, int(n_identity), int(act), float(limit), 1 if weigh_input else 0, _stream())
+    return SliceSums(parts, torch.float32)
 
 
 MOE_FEW_MAX_ROWS = 64          # rows of a step up to which the experts' weights are streamed once for all of them ...

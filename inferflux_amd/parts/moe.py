@@ -182,6 +182,10 @@ class MixtureOfExperts(FeedForward):
         if self.up is None and (isinstance(self.gate, ops.ExpertTiles) or x.shape[0] * self.top >= GROUPED_MIN_ITEMS):
             return self._with_shared(ops.moe_experts_grouped(x, self.gate, self.down, ids, weights, self.act, self.limit,
                                                              self.n_identity, self.weigh_input), x, ctx)      # (partial sums, one per choice)
+        if x.dtype == torch.float32 and self.up is not None:
+            out = self._with_shared(ops.moe_experts_f32(x, self.gate, self.up, self.down, ids, weights, self.act, self.limit,
+                                                        self.n_identity, self.weigh_input), x, ctx)        # (partial sums, one per choice)
+            return out if h.dtype == torch.float32 else out.sum(h.dtype) if isinstance(out, ops.SliceSums) else out.to(h.dtype)
         out = self._with_shared(ops.moe_experts(x, self.gate, self.up, self.down, ids, weights, self.act, self.limit,
                                                 self.n_identity, self.weigh_input), x, ctx)
         return out if out.dtype == h.dtype else out.to(h.dtype)
