@@ -4,7 +4,7 @@
 // every lane accumulates its output elements over the tile's keys in ascending order.  The parts' running maxima, sums and
 // outputs are joined in the parts' order.  So the sequence of operations for a (position, head) is the same however the request was
 // cut into steps and whatever is beside it: results are bit-equal across cuttings.  This is the attention of the 32-bit
-// path and the reference beside the matrix-core kernels.
+// path, whose prompts a kernel on the matrix cores gives the same bits, and the reference beside the bfloat16 kernels.
 //
 // What bounds a step of few rows is the chain of a tile's trips to memory, shuffles and dependent additions, about 4 us, so
 // four waves take a part each (four rows of 14 heads and 150 keys 9 us, 2,000 keys 57, where one wave takes 19 and 190).  Steps
@@ -71,7 +71,8 @@ struct AttnArgs {
   const float* sinks;
   int chunk;
   float lambda, out_scale, norm_eps;
-  int row0, n_rows;         // the launch's rows
+  const int* rows;          // the rows to do (null: all)
+  int row0, n_rows;         // the launch's, of them
 };
 
 // One map's running maximum, sum of weights and weighted values (element e of the values in lane e % 64).
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(WAVE * WAVES_PER_BLOCK) void attn_plain_kernel(Attn
   const long long item = ROW_WAVES == 1 ? (long long)blockIdx.x * WAVES_PER_BLOCK + wid : (long long)blockIdx.x;
   // (ROW_WAVES 1: all lanes of a wave leave together, and no barrier of the workgroup follows)
   if (ROW_WAVES == 1 && item >= (long long)a.n_rows * a.nH) return;
-  const int row = a.row0 + (int)(item / a.nH), head = (int)(item % a.nH);
+  const int nth = a.row0 + (int)(item / a.nH), head = (int)(item % a.nH), row = a.rows ? a.rows[nth] : nth;
   const int d = a.d, dv = a.dv, P = a.page_size;
   const int kvh = head / (a.nH / a.nKV);
   const int pos = a.positions[row];
@@ -355,7 +356,7 @@ extern "C" int ifx_attn_plain(const void* q, const void* k_cache, const void* v_
                               const int* row_req, const int* positions, const int* block_table,
                               int max_blocks, int T, int nH, int nKV, int d, int dv, int page_size, int window,
                               float scale, int keep_first, int has_sink, float sink_score, const float* gate, const float* sinks,
-                              int chunk, int maps, float lambda, float out_scale, float norm_eps, int row_waves, void* stream) {
+                              int chunk, int maps, float lambda, float out_scale, float norm_eps, int row_waves, const int* rows_of, void* stream) {
   IFX_REQUIRE(keep_first >= 0, "attn_plain: keep_first %d", keep_first);
   IFX_REQUIRE(T >= 0 && nH > 0 && nKV > 0 && nH % nKV == 0, "attn_plain: bad head counts nH=%d nKV=%d", nH, nKV);
   IFX_REQUIRE(maps == 1 || maps == 2, "attn_plain: %d maps (1 or 2)", maps);
@@ -367,7 +368,7 @@ extern "C" int ifx_attn_plain(const void* q, const void* k_cache, const void* v_
   IFX_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "attn_plain: unknown dtype %d", dtype);
   IFX_REQUIRE(row_waves == 0 || row_waves == 1 || row_waves == 4, "attn_plain: %d waves to a row and head (0, 1 or 4)", row_waves);
   if (row_waves == 0) row_waves = choose_row_waves((long long)T * nH, (long long)max_blocks * page_size, maps * d);
-  AttnArgs a{q, k_cache, v_cache, out, row_req, positions, block_table, max_blocks, T, nH, nKV, d, dv, page_size, window, scale, keep_first, has_sink, sink_score, gate, sinks, chunk, lambda, out_scale, norm_eps, 0, 0};
+  AttnArgs a{q, k_cache, v_cache, out, row_req, positions, block_table, max_blocks, T, nH, nKV, d, dv, page_size, window, scale, keep_first, has_sink, sink_score, gate, sinks, chunk, lambda, out_scale, norm_eps, rows_of, 0, 0};
   hipStream_t s = (hipStream_t)stream;
   // (a tile's values take registers: two waves to a SIMD of up to 64 elements, one of up to 128, so the items that are there at once)
   const bool at_once = d % 8 == 0 && d <= 64 && dv <= 128 && page_size % 8 == 0 && (long long)T * nH <= (dv <= 64 ? 512 : 256);

@@ -5,7 +5,8 @@ over the paged cache); they differ in speed and in which sizes they accept.  In 
 head size the matrix-core module takes (up to 128, values as wide as keys), requests that bring at least TILE_MIN rows go to the
 tile kernel (tiles of as many rows as the compiled module says; keys in splits when the tiles are
 few and their pasts long) and all other rows (decode tokens, short portions) to the row kernel;
-everything else (float32, other head sizes) goes to the plain kernel.
+everything else (float32, other head sizes) goes to the plain kernel, whose bits the 32-bit
+tile kernel repeats for whole tiles of rows.
 """
 from __future__ import annotations
 
@@ -17,6 +18,14 @@ import torch
 from . import ops
 
 TILE_MIN = 16       # fewer rows than this are cheaper one by one
+F32_TILE_MIN = 16   # ... in 32 bits,
+F32_TILE_MIN_WORK = 1 << 18     # and steps of less than this many (row, head, map) items times the longest context: us plain / in tiles with 14 heads
+                                # of 64 and 8 of 128 elements, one prompt of 80 rows 13 / 15, 16 / 23; of 200 30 / 16, 36 / 28; 64 of 40 rows 67 / 22,
+                                # 66 / 25; 64 rows behind 500 keys 35 / 23, 36 / 47, 128 rows 73 / 24, 85 / 48; two of 2,000 rows 2,470 / 208, 2,770 / 246
+F32_SPLIT = ((64, 128), (128, 255), (256, 768))    # 32-bit tiles by four workgroups each: up to so many workgroups without that, longer contexts
+                                # than this.  us whole / split: 44 workgroups of 64 elements and 200 keys 23 / 16, 112 and 256 keys 23 / 22, 220 and
+                                # 1,000 keys 72 / 52; but 104 and 112 keys 15 / 20, 224 and 256 keys 23 / 34; of 128 elements 14 and 200 keys 43 / 28,
+                                # 152 and 600 keys 110 / 97, 252 and 2,000 keys 320 / 246, but 112 and 200 keys 45 / 54, 256 and 500 keys 96 / 126
 TILE_QT2_MIN_WORKGROUPS = 512   # two workgroups of the tile kernel for each of the 256 compute units
 TILE_QT2_MIN_KEYS = 1536        # ... or rows that see this many keys on average, so that reading them from LDS half as often decides
 TILE_SPLIT_BELOW = 384          # fewer workgroups than this: the tile kernel splits the keys
@@ -268,6 +277,48 @@ def row_launch_shape(n_rows: int, n_kv_heads: int, max_kv: int, max_waves: int =
     return chunk, 0, -(-max_kv // chunk)
 
 
+def _f32_tiles(ctx, n_heads: int, n_kv: int, maps: int, cols: int):
+    """(tiles, rows that are not in one, whether parts go by workgroups of their own) of a step for ``ops.attention_f32``; the first None:
+    the step has no tiles, the second None: no further rows."""
+    tiled = ctx.h_q_len >= F32_TILE_MIN
+    if not tiled.any() or int(ctx.h_q_len[tiled].sum()) * n_heads * maps * int(ctx.h_kv_len[tiled].max()) < F32_TILE_MIN_WORK:
+        return None, None, False
+    group = n_heads // n_kv
+    tiles = [(r, c) for r in np.nonzero(tiled)[0] for c in range(0, int(ctx.h_q_len[r]) * group, cols)]
+    past = ctx.h_kv_len - ctx.h_q_len
+    tiles.sort(key=lambda t: -int(past[t[0]]) - t[1] // group)                  # the longest walks first
+    rows = np.nonzero(~tiled[ctx.h_row_req])[0].astype(np.int32)
+    packed = ctx.upload(np.concatenate([np.asarray(tiles, np.int32).ravel(), rows]))       # (each copy is a call of its own)
+    groups, longest = len(tiles) * n_kv * maps, int(ctx.h_kv_len[tiled].max())
+    split = any(groups <= g and longest > n for g, n in F32_SPLIT)
+    return packed[:2 * len(tiles)].view(-1, 2), packed[2 * len(tiles):] if rows.size else None, split
+
+
+def plain_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: float, keep_first: int = 0, sink: Optional[float] = None,
+                    gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, block: Optional[int] = None,
+                    differential=None) -> torch.Tensor:
+    """The plain kernel, and in 32 bits, where there is a kernel for the sizes, the matrix cores for requests of at least F32_TILE_MIN
+    rows in steps with work enough (the same bits by either)."""
+    table = ctx.block_table(cache.group)
+    T, nH, d = q.shape
+    n_kv, page_size = cache.k.shape[1:3]
+    dv = cache.v.shape[2]
+    maps = 2 if differential is not None else 1
+    cols = ops.attention_f32_cols(q.dtype, d // maps, dv, maps, page_size)
+    tiles, rows, split = (ctx.derived(("attention_f32_tiles", nH, n_kv, maps, cols), lambda: _f32_tiles(ctx, nH, n_kv, maps, cols)) if cols
+                          else (None, None, False))
+    if tiles is None:
+        return ops.attention_plain(q, cache.k, cache.v, ctx.row_req, ctx.positions, table, window, scale, keep_first, sink, gate,
+                                   sinks=sinks, chunk=block, differential=differential)
+    out = ops.empty((T, nH * dv), q.dtype, q)
+    ops.attention_f32(q, cache.k, cache.v, out, tiles, ctx.q_start, ctx.q_len, ctx.kv_len, table, window, scale, keep_first, sink, gate,
+                      sinks, block, differential, split)
+    if rows is not None:
+        ops.attention_plain(q, cache.k, cache.v, ctx.row_req, ctx.positions, table, window, scale, keep_first, sink, gate,
+                            sinks=sinks, chunk=block, differential=differential, rows=rows, out=out)
+    return out
+
+
 def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: float, keep_first: int = 0,
                     sink: Optional[float] = None, gate: Optional[torch.Tensor] = None,
                     sinks: Optional[torch.Tensor] = None, block: Optional[int] = None) -> torch.Tensor:
@@ -291,8 +342,7 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
         if not other and ops.wide_attention_supported(q.dtype, cache.k.shape[1], d, cache.v.shape[2], cache.page_size):
             chunk, splits = ops.wide_launch_shape(T, nH, ctx.kv_bound)
             return ops.attention_wide(q, cache.k, cache.v, ctx.row_req, ctx.positions, table, window, scale, chunk, splits, sinks)
-        return ops.attention_plain(q, cache.k, cache.v, ctx.row_req, ctx.positions, table, window, scale, keep_first, sink, gate,
-                                   sinks=sinks, chunk=block)
+        return plain_attention(q, cache, ctx, window, scale, keep_first, sink, gate, sinks, block)
     n_kv = cache.k.shape[1]
 
     def plan():

@@ -81,6 +81,7 @@ def module_variants() -> Iterable[Tuple[str, Variant]]:
     yield ("grouped_gemm", ())
     yield ("moe_few", ())
     yield ("moe_f32", ())
+    yield ("attn_f32", ())
     yield ("gemm_tiles", ())
     yield ("ceilings", ())            # measurement only: what the memory gives a kernel that just reads
     for d in MFMA_HEAD_DIMS_PREBUILT:
@@ -1760,7 +1761,8 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                     positions: torch.Tensor, block_table: torch.Tensor, window: Optional[int],
                     scale: float, keep_first: int = 0, sink: Optional[float] = None,
                     gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, chunk: Optional[int] = None,
-                    differential: Optional[Tuple[float, float, float]] = None, row_waves: int = 0) -> torch.Tensor:
+                    differential: Optional[Tuple[float, float, float]] = None, row_waves: int = 0,
+                    rows: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Causal (optionally windowed) attention of q [T, nH, d] over the paged cache (K [pages, nKV, page, d],
     V [pages, nKV, dv, page]; dv may differ from d); returns [T, nH*dv].  ``keep_first``: a windowed query also sees
     the first so many positions of its request; ``sink``: the score of a key without value that is added to the
@@ -1769,7 +1771,7 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     counted from the sequence's start.  ``differential`` (lambda, out_scale, eps): q and the keys hold two vectors of
     d / 2 elements per head, each pair a softmax map of its own over the same values; a head's output is map 1 minus
     lambda times map 2, divided by its root mean square (eps inside the root), times out_scale.  ``row_waves``: waves to a row and
-    head, 1 or 4 (0 lets the kernel choose; the same bits either way)."""
+    head, 1 or 4 (0 lets the kernel choose; the same bits either way).  ``rows`` int32: only these rows of ``out`` are written."""
     _check(q, "q", (None, None, None))
     T, nH, d = q.shape
     maps = 2 if differential is not None else 1
@@ -1787,13 +1789,68 @@ def attention_plain(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     _check(block_table, "block_table", (None, None), torch.int32)
     if gate is not None:
         _check(gate, "gate", (T, nH), torch.float32)
-    out = empty((T, nH * dv), q.dtype, q)
-    _call(load_module("attn_plain"), "ifx_attn_plain", (P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, P, P, I, I, F, F, F, I, P),
+    if out is None:
+        out = empty((T, nH * dv), q.dtype, q)
+    else:
+        _check(out, "out", (T, nH * dv), q.dtype)
+    if rows is not None:
+        _check(rows, "rows", (None,), torch.int32)
+        T = rows.shape[0]
+    _call(load_module("attn_plain"), "ifx_attn_plain", (P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, P, P, I, I, F, F, F, I, P, P),
           q, k_cache, v_cache, out, _dt(q), row_req,
           positions, block_table, block_table.shape[1], T, nH, nKV, d // maps, dv, page_size,
           int(window or 0), float(scale), int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), gate,
-          sinks, int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), int(row_waves), _stream())
+          sinks, int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), int(row_waves), rows, _stream())
     return out
+
+
+@functools.lru_cache(maxsize=None)
+def _attention_f32_cols(d: int, dv: int, maps: int, page_size: int) -> int:
+    return load_module("attn_f32").fn("ifx_attn_f32_cols", (I, I, I, I))(d, dv, maps, page_size)
+
+
+def attention_f32_cols(dtype: torch.dtype, d: int, dv: int, maps: int, page_size: int) -> int:
+    """(row, query head) pairs to a workgroup of ``attention_f32`` for keys of ``maps`` vectors of ``d`` elements and values of ``dv``;
+    0: it has no kernel for them."""
+    return _attention_f32_cols(d, dv, maps, page_size) if dtype == torch.float32 else 0
+
+
+def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor, tiles: torch.Tensor,
+                  q_start: torch.Tensor, q_len: torch.Tensor, kv_len: torch.Tensor, block_table: torch.Tensor, window: Optional[int],
+                  scale: float, keep_first: int = 0, sink: Optional[float] = None, gate: Optional[torch.Tensor] = None,
+                  sinks: Optional[torch.Tensor] = None, chunk: Optional[int] = None,
+                  differential: Optional[Tuple[float, float, float]] = None, split: bool = False) -> None:
+    """What ``attention_plain`` computes, the same bits, for whole tiles of rows in 32 bits on the matrix cores: ``tiles`` int32 [n, 2]
+    (request, first of ``attention_f32_cols`` columns; the columns of a request are its rows in this step times the query heads
+    of a kv head, and the first must lie among them).  Rows of requests without tiles stay as they are in ``out``.
+    ``split``: the four parts of a row's keys by workgroups of their own (the same bits)."""
+    _check(q, "q", (None, None, None), torch.float32)
+    T, nH, d = q.shape
+    maps = 2 if differential is not None else 1
+    if d % maps:
+        raise KernelError(f"attention_f32: two maps need an even row, got {d}")
+    lam, out_scale, norm_eps = differential if differential is not None else (0.0, 1.0, 0.0)
+    if sinks is not None:
+        _check(sinks, "sinks", (nH,), torch.float32)
+    _check(k_cache, "k_cache", (None, None, None, d), torch.float32)
+    n_pages, nKV, page_size, _ = k_cache.shape
+    _check(v_cache, "v_cache", (n_pages, nKV, None, page_size), torch.float32)
+    dv = v_cache.shape[2]
+    _check(out, "out", (T, nH * dv), torch.float32)
+    _check(tiles, "tiles", (None, 2), torch.int32)
+    R = q_start.shape[0]
+    for t, nm in ((q_start, "q_start"), (q_len, "q_len"), (kv_len, "kv_len")):
+        _check(t, nm, (R,), torch.int32)
+    _check(block_table, "block_table", (R, None), torch.int32)
+    if gate is not None:
+        _check(gate, "gate", (T, nH), torch.float32)
+    part_o = part_ml = None
+    if split or maps > 1:
+        part_o, part_ml = (empty((T, nH, maps, 4 if split else 1, n), torch.float32, q) for n in (dv, 2))
+    _call(load_module("attn_f32"), "ifx_attn_f32", (P, P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, I, F, I, I, F, P, P, I, I, F, F, F, I, P, P, P),
+          q, k_cache, v_cache, out, tiles, tiles.shape[0], q_start, q_len, kv_len, block_table, block_table.shape[1], nH, nKV, d // maps,
+          dv, page_size, int(window or 0), float(scale), int(keep_first or 0), 0 if sink is None else 1, float(sink or 0.0), gate,
+          sinks, int(chunk or 0), maps, float(lam), float(out_scale), float(norm_eps), int(split), part_o, part_ml, _stream())
 
 
 # ----------------------------------------------------------------------------------------

@@ -51,7 +51,7 @@ from typing import Dict, Mapping, Optional
 import torch
 
 from ..kernels import ops
-from ..kernels.attention import paged_attention
+from ..kernels.attention import paged_attention, plain_attention
 from .base import Mixer, MixerBinding, build_part, register_part
 from .position import PositionEncoding
 from .ffn import concat_weights
@@ -224,9 +224,9 @@ class PagedAttention(Mixer):
             # kernel joins the two outputs.
             a = paged_attention(ops.diff_expand(q), cache, ctx, self.window, self.scale, block=self.chunk)
             return ops.diff_combine(a, self.n_heads, self.v_head_dim, lam, out_scale, eps)
-        # any other sizes, and 32-bit: the kernel that knows two maps, one wave per (row, head), float math
-        return ops.attention_plain(q, cache.k, cache.v, ctx.row_req, ctx.positions, ctx.block_table(cache.group), self.window,
-                                   self.scale, self.keep_first, self.sink, gate, chunk=self.chunk, differential=(lam, out_scale, eps))
+        # any other sizes, and 32-bit: the kernels that know two maps, float math
+        return plain_attention(q, cache, ctx, self.window, self.scale, self.keep_first, self.sink, gate, block=self.chunk,
+                               differential=(lam, out_scale, eps))
 
     def _forward_extras(self, h, ctx, binding: MixerBinding, sink):
         """The step with the optional mechanisms: the fused projection (with the gate's rows), one row kernel for bias,
