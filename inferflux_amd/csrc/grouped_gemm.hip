@@ -34,7 +34,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
-#define TM 128         // items to a tile of the eight-wave kernel
+#define TM 128         // items to a tile of the eight-wave kernel,
+#define FEW_ITEMS 64   // where experts have few,
 #define WAVE_ITEMS 192 // ... of the kernel by four large waves
 #define EXPERTS_GROUP 4          // tiles of items that meet a tile of W one after the other
 #define MAX_EXPERTS 1024
@@ -131,18 +132,20 @@ struct ExpertsArgs {
 // took 718 us where these take 644; waves of 64 x 64 653; W from global memory into registers, in place of LDS, 624 to 714
 // by the shape.)  22,800 items of 64 experts (2,048 wide, 1,408 inner, 356 items each): 532 + 328 us for the two products
 // before, with the pieces through registers into LDS and rows of 64 k-values padded, now 362 + 241 (730 TFLOP/s with the tiles
-// that are not full).  One size of tile for all: tiles of 64 items were 0.91 of the time where experts have 88 items and
-// matrices are small (37 for 41 us), 1.03 to 1.2 of it everywhere else.
+// that are not full).  Experts of few items are bound by their weights' way from memory instead: tiles of 64 items, waves of
+// 32 x 32, leave room for a third stage of loads on their way (64 experts of 6 to a row, 150 rows 215 -> 199 us for the whole mixture, 512 rows
+// 234 -> 231; 32 experts, 4 to a row, 120 -> 106, 155 -> 145; 16 of 1,024 x 704, 2 to a row, 30 -> 23, 35 -> 27; with two stages 206, 108
+// and 27 at 150 rows; tiles of 32 items in three or four 208, 116 and 23, but from 30 items to an expert on 1.1 times the tiles of 64 and more).
 constexpr int TILE_BN = 128;
-typedef ProductTiles<TILE_BN, TM, 32, 64, false> RowTiles;
-template <int MODE, bool TILED>
-__global__ __launch_bounds__(RowTiles::THREADS, 4) void experts_kernel(ExpertsArgs a) {
-  typedef ProductTiles<TILE_BN, TM, 32, 64, TILED> P;
+template <int MODE, bool TILED, int BM, int WM, int STAGES>
+__global__ __launch_bounds__(512, 4) void experts_kernel(ExpertsArgs a) {
+  typedef ProductTiles<TILE_BN, BM, 32, WM, TILED, STAGES> P;
+  static_assert(P::THREADS == 512, "eight waves");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[P::LDS];
   const int tid = threadIdx.x;
   int tn, tm;
   if (!product_tile((a.NW + TILE_BN - 1) / TILE_BN, *a.n_tiles, 2, &tn, &tm)) return;
-  const int e = a.tile_expert[tm], start = a.tile_start[tm], count = min(a.tile_count[tm], TM), n0 = tn * TILE_BN;
+  const int e = a.tile_expert[tm], start = a.tile_start[tm], count = min(a.tile_count[tm], BM), n0 = tn * TILE_BN;
   const int* items = a.sorted + start;
   if (e >= a.n_real) {        // an identity expert's tile
     if (MODE == MODE_DOWN)
@@ -339,10 +342,11 @@ __global__ __launch_bounds__(256, 1) void experts_waves_kernel(ExpertsArgs a) {
 }
 
 template <int MODE>
-static void launch_experts(const ExpertsArgs& a, int max_tiles, int tiled, hipStream_t s) {
-  const dim3 blocks((max_tiles * ((a.NW + TILE_BN - 1) / TILE_BN) + 7) / 8 * 8), threads(RowTiles::THREADS);
-  if (tiled) hipLaunchKernelGGL((experts_kernel<MODE, true>), blocks, threads, 0, s, a);
-  else hipLaunchKernelGGL((experts_kernel<MODE, false>), blocks, threads, 0, s, a);
+static void launch_experts(const ExpertsArgs& a, int max_tiles, int tiled, int items, hipStream_t s) {
+  const dim3 blocks((max_tiles * ((a.NW + TILE_BN - 1) / TILE_BN) + 7) / 8 * 8), threads(512);
+  if (items == FEW_ITEMS) hipLaunchKernelGGL((experts_kernel<MODE, true, FEW_ITEMS, 32, 3>), blocks, threads, 0, s, a);
+  else if (tiled) hipLaunchKernelGGL((experts_kernel<MODE, true, TM, 64, 2>), blocks, threads, 0, s, a);
+  else hipLaunchKernelGGL((experts_kernel<MODE, false, TM, 64, 2>), blocks, threads, 0, s, a);
 }
 
 template <int MODE>
@@ -493,9 +497,9 @@ extern "C" int ifx_moe_gate_up_grouped(const void* x, const void* w, void* act, 
   if (max_tiles <= 0 || T == 0) return 0;
   const ExpertsArgs a{(const bf16_t*)x, (const bf16_t*)w, act, sorted, tile_expert, tile_start, tile_count, n_tiles, in_weights,
                       nullptr, T, top, K, 2 * ff, n_real, act_kind, limit, in_weights ? 1 : 0};
-  IFX_REQUIRE(wave_items == 0 || (tiled && wave_items == WAVE_ITEMS), "moe_gate_up_grouped: tiles of %d items", wave_items);
-  if (wave_items) launch_experts_waves<MODE_GATE_UP>(a, max_tiles, (hipStream_t)stream);
-  else launch_experts<MODE_GATE_UP>(a, max_tiles, tiled, (hipStream_t)stream);
+  IFX_REQUIRE(wave_items == 0 || (tiled && (wave_items == WAVE_ITEMS || wave_items == FEW_ITEMS)), "moe_gate_up_grouped: tiles of %d items", wave_items);
+  if (wave_items == WAVE_ITEMS) launch_experts_waves<MODE_GATE_UP>(a, max_tiles, (hipStream_t)stream);
+  else launch_experts<MODE_GATE_UP>(a, max_tiles, tiled, wave_items, (hipStream_t)stream);
   IFX_LAUNCH_CHECK();
 }
 
@@ -509,9 +513,9 @@ extern "C" int ifx_moe_down_grouped(const void* act, const void* w, float* parts
   if (max_tiles <= 0 || T == 0) return 0;
   const ExpertsArgs a{(const bf16_t*)act, (const bf16_t*)w, parts, sorted, tile_expert, tile_start, tile_count, n_tiles, weights,
                       (const bf16_t*)identity, T, top, ff, N, n_real, 0, 0.f, weigh_input};
-  IFX_REQUIRE(wave_items == 0 || (tiled && wave_items == WAVE_ITEMS), "moe_down_grouped: tiles of %d items", wave_items);
-  if (wave_items) launch_experts_waves<MODE_DOWN>(a, max_tiles, (hipStream_t)stream);
-  else launch_experts<MODE_DOWN>(a, max_tiles, tiled, (hipStream_t)stream);
+  IFX_REQUIRE(wave_items == 0 || (tiled && (wave_items == WAVE_ITEMS || wave_items == FEW_ITEMS)), "moe_down_grouped: tiles of %d items", wave_items);
+  if (wave_items == WAVE_ITEMS) launch_experts_waves<MODE_DOWN>(a, max_tiles, (hipStream_t)stream);
+  else launch_experts<MODE_DOWN>(a, max_tiles, tiled, wave_items, (hipStream_t)stream);
   IFX_LAUNCH_CHECK();
 }
 

@@ -2,11 +2,11 @@
 // tile of BN weight rows and BM rows of x, by (BN / WN) (BM / WM) waves that hold WN x WM sums each.
 //
 // Steps of 64 k-values of both operands are staged in LDS by loads that go there directly (no registers, no instructions to
-// store them; rows beyond the operands' ends arrive as zeros), two stages in turn.  What bounds it is LDS: a step's
+// store them; rows beyond the operands' ends arrive as zeros), STAGES stages in turn.  What bounds it is LDS: a step's
 // matrix instructions take 2 BN BM 64 / 4,096 cycles of a CU, its reads from LDS (WN + WM) 128 bytes a wave at 128 bytes a
 // cycle, and the direct loads' writes (BN + BM) 128 bytes besides.  So the loop is software-pipelined by half steps: the
 // fragments of the second half are read while the first half is multiplied; then the step's slot is free, the loads of
-// the step after next go out to it, and the next step's first half is read while the second half is multiplied.  Fetch
+// the step after next (STAGES steps on) go out to it, and the next step's first half is read while the second half is multiplied.  Fetch
 // and wait thus stand a whole step apart, and the only wait of a step is the barrier in its middle.
 //
 // A row of x is 128 bytes in LDS, 8 pieces of 16; piece p of row r lies at p ^ (r & 7) ^ (r >> 3 & 1), so that the 16 rows a
@@ -45,10 +45,10 @@ __device__ __forceinline__ void tile_meet() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
-template <int BN, int BM, int WN, int WM, bool TILED>
+template <int BN, int BM, int WN, int WM, bool TILED, int STAGES = 2>
 struct ProductTiles {
   static constexpr int ROW = 128, WAVES = (BN / WN) * (BM / WM), THREADS = 64 * WAVES;
-  static constexpr int W_BYTES = BN * ROW, STAGE = (BN + BM) * ROW, LDS = 2 * STAGE;
+  static constexpr int W_BYTES = BN * ROW, STAGE = (BN + BM) * ROW, LDS = STAGES * STAGE;
   static constexpr int FN = WN / 16, FM = WM / 16;      // this wave's fragments
   static constexpr int LW = BN / 8 / WAVES, LX = BM / 8 / WAVES;      // direct loads of a wave and a step (1 KB each)
   static_assert(BN % (8 * WAVES) == 0 && BM % (8 * WAVES) == 0 && BN % WN == 0 && BM % WM == 0, "tiles");
@@ -124,18 +124,20 @@ struct ProductTiles {
 #pragma unroll
       for (int b = 0; b < FM; ++b) acc[a][b] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
     __builtin_amdgcn_s_waitcnt(0);
-    issue(0, 0);
-    issue(1, 1);
-    tile_meet<LW + LX>();
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) issue(s, s);
+    tile_meet<(STAGES - 1) * (LW + LX)>();
     read(0, 0);
+    int slot = 0;
     for (int s = 0; s < steps; ++s) {
-      const int slot = s & 1;
+      const int next = STAGES == 2 ? slot ^ 1 : slot == STAGES - 1 ? 0 : slot + 1;
       read(slot, 1);
       multiply(0);
-      tile_meet<0>();
-      issue(s + 2, slot);
-      read(slot ^ 1, 0);
+      tile_meet<(STAGES - 2) * (LW + LX)>();
+      issue(s + STAGES, slot);
+      read(next, 0);
       multiply(1);
+      slot = next;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }

@@ -630,7 +630,10 @@ def moe_experts(h: torch.Tensor, gate: torch.Tensor, up: Optional[torch.Tensor],
     return out
 
 
-GROUPED_TILE_ITEMS = 128          # items of one expert to a workgroup of the grouped product (TM in csrc/grouped_gemm.hip)
+GROUPED_TILE_ITEMS = 128          # items of one expert to a workgroup of the grouped product (TM in csrc/grouped_gemm.hip),
+GROUPED_FEW_ITEMS = 64            # ... of weights in tiles where experts have, on average, up to
+GROUPED_FEW_MAX_ITEMS = 90        # so many (us by 128 / by 64 at 1,024 x 704 and 88, 125, 175 items 36 / 31, 37 / 35, 41 / 43; at 2,048 x 1,408 and 64 to 73 items
+                                  # 155 / 145, 132 / 128 and 264 / 260, 88 to 100 items 161 / 159, 156 / 153 and 292 / 303, 125 items 179 / 187)
 GROUPED_MAX_VALUES = 2 ** 30 - 8192          # values of the rows that the product's offsets of 32 bits reach
 
 
@@ -648,6 +651,11 @@ def grouped_wave_items(n_items: int, n_experts: int, pair_rows: int) -> int:
     tiles = n_items / GROUPED_WAVE_ITEMS + n_experts / 2
     fits = n_items >= GROUPED_WAVE_MIN_ITEMS * n_experts and tiles * -(-pair_rows // 256) >= GROUPED_WAVE_MIN_ROUNDS * COMPUTE_UNITS
     return GROUPED_WAVE_ITEMS if fits else 0
+
+
+def grouped_items(n_items: int, n_experts: int, pair_rows: int) -> int:
+    """Items to a tile where that is not GROUPED_TILE_ITEMS (0)."""
+    return GROUPED_FEW_ITEMS if n_items <= GROUPED_FEW_MAX_ITEMS * n_experts else grouped_wave_items(n_items, n_experts, pair_rows)
 
 
 def grouped_takes(dtype: torch.dtype, K: int, ff: int) -> bool:
@@ -687,7 +695,7 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
     choices' weighted outputs as ``SliceSums`` [top, T, N] (float32), which the kernel that adds them to the stream sums
     in the order of the choices.  ``n_identity``: ids from E up to E + n_identity name identity experts, whose output is
     the row itself (N = K then); ``act``, ``limit`` and ``weigh_input`` as for ``moe_experts``.  ``wave_items`` (both weights as
-    ``ExpertTiles``): tiles of so many items by four large waves (128 or 192), 0 those by eight, -1 chooses (``grouped_wave_items``)."""
+    ``ExpertTiles``): tiles of so many items, 192 by four large waves, 64 by eight small ones, 0 of 128, -1 chooses."""
     _check(h, "h", (None, None), torch.bfloat16)
     T, K = h.shape
     gu_shape, gu_ptr, gu_tiled = _experts(gate_up, "gate_up", (None, None, K))
@@ -711,7 +719,7 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
                                                           limit, n_identity, weigh_input, wave_items).parts
         return SliceSums(parts, torch.bfloat16)
     if wave_items < 0:
-        wave_items = grouped_wave_items(n_items, n_real, 2 * ff) if gu_tiled and down_tiled else 0
+        wave_items = grouped_items(n_items, n_real, 2 * ff) if gu_tiled and down_tiled else 0
     tile_items = wave_items or GROUPED_TILE_ITEMS
     max_tiles = -(-n_items // tile_items) + E          # every expert may end on a tile that is not full
     lists = empty((n_items + 3 * max_tiles + 2,), torch.int32, h)
