@@ -5,7 +5,7 @@
 // The library's product followed by a launch for the activation writes the N columns and reads them back (2,048 rows of
 // 37,888 columns: 233 MB, 40 us of 552) and rounds them to bfloat16 in between.
 //
-// The inner loop is wave_tiles.h, and for small tiles, of which two workgroups to a CU hide each other's ends, product_tiles.h.
+// The inner loop is wave_tiles.h, and for small tiles, of which up to three workgroups to a CU hide each other's ends, product_tiles.h.
 // What is chosen here is the tile.  A large tile reads less of LDS and of the caches for its products, but there are few of
 // them, and the last of the rounds that they take on 256 CUs may be nearly empty (600 rows of 22,016 x 2,048: 258 tiles of
 // 256 x 256 take 89 us, 232 of 384 x 160 49 us).  So choose_tile() takes the tile whose rounds are estimated to take least, from
@@ -190,77 +190,127 @@ __global__ __launch_bounds__(256, 1) void tiles_kernel(TilesArgs a) {
   }
 }
 
-template <int BN, int BM, int WN, int WM, int PER_CU>
-__global__ __launch_bounds__(64 * (BN / WN) * (BM / WM), 2 * PER_CU) void pairs_kernel(TilesArgs a) {
-  typedef ProductTiles<BN, BM, WN, WM, false> P;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[P::LDS];
-  int tn, tm;
-  if (!product_tile((a.N + BN - 1) / BN, (a.M + BM - 1) / BM, 4, &tn, &tm)) return;
-  const int n0 = tn * BN, m0 = tm * BM, rows = min(BN, a.N - n0), count = min(BM, a.M - m0);
-  const tile_uintx4 w = tile_buffer(a.w + (size_t)n0 * a.K, (unsigned)rows * (unsigned)a.K * 2u);
-  const tile_uintx4 x = tile_buffer(a.x + (size_t)m0 * a.K, (unsigned)count * (unsigned)a.K * 2u);
-  tile_floatx4 acc[P::FN][P::FM];
-  P::run(lds, w, x, a.K, [&](int i) { return i * a.K * 2; }, acc);
+// Tiles by small waves on product_tiles.h, a tile to a workgroup: for products of some hundred rows, whose tiles of 256 x 256 are few.
+// They are bound by the trips to memory of a short walk (three stages of loads stand between a request and its use) and, large ones,
+// by the caches: tiles of 64 x 64 by four waves, three workgroups to a CU, of 128 x 64 by eight, two, of 128 x 128 by eight, one.  us of
+// sums, cold weights, by large tiles (slices and what they cost the reader included) / the library / here: 150 rows of 896 x 896
+// 10.7 / 7.7 / 5.6, of 896 x 4,864 16.3 / 11.3 / 8.5, 300 of 1,536 x 8,960 29.4 / 30.2 / 22.8, 512 of 2,048 x 2,048 19.0 / 11.3 / 11.2; 100 rows by
+// the product that shares x through LDS / here of 2,048 x 2,048 12.2 / 7.4, of 2,048 x 11,008 27.8 / 19.3; gate/up of 150 and 300 rows of 9,728 x 896 17.2 / 16.2 / 11.1 and 17.3 / 19.3 / 14.0.
+// Four stages of 64 x 64 and 64 rows by 128 items were within 2 % of these; the two tiles of two stages that were here before (192 x 128,
+// 128 x 128) nowhere better.
+template <int BN, int BM, int WN, int WM, int OUT, int ACT>
+__device__ __forceinline__ void small_out(const TilesArgs& a, tile_floatx4 (&acc)[WN / 16][WM / 16], int slice, int m0, int n0) {
   const int lane = threadIdx.x % 64, g = lane / 16;
 #pragma unroll
-  for (int b = 0; b < P::FM; ++b) {
-    const int m = m0 + P::wm() + 16 * b + lane % 16;
+  for (int b = 0; b < WM / 16; ++b) {
+    const int m = m0 + 16 * b + lane % 16;
     if (m >= a.M) continue;
-    bf16_t* out = (bf16_t*)a.out + (size_t)m * (a.N / 2);
 #pragma unroll
-    for (int c = 0; c < P::FN; ++c) {
-      const int n = n0 + P::wn() + 16 * c + 4 * g;
+    for (int c = 0; c < WN / 16; ++c) {
+      const int n = n0 + 16 * c + 4 * g;
       if (n >= a.N) continue;
-      bf16x2 y;
-      y[0] = (__bf16)gated_act(acc[c][b][0], acc[c][b][1], a.act, a.limit);
-      y[1] = (__bf16)gated_act(acc[c][b][2], acc[c][b][3], a.act, a.limit);
-      *(bf16x2*)(out + n / 2) = y;
+      const tile_floatx4 v = acc[c][b];
+      if constexpr (OUT == OUT_PAIRS) {
+        bf16x2 y;
+        y[0] = (__bf16)tile_gated<ACT>(v[0], v[1], a.limit);
+        y[1] = (__bf16)tile_gated<ACT>(v[2], v[3], a.limit);
+        *(bf16x2*)((bf16_t*)a.out + (size_t)m * (a.N / 2) + n / 2) = y;
+      } else if constexpr (OUT == OUT_SUMS) {
+        *(tile_floatx4*)((float*)a.out + ((size_t)slice * a.M + m) * a.N + n) = v;
+      } else {
+        bf16_t* out = (bf16_t*)a.out + (size_t)m * a.N + n;
+        bf16x4 y;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = (__bf16)tile_act<ACT>(v[r]);
+        if (a.N % 4 == 0) *(bf16x4*)out = y;
+        else {          // (N is even)
+          *(bf16x2*)out = bf16x2{y[0], y[1]};
+          if (n + 2 < a.N) *(bf16x2*)(out + 2) = bf16x2{y[2], y[3]};
+        }
+      }
     }
   }
 }
 
-enum { TILE_256_256, TILE_320_192, TILE_192_128, TILE_128_128, TILE_384_160, TILE_256_192, TILE_192_256, TILE_256_128, TILE_KINDS };
-
-// us of a launch with tiles of a kind: workgroups to a CU; a launch, a full round of the chip (and each 1,000 k-values of it), the
-// last round (and each 1,000 k-values, and those times the share of CUs that have a tile: fewer of them find memory faster, and
-// the chip's power goes further).  For two workgroups to a CU the last round is one of one to a CU at most, others count as full.
-static const struct { int bn, bm, per_cu; double launch, base, per_k, last_base, last_per_k, last_fill; } kinds[TILE_KINDS] = {
-    {256, 256, 1, 3.07, 9.00, 22.71, 8.66, 15.99, 5.92}, {320, 192, 1, 2.39, 9.30, 21.06, 8.14, 14.48, 4.28},
-    {192, 128, 2, 2.84, 8.25, 20.48, 4.30, 12.97, 0.00}, {128, 128, 2, 2.21, 5.82, 15.77, 3.16, 10.50, 0.00},
-    {384, 160, 1, 3.16, 8.88, 22.56, 7.07, 14.47, 5.78}, {256, 192, 1, 2.32, 7.33, 17.34, 6.39, 12.35, 4.09},
-    {192, 256, 1, 2.81, 7.66, 16.78, 5.97, 11.85, 4.51}, {256, 128, 1, 2.82, 5.06, 14.36, 4.16, 9.91, 4.28}};
-
-static double tiles_us(int kind, int M, int N, int K) {
-  const auto& k = kinds[kind];
-  const long long tiles = (long long)((N + k.bn - 1) / k.bn) * ((M + k.bm - 1) / k.bm), per = (tiles + 7) / 8, round = 32 * k.per_cu;      // (of an XCD)
-  const long long rest = per % round;
-  const double kk = K / 1000.0, full = k.base + k.per_k * kk;
-  const double last = rest == 0 ? 0.0 : k.per_cu == 2 && rest > 32 ? full : k.last_base + kk * (k.last_per_k + k.last_fill * (double)rest / 32);
-  return k.launch + (double)(per / round) * full + last;
+template <int BN, int BM, int WN, int WM, int PER_CU, int OUT>
+__global__ __launch_bounds__(64 * (BN / WN) * (BM / WM), PER_CU * (BN / WN) * (BM / WM) / 4) void small_kernel(TilesArgs a) {
+  typedef ProductTiles<BN, BM, WN, WM, false, 3> P;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[P::LDS];
+  static_assert(PER_CU * P::LDS <= 160 * 1024, "LDS");
+  const int mt = (a.M + BM - 1) / BM;
+  int tn, tm;
+  if (!product_tile((a.N + BN - 1) / BN, mt * a.slices, min(mt, GROUP), &tn, &tm)) return;
+  const int slice = tm / mt, k0 = slice * a.slice_k, K = min(a.slice_k, a.K - k0), m0 = (tm - slice * mt) * BM, n0 = tn * BN;
+  const int rows = min(BN, a.N - n0), count = min(BM, a.M - m0);
+  const tile_uintx4 w = tile_buffer(a.w + (size_t)n0 * a.K + k0, ((unsigned)rows * (unsigned)a.K - (unsigned)k0) * 2u);
+  const tile_uintx4 x = tile_buffer(a.x + (size_t)m0 * a.K + k0, ((unsigned)count * (unsigned)a.K - (unsigned)k0) * 2u);
+  tile_floatx4 acc[P::FN][P::FM];
+  P::run(lds, w, x, K, a.K, [&](int i) { return i < count ? i * a.K * 2 : TILE_NO_ROW; }, acc);
+  const int m = m0 + P::wm(), n = n0 + P::wn();
+  if constexpr (OUT == OUT_SUMS) small_out<BN, BM, WN, WM, OUT, ACT_NONE>(a, acc, slice, m, n);
+  else switch (a.act) {
+    case ACT_GELU_TANH: small_out<BN, BM, WN, WM, OUT, ACT_GELU_TANH>(a, acc, 0, m, n); break;
+    case ACT_SILU: small_out<BN, BM, WN, WM, OUT, ACT_SILU>(a, acc, 0, m, n); break;
+    case ACT_NONE: if constexpr (OUT == OUT_ACT) small_out<BN, BM, WN, WM, OUT, ACT_NONE>(a, acc, 0, m, n); break;
+    default: small_out<BN, BM, WN, WM, OUT, OUT == OUT_PAIRS ? ACT_CLAMPED_SWISH : ACT_RELU_SQUARED>(a, acc, 0, m, n); break;
+  }
 }
 
-static bool eight_waves(int kind) { return kind == TILE_192_128 || kind == TILE_128_128; }
+enum { TILE_256_256, TILE_320_192, TILE_128_64, TILE_128_128, TILE_384_160, TILE_256_192, TILE_192_256, TILE_256_128, TILE_64_64, TILE_KINDS };
+
+// A tile's size and the workgroups of it to a CU.
+static const struct { int bn, bm, per_cu; } kinds[TILE_KINDS] = {
+    {256, 256, 1}, {320, 192, 1}, {128, 64, 2}, {128, 128, 1}, {384, 160, 1}, {256, 192, 1}, {192, 256, 1}, {256, 128, 1}, {64, 64, 3}};
+
+// us of a launch with tiles of a kind: a launch, a full round of the chip (and each 1,000 k-values of it), the last round by the workgroups on its
+// fullest CU (and each 1,000 k-values, and those times the share of CUs that have the last of them: fewer of them find memory faster, and
+// the chip's power goes further).
+struct TileCost { double launch, base, per_k, last[3][3]; };
+
+// ... of gate/up.  Tiles by small waves: fitted to 5,534 sizes of 65 to 1,200 rows, 1,024 to 38,000 weight rows, 128 to 4,096 k-values, off by 9 to 10 %
+// in the mean square.
+static const TileCost pairs_cost[TILE_KINDS] = {
+    {3.07, 9.00, 22.71, {{8.66, 15.99, 5.92}}}, {2.39, 9.30, 21.06, {{8.14, 14.48, 4.28}}},
+    {2.92, 2.70, 15.15, {{1.44, 5.26, 3.15}, {1.97, 13.46, 3.98}}}, {1.96, 4.47, 11.42, {{4.08, 7.21, 4.81}}},
+    {3.16, 8.88, 22.56, {{7.07, 14.47, 5.78}}}, {2.32, 7.33, 17.34, {{6.39, 12.35, 4.09}}},
+    {2.81, 7.66, 16.78, {{5.97, 11.85, 4.51}}}, {2.82, 5.06, 14.36, {{4.16, 9.91, 4.28}}},
+    {3.64, 2.14, 13.25, {{0.67, 3.48, 1.61}, {0.96, 7.60, 2.26}, {1.19, 12.75, 2.54}}}};
+
+// ... of the partial sums of a slice (380 sizes of 896 to 20,000 k-values in 1 to 8 slices: off by 5 to 7 % in the mean square; 160 more of cold
+// weights: 6 to 7.5 %, tiles of 256 x 128, which have got three slots since, 9.7 %, of which 4 % too long; the choice is 1.0 % off the best in the mean,
+// 0.7 % with those fitted again).  Tiles by small waves: 51,415 products of 8,424 sizes of 65 to 1,200 rows, 256 to 8,192 weight rows, 256 to 19,000
+// k-values in 1 to 16 slices, 11 to 12 %.
+static const TileCost sums_cost[TILE_KINDS] = {
+    {1.71, 9.86, 22.96, {{10.23, 15.63, 6.15}}}, {3.43, 8.36, 21.49, {{8.44, 15.09, 4.84}}}, {}, {1.87, 4.35, 11.28, {{2.98, 7.07, 5.83}}},
+    {2.80, 7.93, 22.05, {{9.30, 15.29, 4.32}}}, {2.78, 6.62, 18.46, {{7.16, 11.93, 5.03}}}, {1.58, 6.75, 18.74, {{7.87, 11.78, 5.63}}},
+    {1.86, 4.34, 15.21, {{5.42, 10.92, 3.72}}}, {3.05, 2.46, 13.31, {{0.21, 3.68, 1.72}, {1.07, 7.25, 2.71}, {1.90, 12.21, 2.60}}}};
+
+static double tile_us(int kind, const TileCost* costs, int M, int N, int slices, int slice_k) {
+  const auto& k = kinds[kind];
+  const TileCost& c = costs[kind];
+  const long long tiles = (long long)((N + k.bn - 1) / k.bn) * ((M + k.bm - 1) / k.bm) * slices, per = (tiles + 7) / 8, round = 32 * k.per_cu;      // (of an XCD)
+  const int rest = (int)(per % round), fullest = (rest + 31) / 32;
+  const double kk = slice_k / 1000.0;
+  double us = c.launch + (double)(per / round) * (c.base + c.per_k * kk);
+  if (rest > 0) {
+    const double* last = c.last[fullest - 1];
+    us += last[0] + kk * (last[1] + last[2] * (rest - 32 * (fullest - 1)) / 32.0);
+  }
+  return us;
+}
+
+static bool small_waves(int kind) { return kind == TILE_128_64 || kind == TILE_128_128 || kind == TILE_64_64; }
 
 static int choose_tile(int M, int N, int K, int out) {
   int best = 0;
   for (int i = 1; i < TILE_KINDS; ++i)
-    if (!(out == OUT_ACT && eight_waves(i)) && tiles_us(i, M, N, K) < tiles_us(best, M, N, K)) best = i;
+    if (!(out == OUT_ACT && i == TILE_128_64) && tile_us(i, pairs_cost, M, N, 1, K) < tile_us(best, pairs_cost, M, N, 1, K)) best = i;
   return best;
 }
 
-// us of the partial sums of a slice of slice_k values, the coefficients as for `kinds` but of this product (380 sizes of 896 to 20,000
-// k-values in 1 to 8 slices: off by 5 to 7 % in the mean square; 160 more of cold weights: 6 to 7.5 %, tiles of 256 x 128, which have got three
-// slots since, 9.7 %, of which 4 % too long; the choice is 1.0 % off the best in the mean, 0.7 % with those fitted again) and, for every slice after the first, of what the reader of the sums pays
+// ... and what the reader of the sums pays for every slice after the first
 static double sums_us(int kind, int M, int N, int slices, int slice_k) {
-  static const double sums[TILE_KINDS][6] = {
-      {1.71, 9.86, 22.96, 10.23, 15.63, 6.15}, {3.43, 8.36, 21.49, 8.44, 15.09, 4.84}, {}, {}, {2.80, 7.93, 22.05, 9.30, 15.29, 4.32},
-      {2.78, 6.62, 18.46, 7.16, 11.93, 5.03}, {1.58, 6.75, 18.74, 7.87, 11.78, 5.63}, {1.86, 4.34, 15.21, 5.42, 10.92, 3.72}};
-  const double* c = sums[kind];
-  const long long tiles = (long long)((N + kinds[kind].bn - 1) / kinds[kind].bn) * ((M + kinds[kind].bm - 1) / kinds[kind].bm) * slices;
-  const long long per = (tiles + 7) / 8, rest = per % 32;
-  const double kk = slice_k / 1000.0;
-  const double last = rest == 0 ? 0.0 : c[3] + kk * (c[4] + c[5] * (double)rest / 32);
-  return c[0] + (double)(per / 32) * (c[1] + c[2] * kk) + last + (slices > 1 ? 0.5 + 1.2e-6 * (double)M * (double)N * (slices - 1) : 0.0);
+  return tile_us(kind, sums_cost, M, N, slices, slice_k) + (slices > 1 ? 0.5 + 1.2e-6 * (double)M * (double)N * (slices - 1) : 0.0);
 }
 
 #define SUMS_MIN_ROWS 257
@@ -312,7 +362,24 @@ extern "C" int ifx_gemm_tiles_sums_plan(int M, int N, int K, int library_slices,
     const int slice_k = ((K + s - 1) / s + 63) / 64 * 64;
     if ((K + slice_k - 1) / slice_k != s || (s > 1 && (long long)s * M * N * 4 > SUMS_MAX_BYTES)) continue;
     for (int kind = 0; kind < TILE_KINDS; ++kind) {
-      if (eight_waves(kind)) continue;
+      if (small_waves(kind)) continue;
+      const double us = sums_us(kind, M, N, s, slice_k);
+      if (best == 0 || us < least) best = s << 8 | kind, least = us;
+    }
+  }
+  return best;
+}
+
+// The same for up to FEW_MOST multiplications, with tiles by small waves, too: slices (1 without `keep`: the plain product) << 8 | tile.
+#define FEW_MAX_SLICES 16
+extern "C" int ifx_gemm_tiles_few_plan(int M, int N, int K, int keep) {
+  int best = 0;
+  double least = 0;
+  for (int s = 1; s <= (keep ? FEW_MAX_SLICES : 1); ++s) {
+    const int slice_k = ((K + s - 1) / s + 63) / 64 * 64;
+    if ((K + slice_k - 1) / slice_k != s || (s > 1 && (slice_k < 128 || (long long)s * M * N * 4 > SUMS_MAX_BYTES))) continue;
+    for (int kind = 0; kind < TILE_KINDS; ++kind) {
+      if (kind == TILE_128_64) continue;
       const double us = sums_us(kind, M, N, s, slice_k);
       if (best == 0 || us < least) best = s << 8 | kind, least = us;
     }
@@ -330,17 +397,22 @@ static void launch_waves(const TilesArgs& a, int out, hipStream_t s) {
 }
 
 template <int BN, int BM, int WN, int WM, int PER_CU>
-static void launch_pairs(const TilesArgs& a, hipStream_t s) {
-  const int blocks = ((a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) + 7) / 8 * 8;
-  hipLaunchKernelGGL((pairs_kernel<BN, BM, WN, WM, PER_CU>), dim3(blocks), dim3(64 * (BN / WN) * (BM / WM)), 0, s, a);
+static void launch_small(const TilesArgs& a, int out, hipStream_t s) {
+  const dim3 blocks(((a.N + BN - 1) / BN * ((a.M + BM - 1) / BM) * a.slices + 7) / 8 * 8), threads(64 * (BN / WN) * (BM / WM));
+  if (out == OUT_PAIRS) hipLaunchKernelGGL((small_kernel<BN, BM, WN, WM, PER_CU, OUT_PAIRS>), blocks, threads, 0, s, a);
+  if constexpr (BN == BM) {
+    if (out == OUT_ACT) hipLaunchKernelGGL((small_kernel<BN, BM, WN, WM, PER_CU, OUT_ACT>), blocks, threads, 0, s, a);
+    else if (out == OUT_SUMS) hipLaunchKernelGGL((small_kernel<BN, BM, WN, WM, PER_CU, OUT_SUMS>), blocks, threads, 0, s, a);
+  }
 }
 
 static void launch_kind(const TilesArgs& a, int kind, int out, hipStream_t s) {
   switch (kind) {
     case TILE_256_256: launch_waves<8, 8>(a, out, s); break;
     case TILE_320_192: launch_waves<10, 6>(a, out, s); break;
-    case TILE_192_128: launch_pairs<192, 128, 48, 64, 2>(a, s); break;
-    case TILE_128_128: launch_pairs<128, 128, 32, 64, 2>(a, s); break;
+    case TILE_128_64: launch_small<128, 64, 32, 32, 2>(a, out, s); break;
+    case TILE_128_128: launch_small<128, 128, 64, 32, 1>(a, out, s); break;
+    case TILE_64_64: launch_small<64, 64, 32, 32, 3>(a, out, s); break;
     case TILE_384_160: launch_waves<12, 5>(a, out, s); break;
     case TILE_256_192: launch_waves<8, 6>(a, out, s); break;
     case TILE_192_256: launch_waves<6, 8>(a, out, s); break;
@@ -362,7 +434,7 @@ extern "C" int ifx_gemm_tiles(const void* x, const void* w, void* result, int M,
   if (M == 0) return 0;
   const TilesArgs a{(const bf16_t*)x, (const bf16_t*)w, result, M, N, K, act, limit, 1, K};
   const int kind = tile < 0 ? choose_tile(M, N, K, out) : tile;
-  IFX_REQUIRE(kind < TILE_KINDS && !(out == OUT_ACT && eight_waves(kind)), "gemm_tiles: tile %d", tile);
+  IFX_REQUIRE(kind < TILE_KINDS && !(out == OUT_ACT && kind == TILE_128_64), "gemm_tiles: tile %d", tile);
   launch_kind(a, kind, out, (hipStream_t)stream);
   IFX_LAUNCH_CHECK();
 }
@@ -373,7 +445,7 @@ extern "C" int ifx_gemm_tiles_sums(const void* x, const void* w, float* parts, i
   IFX_REQUIRE(slices > 0 && slice_k > 0 && slice_k % 64 == 0 && (long long)slices * slice_k >= K && (long long)(slices - 1) * slice_k < K,
               "gemm_tiles_sums: %d slices of %d values of K=%d", slices, slice_k, K);
   IFX_REQUIRE(((size_t)x | (size_t)w | (size_t)parts) % 16 == 0, "gemm_tiles_sums: x, the weight and the result must lie on 16 bytes");
-  IFX_REQUIRE(tile >= 0 && tile < TILE_KINDS && !eight_waves(tile), "gemm_tiles_sums: tile %d", tile);
+  IFX_REQUIRE(tile >= 0 && tile < TILE_KINDS && tile != TILE_128_64, "gemm_tiles_sums: tile %d", tile);
   if (M == 0) return 0;
   const TilesArgs a{(const bf16_t*)x, (const bf16_t*)w, parts, M, N, K, ACT_NONE, 0.f, slices, slice_k};
   launch_kind(a, tile, OUT_SUMS, (hipStream_t)stream);

@@ -162,7 +162,7 @@ __global__ __launch_bounds__(512, 4) void experts_kernel(ExpertsArgs a) {
   const tile_uintx4 x = MODE == MODE_GATE_UP ? tile_buffer(a.x, (unsigned)a.T * (unsigned)a.K * 2u)
                                              : tile_buffer(a.x + (size_t)start * a.K, (unsigned)count * (unsigned)a.K * 2u);
   tile_floatx4 acc[P::FN][P::FM];
-  P::run(lds, w, x, a.K, [&](int i) { return i >= count ? TILE_NO_ROW : (MODE == MODE_GATE_UP ? items[i] / a.top : i) * a.K * 2; }, acc);
+  P::run(lds, w, x, a.K, a.K, [&](int i) { return i >= count ? TILE_NO_ROW : (MODE == MODE_GATE_UP ? items[i] / a.top : i) * a.K * 2; }, acc);
   const int lane = tid % 64, g = lane / 16;
 #pragma unroll
   for (int b = 0; b < P::FM; ++b) {

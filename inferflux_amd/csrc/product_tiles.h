@@ -59,9 +59,10 @@ struct ProductTiles {
   static __device__ __forceinline__ int wm() { return wave() / (BN / WN) * WM; }
 
   // w: the tile's BN weight rows of K values each (TILED: from the tile's first row tile on, k_tiles tiles of 32 k-values to
-  // a row tile, an even number); x: row m of the tile starts at byte x_offset(m) (TILE_NO_ROW: zeros).  K a multiple of 8.
+  // a row tile, an even number); x: row m of the tile starts at byte x_offset(m) (TILE_NO_ROW: zeros).  K a multiple of 8; rows of
+  // W (not TILED) w_pitch values apart.
   template <class XOffset>
-  static __device__ __forceinline__ void run(unsigned char* lds, const tile_uintx4& w, const tile_uintx4& x, int K, XOffset x_offset,
+  static __device__ __forceinline__ void run(unsigned char* lds, const tile_uintx4& w, const tile_uintx4& x, int K, int w_pitch, XOffset x_offset,
                                              tile_floatx4 (&acc)[FN][FM]) {
     const int wid = wave(), lane = threadIdx.x % 64, col = lane % 16, g = lane / 16;
     const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
@@ -72,7 +73,7 @@ struct ProductTiles {
     for (int i = 0; i < LW; ++i) {
       const int j = wid * LW + i, row = 8 * j + lane / 8;
       wk[i] = TILED ? 0 : 8 * (lane % 8 ^ place(row));
-      wo[i] = TILED ? (j / 2) * steps * 2048 + j % 2 * 1024 + lane * 16 : row * K * 2 + wk[i] * 2;
+      wo[i] = TILED ? (j / 2) * steps * 2048 + j % 2 * 1024 + lane * 16 : row * w_pitch * 2 + wk[i] * 2;
     }
 #pragma unroll
     for (int i = 0; i < LX; ++i) {

@@ -1508,7 +1508,8 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
     tile_rows = 16
     if isinstance(x, ScaledRows) and not takes_scaled_rows(x.shape[0], weight):
         raise KernelError(f"linear: scaled rows are not taken for {x.shape[0]} rows and this weight")
-    if isinstance(weight, LinearWeight):
+    prepared = isinstance(weight, LinearWeight)
+    if prepared:
         weight, tiled, order, tile_rows = weight.rows, weight.tiled, weight.order, weight.tile_rows
     columns = columns_on_16_bytes(x)      # (the product for few rows reads them where they lie, every other one takes a copy)
     if weight.dtype == torch.float32:
@@ -1525,6 +1526,10 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
     kind = _small_m_kernel(M, weight.shape[0], K, tiled is not None)
     if columns and kind != "skinny":
         x = x.contiguous()
+    if prepared and M > SKINNY_MAX_M and (keep_slices or kind is None) and out_dtype == torch.bfloat16 and not torch.cuda.tunable.is_enabled():
+        plan = few_tiles_plan(M, weight.shape[0], K, bool(keep_slices))
+        if plan and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and weight.is_contiguous():
+            return _by_plan(x, weight, plan)
     if kind == "skinny":
         ring = ring_takes_few(x, LinearWeight(weight, tiled, order, tile_rows), keep_slices and out_dtype == torch.bfloat16)
         if ring:
@@ -1541,8 +1546,7 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
         if plan and torch.cuda.is_current_stream_capturing():
             plan = _tiles_sums_plan(M, weight.shape[0], K, True)
         if plan and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0:
-            slices, tile = plan >> 8, plan & 255
-            return sums_tiles(x, weight, slices, -(-(-(-K // slices)) // 64) * 64, tile) if slices > 1 else act_tiles(x, weight, ACT_NONE, tile)
+            return _by_plan(x, weight, plan)
     if keep_slices:
         S = library_k_slices(M, weight.shape[0], K)
         if S > 1 and not torch.cuda.is_current_stream_capturing():
@@ -1551,6 +1555,43 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
             ws = weight.view(weight.shape[0], S, K // S).permute(1, 2, 0)
             return SliceSums(torch.bmm(xs, ws, out_dtype=torch.float32), out_dtype)
     return torch.matmul(x, weight.t())
+
+
+def _by_plan(x: torch.Tensor, weight: torch.Tensor, plan: int):
+    slices, tile, K = plan >> 8, plan & 255, x.shape[1]
+    return sums_tiles(x, weight, slices, -(-(-(-K // slices)) // 64) * 64, tile) if slices > 1 else act_tiles(x, weight, ACT_NONE, tile)
+
+
+FEW_MAX_ROWS = 2048              # rows, weight rows and k-values that ``few_tiles_plan`` was measured for
+FEW_MIN_N, FEW_MAX_N, FEW_PAIRS_MAX_N = 256, 8192, 65536
+FEW_MIN_K, FEW_MAX_K = 256, 20000
+# products whose reader adds slices: k-values from which ..., multiplications up to which ..., against the library and against the product that shares x through LDS
+FEW_SLICED = ((8192, 6.4e9, 3.2e9), (4096, 6.4e9, 1.6e9), (0, 3.2e9, 1.6e9))
+FEW_WHOLE = ((512, 1, 1024), (1024, 1, 512), (3072, 128, 256))          # the plain product: k-values up to which ..., tiles of 64 x 64 from and up to which
+
+
+@functools.lru_cache(maxsize=4096)
+def few_tiles_plan(M: int, N: int, K: int, keep_slices: bool) -> int:
+    """slices << 8 | tile of the tiles of ``gemm_tiles`` that take a model's weight [N, K] (a ``LinearWeight``) at 65 to 2,048 rows, 0: another product
+    does.  Tiles of 64 x 64 and of 128 x 128 in three stages are made for these sizes, where tiles of 256 x 256 are few.  What the others take over
+    their time, geometric mean and worst, 6,700 products of cold weights with what the slices cost their reader, by M N K:
+        against the library's and large tiles', 129 rows on: up to 4e8 1.45 and 0.94, 4e8 to 1.6e9 1.6 and 0.95, 1.6e9 to 3.2e9 1.35 and 0.85 (3 % slower
+        than 0.97), 3.2e9 to 6.4e9 with K up to 4,096 1.03 and 0.66 (38 %), deeper 1.27 and 0.88 (6 %); weights of more than 8,192 rows 0.79 to 0.9
+        against the product that shares x through LDS, 65 to 128 rows: up to 8e8 1.7 and 1.08, 8e8 to 1.6e9 1.47 and 1.07, 1.6e9 to 3.2e9 with K of 4,096 to
+        8,192 1.13 and 0.81 (30 %), deeper 1.4 and 0.89
+    and, without slices, of 2,900 against the library: K up to 512 1.35 and 1.01, 512 to 1,024 1.2 and 0.84 (up to 512 tiles of 64 x 64; 18 to 24 % of more are
+    slower), 1,024 to 3,072 with 128 to 256 tiles 1.18 and 0.87 (9 %), otherwise 1.05 with a third slower.  A bare tensor goes where ``_tiles_sums_plan`` says."""
+    if not (SKINNY_MAX_M < M <= FEW_MAX_ROWS and FEW_MIN_N <= N <= FEW_MAX_N and FEW_MIN_K <= K <= FEW_MAX_K) or N % 8 or K % 8:
+        return 0
+    if keep_slices:
+        _, most, most_streamed = next(line for line in FEW_SLICED if K >= line[0])
+        if M * N * K > (most if M > WIDE_MAX_M else most_streamed):
+            return 0
+    else:
+        tiles = -(-M // 64) * -(-N // 64)
+        if not any(K <= deepest and least <= tiles < most for deepest, least, most in FEW_WHOLE):
+            return 0
+    return load_module("gemm_tiles").fn("ifx_gemm_tiles_few_plan", (I, I, I, I))(M, N, K, int(keep_slices))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1689,6 +1730,18 @@ def pairs_tiles_take(M: int, N: int, K: int) -> bool:
     return any(K <= deepest and M * N >= 65536 * tiles for deepest, tiles in FEW_TILES) and not torch.cuda.tunable.is_enabled()
 
 
+def few_pairs_take(M: int, N: int, K: int) -> bool:
+    """Whether that product takes a model's gate/up pairs [N, K] (a ``LinearWeight``) at 65 to 2,048 rows, where tiles by small waves are among its
+    choices.  The library's product and the activation, or up to 128 rows the product that shares x through LDS, over this one's time, geometric mean
+    and worst of 7,100: up to 128 rows 2.0 and 0.90; more, K up to 1,536 1.2 to 1.7 and 0.92, 1,536 to 2,560 and up to 64 tiles of 256 x 256 1.25 and 0.84,
+    2,560 to 4,096 and 2 to 16 tiles 1.23 and 0.93 (fewer 0.96 and 0.83); 1,536 to 2,560 and more tiles 1.0, from 700 rows on 0.98 and 0.88."""
+    if not (SKINNY_MAX_M < M <= FEW_MAX_ROWS and FEW_MIN_N <= N <= FEW_PAIRS_MAX_N and N % 4 == 0 and FEW_MIN_K <= K <= 4096 and K % 8 == 0):
+        return False
+    tiles = M * N / 65536
+    fits = K <= 1536 or (M <= 300 or tiles <= 64 if K <= 2560 else (M <= WIDE_MAX_M or tiles >= 2) and tiles <= 16)
+    return fits and not torch.cuda.tunable.is_enabled()
+
+
 def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limit: float = 0.0, tile: int = -1) -> torch.Tensor:
     """``linear_swiglu`` of many rows in bfloat16 as one launch ([N, K] ``pairs``, N a multiple of 4 and K of 8, both on 16 bytes);
     ``tile``: one of the kernel's tiles instead of its choice."""
@@ -1741,7 +1794,8 @@ def linear_swiglu(x: torch.Tensor, weight_pairs, act: int = ACT_SILU, limit: flo
         raise KernelError("linear_swiglu: a tile order is not supported for gate/up pairs")
     columns = columns_on_16_bytes(x)          # (as for ``linear``)
     if not isinstance(x, ScaledRows) and rows.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and K == rows.shape[1] \
-            and (pairs_tiles_take(M, rows.shape[0], K) or many_tiles_take(M, rows.shape[0], K)):
+            and (pairs_tiles_take(M, rows.shape[0], K) or many_tiles_take(M, rows.shape[0], K)
+                 or isinstance(weight_pairs, LinearWeight) and few_pairs_take(M, rows.shape[0], K)):
         whole = x.contiguous() if columns else x
         if whole.data_ptr() % 16 == 0 and rows.is_contiguous() and rows.data_ptr() % 16 == 0:
             return swiglu_tiles(whole, rows, act, limit)
