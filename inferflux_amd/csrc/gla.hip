@@ -32,6 +32,7 @@
 //              S <- exp(sum log alpha) S + S_c; the request's new state goes into its slot.
 // MODE 2: a chunk from the state it starts from; writes y.
 #include "common.h"
+#include "tile_acts.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -279,6 +280,274 @@ __global__ __launch_bounds__(256) void gla_combine_kernel(CombineArgs a) {
   *slot = S;
 }
 
+#if !TIME_MIX
+// ---- chunks on the matrix cores ------------------------------------------------------------------------------------------
+// A chunk's walk (MODE 1 and 2 for bfloat16 rows, heads of up to 64 x 128) by blocks of 16 tokens, with B_t the sum of the block's log alpha up to
+// token t, per channel, and the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: float products, float sums) for every product:
+//   o_t = (q_t exp(B_t))^T S + sum_(s <= t) (sum_i q_t[i] exp(B_t - B_7)[i] k_s[i] exp(B_7 - B_s)[i]) v_s
+//   S  <- exp(B_15) S + sum_s (k_s exp(B_15 - B_s)) v_s^T
+// A workgroup is one head of a chunk; a wave owns 32 columns of S in the instruction's output layout, whose registers are at the same time
+// the operand that the read-out wants (with its channels in another order), so S never leaves them.  A block whose decays are strong
+// (B_15 below -8 in some channel: exp(B_7 - B_s) would lose digits, and overflow) is walked token by token as the kernel above does.
+// What bounds it is the matrix instruction (88 of 32 cycles a wave and block in MODE 2), the exponentials beside it and the block's four meeting
+// points.  Both walks and what joins the chunks, 16 heads of 64 x 128, by the kernel above / here: 4,026 rows of 16 requests 268 / 113 us, 8,192 of
+// four 450 / 167, a request of 200 71 / 25.  (With expf() and log1pf() 217 of the 113 us.)  The state against 64 bits, tau 16, decays' logits of
+// deviation 1 about 0 and 0.3 about 4, chunks of 32: 9.0e-8 and 2.0e-7 there, 8.3e-8 and 1.6e-7 here.
+#define BLOCK 16
+#define BLOCK_MIN_DECAY -8.f
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gla_f4;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 gla_bf16x4;
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 gla_bf16x8;
+
+// exp(x) for |x| <= 8 by the hardware's exp2 of x log2(e) in two parts, and log_sigmoid by its exp2 and log2: an eighth of the instructions of expf(),
+// whose ranges are not needed here, and of log1pf().  The logarithm's error is 2^-23 of 1 + exp(-|x|), as alpha's own rounding.
+__device__ __forceinline__ float block_exp(float x) {
+  const float h = x * 1.44269504f, e = __builtin_amdgcn_exp2f(h);
+  return fmaf(e, 0.693147181f * fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504f, -h)), e);
+}
+__device__ __forceinline__ float block_log_sigmoid(float x) {
+  return fminf(x, 0.f) - 0.693147181f * __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * fabsf(x)));
+}
+// Over the lanes of a row of 16: those up to this one, and those behind it.  (What a token leaves of its write is summed from the block's end, not
+// formed as a difference: the last tokens' sums are then small, and exact to their own last digit.)
+#define SHIFTED(v, ctrl) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), (ctrl), 0xf, 0xf, true))
+__device__ __forceinline__ float sum_up_to(float v) {
+  v += SHIFTED(v, 0x111);
+  v += SHIFTED(v, 0x112);
+  v += SHIFTED(v, 0x114);
+  v += SHIFTED(v, 0x118);
+  return v;
+}
+__device__ __forceinline__ float sum_behind(float v) {
+  v = SHIFTED(v, 0x101);
+  v += SHIFTED(v, 0x101);
+  v += SHIFTED(v, 0x102);
+  v += SHIFTED(v, 0x104);
+  v += SHIFTED(v, 0x108);
+  return v;
+}
+#undef SHIFTED
+
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void gla_blocks_kernel(GlaArgs a) {
+  constexpr int D = 64, DV = 128, P = D + 4, PV = DV + 4;
+  __shared__ __attribute__((aligned(16))) float lq[BLOCK][P], lk[BLOCK][P], la[BLOCK][P], lqm[MODE == 2 ? BLOCK : 1][P], lkm[MODE == 2 ? BLOCK : 1][P], lv[BLOCK][PV];
+  __shared__ __attribute__((aligned(16))) float keep[D];
+  __shared__ float squares[4][BLOCK];
+  const int unit = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, wid = tid / WAVE, lane = tid % WAVE, i16 = lane % 16, g = lane / 16;
+  const int t0 = a.chunk_t0[unit], n = a.chunk_len[unit], H = a.H;
+  if (n <= 0) return;
+  const bf16_t *rq = (const bf16_t*)a.q, *rk = (const bf16_t*)a.k, *rv = (const bf16_t*)a.v, *rg = (const bf16_t*)a.g;
+  // S[ib][jb][r]: channel 16 ib + 4 g + r of column 32 wid + 16 jb + i16
+  gla_f4 S[4][2];
+  float* sp = a.chunk_state + ((size_t)unit * H + head) * DV * D + (size_t)(32 * wid + i16) * D + 4 * g;
+#pragma unroll
+  for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) S[ib][jb] = MODE == 2 ? *(const gla_f4*)(sp + (size_t)16 * jb * D + 16 * ib) : gla_f4{0.f, 0.f, 0.f, 0.f};
+  float w[2][4];
+  if (MODE == 2) {
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[jb][r] = load_dyn(a.norm_w, a.norm_dtype, 32 * wid + 16 * jb + 4 * g + r);
+  }
+  // a block's rows on their way: token tid / 16, four channels and eight values of it a thread
+  // (channels from d on count as zero keys and queries that do not decay)
+  const int lt = tid / 16, lc = 4 * (tid % 16), d = a.d, at = head * d + (lc < d ? lc : 0);
+  gla_f4 bias = {0.f, 0.f, 0.f, 0.f};
+  if (a.z_bias) bias = *(const gla_f4*)(a.z_bias + at);
+  gla_bf16x4 nq, nk;
+  gla_bf16x8 nv;
+  gla_f4 nz;
+  gla_bf16x4 ng[2], gate[2];
+  auto fetch = [&](int s0) {          // (rows beyond the chunk are asked for as its last)
+    const size_t t = t0 + min(s0 + lt, n - 1);
+    if (MODE == 2) nq = *(const gla_bf16x4*)(rq + t * a.ld + at);
+    nk = *(const gla_bf16x4*)(rk + t * a.ld + at);
+    nz = *(const gla_f4*)(a.z + t * (size_t)(H * d) + at);
+    nv = *(const gla_bf16x8*)(rv + t * a.ld + head * DV + 2 * lc);
+    if (MODE == 2) {
+      const size_t tg = t0 + min(s0 + i16, n - 1);
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) ng[jb] = *(const gla_bf16x4*)(rg + tg * a.ld + head * DV + 32 * wid + 16 * jb + 4 * g);
+    }
+  };
+  fetch(0);
+  gla_f4 loga = {0.f, 0.f, 0.f, 0.f};          // of the channels ch .. ch + 3 below
+  const int ch = 16 * wid + 4 * g;             // with token i16 this thread's of the block's transformed rows
+#pragma unroll 1
+  for (int s0 = 0; s0 < n; s0 += BLOCK) {
+    const bool row = s0 + lt < n, in = row && lc < d;
+    gla_f4 x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = in ? block_log_sigmoid(nz[e] + bias[e]) * a.inv_tau : 0.f;
+    *(gla_f4*)&la[lt][lc] = x;
+    *(gla_f4*)&lk[lt][lc] = in ? gla_f4{(float)nk[0], (float)nk[1], (float)nk[2], (float)nk[3]} : gla_f4{0.f, 0.f, 0.f, 0.f};
+    if (MODE == 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = in ? (float)nq[e] * a.q_scale : 0.f;
+      *(gla_f4*)&lq[lt][lc] = x;
+      gate[0] = ng[0], gate[1] = ng[1];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = row ? (float)nv[4 * h + e] : 0.f;
+      *(gla_f4*)&lv[lt][2 * lc + 4 * h] = x;
+    }
+    if (s0 + BLOCK < n) fetch(s0 + BLOCK);
+    __syncthreads();
+    const gla_f4 mine = *(const gla_f4*)&la[i16][ch];
+    gla_f4 upto, whole, half;
+    bool strong = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      upto[e] = sum_up_to(mine[e]);
+      whole[e] = __shfl(upto[e], lane | 15, WAVE);
+      half[e] = __shfl(upto[e], (lane & 48) + 7, WAVE);
+      strong = strong || !(whole[e] > BLOCK_MIN_DECAY);
+      loga[e] += whole[e];
+    }
+    gla_f4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    if (__syncthreads_or(strong)) {
+      const int ns = min(BLOCK, n - s0);
+#pragma unroll 1
+      for (int tt = 0; tt < ns; ++tt) {
+        float v[2], sum[2] = {0.f, 0.f};
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb) v[jb] = lv[tt][32 * wid + 16 * jb + i16];
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          const gla_f4 l = *(const gla_f4*)&la[tt][16 * ib + 4 * g], k = *(const gla_f4*)&lk[tt][16 * ib + 4 * g];
+          const gla_f4 q = MODE == 2 ? *(const gla_f4*)&lq[tt][16 * ib + 4 * g] : gla_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float al = expf(l[r]);
+#pragma unroll
+            for (int jb = 0; jb < 2; ++jb) {
+              S[ib][jb][r] = fmaf(al, S[ib][jb][r], k[r] * v[jb]);
+              if (MODE == 2) sum[jb] = fmaf(S[ib][jb][r], q[r], sum[jb]);
+            }
+          }
+        }
+        if (MODE == 2) {
+#pragma unroll
+          for (int jb = 0; jb < 2; ++jb) {
+            sum[jb] += __shfl_xor(sum[jb], 16, WAVE);
+            sum[jb] += __shfl_xor(sum[jb], 32, WAVE);
+            if (g == 0) lv[tt][32 * wid + 16 * jb + i16] = sum[jb];          // (in place of the values, this wave's own)
+          }
+        }
+      }
+      if (MODE == 2) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb) o[jb] = *(const gla_f4*)&lv[i16][32 * wid + 16 * jb + 4 * g];
+      }
+    } else {
+      gla_f4 k = *(const gla_f4*)&lk[i16][ch], kl, km, q1, qm;
+      const gla_f4 q = MODE == 2 ? *(const gla_f4*)&lq[i16][ch] : k;
+      if (i16 == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kl[e] = block_exp(whole[e]);
+        *(gla_f4*)&keep[ch] = kl;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kl[e] = k[e] * block_exp(sum_behind(mine[e]));
+        if (MODE == 2) {
+          km[e] = k[e] * block_exp(half[e] - upto[e]);
+          qm[e] = q[e] * block_exp(upto[e] - half[e]);
+          q1[e] = q[e] * block_exp(upto[e]);
+        }
+      }
+      *(gla_f4*)&lk[i16][ch] = kl;          // (each thread in place of what it read)
+      if (MODE == 2) {
+        *(gla_f4*)&lq[i16][ch] = q1;
+        *(gla_f4*)&lqm[i16][ch] = qm;
+        *(gla_f4*)&lkm[i16][ch] = km;
+      }
+      __syncthreads();
+      float v[2][4];
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[jb][r] = lv[4 * g + r][32 * wid + 16 * jb + i16];
+      if (MODE == 2) {
+        gla_f4 pairs = {0.f, 0.f, 0.f, 0.f};          // what token i16 takes of tokens 4 g + r
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          const gla_f4 ks = *(const gla_f4*)&lkm[i16][16 * ib + 4 * g], qs = *(const gla_f4*)&lqm[i16][16 * ib + 4 * g], qo = *(const gla_f4*)&lq[i16][16 * ib + 4 * g];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            pairs = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[r], qs[r], pairs, 0, 0, 0);
+#pragma unroll
+            for (int jb = 0; jb < 2; ++jb) o[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[ib][jb][r], qo[r], o[jb], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float p = 4 * g + r <= i16 ? pairs[r] : 0.f;
+#pragma unroll
+          for (int jb = 0; jb < 2; ++jb) o[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[jb][r], p, o[jb], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib) {
+        const gla_f4 kept = *(const gla_f4*)&keep[16 * ib + 4 * g];
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[ib][jb][r] *= kept[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          const float kt = lk[4 * g + r][16 * ib + i16];
+#pragma unroll
+          for (int jb = 0; jb < 2; ++jb) S[ib][jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt, v[jb][r], S[ib][jb], 0, 0, 0);
+        }
+    }
+    if (MODE == 2) {
+      float ss = 0.f;
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ss = fmaf(o[jb][r], o[jb][r], ss);
+      ss += __shfl_xor(ss, 16, WAVE);
+      ss += __shfl_xor(ss, 32, WAVE);
+      if (g == 0) squares[wid][i16] = ss;
+    }
+    __syncthreads();                         // (and the next block's rows overwrite what this one read)
+    if (MODE == 2 && s0 + i16 < n) {
+      const float inv = rsqrtf((((squares[0][i16] + squares[1][i16]) + squares[2][i16]) + squares[3][i16]) / (float)DV + a.eps);
+      bf16_t* out = (bf16_t*)a.out + (size_t)(t0 + s0 + i16) * (size_t)(H * DV) + head * DV + 32 * wid + 4 * g;
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) {
+        gla_bf16x4 y;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = (__bf16)(o[jb][r] * inv * w[jb][r] * over_one_plus_exp<false>((float)gate[jb][r], (float)gate[jb][r]));
+        *(gla_bf16x4*)(out + 16 * jb) = y;
+      }
+    }
+  }
+  if (MODE == 1) {
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) *(gla_f4*)(sp + (size_t)16 * jb * D + 16 * ib) = S[ib][jb];
+    if (i16 == 0 && ch < d) *(gla_f4*)(a.chunk_loga + (size_t)unit * H * d + head * d + ch) = loga;
+  }
+}
+
+static bool blocks_take(const GlaArgs& a, int dp) {
+  return a.d <= 64 && a.d % 4 == 0 && a.dv == 128 && a.parts * dp == 64 && a.ld % 8 == 0
+         && ((size_t)a.q | (size_t)a.k | (size_t)a.v | (size_t)a.g | (size_t)a.z | (size_t)a.z_bias | (size_t)a.out | (size_t)a.chunk_state | (size_t)a.chunk_loga) % 16 == 0;
+}
+#endif
+
 template <typename T, typename TO, int DP, int MODE, int COLS>
 static void launch_gla_mode(const GlaArgs& a, int units, int threads, size_t lds, hipStream_t s) {
   if constexpr (DP <= 32) {
@@ -318,11 +587,19 @@ static int launch_gla(const GlaArgs& a, int R, int n_chunks, const int* req_chun
     launch_gla_cols<T, TO, DP, 0>(a, R, cols_walk, threads_for(cols_walk), lds, s);
     IFX_LAUNCH_CHECK();
   }
-  launch_gla_cols<T, TO, DP, 1>(a, n_chunks, cols_chunk, threads_for(cols_chunk), lds, s);
+  bool blocks = false;
+#if !TIME_MIX
+  if constexpr (sizeof(T) == 2) blocks = blocks_take(a, DP);
+  if (blocks) hipLaunchKernelGGL(gla_blocks_kernel<1>, dim3(n_chunks, a.H), dim3(256), 0, s, a);
+#endif
+  if (!blocks) launch_gla_cols<T, TO, DP, 1>(a, n_chunks, cols_chunk, threads_for(cols_chunk), lds, s);
   CombineArgs c{a.state, a.state_stride, a.state_offset, a.slots, req_chunk0, a.chunk_state, a.chunk_loga, a.H, a.d, a.dv, a.parts, DP};
   const size_t per = (size_t)a.H * a.dv * a.parts * DP;
   hipLaunchKernelGGL(gla_combine_kernel, dim3((unsigned)((per + 255) / 256), R), dim3(256), 0, s, c);
-  launch_gla_cols<T, TO, DP, 2>(a, n_chunks, cols_chunk, threads_for(cols_chunk), lds, s);
+#if !TIME_MIX
+  if (blocks) hipLaunchKernelGGL(gla_blocks_kernel<2>, dim3(n_chunks, a.H), dim3(256), 0, s, a);
+#endif
+  if (!blocks) launch_gla_cols<T, TO, DP, 2>(a, n_chunks, cols_chunk, threads_for(cols_chunk), lds, s);
   IFX_LAUNCH_CHECK();
 }
 

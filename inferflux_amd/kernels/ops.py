@@ -2147,6 +2147,13 @@ def gla_layout(d: int, dv: int) -> Tuple[int, int]:
     raise KernelError(f"gla: a head of {d} key channels and {dv} values does not fit a workgroup")
 
 
+def gla_takes_blocks(d: int, dv: int) -> bool:
+    """Whether ``gla_scan`` runs chunks of bfloat16 rows on the matrix cores for heads of d key channels and dv values (rows and decays on 16
+    bytes, as ``linear`` leaves them)."""
+    dp, parts = gla_layout(d, dv)
+    return dp * parts == 64 and d % 4 == 0 and dv == 128
+
+
 def gla_state_floats(n_heads: int, d: int, dv: int) -> int:
     dp, parts = gla_layout(d, dv)
     return n_heads * dv * parts * dp

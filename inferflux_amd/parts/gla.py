@@ -32,6 +32,21 @@ from .plan import ParamSpec, StateSpec
 
 SCAN_CHUNK = 32             # rows of a chunk where long portions are cut into chunks that run side by side
 SCAN_CHUNK_MIN_ROWS = 128   # ... which happens in steps that bring some request this many rows or more
+BLOCKS_MIN_ROWS = 48        # ... of heads whose chunks run on the matrix cores, where this many do,
+BLOCKS_FEW_MIN_ROWS, BLOCKS_FEW_REQUESTS = 24, 8          # or this many in steps of so few requests,
+BLOCKS_LONG_CHUNK, BLOCKS_LONG_ROWS = 64, 2048            # and whose chunks are longer in steps of so many rows
+
+
+def chunk_rows(longest: int, n_rows: int, n_requests: int, blocks: bool) -> int:
+    """Rows of a chunk in a step whose longest request brings ``longest`` rows, 0: its requests are walked whole.  us walked / in chunks of 32 on the
+    matrix cores, 16 and 8 heads of 64 x 128: a request of 24 rows 33 / 21, 32 / 21, of 100 122 / 23, 122 / 22; 16 of 32 44 / 42, 43 / 32, of 48 63 / 48,
+    62 / 34; 64 of 24 82 / 112, 40 / 62, of 48 146 / 146, 79 / 83, of 64 192 / 150, 103 / 84; a request of 64 beside 16 of one 80 / 47, 79 / 32.  Chunks of 32 /
+    64: 200 rows 25 / 34, 23 / 33, 1,000 40 / 41, 33 / 37, 4,026 of 16 requests 123 / 113, 73 / 72, 8,192 of four 212 / 167, 114 / 92."""
+    if not blocks:
+        return SCAN_CHUNK if longest >= SCAN_CHUNK_MIN_ROWS else 0
+    if longest < (BLOCKS_FEW_MIN_ROWS if n_requests <= BLOCKS_FEW_REQUESTS else BLOCKS_MIN_ROWS):
+        return 0
+    return BLOCKS_LONG_CHUNK if n_rows >= BLOCKS_LONG_ROWS else SCAN_CHUNK
 
 
 @register_part("mixer", "gated_linear_attention")
@@ -93,8 +108,10 @@ class GatedLinearAttention(Mixer):
         # chunks that run side by side.  In 32-bit the walk stays in one piece, so that a token's sums do not depend on
         # where its request was cut.  (Steps of single tokens never take the chunks: a captured layout keeps its launches.)
         chunks = None
-        if rows.dtype == torch.bfloat16 and ctx.n_tokens > ctx.n_requests and int(ctx.h_q_len.max()) >= SCAN_CHUNK_MIN_ROWS:
-            chunks = ctx.derived(("scan_chunks", SCAN_CHUNK), lambda: ops.scan_chunks(ctx.h_q_start, ctx.h_q_len, SCAN_CHUNK, ctx.device))
+        if rows.dtype == torch.bfloat16 and ctx.n_tokens > ctx.n_requests:
+            chunk = chunk_rows(int(ctx.h_q_len.max()), ctx.n_tokens, ctx.n_requests, ops.gla_takes_blocks(self.head_dim, self.v_head_dim))
+            if chunk:
+                chunks = ctx.derived(("scan_chunks", chunk), lambda: ops.scan_chunks(ctx.h_q_start, ctx.h_q_len, chunk, ctx.device))
         y = ops.gla_scan(rows, (0, HD, 2 * HD, 2 * HD + HV), z, self.a2_bias, self.tau, self.head_dim ** -0.5, self.norm_w,
                          self.norm_eps, self.n_heads, self.head_dim, self.v_head_dim, state, 0, ctx.q_start, ctx.q_len,
                          ctx.state_slots, chunks)

@@ -309,6 +309,34 @@ def test_gated_linear_attention_in_chunks_side_by_side(dtype, H, d, dv, tau, chu
     assert warm.cpu().abs().max() > 0 and not torch.equal(states[0], warm.cpu())
 
 
+@pytest.mark.parametrize("H,d,chunk,decay", [(2, 64, 32, 0.0), (3, 36, 64, 0.0), (1, 60, 7, -3.0), (2, 64, 48, -30.0), (2, 64, 64, -400.0), (1, 64, 16, -1e30)])
+def test_chunks_on_the_matrix_cores(H, d, chunk, decay):
+    """Heads of up to 64 x 128 in chunks by blocks of 16 tokens, blocks full and not, against the recurrence in 64 bits: outputs to a rounding of
+    bfloat16 (2^-9 of them) and what their 128 values' norm carries over of the sums' errors, the state to 16 roundings of float and the
+    decays' exponents (at most 16 of 2^-24).  Decays whose exponents would leave float's range, on some channels and tokens."""
+    eps, tau, dv = 1e-6, 1.0, 128
+    lens = [150, 1, 33, 16, 63]
+    rows, cols, z, bias, w = _gla_inputs(75, sum(lens), H, d, dv, torch.bfloat16, extra=0)
+    g = torch.Generator().manual_seed(76)
+    z = torch.where(torch.rand(z.shape, generator=g) < 0.02, z + decay, z + 2.0)
+    q_start, q_len = _step_arrays(lens)
+    slots = torch.tensor([2, 0, 4, 1, 3], dtype=torch.int32)
+    state = torch.zeros((5, ops.gla_state_floats(H, d, dv)), dtype=torch.float32, device=DEV)
+    out = ops.gla_scan(rows.to(DEV), cols, z.to(DEV), bias.to(DEV), tau, d ** -0.5, w.to(DEV), eps, H, d, dv, state, 0, q_start.to(DEV), q_len.to(DEV),
+                       slots.to(DEV), ops.scan_chunks(q_start.numpy(), q_len.numpy(), chunk, DEV)).cpu()
+    at = 0
+    for r, n in enumerate(lens):
+        want, S = _gla_plain(rows[at:at + n], cols, z[at:at + n], bias, w, H, d, dv, tau, eps)
+        got = out[at:at + n].double()
+        assert torch.isfinite(got).all()
+        assert ((got - T64(want)).abs() <= 2.0 ** -8 * T64(want).abs() + 1e-4).all(), r
+        mine = state[slots[r]].cpu().double().reshape(H, dv, 64)
+        assert not mine[:, :, d:].any()
+        S = T64(S).reshape(H, d, dv).transpose(1, 2)
+        assert (mine[:, :, :d] - S).abs().max() < 64 * 2.0 ** -24 * max(1.0, float(S.abs().max())) * 4, r
+        at += n
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("chunk", [0, 5, 64])
 @pytest.mark.parametrize("H,d,left,dv", [(2, 16, 2, 24), (3, 32, 2, 16), (2, 64, 4, 128), (1, 64, 14, 6), (2, 128, 4, 192)])
