@@ -257,17 +257,22 @@ __global__ __launch_bounds__(256, 1) void experts_waves_kernel(ExpertsArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[O::LDS];
   static_assert(O::LDS <= 160 * 1024 && FN % 4 == 0, "LDS");
   const int nt = (a.NW + P::BN - 1) / P::BN, mt = a.n_tiles[1], total = nt * mt;
-  if (MODE == MODE_DOWN)          // identity experts' tiles
-    for (int tm = mt + blockIdx.x; tm < a.n_tiles[0]; tm += gridDim.x) {
-      const int* items = a.sorted + a.tile_start[tm];
-      const int count = a.tile_count[tm];
-      for (int i = 0; i < count; ++i) {
-        const int m = items[i], t = m / a.top;
-        const float w = a.weights[m];
-        float* out = (float*)a.out + ((size_t)(m - t * a.top) * a.T + t) * a.NW;
-        for (int n = threadIdx.x; n < a.NW; n += P::THREADS) out[n] = w * (float)a.identity[(size_t)t * a.NW + n];
+  if (MODE == MODE_DOWN) {          // identity experts' items, a wave to an item (NW is the rows' width then, a multiple of 8)
+    const int places = (a.n_tiles[0] - mt) * WAVE_ITEMS;
+    for (int p = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + threadIdx.x / 64); p < places; p += gridDim.x * 4) {
+      const int tm = mt + p / WAVE_ITEMS, i = p % WAVE_ITEMS;
+      if (i >= a.tile_count[tm]) continue;
+      const int m = a.sorted[a.tile_start[tm] + i], t = m / a.top;
+      const float w = a.weights[m];
+      const bf16_t* x = a.identity + (size_t)t * a.NW;
+      float* out = (float*)a.out + ((size_t)(m - t * a.top) * a.T + t) * a.NW;
+      for (int n = threadIdx.x % 64 * 8; n < a.NW; n += 512) {
+        const bf16x8 v = *(const bf16x8*)(x + n);
+        *(floatx4*)(out + n) = floatx4{w * (float)v[0], w * (float)v[1], w * (float)v[2], w * (float)v[3]};
+        *(floatx4*)(out + n + 4) = floatx4{w * (float)v[4], w * (float)v[5], w * (float)v[6], w * (float)v[7]};
       }
     }
+  }
   const int per = (total + 7) / 8, end = min(total, (int)(blockIdx.x % 8 + 1) * per), stride = gridDim.x / 8;
   int id = blockIdx.x % 8 * per + blockIdx.x / 8;
   if (id >= end) return;
