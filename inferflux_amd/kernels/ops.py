@@ -1680,7 +1680,8 @@ def _small_m_kernel(M: int, N: int, K: int, has_tiled: bool = False) -> Optional
     rows on narrow weights); from 65 to 128 rows the same product for weights of few rows, whose K it cuts into
     slices to fill the chip where the library has too few output tiles to (down, o and q/k/v of the 7B shape:
     37-50, 15-21 and 16-22 us against 58-66, 30-34 and 30-37); beyond that, and for tall weights such as gate/up
-    and the head, the library's tiles reuse the rows better."""
+    and the head, the library's tiles reuse the rows better.  (A model's weights go to small tiles first from 65 rows on where those
+    are faster than either: ``few_tiles_plan``, ``few_pairs_take``.)"""
     if K % 8:
         return None
     if M <= 16:
