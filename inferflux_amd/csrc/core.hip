@@ -402,7 +402,7 @@ extern "C" int ifx_rope_table(const int* positions, const float* inv_freq, float
 // cos/sin come from the step's table [T, rotary_dim / 2]; elements at or beyond rotary_dim are
 // copied.  One block per (token, head): q heads, then k heads, then v heads.
 struct RopeArgs {
-  const void* qkv;       // [T, row width] of the activation type, or with n_slices > 1 float partial sums
+  const void* qkv;       // [T, row width] of the activation type (n_slices 0), or float partial sums
   int n_slices;          // [n_slices][T, row width], slice_stride elements apart, added in order
   size_t slice_stride;
   const void* bias;
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(64) void rope_append_kernel(RopeArgs a) {
   // Elements i0 and i1 of the row; partial sums are added in slice order, eight slices of both elements asked for
   // together (one after the other every slice would cost a trip to the L2).
   auto in2 = [&](int i0, int i1, float& x0, float& x1) {
-    if (a.n_slices <= 1) { x0 = to_f(row[i0]); x1 = to_f(row[i1]); return; }
+    if (a.n_slices == 0) { x0 = to_f(row[i0]); x1 = to_f(row[i1]); return; }
     for (int s0 = 0; s0 < a.n_slices; s0 += 8) {
       float p0[8], p1[8];
 #pragma unroll
@@ -765,7 +765,7 @@ __global__ __launch_bounds__(256) void rope_append_vec_x_kernel(RopeArgs a, int 
   }
 }
 
-// dtype: the type of q_out and the cache, and of qkv unless n_slices > 1 (then qkv holds float partial sums,
+// dtype: the type of q_out and the cache, and of qkv unless n_slices > 0 (then qkv holds so many float partial sums,
 // slice_stride elements apart).
 extern "C" int ifx_rope_append(const void* qkv, int dtype, const void* bias, int bias_dtype, const int* slots,
                                const float* cs, const float* sn, int rope_style, int rotary_dim, int T, int nH,
@@ -774,7 +774,7 @@ extern "C" int ifx_rope_append(const void* qkv, int dtype, const void* bias, int
                                const void* v_first, float v_mix, void* v_out, const void* q_norm_w, const void* k_norm_w,
                                int pre_norm_dtype, float pre_norm_eps, int extra_cols, const float* q_mult, void* stream) {
   IFX_REQUIRE((q_norm_w != nullptr) == (k_norm_w != nullptr) && extra_cols >= 0, "rope_append: norms for q and k come together");
-  IFX_REQUIRE(n_slices >= 1 && (n_slices == 1 || slice_stride > 0), "rope_append: %d slices, %lld apart", n_slices, slice_stride);
+  IFX_REQUIRE(n_slices >= 0 && (n_slices <= 1 || slice_stride > 0), "rope_append: %d slices, %lld apart", n_slices, slice_stride);
   IFX_REQUIRE(T >= 0 && nH > 0 && nKV >= 0 && d > 0 && d % 2 == 0 && dv > 0, "rope_append: bad sizes T=%d nH=%d nKV=%d d=%d dv=%d", T, nH, nKV, d, dv);
   IFX_REQUIRE(rope_style >= 0 && rope_style <= 2, "rope_append: unknown rope style %d", rope_style);
   IFX_REQUIRE(rope_style == 0 || (rotary_dim > 0 && rotary_dim <= d && rotary_dim % 2 == 0 && cs && sn),
@@ -790,7 +790,7 @@ extern "C" int ifx_rope_append(const void* qkv, int dtype, const void* bias, int
   const bool extras = gate_cols || unit_norm || v_first || v_out || q_norm_w || extra_cols || q_mult;
   hipStream_t s = (hipStream_t)stream;
   // (a few tokens are quicker with one small block per token and head: nothing waits on a loop over tokens)
-  if (!extras && dv == d && T >= 128 && n_slices == 1 && dtype == DT_BF16 && rope_style == 1 && rotary_dim == d && d % 16 == 0 && (!bias || bias_dtype == DT_BF16) &&
+  if (!extras && dv == d && T >= 128 && n_slices == 0 && dtype == DT_BF16 && rope_style == 1 && rotary_dim == d && d % 16 == 0 && (!bias || bias_dtype == DT_BF16) &&
       (!slots || page_size % 8 == 0)) {
     const size_t qk_threads = (size_t)T * (nH + (slots ? nKV : 0)) * (d / 16);
     const size_t v_threads = slots ? (size_t)((T + 7) / 8) * nKV * d : 0;
@@ -799,7 +799,7 @@ extern "C" int ifx_rope_append(const void* qkv, int dtype, const void* bias, int
     IFX_LAUNCH_CHECK();
   }
   const int rot = rope_style != 0 ? rotary_dim : 0;
-  if (extras && T >= 128 && n_slices == 1 && dtype == DT_BF16 && rope_style <= 1 && (d == 16 || d == 32 || d == 64 || d == 128) &&
+  if (extras && T >= 128 && n_slices == 0 && dtype == DT_BF16 && rope_style <= 1 && (d == 16 || d == 32 || d == 64 || d == 128) &&
       rot % 16 == 0 && (nH * d + nKV * (d + dv) + gate_cols + extra_cols) % 8 == 0 && (!bias || bias_dtype == DT_BF16) &&
       (!q_norm_w || pre_norm_dtype == DT_BF16) &&
       (!slots || page_size % 8 == 0) && (slots || (!v_first && !v_out))) {

@@ -84,7 +84,7 @@ extern "C" int ifx_activation_slices(const float* parts, int n_slices, long long
   IFX_LAUNCH_CHECK();
 }
 
-// x [T, C] of type T; g: columns g_col .. g_col + C - 1 of rows ld apart, of type T, or (n_slices > 1) float partial sums
+// x [T, C] of type T; g: columns g_col .. g_col + C - 1 of rows ld apart, of type T (n_slices 0), or so many float partial sums
 template <typename T>
 __global__ __launch_bounds__(256) void sigmoid_gate_kernel(const T* __restrict__ x, const void* __restrict__ g, int ld, int g_col,
                                                            int n_slices, size_t slice_stride, T* __restrict__ out, int C, size_t n) {
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void sigmoid_gate_kernel(const T* __restrict__
   const size_t t = i / C;
   const int c = (int)(i % C);
   float gv;
-  if (n_slices > 1) {
+  if (n_slices > 0) {
     const float* p = (const float*)g + t * ld + g_col + c;
     gv = p[0];
     for (int k = 1; k < n_slices; ++k) gv += p[(size_t)k * slice_stride];
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void sigmoid_gate_kernel(const T* __restrict__
 
 extern "C" int ifx_sigmoid_gate(const void* x, const void* g, int ld, int g_col, int n_slices, long long slice_stride, void* out,
                                 int dtype, int T, int C, void* stream) {
-  IFX_REQUIRE(T >= 0 && C > 0 && ld >= g_col + C && g_col >= 0 && n_slices >= 1, "sigmoid_gate: T=%d C=%d ld=%d g_col=%d", T, C, ld, g_col);
+  IFX_REQUIRE(T >= 0 && C > 0 && ld >= g_col + C && g_col >= 0 && n_slices >= 0, "sigmoid_gate: T=%d C=%d ld=%d g_col=%d", T, C, ld, g_col);
   if (T == 0) return 0;
   const size_t n = (size_t)T * C;
   hipStream_t s = (hipStream_t)stream;

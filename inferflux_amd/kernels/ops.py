@@ -352,10 +352,10 @@ def rope_append(qkv: torch.Tensor, bias: Optional[torch.Tensor], slots: Optional
     dv = head_dim if v_head_dim is None else int(v_head_dim)
     gate_cols = n_heads if gate_out is not None else 0
     width = (n_heads + n_kv_heads) * head_dim + n_kv_heads * dv + gate_cols + int(extra_cols)
-    n_slices = 1
+    n_slices = stride = 0
     if isinstance(qkv, SliceSums):                  # partial sums: the kernel adds them in slice order
         _check(qkv.parts, "qkv", (None, T, width), torch.float32)
-        n_slices, dtype, qkv = qkv.parts.shape[0], qkv.dtype, qkv.parts
+        n_slices, stride, dtype, qkv = qkv.parts.shape[0], T * width, qkv.dtype, qkv.parts
     else:
         _check(qkv, "qkv", (T, width))
         dtype = qkv.dtype
@@ -388,7 +388,7 @@ def rope_append(qkv: torch.Tensor, bias: Optional[torch.Tensor], slots: Optional
           qkv, _DT[dtype], bias, _dt(bias) if bias is not None else 0, slots,
           cos if rope_style != ROPE_NONE else None, sin if rope_style != ROPE_NONE else None, rope_style,
           rotary_dim, T, n_heads, n_kv_heads, head_dim, page_size, q, k_cache, v_cache,
-          n_slices, T * width, dv, gate_cols, gate_out, 1 if unit_norm_eps is not None else 0,
+          n_slices, stride, dv, gate_cols, gate_out, 1 if unit_norm_eps is not None else 0,
           float(unit_norm_eps or 0.0), v_first, float(v_mix), v_out, qn, kn,
           _dt(qn) if qn is not None else 0, float(pre_eps) if qn is not None else 0.0, int(extra_cols), q_mult, _stream())
     return q
@@ -1529,7 +1529,7 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
     if prepared and M > SKINNY_MAX_M and (keep_slices or kind is None) and out_dtype == torch.bfloat16 and not torch.cuda.tunable.is_enabled():
         plan = few_tiles_plan(M, weight.shape[0], K, bool(keep_slices))
         if plan and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and weight.is_contiguous():
-            return _by_plan(x, weight, plan)
+            return _by_plan(x, weight, plan, keep_slices)
     if kind == "skinny":
         ring = ring_takes_few(x, LinearWeight(weight, tiled, order, tile_rows), keep_slices and out_dtype == torch.bfloat16)
         if ring:
@@ -1557,9 +1557,13 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
     return torch.matmul(x, weight.t())
 
 
-def _by_plan(x: torch.Tensor, weight: torch.Tensor, plan: int):
+def _by_plan(x: torch.Tensor, weight: torch.Tensor, plan: int, whole_in_float: bool = False):
+    """The product that ``plan`` names; ``whole_in_float``: one slice stays a float sum, too, as the slices of the products that it is taken
+    instead of are."""
     slices, tile, K = plan >> 8, plan & 255, x.shape[1]
-    return sums_tiles(x, weight, slices, -(-(-(-K // slices)) // 64) * 64, tile) if slices > 1 else act_tiles(x, weight, ACT_NONE, tile)
+    if slices > 1 or whole_in_float:
+        return sums_tiles(x, weight, slices, -(-(-(-K // slices)) // 64) * 64, tile)
+    return act_tiles(x, weight, ACT_NONE, tile)
 
 
 FEW_MAX_ROWS = 2048              # rows, weight rows and k-values that ``few_tiles_plan`` was measured for
@@ -2591,7 +2595,7 @@ def sigmoid_gate(x: torch.Tensor, rows, g_col: int) -> torch.Tensor:
     element by element, the sigmoid in float."""
     _check(x, "x", (None, None))
     T, C = x.shape
-    n_slices, stride = 1, 0
+    n_slices = stride = 0
     if isinstance(rows, SliceSums):
         _check(rows.parts, "rows", (None, T, None), torch.float32)
         n_slices, ld, stride, ptr = rows.parts.shape[0], rows.parts.shape[2], T * rows.parts.shape[2], rows.parts.data_ptr()
