@@ -337,6 +337,24 @@ def test_chunks_on_the_matrix_cores(H, d, chunk, decay):
         at += n
 
 
+@pytest.mark.parametrize("chunk", [32, 64])
+@pytest.mark.parametrize("tau,logit,spread,drift", [(1.0, 8.0, 0.0, 0.5), (1.0, 20.0, 0.0, 0.5), (1.0, 8.0, 0.3, 0.0), (1.0, 2.0, 1.0, 0.0), (16.0, 10.0, 1.0, 0.0), (16.0, 0.0, 1.0, 0.0)])
+def test_slow_decays_on_the_matrix_cores_keep_their_digits(chunk, tau, logit, spread, drift):
+    """The state that a long request leaves in chunks, where every decay is close to 1 and its logarithm is all that says how close: against the recurrence in
+    64 bits, in the mean square within what the 2 x 125 roundings of S (0.4 of 2^-24 each) and a few of its decays' exponents leave, 12 of 2^-24."""
+    H, d, dv, T, eps = 1, 64, 128, 2000, 1e-6
+    rows, cols, _, bias, w = _gla_inputs(77, T, H, d, dv, torch.bfloat16, extra=0)
+    g = torch.Generator().manual_seed(78)
+    z = logit + spread * torch.randn(T, H * d, generator=g) + drift * torch.rand(1, H * d, generator=g)        # (a channel's own, where it does not vary)
+    q_start, q_len = _step_arrays([T])
+    state = torch.zeros((1, ops.gla_state_floats(H, d, dv)), dtype=torch.float32, device=DEV)
+    ops.gla_scan(rows.to(DEV), cols, z.to(DEV), None, tau, d ** -0.5, w.to(DEV), eps, H, d, dv, state, 0, q_start.to(DEV), q_len.to(DEV),
+                 torch.zeros(1, dtype=torch.int32, device=DEV), ops.scan_chunks(q_start.numpy(), q_len.numpy(), chunk, DEV))
+    _, S = _gla_plain(rows, cols, z, torch.zeros_like(bias), w, H, d, dv, tau, eps)
+    S = T64(S).reshape(H, d, dv).transpose(1, 2)
+    assert (state.cpu().double().reshape(H, dv, 64) - S).norm() < 12 * 2.0 ** -24 * S.norm()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("chunk", [0, 5, 64])
 @pytest.mark.parametrize("H,d,left,dv", [(2, 16, 2, 24), (3, 32, 2, 16), (2, 64, 4, 128), (1, 64, 14, 6), (2, 128, 4, 192)])
