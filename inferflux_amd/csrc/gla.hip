@@ -288,7 +288,8 @@ __global__ __launch_bounds__(256) void gla_combine_kernel(CombineArgs a) {
 //   S  <- exp(B_15) S + sum_s (k_s exp(B_15 - B_s)) v_s^T
 // A workgroup is one head of a chunk; a wave owns 32 columns of S in the instruction's output layout, whose registers are at the same time
 // the operand that the read-out wants (with its channels in another order), so S never leaves them.  A block whose decays are strong
-// (B_15 below -8 in some channel: exp(B_7 - B_s) would lose digits, and overflow) is walked token by token as the kernel above does.
+// (B_15 below -8 in some channel: exp(B_7 - B_s) would lose digits, and overflow), or that has a value that is not finite (which a weight of zero would hand
+// to the tokens before it), is walked token by token as the kernel above does.
 // What bounds it is the matrix instruction (88 of 32 cycles a wave and block in MODE 2), the exponentials beside it and the block's four meeting
 // points.  Both walks and what joins the chunks, 16 heads of 64 x 128, by the kernel above / here: 4,026 rows of 16 requests 268 / 113 us, 8,192 of
 // four 450 / 167, a request of 200 71 / 25.  (With expf() and log1pf() 217 of the 113 us.)  The state against 64 bits, tau 16, decays' logits of
@@ -397,27 +398,31 @@ __global__ __launch_bounds__(256, 2) void gla_blocks_kernel(GlaArgs a) {
       *(gla_f4*)&lq[lt][lc] = x;
       gate[0] = ng[0], gate[1] = ng[1];
     }
+    float odd = 0.f;              // NaN where a value is not finite
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = row ? (float)nv[4 * h + e] : 0.f;
+      for (int e = 0; e < 4; ++e) {
+        x[e] = row ? (float)nv[4 * h + e] : 0.f;
+        odd = fmaf(x[e], 0.f, odd);
+      }
       *(gla_f4*)&lv[lt][2 * lc + 4 * h] = x;
     }
     if (s0 + BLOCK < n) fetch(s0 + BLOCK);
     __syncthreads();
     const gla_f4 mine = *(const gla_f4*)&la[i16][ch];
     gla_f4 upto, whole, half;
-    bool strong = false;
+    bool walk = !(odd == 0.f);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       upto[e] = sum_up_to(mine[e]);
       whole[e] = __shfl(upto[e], lane | 15, WAVE);
       half[e] = __shfl(upto[e], (lane & 48) + 7, WAVE);
-      strong = strong || !(whole[e] > BLOCK_MIN_DECAY);
+      walk = walk || !(whole[e] > BLOCK_MIN_DECAY);
       loga[e] += whole[e];
     }
     gla_f4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    if (__syncthreads_or(strong)) {
+    if (__syncthreads_or(walk)) {
       const int ns = min(BLOCK, n - s0);
 #pragma unroll 1
       for (int tt = 0; tt < ns; ++tt) {
@@ -426,6 +431,7 @@ __global__ __launch_bounds__(256, 2) void gla_blocks_kernel(GlaArgs a) {
         for (int jb = 0; jb < 2; ++jb) v[jb] = lv[tt][32 * wid + 16 * jb + i16];
 #pragma unroll
         for (int ib = 0; ib < 4; ++ib) {
+          if (16 * ib + 4 * g >= d) continue;          // (no channels: zero by a value that is not finite would be none)
           const gla_f4 l = *(const gla_f4*)&la[tt][16 * ib + 4 * g], k = *(const gla_f4*)&lk[tt][16 * ib + 4 * g];
           const gla_f4 q = MODE == 2 ? *(const gla_f4*)&lq[tt][16 * ib + 4 * g] : gla_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -355,6 +355,27 @@ def test_slow_decays_on_the_matrix_cores_keep_their_digits(chunk, tau, logit, sp
     assert (state.cpu().double().reshape(H, dv, 64) - S).norm() < 12 * 2.0 ** -24 * S.norm()
 
 
+@pytest.mark.parametrize("odd", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("d,chunk,at", [(64, 64, 37), (36, 32, 15), (60, 48, 48), (64, 32, 0)])
+def test_values_that_are_not_finite_reach_no_earlier_token_in_chunks(d, chunk, at, odd):
+    """One value of one head in one of two requests: what came before it, the other head and the other request have the recurrence's outputs (to the
+    tolerance of test_chunks_on_the_matrix_cores), and the tokens from it on are finite where those of the walk in one piece are."""
+    H, dv, lens, eps, tau = 2, 128, [100, 70], 1e-6, 4.0
+    rows, cols, z, bias, w = _gla_inputs(79, sum(lens), H, d, dv, torch.bfloat16, extra=0)
+    q_start, q_len = _step_arrays(lens)
+    want = torch.cat([T64(_gla_plain(rows[a:a + n], cols, z[a:a + n], bias, w, H, d, dv, tau, eps)[0]) for a, n in ((0, 100), (100, 70))])
+    rows[at, cols[2] + dv + 77] = odd
+    outs = []
+    for chunks in (None, ops.scan_chunks(q_start.numpy(), q_len.numpy(), chunk, DEV)):
+        state = torch.zeros((2, ops.gla_state_floats(H, d, dv)), dtype=torch.float32, device=DEV)
+        outs.append(ops.gla_scan(rows.to(DEV), cols, z.to(DEV), bias.to(DEV), tau, d ** -0.5, w.to(DEV), eps, H, d, dv, state, 0, q_start.to(DEV), q_len.to(DEV),
+                                 torch.arange(2, dtype=torch.int32, device=DEV), chunks).cpu().double())
+    sound = torch.ones(sum(lens), H * dv, dtype=torch.bool)
+    sound[at:100, dv:] = False
+    assert ((outs[1] - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4)[sound].all()
+    assert torch.equal(torch.isfinite(outs[1]), torch.isfinite(outs[0])) and not torch.isfinite(outs[1]).all()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("chunk", [0, 5, 64])
 @pytest.mark.parametrize("H,d,left,dv", [(2, 16, 2, 24), (3, 32, 2, 16), (2, 64, 4, 128), (1, 64, 14, 6), (2, 128, 4, 192)])
