@@ -2152,11 +2152,12 @@ def gla_layout(d: int, dv: int) -> Tuple[int, int]:
     raise KernelError(f"gla: a head of {d} key channels and {dv} values does not fit a workgroup")
 
 
-def gla_takes_blocks(d: int, dv: int) -> bool:
-    """Whether ``gla_scan`` runs chunks of bfloat16 rows on the matrix cores for heads of d key channels and dv values (rows and decays on 16
-    bytes, as ``linear`` leaves them)."""
+def gla_takes_blocks(rows: torch.Tensor, cols: Tuple[int, int, int, int], z: torch.Tensor, z_bias: Optional[torch.Tensor], d: int, dv: int) -> bool:
+    """Whether ``gla_scan`` runs these rows' chunks on the matrix cores: bfloat16, heads of the layout for 64 key channels and 128 values, everything it reads on
+    16 bytes (the rule of blocks_take in csrc/gla.hip)."""
     dp, parts = gla_layout(d, dv)
-    return dp * parts == 64 and d % 4 == 0 and dv == 128
+    return (rows.dtype == torch.bfloat16 and dp * parts == 64 and d % 4 == 0 and dv == 128 and rows.shape[1] % 8 == 0
+            and all((rows.data_ptr() + 2 * c) % 16 == 0 for c in cols) and z.data_ptr() % 16 == 0 and (z_bias is None or z_bias.data_ptr() % 16 == 0))
 
 
 def gla_state_floats(n_heads: int, d: int, dv: int) -> int:

@@ -98,6 +98,7 @@ class GatedLinearAttention(Mixer):
             raise ValueError(f"{self.name}: the mixer was given no per-request state")
         HD, HV, r = self.n_heads * self.head_dim, self.n_heads * self.v_head_dim, self.decay_rank
         rows = ops.linear(h, self.w_in)                                 # [T, q | k | v | g | a1]
+        cols = (0, HD, 2 * HD, 2 * HD + HV)
         a1 = rows[:, 2 * HD + 2 * HV:] if rows.shape[0] else rows.new_empty((0, r))
         if not ops.columns_on_16_bytes(a1):
             a1 = a1.contiguous()              # (``linear`` takes columns in bfloat16 on 16 bytes)
@@ -109,10 +110,11 @@ class GatedLinearAttention(Mixer):
         # where its request was cut.  (Steps of single tokens never take the chunks: a captured layout keeps its launches.)
         chunks = None
         if rows.dtype == torch.bfloat16 and ctx.n_tokens > ctx.n_requests:
-            chunk = chunk_rows(int(ctx.h_q_len.max()), ctx.n_tokens, ctx.n_requests, ops.gla_takes_blocks(self.head_dim, self.v_head_dim))
+            chunk = chunk_rows(int(ctx.h_q_len.max()), ctx.n_tokens, ctx.n_requests,
+                               ops.gla_takes_blocks(rows, cols, z, self.a2_bias, self.head_dim, self.v_head_dim))
             if chunk:
                 chunks = ctx.derived(("scan_chunks", chunk), lambda: ops.scan_chunks(ctx.h_q_start, ctx.h_q_len, chunk, ctx.device))
-        y = ops.gla_scan(rows, (0, HD, 2 * HD, 2 * HD + HV), z, self.a2_bias, self.tau, self.head_dim ** -0.5, self.norm_w,
+        y = ops.gla_scan(rows, cols, z, self.a2_bias, self.tau, self.head_dim ** -0.5, self.norm_w,
                          self.norm_eps, self.n_heads, self.head_dim, self.v_head_dim, state, 0, ctx.q_start, ctx.q_len,
                          ctx.state_slots, chunks)
         if t is not None:

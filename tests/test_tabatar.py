@@ -295,3 +295,26 @@ def test_random_weights_folder_roundtrips(tmp_path):
     assert float(t["l0.mix.a2.b"].float().min()) >= 0.0 and t["l0.hc1.mix"].shape == (5, 5)
     logits = pt.forward(tm.config("D"), {k: v.double().numpy() for k, v in t.items()}, [1, 2, 3, 4])
     assert np.isfinite(logits).all() and np.abs(logits).max() <= 8.0
+
+
+def test_linear_attention_is_cut_into_chunks_where_they_pay():
+    """Both sides of every line: heads whose chunks run on the matrix cores, and others."""
+    from inferflux_amd.parts.gla import chunk_rows
+    assert [chunk_rows(n, n, 1, False) for n in (127, 128, 5000)] == [0, 32, 32]
+    assert [chunk_rows(n, 200, 8, True) for n in (23, 24)] == [0, 32] and [chunk_rows(n, 200, 9, True) for n in (24, 47, 48)] == [0, 0, 32]
+    assert [chunk_rows(100, rows, 20, True) for rows in (2047, 2048)] == [32, 64]
+
+
+@pytest.mark.parametrize("H,d,dv,rank,takes", [(2, 64, 128, 16, True), (2, 36, 128, 16, True), (2, 64, 128, 4, False), (1, 60, 128, 16, False), (2, 60, 128, 16, True),
+                                               (3, 44, 128, 16, False), (2, 32, 128, 16, False), (2, 62, 128, 16, False), (2, 64, 96, 16, False)])
+def test_chunks_on_the_matrix_cores_are_promised_only_where_they_run(H, d, dv, rank, takes):
+    """Rows as the projection leaves them, q | k | v | g | a1: what the kernel reads in pieces of 16 bytes must lie on 16 (a head of 128 values and 33 to 64 channels)."""
+    import torch
+
+    from inferflux_amd.kernels import ops
+    HD, HV = H * d, H * dv
+    rows, z, bias = torch.zeros(40, 2 * HD + 2 * HV + rank, dtype=torch.bfloat16), torch.zeros(40, HD), torch.zeros(HD + 4)
+    cols = (0, HD, 2 * HD, 2 * HD + HV)
+    assert ops.gla_takes_blocks(rows, cols, z, bias[:HD], d, dv) == takes and ops.gla_takes_blocks(rows, cols, z, None, d, dv) == takes
+    assert not ops.gla_takes_blocks(rows, cols, z, bias[1:HD + 1], d, dv)
+    assert not ops.gla_takes_blocks(rows.float(), cols, z, None, d, dv)
