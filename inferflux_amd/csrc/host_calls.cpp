@@ -11,7 +11,7 @@
 //   call(module, function, types, *arguments)        the library's function with these arguments, as ctypes would call it; an error code is
 //                                                    handed to the Python side; whatever is not plain (other types, other objects) is
 //                                                    left to ctypes
-//   connect(check, call, failed, entry)              the Python functions for all that
+//   connect(check, call, failed, entry, array)       the Python functions for all that, and the type of ctypes' arrays
 //
 // The call: by the C calling convention of x86-64 the first six whole numbers and pointers of a call are in registers, the first eight
 // floating-point ones in others, and all further whole numbers on the stack in order, whatever stands between them.  So one function type
@@ -25,6 +25,7 @@
 
 #include <cstring>
 #include <string>
+#include <vector>
 
 #if !defined(__x86_64__)
 #error "host_calls.cpp knows the calling convention of x86-64 only"
@@ -36,7 +37,11 @@ constexpr int REGISTERS = 6, FLOATS = 8, STACK = 32;
 
 struct Entry {
   void* function;
-  std::string types;        // p: pointer (a tensor's address, a number, None), a: pointer to an object's buffer, i: 32 bits, l: 64 bits, f: float
+  std::string types;        // p: pointer (a tensor's address, a number, None), a: a ctypes array's address, i: 32 bits, l: 64 bits, f: float
+  std::vector<PyObject*> elements;        // of the arrays, in order
+  ~Entry() {
+    for (PyObject* e : elements) Py_DECREF(e);
+  }
 };
 
 struct WithoutGil {
@@ -44,7 +49,8 @@ struct WithoutGil {
   ~WithoutGil() { PyEval_RestoreThread(state); }
 };
 
-PyObject *slow_check = nullptr, *slow_call = nullptr, *call_failed = nullptr, *make_entry = nullptr, *entries_name = nullptr;
+PyObject *slow_check = nullptr, *slow_call = nullptr, *call_failed = nullptr, *make_entry = nullptr, *array_type = nullptr, *entries_name = nullptr,
+         *type_name = nullptr;
 
 bool as_expected(PyObject* const* a, Py_ssize_t n) {
   if (!THPVariable_Check(a[0])) return false;
@@ -109,26 +115,39 @@ PyObject* stream(PyObject*, PyObject*) {
 
 void free_entry(PyObject* capsule) { delete static_cast<Entry*>(PyCapsule_GetPointer(capsule, "entry")); }
 
-// entry(address, types): what ``call`` keeps of a function, or None where the types do not fit the one call there is
+// entry(address, types, elements): what ``call`` keeps of a function, or None where the types do not fit the one call there is
 PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  const char* types = n == 2 ? PyUnicode_AsUTF8(a[1]) : nullptr;
+  const char* types = n == 3 && PyTuple_Check(a[2]) ? PyUnicode_AsUTF8(a[1]) : nullptr;
   if (!types) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "entry(address, types)");
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "entry(address, types, elements: tuple)");
     return nullptr;
   }
-  int floats = 0, others = 0;
+  int floats = 0, others = 0, arrays = 0;
   for (const char* c = types; *c; ++c) {
     if (*c == 'f') ++floats;
     else if (*c == 'p' || *c == 'a' || *c == 'i' || *c == 'l') ++others;
     else Py_RETURN_NONE;
+    arrays += *c == 'a';
   }
   if (floats > FLOATS || others > REGISTERS + STACK) Py_RETURN_NONE;
+  if (arrays != PyTuple_GET_SIZE(a[2])) {
+    PyErr_SetString(PyExc_TypeError, "entry: an element type for every array");
+    return nullptr;
+  }
   void* function = PyLong_AsVoidPtr(a[0]);
   if (!function) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "entry: no address");
     return nullptr;
   }
-  return PyCapsule_New(new Entry{function, types}, "entry", free_entry);
+  Entry* made = new Entry{function, types, {}};
+  for (int i = 0; i < arrays; ++i) {
+    PyObject* e = PyTuple_GET_ITEM(a[2], i);
+    Py_INCREF(e);
+    made->elements.push_back(e);
+  }
+  PyObject* capsule = PyCapsule_New(made, "entry", free_entry);
+  if (!capsule) delete made;
+  return capsule;
 }
 
 typedef uint64_t W;
@@ -144,8 +163,21 @@ struct Buffers {
   }
 };
 
+// Whether v is a ctypes array of these elements, as a pointer to them takes it: other objects with a buffer, a ctypes pointer among them, hold something else there.
+bool is_array_of(PyObject* v, PyObject* element) {
+  if (!PyType_IsSubtype(Py_TYPE(v), reinterpret_cast<PyTypeObject*>(array_type))) return false;
+  PyObject* of = PyObject_GetAttr(reinterpret_cast<PyObject*>(Py_TYPE(v)), type_name);
+  if (!of) {
+    PyErr_Clear();
+    return false;
+  }
+  Py_DECREF(of);        // (its type keeps it)
+  return of == element;
+}
+
 // The arguments as words; false: one is not plain
-bool words(const std::string& types, PyObject* const* a, W* whole, double* floats, Buffers& buffers) {
+bool words(const Entry& entry, PyObject* const* a, W* whole, double* floats, Buffers& buffers) {
+  const std::string& types = entry.types;
   int w = 0, f = 0;
   for (size_t i = 0; i < types.size(); ++i) {
     PyObject* v = a[i];
@@ -167,6 +199,7 @@ bool words(const std::string& types, PyObject* const* a, W* whole, double* float
       else if (PyLong_CheckExact(v)) whole[w++] = (W)PyLong_AsVoidPtr(v);
       else return false;
     } else if (types[i] == 'a') {
+      if (!is_array_of(v, entry.elements[buffers.n])) return false;
       Py_buffer* view = &buffers.views[buffers.n];
       if (PyObject_GetBuffer(v, view, PyBUF_SIMPLE) != 0) {
         PyErr_Clear();
@@ -207,7 +240,7 @@ PyObject* call_or_throw(PyObject* const* a, Py_ssize_t n) {
     W w[REGISTERS + STACK] = {};
     double d[FLOATS] = {};
     Buffers buffers;
-    if ((size_t)(n - 3) == e->types.size() && words(e->types, a + 3, w, d, buffers)) {
+    if ((size_t)(n - 3) == e->types.size() && words(*e, a + 3, w, d, buffers)) {
       const Function f = reinterpret_cast<Function>(e->function);
       int rc;
       Py_BEGIN_ALLOW_THREADS
@@ -233,12 +266,12 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 PyObject* connect(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 4) {
-    PyErr_SetString(PyExc_TypeError, "connect(check, call, failed, entry)");
+  if (n != 5 || !PyType_Check(a[4])) {
+    PyErr_SetString(PyExc_TypeError, "connect(check, call, failed, entry, array: type)");
     return nullptr;
   }
-  PyObject** to[4] = {&slow_check, &slow_call, &call_failed, &make_entry};
-  for (int i = 0; i < 4; ++i) {
+  PyObject** to[5] = {&slow_check, &slow_call, &call_failed, &make_entry, &array_type};
+  for (int i = 0; i < 5; ++i) {
     Py_INCREF(a[i]);
     Py_XDECREF(*to[i]);
     *to[i] = a[i];
@@ -259,5 +292,6 @@ PyModuleDef definition = {PyModuleDef_HEAD_INIT, "host_calls", nullptr, -1, meth
 
 PyMODINIT_FUNC PyInit_host_calls() {
   entries_name = PyUnicode_InternFromString("entries");
-  return entries_name ? PyModule_Create(&definition) : nullptr;
+  type_name = PyUnicode_InternFromString("_type_");
+  return entries_name && type_name ? PyModule_Create(&definition) : nullptr;
 }

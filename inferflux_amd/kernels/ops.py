@@ -157,12 +157,13 @@ def _entry(mod: KernelModule, fname: str, argtypes):
     """What the native call keeps of a function: its address and argument types, or None where one of them is no plain word."""
     f = mod.fn(fname, argtypes)
     types = "".join(_WORDS.get(t) or ("a" if issubclass(t, ctypes._Pointer) else "?") for t in argtypes)
-    found = mod.entries[fname] = _native.entry(ctypes.cast(f, P).value, types)
+    elements = tuple(t._type_ for t, word in zip(argtypes, types) if word == "a")
+    found = mod.entries[fname] = _native.entry(ctypes.cast(f, P).value, types, elements)
     return found
 
 
 _native = load_extension("host_calls")
-_native.connect(_check_in_python, _call_by_ctypes, _call_failed, _entry)
+_native.connect(_check_in_python, _call_by_ctypes, _call_failed, _entry, ctypes.Array)
 _check, _call, empty, _stream = _native.check, _native.call, _native.empty, _native.stream      # (see csrc/host_calls.cpp)
 
 

@@ -110,17 +110,50 @@ def test_native_calls_leave_the_rest_to_ctypes():
     f = _Function("i" * 39)                              # more than the native call has places for
     ops._call(f, "fake", f.argtypes, *range(39))
     assert f.entries["fake"] is None and f.got == tuple(range(39))
-    f = _Function("if")
-    for wrong in ((1,), (1, 2.0, "three"), ("one", 2.0), (1, "two"), (np.int64(1), None)):
+    for wrong in ((1,), ("one", 2.0), (1, "two"), (np.int64(1), None)):
+        g = _Function("if")
+        g.keep.argtypes = list(g.argtypes)
         with pytest.raises((TypeError, ctypes.ArgumentError)):
-            g = _Function("if")
-            g.keep.argtypes = list(g.argtypes)
             ops._call(g, "fake", g.argtypes, *wrong)
-            assert len(wrong) <= 2 or g.got == (1, 2.0)  # (ctypes takes further arguments)
-            raise TypeError
+        assert g.got is None
+    g = _Function("if")
+    g.keep.argtypes = list(g.argtypes)
+    with pytest.raises((TypeError, ctypes.ArgumentError)):                   # (what comes after is converted by ctypes' own rules, too)
+        ops._call(g, "fake", g.argtypes, 1, 2.0, "three", object())
+    g = _Function("if")
+    ops._call(g, "fake", g.argtypes, 1, 2.0, 3)          # (a C function called with more than it takes, which ctypes allows)
+    assert g.got[:2] == (1, 2.0)
     f = _Function("p", rc=-7)
     with pytest.raises(ops.KernelError, match=r"fake: an error of its own \(code -7\)"):
         ops._call(f, "fake", f.argtypes, None)
+
+
+def test_native_calls_take_a_pointers_array_only_as_ctypes_does():
+    """For a pointer to 32-bit numbers: an array of them by its address, a pointer by what it points to (an object's own buffer would be the pointer
+    itself), None as none, and nothing else."""
+    import ctypes
+
+    import numpy as np
+
+    from inferflux_amd.kernels import ops
+
+    def given(v):
+        f = _Function("ia")
+        f.keep.argtypes = list(f.argtypes)
+        got = []
+        f.keep = ctypes.CFUNCTYPE(ctypes.c_int, ops.I, ctypes.POINTER(ops.I))(lambda i, p: got.append(ctypes.cast(p, ops.P).value) or 0)
+        ops._call(f, "fake", f.argtypes, 1, v)
+        return got[0]
+    ints = (ctypes.c_int * 3)(4, 5, 6)
+    numbers = np.arange(3, dtype=np.int32)
+    assert given(ints) == ctypes.addressof(ints) and given(None) is None
+    first = ctypes.c_int.from_buffer(ints)
+    for pointer in (ctypes.cast(ints, ctypes.POINTER(ctypes.c_int)), ctypes.pointer(first), ctypes.byref(first)):
+        assert given(pointer) == ctypes.addressof(ints)
+    assert given(numbers.ctypes.data_as(ctypes.POINTER(ctypes.c_int))) == numbers.ctypes.data
+    for wrong in (numbers, np.arange(3), b"ab", bytearray(8), (ctypes.c_float * 3)(), (ctypes.c_longlong * 2)(), memoryview(b"abcd")):
+        with pytest.raises(ctypes.ArgumentError):
+            given(wrong)
 
 
 def test_native_checks_raise_what_the_python_check_raises():
