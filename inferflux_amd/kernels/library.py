@@ -9,7 +9,8 @@ is compiled when it is first used, which means a run compiles what its model nee
 more.  Libraries are written next to the sources when that folder is writable (so they travel
 with the tree) and to a per-user folder under the temporary directory otherwise.
 
-There is no fallback: if hipcc is missing or a module does not compile, loading raises.
+There is no fallback: if hipcc is missing or a module does not compile, loading raises.  (Only what a launch does on the host, a Python extension,
+has a slower form in Python: ``ops._host_forms``.)
 """
 from __future__ import annotations
 
@@ -37,13 +38,14 @@ from .device import ARCH
 FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-result"]
 
-HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC"]
-# INFERFLUX_HOST_SANITIZE=1 builds the host-only modules (the cache's bookkeeping) with the address and
+HOST_OPTIONS = ["-O2"]
+# INFERFLUX_HOST_SANITIZE=1 builds the host-only modules (the cache's bookkeeping, the calls of launches) with the address and
 # undefined-behaviour sanitizers, for test runs on the CPU (the process then needs libasan preloaded:
 # LD_PRELOAD=$(g++ -print-file-name=libasan.so)).  Device code is never built with a sanitizer.
 HOST_SANITIZE = os.environ.get("INFERFLUX_HOST_SANITIZE", "") == "1"
 if HOST_SANITIZE:
-    HOST_FLAGS = ["-O1", "-g", "-fno-omit-frame-pointer", "-fsanitize=address,undefined", "-std=c++17", "-shared", "-fPIC"]
+    HOST_OPTIONS = ["-O1", "-g", "-fno-omit-frame-pointer", "-fsanitize=address,undefined"]
+HOST_FLAGS = [*HOST_OPTIONS, "-std=c++17", "-shared", "-fPIC"]
 
 # Host modules that are Python extensions over torch's tensors: they are built against this interpreter and this torch, which their hash covers.
 EXTENSIONS = ("host_calls",)
@@ -86,7 +88,7 @@ def _extension_flags() -> Tuple[str, ...]:
     include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
     lib = os.path.join(root, "lib")
-    return ("-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+    return (*HOST_FLAGS, "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in include),
             f"-L{lib}", f"-Wl,-rpath,{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip")
 
@@ -149,7 +151,7 @@ def _fallback_dir(create: bool = False) -> Optional[str]:
 def _stem(name: str, variant: Variant) -> str:
     """A library's file name up to its hash (a sanitized host build has a name of its own, so that it and the
     ordinary build do not take each other for stale)."""
-    san = "-hostsan" if HOST_SANITIZE and _is_host_module(name) and name not in EXTENSIONS else ""
+    san = "-hostsan" if HOST_SANITIZE and _is_host_module(name) else ""
     return f"{name}{san}{_variant_tag(variant)}"
 
 

@@ -15,7 +15,7 @@ import torch
 
 from .. import log
 from .device import ARCH, COMPUTE_UNITS, N_XCD
-from .library import KernelModule, Variant, load_extension, load_module
+from .library import KernelBuildError, KernelModule, Variant, load_extension, load_module
 
 P = ctypes.c_void_p
 I = ctypes.c_int
@@ -162,9 +162,28 @@ def _entry(mod: KernelModule, fname: str, argtypes):
     return found
 
 
-_native = load_extension("host_calls")
-_native.connect(_check_in_python, _call_by_ctypes, _call_failed, _entry, ctypes.Array)
-_check, _call, empty, _stream = _native.check, _native.call, _native.empty, _native.stream      # (see csrc/host_calls.cpp)
+def _empty_in_python(shape: Tuple[int, ...], dtype: torch.dtype, like: torch.Tensor) -> torch.Tensor:
+    return torch.empty(shape, dtype=dtype, device=like.device)
+
+
+def _stream_in_python() -> int:
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _host_forms(load):
+    """(the native module or None, check, call, empty, stream): what every launch does on the host, from the extension that ``load`` gives.  Where that cannot
+    be built (no compiler, no ROCm headers, another processor: hosts without this GPU, where the package is imported for its configuration and plans) the
+    Python forms do the same work; the kernels themselves have no other form."""
+    try:
+        native = load("host_calls")
+    except (KernelBuildError, ImportError, OSError) as e:
+        log.warn("kernels", f"launches are checked and called in Python, several times slower: {str(e).splitlines()[0]}")
+        return None, _check_in_python, _call_by_ctypes, _empty_in_python, _stream_in_python
+    native.connect(_check_in_python, _call_by_ctypes, _call_failed, _entry, ctypes.Array)
+    return native, native.check, native.call, native.empty, native.stream
+
+
+_native, _check, _call, empty, _stream = _host_forms(load_extension)      # (see csrc/host_calls.cpp)
 
 
 # ----------------------------------------------------------------------------------------

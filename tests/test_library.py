@@ -174,6 +174,46 @@ def test_native_checks_raise_what_the_python_check_raises():
             ops.empty(*wrong)
 
 
+@pytest.mark.parametrize("failure", [library.KernelBuildError("g++ failed\nwith many lines"), ImportError("built for another interpreter"), OSError("no such library")])
+def test_without_the_native_calls_python_does_their_work(failure, capfd):
+    """A host that cannot build the extension imports the package all the same: the same checks, calls and tensors by the Python forms, and a line that says so."""
+    from inferflux_amd.kernels import ops
+
+    def load(name):
+        raise failure
+    native, check, call, empty, stream = ops._host_forms(load)
+    assert native is None and str(failure).split("\n")[0] in capfd.readouterr().err
+    x = torch.zeros(2, 3)
+    with pytest.raises(ops.KernelError, match="GPU"):
+        check(x, "x", (2, 3))
+    y = empty((2, 0, 5), torch.bfloat16, x)
+    assert y.shape == (2, 0, 5) and y.dtype == torch.bfloat16 and y.device == x.device
+    f = _Function("pif")
+    call(f, "fake", f.argtypes, x, 7, 0.5)
+    assert f.got == (x.data_ptr(), 7, 0.5) and callable(stream)
+    f = _Function("p", rc=-7)
+    with pytest.raises(ops.KernelError, match=r"fake: an error of its own \(code -7\)"):
+        call(f, "fake", f.argtypes, None)
+
+
+def test_the_package_imports_where_nothing_can_be_built(tmp_path):
+    """Its configurations and plans do not need a compiler: a copy of the Python files alone, with no compiler to be found."""
+    import shutil
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(library.CSRC))
+    shutil.copytree(os.path.join(root, "inferflux_amd"), tmp_path / "inferflux_amd", ignore=shutil.ignore_patterns("*.so", "__pycache__", ".*.lock"))
+    env = {**os.environ, "PATH": "", "CXX": "/nonexistent", "HIPCC": "", "ROCM_PATH": "/nonexistent", "TMPDIR": str(tmp_path), "PYTHONDONTWRITEBYTECODE": "1"}
+    code = ("from inferflux_amd.kernels import library\n"
+            "def absent():\n    raise library.KernelBuildError('no compiler')\n"
+            "library._cxx = absent\n"
+            "from inferflux_amd.engine import engine, context\n"
+            "from inferflux_amd.kernels import ops\n"
+            "print('native', ops._native)\n")
+    out = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, env=env, capture_output=True, text=True, timeout=110)
+    assert out.returncode == 0 and "native None" in out.stdout and "no compiler" in out.stderr, out.stderr[-2000:]
+
+
 @pytest.mark.gpu
 def test_native_checks_on_the_gpu():
     from inferflux_amd.kernels import ops
