@@ -19,9 +19,12 @@ from . import ops
 
 TILE_MIN = 16       # fewer rows than this are cheaper one by one
 F32_TILE_MIN = 16   # ... in 32 bits,
-F32_TILE_MIN_WORK = 1 << 18     # and steps of less than this many (row, head, map) items times the longest context: us plain / in tiles with 14 heads
-                                # of 64 and 8 of 128 elements, one prompt of 80 rows 13 / 15, 16 / 23; of 200 30 / 16, 36 / 28; 64 of 40 rows 67 / 22,
-                                # 66 / 25; 64 rows behind 500 keys 35 / 23, 36 / 47, 128 rows 73 / 24, 85 / 48; two of 2,000 rows 2,470 / 208, 2,770 / 246
+F32_TILE_MIN_WORK, F32_WIDE_TILE_MIN_WORK = 1 << 18, 300_000    # and steps of less than this many (row, head, map) items times the longest context,
+                                # the second for tiles of 128 columns, 8 heads of 128 on two in what follows beside 14 of 64 on two.  us plain / in tiles, a prompt of
+                                # 80 rows 16 / 24, 13 / 15; of 200 37 / 28, 30 / 16; 64 of 40 rows 68 / 25, 67 / 22; 64 rows behind 500 keys 36 / 46 (289,000 items), 34 / 23, 128
+                                # rows 87 / 47, 73 / 23; 64 behind 400 beside 32 prompts of 16 70 / 38, 49 / 27, 16 behind 3,000 beside 16 of 16 387 / 82, 258 / 61; two of 2,000
+                                # rows 2,760 / 247, 2,460 / 210.  480 steps drawn around the lines: 0.91 of the plain kernel's speed at worst in tiles beyond
+                                # them, 0.59 and a tenth slower with a line at 1 << 17 for tiles of 128 columns; counting each request's own context is no better
 F32_SPLIT = ((64, 128), (128, 255), (256, 768))    # 32-bit tiles by four workgroups each: up to so many workgroups without that, longer contexts
                                 # than this.  us whole / split: 44 workgroups of 64 elements and 200 keys 23 / 16, 112 and 256 keys 23 / 22, 220 and
                                 # 1,000 keys 72 / 52; but 104 and 112 keys 15 / 20, 224 and 256 keys 23 / 34; of 128 elements 14 and 200 keys 43 / 28,
@@ -281,7 +284,8 @@ def _f32_tiles(ctx, n_heads: int, n_kv: int, maps: int, cols: int):
     """(tiles, rows that are not in one, whether parts go by workgroups of their own) of a step for ``ops.attention_f32``; the first None:
     the step has no tiles, the second None: no further rows."""
     tiled = ctx.h_q_len >= F32_TILE_MIN
-    if not tiled.any() or int(ctx.h_q_len[tiled].sum()) * n_heads * maps * int(ctx.h_kv_len[tiled].max()) < F32_TILE_MIN_WORK:
+    least = F32_WIDE_TILE_MIN_WORK if cols > 64 else F32_TILE_MIN_WORK
+    if not tiled.any() or int(ctx.h_q_len[tiled].sum()) * n_heads * maps * int(ctx.h_kv_len[tiled].max()) < least:
         return None, None, False
     group = n_heads // n_kv
     tiles = [(r, c) for r in np.nonzero(tiled)[0] for c in range(0, int(ctx.h_q_len[r]) * group, cols)]

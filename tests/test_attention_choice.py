@@ -1,11 +1,12 @@
 """How the tile attention kernel's launch is chosen (no GPU needed): the choices that were measured, and what every
 choice must satisfy for the kernel to be right."""
 import random
+import types
 
 import numpy as np
 import torch
 
-from inferflux_amd.kernels.attention import TILE_MAX_SPLITS, choose_tiling, tile_order
+from inferflux_amd.kernels.attention import F32_TILE_MIN, TILE_MAX_SPLITS, _f32_tiles, choose_tiling, tile_order
 
 ROWS_OF = lambda qt: 64 * qt          # head size 128
 
@@ -212,3 +213,40 @@ def test_row_launch_shape():
         chunk, waves, splits = row_launch_shape(rows, kv_heads, bound)
         assert waves == 0 and chunk % 32 == 0 and chunk >= 64
         assert splits * chunk >= bound > (splits - 1) * chunk and splits <= ROW_MAX_SPLITS
+
+
+def _f32_step(rows, past):
+    """What ``_f32_tiles`` reads of a step whose requests bring ``rows`` behind ``past`` keys."""
+    q_len = np.asarray(rows, np.int32)
+    return types.SimpleNamespace(h_q_len=q_len, h_kv_len=q_len + np.asarray(past, np.int32), h_row_req=np.repeat(np.arange(len(rows)), rows), upload=torch.from_numpy)
+
+
+def test_prompts_in_32_bits_take_tiles_where_those_are_faster():
+    """The steps that were measured on either side (us plain / in tiles), heads of 128 elements in tiles of 128 columns and of 64 in tiles of 64."""
+    for rows, past, wide, narrow in [  # 8 heads of 128 on two, 14 of 64 on two
+        ([80], [0], False, False),                               # 16 / 24, 13 / 15
+        ([200], [0], True, True),                                # 37 / 28, 30 / 16
+        ([40] * 64, [0] * 64, True, True),                       # 68 / 25, 67 / 22
+        ([64], [500], False, True),                              # 36 / 46, 34 / 23
+        ([128], [500], True, True),                              # 87 / 47, 73 / 23
+        ([64] + [16] * 32, [400] + [0] * 32, True, True),        # 70 / 38, 49 / 27
+        ([16] * 17, [3000] + [0] * 16, True, True),              # 387 / 82, 258 / 61
+        ([2000] * 2, [0] * 2, True, True),                       # 2,760 / 247, 2,460 / 210
+        ([15] * 500, [2000] * 500, False, False),                # (fewer rows a request than a tile is worth)
+    ]:
+        step = _f32_step(rows, past)
+        assert (_f32_tiles(step, 8, 2, 1, 128)[0] is not None) == wide, (rows, past)
+        assert (_f32_tiles(step, 14, 2, 1, 64)[0] is not None) == narrow, (rows, past)
+
+
+def test_32_bit_tiles_hold_every_row_once_and_the_longest_walks_come_first():
+    rng = random.Random(3)
+    for cols, n_heads, n_kv, maps in ((64, 14, 2, 1), (128, 8, 8, 1), (64, 8, 2, 2), (64, 6, 2, 1)):
+        rows, past = zip(*[(rng.choice([1, 15, 16, 17, 100, 333]), rng.choice([0, 1, 500])) for _ in range(40)])
+        step, group = _f32_step(rows, past), n_heads // n_kv
+        tiles, rest, split = _f32_tiles(step, n_heads, n_kv, maps, cols)
+        assert sorted(map(tuple, tiles.tolist())) == [(r, c) for r, n in enumerate(rows) if n >= F32_TILE_MIN for c in range(0, n * group, cols)]
+        starts = [past[r] + c // group for r, c in tiles.tolist()]
+        assert starts == sorted(starts, reverse=True)
+        assert rest.tolist() == [t for t, r in enumerate(step.h_row_req) if rows[r] < F32_TILE_MIN] and not split      # (more workgroups than are worth four each)
+    assert _f32_tiles(_f32_step([200], [0]), 8, 2, 1, 128)[1:] == (None, True)
