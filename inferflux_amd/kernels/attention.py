@@ -25,6 +25,7 @@ F32_TILE_MIN_WORK, F32_WIDE_TILE_MIN_WORK = 1 << 18, 300_000    # and steps of l
                                 # rows 87 / 47, 73 / 23; 64 behind 400 beside 32 prompts of 16 70 / 38, 49 / 27, 16 behind 3,000 beside 16 of 16 387 / 82, 258 / 61; two of 2,000
                                 # rows 2,760 / 247, 2,460 / 210.  480 steps drawn around the lines: 0.91 of the plain kernel's speed at worst in tiles beyond
                                 # them, 0.59 and a tenth slower with a line at 1 << 17 for tiles of 128 columns; counting each request's own context is no better
+F32_MAX_COLUMNS = 1 << 26        # (row, head) columns of whole tiles that a launch holds; larger steps stay with the plain kernel, which goes portion by portion
 F32_SPLIT = ((64, 128), (128, 255), (256, 768))    # 32-bit tiles by four workgroups each: up to so many workgroups without that, longer contexts
                                 # than this.  us whole / split: 44 workgroups of 64 elements and 200 keys 23 / 16, 112 and 256 keys 23 / 22, 220 and
                                 # 1,000 keys 72 / 52; but 104 and 112 keys 15 / 20, 224 and 256 keys 23 / 34; of 128 elements 14 and 200 keys 43 / 28,
@@ -288,6 +289,8 @@ def _f32_tiles(ctx, n_heads: int, n_kv: int, maps: int, cols: int):
     if not tiled.any() or int(ctx.h_q_len[tiled].sum()) * n_heads * maps * int(ctx.h_kv_len[tiled].max()) < least:
         return None, None, False
     group = n_heads // n_kv
+    if int((-(-ctx.h_q_len[tiled].astype(np.int64) * group // cols)).sum()) * n_kv * cols >= F32_MAX_COLUMNS:
+        return None, None, False
     tiles = [(r, c) for r in np.nonzero(tiled)[0] for c in range(0, int(ctx.h_q_len[r]) * group, cols)]
     past = ctx.h_kv_len - ctx.h_q_len
     tiles.sort(key=lambda t: -int(past[t[0]]) - t[1] // group)                  # the longest walks first

@@ -250,3 +250,14 @@ def test_32_bit_tiles_hold_every_row_once_and_the_longest_walks_come_first():
         assert starts == sorted(starts, reverse=True)
         assert rest.tolist() == [t for t, r in enumerate(step.h_row_req) if rows[r] < F32_TILE_MIN] and not split      # (more workgroups than are worth four each)
     assert _f32_tiles(_f32_step([200], [0]), 8, 2, 1, 128)[1:] == (None, True)
+
+
+def test_steps_beyond_a_launch_of_32_bit_tiles_stay_with_the_plain_kernel():
+    """The entry point takes fewer than 2^26 columns of whole tiles; the plain kernel takes any number of rows."""
+    for rows, n_heads, n_kv, cols, takes in (([16], 64 * 16, 16, 64, True), ([1 << 20], 64, 64, 64, False), ([(1 << 20) - 64], 64, 64, 64, True),
+                                             ([1 << 19, 1 << 19], 64, 1, 128, False), ([17] * 4, 1 << 20, 1 << 20, 64, False)):
+        step = types.SimpleNamespace(h_q_len=np.asarray(rows, np.int32), h_kv_len=np.asarray(rows, np.int32), h_row_req=np.zeros(0, np.int64),
+                                     upload=torch.from_numpy)
+        tiles = _f32_tiles(step, n_heads, n_kv, 1, cols)[0]
+        assert (tiles is not None) == takes, (rows, n_heads, n_kv)
+        assert tiles is None or len(tiles) * n_kv * cols // 4 < 1 << 24
