@@ -13,13 +13,16 @@
 //   few    a wave takes four columns of an item (of gate and of up) by vector instructions: the matrix instruction adds its four products to the
 //          sum one after the other, each rounded once, so fmaf() in its order gives the same bits.  (By matrix instructions, of whose 256
 //          sums an item wants 16, 16 items of 1,024 x 1,408 took 57 us where these take 43.)  Every item streams its expert's weights: for steps of few rows, which rarely share
-//          an expert.
+//          an expert.  Bound by the caches then (227 us for the 1.66 GB that 192 items of 704 ask for).
+//   four   the same for up to four items of an expert at a time (ifx_moe_sort's tiles of four), whose weights are asked for once: for experts of one to
+//          eight items, of which tiles of 64 would be empty for the most part.
 //   tiles  items ordered by expert (ifx_moe_sort), 64 items by 64 weight rows through LDS as in gemm_f32_tiles_kernel; a wave's two tiles of
 //          weight rows are gate's and up's of the same columns.
 //
-// Before, a wave of moe.hip formed the outputs of an item and the weights were read again for every row.  us of both products, that way : these (16
-// experts 1,024 wide and 1,408 inner, two to a row) 1 row 15 : 12, 8 45 : 43, 32 134 : 147, 64 215 : 146, 1,720 3,298 : 468 (93 TFLOP/s); 64 of 704, six to
-// a row, 1 22 : 15, 16 121 : 120, 32 201 : 227, 64 358 : 241, 1,720 6,354 : 744.
+// Before, a wave of moe.hip formed the outputs of an item and the weights were read again for every row.  us of both products, that way : few : four : tiles (16
+// experts 1,024 wide and 1,408 inner, two to a row) 1 row 15 : 12 : 21 : 93, 8 45 : 43 : 35 : 112, 32 132 : 151 : 79 : 145, 64 212 : 274 : 114 : 145, 128 351 : 555 : 180 : 149, 1,720
+// 3,298 : - : - : 468 (93 TFLOP/s); 64 of 704, six to a row, 1 21 : 15 : 36 : 71, 8 68 : 67 : 75 : 133, 16 122 : 122 : 112 : 217, 32 199 : 227 : 146 : 240, 64 365 : 443 : 213 : 242, 1,720 6,354 :
+// - : - : 744; 32 2,048 wide and 1,408 inner, four to a row, 4 90 : 94 : 100 : 246, 8 163 : 175 : 149 : 331, 64 859 : 1,217 : 425 : 460.
 #include "common.h"
 #include "f32_slices.h"
 
@@ -54,20 +57,21 @@ __device__ __forceinline__ float halve(float first, float second, bool odd) {
   return (odd ? second : first) + dpp<CTRL>(odd ? first : second);
 }
 
-// x . w[r] for R (4 or 8) rows of K values; lane l takes the k-values 4 l ... 4 l + 3 of a block of 256, AT_ONCE blocks asked for at a time, and is left
-// with the sum of row (l & 3) + (l & 4): of 8 rows the lanes of bit 2 have the later four.
-template <int R, bool VEC>
-__device__ __forceinline__ float dots(const float* __restrict__ x, const float* const (&w)[R], int K, int lane) {
+// total[j] = x[j] . w[r] for R (4 or 8) rows of K values and the first `count` of ITEMS rows of x; lane l takes the k-values 4 l ... 4 l + 3 of a block of
+// 256, AT_ONCE blocks asked for at a time, and is left with the sum of row (l & 3) + (l & 4): of 8 rows the lanes of bit 2 have the later four.
+template <int R, bool VEC, int ITEMS>
+__device__ __forceinline__ void dots(const float* const (&x)[ITEMS], int count, const float* const (&w)[R], int K, int lane, float (&total)[ITEMS]) {
   constexpr int AT_ONCE = R > 4 ? 2 : 4;
   const bool one = lane & 1, two = lane & 2, four = lane & 4;
-  float total = 0.f;
   for (int k0 = 0; k0 < K; k0 += 256 * AT_ONCE) {
-    f32x4 xv[AT_ONCE], wv[AT_ONCE][R];
+    f32x4 xv[AT_ONCE][ITEMS], wv[AT_ONCE][R];
     if (VEC && k0 + 256 * AT_ONCE <= K) {          // (no lane's place lies beyond K)
 #pragma unroll
       for (int b = 0; b < AT_ONCE; ++b) {
         const int k = k0 + 256 * b + 4 * lane;
-        xv[b] = *(const f32x4*)(x + k);
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j)
+          if (j < count) xv[b][j] = *(const f32x4*)(x[j] + k);
 #pragma unroll
         for (int r = 0; r < R; ++r) wv[b][r] = *(const f32x4*)(w[r] + k);
       }
@@ -75,7 +79,9 @@ __device__ __forceinline__ float dots(const float* __restrict__ x, const float* 
 #pragma unroll
       for (int b = 0; b < AT_ONCE; ++b) {
         const int k = k0 + 256 * b + 4 * lane;
-        xv[b] = load4<VEC>(x, k, K);
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j)
+          if (j < count) xv[b][j] = load4<VEC>(x[j], k, K);
 #pragma unroll
         for (int r = 0; r < R; ++r) wv[b][r] = load4<VEC>(w[r], k, K);
       }
@@ -83,62 +89,89 @@ __device__ __forceinline__ float dots(const float* __restrict__ x, const float* 
 #pragma unroll
     for (int b = 0; b < AT_ONCE; ++b) {
       if (k0 + 256 * b >= K) break;
-      float v[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {          // (the matrix instruction adds its four products one after the other, each rounded once: so does this)
-        v[r] = 0.f;
+      for (int j = 0; j < ITEMS; ++j) {
+        if (j >= count) break;
+        float v[R];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[r] = fmaf(xv[b][q], wv[b][r][q], v[r]);
+        for (int r = 0; r < R; ++r) {          // (the matrix instruction adds its four products one after the other, each rounded once: so does this)
+          v[r] = 0.f;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[r] = fmaf(xv[b][j][q], wv[b][r][q], v[r]);
+        }
+        float u[R / 2], t[R / 4];
+#pragma unroll
+        for (int r = 0; r < R / 2; ++r) u[r] = halve<0xb1>(v[2 * r], v[2 * r + 1], one);             // lanes l and l ^ 1
+#pragma unroll
+        for (int r = 0; r < R / 4; ++r) {
+          t[r] = halve<0x4e>(u[2 * r], u[2 * r + 1], two);                                          // ... ^ 2: steps of 16
+          t[r] += dpp<0x128>(t[r]);                                                                 // ... ^ 8 (a rotation of a row of 16 by 8)
+        }
+        // ... ^ 4: by a rotation by 4, which is right where lanes 8 apart hold the same
+        float g = R > 4 ? halve<0x124>(t[0], t[R / 4 - 1], four) : t[0] + dpp<0x124>(t[0]);        // groups of 64
+        const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(g), __float_as_uint(g), false, false);
+        g = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
+        const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(g), __float_as_uint(g), false, false);
+        g = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);                                     // a block
+        total[j] = k0 + b == 0 ? g : total[j] + g;
       }
-      float u[R / 2], t[R / 4];
-#pragma unroll
-      for (int r = 0; r < R / 2; ++r) u[r] = halve<0xb1>(v[2 * r], v[2 * r + 1], one);             // lanes l and l ^ 1
-#pragma unroll
-      for (int r = 0; r < R / 4; ++r) {
-        t[r] = halve<0x4e>(u[2 * r], u[2 * r + 1], two);                                          // ... ^ 2: steps of 16
-        t[r] += dpp<0x128>(t[r]);                                                                 // ... ^ 8 (a rotation of a row of 16 by 8)
-      }
-      // ... ^ 4: by a rotation by 4, which is right where lanes 8 apart hold the same
-      float g = R > 4 ? halve<0x124>(t[0], t[R / 4 - 1], four) : t[0] + dpp<0x124>(t[0]);        // groups of 64
-      const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(g), __float_as_uint(g), false, false);
-      g = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
-      const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(g), __float_as_uint(g), false, false);
-      g = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);                                     // a block
-      total = k0 + b == 0 ? g : total + g;
     }
   }
-  return total;
 }
 
 #define COLUMNS 4          // of a wave
 #define ITEMS_FIRST 12
-template <int MODE, bool VEC>
+#define TOGETHER 4         // items of one expert that a wave takes at a time
+// ITEMS 1: the grid's items one by one.  TOGETHER: the lists' tiles of up to so many.
+template <int MODE, bool VEC, int ITEMS>
 __global__ __launch_bounds__(256) void experts_f32_few_kernel(ExpertsF32 a) {
-  const int item = a.items_first ? blockIdx.x : blockIdx.y, e = a.ids[item], t = item / a.top, lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int nth = a.items_first ? blockIdx.x : blockIdx.y, lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  if (ITEMS > 1 && nth >= *a.n_tiles) return;
   const int n0 = ((a.items_first ? blockIdx.y : blockIdx.x) * 4 + wave) * COLUMNS, K = a.K;
+  const int e = ITEMS > 1 ? a.tile_expert[nth] : a.ids[nth];
   if (n0 >= a.N || (MODE == MODE_GATE_UP && e >= a.n_real)) return;
-  const float weight = a.weights[item];
-  float* out = MODE == MODE_GATE_UP ? a.out + (size_t)item * a.N : a.out + ((size_t)(item - t * a.top) * a.T + t) * a.N;
+  const int count = ITEMS > 1 ? min(a.tile_count[nth], ITEMS) : 1, start = ITEMS > 1 ? a.tile_start[nth] : 0;
+  int item[ITEMS];
+  float weight[ITEMS];
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    item[j] = ITEMS > 1 ? a.sorted[start + min(j, count - 1)] : nth;
+    weight[j] = a.weights[item[j]];
+  }
+  const auto place = [&](int m) {        // of an item's row of results
+    const int t = m / a.top;
+    return a.out + (MODE == MODE_GATE_UP ? (size_t)m : (size_t)(m - t * a.top) * a.T + t) * a.N;
+  };
   if (e >= a.n_real) {
-    if (lane < COLUMNS && n0 + lane < a.N) out[n0 + lane] = weight * a.identity[(size_t)t * a.N + n0 + lane];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (j < count && lane < COLUMNS && n0 + lane < a.N) place(item[j])[n0 + lane] = weight[j] * a.identity[(size_t)(item[j] / a.top) * a.N + n0 + lane];
     return;
   }
   constexpr int R = MODE == MODE_GATE_UP ? 2 * COLUMNS : COLUMNS;
   const float* rows[R];
+  const float* x[ITEMS];
 #pragma unroll
   for (int c = 0; c < COLUMNS; ++c) {
     const size_t at = ((size_t)e * a.N + min(n0 + c, a.N - 1)) * K;          // (columns beyond N are computed and dropped)
     rows[c] = a.w + at;
     if (MODE == MODE_GATE_UP) rows[R / 2 + c] = a.up + at;
   }
-  const float v = dots<R, VEC>(a.x + (size_t)(MODE == MODE_GATE_UP ? t : item) * K, rows, K, lane);
-  const float up = MODE == MODE_GATE_UP ? __shfl(v, lane ^ 4) : 0.f;
-  if (lane >= COLUMNS || n0 + lane >= a.N) return;
-  if (MODE == MODE_GATE_UP) {
-    const float wi = a.weigh_input ? weight : 1.f;
-    out[n0 + lane] = gated_act(wi * v, wi * up, a.act, a.limit);
-  } else {
-    out[n0 + lane] = (a.weigh_input ? 1.f : weight) * v;
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) x[j] = a.x + (size_t)(MODE == MODE_GATE_UP ? item[j] / a.top : item[j]) * K;
+  float v[ITEMS] = {};
+  dots<R, VEC, ITEMS>(x, count, rows, K, lane, v);
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    if (j >= count) break;
+    const float up = MODE == MODE_GATE_UP ? __shfl(v[j], lane ^ 4) : 0.f;
+    if (lane >= COLUMNS || n0 + lane >= a.N) continue;
+    if (MODE == MODE_GATE_UP) {
+      const float wi = a.weigh_input ? weight[j] : 1.f;
+      place(item[j])[n0 + lane] = gated_act(wi * v[j], wi * up, a.act, a.limit);
+    } else {
+      place(item[j])[n0 + lane] = (a.weigh_input ? 1.f : weight[j]) * v[j];
+    }
   }
 }
 
@@ -275,16 +308,17 @@ __global__ __launch_bounds__(256, 2) void experts_f32_tiles_kernel(ExpertsF32 a)
 static bool check_act(int act, float limit) { return act == ACT_SILU || act == ACT_GELU_TANH || (act == ACT_CLAMPED_SWISH && limit > 0.f); }
 static bool on16(const void* p) { return (uintptr_t)p % 16 == 0; }
 
-// Both products.  act [items][ff] is scratch; parts [top][T][N].  sorted ... n_tiles: the lists of ifx_moe_sort with tiles of 64 items, or null: few items,
-// each with its expert's weights for itself.
+// Both products.  act [items][ff] is scratch; parts [top][T][N].  sorted ... n_tiles: the lists of ifx_moe_sort with tiles of tile_items items, 64 for the matrix
+// instruction's tiles or 4 for the vector instructions' that share their weights, or null: few items, each with its expert's weights for itself.
 extern "C" int ifx_moe_f32(const float* h, const float* gate, const float* up, const float* down, const int* ids, const float* weights,
                            float* act, float* parts, const int* sorted, const int* tile_expert, const int* tile_start, const int* tile_count,
-                           const int* n_tiles, int max_tiles, int T, int K, int ff, int N, int top, int n_real, int n_identity, int act_kind,
+                           const int* n_tiles, int max_tiles, int tile_items, int T, int K, int ff, int N, int top, int n_real, int n_identity, int act_kind,
                            float limit, int weigh_input, void* stream) {
   IFX_REQUIRE(T >= 0 && K > 0 && ff > 0 && N > 0 && top > 0 && n_real > 0, "moe_f32: bad sizes T=%d K=%d ff=%d N=%d top=%d", T, K, ff, N, top);
   IFX_REQUIRE(check_act(act_kind, limit), "moe_f32: gated activation %d (limit %g)", act_kind, (double)limit);
   IFX_REQUIRE(n_identity == 0 || N == K, "moe_f32: identity experts hand back the row itself, so N=%d must equal K=%d", N, K);
   IFX_REQUIRE((sorted ? (long long)max_tiles : (long long)T * top) <= 65535, "moe_f32: %lld items or tiles are too many for one launch", sorted ? (long long)max_tiles : (long long)T * top);
+  IFX_REQUIRE(sorted ? tile_items == TILE_ITEMS || tile_items == TOGETHER : tile_items == 1, "moe_f32: tiles of %d items", tile_items);
   if (T == 0) return 0;
   // (us with the items : the columns running fastest, 16 experts of 704: 4 items 11.9 : 14.1, 8 16.2 : 18.0, 16 27.9 : 24.6, 32 46 : 38, 64 84 : 65;
   // 64 experts: 12 21 : 24, 24 42 : 37.  With 1,000,000 columns the grid's second dimension is at its end.)
@@ -293,19 +327,24 @@ extern "C" int ifx_moe_f32(const float* h, const float* gate, const float* up, c
   ExpertsF32 d{act, down, nullptr, parts, ids, weights, h, sorted, tile_expert, tile_start, tile_count, n_tiles, T, top, ff, N, n_real, act_kind, limit, weigh_input, items_first};
   const bool vec_g = K % 4 == 0 && on16(h) && on16(gate) && on16(up), vec_d = ff % 4 == 0 && on16(act) && on16(down);
   hipStream_t s = (hipStream_t)stream;
-#define GO(KERNEL, MODE, VEC, ARGS, COLS) \
-  hipLaunchKernelGGL((KERNEL<MODE, VEC>), items_first ? dim3(T * top, (ARGS.N + COLS - 1) / COLS) : dim3((ARGS.N + COLS - 1) / COLS, sorted ? max_tiles : T * top), dim3(256), 0, s, ARGS)
-  if (sorted) {
-    if (vec_g) GO(experts_f32_tiles_kernel, MODE_GATE_UP, true, g, 32);
-    else GO(experts_f32_tiles_kernel, MODE_GATE_UP, false, g, 32);
-    if (vec_d) GO(experts_f32_tiles_kernel, MODE_DOWN, true, d, 64);
-    else GO(experts_f32_tiles_kernel, MODE_DOWN, false, d, 64);
+#define GO(KERNEL, ARGS, COLS) \
+  hipLaunchKernelGGL(KERNEL, items_first ? dim3(T * top, (ARGS.N + COLS - 1) / COLS) : dim3((ARGS.N + COLS - 1) / COLS, sorted ? max_tiles : T * top), dim3(256), 0, s, ARGS)
+#define FEW(ITEMS) \
+  if (vec_g) GO((experts_f32_few_kernel<MODE_GATE_UP, true, ITEMS>), g, 4 * COLUMNS); \
+  else GO((experts_f32_few_kernel<MODE_GATE_UP, false, ITEMS>), g, 4 * COLUMNS); \
+  if (vec_d) GO((experts_f32_few_kernel<MODE_DOWN, true, ITEMS>), d, 4 * COLUMNS); \
+  else GO((experts_f32_few_kernel<MODE_DOWN, false, ITEMS>), d, 4 * COLUMNS)
+  if (!sorted) {
+    FEW(1);
+  } else if (tile_items == TOGETHER) {
+    FEW(TOGETHER);
   } else {
-    if (vec_g) GO(experts_f32_few_kernel, MODE_GATE_UP, true, g, 4 * COLUMNS);
-    else GO(experts_f32_few_kernel, MODE_GATE_UP, false, g, 4 * COLUMNS);
-    if (vec_d) GO(experts_f32_few_kernel, MODE_DOWN, true, d, 4 * COLUMNS);
-    else GO(experts_f32_few_kernel, MODE_DOWN, false, d, 4 * COLUMNS);
+    if (vec_g) GO((experts_f32_tiles_kernel<MODE_GATE_UP, true>), g, 32);
+    else GO((experts_f32_tiles_kernel<MODE_GATE_UP, false>), g, 32);
+    if (vec_d) GO((experts_f32_tiles_kernel<MODE_DOWN, true>), d, 64);
+    else GO((experts_f32_tiles_kernel<MODE_DOWN, false>), d, 64);
   }
+#undef FEW
 #undef GO
   IFX_LAUNCH_CHECK();
 }

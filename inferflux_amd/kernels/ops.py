@@ -760,16 +760,28 @@ def moe_experts_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
 
 
 MOE_F32_TILE_ITEMS = 64          # items of one expert to a workgroup of the 32-bit tiles
-MOE_F32_FEW_ITEMS = 3.25         # (row, choice) items for each expert up to which each streams its expert's weights for itself (see csrc/moe_f32.hip)
+MOE_F32_TOGETHER = 4             # ... or to a wave, whose items then share their expert's weights (see csrc/moe_f32.hip)
+MOE_F32_TOGETHER_MIN_VALUES = 20_000_000     # k-values times inner columns of all items from which that pays for the items' order, and
+MOE_F32_TOGETHER_MAX_ITEMS = 8               # items to an expert up to which it is faster than tiles
 MOE_F32_PORTION = 16384          # rows of a launch at most (a grid has up to 65,535 tiles)
+
+
+def moe_f32_way(n_items: int, n_experts: int, K: int, ff: int) -> int:
+    """Items to a tile of the 32-bit experts: 1, each streams its expert's weights for itself, MOE_F32_TOGETHER or MOE_F32_TILE_ITEMS.  us by 1 / 4 / 64, by items to
+    an expert: 0.5 to 0.75 94 / 100 / 246 (32 experts of 2,048 x 1,408), 67 / 75 / 133 (64 of 1,024 x 704); 1 43 / 35 / 112 (16 of 1,024 x 1,408), 175 / 149 / 331 (the 32), but 25 /
+    31 / 73 of 16 small ones (16 items of 1,024 x 704, 1.2e7); 2 40 / 38 / 89 of those; 6 443 / 213 / 242 (the 64); 8 274 / 114 / 145 (the 16), 1,217 / 425 / 460 (the 32); 12 to
+    16 866 / 333 / 245, 555 / 180 / 149, 2,401 / 698 / 467, and 103 / 62 / 73 of 8 experts."""
+    if n_items > MOE_F32_TOGETHER_MAX_ITEMS * n_experts:
+        return MOE_F32_TILE_ITEMS
+    return MOE_F32_TOGETHER if n_items >= n_experts and n_items * K * ff >= MOE_F32_TOGETHER_MIN_VALUES else 1
 
 
 def moe_experts_f32(h: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
                     act: int = ACT_SILU, limit: float = 0.0, n_identity: int = 0, weigh_input: bool = False,
-                    few: Optional[bool] = None) -> "SliceSums":
+                    few: Optional[bool] = None, tile_items: int = 0) -> "SliceSums":
     """``moe_experts`` in 32 bits on the matrix cores (``gate`` / ``up`` [E, ff, K], ``down`` [E, N, ff], float32): the choices' weighted
     outputs as ``SliceSums`` [top, T, N].  An element's sum has one order whatever the number of rows; ``few``: each item streams its
-    expert's weights for itself, or items are ordered by expert and meet them in tiles (None chooses)."""
+    expert's weights for itself, or items are ordered by expert and meet them in tiles of ``tile_items``, 64 or 4 (None and 0 choose)."""
     _check(h, "h", (None, None), torch.float32)
     T, K = h.shape
     _check(gate, "gate", (None, None, K), torch.float32)
@@ -786,20 +798,19 @@ def moe_experts_f32(h: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down:
     if T > portion:
         for r in range(0, T, portion):
             parts[:, r:r + portion] = moe_experts_f32(h[r:r + portion], gate, up, down, ids[r:r + portion].contiguous(), weights[r:r + portion].contiguous(),
-                                                      act, limit, n_identity, weigh_input, few).parts
+                                                      act, limit, n_identity, weigh_input, few, tile_items).parts
         return SliceSums(parts, torch.float32)
     n_items = T * top
-    if few is None:
-        few = n_items <= MOE_F32_FEW_ITEMS * n_real
+    tile_items = moe_f32_way(n_items, n_real, K, ff) if few is None else 1 if few else tile_items or MOE_F32_TILE_ITEMS
     lists, max_tiles = (None, None, None, None, None), 0
-    if not few:
-        max_tiles = -(-n_items // MOE_F32_TILE_ITEMS) + E          # every expert may end on a tile that is not full
+    if tile_items > 1:
+        max_tiles = -(-n_items // tile_items) + E          # every expert may end on a tile that is not full
         ints = empty((n_items + 3 * max_tiles + 2,), torch.int32, h)
         lists = (ints[:n_items], *(ints[n_items + i * max_tiles:n_items + (i + 1) * max_tiles] for i in range(3)), ints[n_items + 3 * max_tiles:])
-        _call(load_module("grouped_gemm"), "ifx_moe_sort", (P, I, I, I, I, P, P, P, P, P, P), ids, n_items, E, n_real, MOE_F32_TILE_ITEMS, *lists, _stream())
+        _call(load_module("grouped_gemm"), "ifx_moe_sort", (P, I, I, I, I, P, P, P, P, P, P), ids, n_items, E, n_real, tile_items, *lists, _stream())
     a = empty((n_items, ff), torch.float32, h)
-    _call(load_module("moe_f32"), "ifx_moe_f32", (P,) * 13 + (I,) * 9 + (F, I, P), h, gate, up, down, ids, weights, a, parts, *lists, max_tiles,
-          T, K, ff, N, top, n_real, int(n_identity), int(act), float(limit), 1 if weigh_input else 0, _stream())
+    _call(load_module("moe_f32"), "ifx_moe_f32", (P,) * 13 + (I,) * 10 + (F, I, P), h, gate, up, down, ids, weights, a, parts, *lists, max_tiles,
+          tile_items, T, K, ff, N, top, n_real, int(n_identity), int(act), float(limit), 1 if weigh_input else 0, _stream())
     return SliceSums(parts, torch.float32)
 
 
