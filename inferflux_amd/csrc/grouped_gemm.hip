@@ -207,8 +207,8 @@ __global__ __launch_bounds__(512, 4) void experts_kernel(ExpertsArgs a) {
 // not full and the last round of the chip: 20,400 items of 32 experts (2,048 wide, 1,408 inner) both products and the order of the items
 // 537 -> 477 us (740 TFLOP/s), 65,536 items 1,414 -> 1,219 (930).  Tiles of 128 items (three slots) were
 // 1.0 to 1.2 x the eight waves' time; with tiles of 256 the sums, the fragments and the rows' addresses fill the registers, and the compiler
-// moves sums about between the products in assembly, whose results it does not wait for: wrong sums.  So whoever changes this kernel looks
-// for such moves (v_accvgpr_read within 14 instructions of the product that writes it) in its assembly.
+// moves sums about between the products in assembly, whose results it does not wait for: wrong sums.  A test looks for
+// such moves (a sum read within 14 wait states of the product that writes it) in the built kernels, along every path.
 template <int MODE, int FN, int FM>
 struct ExpertWaves {
   typedef WaveTiles<FN, FM, true> P;

@@ -1,6 +1,9 @@
 """Where built libraries are looked for and written (no GPU)."""
 import os
+import re
+import shutil
 import stat
+import subprocess
 
 import pytest
 import torch
@@ -41,6 +44,88 @@ def test_barriers_in_assembly_stand_behind_a_wait_for_what_was_read_from_lds():
                 before = "\n".join(lines[max(0, i - 5):i])
                 assert "lgkmcnt(0)" in line.split("//")[0] or "__builtin_amdgcn_s_waitcnt(0xc07f)" in before, f"{name}:{i + 1}"
     assert found >= 4
+
+
+def _sums_read_early(kernel, states=14):
+    """Of a kernel's disassembled lines: those that may read an accumulation register fewer than ``states`` wait states (an instruction is one, s_nop n is n + 1)
+    after a matrix product that writes it, on any path, branches taken and not."""
+    def registers(operand):
+        m = re.fullmatch(r"a(\d+)|a\[(\d+):(\d+)\]", operand)
+        return set() if not m else {int(m[1])} if m[1] else set(range(int(m[2]), int(m[3]) + 1))
+    code, at = [], {}
+    for line in kernel:
+        text, _, comment = line.partition("//")
+        op, _, rest = text.strip().partition(" ")
+        target = re.search(r"<.*?(?:\+0x([0-9a-f]+))?>", comment) if op.startswith(("s_branch", "s_cbranch")) else None
+        at[int(comment.split(":")[0], 16)] = len(code)
+        code.append((op, [o.strip().split(" ")[0] for o in rest.split(",")], int(target[1] or "0", 16) if target else None, text.strip()))
+    first = min(at)
+    starts = {0} | {at[first + t] for _, _, t, _ in code if t is not None} | {i + 1 for i, c in enumerate(code) if c[2] is not None}
+    since, todo, early = {0: {}}, [0], set()          # (where a block starts: registers written shortly before, with the states since)
+    while todo:
+        i = todo.pop()
+        recent = dict(since[i])
+        after = []
+        while i < len(code):
+            op, operands, target, text = code[i]
+            if op.startswith("v_mfma"):
+                recent = {**{r: n + 1 for r, n in recent.items() if n + 1 < states}, **dict.fromkeys(registers(operands[0]), 0)}
+            else:
+                read = set().union(*map(registers, operands if "store" in op or op.startswith("ds_write") else operands[1:]))
+                if read & recent.keys():
+                    early.add(text)
+                took = int(operands[0], 0) + 1 if op == "s_nop" else 1
+                recent = {r: n + took for r, n in recent.items() if n + took < states}
+            i += 1
+            if target is not None:
+                after.append(at[first + target])
+            if op in ("s_branch", "s_endpgm"):
+                break
+            if i in starts:
+                after.append(i)
+                break
+        for j in after:
+            known = since.get(j)
+            joined = {r: min(n, (known or {}).get(r, states)) for r, n in recent.items()} | {r: n for r, n in (known or {}).items() if r not in recent}
+            if joined != known:
+                since[j] = joined
+                todo.append(j)
+    return early
+
+
+def _line(address, text, target=None):
+    return f"\t{text}  // {address:012X}: 00000000" + (f" <k+0x{target:x}>" if target is not None else "")
+
+
+def test_sums_read_early_are_found_along_every_path():
+    product, read = "v_mfma_f32_16x16x32_bf16 a[4:7], v[0:3], v[4:7], a[4:7]", "v_accvgpr_read_b32 v9, a6"
+    assert _sums_read_early([_line(0, product), _line(8, read), _line(16, "s_endpgm")]) == {read}
+    assert not _sums_read_early([_line(0, product), _line(8, "s_nop 12"), _line(12, read.replace("a6", "a8")), _line(16, read), _line(20, "s_endpgm")])
+    assert _sums_read_early([_line(0, product), _line(8, "s_nop 12"), _line(12, read), _line(16, "s_endpgm")]) == {read}
+    # around a loop, and over a branch to a place before
+    assert _sums_read_early([_line(0, read), _line(8, "s_nop 15"), _line(16, product), _line(24, "s_cbranch_scc1 65530", 0), _line(32, "s_endpgm")]) == {read}
+    assert _sums_read_early([_line(0, "s_branch 4", 24), _line(8, read), _line(16, "s_endpgm"), _line(24, product), _line(32, "s_cbranch_scc0 1", 8), _line(40, "s_nop 15"),
+                             _line(48, read.replace("v9", "v8")), _line(56, "s_endpgm")]) == {read}
+    assert _sums_read_early([_line(0, product), _line(8, "buffer_store_dwordx4 a[4:7], v1, s[0:3], 0 offen"), _line(16, "s_endpgm")])
+
+
+@pytest.mark.parametrize("name", ["grouped_gemm", "gemm_tiles"])
+def test_nothing_reads_a_sum_of_a_product_in_assembly_too_early(name, tmp_path):
+    """The tiles by four large waves keep their sums in registers that products in assembly write.  The compiler does not know how long such a product takes,
+    so a move of a sum that it puts shortly behind one (as it did with 256 items to a tile) reads what was there before: there is none in the built kernels."""
+    dump, built = "/opt/rocm/llvm/bin/llvm-objdump", library.find_library(name)
+    if built is None or not os.path.isfile(dump):
+        pytest.skip("needs the built module and the disassembler")
+    shutil.copy(built, tmp_path / "module.so")
+    subprocess.run([dump, "--offloading", "module.so"], cwd=tmp_path, check=True, capture_output=True)
+    image = next(f for f in os.listdir(tmp_path) if library.ARCH in f)
+    text = subprocess.run([dump, "-d", "--no-show-raw-insn", image], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+    kernels = [k.split("\n") for k in re.split(r"\n(?=[0-9a-f]+ <)", text) if re.match(r"[0-9a-f]+ <.*(experts_waves|tiles)_kernel.*>:", k)]
+    assert kernels
+    for name_line, *lines in kernels:
+        lines = [line for line in lines if "//" in line]
+        assert sum("v_mfma" in line for line in lines) > 50
+        assert not _sums_read_early(lines), name_line
 
 
 class _Function:
@@ -198,8 +283,6 @@ def test_without_the_native_calls_python_does_their_work(failure, capfd):
 
 def test_the_package_imports_where_nothing_can_be_built(tmp_path):
     """Its configurations and plans do not need a compiler: a copy of the Python files alone, with no compiler to be found."""
-    import shutil
-    import subprocess
     import sys
     root = os.path.dirname(os.path.dirname(library.CSRC))
     shutil.copytree(os.path.join(root, "inferflux_amd"), tmp_path / "inferflux_amd", ignore=shutil.ignore_patterns("*.so", "__pycache__", ".*.lock"))
