@@ -1,13 +1,8 @@
-// What the true 32-bit products share (gemm_f32.hip, moe_f32.hip): the sixteen slices that K is cut into, whatever the other sizes are, and
-// the loads of a slice's steps of 16 k-values.  See gemm_f32.hip for the order of an element's sum.
+// What the true 32-bit products share (gemm_f32.hip, moe_f32.hip): the loads of four k-values of a row.
 #pragma once
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-#define N_SLICES 16
-
-__device__ __forceinline__ int slice_len(int K) { return ((K + N_SLICES - 1) / N_SLICES + 15) / 16 * 16; }
 
 // Four consecutive elements k .. k + 3 of a row of K, zeros behind its end.  VEC: the row starts on 16 bytes (8 for bf16)
 // and K is a multiple of 4, so four elements are all there or all not.

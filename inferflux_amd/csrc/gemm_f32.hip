@@ -10,9 +10,13 @@
 // (runtime/backends/cuda/native/transformer_forward.cu:4600-4601 instantiates half and bf16
 // only), its library call with float accumulation is runtime/backends/cuda/native/cublas_gemm.cpp:99-117.
 #include "common.h"
-#include "f32_slices.h"
+#include "f32_loads.h"
 
 IFX_DEFINE_LAST_ERROR()
+
+#define N_SLICES 16
+
+__device__ __forceinline__ int slice_len(int K) { return ((K + N_SLICES - 1) / N_SLICES + 15) / 16 * 16; }
 
 // ---- the results ---------------------------------------------------------------------------------------------------------
 // Either the sums as they are, C [M][N], or, with an activation, weight rows of gate and up in turn and C [M][N / 2] = act(gate) * up:

@@ -370,7 +370,8 @@ extern "C" int ifx_gemm_tiles_sums_plan(int M, int N, int K, int library_slices,
   return best;
 }
 
-// The same for up to FEW_MOST multiplications, with tiles by small waves, too: slices (1 without `keep`: the plain product) << 8 | tile.
+// The same for a model's weights and 65 to 2,048 rows (few_tiles_plan in ops.py has the limits and the lines), with tiles by small waves, too: slices (1 without `keep`: the
+// plain product) << 8 | tile.
 #define FEW_MAX_SLICES 16
 extern "C" int ifx_gemm_tiles_few_plan(int M, int N, int K, int keep) {
   int best = 0;

@@ -18,7 +18,7 @@
 // step's layout alone.  One wave forms one output element at a time (lanes across k, the fixed-order sum of
 // common.h), so a row's result does not depend on what shares its batch.  They are the path of bfloat16 sizes that the
 // others do not take; the 32-bit mode has moe_f32.hip, bfloat16 steps of up to 64 rows stream every expert once (moe_few.hip), longer ones take
-// the grouped matrix-core product (grouped_gemm.hip).
+// the grouped matrix-core product (grouped_gemm.hip).  (No model reaches their float forms any more: tests hold these kernels' sums by them.)
 #include "common.h"
 
 IFX_DEFINE_LAST_ERROR()

@@ -24,7 +24,7 @@
 // 3,298 : - : - : 468 (93 TFLOP/s); 64 of 704, six to a row, 1 21 : 15 : 36 : 71, 8 68 : 67 : 75 : 133, 16 122 : 122 : 112 : 217, 32 199 : 227 : 146 : 240, 64 365 : 443 : 213 : 242, 1,720 6,354 :
 // - : - : 744; 32 2,048 wide and 1,408 inner, four to a row, 4 90 : 94 : 100 : 246, 8 163 : 175 : 149 : 331, 64 859 : 1,217 : 425 : 460.
 #include "common.h"
-#include "f32_slices.h"
+#include "f32_loads.h"
 
 IFX_DEFINE_LAST_ERROR()
 

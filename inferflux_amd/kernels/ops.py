@@ -1792,7 +1792,7 @@ def swiglu_tiles(x: torch.Tensor, pairs: torch.Tensor, act: int = ACT_SILU, limi
 
 def act_tiles(x: torch.Tensor, weight: torch.Tensor, act: int, tile: int = -1) -> torch.Tensor:
     """``linear_act`` of many rows in bfloat16 as one launch ([N, K] ``weight``, N even and K a multiple of 8, both on 16 bytes);
-    ``tile`` as for ``swiglu_tiles``, one by four waves."""
+    ``tile`` as for ``swiglu_tiles``, but not 2."""
     _check(weight, "weight", (None, None), torch.bfloat16)
     N, K = weight.shape
     _check(x, "x", (None, K), torch.bfloat16)
@@ -1804,7 +1804,7 @@ def act_tiles(x: torch.Tensor, weight: torch.Tensor, act: int, tile: int = -1) -
 
 def sums_tiles(x: torch.Tensor, weight: torch.Tensor, slices: int, slice_k: int, tile: int) -> "SliceSums":
     """bfloat16 x [M, K] times ``weight`` [N, K] transposed as ``SliceSums`` over ``slices`` of ``slice_k`` values of K (a multiple of
-    64), N a multiple of 4, K of 8, both on 16 bytes; ``tile``: one of the kernel's tiles by four waves."""
+    64), N a multiple of 4, K of 8, both on 16 bytes; ``tile``: one of the kernel's tiles but 2."""
     _check(weight, "weight", (None, None), torch.bfloat16)
     N, K = weight.shape
     _check(x, "x", (None, K), torch.bfloat16)
