@@ -131,9 +131,12 @@ def _check_in_python(t: torch.Tensor, name: str, shape=None, dtype=None) -> None
 
 def upload(array, device) -> torch.Tensor:
     """The numpy ``array`` on ``device``, by a copy on the current stream that the host does not wait for: from pinned memory of its own,
-    which torch's allocator hands out again only after the copy (from ordinary memory ``to`` waits for everything launched before it)."""
+    which torch's allocator hands out again only after the copy (from ordinary memory ``to`` waits for everything launched before it).  Not in a capture, whose
+    replays would copy what that memory holds by then."""
     if torch.device(device).type != "cuda":
         return torch.from_numpy(array).to(device)
+    if torch.cuda.is_current_stream_capturing():
+        raise KernelError("upload: a captured step's arrays go into buffers that outlive it")
     pageable = torch.from_numpy(array)
     pinned = torch.empty(pageable.shape, dtype=pageable.dtype, pin_memory=True)
     pinned.copy_(pageable)

@@ -318,3 +318,12 @@ def test_native_checks_on_the_gpu():
         assert ops._stream() == side.cuda_stream != 0
     a = ops.upload(__import__("numpy").arange(1000, dtype="int32"), x.device)
     assert torch.equal(a.cpu(), torch.arange(1000, dtype=torch.int32))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):                  # (from ordinary memory the copy was refused there, too)
+        b = a + 1
+        with pytest.raises(ops.KernelError, match="captured"):
+            ops.upload(__import__("numpy").arange(1000, dtype="int32"), x.device)
+    for n in (1, 2):
+        a += 1
+        graph.replay()
+        assert torch.equal(b.cpu(), torch.arange(1000, dtype=torch.int32) + n + 1)
