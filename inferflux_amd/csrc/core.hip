@@ -566,12 +566,56 @@ __global__ __launch_bounds__(64) void rope_append_kernel(RopeArgs a) {
 // blocks append v: a thread takes one dimension of one kv head for 8 consecutive tokens and, when
 // their slots are 8 consecutive offsets of one page starting at a multiple of 8, writes them as one
 // piece of the transposed page; otherwise element by element.
+// SUMS: the rows are float partial sums, added in slice order (four slices asked for together).  One element at a time, as the kernel above takes them, they
+// cost 20 heads of 128 8.8 us at 512 rows and 24 at 2,048 in one slice, 8.8 and 25 in four; like this 4.2 and 7.0, 5.6 and 16.5 (rows of bfloat16 4.8 and 7.4).
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 rope_bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float rope_f4;
 
+template <bool SUMS>
+__device__ __forceinline__ void rope_in8(const RopeArgs& a, size_t at, float (&f)[8]) {
+  if (!SUMS) {
+    const rope_bf16x8 x = *(const rope_bf16x8*)((const bf16_t*)a.qkv + at);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = (float)x[e];
+    return;
+  }
+  const float* p = (const float*)a.qkv + at;
+  for (int s0 = 0; s0 < a.n_slices; s0 += 4) {
+    rope_f4 x[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (s0 + u < a.n_slices) {
+        x[u][0] = *(const rope_f4*)(p + (size_t)(s0 + u) * a.slice_stride);
+        x[u][1] = *(const rope_f4*)(p + (size_t)(s0 + u) * a.slice_stride + 4);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (s0 + u < a.n_slices)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = s0 + u == 0 ? x[u][e / 4][e % 4] : f[e] + x[u][e / 4][e % 4];
+  }
+}
+
+// One element of each of 8 rows, row_width apart (those of `live` are there).
+template <bool SUMS>
+__device__ __forceinline__ void rope_in_rows(const RopeArgs& a, size_t at, int row_width, int live, float (&f)[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) f[k] = k < live ? (SUMS ? ((const float*)a.qkv)[at + (size_t)k * row_width] : (float)((const bf16_t*)a.qkv)[at + (size_t)k * row_width]) : 0.f;
+  if (!SUMS) return;
+  for (int s = 1; s < a.n_slices; ++s) {
+    const float* p = (const float*)a.qkv + (size_t)s * a.slice_stride + at;
+    float x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = k < live ? p[(size_t)k * row_width] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) f[k] += x[k];
+  }
+}
+
+template <bool SUMS>
 __global__ __launch_bounds__(256) void rope_append_vec_kernel(RopeArgs a, int T, int n_qk_blocks) {
   const int d = a.d, half = d / 2;
   const int q_width = a.nH * d, kv_width = a.nKV * d, row_width = q_width + 2 * kv_width;
-  const bf16_t* qkv = (const bf16_t*)a.qkv;
   const bf16_t* bias = (const bf16_t*)a.bias;
   if ((int)blockIdx.x < n_qk_blocks) {
     const int per_head = d / 16, heads = a.nH + (a.slots ? a.nKV : 0);
@@ -579,11 +623,9 @@ __global__ __launch_bounds__(256) void rope_append_vec_kernel(RopeArgs a, int T,
     if (idx >= (size_t)T * heads * per_head) return;
     const int j = (int)(idx % per_head), head = (int)(idx / per_head % heads), t = (int)(idx / per_head / heads);
     const int col = head * d + 8 * j;
-    const bf16_t* row = qkv + (size_t)t * row_width + col;
-    rope_bf16x8 x0 = *(const rope_bf16x8*)row, x1 = *(const rope_bf16x8*)(row + half);
     float f0[8], f1[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { f0[e] = (float)x0[e]; f1[e] = (float)x1[e]; }
+    rope_in8<SUMS>(a, (size_t)t * row_width + col, f0);
+    rope_in8<SUMS>(a, (size_t)t * row_width + col + half, f1);
     if (bias) {
       const rope_bf16x8 b0 = *(const rope_bf16x8*)(bias + col), b1 = *(const rope_bf16x8*)(bias + col + half);
 #pragma unroll
@@ -620,10 +662,10 @@ __global__ __launch_bounds__(256) void rope_append_vec_kernel(RopeArgs a, int T,
   int slot[8];
   float x[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {   // all loads of the group are independent: they go out together
-    slot[k] = t0 + k < T ? a.slots[t0 + k] : -1;
-    x[k] = t0 + k < T ? (float)qkv[(size_t)(t0 + k) * row_width + col] + b : 0.f;
-  }
+  for (int k = 0; k < 8; ++k) slot[k] = t0 + k < T ? a.slots[t0 + k] : -1;   // all loads of the group are independent: they go out together
+  rope_in_rows<SUMS>(a, (size_t)t0 * row_width + col, row_width, T - t0, x);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) x[k] += b;
   bool run = slot[0] >= 0 && slot[0] % 8 == 0;
 #pragma unroll
   for (int k = 1; k < 8; ++k) run = run && slot[k] == slot[0] + k;
@@ -649,10 +691,10 @@ __global__ __launch_bounds__(256) void rope_append_vec_kernel(RopeArgs a, int T,
 // A head is d / 16 threads, each with two pieces of 8: in the rotated part piece j and its partner rot / 2 further, behind
 // it two neighbours.  The head's sum of squares is added across its threads by shuffles.  The other blocks append v as
 // above, dv wide, mixed and handed on where asked.
+template <bool SUMS>
 __global__ __launch_bounds__(256) void rope_append_vec_x_kernel(RopeArgs a, int T, int n_qk_blocks) {
   const int d = a.d, dv = a.dv, rot = a.rope_style != 0 ? a.rotary_dim : 0;
   const int q_width = a.nH * d, kv_width = a.nKV * d, v_width = a.nKV * dv, row_width = q_width + kv_width + v_width + a.gate_cols + a.extra_cols;
-  const bf16_t* qkv = (const bf16_t*)a.qkv;
   const bf16_t* bias = (const bf16_t*)a.bias;
   if ((int)blockIdx.x < n_qk_blocks) {
     const int per_head = d / 16, heads = a.nH + (a.slots ? a.nKV : 0);
@@ -661,11 +703,9 @@ __global__ __launch_bounds__(256) void rope_append_vec_x_kernel(RopeArgs a, int 
     const int j = (int)(idx % per_head), head = (int)(idx / per_head % heads), t = (int)(idx / per_head / heads);
     const bool rotate = 16 * j < rot;
     const int first = rotate ? 8 * j : rot + 16 * (j - rot / 16), second = rotate ? first + rot / 2 : first + 8;
-    const bf16_t* row = qkv + (size_t)t * row_width + head * d;
-    const rope_bf16x8 x0 = *(const rope_bf16x8*)(row + first), x1 = *(const rope_bf16x8*)(row + second);
     float f0[8], f1[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { f0[e] = (float)x0[e]; f1[e] = (float)x1[e]; }
+    rope_in8<SUMS>(a, (size_t)t * row_width + head * d + first, f0);
+    rope_in8<SUMS>(a, (size_t)t * row_width + head * d + second, f1);
     if (bias) {
       const rope_bf16x8 b0 = *(const rope_bf16x8*)(bias + head * d + first), b1 = *(const rope_bf16x8*)(bias + head * d + second);
 #pragma unroll
@@ -702,7 +742,9 @@ __global__ __launch_bounds__(256) void rope_append_vec_x_kernel(RopeArgs a, int 
     }
     if (head < a.nH && a.gate_cols && j == 0) {
       const int gc = q_width + kv_width + v_width + head;
-      float g = (float)qkv[(size_t)t * row_width + gc];
+      float g = SUMS ? ((const float*)a.qkv)[(size_t)t * row_width + gc] : (float)((const bf16_t*)a.qkv)[(size_t)t * row_width + gc];
+      if (SUMS)
+        for (int s = 1; s < a.n_slices; ++s) g += ((const float*)a.qkv)[(size_t)s * a.slice_stride + (size_t)t * row_width + gc];
       if (bias) g += (float)bias[gc];
       a.gate_out[(size_t)t * a.nH + head] = 1.0f / (1.0f + expf(-g));
     }
@@ -737,9 +779,11 @@ __global__ __launch_bounds__(256) void rope_append_vec_x_kernel(RopeArgs a, int 
   for (int k = 0; k < 8; ++k) {   // all loads of the group are independent: they go out together
     const bool live = t0 + k < T;
     slot[k] = live && a.slots ? a.slots[t0 + k] : -1;
-    x[k] = live ? (float)qkv[(size_t)(t0 + k) * row_width + col] + b : 0.f;
     m[k] = live && vf ? (float)vf[((size_t)(t0 + k) * a.nKV + kh) * dv + e] : 0.f;
   }
+  rope_in_rows<SUMS>(a, (size_t)t0 * row_width + col, row_width, T - t0, x);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) x[k] += b;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     if (vo && t0 + k < T) vo[((size_t)(t0 + k) * a.nKV + kh) * dv + e] = (__bf16)x[k];
@@ -789,26 +833,31 @@ extern "C" int ifx_rope_append(const void* qkv, int dtype, const void* bias, int
              q_norm_w, k_norm_w, pre_norm_dtype, pre_norm_eps, extra_cols, q_mult};
   const bool extras = gate_cols || unit_norm || v_first || v_out || q_norm_w || extra_cols || q_mult;
   hipStream_t s = (hipStream_t)stream;
+  const bool in_pieces = n_slices == 0 || (slice_stride % 4 == 0 && (size_t)qkv % 16 == 0);
+#define ROPE_GO(KERNEL, BLOCKS) \
+  if (n_slices > 0) hipLaunchKernelGGL(KERNEL<true>, dim3(BLOCKS), dim3(256), 0, s, a, T, (int)qk_blocks); \
+  else hipLaunchKernelGGL(KERNEL<false>, dim3(BLOCKS), dim3(256), 0, s, a, T, (int)qk_blocks)
   // (a few tokens are quicker with one small block per token and head: nothing waits on a loop over tokens)
-  if (!extras && dv == d && T >= 128 && n_slices == 0 && dtype == DT_BF16 && rope_style == 1 && rotary_dim == d && d % 16 == 0 && (!bias || bias_dtype == DT_BF16) &&
+  if (!extras && dv == d && T >= 128 && in_pieces && dtype == DT_BF16 && rope_style == 1 && rotary_dim == d && d % 16 == 0 && (!bias || bias_dtype == DT_BF16) &&
       (!slots || page_size % 8 == 0)) {
     const size_t qk_threads = (size_t)T * (nH + (slots ? nKV : 0)) * (d / 16);
     const size_t v_threads = slots ? (size_t)((T + 7) / 8) * nKV * d : 0;
     const unsigned qk_blocks = (unsigned)((qk_threads + 255) / 256), v_blocks = (unsigned)((v_threads + 255) / 256);
-    hipLaunchKernelGGL(rope_append_vec_kernel, dim3(qk_blocks + v_blocks), dim3(256), 0, s, a, T, (int)qk_blocks);
+    ROPE_GO(rope_append_vec_kernel, qk_blocks + v_blocks);
     IFX_LAUNCH_CHECK();
   }
   const int rot = rope_style != 0 ? rotary_dim : 0;
-  if (extras && T >= 128 && n_slices == 0 && dtype == DT_BF16 && rope_style <= 1 && (d == 16 || d == 32 || d == 64 || d == 128) &&
+  if (extras && T >= 128 && in_pieces && dtype == DT_BF16 && rope_style <= 1 && (d == 16 || d == 32 || d == 64 || d == 128) &&
       rot % 16 == 0 && (nH * d + nKV * (d + dv) + gate_cols + extra_cols) % 8 == 0 && (!bias || bias_dtype == DT_BF16) &&
       (!q_norm_w || pre_norm_dtype == DT_BF16) &&
       (!slots || page_size % 8 == 0) && (slots || (!v_first && !v_out))) {
     const size_t qk_threads = (size_t)T * (nH + (slots ? nKV : 0)) * (d / 16);
     const size_t v_threads = (slots || v_out) ? (size_t)((T + 7) / 8) * nKV * dv : 0;
     const unsigned qk_blocks = (unsigned)((qk_threads + 255) / 256), v_blocks = (unsigned)((v_threads + 255) / 256);
-    hipLaunchKernelGGL(rope_append_vec_x_kernel, dim3(qk_blocks + v_blocks), dim3(256), 0, s, a, T, (int)qk_blocks);
+    ROPE_GO(rope_append_vec_x_kernel, qk_blocks + v_blocks);
     IFX_LAUNCH_CHECK();
   }
+#undef ROPE_GO
   const dim3 grid(T, nH + 2 * nKV);
   if (dtype == DT_F32) hipLaunchKernelGGL(rope_append_kernel<float>, grid, dim3(64), 0, s, a);
   else if (dtype == DT_BF16) hipLaunchKernelGGL(rope_append_kernel<bf16_t>, grid, dim3(64), 0, s, a);
