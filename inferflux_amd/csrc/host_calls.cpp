@@ -2,7 +2,7 @@
 //
 // A step that is not replayed as a graph issues 100 to 350 launches, and in Python the checks (0.47 us a tensor), the allocation (1.7),
 // the stream (0.35) and the call through ctypes (1.5 beyond the launch itself) of each took longer than most of the kernels.
-// Here: 0.1, 0.7, 0.05 and 0.3.
+// Here: 0.06, 1.5, 0.13 and 0.25.
 //
 //   check(tensor, name, shape = None, dtype = None)      nothing if the tensor is on the GPU, contiguous and as expected; anything else is
 //                                                    handed to the Python check, whose errors it raises

@@ -1612,13 +1612,15 @@ FEW_WHOLE = ((512, 1, 1024), (1024, 1, 512), (3072, 128, 256))          # the pl
 def few_tiles_plan(M: int, N: int, K: int, keep_slices: bool) -> int:
     """slices << 8 | tile of the tiles of ``gemm_tiles`` that take a model's weight [N, K] (a ``LinearWeight``) at 65 to 2,048 rows, 0: another product
     does.  Tiles of 64 x 64 and of 128 x 128 in three stages are made for these sizes, where tiles of 256 x 256 are few.  What the others take over
-    their time, geometric mean and worst, 6,700 products of cold weights with what the slices cost their reader, by M N K:
-        against the library's and large tiles', 129 rows on: up to 4e8 1.45 and 0.94, 4e8 to 1.6e9 1.6 and 0.95, 1.6e9 to 3.2e9 1.35 and 0.85 (3 % slower
-        than 0.97), 3.2e9 to 6.4e9 with K up to 4,096 1.03 and 0.66 (38 %), deeper 1.27 and 0.88 (6 %); weights of more than 8,192 rows 0.79 to 0.9
-        against the product that shares x through LDS, 65 to 128 rows: up to 8e8 1.7 and 1.08, 8e8 to 1.6e9 1.47 and 1.07, 1.6e9 to 3.2e9 with K of 4,096 to
-        8,192 1.13 and 0.81 (30 %), deeper 1.4 and 0.89
-    and, without slices, of 2,900 against the library: K up to 512 1.35 and 1.01, 512 to 1,024 1.2 and 0.84 (up to 512 tiles of 64 x 64; 18 to 24 % of more are
-    slower), 1,024 to 3,072 with 128 to 256 tiles 1.18 and 0.87 (9 %), otherwise 1.05 with a third slower.  A bare tensor goes where ``_tiles_sums_plan`` says."""
+    their time, geometric mean and worst, 16,100 products of cold weights with what the slices cost their reader, by M N K:
+        against the library's and large tiles', 129 rows on: up to 4e8 1.47 and 0.90, 4e8 to 1.6e9 1.6 and 0.72 (0.3 % below 0.97), 1.6e9 to 3.2e9 1.43 and
+        0.71 (2 %), 3.2e9 to 6.4e9 with K of 4,096 to 8,192 1.15 and 0.82 (10 %), deeper 1.40 and 0.96; beyond the lines 3.2e9 to 6.4e9 with K up to 4,096 1.03
+        and 0.66 (38 %), weights of more than 8,192 rows 0.79 to 0.9
+        against the product that shares x through LDS, 65 to 128 rows: up to 8e8 1.7 and 1.09, 8e8 to 1.6e9 1.52 and 1.04, 1.6e9 to 3.2e9 with K from 8,192 on 1.40
+        and 0.87 (8 %); beyond, with K of 4,096 to 8,192, 1.13 and 0.81 (30 %)
+        in one slice (a float sum, as the slices are) 1.42, in more 1.60
+    and, without slices, of 3,400 against the library: K up to 512 1.21 and 0.96, 512 to 1,024 1.16 and 0.84 (4 %; up to 512 tiles of 64 x 64: 18 to 24 % of more are
+    slower), 1,024 to 3,072 with 128 to 256 tiles 1.11 and 0.89 (7 %), otherwise 1.05 with a third slower.  A bare tensor goes where ``_tiles_sums_plan`` says."""
     if not (SKINNY_MAX_M < M <= FEW_MAX_ROWS and FEW_MIN_N <= N <= FEW_MAX_N and FEW_MIN_K <= K <= FEW_MAX_K) or N % 8 or K % 8:
         return 0
     if keep_slices:
@@ -1772,8 +1774,9 @@ def pairs_tiles_take(M: int, N: int, K: int) -> bool:
 def few_pairs_take(M: int, N: int, K: int) -> bool:
     """Whether that product takes a model's gate/up pairs [N, K] (a ``LinearWeight``) at 65 to 2,048 rows, where tiles by small waves are among its
     choices.  The library's product and the activation, or up to 128 rows the product that shares x through LDS, over this one's time, geometric mean
-    and worst of 7,100: up to 128 rows 2.0 and 0.90; more, K up to 1,536 1.2 to 1.7 and 0.92, 1,536 to 2,560 and up to 64 tiles of 256 x 256 1.25 and 0.84,
-    2,560 to 4,096 and 2 to 16 tiles 1.23 and 0.93 (fewer 0.96 and 0.83); 1,536 to 2,560 and more tiles 1.0, from 700 rows on 0.98 and 0.88."""
+    and worst of 8,700: up to 128 rows 2.0 and 0.88; more, K up to 1,536 and 16 tiles of 256 x 256 1.46 and 0.94 (beyond, ``many_tiles_take`` has most of them
+    anyway), 1,536 to 2,560 and up to 64 tiles 1.29 and 0.87, 2,560 to 4,096 and 2 to 16 tiles 1.24 and 0.78 (3 % below 0.97; fewer 0.96 and 0.83); 1,536 to 2,560
+    and more tiles 1.0, from 700 rows on 0.98 and 0.88."""
     if not (SKINNY_MAX_M < M <= FEW_MAX_ROWS and FEW_MIN_N <= N <= FEW_PAIRS_MAX_N and N % 4 == 0 and FEW_MIN_K <= K <= 4096 and K % 8 == 0):
         return False
     tiles = M * N / 65536
