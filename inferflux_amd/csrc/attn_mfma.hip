@@ -27,6 +27,7 @@
 // Softmax runs in float on the accumulators (base-2 exponent with the scale folded in); P is
 // rounded to bf16 for the second product, the row sum is kept in float.
 #include "common.h"
+#include "split_rows.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -338,12 +339,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // (``max_splits`` * chunk must reach past every row's position; part_o / part_ml are the partial results).
 // ``waves`` 1-8: one workgroup of that many waves per (row, kv head), which shares the row's keys evenly and writes
 // the output itself; chunk, max_splits and the scratch are not used.
+// ``merge`` 0: the merge launch is left out, whoever reads the rows joins the splits (split_rows.h).
 // ``req_is_row``: the caller knows that row_req[r] == r for every row of the step (each request brings one row).
 extern "C" int ifx_attn_rows(const void* q, const void* k_cache, const void* v_cache, void* out, const int* rows,
                              const int* row_req, const int* positions, const int* block_table, int max_blocks,
                              int n_rows, int nH, int nKV, int d, int page_size, int window, int chunk,
                              int max_splits, float scale, float* part_o, float* part_ml, int waves, int req_is_row,
-                             int keep_first, int has_sink, float sink_score, const float* gate, const float* sinks, int block, void* stream) {
+                             int keep_first, int has_sink, float sink_score, const float* gate, const float* sinks, int block, int merge,
+                             void* stream) {
   IFX_REQUIRE(d == D, "attn_rows: built for head_dim %d, called with %d", D, d);
   IFX_REQUIRE(n_rows >= 0 && nH > 0 && nKV > 0 && nH % nKV == 0, "attn_rows: bad head counts nH=%d nKV=%d", nH, nKV);
   IFX_REQUIRE(page_size > 0 && page_size % 16 == 0, "attn_rows: page_size %d must be a multiple of 16", page_size);
@@ -378,7 +381,7 @@ extern "C" int ifx_attn_rows(const void* q, const void* k_cache, const void* v_c
     if (streaming) hipLaunchKernelGGL((attn_rows_kernel<true, false>), dim3(max_splits, nKV, n_rows), dim3(WAVE), 0, s, a);
     else hipLaunchKernelGGL((attn_rows_kernel<false, false>), dim3(max_splits, nKV, n_rows), dim3(WAVE), 0, s, a);
   }
-  hipLaunchKernelGGL(attn_rows_merge_kernel, dim3(n_rows, nH), dim3(WAVE * merge_waves(max_splits)), 0, s, a);
+  if (merge) hipLaunchKernelGGL(attn_rows_merge_kernel, dim3(n_rows, nH), dim3(WAVE * merge_waves(max_splits)), 0, s, a);
   IFX_LAUNCH_CHECK();
 }
 

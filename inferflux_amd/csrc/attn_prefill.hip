@@ -28,6 +28,7 @@
 // row j of score tile t is key 32 (t / 2) + 8 (j / 4) + 4 (t % 2) + j % 4 of the 64.  V^T is then read in
 // plain 16-byte pieces of 8 consecutive keys, as the cache holds them.
 #include "common.h"
+#include "split_rows.h"
 
 IFX_DEFINE_LAST_ERROR()
 

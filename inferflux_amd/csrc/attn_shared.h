@@ -2,6 +2,7 @@
 // lanes that hold one query column, and the merge of split key ranges.
 #pragma once
 #include "common.h"
+#include "split_rows.h"      // finish_factor (includers name it, too: what they are built from is read from their own lines)
 
 #ifndef HEAD_DIM
 #error "compile with -DHEAD_DIM=<multiple of 16>"
@@ -97,25 +98,6 @@ struct RowArgs {
 __device__ __forceinline__ int first_seen(int pos, int window, int block) {
   const int lo = window > 0 ? max(0, pos - window + 1) : 0;
   return block > 0 ? max(lo, pos - pos % block) : lo;
-}
-
-// The sink joins a finished (maximum M, sum L, unnormalised output) once, where the output is written: returns the
-// factor on the output, 1 / (L + 2^(sink - M)) (times the head's gate), with care for a maximum below the sink's score.
-// ``at`` is row * nH + head; with ``sinks`` the head's own score is taken.
-__device__ __forceinline__ float finish_factor(float M, float L, int has_sink, float sink_l2, const float* gate, size_t gate_at,
-                                               const float* sinks = nullptr, int nH = 1) {
-  float f = 1.f;
-  if (sinks) {
-    has_sink = 1;
-    sink_l2 = sinks[gate_at % (size_t)nH] * 1.4426950408889634f;
-  }
-  if (has_sink) {
-    const float Ms = fmaxf(M, sink_l2);
-    f = M == -INFINITY ? 0.f : exp2f(M - Ms);
-    L = L * f + exp2f(sink_l2 - Ms);
-  }
-  const float inv = L > 0.f ? f / L : 0.f;
-  return gate ? inv * gate[gate_at] : inv;
 }
 
 // out[row, head] = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s over the row's splits, M = max m_s.

@@ -12,6 +12,7 @@
 //
 // Compile with -DK_DIM=<multiple of 8> -DV_DIM=<multiple of 16>.
 #include "common.h"
+#include "split_rows.h"
 
 IFX_DEFINE_LAST_ERROR()
 

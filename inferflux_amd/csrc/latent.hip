@@ -16,9 +16,13 @@
 //                       (the rotated query part); optionally out[t, h, n] is multiplied by sigmoid of a column of a wider
 //                       projected row, one column per output element (the output gate on W_uv's product)
 //
+//   ifx_headwise_splits the same from the row kernel's splits of attention (split_rows.h): W_uv's product of up to 16 rows
+//   ifx_latent_query    ifx_headwise of the queries and ifx_latent_finish of the latent without a query latent, in one launch
+//
 // All sums in float in ascending k, one output element per thread: a row's result does not depend on the batch.
 #include "common.h"
 #include "column_gate.h"
+#include "split_rows.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -29,18 +33,35 @@ __device__ __forceinline__ float sliced(const TY* __restrict__ y, int i, int n_s
   return v;
 }
 
-// y [T][ld], a row's first q_rank + kv_rank + rot_dim numbers (n_slices partial sums, slice_stride elements apart)
-// LF_EACH: numbers of each latent that a thread keeps in registers (wider latents are read again)
+// y [T][ld], a row's q_rank + kv_rank + rot_dim numbers from ``y`` on (n_slices partial sums, slice_stride elements apart)
+template <typename TY, typename T>
+struct FinishArgs {
+  const TY* y;
+  int n_slices;
+  size_t slice_stride;
+  const void* wq; const void* wkv;
+  int w_dtype;
+  const float* cs; const float* sn;
+  int rot_dims;
+  const int* slots;
+  T* cq; T* k_cache; T* v_cache;
+  int q_rank, kv_rank, rot_dim, page_size;
+  float eps;
+  int v_rows, ld;
+};
+
+// Row t by the workgroup's 256 threads.  LF_EACH: numbers of each latent that a thread keeps in registers (wider latents are read
+// again); ``red``: 32 floats of LDS.
 template <typename TY, typename T, int LF_EACH>
-__global__ __launch_bounds__(256) void latent_finish_kernel(const TY* __restrict__ y, int n_slices, size_t slice_stride,
-                                                            const void* __restrict__ wq, const void* __restrict__ wkv, int w_dtype,
-                                                            const float* __restrict__ cs, const float* __restrict__ sn, int rot_dims,
-                                                            const int* __restrict__ slots, T* __restrict__ cq,
-                                                            T* __restrict__ k_cache, T* __restrict__ v_cache, int q_rank,
-                                                            int kv_rank, int rot_dim, int page_size, float eps, int v_rows, int ld) {
-  __shared__ float red[32];
-  const size_t t = blockIdx.x;
-  const TY* yr = y + t * ld;
+__device__ __forceinline__ void finish_row(const FinishArgs<TY, T>& a, size_t t, float* red) {
+  const int n_slices = a.n_slices, rot_dims = a.rot_dims, q_rank = a.q_rank, kv_rank = a.kv_rank, rot_dim = a.rot_dim, page_size = a.page_size;
+  const int v_rows = a.v_rows, w_dtype = a.w_dtype;
+  const size_t slice_stride = a.slice_stride;
+  const float eps = a.eps, *cs = a.cs, *sn = a.sn;
+  const int* slots = a.slots;
+  const void *wq = a.wq, *wkv = a.wkv;
+  T *cq = a.cq, *k_cache = a.k_cache, *v_cache = a.v_cache;
+  const TY* yr = a.y + t * a.ld;
   const TY* yc = yr + q_rank;
   const TY* yk = yc + kv_rank;
   const int slot = slots ? slots[t] : -1, half = rot_dims / 2, tid = threadIdx.x;
@@ -126,6 +147,12 @@ __global__ __launch_bounds__(256) void latent_finish_kernel(const TY* __restrict
   }
 }
 
+template <typename TY, typename T, int LF_EACH>
+__global__ __launch_bounds__(256) void latent_finish_kernel(FinishArgs<TY, T> a) {
+  __shared__ float red[32];
+  finish_row<TY, T, LF_EACH>(a, blockIdx.x, red);
+}
+
 extern "C" int ifx_latent_finish(const void* y, int y_dtype, int n_slices, long long slice_stride, const void* wq, const void* wkv,
                                  int w_dtype, const float* cs, const float* sn, int rot_dims, const int* slots, void* cq,
                                  void* k_cache, void* v_cache, int dtype, int T, int q_rank, int kv_rank, int rot_dim,
@@ -149,8 +176,9 @@ extern "C" int ifx_latent_finish(const void* y, int y_dtype, int n_slices, long 
     else LF_GO(TY, TT, 6);                                               \
   } while (0)
 #define LF_GO(TY, TT, EACH) \
-  hipLaunchKernelGGL((latent_finish_kernel<TY, TT, EACH>), dim3(T), dim3(256), 0, s, (const TY*)y, n_slices, (size_t)slice_stride, wq, wkv, \
-                     w_dtype, cs, sn, rot_dims, slots, (TT*)cq, (TT*)k_cache, (TT*)v_cache, q_rank, kv_rank, rot_dim, page_size, eps, v_rows, ld)
+  hipLaunchKernelGGL((latent_finish_kernel<TY, TT, EACH>), dim3(T), dim3(256), 0, s,                                                          \
+                     FinishArgs<TY, TT>{(const TY*)y, n_slices, (size_t)slice_stride, wq, wkv, w_dtype, cs, sn, rot_dims, slots, (TT*)cq,       \
+                                        (TT*)k_cache, (TT*)v_cache, q_rank, kv_rank, rot_dim, page_size, eps, v_rows, ld})
   if (y_dtype == DT_F32 && dtype == DT_F32) LF_LAUNCH(float, float);
   else if (y_dtype == DT_F32 && dtype == DT_BF16) LF_LAUNCH(float, bf16_t);
   else if (y_dtype == DT_BF16 && dtype == DT_BF16) LF_LAUNCH(bf16_t, bf16_t);
@@ -247,8 +275,7 @@ __device__ __forceinline__ void hw_load8(const float* p, float* v) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void headwise_rows_kernel(HeadwiseArgs a) {
-  const int t = blockIdx.x, h = blockIdx.y, n = blockIdx.z * 256 + threadIdx.x;
+__device__ __forceinline__ void headwise_row(const HeadwiseArgs& a, int t, int h, int n) {
   const int out_head = a.N + a.tail;
   const T* xt = (const T*)a.x + (size_t)t * a.x_row + (size_t)h * a.x_head;
   T* out = (T*)a.out + ((size_t)t * a.H + h) * out_head;
@@ -275,6 +302,55 @@ __global__ __launch_bounds__(256) void headwise_rows_kernel(HeadwiseArgs a) {
     }
     out[n] = from_f<T>(v);
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void headwise_rows_kernel(HeadwiseArgs a) {
+  headwise_row<T>(a, blockIdx.x, blockIdx.y, blockIdx.z * 256 + threadIdx.x);
+}
+
+// The queries' side of a step and the cache's, which do not need each other: workgroups (row, head) for the product, and one a row
+// behind them for ``finish_row``.  Bound by the launch and a chain of two trips: one row of 16 heads 4.0 us, apart 4.6 and 4.6.
+template <int LF_EACH>
+__global__ __launch_bounds__(256) void latent_query_kernel(HeadwiseArgs a, FinishArgs<bf16_t, bf16_t> f) {
+  __shared__ float red[32];
+  if ((int)blockIdx.y < a.H) headwise_row<bf16_t>(a, blockIdx.x, blockIdx.y, blockIdx.z * 256 + threadIdx.x);
+  else if (blockIdx.z == 0) finish_row<bf16_t, bf16_t, LF_EACH>(f, blockIdx.x, red);
+}
+
+// W_uv's product from attention's splits: a workgroup's four waves join a head's splits (in float, no rounding between) while the
+// weights, a thread its whole row, are on their way.  Bound by its launch and one trip to memory: 8 rows of 16 heads in 16 splits 4.8 us, where
+// the launch that joined them took 5.1 and the product from rows 4.7.
+__global__ __launch_bounds__(256) void headwise_splits_kernel(HeadwiseArgs a, SplitRows p) {
+  typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+  __shared__ __attribute__((aligned(16))) float xs[SPLITS_MAX_WIDTH];
+  __shared__ float sums[4][SPLITS_MAX_WIDTH];
+  const int t = blockIdx.x, h = blockIdx.y, n = blockIdx.z * 256 + threadIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const size_t at = (size_t)t * a.H + h;
+  SplitMerge<4> m;
+  m.ask(p, at, a.K, wave, lane);
+  const bf16_t* w = (const bf16_t*)a.w + ((size_t)h * a.N + min(n, a.N - 1)) * a.K;
+  bf16x8 wv[SPLITS_MAX_WIDTH / 8];
+#pragma unroll
+  for (int i = 0; i < SPLITS_MAX_WIDTH / 8; ++i) wv[i] = *(const bf16x8*)(w + min(8 * i, a.K - 8));
+  const float gate = a.gate.rows && n < a.N ? a.gate.at<bf16_t>(t, h * a.N + n) : 1.f;
+  const float inv = m.weigh(p, at, a.H);
+  m.sums(wave, sums[wave], lane);
+  __syncthreads();
+  const int e = threadIdx.x;
+  if (e < SPLITS_MAX_WIDTH) xs[e] = ((sums[0][e] + sums[1][e]) + (sums[2][e] + sums[3][e])) * inv;
+  __syncthreads();
+  if (n >= a.N) return;
+  float y = 0.f;
+#pragma unroll
+  for (int i = 0; i < SPLITS_MAX_WIDTH / 8; ++i)
+    if (8 * i < a.K) {
+      float x[8];
+      hw_load8(xs + 8 * i, x);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y = fmaf(x[j], (float)wv[i][j], y);
+    }
+  ((bf16_t*)a.out)[at * a.N + n] = (bf16_t)(y * gate);
 }
 
 #define HW_ROWS_MAX_T 16
@@ -306,5 +382,41 @@ extern "C" int ifx_headwise(const void* x, const void* w, void* out, int dtype, 
   if (dtype == DT_F32) hipLaunchKernelGGL(headwise_kernel<float>, grid, dim3(256), 0, s, a);
   else if (dtype == DT_BF16) hipLaunchKernelGGL(headwise_kernel<bf16_t>, grid, dim3(256), 0, s, a);
   else IFX_FAIL("headwise: unknown dtype %d", dtype);
+  IFX_LAUNCH_CHECK();
+}
+
+extern "C" int ifx_headwise_splits(const float* part_o, const float* part_ml, const float* sinks, int splits, int D, const void* w, void* out, int T,
+                                   int H, int K, int N, const void* gate, int gate_ld, int gate_col, int gate_slices, long long gate_stride, void* stream) {
+  IFX_REQUIRE(T >= 0 && T <= HW_ROWS_MAX_T && H > 0 && H <= 65535 && N > 0, "headwise_splits: bad sizes T=%d H=%d N=%d", T, H, N);
+  IFX_REQUIRE(K > 0 && K % 8 == 0 && K <= SPLITS_MAX_WIDTH && K <= D, "headwise_splits: K=%d (a multiple of 8 up to %d) of heads of %d", K, SPLITS_MAX_WIDTH, D);
+  IFX_REQUIRE(part_o && part_ml && splits > 0 && splits <= SPLITS_MAX, "headwise_splits: %d splits (1-%d)", splits, SPLITS_MAX);
+  IFX_REQUIRE(!gate || (gate_col >= 0 && gate_col + H * N <= gate_ld && gate_slices >= 0), "headwise_splits: %d gates from column %d on do not fit rows of %d", H * N, gate_col, gate_ld);
+  if (T == 0) return 0;
+  HeadwiseArgs a{nullptr, w, out, nullptr, nullptr, T, H, K, N, 0, 0, 0, 0, ColumnGate{gate, gate_ld, gate_col, gate_slices, (size_t)gate_stride}, 0};
+  hipLaunchKernelGGL(headwise_splits_kernel, dim3(T, H, (N + 255) / 256), dim3(256), 0, (hipStream_t)stream, a, SplitRows{part_o, part_ml, sinks, splits, D});
+  IFX_LAUNCH_CHECK();
+}
+
+// x [T][x_row]: the queries; y [T][ld]: a row's kv_rank + rot_dim numbers, the latent and the key part (columns of the same rows or of others).
+extern "C" int ifx_latent_query(const void* x, int x_row, const void* y, int ld, const void* w, void* out, int T, int H, int K, int N, int x_head,
+                                int tail, const float* cs, const float* sn, int rot_dims, const void* wkv, int w_dtype, const int* slots,
+                                void* k_cache, void* v_cache, int kv_rank, int rot_dim, int page_size, float eps, int v_rows, void* stream) {
+  IFX_REQUIRE(T >= 0 && T <= HW_ROWS_MAX_T && H > 0 && H < 65535 && K > 0 && N > 0 && tail >= 0 && x_head >= K + tail, "latent_query: bad sizes T=%d H=%d K=%d N=%d tail=%d", T, H, K, N, tail);
+  IFX_REQUIRE(K % 8 == 0 && x_head % 8 == 0 && x_row % 8 == 0 && (uintptr_t)x % 16 == 0, "latent_query: K=%d, heads of %d and rows of %d must be multiples of 8", K, x_head, x_row);
+  IFX_REQUIRE(x_row >= (H - 1) * x_head + K + tail, "latent_query: the heads do not fit the rows of x");
+  IFX_REQUIRE(kv_rank > 0 && rot_dim >= 0 && kv_rank <= 1536 && ld >= kv_rank + rot_dim, "latent_query: rows of %d are too short", ld);
+  IFX_REQUIRE(rot_dims >= 0 && rot_dims % 2 == 0 && rot_dims <= rot_dim && rot_dims <= tail, "latent_query: %d of %d dimensions rotate", rot_dims, rot_dim);
+  IFX_REQUIRE(rot_dims == 0 || (cs && sn), "latent_query: a rotation needs its table");
+  IFX_REQUIRE(slots && k_cache && v_cache && page_size > 0, "latent_query: no cache");
+  IFX_REQUIRE(v_rows == kv_rank || v_rows == kv_rank + rot_dim, "latent_query: values of %d rows (the latent's %d, or %d with the key part)", v_rows, kv_rank, kv_rank + rot_dim);
+  IFX_REQUIRE(w_dtype == DT_F32 || w_dtype == DT_BF16, "latent_query: unknown weight dtype %d", w_dtype);
+  if (T == 0) return 0;
+  HeadwiseArgs a{x, w, out, cs, sn, T, H, K, N, x_row, x_head, tail, rot_dims, ColumnGate{nullptr, 0, 0, 0, 0}, 0};
+  FinishArgs<bf16_t, bf16_t> f{(const bf16_t*)y, 1, 0, nullptr, wkv, w_dtype, cs, sn, rot_dims, slots, nullptr, (bf16_t*)k_cache,
+                               (bf16_t*)v_cache, 0, kv_rank, rot_dim, page_size, eps, v_rows, ld};
+  const dim3 grid(T, H + 1, (N + tail + 255) / 256);
+  if (kv_rank <= 256) hipLaunchKernelGGL(latent_query_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, a, f);
+  else if (kv_rank <= 512) hipLaunchKernelGGL(latent_query_kernel<2>, grid, dim3(256), 0, (hipStream_t)stream, a, f);
+  else hipLaunchKernelGGL(latent_query_kernel<6>, grid, dim3(256), 0, (hipStream_t)stream, a, f);
   IFX_LAUNCH_CHECK();
 }

@@ -10,9 +10,10 @@
 //   diff_expand    q [T][H][2 d] -> [T][2 H][2 d]: head 2 h holds [q1 | 0] and head 2 h + 1 holds [0 | q2], so that attention
 //                  kernels for heads of 2 d elements score each half against its half of the keys' rows [k1 | k2]
 //   diff_combine   out[t, h, :] = o / sqrt(mean(o^2) + eps) * out_scale with o = a[t, 2 h, :] - lambda a[t, 2 h + 1, :]: the two
-//                  maps of differential attention joined, a wave per (row, head)
+//                  maps of differential attention joined, a wave per (row, head); from the row kernel's splits a workgroup each
 // All arithmetic is float.
 #include "common.h"
+#include "split_rows.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -330,5 +331,45 @@ extern "C" int ifx_diff_combine(const void* a, void* out, int dtype, long long r
   else if (dtype == DT_F32)
     hipLaunchKernelGGL(diff_combine_kernel<float>, dim3(blocks), dim3(256), 0, s, (const float*)a, (float*)out, (size_t)rows_heads, dv, lambda, out_scale, eps);
   else IFX_FAIL("diff_combine: unknown dtype %d", dtype);
+  IFX_LAUNCH_CHECK();
+}
+
+// The same with the two maps' outputs still in the row kernel's splits (map c of head h is head 2 h + c of the partial results, p.D = dv
+// wide): two waves join each map's, and all four meet once, in float.  One row of 16 heads in 16 splits 4.2 us, as a launch that joins and one that
+// combines 5.2 + 4.8.
+__global__ __launch_bounds__(256) void diff_combine_splits_kernel(SplitRows p, bf16_t* __restrict__ out, int H, float lambda, float out_scale,
+                                                                  float eps) {
+  __shared__ float sums[4][SPLITS_MAX_WIDTH];
+  __shared__ float factor[2];
+  const int t = blockIdx.x, h = blockIdx.y, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, map = wave / 2, w = wave % 2;
+  const size_t at = ((size_t)t * H + h) * 2 + map;
+  SplitMerge<2> m;
+  m.ask(p, at, p.D, w, lane);
+  const float inv = m.weigh(p, at, 2 * H);
+  if (w == 0 && lane == 0) factor[map] = inv;
+  m.sums(w, sums[wave], lane);
+  __syncthreads();
+  if (wave > 0) return;
+  constexpr int C = SPLITS_MAX_WIDTH / WAVE;
+  float o[C], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int e = lane + WAVE * c;
+    o[c] = (sums[0][e] + sums[1][e]) * factor[0] - lambda * ((sums[2][e] + sums[3][e]) * factor[1]);      // (past dv: zeros)
+    ss = fmaf(o[c], o[c], ss);
+  }
+  const float f = out_scale / sqrtf(wave_sum(ss) / (float)p.D + eps);
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    if (lane + WAVE * c < p.D) out[((size_t)t * H + h) * p.D + lane + WAVE * c] = (bf16_t)(o[c] * f);
+}
+
+extern "C" int ifx_diff_combine_splits(const float* part_o, const float* part_ml, int splits, void* out, int T, int H, int dv, float lambda,
+                                       float out_scale, float eps, void* stream) {
+  IFX_REQUIRE(part_o && part_ml && splits > 0 && splits <= SPLITS_MAX, "diff_combine: %d splits (1-%d)", splits, SPLITS_MAX);
+  IFX_REQUIRE(T >= 0 && H > 0 && H <= 65535 && dv > 0 && dv <= SPLITS_MAX_WIDTH, "diff_combine: T=%d H=%d dv=%d (at most %d)", T, H, dv, SPLITS_MAX_WIDTH);
+  if (T == 0) return 0;
+  hipLaunchKernelGGL(diff_combine_splits_kernel, dim3(T, H), dim3(256), 0, (hipStream_t)stream, SplitRows{part_o, part_ml, nullptr, splits, dv},
+                     (bf16_t*)out, H, lambda, out_scale, eps);
   IFX_LAUNCH_CHECK();
 }

@@ -328,8 +328,9 @@ def plain_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
 
 def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: float, keep_first: int = 0,
                     sink: Optional[float] = None, gate: Optional[torch.Tensor] = None,
-                    sinks: Optional[torch.Tensor] = None, block: Optional[int] = None) -> torch.Tensor:
-    """q [T, nH, d] of this step's rows against ``cache`` (a LayerCache); returns [T, nH*d].  ``keep_first``: the first
+                    sinks: Optional[torch.Tensor] = None, block: Optional[int] = None, keep_splits: bool = False):
+    """q [T, nH, d] of this step's rows against ``cache`` (a LayerCache); returns [T, nH*d], with ``keep_splits`` also ``SplitRows`` (where
+    one launch has all rows in splits).  ``keep_first``: the first
     positions a windowed query sees beside its window; ``sink``: the score of a key without value in the softmax's
     denominator (None: none), ``sinks`` float32 [nH]: such a score for every head; ``gate`` float32
     [T, nH]: a factor on every head's output; ``block``: a row sees only the keys of its own block of that many positions,
@@ -365,13 +366,14 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
 
     # (once a step for all layers of a kind)
     qt, w = ctx.derived(("attention_plan", n_kv, nH, d, window, keep_first, block), plan)
-    out = ops.empty((T, nH * d), q.dtype, q)
+    left = keep_splits and w["waves"] == 0 and w["n_rows"] == T > 0 and w["max_splits"] <= ops.SPLITS_READ_MAX and sink is None and gate is None
+    out = None if left else ops.empty((T, nH * d), q.dtype, q)
     more = dict(keep_first=keep_first, sink=sink, gate=gate, sinks=sinks, block=block) if extras else {}
     if w["n_tiles"]:
         ops.attention_tiles(q, cache.k, cache.v, out, w["tile_req"], w["tile_q0"], ctx.q_start, ctx.q_len, ctx.kv_len,
                             table, window, scale, qt, w["tile_chunk"], w["tile_splits"], w["tile_row_list"], ctx.row_req,
                             ctx.positions, w["tile_order"], **more)
     if w["n_rows"]:
-        ops.attention_rows(q, cache.k, cache.v, out, w["rows"], w["n_rows"], ctx.row_req, ctx.positions, table,
-                           window, scale, w["chunk"], w["max_splits"], w["waves"], ctx.n_tokens == ctx.n_requests, **more)
-    return out
+        splits = ops.attention_rows(q, cache.k, cache.v, out, w["rows"], w["n_rows"], ctx.row_req, ctx.positions, table,
+                                    window, scale, w["chunk"], w["max_splits"], w["waves"], ctx.n_tokens == ctx.n_requests, **more)
+    return splits if left else out

@@ -530,19 +530,64 @@ def latent_finish(y, q_norm: Optional[torch.Tensor], kv_norm: Optional[torch.Ten
     return cq
 
 
+LATENT_QUERY_MAX_RANK = 1536
+
+
+def latent_query_takes(T: int, dtype: torch.dtype, dim: int, rot_dim: int, kv_rank: int) -> bool:
+    """Whether ``latent_query`` takes a step of ``T`` rows."""
+    return (dtype == torch.bfloat16 and 0 < T <= HEADWISE_ROWS_MAX and dim % 8 == 0 and (dim + rot_dim) % 8 == 0 and (kv_rank + rot_dim) % 8 == 0
+            and kv_rank <= LATENT_QUERY_MAX_RANK)
+
+
+def latent_query(y: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, kv_norm: torch.Tensor, eps: float,
+                 cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], rot_dims: int, slots: torch.Tensor, kv_rank: int, rot_dim: int,
+                 k_cache: torch.Tensor, v_cache: torch.Tensor, page_size: int) -> torch.Tensor:
+    """``headwise`` of the queries (a tail of ``rot_dim`` elements behind each head's) and ``latent_finish`` of the latent in one launch, for
+    steps of few rows (``latent_query_takes``): ``y`` [T, n_heads * x_head + kv_rank + rot_dim] in bfloat16 holds both side by side."""
+    T, width = y.shape
+    n_q = n_heads * x_head
+    _check(y, "y", (None, n_q + kv_rank + rot_dim), torch.bfloat16)
+    _check(weight, "weight", (n_heads, None, None), y.dtype)
+    _, N, K = weight.shape
+    if not latent_query_takes(T, y.dtype, K, x_head - K, kv_rank) or x_head != K + rot_dim:
+        raise KernelError(f"latent_query: {T} rows (1-{HEADWISE_ROWS_MAX}) of {n_heads} heads of {K} + {x_head - K}, a latent of {kv_rank}")
+    _check(kv_norm, "kv_norm", (kv_rank,))
+    if rot_dims:
+        _check(cos, "cos", (T, rot_dims // 2), torch.float32)
+        _check(sin, "sin", (T, rot_dims // 2), torch.float32)
+    _check(slots, "slots", (T,), torch.int32)
+    _check(k_cache, "k_cache", (None, 1, page_size, kv_rank + rot_dim), y.dtype)
+    _check(v_cache, "v_cache", (k_cache.shape[0], 1, None, page_size), y.dtype)
+    out = empty((T, n_heads, N + rot_dim), y.dtype, y)
+    _call(load_module("latent"), "ifx_latent_query", (P, I, P, I, P, P, I, I, I, I, I, I, P, P, I, P, I, P, P, P, I, I, I, F, I, P),
+          y, width, y.data_ptr() + 2 * n_q, width, weight, out, T, n_heads, K, N, x_head, rot_dim, cos if rot_dims else None,
+          sin if rot_dims else None, rot_dims, kv_norm, _dt(kv_norm), slots, k_cache, v_cache, kv_rank, rot_dim, page_size, float(eps),
+          v_cache.shape[2], _stream())
+    return out
+
+
+HEADWISE_ROWS_MAX = 16             # rows of a step up to which a thread forms an output element by itself
 HEADWISE_GROUPED_MIN_ROWS = 32     # rows of a step from which the per-head products go to the matrix cores
 
 
-def headwise(x: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, tail: int = 0,
+def headwise_takes_splits(T: int, K: int) -> bool:
+    """Whether ``headwise`` takes ``SplitRows`` of ``T`` rows (``K`` elements of each head)."""
+    return 0 < T <= HEADWISE_ROWS_MAX and K % 8 == 0 and K <= MFMA_MAX_HEAD_DIM
+
+
+def headwise(x, weight: torch.Tensor, n_heads: int, x_head: int, tail: int = 0,
              cos: Optional[torch.Tensor] = None, sin: Optional[torch.Tensor] = None, rot_dims: int = 0,
              gate: Optional[Tuple[object, int]] = None) -> torch.Tensor:
     """A product per head: out[t, h, :N] = ``weight``[h] x[t, h] with ``weight`` [H, N, K] and head h's input the K
     elements of row t of ``x`` [T, >= H * x_head] from h * x_head on.  The ``tail`` elements that follow a head's K
     inputs are appended to its output, the first ``rot_dims`` of them turned by the table ``cos`` / ``sin``
     [T, rot_dims / 2] in split-half pairs.  ``gate`` = (rows, column): out[t, h, n] is multiplied by the sigmoid of column
-    column + h * N + n of ``rows`` [T, ld] (x's type, or ``SliceSums``), in float.  Returns [T, H, N + tail] in x's type; sums in
+    column + h * N + n of ``rows`` [T, ld] (x's type, or ``SliceSums``), in float.  ``x`` may be attention's ``SplitRows`` (without a tail;
+    see ``headwise_takes_splits``), which are joined in float.  Returns [T, H, N + tail] in x's type; sums in
     float."""
-    _check(x, "x", (None, None))
+    splits = x if isinstance(x, SplitRows) else None
+    if splits is None:
+        _check(x, "x", (None, None))
     T = x.shape[0]
     _check(weight, "weight", (n_heads, None, None), x.dtype)
     _, N, K = weight.shape
@@ -551,7 +596,7 @@ def headwise(x: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, t
     if rot_dims:
         _check(cos, "cos", (T, rot_dims // 2), torch.float32)
         _check(sin, "sin", (T, rot_dims // 2), torch.float32)
-    out = empty((T, n_heads, N + tail), x.dtype, x)
+    out = empty((T, n_heads, N + tail), x.dtype, weight)
     gate_args = (0, 0, 0, 0, 0)
     if gate is not None:
         rows, col = gate
@@ -564,6 +609,12 @@ def headwise(x: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, t
             gate_args = (rows.data_ptr(), rows.shape[1], int(col), 0, 0)
         if col < 0 or col + n_heads * N > gate_args[1]:
             raise KernelError(f"headwise: {n_heads * N} gates from column {col} on do not fit rows of {gate_args[1]}")
+    if splits is not None:
+        if tail or splits.n_heads != n_heads or splits.width != x_head or not headwise_takes_splits(T, K):
+            raise KernelError(f"headwise: splits of {splits.n_heads} heads of {splits.width} where {n_heads} of {x_head} (K={K}, {T} rows) are read")
+        _call(load_module("latent"), "ifx_headwise_splits", (P, P, P, I, I, P, P, I, I, I, I, P, I, I, I, LL, P),
+              splits.part_o, splits.part_ml, splits.sinks, splits.n_splits, splits.width, weight, out, T, n_heads, K, N, *gate_args, _stream())
+        return out
     tail_only = 0
     if x.dtype == torch.bfloat16 and T >= HEADWISE_GROUPED_MIN_ROWS and K % 8 == 0 and x_head % 8 == 0 and x.shape[1] % 8 == 0:
         # many rows: the products on the matrix cores, and of the other kernel only the tails
@@ -1137,6 +1188,29 @@ class DeltaSum:
         for v, s in self.terms:
             out += (v.sum(torch.float32) if isinstance(v, SliceSums) else v.float()) * s
         return out
+
+
+class SplitRows:
+    """Attention of a step of single rows [T, n_heads * width] (bfloat16) whose splits of the keys its reader joins: ``part_o`` float32
+    [T, n_heads, splits, width] and ``part_ml`` [T, n_heads, splits, 2] as ``attention_rows`` leaves them, ``sinks`` float32 [n_heads] (or None) a
+    score per head that joins the softmax's denominator.  ``headwise`` and ``diff_combine`` take it, which saves the launch that would join them."""
+
+    __slots__ = ("part_o", "part_ml", "sinks")
+    dtype = torch.bfloat16
+
+    def __init__(self, part_o: torch.Tensor, part_ml: torch.Tensor, sinks: Optional[torch.Tensor] = None):
+        self.part_o, self.part_ml, self.sinks = part_o, part_ml, sinks
+
+    n_heads = property(lambda self: self.part_o.shape[1])
+    n_splits = property(lambda self: self.part_o.shape[2])
+    width = property(lambda self: self.part_o.shape[3])
+
+    @property
+    def shape(self):
+        return torch.Size((self.part_o.shape[0], self.part_o.shape[1] * self.part_o.shape[3]))
+
+
+SPLITS_READ_MAX = 32        # splits of a row that the readers of SplitRows take
 
 
 class SliceSums:
@@ -2052,9 +2126,16 @@ def diff_expand(q: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def diff_combine(a: torch.Tensor, n_heads: int, dv: int, lam: float, out_scale: float, eps: float) -> torch.Tensor:
-    """a [T, 2 H dv] (per head the two maps' outputs, one after the other) -> [T, H dv]: o = a1 - lam a2, divided by its root
-    mean square over dv (eps inside the root), times out_scale."""
+def diff_combine(a, n_heads: int, dv: int, lam: float, out_scale: float, eps: float) -> torch.Tensor:
+    """a [T, 2 H dv] (per head the two maps' outputs, one after the other; also ``SplitRows``) -> [T, H dv]: o =
+    a1 - lam a2, divided by its root mean square over dv (eps inside the root), times out_scale."""
+    if isinstance(a, SplitRows):
+        if a.n_heads != 2 * n_heads or a.width != dv or a.sinks is not None:
+            raise KernelError(f"diff_combine: splits of {a.n_heads} heads of {a.width} where two maps of {n_heads} of {dv} are joined")
+        out = empty((a.shape[0], n_heads * dv), a.dtype, a.part_o)
+        _call(load_module("rowwise"), "ifx_diff_combine_splits", (P, P, I, P, I, I, I, F, F, F, P), a.part_o, a.part_ml, a.n_splits, out, a.shape[0],
+              n_heads, dv, float(lam), float(out_scale), float(eps), _stream())
+        return out
     _check(a, "a", (None, 2 * n_heads * dv))
     T = a.shape[0]
     out = empty((T, n_heads * dv), a.dtype, a)
@@ -2777,9 +2858,10 @@ def attention_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
                    rows: Optional[torch.Tensor], n_rows: int, row_req: torch.Tensor, positions: torch.Tensor,
                    block_table: torch.Tensor, window: Optional[int], scale: float, chunk: int, max_splits: int,
                    waves: int = 0, req_is_row: bool = False, keep_first: int = 0, sink: Optional[float] = None,
-                   gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, block: Optional[int] = None) -> None:
+                   gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, block: Optional[int] = None) -> Optional["SplitRows"]:
     """Attention of single rows (``rows`` int32, or None for rows 0..n_rows-1) into ``out`` [T, nH*d].  ``keep_first``,
-    ``sink``, ``gate``: as for ``attention_plain``.
+    ``sink``, ``gate``: as for ``attention_plain``.  Without ``out`` (every row, in splits, no ``sink`` and no ``gate``) the splits are left
+    to the reader and returned.
 
     ``waves`` 0: split s of a row covers key positions [s*chunk, (s+1)*chunk), one wave each, and a second launch
     merges a row's splits; ``max_splits`` * chunk must reach past the largest position among the rows.
@@ -2788,7 +2870,10 @@ def attention_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     ``req_is_row``: the caller vouches that ``row_req`` is 0, 1, 2, ... (every request brings one row), which lets
     a wave ask for its block-table entries before it knows anything else."""
     T, nH, d, nKV, page_size, mod = _attn_common(q, k_cache, v_cache)
-    _check(out, "out", (T, nH * d), torch.bfloat16)
+    if out is not None:
+        _check(out, "out", (T, nH * d), torch.bfloat16)
+    elif rows is not None or waves or sink is not None or gate is not None or not 0 < max_splits <= SPLITS_READ_MAX:
+        raise KernelError(f"attention_rows: {max_splits} splits are not left to the reader (1-{SPLITS_READ_MAX} of every row, no sink, no gate)")
     _check(row_req, "row_req", (T,), torch.int32)
     _check(positions, "positions", (T,), torch.int32)
     _check(block_table, "block_table", (None, None), torch.int32)
@@ -2805,11 +2890,12 @@ def attention_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
         part_ml = empty((n_rows, nH, max_splits, 2), torch.float32, q)
     if req_is_row and block_table.shape[0] < T:
         raise KernelError("attention_rows: req_is_row needs a block-table row for every row of the step")
-    _call(mod, "ifx_attn_rows", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, I, I, I, I, F, P, P, I, P),
+    _call(mod, "ifx_attn_rows", (P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, I, I, I, I, F, P, P, I, I, P),
           q, k_cache, v_cache, out, rows, row_req,
           positions, block_table, block_table.shape[1], n_rows, nH, nKV, d, page_size,
           int(window or 0), chunk, max_splits, float(scale), part_o, part_ml, waves, 1 if req_is_row else 0,
-          *_attn_extras(T, nH, keep_first, sink, gate, sinks, block), _stream())
+          *_attn_extras(T, nH, keep_first, sink, gate, sinks, block), 0 if out is None else 1, _stream())
+    return SplitRows(part_o, part_ml, sinks) if out is None else None
 
 
 def attention_tile_rows(head_dim: int, qt: int = 1) -> int:

@@ -222,7 +222,7 @@ class PagedAttention(Mixer):
             # Values as wide as both maps' keys together: each map becomes a head of its own whose query is padded with
             # zeros over the other map's half, which the matrix-core kernels score against the keys' whole rows; a small
             # kernel joins the two outputs.
-            a = paged_attention(ops.diff_expand(q), cache, ctx, self.window, self.scale, block=self.chunk)
+            a = paged_attention(ops.diff_expand(q), cache, ctx, self.window, self.scale, block=self.chunk, keep_splits=True)
             return ops.diff_combine(a, self.n_heads, self.v_head_dim, lam, out_scale, eps)
         # any other sizes, and 32-bit: the kernels that know two maps, float math
         return plain_attention(q, cache, ctx, self.window, self.scale, self.keep_first, self.sink, gate, block=self.chunk,

@@ -78,7 +78,7 @@ class LatentAttention(Mixer):
         self.position = build_part("position", position)
         if self.position.needs_apply:
             raise ValueError(f"{name}: latent attention needs a position part that gives the kernels a rotation table")
-        self.w_down = self.w_uq = self.w_uk_t = self.w_uv = self.w_o = self.q_norm = self.kv_norm = None
+        self.w_few = self.w_down = self.w_uq = self.w_uk_t = self.w_uv = self.w_o = self.q_norm = self.kv_norm = None
 
     @property
     def key_width(self) -> int:
@@ -138,8 +138,13 @@ class LatentAttention(Mixer):
             w_q = torch.cat([w_q[:, :self.dim], w_q[:, self.dim:][:, order]], dim=1).reshape(nh * (self.dim + self.rot_dim), -1).contiguous()
             w_dkv = torch.cat([w_dkv[:self.kv_rank], w_dkv[self.kv_rank:][order]], dim=0).contiguous()
         down = [tensors[f"{n}.dq"] if self.q_rank else None, w_dkv, tensors[f"{n}.g"] if self.output_gate else None]
-        self.w_down = ops.prepare_linear(concat_weights([w for w in down if w is not None]))
-        self.w_uq = ops.prepare_linear(w_q)
+        down = concat_weights([w for w in down if w is not None])
+        self.w_few = None
+        if w_q.is_cuda and not (self.q_rank or self.output_gate) and down.dtype == w_q.dtype == torch.bfloat16 and self.hidden_size % 8 == 0:
+            # queries and latent as one product, for steps of few rows (its rows are the two weights' own)
+            self.w_few = ops.prepare_linear(torch.cat([w_q, down]))
+            w_q, down = self.w_few.rows[:w_q.shape[0]], self.w_few.rows[w_q.shape[0]:]
+        self.w_down, self.w_uq = ops.prepare_linear(down), ops.prepare_linear(w_q)
         if self.sinks:
             self.sink_scores = tensors[f"{n}.sink"].float().contiguous()        # scores are float whatever the file holds
         self.w_o = ops.prepare_linear(tensors[f"{n}.o"])
@@ -167,19 +172,20 @@ class LatentAttention(Mixer):
         T, nh, t, dtype = h.shape[0], self.n_heads, ctx.timer, h.dtype
         _, rot_dims, cos, sin = self.position.kernel_args(ctx)
         slots = None if self.shared_latent else ctx.write_slots(cache.group)
-        y = ops.linear(h, self.w_down, keep_slices=True)              # [T, q_rank + kv_rank + rot_dim + gate]
+        few = self.w_few is not None and h.dtype == cache.k.dtype and ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank)
+        y = None if few else ops.linear(h, self.w_down, keep_slices=True)     # [T, q_rank + kv_rank + rot_dim + gate]
         if isinstance(y, ops.SliceSums) and y.parts.shape[0] > SLICES_READ_TWICE:
             y = ops.SliceSums(y.sum(torch.float32)[None], y.dtype)    # (still float, added up by the whole chip)
-        cq = ops.latent_finish(y, self.q_norm, self.kv_norm, self.eps, cos, sin, rot_dims, slots, self.q_rank, self.kv_rank,
-                               self.rot_dim, cache.k, cache.v, cache.page_size, dtype)
-        q = ops.linear(cq if self.q_rank else h, self.w_uq)           # [T, heads (dim + rot_dim)]
-        w_dtype = self.w_uk_t.dtype
-        qa = ops.headwise(q if q.dtype == w_dtype else q.to(w_dtype), self.w_uk_t, nh, self.dim + self.rot_dim, self.rot_dim,
-                          cos, sin, rot_dims)                         # [T, heads, key_width]
+        if few:
+            qa = ops.latent_query(ops.linear(h, self.w_few), self.w_uk_t, nh, self.dim + self.rot_dim, self.kv_norm, self.eps, cos, sin, rot_dims,
+                                  slots, self.kv_rank, self.rot_dim, cache.k, cache.v, cache.page_size)
+        else:
+            qa = self._queries(h, y, cache, slots, cos, sin, rot_dims)        # [T, heads, key_width]
         if t is not None:
             t.mark("mixer.qkv")
-        a = paged_attention(qa if qa.dtype == dtype else qa.to(dtype), cache, ctx, self.window, self.scale,
-                            sinks=self.sink_scores)                    # [T, heads value_width]
+        w_dtype = self.w_uv.dtype
+        a = paged_attention(qa if qa.dtype == dtype else qa.to(dtype), cache, ctx, self.window, self.scale, sinks=self.sink_scores,
+                            keep_splits=w_dtype == dtype and ops.headwise_takes_splits(T, self.kv_rank))     # [T, heads value_width]
         if t is not None:
             t.mark("mixer.attention")
         v = ops.headwise(a if a.dtype == w_dtype else a.to(w_dtype), self.w_uv, nh, self.value_width,
@@ -189,3 +195,12 @@ class LatentAttention(Mixer):
         if sink is not None and ops.adds_into_stream(T, self.w_o, sink.norm_weight):
             return ops.linear_into_stream(v, self.w_o, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(v, self.w_o, keep_slices=True)
+
+    def _queries(self, h, y, cache, slots, cos, sin, rot_dims):
+        """The latent into the cache, and the heads' queries against it, from the down projections ``y`` one launch after the other."""
+        cq = ops.latent_finish(y, self.q_norm, self.kv_norm, self.eps, cos, sin, rot_dims, slots, self.q_rank, self.kv_rank,
+                               self.rot_dim, cache.k, cache.v, cache.page_size, h.dtype)
+        q = ops.linear(cq if self.q_rank else h, self.w_uq)           # [T, heads (dim + rot_dim)]
+        w_dtype = self.w_uk_t.dtype
+        return ops.headwise(q if q.dtype == w_dtype else q.to(w_dtype), self.w_uk_t, self.n_heads, self.dim + self.rot_dim, self.rot_dim,
+                            cos, sin, rot_dims)

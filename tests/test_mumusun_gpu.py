@@ -249,6 +249,82 @@ def test_headwise_product_on_the_matrix_cores(T, H, K, N, tail, rot):
     assert torch.equal(got[..., N:], few[..., N:])
 
 
+def split_rows(seed, T, H, splits, D, sinks=False):
+    """Partial results of attention's splits as the row kernel leaves them, and what they join to in 64 bits.  Splits that saw no key hold anything."""
+    o, m, l = rnd(seed, T, H, splits, D), rnd(seed + 1, T, H, splits, scale=6.0), rnd(seed + 2, T, H, splits).abs() + 0.1
+    unseen = torch.rand(T, H, splits, generator=torch.Generator().manual_seed(seed)) < 0.4
+    unseen[..., 0] = False
+    if T > 1:
+        unseen[1, :, :] = True              # (a row that sees nothing: zeros)
+    m[unseen], l[unseen], o[unseen] = -math.inf, 0.0, math.nan
+    sink = rnd(seed + 3, H, scale=4.0).float() if sinks else None
+    top = m.double().amax(-1, keepdim=True).clamp(min=-1e30)
+    w = torch.exp2(m.double() - top)
+    total = (w * l.double()).sum(-1)
+    if sinks:
+        total = total + torch.exp2(sink.double() * math.log2(math.e) - top[..., 0])
+    want = (w[..., None] * torch.where(unseen[..., None], 0.0, o.double())).sum(2)
+    want = torch.where(w.sum(-1, keepdim=True) > 0, want / total[..., None], 0.0)
+    ml = torch.stack([m, l], -1).float().contiguous()
+    return ops.SplitRows(o.float().to(DEV), ml.to(DEV), None if sink is None else sink.to(DEV)), want
+
+
+@pytest.mark.parametrize("T,H,K,D,N,splits,gate", [(1, 3, 8, 16, 9, 1, 0), (16, 2, 96, 128, 128, 16, 0), (3, 16, 128, 128, 300, 32, 0), (5, 1, 40, 48, 44, 5, 1),
+                                                   (2, 4, 120, 128, 64, 31, 3)])
+def test_headwise_joins_the_splits_of_attention(T, H, K, D, N, splits, gate):
+    x, joined = split_rows(40 + T, T, H, splits, D, sinks=splits % 2 == 0)
+    w = rnd(44, H, N, K, scale=K ** -0.5).bfloat16()
+    want, rows = torch.einsum("thk,hnk->thn", joined[..., :K], w.double()), None
+    if gate:                      # columns 3 .. of wider rows, as they are or in so many partial sums
+        z = rnd(45, gate, T, H * N + 5).float()
+        z = z if gate > 1 else z.bfloat16().float()
+        want = want * torch.sigmoid(z.double().sum(0)[:, 3:3 + H * N]).view(T, H, N)
+        rows = (ops.SliceSums(z.to(DEV), torch.bfloat16) if gate > 1 else z[0].bfloat16().to(DEV), 3)
+    got = ops.headwise(x, w.to(DEV), H, D, gate=rows).cpu()
+    assert rel_err(got, want) < 4e-3                # (one rounding to bfloat16)
+    with pytest.raises(ops.KernelError):
+        ops.headwise(x, w.to(DEV), H, D, tail=2)
+    with pytest.raises(ops.KernelError):
+        ops.headwise(split_rows(3, 17, H, 4, D)[0], w.to(DEV), H, D)
+
+
+@pytest.mark.parametrize("T,H,dim,rot_dim,rot,kv_rank,N,wide", [(1, 3, 16, 8, 8, 32, 32, True), (16, 2, 64, 32, 16, 96, 96, True), (7, 5, 8, 0, 0, 264, 264, False),
+                                                               (2, 1, 24, 16, 16, 600, 300, False)])
+def test_queries_and_cache_in_one_launch(T, H, dim, rot_dim, rot, kv_rank, N, wide):
+    """The bits of the two launches that it stands for."""
+    P, pages = 16, 9
+    y = rnd(50, T, H * (dim + rot_dim) + kv_rank + rot_dim, scale=2.0).bfloat16().to(DEV)
+    w, norm = rnd(51, H, N, dim, scale=dim ** -0.5).bfloat16().to(DEV), (rnd(52, kv_rank) + 1).bfloat16().to(DEV)
+    cos = sin = None
+    if rot:
+        inv = torch.tensor([50.0 ** (-2.0 * i / rot) for i in range(rot // 2)], dtype=torch.float32, device=DEV)
+        cos, sin = ops.rope_table(torch.arange(T, dtype=torch.int32, device=DEV) * 3 + 1, inv)
+    slots = torch.randperm(pages * P, generator=torch.Generator().manual_seed(7))[:T].to(torch.int32).to(DEV)
+    caches = [(torch.zeros((pages, 1, P, kv_rank + rot_dim), dtype=torch.bfloat16, device=DEV),
+               torch.zeros((pages, 1, kv_rank + (rot_dim if wide else 0), P), dtype=torch.bfloat16, device=DEV)) for _ in range(2)]
+    got = ops.latent_query(y, w, H, dim + rot_dim, norm, 1e-5, cos, sin, rot, slots, kv_rank, rot_dim, *caches[0], P)
+    n_q = H * (dim + rot_dim)
+    want = ops.headwise(y[:, :n_q].contiguous(), w, H, dim + rot_dim, rot_dim, cos, sin, rot)
+    ops.latent_finish(y[:, n_q:].contiguous(), None, norm, 1e-5, cos, sin, rot, slots, 0, kv_rank, rot_dim, *caches[1], P, torch.bfloat16)
+    assert torch.equal(got, want) and all(torch.equal(a, b) and a.any() for a, b in zip(*caches))
+
+
+def test_rows_leave_their_splits_to_the_reader():
+    q, kc, vc, table, want = _paged_case("bfloat16", 300, None, 48, 48, 4)
+    rows, pos = torch.tensor([0, 17, 64, 299]), torch.tensor([0, 17, 64, 299], dtype=torch.int32, device=DEV)
+    args = (q[rows].to(DEV), kc.to(DEV), vc.to(DEV))
+    tail = (None, 4, torch.zeros(4, dtype=torch.int32, device=DEV), pos, table.to(DEV), None, 1.0, 64, 5)
+    left = ops.attention_rows(*args, None, *tail)
+    assert left.shape == (4, 4 * 48) and (left.n_heads, left.n_splits, left.width) == (4, 5, 48)
+    eye = torch.eye(48).expand(4, 48, 48).contiguous().bfloat16().to(DEV)
+    assert rel_err(ops.headwise(left, eye, 4, 48).view(4, -1).cpu(), want[rows]) < 2e-2
+    out = torch.empty(4, 4 * 48, dtype=torch.bfloat16, device=DEV)
+    assert ops.attention_rows(*args, out, *tail) is None and rel_err(out.cpu(), want[rows]) < 2e-2
+    for more in (dict(waves=4), dict(sink=1.0)):
+        with pytest.raises(ops.KernelError):
+            ops.attention_rows(*args, None, *tail, **more)
+
+
 def _paged_case(dtype, n, window, d, dv, nH, P=16, seed=20):
     """One request of n positions whose rows are all queried at once, its pages scattered over the pool; every query
     is aimed at two keys, the one on the window's inner edge and, twice as hard, the one just outside it, so that a

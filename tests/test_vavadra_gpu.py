@@ -347,6 +347,18 @@ def test_two_maps_as_heads_of_their_own_and_joined_again(dtype):
     assert rel_err(got, T64(want.reshape(T, H * dv))) < (1e-6 if dtype == "float32" else 1e-2)
 
 
+@pytest.mark.parametrize("T,H,dv,splits", [(1, 3, 16, 1), (37, 2, 128, 32), (8, 16, 112, 16), (64, 1, 48, 3)])
+def test_two_maps_joined_from_the_splits_of_attention(T, H, dv, splits):
+    from test_mumusun_gpu import split_rows
+    lam, scale, eps = 0.63, 0.7, 1e-5
+    a, joined = split_rows(60 + T, T, 2 * H, splits, dv)
+    pairs = N64(joined).reshape(T, H, 2, dv)
+    want = pv.rms_norm(pairs[:, :, 0] - lam * pairs[:, :, 1], None, eps) * scale
+    assert rel_err(ops.diff_combine(a, H, dv, lam, scale, eps).cpu(), T64(want.reshape(T, H * dv))) < 4e-3      # (one rounding to bfloat16)
+    with pytest.raises(ops.KernelError):
+        ops.diff_combine(a, 2 * H, dv, lam, scale, eps)
+
+
 # ---- the model through the engine -----------------------------------------------------------------
 @pytest.mark.parametrize("chunk", [17, 48, 100, 64, None])
 def test_blocks_and_two_maps_on_the_matrix_cores(chunk, tmp_path):
