@@ -38,6 +38,9 @@ __device__ __forceinline__ bf16x8 zero8() {
 
 // EPI 2: the product is added to the float stream [M, N] in place, and what the norm that follows needs is
 // written beside it: rows[m, n] = bf16(stream[m, n] * norm_w[n]) and pieces[n / 16][m] (see RowScale).
+// EPI 6: the same of the product itself, without a stream (a norm over some of a projection's columns: whoever wants the sum takes their pieces).
+// Latent attention's query norm so needs no launch between its two products: eight requests of 8 such layers 43.9 -> 43.3 ms (248 launches
+// of 5.5 us, whose other half, the cache's rows, goes with the queries' launch).
 struct StreamOut {
   float* stream;
   const void* norm_w;      // bfloat16, or float (a weight formed at load: norm_f32)
@@ -206,7 +209,7 @@ __device__ __forceinline__ bool skinny_accumulate(const bf16_t* __restrict__ x, 
 
 // EPI 0: out[m, n] = acc.  EPI 1: the rows of W alternate gate, up, gate, up ...; a lane holds two
 // such pairs of one output row and writes silu(gate) * up to out[m, n / 2] (out is [M, N / 2]).
-// EPI 2 (up to 16 rows, N a multiple of 4): see StreamOut; ``out`` is not used.  EPI 4: out[m, n] = max(acc, 0)^2.  EPI 5: gelu(acc).
+// EPI 2 and 6 (up to 16 rows, N a multiple of 4): see StreamOut; ``out`` is not used.  EPI 4: out[m, n] = max(acc, 0)^2.  EPI 5: gelu(acc).
 // ``order`` (tiled copies only): tile t of the copy holds the weight's rows 16 order[t] ...; null: in order.
 // ``scale`` (up to 16 rows): the results of row m are multiplied by the row's factor first.
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
@@ -241,14 +244,14 @@ __global__ __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_gemm_kernel(co
   union Two { floatx2 f; bf16x2 h; };
   floatx2 was[NT][2];
   Two nw[NT][2];
-  if (EPI == 2 && first_wave) {
+  if ((EPI == 2 || EPI == 6) && first_wave) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const int n = tile_rows * (first_tile + nt) + 4 * g + 2 * q;
         const bool ok = 4 * g + 2 * q < tile_rows && n < N && col < M;
-        was[nt][q] = ok ? *(const floatx2*)(so.stream + (size_t)col * N + n) : floatx2{0.f, 0.f};
+        was[nt][q] = EPI == 2 && ok ? *(const floatx2*)(so.stream + (size_t)col * N + n) : floatx2{0.f, 0.f};
         nw[nt][q].f = floatx2{0.f, 0.f};
         if (ok && so.norm_f32) nw[nt][q].f = *(const floatx2*)((const float*)so.norm_w + n);
         else if (ok) nw[nt][q].h = *(const bf16x2*)((const bf16_t*)so.norm_w + n);
@@ -261,7 +264,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_gemm_kernel(co
       })) return;
   if (shared_sums) rs = gathered_row_factor(scale, col, waves);
   // acc[nt][mt][r] = out[m = 16 mt + col][n = tile_rows (row tile of the weight) + 4 g + r], for 4 g + r < tile_rows
-  if (EPI == 2) {
+  if (EPI == 2 || EPI == 6) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       if (first_tile + nt >= n_tiles) continue;   // the same for the whole wave
@@ -278,7 +281,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_gemm_kernel(co
             y[r] = (__bf16)(v[r] * (so.norm_f32 ? nw[nt][q].f[r] : (float)nw[nt][q].h[r]));
             sq += v[r] * v[r];
           }
-          *(floatx2*)(so.stream + (size_t)col * N + n) = v;
+          if (EPI == 2) *(floatx2*)(so.stream + (size_t)col * N + n) = v;
           *(bf16x2*)(so.rows + (size_t)col * N + n) = y;
         }
       }
@@ -430,6 +433,9 @@ static int launch(const void* x, const void* W, void* out, int out_dtype, int M,
   if (epi == 2) {
     if constexpr (MT == 1) GO(float, 2);
     else IFX_FAIL("skinny_gemm: the stream epilogue takes at most 16 rows");
+  } else if (epi == 6) {
+    if constexpr (MT == 1) GO(float, 6);
+    else IFX_FAIL("skinny_gemm: the norm's epilogue takes at most 16 rows");
   } else if (epi == 4) {
     GO(bf16_t, 4);
   } else if (epi == 5) {
@@ -527,6 +533,7 @@ extern "C" int ifx_qkv_rope(const void* x, const void* Wt, int M, int K, const v
 // epi 2: the product is added to ``stream`` [M, N] (float, in place), rows_out [M, N] = bf16(stream * norm_w) and
 //        pieces_out [ceil(N / 16)][16] = sums of squares of the stream in runs of 16, for the norm that follows
 //        (M <= 16, N a multiple of 4, norm_w [N] bfloat16, or float with norm_f32); ``out`` is not used.
+// epi 6: the same of the product itself, without ``stream``.
 // epi 4: out = max(product, 0)^2, epi 5: out = gelu(product) (the tanh form), in bfloat16.
 // block_tiles, n_blocks: row tiles in blocks that read inputs of their own (see XBlocks; block_tiles 0: one input, its rows
 //        n_blocks elements apart, a multiple of 8, 0: K).
@@ -542,8 +549,8 @@ extern "C" int ifx_skinny_gemm(const void* x, const void* W, void* out, int out_
   const int tile_rows = tiled >= 8 ? tiled : 16;
   IFX_REQUIRE((tiled && tile_rows == 16) || !order, "skinny_gemm: a tile order goes with a tiled copy of 16-row tiles");
   IFX_REQUIRE(epi == 0 || !order, "skinny_gemm: only the plain epilogue takes a tile order");
-  IFX_REQUIRE(epi == 0 || ((epi == 1 || epi == 3) && N % 2 == 0) || (epi == 2 && N % 4 == 0) || ((epi == 4 || epi == 5) && out_dtype == DT_BF16), "skinny_gemm: epilogue %d with N=%d", epi, N);
-  IFX_REQUIRE(epi != 2 || (M <= 16 && stream_io && norm_w && rows_out && pieces_out),
+  IFX_REQUIRE(epi == 0 || ((epi == 1 || epi == 3) && N % 2 == 0) || ((epi == 2 || epi == 6) && N % 4 == 0) || ((epi == 4 || epi == 5) && out_dtype == DT_BF16), "skinny_gemm: epilogue %d with N=%d", epi, N);
+  IFX_REQUIRE((epi != 2 && epi != 6) || (M <= 16 && (epi == 6 || stream_io) && norm_w && rows_out && pieces_out),
               "skinny_gemm: the stream epilogue takes at most 16 rows (M=%d) and needs the stream, the norm's weight and two outputs", M);
   IFX_REQUIRE(!scale_pieces || (M <= 16 && n_scale_pieces > 0 && scale_width > 0.f),
               "skinny_gemm: row factors take at most 16 rows (M=%d, %d pieces, width %g)", M, n_scale_pieces, (double)scale_width);
@@ -606,7 +613,7 @@ extern "C" int ifx_skinny_gemm(const void* x, const void* W, void* out, int out_
   }
   while (waves > 1 && (size_t)(waves - 1) * nt * mt * WAVE * 16 > 64 * 1024) waves /= 2;
   IFX_REQUIRE(waves >= 1 && waves <= 16, "skinny_gemm: waves=%d outside 1..16", waves);
-  if (epi == 2 && nt == 2 && unroll == 4) unroll = 2;   // that instantiation spills
+  if ((epi == 2 || epi == 6) && nt == 2 && unroll == 4) unroll = 2;   // that instantiation spills
   hipStream_t s = (hipStream_t)stream;
   const int k_tiles = ifx_tiled_cols(K) / 32;
   const RowScale scale{scale_pieces, n_scale_pieces, scale_width, scale_eps};

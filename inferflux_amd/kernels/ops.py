@@ -539,31 +539,71 @@ def latent_query_takes(T: int, dtype: torch.dtype, dim: int, rot_dim: int, kv_ra
             and kv_rank <= LATENT_QUERY_MAX_RANK)
 
 
-def latent_query(y: torch.Tensor, weight: torch.Tensor, n_heads: int, x_head: int, kv_norm: torch.Tensor, eps: float,
-                 cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], rot_dims: int, slots: torch.Tensor, kv_rank: int, rot_dim: int,
+def _columns(t: torch.Tensor, name: str, T: int, width: int) -> int:
+    """How far apart the rows of ``t`` are: [T, width] in bfloat16, whole or columns of wider rows."""
+    if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.bfloat16 and t.shape == (T, width) and t.stride(1) == 1 and t.stride(0) >= width):
+        raise KernelError(f"{name}: expected bfloat16 rows or columns of rows [{T}, {width}] on the GPU")
+    return t.stride(0)
+
+
+def latent_query(q: torch.Tensor, latent: torch.Tensor, weight: torch.Tensor, n_heads: int, kv_norm: torch.Tensor, eps: float,
+                 cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], rot_dims: int, slots: torch.Tensor, rot_dim: int,
                  k_cache: torch.Tensor, v_cache: torch.Tensor, page_size: int) -> torch.Tensor:
-    """``headwise`` of the queries (a tail of ``rot_dim`` elements behind each head's) and ``latent_finish`` of the latent in one launch, for
-    steps of few rows (``latent_query_takes``): ``y`` [T, n_heads * x_head + kv_rank + rot_dim] in bfloat16 holds both side by side."""
-    T, width = y.shape
-    n_q = n_heads * x_head
-    _check(y, "y", (None, n_q + kv_rank + rot_dim), torch.bfloat16)
-    _check(weight, "weight", (n_heads, None, None), y.dtype)
+    """``headwise`` of the queries ``q`` [T, n_heads * (K + rot_dim)] (a tail of ``rot_dim`` elements behind each head's K) and ``latent_finish``
+    of ``latent`` [T, kv_rank + rot_dim] in one launch, for steps of few rows (``latent_query_takes``).  Both in bfloat16, whole rows or columns of
+    wider ones (on 16 bytes the queries)."""
+    T = q.shape[0]
+    _check(weight, "weight", (n_heads, None, None), q.dtype)
     _, N, K = weight.shape
-    if not latent_query_takes(T, y.dtype, K, x_head - K, kv_rank) or x_head != K + rot_dim:
-        raise KernelError(f"latent_query: {T} rows (1-{HEADWISE_ROWS_MAX}) of {n_heads} heads of {K} + {x_head - K}, a latent of {kv_rank}")
+    kv_rank, x_head = kv_norm.shape[0], K + rot_dim
+    q_ld, ld = _columns(q, "q", T, n_heads * x_head), _columns(latent, "latent", T, kv_rank + rot_dim)
+    if not latent_query_takes(T, q.dtype, K, rot_dim, kv_rank) or q_ld % 8 or q.data_ptr() % 16:
+        raise KernelError(f"latent_query: {T} rows (1-{HEADWISE_ROWS_MAX}), {q_ld} apart, of {n_heads} heads of {K} + {rot_dim}, a latent of {kv_rank}")
     _check(kv_norm, "kv_norm", (kv_rank,))
     if rot_dims:
         _check(cos, "cos", (T, rot_dims // 2), torch.float32)
         _check(sin, "sin", (T, rot_dims // 2), torch.float32)
     _check(slots, "slots", (T,), torch.int32)
-    _check(k_cache, "k_cache", (None, 1, page_size, kv_rank + rot_dim), y.dtype)
-    _check(v_cache, "v_cache", (k_cache.shape[0], 1, None, page_size), y.dtype)
-    out = empty((T, n_heads, N + rot_dim), y.dtype, y)
+    _check(k_cache, "k_cache", (None, 1, page_size, kv_rank + rot_dim), q.dtype)
+    _check(v_cache, "v_cache", (k_cache.shape[0], 1, None, page_size), q.dtype)
+    out = empty((T, n_heads, N + rot_dim), q.dtype, q)
     _call(load_module("latent"), "ifx_latent_query", (P, I, P, I, P, P, I, I, I, I, I, I, P, P, I, P, I, P, P, P, I, I, I, F, I, P),
-          y, width, y.data_ptr() + 2 * n_q, width, weight, out, T, n_heads, K, N, x_head, rot_dim, cos if rot_dims else None,
+          q, q_ld, latent, ld, weight, out, T, n_heads, K, N, x_head, rot_dim, cos if rot_dims else None,
           sin if rot_dims else None, rot_dims, kv_norm, _dt(kv_norm), slots, k_cache, v_cache, kv_rank, rot_dim, page_size, float(eps),
           v_cache.shape[2], _stream())
     return out
+
+
+def linear_normed_takes(x, weight, rank: int) -> bool:
+    """Whether ``linear_normed`` takes ``x`` and this weight, a norm over the first ``rank`` columns of whose product follows."""
+    if not isinstance(weight, LinearWeight) or weight.order is not None or weight.tiled is None or x.dtype != torch.bfloat16:
+        return False
+    N, K = weight.rows.shape
+    return (weight.rows.dtype == torch.bfloat16 and x.shape[0] <= 16 and N % 8 == 0 and 0 < rank <= N and rank % weight.tile_rows == 0
+            and _small_m_kernel(x.shape[0], N, K, True) == "skinny" and not ring_takes_few(x, weight))
+
+
+def normed_columns_take(n_rows: int, weight, rank: int) -> bool:
+    """Whether ``linear`` takes ``linear_normed``'s ``ScaledRows`` of ``n_rows`` rows with this weight."""
+    return (isinstance(weight, LinearWeight) and weight.rows.dtype == torch.bfloat16 and n_rows <= 16 and rank % 8 == 0 and weight.rows.shape[1] == rank
+            and _small_m_kernel(n_rows, weight.rows.shape[0], rank, weight.tiled is not None) == "skinny")
+
+
+def linear_normed(x, weight: LinearWeight, column_scale: torch.Tensor, rank: int, eps: float):
+    """x [M <= 16, K] (a tensor or ``ScaledRows``) times ``weight`` [N, K] transposed, times ``column_scale`` [N], as bfloat16 [M, N], and its first
+    ``rank`` columns as ``ScaledRows``: the rows of an RMS norm over them (whose weight the scale's first ``rank`` numbers are) up to the factor."""
+    if not linear_normed_takes(x, weight, rank):
+        raise KernelError(f"linear_normed: not for {x.shape[0]} rows times a {tuple(weight.rows.shape)} weight and a norm over {rank} columns")
+    x, scale = _scale_args(x)
+    _check(x, "x", (None, weight.rows.shape[1]), torch.bfloat16)
+    (M, K), N = x.shape, weight.rows.shape[0]
+    _check(column_scale, "column_scale", (N,))
+    y = empty((M, N), torch.bfloat16, x)
+    pieces = empty((-(-N // weight.tile_rows), 16), torch.float32, x)
+    _call(load_module("gemm_bf16"), "ifx_skinny_gemm", _SKINNY_ARGS,
+          x, weight.tiled, 0, DT_F32, M, N, K, 0, 0, 0, 6, weight.tile_rows, 0, *scale, 0, column_scale,
+          1 if column_scale.dtype == torch.float32 else 0, y, pieces, 1.0, 0, 0, _stream())
+    return y, ScaledRows(y[:, :rank], pieces[:rank // weight.tile_rows], rank, eps, None)
 
 
 HEADWISE_ROWS_MAX = 16             # rows of a step up to which a thread forms an output element by itself
@@ -1235,13 +1275,14 @@ class SliceSums:
         return out
 
 
-def _scale_args(x):
-    """(rows, the four row-factor arguments of the kernels) of a tensor or a ``ScaledRows``."""
+def _scale_args(x, columns: bool = False):
+    """(rows, the four row-factor arguments of the kernels) of a tensor or a ``ScaledRows``; ``columns``: whose rows may be columns of wider ones."""
     if isinstance(x, ScaledRows):
         _check(x.pieces, "pieces", (None, 16), torch.float32)
         if not 1 <= x.pieces.shape[0] <= x.width:
             raise KernelError(f"scaled rows: {x.pieces.shape[0]} pieces for a width of {x.width}")
-        _check(x.rows, "rows", (None, x.width), torch.bfloat16)
+        if not (columns and columns_on_16_bytes(x.rows) and x.rows.shape[1] == x.width):
+            _check(x.rows, "rows", (None, x.width), torch.bfloat16)
         if x.rows.shape[0] > 16:
             raise KernelError(f"scaled rows: {x.rows.shape[0]} rows, at most 16")
         return x.rows, (x.pieces.data_ptr(), x.pieces.shape[0], float(x.width), x.eps)
@@ -1355,7 +1396,7 @@ def skinny_gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     ``x`` may be ``ScaledRows``, or a tensor whose rows are further apart than K (columns of wider rows, on 16 bytes).
     ``plain_act`` (ACT_RELU_SQUARED, ACT_GELU_TANH; bfloat16 output): the activation of a feed-forward without a gate on the
     float sums."""
-    x, scale = _scale_args(x)
+    x, scale = _scale_args(x, True)
     apart = 0
     if columns_on_16_bytes(x):
         apart = x.stride(0)
@@ -1619,6 +1660,8 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
     prepared = isinstance(weight, LinearWeight)
     if prepared:
         weight, tiled, order, tile_rows = weight.rows, weight.tiled, weight.order, weight.tile_rows
+    if isinstance(x, ScaledRows) and columns_on_16_bytes(x.rows):
+        return skinny_gemm(x, weight, out_dtype or torch.bfloat16, tiled=tiled, order=order, tile_rows=tile_rows)
     columns = columns_on_16_bytes(x)      # (the product for few rows reads them where they lie, every other one takes a copy)
     if weight.dtype == torch.float32:
         return gemm_f32(x.contiguous() if columns else x, weight, None, out_dtype or x.dtype)

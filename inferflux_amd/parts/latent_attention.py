@@ -78,7 +78,7 @@ class LatentAttention(Mixer):
         self.position = build_part("position", position)
         if self.position.needs_apply:
             raise ValueError(f"{name}: latent attention needs a position part that gives the kernels a rotation table")
-        self.w_few = self.w_down = self.w_uq = self.w_uk_t = self.w_uv = self.w_o = self.q_norm = self.kv_norm = None
+        self.w_few = self.few_scale = self.w_down = self.w_uq = self.w_uk_t = self.w_uv = self.w_o = self.q_norm = self.kv_norm = None
 
     @property
     def key_width(self) -> int:
@@ -159,6 +159,10 @@ class LatentAttention(Mixer):
         if self.q_rank and not self.shared_latent and norms[0].dtype != norms[1].dtype:
             norms = [w.float() for w in norms]
         self.q_norm, self.kv_norm = norms
+        self.few_scale = None
+        if self.q_rank and self.q_norm.is_cuda and self.w_down.dtype == torch.bfloat16:
+            # the down projections' columns times this: the query latent's by its norm's weight, the others as they are
+            self.few_scale = torch.cat([self.q_norm, self.q_norm.new_ones(self.w_down.shape[0] - self.q_rank)])
 
     adds_to_stream = True
 
@@ -172,15 +176,25 @@ class LatentAttention(Mixer):
         T, nh, t, dtype = h.shape[0], self.n_heads, ctx.timer, h.dtype
         _, rot_dims, cos, sin = self.position.kernel_args(ctx)
         slots = None if self.shared_latent else ctx.write_slots(cache.group)
-        few = self.w_few is not None and h.dtype == cache.k.dtype and ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank)
-        y = None if few else ops.linear(h, self.w_down, keep_slices=True)     # [T, q_rank + kv_rank + rot_dim + gate]
-        if isinstance(y, ops.SliceSums) and y.parts.shape[0] > SLICES_READ_TWICE:
-            y = ops.SliceSums(y.sum(torch.float32)[None], y.dtype)    # (still float, added up by the whole chip)
-        if few:
-            qa = ops.latent_query(ops.linear(h, self.w_few), self.w_uk_t, nh, self.dim + self.rot_dim, self.kv_norm, self.eps, cos, sin, rot_dims,
-                                  slots, self.kv_rank, self.rot_dim, cache.k, cache.v, cache.page_size)
+        rank, heads_w = self.q_rank, nh * (self.dim + self.rot_dim)
+        q = latent = None
+        if self.w_few is not None and h.dtype == cache.k.dtype and ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank):
+            y = ops.linear(h, self.w_few)
+            q, latent = y[:, :heads_w], y[:, heads_w:]
+        elif (self.few_scale is not None and h.dtype == cache.k.dtype and ops.linear_normed_takes(h, self.w_down, rank)
+                and ops.normed_columns_take(T, self.w_uq, rank)
+                and (self.shared_latent or ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank))):
+            y, cq = ops.linear_normed(h, self.w_down, self.few_scale, rank, self.eps)
+            q, latent = ops.linear(cq, self.w_uq), y[:, rank:rank + self.kv_rank + self.rot_dim]
         else:
-            qa = self._queries(h, y, cache, slots, cos, sin, rot_dims)        # [T, heads, key_width]
+            y = ops.linear(h, self.w_down, keep_slices=True)          # [T, q_rank + kv_rank + rot_dim + gate]
+            if isinstance(y, ops.SliceSums) and y.parts.shape[0] > SLICES_READ_TWICE:
+                y = ops.SliceSums(y.sum(torch.float32)[None], y.dtype)    # (still float, added up by the whole chip)
+        if latent is None or self.shared_latent:
+            qa = self._queries(h, y, q, cache, slots, cos, sin, rot_dims)     # [T, heads, key_width]
+        else:
+            qa = ops.latent_query(q, latent, self.w_uk_t, nh, self.kv_norm, self.eps, cos, sin, rot_dims, slots, self.rot_dim, cache.k, cache.v,
+                                  cache.page_size)
         if t is not None:
             t.mark("mixer.qkv")
         w_dtype = self.w_uv.dtype
@@ -196,11 +210,12 @@ class LatentAttention(Mixer):
             return ops.linear_into_stream(v, self.w_o, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(v, self.w_o, keep_slices=True)
 
-    def _queries(self, h, y, cache, slots, cos, sin, rot_dims):
-        """The latent into the cache, and the heads' queries against it, from the down projections ``y`` one launch after the other."""
-        cq = ops.latent_finish(y, self.q_norm, self.kv_norm, self.eps, cos, sin, rot_dims, slots, self.q_rank, self.kv_rank,
-                               self.rot_dim, cache.k, cache.v, cache.page_size, h.dtype)
-        q = ops.linear(cq if self.q_rank else h, self.w_uq)           # [T, heads (dim + rot_dim)]
+    def _queries(self, h, y, q, cache, slots, cos, sin, rot_dims):
+        """The heads' queries against the cached rows, from ``q``, or from the down projections ``y``, whose latent goes into the cache."""
+        if q is None:
+            cq = ops.latent_finish(y, self.q_norm, self.kv_norm, self.eps, cos, sin, rot_dims, slots, self.q_rank, self.kv_rank,
+                                   self.rot_dim, cache.k, cache.v, cache.page_size, h.dtype)
+            q = ops.linear(cq if self.q_rank else h, self.w_uq)       # [T, heads (dim + rot_dim)]
         w_dtype = self.w_uk_t.dtype
         return ops.headwise(q if q.dtype == w_dtype else q.to(w_dtype), self.w_uk_t, self.n_heads, self.dim + self.rot_dim, self.rot_dim,
                             cos, sin, rot_dims)

@@ -302,11 +302,34 @@ def test_queries_and_cache_in_one_launch(T, H, dim, rot_dim, rot, kv_rank, N, wi
     slots = torch.randperm(pages * P, generator=torch.Generator().manual_seed(7))[:T].to(torch.int32).to(DEV)
     caches = [(torch.zeros((pages, 1, P, kv_rank + rot_dim), dtype=torch.bfloat16, device=DEV),
                torch.zeros((pages, 1, kv_rank + (rot_dim if wide else 0), P), dtype=torch.bfloat16, device=DEV)) for _ in range(2)]
-    got = ops.latent_query(y, w, H, dim + rot_dim, norm, 1e-5, cos, sin, rot, slots, kv_rank, rot_dim, *caches[0], P)
     n_q = H * (dim + rot_dim)
+    got = ops.latent_query(y[:, :n_q], y[:, n_q:], w, H, norm, 1e-5, cos, sin, rot, slots, rot_dim, *caches[0], P)
     want = ops.headwise(y[:, :n_q].contiguous(), w, H, dim + rot_dim, rot_dim, cos, sin, rot)
     ops.latent_finish(y[:, n_q:].contiguous(), None, norm, 1e-5, cos, sin, rot, slots, 0, kv_rank, rot_dim, *caches[1], P, torch.bfloat16)
     assert torch.equal(got, want) and all(torch.equal(a, b) and a.any() for a, b in zip(*caches))
+
+
+@pytest.mark.parametrize("T,N,K,rank,N2,scaled,norm_dtype", [(1, 48, 64, 16, 40, False, torch.bfloat16), (16, 896, 2048, 768, 2048, False, torch.float32),
+                                                             (5, 2944, 320, 384, 100, True, torch.bfloat16), (9, 512, 136, 512, 56, True, torch.float32)])
+def test_norm_over_a_products_first_columns(T, N, K, rank, N2, scaled, norm_dtype):
+    """A down projection's columns times a weight, the first ``rank`` of them under an RMS norm whose factor the next product applies."""
+    x, w, w2 = rnd(70, T, K).bfloat16(), rnd(71, N, K, scale=K ** -0.5).bfloat16(), rnd(72, N2, rank, scale=rank ** -0.5).bfloat16()
+    g = torch.cat([rnd(73, rank) + 1, torch.ones(N - rank)]).to(norm_dtype)
+    y = x.double() @ w.double().T
+    xd = x.to(DEV)
+    if scaled:                # (the rows themselves up to a norm's factor)
+        pieces = torch.zeros(3, 16)
+        pieces[:, :T] = rnd(74, 3, T).abs() + 0.5
+        xd = ops.ScaledRows(xd, pieces.to(DEV), K, 1e-5)
+        y = y / torch.sqrt(pieces[:, :T].double().sum(0)[:, None] / K + 1e-5)
+    down, up = ops.prepare_linear(w.to(DEV)), ops.prepare_linear(w2.to(DEV))
+    assert ops.linear_normed_takes(xd, down, rank) and ops.normed_columns_take(T, up, rank)
+    got, cq = ops.linear_normed(xd, down, g.to(DEV), rank, 1e-5)
+    assert rel_err(got.cpu(), y * g.double()) < 4e-3                                                # (one rounding to bfloat16)
+    want = pm.rms_norm(y[:, :rank], g[:rank].double(), 1e-5) @ w2.double().T
+    assert rel_err(ops.linear(cq, up).cpu(), want) < 8e-3                                           # (two)
+    with pytest.raises(ops.KernelError):
+        ops.linear_normed(xd, down, g.to(DEV), rank + 1, 1e-5)
 
 
 def test_rows_leave_their_splits_to_the_reader():
