@@ -25,7 +25,7 @@
 // the threads put q, k and alpha of the stage's tokens into LDS, a (token, channel) each (and form alpha on the way), everybody walks the
 // stage's tokens, o goes to LDS, and a wave per token norms and gates it.
 //
-// MODE 0: a request's rows in one walk, from its slot and back into it.
+// MODE 0: a request's rows in one walk, from its slot and back into it (steps of single tokens: gla_step_kernel).
 // Long portions are cut into chunks that run side by side (the recurrence is linear in S):
 // MODE 1: a chunk from S = 0; records its final S and the sum of its log alpha per channel.
 // gla_combine: walks a request's chunks: chunk c's record becomes the state chunk c starts from,
@@ -33,6 +33,7 @@
 // MODE 2: a chunk from the state it starts from; writes y.
 #include "common.h"
 #include "tile_acts.h"
+#include "lane_sums.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -238,6 +239,83 @@ __global__ __launch_bounds__(WHOLE ? 512 : GLA_MAX_THREADS(DP)) void gla_kernel(
   }
   if (MODE == 1) put_back();
   if (MODE == 1 && tid < d) a.chunk_loga[(size_t)unit * H * d + head * d + tid] = loga_sum;
+}
+
+// Steps of single tokens (a request's tokens one after the other where it has more): a workgroup takes a head of a request.  Bound by S, which is
+// read and written once.  A thread has four channels of up to STEP_COLS columns, the threads of a column neighbours, so that a wave's load is 1 KB of
+// contiguous memory and q and k are a thread's own; the decays are formed once and go through LDS while S is on its way.  16 heads of 64 x 128, us by
+// the walk above, with runs of 16 channels to a thread / 4 columns / 8 columns, at 1, 8, 16, 32, 48, 64 requests: 5.8 / 4.8 / 5.6, 7.3 / 5.9 / 6.7,
+// 9.4 / 7.1 / 7.9, 14.1 / 10.8 / 11.1, 17.6 / 13.1 / 13.4, 24.5 / 19.6 / 16.4 (67 MB of S at 64); time mixing of 64 x 64 4.2 / 4.2 / 4.8, 4.7 / 4.5 / 4.9,
+// 5.9 / 5.4 / 5.9, 8.2 / 7.1 / 7.4, 10.6 / 9.0 / 8.8, 12.2 / 10.2 / 9.7.
+#define STEP_MANY_HEADS 768      // (request, head) pairs up to which four columns are the better choice
+template <typename T, typename TO, int STEP_COLS>
+__global__ __launch_bounds__(1024) void gla_step_kernel(GlaArgs a, int KS) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // the token's decays [4 KS], its outputs [dv]
+  const int r = blockIdx.x, head = blockIdx.y, n = a.q_len[r];
+  if (n <= 0) return;
+  const int t0 = a.q_start[r], d = a.d, dv = a.dv, H = a.H, dpad = 4 * KS, groups = blockDim.x / KS;
+  const int tid = threadIdx.x, lane = tid % WAVE, s = tid % KS, j0 = tid / KS;      // column i of the thread: j0 + groups i
+  float *la = lds, *lo = lds + dpad;
+  float* sp = a.state + (size_t)a.slots[r] * a.state_stride + a.state_offset + (size_t)head * dv * dpad;      // (the same for all
+  const unsigned own = 4 * s;                                                   // threads: a thread's places are 32-bit offsets from it)
+  float4 S[STEP_COLS];
+#pragma unroll
+  for (int i = 0; i < STEP_COLS; ++i) {
+    const int j = j0 + groups * i;
+    S[i] = j < dv ? *(const float4*)(sp + (own + (unsigned)(j * dpad))) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const T *rq = (const T*)a.q, *rk = (const T*)a.k, *rv = (const T*)a.v, *rg = (const T*)a.g;
+  const LaneSteps steps = lane_steps(KS);
+  const auto weight_of = [&](int c) { return load_dyn(a.norm_w, a.norm_dtype, TIME_MIX ? head * dv + c : c); };
+  const float weight = tid < dv ? weight_of(tid) : 0.f;
+  float u4[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) u4[c] = TIME_MIX && 4 * s + c < d ? a.bonus[head * d + 4 * s + c] : 0.f;
+  for (int t = t0; t < t0 + n; ++t) {
+    const size_t at = (size_t)t * a.ld;
+    const float g = tid < dv ? to_f(rg[at + head * dv + tid]) : 0.f;
+    float q[4], k[4], v[STEP_COLS];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int ch = 4 * s + c;
+      q[c] = ch < d ? to_f(rq[at + head * d + ch]) * a.q_scale : 0.f;
+      k[c] = ch < d ? to_f(rk[at + head * d + ch]) : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < STEP_COLS; ++i) v[i] = j0 + groups * i < dv ? to_f(rv[at + head * dv + j0 + groups * i]) : 0.f;
+    for (int c = tid; c < dpad; c += blockDim.x) {
+      const float z = c < d ? a.z[(size_t)t * (H * d) + head * d + c] + (a.z_bias ? a.z_bias[head * d + c] : 0.f) : 0.f;
+      la[c] = expf(TIME_MIX ? -expf(z) : log_sigmoid(z) * a.inv_tau);
+    }
+    float b = 0.f;                       // TIME_MIX: sum_i u[i] k[i] q[i]
+    if (TIME_MIX) b = column_sum((u4[0] * k[0] * q[0] + u4[1] * k[1] * q[1]) + (u4[2] * k[2] * q[2] + u4[3] * k[3] * q[3]), steps);
+    LDS_BARRIER();
+    const float4 al = *(const float4*)(la + 4 * s);
+    const bool last = t == t0 + n - 1;
+#pragma unroll
+    for (int i = 0; i < STEP_COLS; ++i) {
+      const int j = j0 + groups * i;
+      float o = 0.f;
+      if (TIME_MIX) o = (S[i].x * q[0] + S[i].y * q[1]) + (S[i].z * q[2] + S[i].w * q[3]);        // (the read-out comes before the write)
+      S[i].x = fmaf(al.x, S[i].x, k[0] * v[i]);
+      S[i].y = fmaf(al.y, S[i].y, k[1] * v[i]);
+      S[i].z = fmaf(al.z, S[i].z, k[2] * v[i]);
+      S[i].w = fmaf(al.w, S[i].w, k[3] * v[i]);
+      if (last && j < dv) *(float4*)(sp + (own + (unsigned)(j * dpad))) = S[i];
+      if (!TIME_MIX) o = (S[i].x * q[0] + S[i].y * q[1]) + (S[i].z * q[2] + S[i].w * q[3]);
+      o = column_sum(o, steps);
+      if (TIME_MIX) o = fmaf(b, v[i], o);
+      if (s == 0 && j < dv) lo[j] = o;
+    }
+    LDS_BARRIER();
+    float ss = 0.f;
+    for (int c = lane; c < dv; c += WAVE) ss = fmaf(lo[c], lo[c], ss);
+    const float inv = rsqrtf(wave_sum(ss) / (float)dv + a.eps);
+    TO* out = (TO*)a.out + (size_t)t * (H * dv) + head * dv;
+    if (tid < dv) out[tid] = from_f<TO>(lo[tid] * inv * weight * act_silu(g));
+    for (int c = tid + blockDim.x; c < dv; c += blockDim.x) out[c] = from_f<TO>(lo[c] * inv * weight_of(c) * act_silu(to_f(rg[at + head * dv + c])));
+    if (!last) LDS_BARRIER();          // (the next token's decays and outputs overwrite what this one read)
+  }
 }
 
 // One thread per number of a request's S: walks the request's chunks in order.  chunk_state[c] holds what chunk c
@@ -580,8 +658,24 @@ static void launch_gla_cols(const GlaArgs& a, int units, int cols, int threads, 
   launch_gla_mode<T, TO, DP, MODE, 1>(a, units, threads, lds, s);
 }
 
+// The threads of gla_step_kernel for a head of these sizes, 0 where it does not take them.
+static int step_threads(int dpad, int dv, int cols) {
+  const int lanes = dpad / 4, threads = (lanes * ((dv + cols - 1) / cols) + WAVE - 1) / WAVE * WAVE;
+  return lanes <= WAVE && threads <= 1024 ? threads : 0;
+}
+
 template <typename T, typename TO, int DP>
-static int launch_gla(const GlaArgs& a, int R, int n_chunks, const int* req_chunk0, hipStream_t s) {
+static int launch_gla(const GlaArgs& a, int T_rows, int R, int n_chunks, const int* req_chunk0, hipStream_t s) {
+  if constexpr (sizeof(TO) == 2) {         // (in 32 bits a token's bits are the same alone and among others of its request: the walk's)
+    const bool many = (long long)R * a.H > STEP_MANY_HEADS || step_threads(a.parts * DP, a.dv, 4) == 0;
+    const int threads = n_chunks == 0 && T_rows <= R ? step_threads(a.parts * DP, a.dv, many ? 8 : 4) : 0;
+    if (threads > 0) {
+      const size_t lds = (size_t)(a.parts * DP + a.dv) * sizeof(float);
+      if (many) hipLaunchKernelGGL((gla_step_kernel<T, TO, 8>), dim3(R, a.H), dim3(threads), lds, s, a, a.parts * DP / 4);
+      else hipLaunchKernelGGL((gla_step_kernel<T, TO, 4>), dim3(R, a.H), dim3(threads), lds, s, a, a.parts * DP / 4);
+      IFX_LAUNCH_CHECK();
+    }
+  }
   // A thread holds 1, 2 or 4 columns of S as its registers allow (4 for runs of 16 channels, 2 for 32): what it reads of a
   // token's q, k and decays from LDS then serves several columns.  Two where possible (steps of single tokens, which are bound
   // by reading and writing S: 23 against 33 us for 64 requests of 16 heads x 64 x 128; chunks side by side: 86 + 64 against
@@ -637,7 +731,7 @@ extern "C" int ifx_gla_scan(const void* q, const void* k, const void* v, const v
             (size_t)state_stride, (size_t)state_offset, q_start, q_len, slots, out, H, d, dv, parts,
             chunk_req, chunk_t0, chunk_len, chunk_state, chunk_loga};
   hipStream_t s = (hipStream_t)stream;
-#define GLA_CASE2(TY, TO, DPV) if (dp == DPV) return launch_gla<TY, TO, DPV>(a, R, n_chunks, req_chunk0, s);
+#define GLA_CASE2(TY, TO, DPV) if (dp == DPV) return launch_gla<TY, TO, DPV>(a, T, R, n_chunks, req_chunk0, s);
 #define GLA_CASE(TY, DPV) GLA_CASE2(TY, TY, DPV)
 #if TIME_MIX
   if (dtype == DT_F32 && out_dtype == DT_BF16) { GLA_CASE2(float, bf16_t, 16) GLA_CASE2(float, bf16_t, 32) GLA_CASE2(float, bf16_t, 64) GLA_CASE2(float, bf16_t, 128) }

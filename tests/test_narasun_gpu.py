@@ -282,6 +282,29 @@ def test_time_mix_over_steps_with_state_in_slots(dtype, H, d):
             assert rel_err(torch.cat(got[r]), T64(want[r])) < (2e-5 if dtype == "float32" else 2e-2), (r, chunked)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float32 to bfloat16"])
+@pytest.mark.parametrize("R,H,d", [(4, 3, 12), (4, 2, 64), (4, 1, 40), (4, 1, 128), (4, 1, 200), (385, 2, 16), (193, 4, 64)])
+def test_single_tokens_of_time_mixing_against_the_walk(dtype, R, H, d):
+    """Requests' tokens, twice, against the walk, which the same tokens take beside a request of two (sums of at most 200 products in another order)."""
+    dt, out_dt = DT[dtype.split()[0]], DT[dtype.split()[-1]]
+    w0 = (-5.0 + 5.0 * torch.rand(H * d, generator=torch.Generator().manual_seed(8))).float().to(DEV)
+    u, norm_w = rnd(9, H, d).float().to(DEV), (1.0 + 0.3 * rnd(10, H * d)).float().to(DEV)
+    data = [x.to(DEV) for x in _time_mix_inputs(20, R + 2, H, d, dt)]
+    order = torch.randperm(R + 2, generator=torch.Generator().manual_seed(2)).to(torch.int32)
+    outs, states = [], []
+    for beside in (False, True):
+        state = torch.zeros(R + 2, ops.gla_state_floats(H, d, d), device=DEV)
+        for turn in range(2):
+            lens = [1] * R + [2] * beside
+            q_start, q_len = _step_arrays(lens)
+            out = ops.time_mix_scan(*(x[:sum(lens)] for x in data), w0, u, norm_w, 1e-5, H, d, state, 0, q_start.to(DEV), q_len.to(DEV),
+                                    order[:len(lens)].to(DEV), out_dt).cpu()
+        outs.append(out[:R].double())
+        states.append(state.cpu()[order[[*range(R), R + 1]].long()].double())
+    assert rel_err(outs[0], outs[1]) < (2e-5 if out_dt == torch.float32 else 2.0 ** -8)
+    assert rel_err(states[0], states[1]) < 2e-6 and states[0][:R].any() and not states[0][R].any()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_a_key_far_back_is_still_in_time_mixings_state(dtype):
     """A channel that hardly decays is written at token 0 alone and read 700 tokens later, decoded one by one at the end: the
@@ -397,6 +420,31 @@ def test_single_tokens_of_the_memory_against_the_walk(dtype, H, d, dv):
         states.append(state[[3, 0, 5, 1, 2]].cpu().double())
     assert rel_err(outs[0], outs[1]) < (2e-5 if out_dt == torch.float32 else 2.0 ** -8)
     assert rel_err(states[0], states[1]) < 2e-6
+
+
+@pytest.mark.parametrize("R,H,d,dv", [(257, 1, 16, 1), (129, 2, 10, 63), (65, 4, 64, 128), (260, 1, 64, 130), (257, 1, 256, 143), (257, 1, 256, 144), (129, 2, 8, 40)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float32 to bfloat16"])
+def test_single_tokens_of_many_heads_of_the_memory_against_the_walk(dtype, R, H, d, dv):
+    """More heads than compute units, on both sides of what a workgroup then takes: as above.  (The states start from random numbers, too: from nothing an
+    output would be one or two outer products, whose q . k may cancel, and the heads' norm would magnify what is left of its rounding, 2^-24 sqrt(d) |q| |k| /
+    |q . k|, without a bound over some hundred heads.)"""
+    dt, out_dt = DT[dtype.split()[0]], DT[dtype.split()[-1]]
+    ib, fb, norm_w = rnd(8, H).float(), (rnd(9, H) * 2 + 3).float(), (1.0 + 0.3 * rnd(10, H * dv)).float()
+    rows, cols, gates, gate_cols = _memory_inputs(5, R + 2, H, d, dv, dt)
+    order = torch.randperm(R + 2, generator=torch.Generator().manual_seed(2)).tolist()
+    outs, states = [], []
+    for beside in (False, True):
+        state = torch.randn(R + 2, ops.matrix_memory_state_floats(H, d, dv), generator=torch.Generator().manual_seed(3)).to(DEV) * 0.5
+        dpad = max(4, 1 << (d - 1).bit_length())
+        state[:, state.shape[1] - H * (dv + 1) * dpad:].view(R + 2, -1, dpad)[:, :, d:] = 0      # (the padded channels hold zeros)
+        first = state[order[R + 1]].clone()
+        for turn in range(2):
+            lens = [1] * R + [2] * beside
+            out = _memory_call(rows[:sum(lens)], cols, gates[:sum(lens)], gate_cols, ib, fb, 9.0, norm_w, 1e-5, H, d, dv, state, lens, order[:len(lens)], out_dt, False, True)
+        outs.append(out[:R].double())
+        states.append(state.cpu()[order[:R] + order[R + 1:]].double())
+    assert rel_err(outs[0], outs[1]) < (2e-5 if out_dt == torch.float32 else 2.0 ** -8)
+    assert rel_err(states[0], states[1]) < 2e-6 and torch.equal(states[0][R], first.cpu().double())
 
 
 @pytest.mark.parametrize("H,d,dv", [(4, 64, 128), (2, 24, 40), (1, 256, 320)])

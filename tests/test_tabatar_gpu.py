@@ -282,6 +282,30 @@ def test_gated_linear_attention_over_steps_with_state_in_slots(dtype, H, d, dv, 
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("R,H,d,dv", [(4, 2, 16, 1), (4, 3, 10, 63), (4, 4, 64, 128), (4, 2, 24, 130), (4, 1, 64, 256), (4, 1, 64, 257), (4, 1, 64, 512), (4, 1, 64, 513),
+                                      (4, 1, 256, 128), (4, 1, 256, 129), (4, 1, 100, 40), (768, 1, 16, 24), (257, 3, 10, 63), (200, 4, 64, 128)])
+def test_single_tokens_of_linear_attention_against_the_walk(dtype, R, H, d, dv):
+    """Heads on both sides of what the kernel of single tokens takes, and numbers of them on both sides of its two forms: requests' tokens, twice, against the
+    walk, which the same tokens take beside a request of two.  Sums of at most 256 products in another order, and one rounding to bfloat16; in 32 bits the walk takes both."""
+    dt = DT[dtype]
+    rows, cols, z, bias, w = _gla_inputs(5, R + 2, H, d, dv, dt)
+    order = torch.randperm(R + 2, generator=torch.Generator().manual_seed(2)).to(torch.int32)
+    outs, states = [], []
+    for beside in (False, True):
+        state = torch.zeros((R + 2, ops.gla_state_floats(H, d, dv) + 4), device=DEV)
+        for turn in range(2):
+            lens = [1] * R + [2] * beside
+            q_start, q_len = _step_arrays(lens)
+            n = sum(lens)
+            out = ops.gla_scan(rows[:n].to(DEV), cols, z[:n].to(DEV), bias.to(DEV), 16.0, d ** -0.5, w.to(DEV), 1e-5, H, d, dv, state, 4,
+                               q_start.to(DEV), q_len.to(DEV), order[:len(lens)].to(DEV)).cpu()
+        outs.append(out[:R].double())
+        states.append(state.cpu()[order[[*range(R), R + 1]].long()].double())
+    assert torch.equal(outs[0], outs[1]) if dtype == "float32" else rel_err(outs[0], outs[1]) < 2.0 ** -8
+    assert rel_err(states[0], states[1]) < 2e-6 and states[0][:R].any() and not states[0][R].any() and not states[0][:, :4].any()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,d,dv,tau,chunk", [(2, 16, 24, 8.0, 64), (3, 8, 16, 3.0, 16), (4, 64, 64, 16.0, 64), (3, 10, 14, 5.0, 7), (2, 128, 128, 16.0, 64),
                                              (1, 32, 8, 20.0, 200), (1, 192, 192, 8.0, 32), (1, 256, 256, 4.0, 64)])
 def test_gated_linear_attention_in_chunks_side_by_side(dtype, H, d, dv, tau, chunk):
