@@ -46,7 +46,10 @@ IFX_DEFINE_LAST_ERROR()
 struct GlaArgs {
   const void* q; const void* k; const void* v; const void* g;      // the head-0 columns of row 0; rows ld elements apart
   int ld;
-  const float* z;          // [T, H * d]
+  const float* z;          // [T, H * d], or null (steps of single tokens):
+  const bf16_t* low;       // ... z_t = w2 low_t with low [T, rank] (rows low_ld apart) and w2 [H * d, rank]
+  const bf16_t* w2;
+  int low_ld, rank;
   const float* z_bias;     // [H * d] or null
   float inv_tau, q_scale, eps;
   const void* norm_w;      // [dv], or with TIME_MIX [H * dv]
@@ -242,69 +245,126 @@ __global__ __launch_bounds__(WHOLE ? 512 : GLA_MAX_THREADS(DP)) void gla_kernel(
 }
 
 // Steps of single tokens (a request's tokens one after the other where it has more): a workgroup takes a head of a request.  Bound by S, which is
-// read and written once.  A thread has four channels of up to STEP_COLS columns, the threads of a column neighbours, so that a wave's load is 1 KB of
-// contiguous memory and q and k are a thread's own; the decays are formed once and go through LDS while S is on its way.  16 heads of 64 x 128, us by
-// the walk above, with runs of 16 channels to a thread / 4 columns / 8 columns, at 1, 8, 16, 32, 48, 64 requests: 5.8 / 4.8 / 5.6, 7.3 / 5.9 / 6.7,
-// 9.4 / 7.1 / 7.9, 14.1 / 10.8 / 11.1, 17.6 / 13.1 / 13.4, 24.5 / 19.6 / 16.4 (67 MB of S at 64); time mixing of 64 x 64 4.2 / 4.2 / 4.8, 4.7 / 4.5 / 4.9,
-// 5.9 / 5.4 / 5.9, 8.2 / 7.1 / 7.4, 10.6 / 9.0 / 8.8, 12.2 / 10.2 / 9.7.
-#define STEP_MANY_HEADS 768      // (request, head) pairs up to which four columns are the better choice
-template <typename T, typename TO, int STEP_COLS>
-__global__ __launch_bounds__(1024) void gla_step_kernel(GlaArgs a, int KS) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];      // the token's decays [4 KS], its outputs [dv]
+// read and written once, and for few requests by a trip to memory and the arithmetic behind it.  A thread has four channels of STEP_COLS columns (4,
+// and 8 where a head's columns want more than STEP_THREADS threads so), the threads of a column neighbours: a wave's load is 1 KB of contiguous
+// memory.  q, k, v and the decays are formed a channel or column a thread and meet in LDS; every load goes out before any is used, without branches
+// between them, so that what meets there is waited for while S is on its way.  16 heads of 64 x 128, us by the walk above, whose threads
+// have 16 channels, / so, at 1, 16, 32, 48, 64 requests: 5.8 / 4.3, 9.4 / 6.7, 14.1 / 9.2, 17.6 / 12.9, 24.5 / 16.7 (67 MB of S at 64); time mixing of
+// 64 x 64 4.2 / 3.9, 5.9 / 5.0, 8.2 / 6.5, 10.6 / 7.7, 12.2 / 8.4.
+// LOW: the decays' second product is formed here, too, by as many neighbouring lanes to a channel as there are, from weights that are asked for first: of
+// rank 128 6.4 us in two launches / 6.2, 9.2 / 7.7, 15.6 / 10.0, 19.5 / 13.8, 24.4 / 18.8.
+#define STEP_THREADS 512
+#define LOW_AHEAD 2              // runs of 8 that a lane has on their way at once
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 gla_bf16x8;
+template <typename T, typename TO, int STEP_COLS, bool LOW>
+__global__ __launch_bounds__(STEP_THREADS) __attribute__((amdgpu_waves_per_eu(STEP_COLS == 8 ? 3 : 4))) void gla_step_kernel(GlaArgs a, int KS) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // the token's decays, q, k, TIME_MIX: u k q [4 KS] each, its outputs [dv]
   const int r = blockIdx.x, head = blockIdx.y, n = a.q_len[r];
   if (n <= 0) return;
   const int t0 = a.q_start[r], d = a.d, dv = a.dv, H = a.H, dpad = 4 * KS, groups = blockDim.x / KS;
   const int tid = threadIdx.x, lane = tid % WAVE, s = tid % KS, j0 = tid / KS;      // column i of the thread: j0 + groups i
-  float *la = lds, *lo = lds + dpad;
+  float *la = lds, *lq = lds + dpad, *lk = lds + 2 * dpad, *lu = lds + 3 * dpad, *lo = lds + 4 * dpad;
   float* sp = a.state + (size_t)a.slots[r] * a.state_stride + a.state_offset + (size_t)head * dv * dpad;      // (the same for all
   const unsigned own = 4 * s;                                                   // threads: a thread's places are 32-bit offsets from it)
-  float4 S[STEP_COLS];
-#pragma unroll
-  for (int i = 0; i < STEP_COLS; ++i) {
-    const int j = j0 + groups * i;
-    S[i] = j < dv ? *(const float4*)(sp + (own + (unsigned)(j * dpad))) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  const T *rq = (const T*)a.q, *rk = (const T*)a.k, *rv = (const T*)a.v, *rg = (const T*)a.g;
+  const T *rq = (const T*)a.q + head * d, *rk = (const T*)a.k + head * d, *rv = (const T*)a.v + head * dv, *rg = (const T*)a.g + head * dv;
+  const float* u_h = TIME_MIX ? a.bonus + head * d : nullptr;
   const LaneSteps steps = lane_steps(KS);
   const auto weight_of = [&](int c) { return load_dyn(a.norm_w, a.norm_dtype, TIME_MIX ? head * dv + c : c); };
-  const float weight = tid < dv ? weight_of(tid) : 0.f;
-  float u4[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) u4[c] = TIME_MIX && 4 * s + c < d ? a.bonus[head * d + 4 * s + c] : 0.f;
+  // LOW: a channel of the decays by ``share`` neighbouring lanes, each its runs of 8 of the rank; else a channel a thread
+  int share = 1;
+  if (LOW)
+    while (2 * share <= WAVE && 2 * share * dpad <= (int)blockDim.x) share *= 2;
+  const LaneSteps shares = lane_steps(share);
+  const int c0 = min(tid / share, d - 1), per_trip = blockDim.x / share;
+  const auto decay = [&](float z) { return expf(TIME_MIX ? -expf(z) : log_sigmoid(z) * a.inv_tau); };
   for (int t = t0; t < t0 + n; ++t) {
-    const size_t at = (size_t)t * a.ld;
-    const float g = tid < dv ? to_f(rg[at + head * dv + tid]) : 0.f;
-    float q[4], k[4], v[STEP_COLS];
+    // (the token's rows: bases that all threads share, a thread's places 32-bit offsets from them)
+    const T *q_t = rq + (size_t)t * a.ld, *k_t = rk + (size_t)t * a.ld, *v_t = rv + (size_t)t * a.ld, *g_t = rg + (size_t)t * a.ld;
+    const bf16_t *low_t = LOW ? a.low + (size_t)t * a.low_ld : nullptr, *w2_h = LOW ? a.w2 + (size_t)head * d * a.rank : nullptr;
+    const float* z_t = LOW ? nullptr : a.z + (size_t)t * (H * d) + head * d;
+    const unsigned my_value = min(tid, dv - 1);
+    // Every load of the token goes out before any is used, without a branch between them (where a thread has nothing it asks for somebody else's): those
+    // of the decays ahead, then q, k and v, then S, which arrives last and is waited for last.
+    gla_bf16x8 lv[LOW_AHEAD], wv[LOW_AHEAD];      // (of the thread's first channel)
+    float z0 = 0.f;
+    if constexpr (LOW) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int ch = 4 * s + c;
-      q[c] = ch < d ? to_f(rq[at + head * d + ch]) * a.q_scale : 0.f;
-      k[c] = ch < d ? to_f(rk[at + head * d + ch]) : 0.f;
+      for (int i = 0; i < LOW_AHEAD; ++i) {
+        const int e = min(8 * (tid % share + share * i), a.rank - 8);
+        lv[i] = *(const gla_bf16x8*)(low_t + (unsigned)e);
+        wv[i] = *(const gla_bf16x8*)(w2_h + (unsigned)(c0 * a.rank + e));
+      }
+    } else {
+      z0 = z_t[(unsigned)c0];
     }
+    const float* zb = a.z_bias ? a.z_bias + head * d : (const float*)sp;      // (without a bias: any float, dropped)
+    const float zb0 = zb[(unsigned)c0];
+    const T v0 = v_t[my_value];
+    const unsigned my_channel = min(tid, d - 1);
+    const T q0 = q_t[my_channel], k0 = k_t[my_channel];
+    const float u0 = TIME_MIX ? u_h[my_channel] : 0.f;
+    float4 S[STEP_COLS];      // (a token's own: where a request has several, a thread reads again what it has written)
 #pragma unroll
-    for (int i = 0; i < STEP_COLS; ++i) v[i] = j0 + groups * i < dv ? to_f(rv[at + head * dv + j0 + groups * i]) : 0.f;
+    for (int i = 0; i < STEP_COLS; ++i) S[i] = *(const float4*)(sp + (own + (unsigned)(min(j0 + groups * i, dv - 1) * dpad)));
+    const T g = g_t[my_value];
+    const float weight = weight_of(my_value);
+    for (int c = tid / share; c < dpad; c += per_trip) {          // (LOW: a channel's lanes are of one wave, and go on or leave together)
+      const bool first = c == tid / share, in = c < d;
+      float z = 0.f;
+      if constexpr (LOW) {
+        if (first) {
+#pragma unroll
+          for (int i = 0; i < LOW_AHEAD; ++i) {
+            float p = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) p = fmaf((float)lv[i][e], (float)wv[i][e], p);
+            z += 8 * (tid % share + share * i) < a.rank ? p : 0.f;
+          }
+        }
+        for (int r8 = 8 * (tid % share + (first ? share * LOW_AHEAD : 0)); r8 < a.rank; r8 += 8 * share) {
+          const gla_bf16x8 l = *(const gla_bf16x8*)(low_t + (unsigned)r8), w = *(const gla_bf16x8*)(w2_h + (unsigned)(min(c, d - 1) * a.rank + r8));
+#pragma unroll
+          for (int e = 0; e < 8; ++e) z = fmaf((float)l[e], (float)w[e], z);
+        }
+        z = column_sum(z, shares);
+      } else {
+        z = first ? z0 : z_t[(unsigned)min(c, d - 1)];
+      }
+      if (a.z_bias) z += first ? zb0 : zb[min(c, d - 1)];
+      if (tid % share == 0) la[c] = in ? decay(z) : 0.f;
+    }
+    // the values lie where the outputs will: a column's is read by its lanes, which are of one wave, before one of them writes the output
+    if (tid < dv) lo[tid] = to_f(v0);
+    for (int c = tid + blockDim.x; c < dv; c += blockDim.x) lo[c] = to_f(v_t[c]);
     for (int c = tid; c < dpad; c += blockDim.x) {
-      const float z = c < d ? a.z[(size_t)t * (H * d) + head * d + c] + (a.z_bias ? a.z_bias[head * d + c] : 0.f) : 0.f;
-      la[c] = expf(TIME_MIX ? -expf(z) : log_sigmoid(z) * a.inv_tau);
+      const bool first = c == tid;
+      const unsigned ch = min(c, d - 1);
+      const float q = c < d ? to_f(first ? q0 : q_t[ch]) * a.q_scale : 0.f, k = c < d ? to_f(first ? k0 : k_t[ch]) : 0.f;
+      lq[c] = q;
+      lk[c] = k;
+      if (TIME_MIX) lu[c] = (first ? u0 : u_h[ch]) * k * q;
     }
-    float b = 0.f;                       // TIME_MIX: sum_i u[i] k[i] q[i]
-    if (TIME_MIX) b = column_sum((u4[0] * k[0] * q[0] + u4[1] * k[1] * q[1]) + (u4[2] * k[2] * q[2] + u4[3] * k[3] * q[3]), steps);
     LDS_BARRIER();
-    const float4 al = *(const float4*)(la + 4 * s);
-    const bool last = t == t0 + n - 1;
+    const float4 al = *(const float4*)(la + 4 * s), q = *(const float4*)(lq + 4 * s), k = *(const float4*)(lk + 4 * s);
+    float b = 0.f;                       // TIME_MIX: sum_i u[i] k[i] q[i]
+    if (TIME_MIX) {
+      const float4 u = *(const float4*)(lu + 4 * s);
+      b = column_sum((u.x + u.y) + (u.z + u.w), steps);
+    }
 #pragma unroll
     for (int i = 0; i < STEP_COLS; ++i) {
       const int j = j0 + groups * i;
+      const float vf = lo[min(j, dv - 1)];
       float o = 0.f;
-      if (TIME_MIX) o = (S[i].x * q[0] + S[i].y * q[1]) + (S[i].z * q[2] + S[i].w * q[3]);        // (the read-out comes before the write)
-      S[i].x = fmaf(al.x, S[i].x, k[0] * v[i]);
-      S[i].y = fmaf(al.y, S[i].y, k[1] * v[i]);
-      S[i].z = fmaf(al.z, S[i].z, k[2] * v[i]);
-      S[i].w = fmaf(al.w, S[i].w, k[3] * v[i]);
-      if (last && j < dv) *(float4*)(sp + (own + (unsigned)(j * dpad))) = S[i];
-      if (!TIME_MIX) o = (S[i].x * q[0] + S[i].y * q[1]) + (S[i].z * q[2] + S[i].w * q[3]);
+      if (TIME_MIX) o = (S[i].x * q.x + S[i].y * q.y) + (S[i].z * q.z + S[i].w * q.w);        // (the read-out comes before the write)
+      S[i].x = fmaf(al.x, S[i].x, k.x * vf);
+      S[i].y = fmaf(al.y, S[i].y, k.y * vf);
+      S[i].z = fmaf(al.z, S[i].z, k.z * vf);
+      S[i].w = fmaf(al.w, S[i].w, k.w * vf);
+      if (j < dv) *(float4*)(sp + (own + (unsigned)(j * dpad))) = S[i];
+      if (!TIME_MIX) o = (S[i].x * q.x + S[i].y * q.y) + (S[i].z * q.z + S[i].w * q.w);
       o = column_sum(o, steps);
-      if (TIME_MIX) o = fmaf(b, v[i], o);
+      if (TIME_MIX) o = fmaf(b, vf, o);
       if (s == 0 && j < dv) lo[j] = o;
     }
     LDS_BARRIER();
@@ -312,9 +372,9 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(GlaArgs a, int KS) {
     for (int c = lane; c < dv; c += WAVE) ss = fmaf(lo[c], lo[c], ss);
     const float inv = rsqrtf(wave_sum(ss) / (float)dv + a.eps);
     TO* out = (TO*)a.out + (size_t)t * (H * dv) + head * dv;
-    if (tid < dv) out[tid] = from_f<TO>(lo[tid] * inv * weight * act_silu(g));
-    for (int c = tid + blockDim.x; c < dv; c += blockDim.x) out[c] = from_f<TO>(lo[c] * inv * weight_of(c) * act_silu(to_f(rg[at + head * dv + c])));
-    if (!last) LDS_BARRIER();          // (the next token's decays and outputs overwrite what this one read)
+    if (tid < dv) out[tid] = from_f<TO>(lo[tid] * inv * weight * act_silu(to_f(g)));
+    for (int c = tid + blockDim.x; c < dv; c += blockDim.x) out[c] = from_f<TO>(lo[c] * inv * weight_of(c) * act_silu(to_f(g_t[c])));
+    if (t + 1 < t0 + n) LDS_BARRIER();          // (the next token's decays and outputs overwrite what this one read)
   }
 }
 
@@ -661,18 +721,26 @@ static void launch_gla_cols(const GlaArgs& a, int units, int cols, int threads, 
 // The threads of gla_step_kernel for a head of these sizes, 0 where it does not take them.
 static int step_threads(int dpad, int dv, int cols) {
   const int lanes = dpad / 4, threads = (lanes * ((dv + cols - 1) / cols) + WAVE - 1) / WAVE * WAVE;
-  return lanes <= WAVE && threads <= 1024 ? threads : 0;
+  return lanes <= WAVE && threads <= STEP_THREADS ? threads : 0;
 }
 
 template <typename T, typename TO, int DP>
 static int launch_gla(const GlaArgs& a, int T_rows, int R, int n_chunks, const int* req_chunk0, hipStream_t s) {
   if constexpr (sizeof(TO) == 2) {         // (in 32 bits a token's bits are the same alone and among others of its request: the walk's)
-    const bool many = (long long)R * a.H > STEP_MANY_HEADS || step_threads(a.parts * DP, a.dv, 4) == 0;
-    const int threads = n_chunks == 0 && T_rows <= R ? step_threads(a.parts * DP, a.dv, many ? 8 : 4) : 0;
+    const int cols = step_threads(a.parts * DP, a.dv, 4) > 0 ? 4 : 8, threads = n_chunks == 0 && T_rows <= R ? step_threads(a.parts * DP, a.dv, cols) : 0;
     if (threads > 0) {
-      const size_t lds = (size_t)(a.parts * DP + a.dv) * sizeof(float);
-      if (many) hipLaunchKernelGGL((gla_step_kernel<T, TO, 8>), dim3(R, a.H), dim3(threads), lds, s, a, a.parts * DP / 4);
-      else hipLaunchKernelGGL((gla_step_kernel<T, TO, 4>), dim3(R, a.H), dim3(threads), lds, s, a, a.parts * DP / 4);
+      const size_t lds = (size_t)(4 * a.parts * DP + a.dv) * sizeof(float);
+#define STEP(COLS, LOW) hipLaunchKernelGGL((gla_step_kernel<T, TO, COLS, LOW>), dim3(R, a.H), dim3(threads), lds, s, a, a.parts * DP / 4)
+      if constexpr (!TIME_MIX && sizeof(T) == 2) {
+        if (a.low) {
+          if (cols == 4) STEP(4, true);
+          else STEP(8, true);
+          IFX_LAUNCH_CHECK();
+        }
+      }
+      if (cols == 4) STEP(4, false);
+      else STEP(8, false);
+#undef STEP
       IFX_LAUNCH_CHECK();
     }
   }
@@ -681,6 +749,7 @@ static int launch_gla(const GlaArgs& a, int T_rows, int R, int n_chunks, const i
   // by reading and writing S: 23 against 33 us for 64 requests of 16 heads x 64 x 128; chunks side by side: 86 + 64 against
   // 95 + 67 us for 2,048 rows), more only where a head's columns would not fit a workgroup otherwise.  The first d threads also
   // load, so a head of few values still gets a thread per key channel.
+  IFX_REQUIRE(a.z, "gla_scan: the decays' second product is formed in steps of single tokens only (bfloat16, heads that gla_step_takes)");
   constexpr int MAX_COLS = DP <= 16 ? 4 : (DP <= 32 ? 2 : 1);
   const auto threads_for = [&](int cols) { return ((max((a.dv + cols - 1) / cols * a.parts, a.d) + WAVE - 1) / WAVE) * WAVE; };
   // (time mixing's heads have as few values as keys: with two columns a thread a head of 64 x 64 would be two waves)
@@ -712,8 +781,11 @@ static int launch_gla(const GlaArgs& a, int T_rows, int R, int n_chunks, const i
 
 // dp: channels a thread holds (16, 32, 64 or 128); parts: a power of two with parts * dp >= d; a head's columns, 1-4 a thread,
 // times parts must fit a workgroup.
+// z null: z = w2 low with low [T, rank] bfloat16, rows low_ld apart, both on 16 bytes, rank a multiple of 8 (see ifx_gla_step_takes).
+extern "C" int ifx_gla_step_takes(int dpad, int dv) { return !TIME_MIX && step_threads(dpad, dv, 8) > 0 ? 1 : 0; }
+
 extern "C" int ifx_gla_scan(const void* q, const void* k, const void* v, const void* g, int dtype, int out_dtype, int ld, const float* z,
-                            const float* z_bias, float inv_tau, float q_scale, float eps, const void* norm_w, int norm_dtype, const float* bonus,
+                            const void* low, int low_ld, const void* w2, int rank, const float* z_bias, float inv_tau, float q_scale, float eps, const void* norm_w, int norm_dtype, const float* bonus,
                             float* state, long long state_stride, long long state_offset, const int* q_start, const int* q_len,
                             const int* slots, void* out, int T, int R, int H, int d, int dv, int dp, int parts,
                             int n_chunks, const int* chunk_req, const int* chunk_t0, const int* chunk_len,
@@ -726,8 +798,11 @@ extern "C" int ifx_gla_scan(const void* q, const void* k, const void* v, const v
   IFX_REQUIRE(n_chunks == 0 || (chunk_req && chunk_t0 && chunk_len && req_chunk0 && chunk_state && chunk_loga), "gla_scan: chunks without their lists");
   IFX_REQUIRE((size_t)STAGE * (4 * d + dv) * sizeof(float) <= 64 * 1024, "gla_scan: d=%d, dv=%d need more LDS than a workgroup has", d, dv);
   IFX_REQUIRE(!TIME_MIX || bonus, "time mixing needs the bonus per channel");
+  IFX_REQUIRE((z == nullptr) == (low != nullptr) && (low != nullptr) == (w2 != nullptr), "gla_scan: the decays' logits, or what they are the product of");
+  IFX_REQUIRE(!low || (rank > 0 && rank % 8 == 0 && low_ld >= rank && low_ld % 8 == 0 && (uintptr_t)low % 16 == 0 && (uintptr_t)w2 % 16 == 0),
+              "gla_scan: a product of rank %d, rows %d apart (multiples of 8, on 16 bytes)", rank, low_ld);
   if (T == 0 || R == 0) return 0;
-  GlaArgs a{q, k, v, g, ld, z, z_bias, inv_tau, q_scale, eps, norm_w, norm_dtype, bonus, state,
+  GlaArgs a{q, k, v, g, ld, z, (const bf16_t*)low, (const bf16_t*)w2, low_ld, rank, z_bias, inv_tau, q_scale, eps, norm_w, norm_dtype, bonus, state,
             (size_t)state_stride, (size_t)state_offset, q_start, q_len, slots, out, H, d, dv, parts,
             chunk_req, chunk_t0, chunk_len, chunk_state, chunk_loga};
   hipStream_t s = (hipStream_t)stream;

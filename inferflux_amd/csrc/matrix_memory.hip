@@ -175,133 +175,94 @@ __global__ __launch_bounds__(256) void memory_finish_kernel(MemoryArgs a) {
     a.state[(size_t)a.slots[r] * a.state_stride + h] = a.m_end[(size_t)r * a.H + h];
 }
 
-// Steps of single tokens: a workgroup takes all columns of a (request, head), CH channels a thread (16, or 32 where a head then fits a
-// workgroup), so that the gates are formed once a head, the normaliser and the norm are there with the outputs, and nothing goes through memory to
-// a second launch.  Bound by S, which is read and written once, and for few requests by two trips to memory (16 heads of 64 x 128, 1 / 16 / 64
-// requests: 8.1 / 11.2 / 24.8 us with the walk and the launch that finishes it, so 5.0 / 7.3 / 22.3, 67 MB of S at 64).  A thread's channels are runs
-// of four, KS runs apart, so that neighbouring lanes ask for neighbouring pieces.  The gates are formed by every wave: S is still on its way.
-template <typename TI, typename TO, int CH>
+// Steps of single tokens (a request's tokens one after the other where it has more): a workgroup takes all columns of a (request, head), so that the gates
+// are formed once a head, the normaliser and the norm are there with the outputs, and nothing goes through memory to a second launch.  Bound by S,
+// which is read and written once, and for few requests by a trip to memory and the arithmetic behind it.  A thread has V runs of four channels (two where
+// a column has more than 256) of COLS columns, the threads of a column neighbours: a wave's load is 1 KB of contiguous memory; the normaliser's column
+// is the first such threads' own.  q, k, v and the gates are formed once and meet in LDS; every load goes out before any is used, without branches
+// between them, so that what meets there is waited for while S is on its way.  16 heads of 64 x 128, us with 16 channels of one column to a thread / 4
+// columns / 8 columns, at 1, 16, 24, 32, 48 requests: 5.0 / 4.9, 7.3 / 7.3, 11.0 / 8.8, 12.0 / 9.7, 16.8 / 13.6, and at 64 22.3 / 18.1 / 16.9 (67 MB of S).
+#define STEP_MANY_HEADS 768      // (request, head) pairs beyond which eight columns, in four waves, are the better choice
+template <typename TI, typename TO, int V, int COLS>
 __global__ __launch_bounds__(1024) void memory_step_kernel(MemoryArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];      // q and k of a token [dpad] each, its outputs [dv + 1]
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // q and k of a token [dpad] each, its values, in whose place its outputs [dv + 1]
+  __shared__ float gate_s[3];                                       // keep, write, exp(-m)
   const int h = blockIdx.x, r = blockIdx.y, n = a.q_len[r];
   if (n <= 0) return;
-  const int t0 = a.q_start[r], d = a.d, dv = a.dv, KS = a.KS, dpad = CH * KS;
+  const int t0 = a.q_start[r], d = a.d, dv = a.dv, KS = a.KS, dpad = 4 * V * KS, groups = blockDim.x / KS;
   float *q_s = lds, *k_s = lds + dpad, *o_s = lds + 2 * dpad;
-  const int tid = threadIdx.x, lane = tid % WAVE, jl = tid / KS, s = tid % KS;
-  const bool owner = jl <= dv, value = jl < dv;
-  float* row = a.state + (size_t)a.slots[r] * a.state_stride;
-  float* Sp = row + a.s_off + ((size_t)h * (dv + 1) + (owner ? jl : 0)) * dpad + 4 * s;
-  float4 S[CH / 4];
-#pragma unroll
-  for (int j = 0; j < CH / 4; ++j) S[j] = owner ? *(const float4*)(Sp + 4 * KS * j) : make_float4(0.f, 0.f, 0.f, 0.f);
-  float m = row[h];
-  const float ib = a.i_bias[h], fb = a.f_bias[h], weight = value ? a.norm_w[(size_t)h * dv + jl] : 0.f;
-  const TI* rows = (const TI*)a.rows;
-  const LaneSteps steps = lane_steps(KS);
-  for (int t = t0; t < t0 + n; ++t) {
-    const TI* x = rows + (size_t)t * a.ld;
-    const float* gates = a.gates + (size_t)t * a.ldg;
-    const float v = value ? to_f(x[a.v_col + (size_t)h * dv + jl]) : 1.f, g = value ? to_f(x[a.g_col + (size_t)h * dv + jl]) : 0.f;
-    for (int c = tid; c < dpad; c += blockDim.x) {
-      q_s[c] = c < d ? to_f(x[a.q_col + (size_t)h * d + c]) * a.q_scale : 0.f;
-      k_s[c] = c < d ? to_f(x[a.k_col + (size_t)h * d + c]) : 0.f;
-    }
-    const float li = soft_cap(gates[a.i_col + h] + ib, a.cap), lf = log_sigmoid(soft_cap(gates[a.f_col + h] + fb, a.cap));
-    const float mt = fmaxf(m + lf, li), keep = expf(lf + m - mt), wv = expf(li - mt) * v;
-    m = mt;
-    __syncthreads();
-    float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int j = 0; j < CH / 4; ++j) {
-      const float4 k = *(const float4*)(k_s + 4 * (s + KS * j)), q = *(const float4*)(q_s + 4 * (s + KS * j));
-      S[j].x = fmaf(k.x, wv, keep * S[j].x), o4.x = fmaf(S[j].x, q.x, o4.x);
-      S[j].y = fmaf(k.y, wv, keep * S[j].y), o4.y = fmaf(S[j].y, q.y, o4.y);
-      S[j].z = fmaf(k.z, wv, keep * S[j].z), o4.z = fmaf(S[j].z, q.z, o4.z);
-      S[j].w = fmaf(k.w, wv, keep * S[j].w), o4.w = fmaf(S[j].w, q.w, o4.w);
-    }
-    const float o = column_sum((o4.x + o4.y) + (o4.z + o4.w), steps);
-    if (owner && s == 0) o_s[jl] = o;
-    if (t == t0 + n - 1 && owner) {
-#pragma unroll
-      for (int j = 0; j < CH / 4; ++j) *(float4*)(Sp + 4 * KS * j) = S[j];
-    }
-    __syncthreads();
-    const float inv_den = 1.0f / (fmaxf(fabsf(o_s[dv]), expf(-mt)) + 1e-6f);      // (as memory_finish_kernel)
-    float ss = 0.f;
-    for (int c = lane; c < dv; c += WAVE) { const float w = o_s[c] * inv_den; ss = fmaf(w, w, ss); }
-    const float f = inv_den / sqrtf(wave_sum(ss) / (float)dv + a.eps);
-    if (value && s == 0) ((TO*)a.out)[((size_t)t * a.H + h) * dv + jl] = from_f<TO>(o * f * weight / (1.0f + expf(-g)));
-    if (t < t0 + n - 1) __syncthreads();          // (the next token's q, k and outputs overwrite what this one read)
-  }
-  if (tid == 0) row[h] = m;
-}
-
-// The same for more (request, head) pairs than compute units, where S is what bounds it: a thread has four channels of up to STEP_COLS columns, the
-// dpad / 4 threads of a column neighbours, so that a wave's load is 1 KB of contiguous memory, q and k are a thread's own, and a workgroup (four waves
-// for 64 x 128) leaves room for three others on its compute unit.  16 heads
-// of 64 x 128, us as above / so at 16, 24, 32, 48, 64 requests: 7.3 / 8.3, 11.0 / 10.3, 12.0 / 11.2, 16.8 / 13.6, 22.3 / 16.4 (67 MB of S at 64); hence
-// the line.  (With 3 to 5 columns to a thread, and more waves, 64 requests take 21 to 27.)
-#define STEP_COLS 9
-#define MANY_HEADS 256
-template <typename TI, typename TO>
-__global__ __launch_bounds__(1024) void memory_steps_kernel(MemoryArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float o_s[];      // the token's outputs [dv + 1]
-  const int h = blockIdx.x, r = blockIdx.y, n = a.q_len[r];
-  if (n <= 0) return;
-  const int t0 = a.q_start[r], d = a.d, dv = a.dv, KS = a.KS, dpad = 4 * KS, groups = blockDim.x / KS;
   const int tid = threadIdx.x, lane = tid % WAVE, s = tid % KS, j0 = tid / KS;      // column i of the thread: j0 + groups i
   float* row = a.state + (size_t)a.slots[r] * a.state_stride;
   float* Sp = row + a.s_off + (size_t)h * (dv + 1) * dpad;      // (the same for all threads: a thread's places are 32-bit offsets from it)
-  const unsigned own = 4 * s;
-  float4 S[STEP_COLS];
-#pragma unroll
-  for (int i = 0; i < STEP_COLS; ++i) {
-    const int j = j0 + groups * i;
-    S[i] = j <= dv ? *(const float4*)(Sp + (own + (unsigned)(j * dpad))) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  float m = row[h];
-  const float ib = a.i_bias[h], fb = a.f_bias[h], weight = tid < dv ? a.norm_w[(size_t)h * dv + tid] : 0.f;
-  const TI* rows = (const TI*)a.rows;
+  const unsigned own = 4 * s, my_channel = min(tid, d - 1), my_value = min(tid, dv - 1);
   const LaneSteps steps = lane_steps(KS);
+  float m = row[h];
+  const float ib = a.i_bias[h], fb = a.f_bias[h];
   for (int t = t0; t < t0 + n; ++t) {
-    const TI* x = rows + (size_t)t * a.ld;
+    const TI* x = (const TI*)a.rows + (size_t)t * a.ld;
+    const TI *q_t = x + a.q_col + (size_t)h * d, *k_t = x + a.k_col + (size_t)h * d, *v_t = x + a.v_col + (size_t)h * dv, *g_t = x + a.g_col + (size_t)h * dv;
     const float* gates = a.gates + (size_t)t * a.ldg;
-    const float g = tid < dv ? to_f(x[a.g_col + (size_t)h * dv + tid]) : 0.f;
-    float q[4], k[4], v[STEP_COLS];
+    const float zi = gates[a.i_col + h], zf = gates[a.f_col + h];
+    const TI q0 = q_t[my_channel], k0 = k_t[my_channel], v0 = v_t[my_value];
+    float4 S[COLS][V], N[V];      // (a token's own: where a request has several, a thread reads again what it has written)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int c = 4 * s + e;
-      q[e] = c < d ? to_f(x[a.q_col + (size_t)h * d + c]) * a.q_scale : 0.f;
-      k[e] = c < d ? to_f(x[a.k_col + (size_t)h * d + c]) : 0.f;
+    for (int i = 0; i < COLS; ++i)
+#pragma unroll
+      for (int u = 0; u < V; ++u) S[i][u] = *(const float4*)(Sp + (own + (unsigned)(min(j0 + groups * i, dv - 1) * dpad + 4 * KS * u)));
+#pragma unroll
+    for (int u = 0; u < V; ++u) N[u] = *(const float4*)(Sp + (own + (unsigned)(dv * dpad + 4 * KS * u)));
+    const TI g = g_t[my_value];
+    const float weight = a.norm_w[(size_t)h * dv + my_value];
+    for (int c = tid; c < dpad; c += blockDim.x) {
+      q_s[c] = c < d ? to_f(c == tid ? q0 : q_t[c]) * a.q_scale : 0.f;
+      k_s[c] = c < d ? to_f(c == tid ? k0 : k_t[c]) : 0.f;
     }
-#pragma unroll
-    for (int i = 0; i < STEP_COLS; ++i) v[i] = j0 + groups * i < dv ? to_f(x[a.v_col + (size_t)h * dv + j0 + groups * i]) : 1.f;
-    const float li = soft_cap(gates[a.i_col + h] + ib, a.cap), lf = log_sigmoid(soft_cap(gates[a.f_col + h] + fb, a.cap));
-    const float mt = fmaxf(m + lf, li), keep = expf(lf + m - mt), write = expf(li - mt);
-    m = mt;
-    const bool last = t == t0 + n - 1;
-#pragma unroll
-    for (int i = 0; i < STEP_COLS; ++i) {
-      const int j = j0 + groups * i;
-      const float wv = write * v[i];
-      S[i].x = fmaf(k[0], wv, keep * S[i].x);
-      S[i].y = fmaf(k[1], wv, keep * S[i].y);
-      S[i].z = fmaf(k[2], wv, keep * S[i].z);
-      S[i].w = fmaf(k[3], wv, keep * S[i].w);
-      if (last && j <= dv) *(float4*)(Sp + (own + (unsigned)(j * dpad))) = S[i];
-      const float o = column_sum((S[i].x * q[0] + S[i].y * q[1]) + (S[i].z * q[2] + S[i].w * q[3]), steps);
-      if (s == 0 && j <= dv) o_s[j] = o;
+    // (a column's value is read by its lanes, which are of one wave, before one of them writes the output in its place)
+    if (tid < dv) o_s[tid] = to_f(v0);
+    for (int c = tid + blockDim.x; c < dv; c += blockDim.x) o_s[c] = to_f(v_t[c]);
+    const float li = soft_cap(zi + ib, a.cap), lf = log_sigmoid(soft_cap(zf + fb, a.cap)), mt = fmaxf(m + lf, li);
+    if (tid < WAVE) {                  // (the first wave, which alone keeps m)
+      if (lane == 0) { gate_s[0] = expf(lf + m - mt); gate_s[1] = expf(li - mt); gate_s[2] = expf(-mt); }
+      m = mt;
     }
     LDS_BARRIER();
-    const float inv_den = 1.0f / (fmaxf(fabsf(o_s[dv]), expf(-mt)) + 1e-6f);      // (as memory_finish_kernel)
+    const float keep = gate_s[0], write = gate_s[1], floor = gate_s[2];
+    float4 q[V], k[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) { q[u] = *(const float4*)(q_s + own + 4 * KS * u); k[u] = *(const float4*)(k_s + own + 4 * KS * u); }
+    auto column = [&](float4 (&S4)[V], float wv, unsigned at, bool held) {
+      float o = 0.f;
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        S4[u].x = fmaf(k[u].x, wv, keep * S4[u].x);
+        S4[u].y = fmaf(k[u].y, wv, keep * S4[u].y);
+        S4[u].z = fmaf(k[u].z, wv, keep * S4[u].z);
+        S4[u].w = fmaf(k[u].w, wv, keep * S4[u].w);
+        if (held) *(float4*)(Sp + (own + at + 4 * KS * u)) = S4[u];
+        o += (S4[u].x * q[u].x + S4[u].y * q[u].y) + (S4[u].z * q[u].z + S4[u].w * q[u].w);
+      }
+      return column_sum(o, steps);
+    };
+#pragma unroll
+    for (int i = 0; i < COLS; ++i) {
+      const int j = j0 + groups * i;
+      const float o = column(S[i], write * o_s[min(j, dv - 1)], (unsigned)(j * dpad), j < dv);
+      if (s == 0 && j < dv) o_s[j] = o;
+    }
+    if (tid < WAVE) {                  // the normaliser's column, of value 1
+      const float o = column(N, write, (unsigned)(dv * dpad), tid < KS);
+      if (tid == 0) o_s[dv] = o;
+    }
+    LDS_BARRIER();
+    const float inv_den = 1.0f / (fmaxf(fabsf(o_s[dv]), floor) + 1e-6f);      // (as memory_finish_kernel)
     float ss = 0.f;
     for (int c = lane; c < dv; c += WAVE) { const float w = o_s[c] * inv_den; ss = fmaf(w, w, ss); }
     const float f = inv_den / sqrtf(wave_sum(ss) / (float)dv + a.eps);
     TO* out = (TO*)a.out + ((size_t)t * a.H + h) * dv;
-    if (tid < dv) out[tid] = from_f<TO>(o_s[tid] * f * weight / (1.0f + expf(-g)));
+    if (tid < dv) out[tid] = from_f<TO>(o_s[tid] * f * weight / (1.0f + expf(-to_f(g))));
     for (int c = tid + blockDim.x; c < dv; c += blockDim.x)
-      out[c] = from_f<TO>(o_s[c] * f * a.norm_w[(size_t)h * dv + c] / (1.0f + expf(-to_f(x[a.g_col + (size_t)h * dv + c]))));
-    if (!last) LDS_BARRIER();          // (the next token's outputs overwrite what this one read)
+      out[c] = from_f<TO>(o_s[c] * f * a.norm_w[(size_t)h * dv + c] / (1.0f + expf(-to_f(g_t[c]))));
+    if (t + 1 < t0 + n) LDS_BARRIER();          // (the next token's q, k, gates and outputs overwrite what this one read)
   }
   if (tid == 0) row[h] = m;
 }
@@ -665,20 +626,20 @@ extern "C" int ifx_matrix_memory(const void* rows, int dtype, int ld, int q_col,
     else hipLaunchKernelGGL((memory_finish_kernel<bf16_t, float>), dim3(blocks), dim3(256), 0, s, a);
     IFX_LAUNCH_CHECK();
   }
-  const int dpad = ch * ks, step_ch = dpad >= 32 && (dv + 1) * (dpad / 16) > 1024 ? 32 : 16, lanes = dpad / 4;
-  const int steps_threads = (lanes * ((dv + STEP_COLS) / STEP_COLS) + WAVE - 1) / WAVE * WAVE;      // (dv + 1 columns)
-  const dim3 step_grid(H, R);
-#define STEP(TI, TO)                                                                                                                               \
-  do {                                                                                                                                             \
-    if (wide) hipLaunchKernelGGL((memory_steps_kernel<TI, TO>), step_grid, dim3(steps_threads), (size_t)(dv + 1) * sizeof(float), s, a);           \
-    else if (step_ch == 16) hipLaunchKernelGGL((memory_step_kernel<TI, TO, 16>), step_grid, step_threads, step_lds, s, a);                         \
-    else hipLaunchKernelGGL((memory_step_kernel<TI, TO, 32>), step_grid, step_threads, step_lds, s, a);                                            \
-  } while (0)
-  const bool wide = T <= R && (long long)H * R > MANY_HEADS && lanes >= 4 && lanes <= WAVE && steps_threads <= 1024;
-  if (wide || (T <= R && dpad >= 16 && (dv + 1) * (dpad / step_ch) <= 1024)) {
-    a.KS = wide ? lanes : dpad / step_ch;
+  const int dpad = ch * ks, runs = dpad > 4 * WAVE ? 2 : 1, lanes = dpad / 4 / runs;
+  const auto threads_of = [&](int cols_) { return (lanes * ((dv + cols_ - 1) / cols_) + WAVE - 1) / WAVE * WAVE; };
+  const bool four = runs > 1 || (threads_of(4) <= 1024 && (long long)H * R <= STEP_MANY_HEADS) || threads_of(8) > 1024;
+  const int step_threads = threads_of(four ? 4 : 8);
+  if (T <= R && lanes >= 4 && lanes <= WAVE && step_threads <= 1024) {
+    a.KS = lanes;
     const size_t step_lds = (size_t)(2 * dpad + dv + 1) * sizeof(float);
-    const dim3 step_threads(((dv + 1) * a.KS + WAVE - 1) / WAVE * WAVE);
+    const dim3 step_grid(H, R);
+#define STEP(TI, TO)                                                                                                             \
+  do {                                                                                                                           \
+    if (runs > 1) hipLaunchKernelGGL((memory_step_kernel<TI, TO, 2, 4>), step_grid, dim3(step_threads), step_lds, s, a);         \
+    else if (four) hipLaunchKernelGGL((memory_step_kernel<TI, TO, 1, 4>), step_grid, dim3(step_threads), step_lds, s, a);        \
+    else hipLaunchKernelGGL((memory_step_kernel<TI, TO, 1, 8>), step_grid, dim3(step_threads), step_lds, s, a);                  \
+  } while (0)
     if (dtype == DT_F32 && out_dtype == DT_F32) STEP(float, float);
     else if (dtype == DT_F32 && out_dtype == DT_BF16) STEP(float, bf16_t);
     else if (dtype == DT_BF16 && out_dtype == DT_BF16) STEP(bf16_t, bf16_t);

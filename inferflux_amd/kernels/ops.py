@@ -2326,14 +2326,26 @@ def gla_state_floats(n_heads: int, d: int, dv: int) -> int:
     return n_heads * dv * parts * dp
 
 
-def gla_scan(rows: torch.Tensor, cols: Tuple[int, int, int, int], z: torch.Tensor, z_bias: Optional[torch.Tensor], tau: float,
+def gla_step_takes(low: torch.Tensor, w2: torch.Tensor, d: int, dv: int) -> bool:
+    """Whether ``gla_scan`` forms the decays' logits of a step of single tokens itself, ``low`` [T, rank] times ``w2`` [n_heads * d, rank] transposed."""
+    rank = w2.shape[1]
+    if low.dtype != torch.bfloat16 or w2.dtype != torch.bfloat16 or rank % 8 or not w2.is_contiguous() or w2.data_ptr() % 16:
+        return False
+    if not columns_on_16_bytes(low) and (not low.is_contiguous() or low.data_ptr() % 16):
+        return False
+    dp, parts = gla_layout(d, dv)
+    return bool(load_module("gla").fn("ifx_gla_step_takes", (I, I))(dp * parts, dv))
+
+
+def gla_scan(rows: torch.Tensor, cols: Tuple[int, int, int, int], z, z_bias: Optional[torch.Tensor], tau: float,
              q_scale: float, norm_weight: torch.Tensor, eps: float, n_heads: int, d: int, dv: int, state: torch.Tensor,
              state_offset: int, q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor,
              chunks: Optional[Dict[str, object]] = None) -> torch.Tensor:
     """Gated linear attention over each request's rows, with the output's norm and gate:
     alpha = sigmoid(z + z_bias) ^ (1 / tau) per key channel; per head S <- diag(alpha) S + k v^T; o = S^T q * q_scale;
     y = o / sqrt(mean(o^2) + eps) * norm_weight * silu(g).  ``rows`` [T, ld] holds q, k (n_heads * d each), v and g
-    (n_heads * dv each) at the columns ``cols`` = (q, k, v, g); ``z`` float32 [T, n_heads * d]; ``state`` float32
+    (n_heads * dv each) at the columns ``cols`` = (q, k, v, g); ``z`` float32 [T, n_heads * d], or in steps of single tokens the two factors that
+    ``gla_step_takes``; ``state`` float32
     [slots, n] with a request's S (``gla_state_floats`` numbers, laid out for the kernel) at ``state_offset`` of its row.
     Decays, S, o, norm and gate are float.  Returns y [T, n_heads * dv] in the rows' type.
 
@@ -2347,7 +2359,15 @@ def gla_scan(rows: torch.Tensor, cols: Tuple[int, int, int, int], z: torch.Tenso
     for c, w, nm in ((q_col, HD, "q"), (k_col, HD, "k"), (v_col, HV, "v"), (g_col, HV, "g")):
         if c < 0 or c + w > ld:
             raise KernelError(f"gla_scan: the {nm} columns {c}..{c + w} lie outside rows of {ld}")
-    _check(z, "z", (T, HD), torch.float32)
+    low_args = (None, 0, None, 0)
+    if isinstance(z, tuple):
+        low, w2 = z
+        if low.shape[0] != T or w2.shape != (HD, low.shape[1]) or rows.dtype != torch.bfloat16 or T > q_start.shape[0] or chunks is not None \
+                or not gla_step_takes(low, w2, d, dv):
+            raise KernelError(f"gla_scan: the product of {tuple(low.shape)} and {tuple(w2.shape)} is not formed for {T} rows of {q_start.shape[0]} requests")
+        low_args, z = (low, low.stride(0), w2, low.shape[1]), None
+    else:
+        _check(z, "z", (T, HD), torch.float32)
     if z_bias is not None:
         _check(z_bias, "z_bias", (HD,), torch.float32)
     _check(norm_weight, "norm_weight", (dv,))
@@ -2363,13 +2383,13 @@ def gla_scan(rows: torch.Tensor, cols: Tuple[int, int, int, int], z: torch.Tenso
     n_chunks, lists, _keep = _chunk_lists(chunks, R, HV * parts * dp, HD, rows.device)
     _call(load_module("gla"), "ifx_gla_scan", _GLA_ARGS,
           base + q_col * size, base + k_col * size, base + v_col * size, base + g_col * size, _dt(rows), _dt(out), ld, z,
-          z_bias, 1.0 / float(tau), float(q_scale), float(eps), norm_weight, _dt(norm_weight), 0, state,
+          *low_args, z_bias, 1.0 / float(tau), float(q_scale), float(eps), norm_weight, _dt(norm_weight), 0, state,
           state.shape[1], int(state_offset), q_start, q_len, slots, out, T, R, n_heads, d, dv,
           dp, parts, n_chunks, *lists, _stream())
     return out
 
 
-_GLA_ARGS = (P, P, P, P, I, I, I, P, P, F, F, F, P, I, P, P, LL, LL, P, P, P, P, I, I, I, I, I, I, I, I, P, P, P, P, P, P, P)
+_GLA_ARGS = (P, P, P, P, I, I, I, P, P, I, P, I, P, F, F, F, P, I, P, P, LL, LL, P, P, P, P, I, I, I, I, I, I, I, I, P, P, P, P, P, P, P)
 
 
 def _chunk_lists(chunks: Optional[Dict[str, object]], R: int, state_floats: int, log_floats: int, device):
@@ -2451,7 +2471,7 @@ def time_mix_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     out = empty((T, HD), out_dtype, r)
     n_chunks, lists, _keep = _chunk_lists(chunks, R, HD * parts * dp, HD, r.device)
     _call(load_module("gla", TIME_MIX), "ifx_gla_scan", _GLA_ARGS,
-          r, k, v, g, _dt(r), _DT[out_dtype], lds[0], z, w0, 1.0, 1.0,
+          r, k, v, g, _dt(r), _DT[out_dtype], lds[0], z, None, 0, None, 0, w0, 1.0, 1.0,
           float(eps), norm_weight, _dt(norm_weight), u, state, state.shape[1], int(state_offset),
           q_start, q_len, slots, out, T, R, n_heads, d, d, dp, parts, n_chunks, *lists, _stream())
     return out

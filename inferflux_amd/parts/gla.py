@@ -102,7 +102,9 @@ class GatedLinearAttention(Mixer):
         a1 = rows[:, 2 * HD + 2 * HV:] if rows.shape[0] else rows.new_empty((0, r))
         if not ops.columns_on_16_bytes(a1):
             a1 = a1.contiguous()              # (``linear`` takes columns in bfloat16 on 16 bytes)
-        z = ops.linear(a1, self.w_a2, out_dtype=torch.float32)         # the decays' logits are never rounded
+        # (steps of single tokens: the recurrence's launch forms them where it can)
+        alone = 0 < ctx.n_tokens == ctx.n_requests and rows.dtype == torch.bfloat16 and ops.gla_step_takes(a1, self.w_a2.rows, self.head_dim, self.v_head_dim)
+        z = (a1, self.w_a2.rows) if alone else ops.linear(a1, self.w_a2, out_dtype=torch.float32)      # the decays' logits are never rounded
         if t is not None:
             t.mark("mixer.project")
         # A prompt's portion walked token by token leaves most of the chip idle: in bfloat16 long portions are cut into

@@ -281,11 +281,36 @@ def test_gated_linear_attention_over_steps_with_state_in_slots(dtype, H, d, dv, 
     assert abs(float((s[0, offset:offset + n_state].double() ** 2).sum()) / float((S ** 2).sum()) - 1.0) < 1e-3
 
 
+@pytest.mark.parametrize("R,H,d,dv,rank,ld", [(4, 2, 16, 1, 8, 8), (4, 3, 10, 63, 24, 32), (1, 16, 64, 128, 128, 200), (16, 16, 64, 128, 128, 128), (60, 16, 64, 128, 72, 80),
+                                              (2, 1, 64, 256, 520, 528), (3, 1, 256, 64, 16, 16), (5, 1, 100, 40, 1000, 1008), (3, 2, 32, 48, 64, 64)])
+def test_single_tokens_of_linear_attention_form_the_decays_product(R, H, d, dv, rank, ld):
+    """The decays' second product formed beside the recurrence, against the same from its float result: sums of at most 1,000 products of bfloat16 values
+    in another order move a logit by up to 1,000 2^-24 of its terms, far below what an output's rounding to bfloat16 shows but for ties of it."""
+    rows, cols, _, bias, w = _gla_inputs(5, R, H, d, dv, torch.bfloat16)
+    low, w2 = rnd(30, R, ld).bfloat16().to(DEV)[:, :rank], rnd(31, H * d, rank, scale=rank ** -0.5).bfloat16().to(DEV)
+    assert ops.gla_step_takes(low, w2, d, dv)
+    q_start, q_len = _step_arrays([1] * R)
+    slots = torch.randperm(R, generator=torch.Generator().manual_seed(2)).to(torch.int32).to(DEV)
+    outs, states = [], []
+    for z in ((low, w2), (low.double() @ w2.double().t()).float()):
+        state = torch.zeros((R, ops.gla_state_floats(H, d, dv)), device=DEV)
+        for turn in range(3):
+            out = ops.gla_scan(rows.to(DEV), cols, z, bias.to(DEV), 16.0, d ** -0.5, w.to(DEV), 1e-5, H, d, dv, state, 0, q_start.to(DEV), q_len.to(DEV), slots)
+        outs.append(out.cpu().double())
+        states.append(state.cpu().double())
+    assert rel_err(outs[0], outs[1]) < 2.0 ** -8 and rel_err(states[0], states[1]) < 1e-5
+    with pytest.raises(ops.KernelError):
+        ops.gla_scan(rows.to(DEV), cols, (low, w2[:, :8 if rank > 8 else 4]), bias.to(DEV), 16.0, 1.0, w.to(DEV), 1e-5, H, d, dv, state, 0, q_start.to(DEV), q_len.to(DEV), slots)
+    with pytest.raises(ops.KernelError):       # (two rows of a request)
+        ops.gla_scan(torch.cat([rows, rows]).to(DEV), cols, (torch.cat([low, low]), w2), bias.to(DEV), 16.0, 1.0, w.to(DEV), 1e-5, H, d, dv, state, 0,
+                     q_start.to(DEV), 2 * q_len.to(DEV), slots)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("R,H,d,dv", [(4, 2, 16, 1), (4, 3, 10, 63), (4, 4, 64, 128), (4, 2, 24, 130), (4, 1, 64, 256), (4, 1, 64, 257), (4, 1, 64, 512), (4, 1, 64, 513),
-                                      (4, 1, 256, 128), (4, 1, 256, 129), (4, 1, 100, 40), (768, 1, 16, 24), (257, 3, 10, 63), (200, 4, 64, 128)])
+@pytest.mark.parametrize("R,H,d,dv", [(4, 2, 16, 1), (4, 3, 10, 63), (4, 4, 64, 128), (4, 2, 24, 130), (4, 1, 64, 128), (4, 1, 64, 129), (4, 1, 64, 256), (4, 1, 64, 257),
+                                      (4, 1, 256, 64), (4, 1, 256, 65), (4, 1, 100, 40), (768, 1, 16, 24), (257, 3, 10, 63), (200, 4, 64, 128)])
 def test_single_tokens_of_linear_attention_against_the_walk(dtype, R, H, d, dv):
-    """Heads on both sides of what the kernel of single tokens takes, and numbers of them on both sides of its two forms: requests' tokens, twice, against the
+    """Heads on both sides of what the kernel of single tokens takes in its two forms, few and many of them: requests' tokens, twice, against the
     walk, which the same tokens take beside a request of two.  Sums of at most 256 products in another order, and one rounding to bfloat16; in 32 bits the walk takes both."""
     dt = DT[dtype]
     rows, cols, z, bias, w = _gla_inputs(5, R + 2, H, d, dv, dt)
