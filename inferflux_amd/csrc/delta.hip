@@ -231,6 +231,152 @@ __global__ __launch_bounds__(256) void delta_finish_kernel(DeltaArgs a) {
   }
 }
 
+// Steps of single tokens in bfloat16 (a request's tokens one after the other where it has more): a workgroup takes a head of a request, so that the norm is
+// there with the outputs, and with TAPS > 0 (heads with q and k of their own) the convolution before it, too.  A thread has four channels of COLS
+// columns of S, the dpad / 4 threads of a column neighbours: a wave's load is 1 KB of contiguous memory.  The convolution is a channel a thread; its
+// results and the gates meet in LDS, and every load goes out before any is used, without branches between them, so that what meets there is waited for
+// while S is on its way.  Everything between the rows and the output is float.  Bound by its launch, a trip to memory and the arithmetic behind it, for
+// many requests by S.  16 heads of 64 x 128, four taps, us in launches for the convolution, the walk and the norm / in one, at 1, 16, 32, 64
+// requests: 13.0 / 5.2, 24.0 / 7.6, 37.8 / 10.1, 70.4 / 19.7 (67 MB of S at 64).  (In 32 bits a token's bits are the same alone and among others of its request: the walk's.)
+struct StepConv {
+  const void* w;          // [2 G d + H dv][TAPS]
+  int w_dtype;
+  float* state;           // a slot's row begins with its last TAPS - 1 inputs of every channel
+};
+#define STEP_THREADS 512
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 step_bf16x4;
+template <int TAPS, int COLS>
+__global__ __launch_bounds__(STEP_THREADS) __attribute__((amdgpu_waves_per_eu(COLS == 8 ? 3 : 4))) void delta_step_kernel(DeltaArgs a, StepConv conv) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // q and k of a token [dpad] each, its values, in whose place its outputs [dv]
+  __shared__ float gate_s[2];                                       // beta, decay
+  const int h = blockIdx.x, r = blockIdx.y, n = a.q_len[r];
+  if (n <= 0) return;
+  const int t0 = a.q_start[r], d = a.d, dv = a.dv, KS = a.KS, dpad = 4 * KS, groups = blockDim.x / KS, g = h / (a.H / a.G);
+  float *q_s = lds, *k_s = lds + dpad, *o_s = lds + 2 * dpad;
+  const int tid = threadIdx.x, lane = tid % WAVE, s = tid % KS, j0 = tid / KS;      // column i of the thread: j0 + groups i
+  const unsigned own = 4 * s, my_value = min(tid, dv - 1);
+  const size_t slot = (size_t)a.slots[r] * a.state_stride;
+  float* Sp = a.state + slot + a.state_offset + (size_t)h * dv * dpad;      // (the same for all threads: a thread's places are 32-bit offsets from it)
+  static_assert(TAPS == 0 || TAPS == 4, "four taps, or no convolution");
+  const int n_in = 2 * d + dv;                     // the head's channels: q, k, v
+  const auto channel_of = [&](int i) { return i < d ? g * d + i : i < 2 * d ? a.G * d + g * d + (i - d) : 2 * a.G * d + h * dv + (i - 2 * d); };
+  const auto place_of = [&](int i) { return i < d ? q_s + i : i < 2 * d ? k_s + (i - d) : o_s + (i - 2 * d); };
+  const LaneSteps steps = lane_steps(KS);
+  const float decay_rate = a.A_log[h], dt_b = a.dt_bias[h], q_mult = 1.0f / sqrtf((float)d);
+  for (int t = t0; t < t0 + n; ++t) {
+    const bf16_t *u = (const bf16_t*)a.u + (size_t)t * a.ldu, *row = (const bf16_t*)a.rows + (size_t)t * a.ldr;
+    const bf16_t zb = row[a.col_b + h], za = row[a.col_a + h];
+    const unsigned c0 = channel_of(min(tid, n_in - 1));
+    const bf16_t x0 = u[c0];
+    float4 wf = {};
+    step_bf16x4 wh = {};
+    float b0 = 0.f, b1 = 0.f, b2 = 0.f;
+    if constexpr (TAPS > 0) {
+      const float* st = conv.state + slot + c0 * 3;
+      b0 = st[0]; b1 = st[1]; b2 = st[2];
+      if (conv.w_dtype == DT_F32) wf = ((const float4*)conv.w)[c0];
+      else wh = ((const step_bf16x4*)conv.w)[c0];
+    }
+    float4 S[COLS];      // (a token's own: where a request has several, a thread reads again what it has written)
+#pragma unroll
+    for (int i = 0; i < COLS; ++i) S[i] = *(const float4*)(Sp + (own + (unsigned)(min(j0 + groups * i, dv - 1) * dpad)));
+    const bf16_t gate = row[a.col_g + h * dv + my_value];
+    const float weight = load_dyn(a.norm_w, a.norm_dtype, my_value);
+    // one input: the convolution over it and the three before it, the last three left in the state
+    const auto put = [&](int i, unsigned c, float x, float last0, float last1, float last2, float4 w) {
+      if constexpr (TAPS > 0) {
+        float* st = conv.state + slot + c * 3;
+        st[0] = last1; st[1] = last2; st[2] = x;
+        x = act_silu(fmaf(w.w, x, fmaf(w.z, last2, fmaf(w.y, last1, w.x * last0))));
+      }
+      *place_of(i) = x;
+    };
+    const auto widened = [&](float4 f, step_bf16x4 h) { return conv.w_dtype == DT_F32 ? f : make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]); };
+    if (tid < n_in) put(tid, c0, to_f(x0), b0, b1, b2, widened(wf, wh));
+    for (int i = tid + blockDim.x; i < n_in; i += blockDim.x) {      // (a head of more channels than threads)
+      const unsigned c = channel_of(i);
+      if constexpr (TAPS > 0) {
+        const float* st = conv.state + slot + c * 3;
+        b0 = st[0]; b1 = st[1]; b2 = st[2];
+        if (conv.w_dtype == DT_F32) wf = ((const float4*)conv.w)[c];
+        else wh = ((const step_bf16x4*)conv.w)[c];
+      }
+      put(i, c, to_f(u[c]), b0, b1, b2, widened(wf, wh));
+    }
+    for (int c = d + tid; c < dpad; c += blockDim.x) { q_s[c] = 0.f; k_s[c] = 0.f; }
+    if (tid == (int)blockDim.x - 1) {               // (a thread of the last wave, which has no channel as a rule)
+      gate_s[0] = 1.0f / (1.0f + expf(-to_f(zb)));
+      gate_s[1] = expf(-expf(decay_rate) * softplus_f(to_f(za) + dt_b));
+    }
+    LDS_BARRIER();
+    const float beta = gate_s[0], decay = gate_s[1];
+    float4 q = *(const float4*)(q_s + own), k = *(const float4*)(k_s + own);
+    const float fq = q_mult / sqrtf(column_sum((q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w), steps) + 1e-6f);
+    const float fk = 1.0f / sqrtf(column_sum((k.x * k.x + k.y * k.y) + (k.z * k.z + k.w * k.w), steps) + 1e-6f);
+    q.x *= fq; q.y *= fq; q.z *= fq; q.w *= fq;
+    k.x *= fk; k.y *= fk; k.z *= fk; k.w *= fk;
+#pragma unroll
+    for (int i = 0; i < COLS; ++i) {
+      const int j = j0 + groups * i;
+      S[i].x *= decay; S[i].y *= decay; S[i].z *= decay; S[i].w *= decay;
+      const float upd = beta * (o_s[min(j, dv - 1)] - column_sum((S[i].x * k.x + S[i].y * k.y) + (S[i].z * k.z + S[i].w * k.w), steps));
+      S[i].x = fmaf(k.x, upd, S[i].x);
+      S[i].y = fmaf(k.y, upd, S[i].y);
+      S[i].z = fmaf(k.z, upd, S[i].z);
+      S[i].w = fmaf(k.w, upd, S[i].w);
+      if (j < dv) *(float4*)(Sp + (own + (unsigned)(j * dpad))) = S[i];
+      const float o = column_sum((S[i].x * q.x + S[i].y * q.y) + (S[i].z * q.z + S[i].w * q.w), steps);
+      if (s == 0 && j < dv) o_s[j] = o;           // (a column's lanes are of one wave, and have read its value)
+    }
+    LDS_BARRIER();
+    float ss = 0.f;
+    for (int c = lane; c < dv; c += WAVE) ss = fmaf(o_s[c], o_s[c], ss);
+    const float f = 1.0f / sqrtf(wave_sum(ss) / (float)dv + a.eps);
+    bf16_t* out = (bf16_t*)a.out + ((size_t)t * a.H + h) * dv;
+    if (tid < dv) out[tid] = (bf16_t)(o_s[tid] * f * weight * act_silu(to_f(gate)));
+    for (int c = tid + blockDim.x; c < dv; c += blockDim.x)
+      out[c] = (bf16_t)(o_s[c] * f * load_dyn(a.norm_w, a.norm_dtype, c) * act_silu(to_f(row[a.col_g + h * dv + c])));
+    if (t + 1 < t0 + n) LDS_BARRIER();          // (the next token's q, k, gates and outputs overwrite what this one read)
+  }
+}
+
+// The threads of delta_step_kernel for a head of these sizes, 0 where it does not take them.
+static int step_threads(int dpad, int dv, int cols) {
+  const int lanes = dpad / 4, threads = (lanes * ((dv + cols - 1) / cols) + WAVE - 1) / WAVE * WAVE;
+  return lanes <= WAVE && threads <= STEP_THREADS ? threads : 0;
+}
+extern "C" int ifx_delta_step_takes(int dpad, int dv) { return dpad >= 4 && step_threads(dpad, dv, 8) > 0 ? 1 : 0; }
+
+// ifx_delta_rule for steps of single tokens in bfloat16 (T <= R).  taps 4: u is the convolution's input, with conv_w [2 G d + H dv][4] (G == H), and
+// a slot's row begins with its state; taps 0: u is its output.  dpad: a column of S.
+extern "C" int ifx_delta_step(const void* u, int ldu, const void* conv_w, int conv_dtype, int taps, const void* rows, int ldr, int col_g, int col_b,
+                              int col_a, const float* A_log, const float* dt_bias, const void* norm_w, int norm_dtype, float eps, float* state,
+                              long long state_stride, long long state_offset, const int* q_start, const int* q_len, const int* slots, void* out,
+                              int T, int R, int H, int G, int d, int dv, int dpad, void* stream) {
+  IFX_REQUIRE(T >= 0 && R >= T && H > 0 && G > 0 && H % G == 0 && d > 0 && dv > 0, "delta_step: bad sizes T=%d R=%d H=%d G=%d d=%d dv=%d", T, R, H, G, d, dv);
+  IFX_REQUIRE(dpad >= d && (dpad & (dpad - 1)) == 0 && ifx_delta_step_takes(dpad, dv), "delta_step: heads of %d (%d) x %d", d, dpad, dv);
+  IFX_REQUIRE(taps == 0 || (taps == 4 && G == H && conv_w && state_offset >= (long long)3 * (2 * G * d + H * dv)), "delta_step: a convolution of %d taps (4, every head its own q and k)", taps);
+  IFX_REQUIRE((uintptr_t)conv_w % 16 == 0, "delta_step: the convolution's weight must start on 16 bytes");
+  IFX_REQUIRE(conv_dtype == DT_F32 || conv_dtype == DT_BF16, "delta_step: unknown weight dtype %d", conv_dtype);
+  IFX_REQUIRE(ldu >= 2 * G * d + H * dv && col_g >= 0 && col_b >= 0 && col_a >= 0 && col_g + H * dv <= ldr && col_b + H <= ldr && col_a + H <= ldr, "delta_step: rows too narrow");
+  IFX_REQUIRE(state_offset % 4 == 0 && state_stride % 4 == 0 && state_stride >= state_offset + (long long)H * dv * dpad, "delta_step: S must lie on 16 bytes within a row of %lld floats", state_stride);
+  IFX_REQUIRE(R <= 65535, "delta_step: too many requests for one launch");
+  if (R == 0 || T == 0) return 0;
+  DeltaArgs a{u, ldu, rows, ldr, col_g, col_b, col_a, A_log, dt_bias, norm_w, norm_dtype, eps, state, (size_t)state_stride,
+              (size_t)state_offset, q_start, q_len, slots, out, nullptr, T, H, G, d, dv, dpad / 4, 0};
+  const StepConv conv{conv_w, conv_dtype, state};
+  const int cols = step_threads(dpad, dv, 4) > 0 ? 4 : 8, threads = step_threads(dpad, dv, cols);
+  const size_t lds_bytes = (size_t)(2 * dpad + dv) * sizeof(float);
+  hipStream_t s = (hipStream_t)stream;
+#define STEP(TAPS, COLS) hipLaunchKernelGGL((delta_step_kernel<TAPS, COLS>), dim3(H, R), dim3(threads), lds_bytes, s, a, conv)
+  if (taps && cols == 4) STEP(4, 4);
+  else if (taps) STEP(4, 8);
+  else if (cols == 4) STEP(0, 4);
+  else STEP(0, 8);
+#undef STEP
+  IFX_LAUNCH_CHECK();
+}
+
 extern "C" int ifx_delta_rule(const void* u, int ldu, const void* rows, int ldr, int col_g, int col_b, int col_a, int dtype,
                               const float* A_log, const float* dt_bias, const void* norm_w, int norm_dtype, float eps, float* state,
                               long long state_stride, long long state_offset, const int* q_start, const int* q_len, const int* slots,

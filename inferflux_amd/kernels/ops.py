@@ -2157,6 +2157,46 @@ def delta_rule(u: torch.Tensor, rows: torch.Tensor, cols: Tuple[int, int, int], 
     return out
 
 
+DELTA_STEP_TAPS = 4         # ... of the convolution that ``delta_step`` takes along
+
+
+def delta_step_takes(dtype: torch.dtype, d: int, dv: int, state_offset: int, state: torch.Tensor) -> bool:
+    """Whether ``delta_step`` takes single tokens of these heads."""
+    return (dtype == torch.bfloat16 and state_offset % 4 == 0 and state.shape[1] % 4 == 0
+            and bool(load_module("delta").fn("ifx_delta_step_takes", (I, I))(delta_padded_dim(d), dv)))
+
+
+def delta_step(u: torch.Tensor, conv_w: Optional[torch.Tensor], rows: torch.Tensor, cols: Tuple[int, int, int], A_log: torch.Tensor,
+               dt_bias: torch.Tensor, norm_w: torch.Tensor, eps: float, n_heads: int, n_kv_heads: int, d: int, dv: int, state: torch.Tensor,
+               state_offset: int, q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:
+    """``delta_rule`` of a step of single tokens in bfloat16 as one launch (``delta_step_takes``), and with ``conv_w`` [2 G d + H dv,
+    DELTA_STEP_TAPS] (as many q and k heads as heads) ``causal_conv_silu`` of the first so many columns of ``u`` before it, whose state begins a
+    request's row.  What lies between the two, and between the walk and its norm, is not rounded."""
+    _check(u, "u", (None, None), torch.bfloat16)
+    T, ldu = u.shape
+    _check(rows, "rows", (T, None), torch.bfloat16)
+    H, G = n_heads, n_kv_heads
+    channels = 2 * G * d + H * dv
+    col_g, col_b, col_a = cols
+    if ldu < channels or col_g + H * dv > rows.shape[1] or max(col_b, col_a) + H > rows.shape[1]:
+        raise KernelError("delta_step: the rows are narrower than the columns named")
+    if conv_w is not None:
+        _check(conv_w, "conv_w", (channels, DELTA_STEP_TAPS))
+    _check(A_log, "A_log", (H,), torch.float32)
+    _check(dt_bias, "dt_bias", (H,), torch.float32)
+    _check(norm_w, "norm_w", (dv,))
+    _check(state, "state", (None, None), torch.float32)
+    R = q_start.shape[0]
+    for t, nm in ((q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
+        _check(t, nm, (R,), torch.int32)
+    out = empty((T, H * dv), u.dtype, u)
+    _call(load_module("delta"), "ifx_delta_step", (P, I, P, I, I, P, I, I, I, I, P, P, P, I, F, P, LL, LL, P, P, P, P, I, I, I, I, I, I, I, P),
+          u, ldu, conv_w, DT_F32 if conv_w is None else _dt(conv_w), 0 if conv_w is None else DELTA_STEP_TAPS, rows, rows.shape[1], col_g, col_b, col_a,
+          A_log, dt_bias, norm_w, _dt(norm_w), float(eps), state, state.shape[1], int(state_offset), q_start, q_len, slots, out, T, R, H, G, d, dv,
+          delta_padded_dim(d), _stream())
+    return out
+
+
 def diff_expand(q: torch.Tensor) -> torch.Tensor:
     """q [T, H, 2 d] -> [T, 2 H, 2 d]: head 2 h is [q1 | 0], head 2 h + 1 is [0 | q2] (the two maps of differential attention as
     heads of their own against keys whose rows hold both maps' vectors)."""

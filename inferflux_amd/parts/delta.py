@@ -95,12 +95,18 @@ class GatedDeltaRule(Mixer):
             raise ValueError(f"{self.name}: the mixer was given no per-request state")
         C, V, nh = self.channels, self.v_width, self.n_heads
         rows = ops.linear(h, self.w_in)                                 # [T, q | k | v | g | b | a]
-        u = ops.causal_conv_silu(rows, C, self.conv_w, None, state, ctx.row_req, ctx.q_start, ctx.q_len, ctx.state_slots)
+        single = 0 < ctx.n_tokens == ctx.n_requests
+        step = single and ops.delta_step_takes(rows.dtype, self.head_dim, self.v_head_dim, self.conv_floats, state)
+        conv = step and nh == self.n_kv_heads and self.taps == ops.DELTA_STEP_TAPS        # (the convolution goes with it)
+        u = rows if conv else ops.causal_conv_silu(rows, C, self.conv_w, None, state, ctx.row_req, ctx.q_start, ctx.q_len, ctx.state_slots)
         if t is not None:
             t.mark("mixer.conv")
-        y = ops.delta_rule(u, rows, (C, C + V, C + V + nh), self.A_log, self.dt_bias, self.norm_w, self.norm_eps, nh,
-                           self.n_kv_heads, self.head_dim, self.v_head_dim, state, self.conv_floats, ctx.q_start, ctx.q_len,
-                           ctx.state_slots, single_tokens=ctx.n_tokens == ctx.n_requests)
+        args = ((C, C + V, C + V + nh), self.A_log, self.dt_bias, self.norm_w, self.norm_eps, nh, self.n_kv_heads, self.head_dim, self.v_head_dim, state,
+                self.conv_floats, ctx.q_start, ctx.q_len, ctx.state_slots)
+        if step:
+            y = ops.delta_step(u, self.conv_w if conv else None, rows, *args)
+        else:
+            y = ops.delta_rule(u, rows, *args, single_tokens=ctx.n_tokens == ctx.n_requests)
         if t is not None:
             t.mark("mixer.scan")
         if sink is not None and ops.adds_into_stream(y.shape[0], self.w_o, sink.norm_weight):

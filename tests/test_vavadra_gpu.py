@@ -347,6 +347,41 @@ def test_two_maps_as_heads_of_their_own_and_joined_again(dtype):
     assert rel_err(got, T64(want.reshape(T, H * dv))) < (1e-6 if dtype == "float32" else 1e-2)
 
 
+@pytest.mark.parametrize("R,H,G,d,dv,conv", [(1, 16, 16, 64, 128, True), (5, 3, 3, 10, 14, True), (3, 2, 2, 128, 128, True), (70, 4, 4, 64, 64, True), (2, 1, 1, 256, 64, True),
+                                             (2, 1, 1, 8, 600, True), (2, 1, 1, 64, 256, True), (4, 4, 2, 16, 24, False), (3, 3, 1, 10, 14, False), (6, 2, 1, 128, 128, False),
+                                             (2, 2, 2, 64, 300, False)])
+def test_single_tokens_of_the_delta_rule_in_one_launch(R, H, G, d, dv, conv):
+    """Against the launches for the convolution, the walk and the norm, in 32 bits from the same bfloat16 rows and the same states, three times: one rounding to
+    bfloat16, and sums of at most 256 products in another order."""
+    eps, channels = 1e-5, 2 * G * d + H * dv
+    A_log, dt_bias = (-3.0 + 3.5 * torch.rand(H, generator=torch.Generator().manual_seed(8))).float().to(DEV), rnd(9, H).float().to(DEV)
+    norm_w, conv_w = (1.0 + 0.3 * rnd(10, dv)).bfloat16().to(DEV), rnd(11, channels, 4, scale=0.5).bfloat16().to(DEV)
+    offset = -(-3 * channels // 4) * 4
+    dpad = ops.delta_padded_dim(d)
+    state = rnd(12, R + 1, -(-(offset + ops.delta_state_floats(H, d, dv)) // 4) * 4, scale=0.5).float().to(DEV)
+    state[:, offset:offset + H * dv * dpad].view(R + 1, -1, dpad)[:, :, d:] = 0          # (the padded channels hold zeros)
+    if not ops.delta_step_takes(torch.bfloat16, d, dv, offset, state):
+        assert -(-dv // 8) * (dpad // 4) > 512
+        return
+    states = [state.clone(), state.clone()]
+    q_start, q_len = (x.to(DEV) for x in _step_arrays([1] * R))
+    slots = torch.randperm(R + 1, generator=torch.Generator().manual_seed(2))[:R].to(torch.int32).to(DEV)
+    row_req = torch.arange(R, dtype=torch.int32, device=DEV)
+    for turn in range(3):
+        u, rows, cols = _delta_inputs(20 + 10 * turn, R, H, G, d, dv, torch.bfloat16)
+        u, rows = u.to(DEV), rows.to(DEV)
+        args = (cols, A_log, dt_bias, norm_w, eps, H, G, d, dv)
+        got = ops.delta_step(u, conv_w if conv else None, rows, *args, states[0], offset, q_start, q_len, slots)
+        uf = ops.causal_conv_silu(u.float(), channels, conv_w.float(), None, states[1], row_req, q_start, q_len, slots) if conv else u.float()
+        want = ops.delta_rule(uf, rows.float(), *args, states[1], offset, q_start, q_len, slots)
+        assert rel_err(got.cpu(), want.cpu()) < 2.0 ** -8
+    a, b = states[0].cpu(), states[1].cpu()
+    assert torch.equal(a[:, :offset], b[:, :offset]) and rel_err(a[:, offset:], b[:, offset:]) < 2e-5 and not torch.equal(a, state.cpu())
+    for wrong in (dict(offset=offset + 1), dict(w=conv_w[:, :3].contiguous())):
+        with pytest.raises(ops.KernelError):
+            ops.delta_step(u, wrong.get("w"), rows, *args, states[0], wrong.get("offset", offset), q_start, q_len, slots)
+
+
 @pytest.mark.parametrize("T,H,dv,splits", [(1, 3, 16, 1), (37, 2, 128, 32), (8, 16, 112, 16), (64, 1, 48, 3)])
 def test_two_maps_joined_from_the_splits_of_attention(T, H, dv, splits):
     from test_mumusun_gpu import split_rows
