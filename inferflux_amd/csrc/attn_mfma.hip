@@ -230,9 +230,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
 constexpr int OPAD = D + 4;       // floats per output row in LDS (the padding spreads the 16 columns over the banks)
 
 template <bool STREAM, bool KEEP>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rows_whole_kernel(RowArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int kvh = blockIdx.x, ri = blockIdx.y;
+__device__ __forceinline__ void row_whole(const RowArgs& a, int kvh, int ri, float* lds) {
   const int tid = threadIdx.x, wid = tid / WAVE, lane = tid % WAVE, col = lane & 15, g4 = lane >> 4;
   const int W = a.waves, n_threads = W * WAVE;
   const int row = a.rows ? a.rows[ri] : ri;
@@ -333,6 +331,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       *(bf16x4*)(a.out + ((size_t)row * a.nH + kvh * ratio + qt + c) * D + e) = w4;
     }
   }
+}
+
+template <bool STREAM, bool KEEP>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rows_whole_kernel(RowArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  row_whole<STREAM, KEEP>(a, blockIdx.x, blockIdx.y, lds);
 }
 
 // ``waves`` 0: one wave per (row, kv head, split of ``chunk`` keys) and a second launch that merges the splits
@@ -449,16 +453,20 @@ struct TileRegs {
 
 // The pages of a tile's four runs of 16 keys (-1: none), the same for every thread and held in scalar
 // registers.  They are looked up one tile before the data is fetched, so that fetching costs one trip
-// to memory, not two.
+// to memory, not two.  The table is read through the constant address space and without branches: four
+// scalar loads on their way together.  As vector loads each waited for itself and for the tile's data that had been
+// asked for before it (1,024 rows of 16 heads of 128 36.6 us then and 32.2 now, 512 rows after 1,500 keys
+// 67.1 and 57.8, 14 heads of 64 52.0 and 44.0).
+typedef const __attribute__((address_space(4))) int* table_ptr;
 static_assert(TK == 64, "a tile is four runs of 16 keys");
 struct TilePages { int p0, p1, p2, p3; };
 
-__device__ __forceinline__ TilePages tile_pages(const TileArgs& a, const int* table, int j0, int pos_last) {
-  auto look = [&](int i) {
-    const int j = j0 + 16 * i, blk = j >> a.page_shift;
-    return __builtin_amdgcn_readfirstlane((j <= pos_last && blk < a.max_blocks) ? table[blk] : -1);
-  };
-  return TilePages{look(0), look(1), look(2), look(3)};
+__device__ __forceinline__ TilePages tile_pages(const TileArgs& a, table_ptr table, int j0, int pos_last) {
+  const int last = a.max_blocks - 1;
+  auto look = [&](int i) { return table[max(0, min((j0 + 16 * i) >> a.page_shift, last))]; };
+  auto held = [&](int i, int page) { return j0 + 16 * i <= pos_last && (j0 + 16 * i) >> a.page_shift <= last ? page : -1; };
+  const int p0 = look(0), p1 = look(1), p2 = look(2), p3 = look(3);
+  return TilePages{held(0, p0), held(1, p1), held(2, p2), held(3, p3)};
 }
 
 __device__ __forceinline__ int pick_page(const TilePages& pg, int sub) {
@@ -653,11 +661,27 @@ __device__ __forceinline__ void tile_math(const bf16_t* k_s, const bf16_t* v_s, 
 #define TILE_WAVES_PER_SIMD 2
 #endif
 #endif
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILE_WAVES_PER_SIMD, TILE_WAVES_PER_SIMD)))
-void attn_tiles_kernel(TileArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16_t k_s[TK * KPAD];
-  __shared__ __attribute__((aligned(16))) bf16_t v_s[D * VPAD];
-  const int tid = threadIdx.x, wid = tid / WAVE, lane = tid % WAVE, col = lane & 15, g4 = lane >> 4;
+// GROUPS 2: two groups of four waves walk every other key tile of the workgroup's each, with LDS of their own, and meet in LDS at the end: for launches
+// of fewer workgroups than compute units, where a workgroup has its unit to itself.  A tile is a serial chain (LDS, scores, maximum, exponentials, output)
+// that four waves, one to a SIMD, wait through: 1.65 us a tile of 128 elements alone, 1.25 in two groups (500 rows of 16 heads 17.9 us and 15.0).
+// ROWS (1, with streaming loads 2): the workgroups behind the first ``tile_blocks`` take a (row, kv head) each as attn_rows_whole_kernel does: the rows of
+// a step's other requests, which do not need the tiles, beside them on units that the tiles leave idle, instead of two launches behind them (500 rows and
+// 23 single ones of up to 299 keys, 16 heads on 2: 28.7 us and 15.6).
+template <int GROUPS, int ROWS>
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(GROUPS == 1 ? TILE_WAVES_PER_SIMD : 2, GROUPS == 1 ? TILE_WAVES_PER_SIMD : 2)))
+void attn_tiles_kernel(TileArgs a, RowArgs rows, int tile_blocks) {
+  constexpr int GROUP_LDS = TK * KPAD + D * VPAD;      // bf16 elements of a group's K and V^T tiles
+  __shared__ __attribute__((aligned(16))) bf16_t lds[GROUPS * GROUP_LDS];
+  if constexpr (ROWS > 0) {
+    if ((int)blockIdx.x >= tile_blocks) {
+      const int i = blockIdx.x - tile_blocks;
+      row_whole<ROWS == 2, false>(rows, i % rows.nKV, i / rows.nKV, (float*)lds);
+      return;
+    }
+  }
+  // (the same for a whole wave, which the compiler has to be told: otherwise each load of a tile becomes a loop over the lanes' descriptors)
+  const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / 256), tid = threadIdx.x % 256, wid = tid / WAVE, lane = tid % WAVE, col = lane & 15, g4 = lane >> 4;
+  bf16_t *k_s = lds + group * GROUP_LDS, *v_s = k_s + TK * KPAD;
   // Workgroups go to the 8 XCDs round-robin by their number, and every XCD has an L2 of its own.
   // Work items are ordered kv head first and dealt to the XCDs in contiguous runs, so that the
   // workgroups that read one kv head's keys and values share an L2 instead of filling all eight with
@@ -674,7 +698,7 @@ void attn_tiles_kernel(TileArgs a) {
   const int req = a.tile_req[ti], q0 = a.tile_q0[ti];
   const int qlen = a.q_len[req], kvlen = a.kv_len[req];
   const int start = kvlen - qlen;                       // position of the request's first row in this step
-  const int* table = a.block_table + (size_t)req * a.max_blocks;
+  const table_ptr table = (table_ptr)(a.block_table + (size_t)req * a.max_blocks);
   const int rows_here = min(TQ, qlen - q0);
   const int pos_first = start + q0, row_last = pos_first + rows_here - 1;
   // the keys of this workgroup: what its rows can see, cut to its split
@@ -720,24 +744,55 @@ void attn_tiles_kernel(TileArgs a) {
   auto tile_at = [&](int n) { return n < n_kept ? k0 + n * TK : w_from + (n - n_kept) * TK; };
 
   TileRegs regs;
-  TilePages pg = tile_pages(a, table, tile_at(0), pos_last);
-  if (n_walk > 0) fetch_tile(regs, a, pg, kvh, tile_at(0), tid);
-  pg = tile_pages(a, table, tile_at(1), pos_last);
-  for (int n = 0; n < n_walk; ++n) {
-    const int j0 = tile_at(n);
+  TilePages pg = tile_pages(a, table, tile_at(group), pos_last);
+  if (group < n_walk) fetch_tile(regs, a, pg, kvh, tile_at(group), tid);
+  pg = tile_pages(a, table, tile_at(group + GROUPS), pos_last);
+  for (int n0 = 0; n0 < n_walk; n0 += GROUPS) {
+    const int n = n0 + group, j0 = tile_at(n);
     __syncthreads();  // everyone is done with the previous tile
-    stage_tile(regs, k_s, v_s, tid);
+    if (GROUPS == 1 || n < n_walk) stage_tile(regs, k_s, v_s, tid);
     __syncthreads();
-    if (n + 1 < n_walk) {  // the next tile's data and the one after's pages: in flight during the arithmetic
-      fetch_tile(regs, a, pg, kvh, tile_at(n + 1), tid);
-      pg = tile_pages(a, table, tile_at(n + 2), pos_last);
+    if (n + GROUPS < n_walk) {  // the next tile's data and the one after's pages: in flight during the arithmetic
+      fetch_tile(regs, a, pg, kvh, tile_at(n + GROUPS), tid);
+      pg = tile_pages(a, table, tile_at(n + 2 * GROUPS), pos_last);
     }
+    if (GROUPS > 1 && n >= n_walk) continue;
     if (j0 > wave_hi || (j0 + TK <= wave_lo && j0 >= keep)) continue;   // uniform over the wave; barriers are at the loop's top
 
     // A tile every key of which every row of this wave sees needs no mask: the common case.
     const bool full = j0 + TK - 1 <= wave_first && j0 >= first_seen(wave_hi, a.window, a.block);
     if (full) tile_math<false>(k_s, v_s, q, a.scale_log2e, j0, col, g4);
     else tile_math<true>(k_s, v_s, q, a.scale_log2e, j0, col, g4, keep);
+  }
+  if constexpr (GROUPS > 1) {      // the second group's lanes leave what they have to the same lanes of the first
+    static_assert(GROUPS == 2 && 256 * QT * (4 * DT + 2) * 2 <= GROUPS * GROUP_LDS, "the meeting fits the tiles' place");
+    floatx4* o_w = (floatx4*)lds;                               // [QT][DT][256]
+    float* ml_w = (float*)(o_w + QT * DT * 256);                // [QT][2][256]
+    __syncthreads();
+    if (group == 1) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o_w[(qt * DT + dt) * 256 + tid] = q[qt].o[dt];
+        ml_w[(2 * qt) * 256 + tid] = q[qt].m;
+        ml_w[(2 * qt + 1) * 256 + tid] = q[qt].l;
+      }
+    }
+    __syncthreads();
+    if (group == 1) return;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const float m1 = ml_w[(2 * qt) * 256 + tid], l1 = ml_w[(2 * qt + 1) * 256 + tid], M = fmaxf(q[qt].m, m1), Ms = M == -INFINITY ? 0.f : M;
+      const float f0 = fast_exp2((q[qt].m - Ms) * a.scale_log2e), f1 = fast_exp2((m1 - Ms) * a.scale_log2e);
+      q[qt].m = M;
+      q[qt].l = q[qt].l * f0 + l1 * f1;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const floatx4 o1 = o_w[(qt * DT + dt) * 256 + tid];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) q[qt].o[dt][r] = q[qt].o[dt][r] * f0 + o1[r] * f1;
+      }
+    }
   }
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -768,13 +823,17 @@ void attn_tiles_kernel(TileArgs a) {
 // splits of ``chunk`` (a multiple of 64; max_splits * chunk reaches past the largest position), the partial
 // results go to part_o [T, nH, max_splits, D] and part_ml [T, nH, max_splits, 2], and the rows named by ``rows``
 // (every row of every tiled request, n_rows of them) are merged into ``out`` at the end.
+// groups 2: eight waves to a workgroup, which share its keys (see attn_tiles_kernel).  beside (groups 2, one split) [n_beside]: rows that are taken whole by
+// workgroups of their own in the same launch.
 extern "C" int ifx_attn_tiles(const void* q, const void* k_cache, const void* v_cache, void* out,
                               const int* tile_req, const int* tile_q0, int n_tiles, const int* q_start,
                               const int* q_len, const int* kv_len, const int* block_table, int max_blocks,
                               int nH, int nKV, int d, int page_size, int window, float scale, int chunk, int max_splits,
                               float* part_o, float* part_ml, const int* rows, int n_rows, const int* row_req,
                               const int* positions, const int* order, int order_per_xcd, int n_xcd, int keep_first,
-                              int has_sink, float sink_score, const float* gate, const float* sinks, int block, void* stream) {
+                              int has_sink, float sink_score, const float* gate, const float* sinks, int block, int groups, const int* beside, int n_beside, void* stream) {
+  IFX_REQUIRE(groups == 1 || (groups == 2 && QT == 1 && max_splits == 1), "attn_tiles: %d groups of waves (2: tiles of 64 rows whose keys are not cut)", groups);
+  IFX_REQUIRE(n_beside == 0 || (n_beside > 0 && n_beside <= 65535 && groups == 2 && beside && row_req && positions && !keep_first), "attn_tiles: %d rows beside the tiles", n_beside);
   IFX_REQUIRE(d == D, "attn_tiles: built for head_dim %d, called with %d", D, d);
   IFX_REQUIRE(keep_first >= 0, "attn_tiles: keep_first %d", keep_first);
   IFX_REQUIRE(n_tiles >= 0 && nH > 0 && nKV > 0 && nH % nKV == 0, "attn_tiles: bad head counts nH=%d nKV=%d", nH, nKV);
@@ -800,7 +859,19 @@ extern "C" int ifx_attn_tiles(const void* q, const void* k_cache, const void* v_
   a.n_xcd = n_xcd;
   a.per_xcd = order ? order_per_xcd : (int)((items + n_xcd - 1) / n_xcd);
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(attn_tiles_kernel, dim3(n_xcd * a.per_xcd), dim3(256), 0, s, a);
+  const int blocks = n_xcd * a.per_xcd;
+  if (groups == 1) {
+    hipLaunchKernelGGL((attn_tiles_kernel<1, 0>), dim3(blocks), dim3(256), 0, s, a, RowArgs{}, blocks);
+  } else if constexpr (QT == 1) {
+    const RowArgs rr{(const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, beside, row_req, positions, block_table, nullptr, nullptr, (bf16_t*)out,
+                     max_blocks, n_beside, nH, nKV, page_size, window, 0, 1, scale * 1.4426950408889634f, 0, 8, 0, 0, has_sink, sink_score * 1.4426950408889634f,
+                     gate, sinks, block};
+    const dim3 grid(blocks + n_beside * nKV);
+    IFX_REQUIRE(n_beside == 0 || 8 * (nH / nKV < 16 ? nH / nKV : 16) * (OPAD + 2) * 4 <= 2 * (TK * KPAD + D * VPAD) * 2, "attn_tiles: rows of %d heads do not fit beside the tiles", nH / nKV);
+    if (n_beside == 0) hipLaunchKernelGGL((attn_tiles_kernel<2, 0>), grid, dim3(512), 0, s, a, rr, blocks);
+    else if (n_beside >= ROW_STREAM_MIN_ROWS && page_size == 16) hipLaunchKernelGGL((attn_tiles_kernel<2, 2>), grid, dim3(512), 0, s, a, rr, blocks);
+    else hipLaunchKernelGGL((attn_tiles_kernel<2, 1>), grid, dim3(512), 0, s, a, rr, blocks);
+  }
   if (max_splits > 1) {
     RowArgs m{(const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, rows, row_req, positions, block_table,
               part_o, part_ml, (bf16_t*)out, max_blocks, n_rows, nH, nKV, page_size, window, chunk, max_splits,

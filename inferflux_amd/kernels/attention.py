@@ -4,7 +4,8 @@ Every choice computes the same function (causal, optionally windowed, grouped-qu
 over the paged cache); they differ in speed and in which sizes they accept.  In bfloat16 with a
 head size the matrix-core module takes (up to 128, values as wide as keys), requests that bring at least TILE_MIN rows go to the
 tile kernel (tiles of as many rows as the compiled module says; keys in splits when the tiles are
-few and their pasts long) and all other rows (decode tokens, short portions) to the row kernel;
+few and their pasts long) and all other rows (decode tokens, short portions) to the row kernel, or into
+the tiles' own launch where those leave compute units idle;
 everything else (float32, other head sizes) goes to the plain kernel, whose bits the 32-bit
 tile kernel repeats for whole tiles of rows.
 """
@@ -42,6 +43,9 @@ TILE_SPLIT_FEW_MIN_LONGEST = 1024   # this many keys on, and may be as short as
 TILE_SPLIT_FEW_MIN_KEYS = 256       # this while the walk is short
 TILE_MAX_SPLITS = 16
 TILE_ORDER_MIN_ITEMS = 64       # launches of more workgroups than this get them in tile_order
+TILE_GROUPS_MAX = 256       # at most this many workgroups of 64-row tiles, one for each compute unit: two groups of waves to a workgroup,
+TILE_GROUPS_KEYS = 1024     # while no workgroup walks more keys than this
+TILE_GROUPS_KEYS_BESIDE = 1536      # ... or than this with the step's other rows in the same launch (see choose_groups)
 ROW_CHUNK = 64      # keys per split of the row kernel: doubled while the launch keeps ROW_MIN_WAVES (ROW_MIN_WAVES_128
 ROW_MIN_WAVES_128 = 1000   # for the step from 64 to 128) waves or more: a split costs a fixed start-up, so longer splits
 ROW_MIN_WAVES = 1536       # pay when there are waves enough; and until a row has at most ROW_MAX_SPLITS splits.  The merge
@@ -122,6 +126,31 @@ def choose_tiling(tiled_rows, tiled_keys, n_heads: int, rows_of, tall_direct: bo
             if splits <= 1:
                 splits, chunk = 1, 0
     return qt, splits, chunk
+
+
+def choose_groups(tiled_rows, tiled_keys, n_heads: int, row_keys, pairs: int, window: Optional[int], splits: int = 1, beside_fits: bool = True):
+    """(two groups of waves to a workgroup of 64-row tiles, and the step's other rows beside them in the same launch) for a step whose requests bring
+    ``tiled_rows`` rows and hold ``tiled_keys`` keys, beside single rows of ``row_keys`` keys in ``pairs`` (row, kv head) pairs; by itself
+    ``choose_tiling`` would cut the tiles' keys into ``splits``.
+
+    A launch of at most a workgroup for each compute unit leaves a workgroup of four waves waiting for itself; with eight, of which each four
+    take every other key tile, a tile of 128 elements costs 1.25 us instead of 1.65.  us as it
+    was / in two groups: 16 heads of 128 on 2, 500 rows 17.9 / 15.0, 300 after 512 keys 26.2 / 21.1, 64 after 700 24.9 / 19.9, 2 prompts of 512 15.5 / 15.5,
+    512 after 512 24.7 / 24.8, 512 after 1,500 43.6 / 43.6, 256 after 3,000 32 / 66; 14 heads of 64 on 2, 500 rows 14.0 / 11.4, 512 after 512 20.6 / 18.4,
+    1,024 24.4 / 18.6, 512 after 1,500 29.7 / 32.1; 336 workgroups of 128 20.5 / 21.5.
+    The other rows beside them cost little while they end no later than the tiles, against 10 to 13 us of their own launches: a row's walk takes some
+    4.5 us and 11 for 1,000 keys, a tile's 5 and 19.5.  us with launches of their own / beside, 16 heads of 128 on 2: 500 rows and 23 rows of up to 299 keys
+    28.7 / 15.6, 20 of up to 992 30.5 / 18.6, 512 after 1,500 and 20 of 981 58 / 44, 128 rows and 6 of 369 17.5 / 9.7, but 4 of 1,900 18.0 / 25.6; more
+    workgroups than compute units, 28 heads on 4, 500 rows and 23 of 283 31.9 / 17.6; 2 prompts of 512, 16 heads, and 4 rows of 1,933 25.6 / 31.6."""
+    blocks = sum(-(-int(n) // 64) for n in tiled_rows) * n_heads
+    walk = int(max(tiled_keys)) if window is None else min(int(max(tiled_keys)), window + 64)
+    if blocks > TILE_GROUPS_MAX or walk > TILE_GROUPS_KEYS_BESIDE:
+        return False, False
+    if pairs and beside_fits and pairs <= TILE_GROUPS_MAX:
+        row_walk = int(max(row_keys)) if window is None else min(int(max(row_keys)), window)
+        if row_walk * 4 <= walk * 7 + (2800 if blocks + pairs <= TILE_GROUPS_MAX else 0):
+            return True, True
+    return splits == 1 and walk <= TILE_GROUPS_KEYS, False
 
 
 from .device import CUS_PER_XCD, N_XCD      # the launch deals workgroups to the XCDs in turn, and an XCD its share to its compute units in turn
@@ -360,20 +389,27 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
         if tiled.any():
             qt, splits, chunk = choose_tiling(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, lambda t: ops.attention_tile_rows(d, t),
                                               tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not keep_first and not block)
+        two = beside = False
+        if tiled.any():
+            row_req = np.nonzero(~tiled & (ctx.h_q_len > 0))[0]
+            two, beside = choose_groups(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, ctx.h_kv_len[row_req], int(ctx.h_q_len[row_req].sum()) * n_kv,
+                                        window, splits, not keep_first)
+            if two:
+                qt, splits, chunk = 1, 1, 0
         tile_rows = ops.attention_tile_rows(d, qt)
-        return qt, ctx.derived(("attention_work_lists", n_kv, tile_rows, nH, splits, chunk, window, d),
+        return qt, 2 if two else 1, beside, ctx.derived(("attention_work_lists", n_kv, tile_rows, nH, splits, chunk, window, d),
                                lambda: _work_lists(ctx, n_kv, tile_rows, nH, splits, chunk, window, ops.row_waves_fit(nH, n_kv, d, ops.ROW_MAX_WAVES), d))
 
     # (once a step for all layers of a kind)
-    qt, w = ctx.derived(("attention_plan", n_kv, nH, d, window, keep_first, block), plan)
+    qt, groups, beside, w = ctx.derived(("attention_plan", n_kv, nH, d, window, keep_first, block), plan)
     left = keep_splits and w["waves"] == 0 and w["n_rows"] == T > 0 and w["max_splits"] <= ops.SPLITS_READ_MAX and sink is None and gate is None
     out = None if left else ops.empty((T, nH * d), q.dtype, q)
     more = dict(keep_first=keep_first, sink=sink, gate=gate, sinks=sinks, block=block) if extras else {}
     if w["n_tiles"]:
         ops.attention_tiles(q, cache.k, cache.v, out, w["tile_req"], w["tile_q0"], ctx.q_start, ctx.q_len, ctx.kv_len,
                             table, window, scale, qt, w["tile_chunk"], w["tile_splits"], w["tile_row_list"], ctx.row_req,
-                            ctx.positions, w["tile_order"], **more)
-    if w["n_rows"]:
+                            ctx.positions, w["tile_order"], groups=groups, beside=w["rows"] if beside else None, **more)
+    if w["n_rows"] and not beside:
         splits = ops.attention_rows(q, cache.k, cache.v, out, w["rows"], w["n_rows"], ctx.row_req, ctx.positions, table,
                                     window, scale, w["chunk"], w["max_splits"], w["waves"], ctx.n_tokens == ctx.n_requests, **more)
     return splits if left else out

@@ -3013,7 +3013,8 @@ def attention_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                     qt: int = 1, chunk: int = 0, max_splits: int = 1, rows: Optional[torch.Tensor] = None,
                     row_req: Optional[torch.Tensor] = None, positions: Optional[torch.Tensor] = None,
                     order: Optional[torch.Tensor] = None, keep_first: int = 0, sink: Optional[float] = None,
-                    gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, block: Optional[int] = None) -> None:
+                    gate: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, block: Optional[int] = None, groups: int = 1,
+                    beside: Optional[torch.Tensor] = None) -> None:
     """Attention of tiles of ``attention_tile_rows(d, qt)`` consecutive rows of one request each (tile t:
     request tile_req[t], rows from tile_q0[t] of that request's rows in this step) into ``out`` [T, nH*d].
 
@@ -3023,8 +3024,14 @@ def attention_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     needs the step's ``row_req`` and ``positions`` [T].
 
     ``order`` (int32 [8 * n], from ``attention.tile_order``) says which work item each workgroup of the launch
-    takes; every item must appear exactly once (-1: a workgroup without work).  The result does not depend on it."""
-    extras = bool(keep_first) or bool(block)      # (the kernel that loads straight into LDS has neither)
+    takes; every item must appear exactly once (-1: a workgroup without work).  The result does not depend on it.
+
+    ``groups`` 2 (``qt`` 1, one split): eight waves to a workgroup, two groups of which share its keys, for launches of fewer workgroups than
+    compute units.  ``beside`` (int32, with ``groups`` 2 and the step's ``row_req`` and ``positions``, not with ``keep_first``): further rows, taken whole
+    by a workgroup for each kv head in the same launch."""
+    extras = bool(keep_first) or bool(block) or groups > 1      # (the kernel that loads straight into LDS has none of them)
+    if groups not in (1, 2) or (groups == 2 and (qt != 1 or max_splits > 1)):
+        raise KernelError(f"attention_tiles: {groups} groups of waves with tiling {qt} and {max_splits} splits (2: tiles of 64 rows, one split)")
     T, nH, d, nKV, page_size, mod = _attn_common(q, k_cache, v_cache, qt, not extras)
     _, _, entry, rows_fn = _tile_module(d, qt, not extras)
     if mod.fn(rows_fn, ())() != attention_tile_rows(d, qt):
@@ -3038,7 +3045,14 @@ def attention_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         _check(t, nm, (R,), torch.int32)
     _check(block_table, "block_table", (R, None), torch.int32)
     part_o = part_ml = None
-    n_rows = 0
+    n_rows = n_beside = 0
+    if beside is not None:
+        n_beside = beside.shape[0]
+        if groups != 2 or keep_first or row_req is None or positions is None or n_beside == 0:
+            raise KernelError("attention_tiles: rows beside the tiles go with two groups of waves, row_req and positions, and without kept first keys")
+        _check(beside, "beside", (n_beside,), torch.int32)
+        _check(row_req, "row_req", (T,), torch.int32)
+        _check(positions, "positions", (T,), torch.int32)
     if max_splits > 1:
         if chunk <= 0 or chunk % 64:
             raise KernelError(f"attention_tiles: splits need a chunk that is a multiple of 64, got {chunk}")
@@ -3061,7 +3075,8 @@ def attention_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             part_o, part_ml, rows, n_rows, row_req, positions, order, per_xcd, N_XCD)
     types = (P, P, P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, F, I, I, P, P, P, I, P, P, P, I, I)
     if entry == "ifx_attn_tiles":
-        _call(mod, entry, types + (I, I, F, P, P, I, P), *args, *_attn_extras(T, nH, keep_first, sink, gate, sinks, block), _stream())
+        _call(mod, entry, types + (I, I, F, P, P, I, I, P, I, P), *args, *_attn_extras(T, nH, keep_first, sink, gate, sinks, block), groups, beside, n_beside,
+              _stream())
     else:
         _call(mod, entry, types + (I, F, P, P, P), *args, *_attn_extras(T, nH, 0, sink, gate, sinks)[1:5], _stream())
 

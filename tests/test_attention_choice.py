@@ -6,7 +6,7 @@ import types
 import numpy as np
 import torch
 
-from inferflux_amd.kernels.attention import F32_TILE_MIN, TILE_MAX_SPLITS, _f32_tiles, choose_tiling, tile_order
+from inferflux_amd.kernels.attention import F32_TILE_MIN, TILE_MAX_SPLITS, _f32_tiles, choose_groups, choose_tiling, tile_order
 
 ROWS_OF = lambda qt: 64 * qt          # head size 128
 
@@ -261,3 +261,28 @@ def test_steps_beyond_a_launch_of_32_bit_tiles_stay_with_the_plain_kernel():
         tiles = _f32_tiles(step, n_heads, n_kv, 1, cols)[0]
         assert (tiles is not None) == takes, (rows, n_heads, n_kv)
         assert tiles is None or len(tiles) * n_kv * cols // 4 < 1 << 24
+
+
+def test_two_groups_of_waves_and_rows_beside_the_tiles_where_both_were_measured():
+    cases = [  # rows of the prompts' portions, their keys, query heads, keys of the other rows, their pairs, window, splits -> (two groups, beside)
+        ([500], [500], 16, [], 0, None, 1, (True, False)),
+        ([500], [500], 16, [299] * 23, 46, None, 1, (True, True)),          # 28.7 us in three launches, 15.6 in one
+        ([500], [500], 16, [1575] + [50] * 3, 8, None, 1, (True, True)),    # 4 x 1,575 = 7 x 500 + 2,800
+        ([500], [500], 16, [1576] + [50] * 3, 8, None, 1, (True, False)),
+        ([512], [2012], 16, [981] * 20, 40, None, 4, (False, False)),       # 2,012 keys: beyond the longest walk
+        ([300], [1500], 16, [981] * 20, 40, None, 4, (True, True)),
+        ([300], [1500], 16, [], 0, None, 4, (False, False)),                # in splits
+        ([128], [128], 16, [1900] * 4, 8, None, 1, (True, False)),          # a row longer than the tiles: 18 us after them, 25.6 beside
+        ([128], [128], 16, [924] * 4, 8, None, 1, (True, True)),
+        ([128], [128], 16, [925] * 4, 8, None, 1, (True, False)),
+        ([128], [128], 16, [1900] * 4, 8, 200, 1, (True, True)),            # ... of which a window leaves 200 keys
+        ([64], [3000], 16, [150] * 4, 8, 512, 1, (True, True)),
+        ([512, 512], [512, 512], 16, [896] * 4, 8, None, 1, (True, True)),  # more workgroups than compute units
+        ([512, 512], [512, 512], 16, [897] * 4, 8, None, 1, (True, False)),
+        ([512, 512, 1], [512, 512, 1], 16, [276] * 23, 46, None, 1, (False, False)),    # more tiles than compute units
+        ([500], [500], 16, [299] * 40, 320, None, 1, (True, False)),
+        ([500], [500], 16, [299] * 20, 40, None, 1, (True, True)),
+    ]
+    for rows, keys, heads, row_keys, pairs, window, splits, want in cases:
+        assert choose_groups(rows, keys, heads, row_keys, pairs, window, splits) == want, (rows, keys, heads, row_keys, pairs, window)
+        assert not choose_groups(rows, keys, heads, row_keys, pairs, window, splits, beside_fits=False)[1]
