@@ -164,6 +164,117 @@ __global__ __launch_bounds__(64 * N_SLICES / SP) void gemm_f32_narrow_kernel(con
   }
 }
 
+// ---- the same of q, k and v -------------------------------------------------------------------------------------------------
+// A workgroup takes both halves of B / 2 rotation pairs, and bias, rotation (split-half pairs over the whole head) and the write into the paged cache
+// are its end, bit for bit those of rope_append, whose launch it saves.  us with the norm's launch before it, two launches / this: 4 rows of 896 in 14 heads of 64
+// on 2 8.3 / 6.2, 1 row 7.8 / 5.7, 8 rows 8.7 / 6.5, 4 rows of 1,536 in 12 heads of 128 on 2 10.9 / 8.5, of 2,048 in 6 on 2 10.7 / 8.5.  (That norm, formed by every
+// workgroup for itself from the stream, gives 0.1 to 0.3 more here, and costs gate/up with its many workgroups 3; a product that adds to the stream itself instead
+// of leaving it to the norm gives nothing.)
+struct QkvArgs {
+  const float *A, *W, *bias;
+  float* q;                 // [M][nH][d]
+  int M, N, K;
+  const int* slots;         // [M] or null: W holds q alone
+  const float *cs, *sn;     // [M][d / 2]
+  int nH, nKV, d, page_size;
+  float *k_cache, *v_cache;
+};
+
+template <int SP>
+__global__ __launch_bounds__(64 * N_SLICES / SP) void narrow_qkv_kernel(QkvArgs a) {
+  constexpr int B = 16 / SP, STEPS = 4;
+  __shared__ float part[N_SLICES][B * B];
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int i = lane % 16, q = lane / 16, r = i % B, slice = SP * wave + i / B;
+  const int M = a.M, K = a.K, half = a.d / 2;
+  // the weight row of column c of this workgroup, its head and where it stands in it (pairs beyond the last are computed and dropped)
+  auto row_at = [&](int c, int& head, int& at) {
+    const int p = min((int)blockIdx.x * (B / 2) + c % (B / 2), a.N / 2 - 1);
+    head = p / half;
+    at = p % half + (c >= B / 2 ? half : 0);
+    return head * a.d + at;
+  };
+  int its_head, its_place;
+  const int len = slice_len(K), k_lo = slice * len, k_hi = min(K, k_lo + len), a_hi = r < M ? k_hi : 0;
+  const float* wrow = a.W + (size_t)row_at(r, its_head, its_place) * K;
+  const float* arow = a.A + (size_t)min(r, M - 1) * K;
+  f32x4 w[STEPS], x[STEPS];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      w[s] = load4<true>(wrow, k_lo + k0 + 16 * s + 4 * q, k_hi);
+      x[s] = load4<true>(arow, k_lo + k0 + 16 * s + 4 * q, a_hi);
+    }
+  };
+  fetch(0);
+  // what the end needs, for the threads that write
+  const int e = threadIdx.x, m = e / B, c = e % B;
+  int head, at;
+  const int n = row_at(c, head, at);
+  const bool in = e < B * B && m < M && (int)blockIdx.x * (B / 2) + c % (B / 2) < a.N / 2;
+  float bias = 0.f, cs = 0.f, sn = 0.f;
+  int slot = -1;
+  if (in) {
+    if (a.bias) bias = a.bias[n];
+    cs = a.cs[(size_t)m * half + at % half], sn = a.sn[(size_t)m * half + at % half];
+    if (a.slots) slot = a.slots[m];
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < len; k0 += 16 * STEPS) {
+    if (k0 > 0) fetch(k0);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s][j], w[s][j], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if ((4 * q + j) / B == i / B) part[slice][(4 * q + j) % B * B + r] = acc[j];
+  __syncthreads();
+  if (e >= B * B) return;
+  float v = part[0][e];
+#pragma unroll
+  for (int s = 1; s < N_SLICES; ++s) v += part[s][e];
+  if (a.bias) v += bias;
+  const float other = __shfl_xor(v, B / 2);
+  if (!in) return;
+  const float turned = other * sn;
+  const float y = __builtin_fmaf(v, cs, c < B / 2 ? -turned : turned);
+  if (head < a.nH) {
+    a.q[(size_t)m * a.nH * a.d + n] = y;
+    return;
+  }
+  if (slot < 0) return;
+  const int page = slot / a.page_size, off = slot % a.page_size, h = (head - a.nH) % a.nKV;
+  if (head < a.nH + a.nKV) a.k_cache[(((size_t)page * a.nKV + h) * a.page_size + off) * a.d + at] = y;
+  else a.v_cache[(((size_t)page * a.nKV + h) * a.d + at) * a.page_size + off] = v;
+}
+
+// The slices to a wave with which the products of up to 8 rows take this size, 0: another kernel does.
+static int narrow_slices(int M, int N) {
+  const double b16 = (N + 15) / 16, full16 = 256.0 * (double)((N + 4095) / 4096);
+  if (M <= 4 && N <= 1024) return 4;
+  return (M <= 8 && N <= 2048) || (M <= 4 && b16 > 256.0 && b16 < 0.85 * full16) ? 2 : 0;
+}
+extern "C" int ifx_gemm_f32_narrow_slices(int M, int N) { return M > 0 && N > 0 ? narrow_slices(M, N) : 0; }
+
+// q, k and v of the rows A [M][K] by W [N][K] (both on 16 bytes, K a multiple of 4, sizes that narrow_slices takes) and ``bias`` [N] or null: q to q [M][nH][d],
+// k and v at ``slots`` [M] (page * page_size + offset, below 0: not) into the cache; slots null: N holds q alone, nKV 0.
+extern "C" int ifx_qkv_rope_f32(const float* A, const float* W, const float* bias, float* q, int M, int N, int K, const int* slots, const float* cs, const float* sn,
+                                int nH, int nKV, int d, int page_size, float* k_cache, float* v_cache, void* stream) {
+  IFX_REQUIRE(M > 0 && N > 0 && K > 0 && K % 4 == 0 && narrow_slices(M, N) > 0, "qkv_rope_f32: not for M=%d N=%d K=%d", M, N, K);
+  IFX_REQUIRE(((uintptr_t)A | (uintptr_t)W) % 16 == 0, "qkv_rope_f32: rows and weight must lie on 16 bytes");
+  IFX_REQUIRE(cs && sn && nH > 0 && nKV >= 0 && d > 0 && d % 2 == 0 && N == (nH + 2 * nKV) * d && (slots ? nKV > 0 && page_size > 0 && k_cache && v_cache : nKV == 0),
+              "qkv_rope_f32: %d rows of weight for %d + %d heads of %d", N, nH, nKV, d);
+  const QkvArgs a{A, W, bias, q, M, N, K, slots, cs, sn, nH, nKV, d, page_size, k_cache, v_cache};
+  const int sp = narrow_slices(M, N);
+  const dim3 grid((N + 16 / sp - 1) / (16 / sp)), threads(64 * N_SLICES / sp);
+  hipStream_t s = (hipStream_t)stream;
+  if (sp == 4) hipLaunchKernelGGL((narrow_qkv_kernel<4>), grid, threads, 0, s, a);
+  else hipLaunchKernelGGL((narrow_qkv_kernel<2>), grid, threads, 0, s, a);
+  IFX_LAUNCH_CHECK();
+}
+
 // ---- many rows: tiles of A and W through LDS -----------------------------------------------------------------------------
 // A workgroup of four waves makes (32 TM) x (32 TN) outputs, two waves by two; a step of 32 k-values goes through LDS, the next
 // one is on its way from memory meanwhile.  Bound by the matrix units: a wave reads TM + TN fragments of 16 bytes a lane for
@@ -273,9 +384,9 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
 #define NARROW(SP, STEPS)                                                                                        \
   hipLaunchKernelGGL((gemm_f32_narrow_kernel<TA, TO, SP, STEPS, VEC>), dim3((N + 16 / SP - 1) / (16 / SP)),      \
                      dim3(64 * N_SLICES / SP), 0, s, A, W, bias, C, M, N, K, gated)
-  const double b16 = blocks(16, 16), full16 = 256.0 * rounds(16, 16);
-  if (M <= 4 && N <= 1024) NARROW(4, 4);
-  else if ((M <= 8 && N <= 2048) || (M <= 4 && b16 > 256.0 && b16 < 0.85 * full16)) NARROW(2, 4);
+  const int narrow = narrow_slices(M, N);
+  if (narrow == 4) NARROW(4, 4);
+  else if (narrow == 2) NARROW(2, 4);
   else if (M <= 16 || (in16 && t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
   else if (in32 && t21 <= t22 && t21 <= tiles) FEW(2, 1);
   else if (in32 && t22 <= tiles) FEW(2, 2);

@@ -1377,6 +1377,46 @@ def qkv_rope_append(x: torch.Tensor, weight: LinearWeight, bias: Optional[torch.
     return q
 
 
+@functools.lru_cache(maxsize=4096)
+def _narrow_f32(M: int, N: int) -> bool:
+    return load_module("gemm_f32").fn("ifx_gemm_f32_narrow_slices", (I, I))(M, N) > 0
+
+
+def qkv_rope_f32_takes(x: torch.Tensor, weight, bias: Optional[torch.Tensor]) -> bool:
+    """Whether ``qkv_rope_f32`` takes these rows, weight and bias: where ``gemm_f32`` has its kernel for up to 8 rows."""
+    if x.dtype != torch.float32 or not 0 < x.shape[0] <= 8 or not isinstance(weight, LinearWeight) or weight.rows.dtype != torch.float32:
+        return False
+    N, K = weight.rows.shape
+    return (K % 4 == 0 and _narrow_f32(x.shape[0], N) and (bias is None or bias.dtype == torch.float32) and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and weight.rows.data_ptr() % 16 == 0)
+
+
+def qkv_rope_f32(x: torch.Tensor, weight: LinearWeight, bias: Optional[torch.Tensor], slots: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor,
+                 n_heads: int, n_kv_heads: int, head_dim: int, k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], page_size: int) -> torch.Tensor:
+    """``qkv_rope_append`` in 32 bits, for up to 8 rows: the bits of ``linear`` and ``rope_append`` (split-half pairs over the whole head, values as wide as
+    keys)."""
+    if not qkv_rope_f32_takes(x, weight, bias):
+        raise KernelError(f"qkv_rope_f32: not for {x.shape[0]} rows times a {tuple(weight.rows.shape)} weight")
+    (M, K), N = x.shape, weight.rows.shape[0]
+    n_kv = n_kv_heads if slots is not None else 0
+    if weight.rows.shape[1] != K or head_dim % 2 or N != (n_heads + 2 * n_kv) * head_dim:
+        raise KernelError(f"qkv_rope_f32: a {tuple(weight.rows.shape)} weight for rows of {K} and {n_heads} + {n_kv} heads of {head_dim}")
+    _check(cos, "cos", (M, head_dim // 2), torch.float32)
+    _check(sin, "sin", (M, head_dim // 2), torch.float32)
+    if bias is not None:
+        _check(bias, "bias", (N,), torch.float32)
+    if slots is not None:
+        _check(slots, "slots", (M,), torch.int32)
+        _check(k_cache, "k_cache", (None, n_kv, page_size, head_dim), torch.float32)
+        _check(v_cache, "v_cache", (k_cache.shape[0], n_kv, head_dim, page_size), torch.float32)
+    else:
+        k_cache = v_cache = None
+    q = empty((M, n_heads, head_dim), torch.float32, x)
+    _call(load_module("gemm_f32"), "ifx_qkv_rope_f32", (P, P, P, P, I, I, I, P, P, P, I, I, I, I, P, P, P),
+          x, weight.rows, bias, q, M, N, K, slots, cos, sin, n_heads, n_kv, head_dim, page_size, k_cache, v_cache, _stream())
+    return q
+
+
 def columns_on_16_bytes(x) -> bool:
     """Whether ``x`` is a bfloat16 matrix on the GPU whose rows are columns of wider rows, each run of eight on 16 bytes: what
     ``skinny_gemm`` reads where it lies."""

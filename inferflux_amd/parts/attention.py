@@ -293,6 +293,16 @@ class PagedAttention(Mixer):
             if t is not None:
                 t.mark("mixer.attention")
             return self._project_out(a, sink)
+        if (style == ops.ROPE_SPLIT_HALF and rotary_dim == d and self.v_head_dim == d and h.dtype == torch.float32 and not self.position.needs_apply
+                and ops.qkv_rope_f32_takes(h, w, b)):      # ... in 32 bits too
+            q = ops.qkv_rope_f32(h, w, b, slots, cos, sin, nH, nKV, d, cache.k if slots is not None else None,
+                                 cache.v if slots is not None else None, cache.page_size)
+            if t is not None:
+                t.mark("mixer.qkv")
+            a = self._attend(q, cache, ctx)
+            if t is not None:
+                t.mark("mixer.attention")
+            return self._project_out(a, sink)
         qkv = ops.linear(h, w, keep_slices=not self.position.needs_apply)     # the rotary kernel adds partial sums itself
         if self.position.needs_apply:
             qkv, b = self._encode_outside(qkv, b, ctx, nKV), None
