@@ -137,7 +137,7 @@ def choose_groups(tiled_rows, tiled_keys, n_heads: int, row_keys, pairs: int, wi
     take every other key tile, a tile of 128 elements costs 1.25 us instead of 1.65.  us as it
     was / in two groups: 16 heads of 128 on 2, 500 rows 17.9 / 15.0, 300 after 512 keys 26.2 / 21.1, 64 after 700 24.9 / 19.9, 2 prompts of 512 15.5 / 15.5,
     512 after 512 24.7 / 24.8, 512 after 1,500 43.6 / 43.6, 256 after 3,000 32 / 66; 14 heads of 64 on 2, 500 rows 14.0 / 11.4, 512 after 512 20.6 / 18.4,
-    1,024 24.4 / 18.6, 512 after 1,500 29.7 / 32.1; 336 workgroups of 128 20.5 / 21.5.
+    1,024 24.4 / 18.6, 512 after 1,500 29.7 / 32.1, 61 (a single tile) 5.7 / 6.2; 336 workgroups of 128 20.5 / 21.5.
     The other rows beside them cost little while they end no later than the tiles, against 10 to 13 us of their own launches: a row's walk takes some
     4.5 us and 11 for 1,000 keys, a tile's 5 and 19.5.  us with launches of their own / beside, 16 heads of 128 on 2: 500 rows and 23 rows of up to 299 keys
     28.7 / 15.6, 20 of up to 992 30.5 / 18.6, 512 after 1,500 and 20 of 981 58 / 44, 128 rows and 6 of 369 17.5 / 9.7, but 4 of 1,900 18.0 / 25.6; more
@@ -150,7 +150,7 @@ def choose_groups(tiled_rows, tiled_keys, n_heads: int, row_keys, pairs: int, wi
         row_walk = int(max(row_keys)) if window is None else min(int(max(row_keys)), window)
         if row_walk * 4 <= walk * 7 + (2800 if blocks + pairs <= TILE_GROUPS_MAX else 0):
             return True, True
-    return splits == 1 and walk <= TILE_GROUPS_KEYS, False
+    return splits == 1 and 64 < walk <= TILE_GROUPS_KEYS, False
 
 
 from .device import CUS_PER_XCD, N_XCD      # the launch deals workgroups to the XCDs in turn, and an XCD its share to its compute units in turn

@@ -266,6 +266,8 @@ def test_steps_beyond_a_launch_of_32_bit_tiles_stay_with_the_plain_kernel():
 def test_two_groups_of_waves_and_rows_beside_the_tiles_where_both_were_measured():
     cases = [  # rows of the prompts' portions, their keys, query heads, keys of the other rows, their pairs, window, splits -> (two groups, beside)
         ([500], [500], 16, [], 0, None, 1, (True, False)),
+        ([61], [64], 14, [], 0, None, 1, (False, False)),                   # a single tile has nothing for the second group
+        ([61], [65], 14, [], 0, None, 1, (True, False)),
         ([500], [500], 16, [299] * 23, 46, None, 1, (True, True)),          # 28.7 us in three launches, 15.6 in one
         ([500], [500], 16, [1575] + [50] * 3, 8, None, 1, (True, True)),    # 4 x 1,575 = 7 x 500 + 2,800
         ([500], [500], 16, [1576] + [50] * 3, 8, None, 1, (True, False)),
