@@ -15,6 +15,11 @@
 // other rows load zeros).  With four tiles of x (33-64 rows) a wave multiplies one of them with all row tiles; with two (17-32
 // rows) two waves share one, half of the step's k-tiles each, with one (9-16 rows) all four, a k-tile each, and add their sums through LDS.
 //
+// Two tiles of 8 rows (weights of up to 2,048 rows) are joined into one of 16 by the loads, half of whose lanes take the one and half the other: alone each would fill half a
+// fragment, and half of its slot with zeros, so that the ring held half as much of W.  us at 16 / 32 / 64 rows, of K in slices, each alone / joined (and cut as
+// ring_plan now does): 1,536 x 8,960 8.9, 9.2, 11.9 / 7.6, 8.0, 10.3, 1,536 x 1,536 4.6, 4.7, 6.0 / 4.2, 4.2, 5.1, 2,048 x 11,008 12.3, 13.7, 16.1 / 10.3, 11.0, 14.2,
+// 1,024 x 4,224 5.5, 5.4, 7.3 / 4.3, 4.8, 6.3, 896 x 896 3.8, 4.0, 4.8 / 3.0, 3.4, 4.0.
+//
 // With more than one slice of K the slices write float partial sums, added in slice order by whoever reads them.
 #include "product_tiles.h"
 
@@ -30,6 +35,7 @@ struct RingArgs {
   void* out;                // [M][N] (epi 0) or [M][N / 2]
   float* part;              // [slices][M][N] where there are several
   int M, N, K, n_tiles, tile_rows, steps;      // steps: of 128 k-values, to a slice
+  int joined;               // the copy's tiles hold 8 rows, two of which make one of 16 here (n_tiles and tile_rows are of those)
   const int* order;         // tile t of the copy holds the weight's rows 16 order[t] ...; null: in order
 };
 
@@ -72,11 +78,13 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(RingArgs a) {
   auto place = [](int row) { return (row & 7) ^ ((row >> 3) & 1); };
   const int k_tiles = (a.K + 63) / 64 * 2, all_steps = (a.K + 127) / 128;
   const int first_tile = blockIdx.x * NTW, s0 = blockIdx.y * a.steps, steps = min(a.steps, all_steps - s0);
-  const int k_tile_bytes = 64 * a.tile_rows;
-  const tile_uintx4 wb = tile_buffer(a.w + (size_t)first_tile * k_tiles * (k_tile_bytes / 2), (unsigned)min(NTW, a.n_tiles - first_tile) * (unsigned)k_tiles * k_tile_bytes);
+  const int k_tile_bytes = 64 * (a.joined ? 8 : a.tile_rows), tile_bytes = (a.joined ? 2 : 1) * k_tiles * k_tile_bytes;
+  // (of joined tiles the last may have one half only: the buffer ends with the copy)
+  const int held_tiles = a.joined ? min(2 * NTW, (a.N + 7) / 8 - 2 * first_tile) : min(NTW, a.n_tiles - first_tile);
+  const tile_uintx4 wb = tile_buffer(a.w + (size_t)first_tile * (tile_bytes / 2), (unsigned)held_tiles * (unsigned)k_tiles * k_tile_bytes);
   const tile_uintx4 xb = tile_buffer(a.x, (unsigned)a.M * (unsigned)a.K * 2u);
   // this wave loads k-tile wid of every row tile's four, and MT runs of eight rows of x
-  const int w_lane = col < a.tile_rows ? (a.tile_rows * g + col) * 16 : TILE_NO_ROW;
+  const int w_lane = a.joined ? col / 8 * (k_tiles * k_tile_bytes) + (8 * g + col % 8) * 16 : col < a.tile_rows ? (a.tile_rows * g + col) * 16 : TILE_NO_ROW;
   int xo[MT], xk[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
@@ -92,7 +100,7 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(RingArgs a) {
     if (s >= steps) x[2] = 0;
 #pragma unroll
     for (int j = 0; j < NTW; ++j)
-      ring_load_streaming(w, w_lane == TILE_NO_ROW ? TILE_NO_ROW : w_lane + j * k_tiles * k_tile_bytes, (at * 4 + wid) * k_tile_bytes, to + (j * 4 + wid) * 1024);
+      ring_load_streaming(w, w_lane == TILE_NO_ROW ? TILE_NO_ROW : w_lane + j * tile_bytes, (at * 4 + wid) * k_tile_bytes, to + (j * 4 + wid) * 1024);
     const bool last = at * 128 + 128 > a.K;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -217,7 +225,9 @@ extern "C" int ifx_ring_gemm(const void* x, const void* w, void* out, int out_dt
   IFX_REQUIRE((size_t)x % 16 == 0, "ring_gemm: x must lie on 16 bytes");
   IFX_REQUIRE((long long)row_tiles * ((K + 63) / 64 * 64) * tile_rows * 2 < (1ll << 31) - 4096 && (long long)M * K * 2 < (1ll << 31) - 4096, "ring_gemm: K=%d is too deep", K);
   if (M == 0) return 0;
-  const RingArgs a{(const bf16_t*)x, (const bf16_t*)w, out, part, M, N, K, (N + tile_rows - 1) / tile_rows, tile_rows, steps, order};
+  const int joined = tile_rows == 8 && slices > 1 && row_tiles % 2 == 0, rows = joined ? 16 : tile_rows;
+  if (joined) row_tiles /= 2;
+  const RingArgs a{(const bf16_t*)x, (const bf16_t*)w, out, part, M, N, K, (N + rows - 1) / rows, rows, steps, joined, order};
   hipStream_t s = (hipStream_t)stream;
 #define CASE(NTW_) case NTW_: return M <= 16 ? launch_ring<NTW_, 1>(a, out_dtype, slices, epi, s) : M <= 32 ? launch_ring<NTW_, 2>(a, out_dtype, slices, epi, s) : launch_ring<NTW_, 4>(a, out_dtype, slices, epi, s)
   switch (row_tiles) {

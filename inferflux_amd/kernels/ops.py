@@ -1546,9 +1546,18 @@ RING_DEEP_STEPS = 48          # steps of 128 k-values from which a slice's own t
 def ring_plan(M: int, N: int, K: int, tile_rows: int, one_slice: bool, row_tiles: int = 0, slices: int = 0) -> Tuple[int, int]:
     """(row tiles to a workgroup, steps of 128 k-values to a slice): about one workgroup to each of the 256 compute units.  Weights that
     are cut into slices of K take two row tiles where K is short (896 x 4,864 at 64 rows 7.3 us, 8.0 with eight) and, where it is
-    deep, four up to 32 rows and eight beyond, whose x is read half as often (1,536 x 8,960 12.3 : 11.8, 3,584 x 18,944 30.1 :
-    28.3, but at 17 rows 8.9 : 9.6 and 24.1 : 25.3)."""
-    n_tiles, steps = -(-N // tile_rows), -(-K // 128)
+    deep, four up to 32 rows and eight beyond, whose x is read half as often (3,584 x 18,944 30.1 :
+    28.3, but at 17 rows 24.1 : 25.3).  Of up to 128 tiles of 16 rows (or pairs of 8, which the kernel joins) K is cut into four, or more where that leaves compute units
+    without a workgroup; a workgroup takes one tile, two where K is deep or there are 96 tiles and 17 rows (us by one, two and four tiles: 1,024 x 4,224 at 16 rows 4.3, 4.9,
+    6.3, 2,048 x 4,096 at 32 6.8, 6.3, 6.8, 1,536 x 8,960 at 16 9.0, 7.5, 8.4, at 64 13.0, 10.3, and 10.1 with twice the partial sums to read)."""
+    steps = -(-K // 128)
+    if not one_slice and row_tiles <= 0 and slices <= 0 and -(-N // (16 if tile_rows == 8 else tile_rows)) <= 128:
+        n_tiles, deep = -(-N // (16 if tile_rows == 8 else tile_rows)), steps >= RING_DEEP_STEPS
+        row_tiles = 2 if deep or (M > 16 and n_tiles >= 96) else 1
+        slices = max(1, min(max(4, COMPUTE_UNITS // -(-n_tiles // row_tiles)), steps // 2))
+        per = -(-steps // slices)
+        return (2 * row_tiles if tile_rows == 8 and per < steps else row_tiles), per
+    n_tiles = -(-N // tile_rows)
     if row_tiles <= 0:
         row_tiles = -(-n_tiles // COMPUTE_UNITS) if one_slice else 2 if steps < RING_DEEP_STEPS else 4 if M <= 32 else 8
         row_tiles = min(8, row_tiles)
@@ -1565,7 +1574,7 @@ def ring_takes(M: int, N: int, K: int, tile_rows: int, one_slice: bool) -> bool:
     six to a workgroup for gate/up and one a compute unit for weights that are cut into slices (us at 17 / 32 / 64 rows, wide : ring)
         gate/up 9,728 x 896 9.4 : 6.8, 9.7 : 7.2, 10.7 : 8.6      17,920 x 1,536 14.4 : 13.4, 14.9 : 13.4, 16.9 : 14.7
                 22,016 x 2,048 22.2 : 19.1, 22.2 : 19.3, 22.1 : 20.0, but 37,888 x 3,584 45.1 : 46.8, 44.1 : 47.5, 50.8 : 54.2
-        896 x 4,864 6.6 : 5.7, 6.7 : 5.6, 9.0 : 7.3     1,536 x 8,960 10.5 : 8.9, 10.3 : 9.2, 13.6 : 11.8    1,024 x 1,024 4.3 : 3.7, 4.5 : 3.8, 5.6 : 4.4
+        896 x 4,864 6.6 : 5.0, 6.7 : 5.0, 9.0 : 6.5     1,536 x 8,960 10.5 : 7.3, 10.3 : 8.0, 13.6 : 10.3    1,024 x 1,024 4.3 : 3.1, 4.5 : 3.2, 5.6 : 3.8
         3,584 x 18,944 25.5 : 24.1, 25.6 : 24.5, 31.0 : 28.3     2,560 x 2,048 5.3 : 5.2, 5.8 : 5.6, 7.6 : 7.1, but 4,608 x 3,584 8.5 : 8.8, 9.1 : 9.2, 11.2 : 11.1."""
     return 17 <= M <= SKINNY_MAX_M and -(-N // tile_rows) <= (6 if one_slice else 1) * COMPUTE_UNITS and K < 1 << 20
 
@@ -1593,9 +1602,9 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
         one slice, weights of 2,049 to 12,288 rows and up to 4,096 k-values: 8,448 x 2,048 10.0, 12.9 : 9.1, 9.4     6,272 x 2,048 8.2, 9.4 : 7.5, 7.7
             11,264 x 2,048 12.2, 12.4 : 11.1, 10.7     9,728 x 896 6.8, 7.1 : 6.6, 6.8     4,224 x 1,024 5.6, 5.9 : 5.5, 5.5     3,136 x 1,024 4.4, 4.8 :
             4.2, 4.3, but 17,920 x 1,536 11.9, 13.9 : 12.9, 12.6, 22,016 x 2,048 16.8, 17.5 : 18.1, 17.7, 2,048 x 8,448 12.9, 14.4 : 13.6, 13.4
-        slices, a row tile for a compute unit at most and 4,096 k-values or more: 2,048 x 8,448 12.9, 14.4 : 10.0, 10.0     1,024 x 4,224 7.2, 8.6 : 5.5, 5.6
-            2,048 x 5,632 9.7, 10.9 : 8.1, 8.2     1,536 x 8,960 12.3, 13.7 : 8.8, 8.9     3,584 x 18,944 26.2, 32.8 : 24.5, 24.2, but 2,048 x 2,048 5.4, 5.8 :
-            5.3, 5.4 and a sum for the reader to form."""
+        slices, a row tile for a compute unit at most and 4,096 k-values or more: 2,048 x 8,448 12.9, 14.4 : 9.0, 8.7     1,024 x 4,224 7.2, 8.6 : 4.2, 4.3
+            2,048 x 5,632 9.7, 10.9 : 8.1, 8.2     1,536 x 8,960 12.3, 13.7 : 7.5, 7.6     3,584 x 18,944 26.2, 32.8 : 24.5, 24.2, but 2,048 x 2,048 5.4, 5.8 :
+            4.5, 4.5 and a sum for the reader to form."""
     if not isinstance(weight, LinearWeight) or isinstance(x, ScaledRows) or weight.tiled is None or weight.rows.dtype != torch.bfloat16 \
             or x.dtype != torch.bfloat16 or not x.is_contiguous() or x.data_ptr() % 16:
         return 0
