@@ -11,6 +11,7 @@
 // only), its library call with float accumulation is runtime/backends/cuda/native/cublas_gemm.cpp:99-117.
 #include "common.h"
 #include "f32_loads.h"
+#include "product_tiles.h"
 
 IFX_DEFINE_LAST_ERROR()
 
@@ -362,7 +363,111 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const TA* __restric
     }
 }
 
-// Which kernel: the one with the lowest estimate of its time, all of them in proportion to K.  A kernel's grid runs in rounds of
+// ---- hundreds of rows: tiles of A and W through LDS, the slices of K side by side --------------------------------------------------
+// Four groups of four waves take four slices of K each and all of them the same (32 TM) x (32 TN) outputs, with a stage of LDS of their own, in step; the slices' sums
+// stay apart, 16 TM TN registers of them, and are added up in their order by the groups one after the other.  Sixteen waves keep the matrix units of a compute unit busy
+// where the walk of the kernel above, four waves through all of K, waits at its barriers, and a step's rows are read once for 32 TM or 32 TN outputs, where the kernel of
+// sixteen slices without LDS reads them from the caches for 16 or 32.  A step of 32 k-values of all groups goes straight to LDS, two or three ahead of its use (one with
+// tiles of 64 x 64; by way of registers, one step ahead, a step took 1.3 to 1.7 times as long).  us, the others' best / here: 470 rows of 896 x 4,864 97 / 56, 1,536 x 8,960
+// 255 / 160, 2,048 x 1,536 51 / 35, 1,152 x 896 28 / 24, 896 x 896 21 / 16; 200 rows of 896 x 4,864 52 / 36, 2,048 x 2,048 42 / 27; 64 of 9,728 x 896 31 / 24; many
+// rounds of them are no faster (470 of 9,728 x 896 101 / 105).
+template <typename TO, int TM, int TN>
+__global__ __launch_bounds__(1024) void gemm_f32_groups_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                                                               TO* __restrict__ C, int M, int N, int K, Gated gated) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, BK = 32, GROUPS = 4, PER = N_SLICES / GROUPS, ROWS = BM + BN;
+  constexpr int SLOTS = TM * TN == 1 ? 4 : TM * TN == 2 ? 3 : 2, LOADS = ROWS / 32;      // direct loads of a wave and a step, 8 rows of 128 bytes each
+  __shared__ __attribute__((aligned(1024))) f32x4 stage[SLOTS][GROUPS][ROWS][BK / 4];
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256), lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x % 256 / WAVE);
+  const int i = lane % 16, q = lane / 16;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int wm = (wave / 2) * 16 * TM, wn = (wave % 2) * 16 * TN;
+  const int len = slice_len(K), steps = (len + BK - 1) / BK;
+  // (rows beyond the last lie beyond the buffer's end and are zeros)
+  const tile_uintx4 ab = tile_buffer(A + (size_t)m0 * K, (unsigned)min(BM, M - m0) * (unsigned)K * 4u), wb = tile_buffer(W + (size_t)n0 * K, (unsigned)min(BN, N - n0) * (unsigned)K * 4u);
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&stage[0][group][0][0];
+  const int piece = 4 * (lane % 8 ^ lane / 8);            // of a row's eight the one that lands at lane % 8
+  int ask_slice = 0, ask_step = 0;                        // the next step to ask for
+  auto ask = [&](int slot) {
+    const int k_lo = (PER * group + ask_slice) * len, k_hi = ask_slice < PER ? min(K, k_lo + len) : 0, k = k_lo + BK * ask_step + piece;
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+      const int eight = wave * LOADS + l, row = 8 * eight + lane / 8;
+      const bool of_a = eight < BM / 8;
+      tile_direct_load(of_a ? ab : wb, k < k_hi ? ((of_a ? row : row - BM) * K + k) * 4 : TILE_NO_ROW, base + slot * (GROUPS * ROWS * 128) + eight * 1024);
+    }
+    if (++ask_step == steps) ask_step = 0, ++ask_slice;
+  };
+  f32x4 acc[PER][TM][TN];
+#pragma unroll
+  for (int s = 0; s < PER; ++s)
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int n = 0; n < TN; ++n) acc[s][m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < SLOTS - 1; ++s) ask(s);
+  int slot = 0;
+#pragma unroll
+  for (int s = 0; s < PER; ++s) {
+    const int k_lo = (PER * group + s) * len, k_hi = min(K, k_lo + len);
+    for (int step = 0; step < steps; ++step) {
+      tile_meet<(SLOTS - 2) * LOADS>();                   // the step is there, and everyone has read the one before it
+      ask(slot == 0 ? SLOTS - 1 : slot - 1);
+      f32x4(*As)[BK / 4] = stage[slot][group], (*Ws)[BK / 4] = stage[slot][group] + BM;
+      slot = slot == SLOTS - 1 ? 0 : slot + 1;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (k_lo + BK * step + 16 * h >= k_hi) break;      // (the end of the slice, whose length is a multiple of 16, or of K)
+        f32x4 a[TM], w[TN];
+#pragma unroll
+        for (int m = 0; m < TM; ++m) a[m] = As[wm + 16 * m + i][(4 * h + q) ^ (i % 8)];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) w[n] = Ws[wn + 16 * n + i][(4 * h + q) ^ (i % 8)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) acc[s][m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][j], w[n][j], acc[s][m][n], 0, 0, 0);
+      }
+    }
+  }
+  tile_meet<0>();                                         // (the loads beyond the end)
+  // the groups in turn: what the ones before have added up, and this one's slices in ascending order
+  f32x4* sums = &stage[0][0][0][0];          // [wave][TM][TN][lane]
+  static_assert(4 * TM * TN * WAVE <= GROUPS * ROWS * (BK / 4), "the sums fit the stages' place");
+#pragma unroll 1
+  for (int g = 0; g < GROUPS; ++g) {
+    __syncthreads();
+    if (g != group) continue;
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        f32x4& at = sums[((wave * TM + m) * TN + n) * WAVE + lane];
+        f32x4 total = g == 0 ? acc[0][m][n] : at + acc[0][m][n];
+#pragma unroll
+        for (int s = 1; s < PER; ++s) total = total + acc[s][m][n];
+        if (g < GROUPS - 1) at = total;
+        else acc[0][m][n] = total;
+      }
+  }
+  if (group < GROUPS - 1) return;
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const int col = n0 + wn + 16 * n + i;
+      const float b = bias && col < N ? bias[col] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + 16 * m + 4 * q + r;
+        put(C, row, col, N, bias ? acc[0][m][n][r] + b : acc[0][m][n][r], row < M && col < N, gated);
+      }
+    }
+}
+
+// Which kernel: the one with the lowest estimate of its time, all but the groups' in proportion to K (of more than 3,000 a fifth less).  A kernel's grid runs in rounds of
 // 256 workgroups (one for each compute unit; sixteen waves fill it, and two workgroups of the tile kernel share one).  A round
 // at K = 896 was measured at 5.6 us for 16 x 16 outputs, 7.5 for 32 x 16 and 10.3 for 32 x 32 with the slices side by side; the
 // tile kernel, which walks K in one go, takes 31 us for up to 256 tiles of 64 x 64 and 0.083 us a tile beyond that (but not
@@ -381,12 +486,28 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
                      dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K, gated)
   // (a grid has at most 65,535 rows: millions of rows by a handful of columns are the tile kernel's, whose limit the caller checks)
   const bool in16 = (M + 15) / 16 <= 65535, in32 = (M + 31) / 32 <= 65535;
+#define GROUPS_(TM, TN)                                                                                          \
+  hipLaunchKernelGGL((gemm_f32_groups_kernel<TO, TM, TN>), dim3((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM)), dim3(1024), 0, s, (const float*)A, W, bias, C, M, N, K, gated)
 #define NARROW(SP, STEPS)                                                                                        \
   hipLaunchKernelGGL((gemm_f32_narrow_kernel<TA, TO, SP, STEPS, VEC>), dim3((N + 16 / SP - 1) / (16 / SP)),      \
                      dim3(64 * N_SLICES / SP), 0, s, A, W, bias, C, M, N, K, gated)
+  // the groups' tiles: a round of them, and each 1,000 k-values of it (which of them, -1: another kernel)
+  static const struct { int bm, bn; double round, per_k; } kinds[4] = {{32, 32, 5.4, 5.75}, {64, 32, 6.2, 9.65}, {32, 64, 6.2, 9.65}, {64, 64, 7.7, 16.7}};
+  int groups = -1;
+  if (VEC && sizeof(TA) == 4 && in32 && K <= 1 << 22) {
+    double least = fmin(fmin(in16 ? t11 : 1e30, fmin(t21, t22)), tiles) * (K / 896.0) * (K > 3000 ? 0.82 : 1.0);
+    for (int k = 0; k < 4; ++k) {
+      const double us = rounds(kinds[k].bm, kinds[k].bn) * (kinds[k].round + kinds[k].per_k * K / 1000.0);
+      if (us < least) least = us, groups = k;
+    }
+  }
   const int narrow = narrow_slices(M, N);
   if (narrow == 4) NARROW(4, 4);
   else if (narrow == 2) NARROW(2, 4);
+  else if (M > 16 && groups == 0) GROUPS_(1, 1);
+  else if (M > 16 && groups == 1) GROUPS_(2, 1);
+  else if (M > 16 && groups == 2) GROUPS_(1, 2);
+  else if (M > 16 && groups == 3) GROUPS_(2, 2);
   else if (M <= 16 || (in16 && t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
   else if (in32 && t21 <= t22 && t21 <= tiles) FEW(2, 1);
   else if (in32 && t22 <= tiles) FEW(2, 2);
