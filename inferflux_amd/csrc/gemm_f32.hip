@@ -363,6 +363,92 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(const TA* __restric
     }
 }
 
+// The same of float rows on 16 bytes: a step's rows go straight to LDS, two steps ahead of their use and with one barrier a step, and three workgroups share a compute unit.
+// 470 rows of 9,728 x 896 108 -> 94 us, 2,000 366 -> 315, 4,000 of 896 x 4,864 413 -> 348 (100 to 113 TFLOP/s).
+template <typename TO, int TM, int TN>
+__global__ __launch_bounds__(256) void gemm_f32_walk_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                                                            TO* __restrict__ C, int M, int N, int K, Gated gated) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, BK = 32, ROWS = BM + BN, SLOTS = 3, LOADS = ROWS / 32;      // direct loads of a wave and a step, 8 rows of 128 bytes each
+  __shared__ __attribute__((aligned(1024))) f32x4 stage[SLOTS][ROWS][BK / 4];
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int i = lane % 16, q = lane / 16;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int wm = (wave / 2) * 16 * TM, wn = (wave % 2) * 16 * TN;
+  const int len = slice_len(K), steps = (len + BK - 1) / BK;
+  // (rows beyond the last lie beyond the buffer's end and are zeros)
+  const tile_uintx4 ab = tile_buffer(A + (size_t)m0 * K, (unsigned)min(BM, M - m0) * (unsigned)K * 4u), wb = tile_buffer(W + (size_t)n0 * K, (unsigned)min(BN, N - n0) * (unsigned)K * 4u);
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&stage[0][0][0];
+  int offset[LOADS];                                      // of this lane's piece (of a row's eight the one that lands at lane % 8) in step 0
+  const int piece = 4 * (lane % 8 ^ lane / 8);
+#pragma unroll
+  for (int l = 0; l < LOADS; ++l) {
+    const int row = 8 * (wave * LOADS + l) + lane / 8;
+    offset[l] = ((row < BM ? row : row - BM) * K + piece) * 4;
+  }
+  int ask_lo = 0, ask_step = 0;                           // the slice and the step in it to ask for next
+  auto ask = [&](int slot) {
+    const int k_hi = min(K, ask_lo + len), k = ask_lo + BK * ask_step;
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+      const int eight = wave * LOADS + l;
+      tile_direct_load(eight < BM / 8 ? ab : wb, k + piece < k_hi ? offset[l] + 4 * k : TILE_NO_ROW, base + slot * (ROWS * 128) + eight * 1024);
+    }
+    if (++ask_step == steps) ask_step = 0, ask_lo += len;
+  };
+  f32x4 acc[TM][TN], total[TM][TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) acc[m][n] = total[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < SLOTS - 1; ++s) ask(s);
+  int slot = 0;
+  for (int k_lo = 0; k_lo < K; k_lo += len) {
+    const int k_hi = min(K, k_lo + len);
+    for (int step = 0; step < steps; ++step) {
+      tile_meet<(SLOTS - 2) * LOADS>();                   // the step is there, and everyone has read the one before it
+      ask(slot == 0 ? SLOTS - 1 : slot - 1);
+      f32x4(*As)[BK / 4] = stage[slot], (*Ws)[BK / 4] = stage[slot] + BM;
+      slot = slot == SLOTS - 1 ? 0 : slot + 1;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (k_lo + BK * step + 16 * h >= k_hi) break;      // (the end of the slice, whose length is a multiple of 16, or of K)
+        f32x4 a[TM], w[TN];
+#pragma unroll
+        for (int m = 0; m < TM; ++m) a[m] = As[wm + 16 * m + i][(4 * h + q) ^ (i % 8)];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) w[n] = Ws[wn + 16 * n + i][(4 * h + q) ^ (i % 8)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][j], w[n][j], acc[m][n], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        total[m][n] = k_lo == 0 ? acc[m][n] : total[m][n] + acc[m][n];
+        acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  tile_meet<0>();                                         // (the loads beyond the end have landed before the workgroup leaves)
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const int col = n0 + wn + 16 * n + i;
+      const float b = bias && col < N ? bias[col] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + 16 * m + 4 * q + r;
+        put(C, row, col, N, bias ? total[m][n][r] + b : total[m][n][r], row < M && col < N, gated);
+      }
+    }
+}
+
 // ---- hundreds of rows: tiles of A and W through LDS, the slices of K side by side --------------------------------------------------
 // Four groups of four waves take four slices of K each and all of them the same (32 TM) x (32 TN) outputs, with a stage of LDS of their own, in step; the slices' sums
 // stay apart, 16 TM TN registers of them, and are added up in their order by the groups one after the other.  Sixteen waves keep the matrix units of a compute unit busy
@@ -471,7 +557,7 @@ __global__ __launch_bounds__(1024) void gemm_f32_groups_kernel(const float* __re
 // 256 workgroups (one for each compute unit; sixteen waves fill it, and two workgroups of the tile kernel share one).  A round
 // at K = 896 was measured at 5.6 us for 16 x 16 outputs, 7.5 for 32 x 16 and 10.3 for 32 x 32 with the slices side by side; the
 // tile kernel, which walks K in one go, takes 31 us for up to 256 tiles of 64 x 64 and 0.083 us a tile beyond that (but not
-// less than 44).  Before these kernels (one thread summing an output, tiles of 64 x 64, scalar loads) a product took 83 us at
+// less than 44), with direct loads 12 us and 16 for each 256 tiles.  Before these kernels (one thread summing an output, tiles of 64 x 64, scalar loads) a product took 83 us at
 // 1 row and 102 at 475 of 896 x 896 (now 4.3 and 20), 449 and 559 of 896 x 4,864 (14.5 and 97), 90 and 266 of 9,728 x 896 (10.2
 // and 105), 410 at one row of 151,936 x 896 (97: 5.6 TB/s); 2,048 rows of 22,016 x 2,048 run at 103 TFLOP/s.  Errors against 64
 // bits fell to a third (5.4e-7 to 2.0e-7 at K = 896, 1.9e-6 to 6.6e-7 at 11,008): shorter chains.
@@ -480,7 +566,8 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
   auto blocks = [&](int m, int n) { return (double)((M + m - 1) / m) * ((N + n - 1) / n); };
   auto rounds = [&](int m, int n) { return (double)(long long)((blocks(m, n) + 255.0) / 256.0); };
   const double t11 = 5.6 * rounds(16, 16), t21 = 7.5 * rounds(32, 16), t22 = 10.3 * rounds(32, 32);
-  const double b64 = blocks(64, 64), tiles = b64 <= 256.0 ? 31.0 : (b64 < 530.0 ? 44.0 : 0.083 * b64);
+  constexpr bool direct = VEC && sizeof(TA) == 4;          // (rows that may go straight to LDS)
+  const double b64 = blocks(64, 64), tiles = direct ? 12.0 + 16.0 * rounds(64, 64) : b64 <= 256.0 ? 31.0 : (b64 < 530.0 ? 44.0 : 0.083 * b64);
 #define FEW(MT, NT)                                                                                              \
   hipLaunchKernelGGL((gemm_f32_few_kernel<TA, TO, MT, NT, 4, VEC>),                                              \
                      dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)), dim3(1024), 0, s, A, W, bias, C, M, N, K, gated)
@@ -494,7 +581,7 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
   // the groups' tiles: a round of them, and each 1,000 k-values of it (which of them, -1: another kernel)
   static const struct { int bm, bn; double round, per_k; } kinds[4] = {{32, 32, 5.4, 5.75}, {64, 32, 6.2, 9.65}, {32, 64, 6.2, 9.65}, {64, 64, 7.7, 16.7}};
   int groups = -1;
-  if (VEC && sizeof(TA) == 4 && in32 && K <= 1 << 22) {
+  if (direct && in32 && K <= 1 << 22) {
     double least = fmin(fmin(in16 ? t11 : 1e30, fmin(t21, t22)), tiles) * (K / 896.0) * (K > 3000 ? 0.82 : 1.0);
     for (int k = 0; k < 4; ++k) {
       const double us = rounds(kinds[k].bm, kinds[k].bn) * (kinds[k].round + kinds[k].per_k * K / 1000.0);
@@ -511,6 +598,8 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
   else if (M <= 16 || (in16 && t11 <= t21 && t11 <= t22 && t11 <= tiles)) FEW(1, 1);
   else if (in32 && t21 <= t22 && t21 <= tiles) FEW(2, 1);
   else if (in32 && t22 <= tiles) FEW(2, 2);
+  else if (direct && K <= 1 << 22)
+    hipLaunchKernelGGL((gemm_f32_walk_kernel<TO, 2, 2>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, (const float*)A, W, bias, C, M, N, K, gated);
   else
     hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K, gated);
 #undef FEW
