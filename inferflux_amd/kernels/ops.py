@@ -1299,7 +1299,17 @@ def takes_scaled_rows(n_rows: int, weight) -> bool:
 
 
 def adds_into_stream(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
-    """Whether ``linear_into_stream`` takes this shape."""
+    """Whether a product of this shape is best added to the stream by ``linear_into_stream``, which takes it then.  Where 9 to 16 rows times a deep weight of up to 2,048 rows go to the ring in slices of K, they and the
+    norm that adds the slices are faster (us of down and the product behind it, into the stream : slices and norm, at 9, 12 and 16 rows: 896 x 4,864 12.0, 13.1, 14.1 : 11.1,
+    11.6, 11.8, 1,024 x 4,224 12.1, 13.1, 13.9 : 11.4, 11.5, 11.8, 1,536 x 8,960 17.3, 18.1, 19.3 : 15.6, 16.0, 16.0, 2,048 x 11,008 33.5, 34.8, 34.4 : 30.6, 30.9, 30.4;
+    but 2,560 x 9,728 22.3, 21.0, 23.5 : 22.8, 21.8, 22.4, 3,584 x 18,944 38.4, 41.8, 47.4 : 40.6, 41.3, 42.0, and at 8 rows all but one slower)."""
+    if not _into_stream_takes(n_rows, weight, norm_weight):
+        return False
+    N, K = weight.rows.shape
+    return not (RING_FEW_MIN_ROWS <= n_rows and N <= RING_FEW_STREAM_MAX_N and K >= RING_FEW_MIN_SLICED_K and weight.tiled is not None)
+
+
+def _into_stream_takes(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
     if not isinstance(weight, LinearWeight) or weight.order is not None:
         return False
     N, K = weight.rows.shape
@@ -1316,7 +1326,7 @@ def linear_into_stream(x: torch.Tensor, weight: LinearWeight, stream: torch.Tens
     _check(x, "x", (None, None), torch.bfloat16)
     M, K = x.shape
     N = weight.rows.shape[0]
-    if not adds_into_stream(M, weight, norm_weight) or weight.rows.shape[1] != K:
+    if not _into_stream_takes(M, weight, norm_weight) or weight.rows.shape[1] != K:
         raise KernelError(f"linear_into_stream: not for {M} rows times a {tuple(weight.rows.shape)} weight")
     _check(stream, "stream", (M, N), torch.float32)
     _check(norm_weight, "norm_weight", (N,))
@@ -1594,6 +1604,7 @@ def _ring_in_one_slice(M: int, N: int, K: int, tile_rows: int, keep_slices: bool
 
 RING_FEW_MIN_ROWS = 9            # (up to 8 rows x is little to read beside W)
 RING_FEW_MIN_SLICED_K = 4096
+RING_FEW_STREAM_MAX_N = 2048         # (see ``adds_into_stream``)
 
 
 def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
