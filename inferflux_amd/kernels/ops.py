@@ -575,12 +575,15 @@ def latent_query(q: torch.Tensor, latent: torch.Tensor, weight: torch.Tensor, n_
 
 
 def linear_normed_takes(x, weight, rank: int) -> bool:
-    """Whether ``linear_normed`` takes ``x`` and this weight, a norm over the first ``rank`` columns of whose product follows."""
+    """Whether ``linear_normed`` takes ``x`` and this weight, a norm over the first ``rank`` columns of whose product follows: a weight whose tiles end where
+    those columns do (weights of 2,049 to 3,584 rows have tiles of 10 to 14, which divide few ranks: there the norm keeps its launch), and rows that
+    ``linear`` would not send to the ring in slices, whose sums reach the norm in float (928 x 4,096 to the heads' queries at 9 and 16 rows 17.2, 17.1 us,
+    joined 15.0, 17.0, but a cached latent's error against 64 bits is 1.65e-3 so and 2.35e-3 through bfloat16)."""
     if not isinstance(weight, LinearWeight) or weight.order is not None or weight.tiled is None or x.dtype != torch.bfloat16:
         return False
     N, K = weight.rows.shape
     return (weight.rows.dtype == torch.bfloat16 and x.shape[0] <= 16 and N % 8 == 0 and 0 < rank <= N and rank % weight.tile_rows == 0
-            and _small_m_kernel(x.shape[0], N, K, True) == "skinny" and not ring_takes_few(x, weight))
+            and _small_m_kernel(x.shape[0], N, K, True) == "skinny" and not ring_takes_few(x, weight, True))
 
 
 def normed_columns_take(n_rows: int, weight, rank: int) -> bool:
@@ -1626,6 +1629,12 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
     if keep_slices and tiles <= COMPUTE_UNITS and RING_FEW_MIN_SLICED_K <= K < 1 << 20:
         return 2
     return 1 if 2048 < N and tiles <= 3 * COMPUTE_UNITS and K <= RING_FEW_MIN_SLICED_K else 0
+
+
+def leaves_few_rows_in_sums(x, weight) -> bool:
+    """Whether ``linear`` with ``keep_slices`` leaves these up to 16 rows times ``weight`` as partial sums in float."""
+    N, K = weight.rows.shape
+    return ring_takes_few(x, weight, True) == 2 or (weight.tiled is not None and N < WIDE_FEW_ROWS_MIN_N and _small_m_kernel(x.shape[0], N, K, True) == "wide")
 
 
 def streams_weight(n_rows: int, weight) -> bool:

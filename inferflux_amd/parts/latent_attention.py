@@ -178,7 +178,9 @@ class LatentAttention(Mixer):
         slots = None if self.shared_latent else ctx.write_slots(cache.group)
         rank, heads_w = self.q_rank, nh * (self.dim + self.rot_dim)
         q = latent = None
-        if self.w_few is not None and h.dtype == cache.k.dtype and ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank):
+        # (the joined products write bfloat16: where the latent would reach its norm as float sums the products stay apart)
+        if (self.w_few is not None and h.dtype == cache.k.dtype and ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank)
+                and not ops.leaves_few_rows_in_sums(h, self.w_down)):
             y = ops.linear(h, self.w_few)
             q, latent = y[:, :heads_w], y[:, heads_w:]
         elif (self.few_scale is not None and h.dtype == cache.k.dtype and ops.linear_normed_takes(h, self.w_down, rank)

@@ -1,0 +1,59 @@
+"""Which products a step of few rows takes in attention through a latent, seen on the CPU: the first product that the layer asks for stands
+for the route, before anything is launched."""
+import types
+
+import pytest
+import torch
+
+from inferflux_amd.kernels import ops
+from inferflux_amd.parts.latent_attention import LatentAttention
+from inferflux_amd.parts.plan import PartSpec
+
+BF16 = torch.bfloat16
+
+
+class Asked(Exception):
+    pass
+
+
+def tiled(rows):
+    """A weight with a copy, of which only its existence is looked at here."""
+    return ops.LinearWeight(rows, torch.empty(0, dtype=rows.dtype), None, ops.choose_tile_rows(rows.shape[0]))
+
+
+def route(monkeypatch, hidden, rows, q_rank, gate):
+    """("joined" | "normed" | "apart", whether partial sums are taken) of a step of ``rows`` plain rows."""
+    a = LatentAttention("a", hidden, 8, 64, 32, 64, q_rank, 96, 0.1, 1e-5, PartSpec("none"), output_gate=gate)
+    zeros = lambda *shape: torch.zeros(shape, dtype=BF16)
+    a.load({n: zeros(*s.shape) for n, s in a.param_specs().items()})
+    a.w_down, a.w_uq = tiled(a.w_down.rows), tiled(a.w_uq.rows)
+    if q_rank:
+        a.few_scale = torch.ones(a.w_down.shape[0], dtype=BF16)
+    elif not gate:
+        a.w_few = tiled(torch.cat([a.w_uq.rows, a.w_down.rows]))
+    a.position = types.SimpleNamespace(kernel_args=lambda ctx: (None, 0, None, None))
+
+    def linear(x, weight, out_dtype=None, keep_slices=False):
+        raise Asked("joined" if weight is a.w_few else "apart", keep_slices and ops.ring_takes_few(x, weight, True) == 2)
+
+    def normed(*args):
+        raise Asked("normed", False)
+    monkeypatch.setattr(ops, "linear", linear)
+    monkeypatch.setattr(ops, "linear_normed", normed)
+    cache = types.SimpleNamespace(group=0, k=zeros(1, 1, 16, 128))
+    ctx = types.SimpleNamespace(timer=None, write_slots=lambda group: None)
+    with pytest.raises(Asked) as asked:
+        a.forward(zeros(rows, hidden), ctx, types.SimpleNamespace(cache=cache, writes_cache=True))
+    return asked.value.args
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 12, 16])
+@pytest.mark.parametrize("q_rank,gate", [(768, False), (768, True), (None, False)])
+@pytest.mark.parametrize("hidden", [2048, 4088, 4096, 5120])
+def test_down_products_whose_sums_stayed_in_float_still_do(monkeypatch, hidden, q_rank, gate, rows):
+    """9 to 16 plain rows times a deep down projection go to the ring in slices of K, whose float sums the latent's norm, the rotation and the
+    output gate's sigmoid read: neither of the joined products, which write bfloat16, may take them away."""
+    way, sums = route(monkeypatch, hidden, rows, q_rank, gate)
+    deep = rows >= 9 and hidden >= 4096
+    assert sums == deep
+    assert way == ("apart" if deep else "normed" if q_rank else "joined")
