@@ -1302,14 +1302,15 @@ def takes_scaled_rows(n_rows: int, weight) -> bool:
 
 
 def adds_into_stream(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
-    """Whether a product of this shape is best added to the stream by ``linear_into_stream``, which takes it then.  Where 9 to 16 rows times a deep weight of up to 2,048 rows go to the ring in slices of K, they and the
-    norm that adds the slices are faster (us of down and the product behind it, into the stream : slices and norm, at 9, 12 and 16 rows: 896 x 4,864 12.0, 13.1, 14.1 : 11.1,
+    """Whether a product of this shape is best added to the stream by ``linear_into_stream``, which takes it then.
+
+    Where 9 to 16 rows times a deep weight of up to 2,048 rows go to the ring in slices of K, they and the norm that adds the slices are faster (us of down and the
+    product behind it, into the stream : slices and norm, at 9, 12 and 16 rows: 896 x 4,864 12.0, 13.1, 14.1 : 11.1,
     11.6, 11.8, 1,024 x 4,224 12.1, 13.1, 13.9 : 11.4, 11.5, 11.8, 1,536 x 8,960 17.3, 18.1, 19.3 : 15.6, 16.0, 16.0, 2,048 x 11,008 33.5, 34.8, 34.4 : 30.6, 30.9, 30.4;
     but 2,560 x 9,728 22.3, 21.0, 23.5 : 22.8, 21.8, 22.4, 3,584 x 18,944 38.4, 41.8, 47.4 : 40.6, 41.3, 42.0, and at 8 rows all but one slower)."""
     if not _into_stream_takes(n_rows, weight, norm_weight):
         return False
-    N, K = weight.rows.shape
-    return not (RING_FEW_MIN_ROWS <= n_rows and N <= RING_FEW_STREAM_MAX_N and K >= RING_FEW_MIN_SLICED_K and weight.tiled is not None)
+    return weight.rows.shape[0] > RING_FEW_STREAM_MAX_N or not _few_in_slices(n_rows, weight)
 
 
 def _into_stream_takes(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
@@ -1610,6 +1611,13 @@ RING_FEW_MIN_SLICED_K = 4096
 RING_FEW_STREAM_MAX_N = 2048         # (see ``adds_into_stream``)
 
 
+def _few_in_slices(n_rows: int, weight: LinearWeight) -> bool:
+    """Whether ``n_rows`` rows times ``weight`` go to ``ring_gemm`` in slices of K where their reader adds the slices (see ``ring_takes_few``)."""
+    N, K = weight.rows.shape
+    return (RING_FEW_MIN_ROWS <= n_rows <= 16 and weight.tiled is not None and weight.rows.dtype == torch.bfloat16 and -(-N // weight.tile_rows) <= COMPUTE_UNITS
+            and RING_FEW_MIN_SLICED_K <= K < 1 << 20 and K % 8 == 0 and _small_m_kernel(n_rows, N, K, True) == "skinny")
+
+
 def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
     """Whether 9 to 16 rows that would go to the product whose waves each read x from the L2 go to ``ring_gemm``, whose workgroups read it
     once: 1 in one slice of K, 2 in slices whose sum the caller takes, 0 not (us at 9 and 16 rows, that product : this one)
@@ -1625,9 +1633,9 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
     (M, K), N = x.shape, weight.rows.shape[0]
     if not RING_FEW_MIN_ROWS <= M <= 16 or K % 8 or K != weight.rows.shape[1] or _small_m_kernel(M, N, K, True) != "skinny":
         return 0
-    tiles = -(-N // weight.tile_rows)
-    if keep_slices and tiles <= COMPUTE_UNITS and RING_FEW_MIN_SLICED_K <= K < 1 << 20:
+    if keep_slices and _few_in_slices(M, weight):
         return 2
+    tiles = -(-N // weight.tile_rows)
     return 1 if 2048 < N and tiles <= 3 * COMPUTE_UNITS and K <= RING_FEW_MIN_SLICED_K else 0
 
 

@@ -1,5 +1,5 @@
-"""Which products a step of few rows takes in attention through a latent, seen on the CPU: the first product that the layer asks for stands
-for the route, before anything is launched."""
+"""Which products a step of few rows takes, seen on the CPU, before anything is launched: in attention through a latent the first product that the layer
+asks for stands for the route."""
 import types
 
 import pytest
@@ -57,3 +57,16 @@ def test_down_products_whose_sums_stayed_in_float_still_do(monkeypatch, hidden, 
     deep = rows >= 9 and hidden >= 4096
     assert sums == deep
     assert way == ("apart" if deep else "normed" if q_rank else "joined")
+
+
+@pytest.mark.parametrize("N,K", [(8, 4096), (2048, 4096), (2048, 4088), (2048, 4104), (2052, 4096), (896, 4864), (8, 1 << 20), (16, (1 << 20) - 8), (64, 4100)])
+def test_what_is_not_added_into_the_stream_leaves_its_sums_in_float(N, K):
+    """``adds_into_stream`` gives a product to the norm only where ``linear`` then leaves partial sums: a rounded one would lose what the stream's
+    epilogue keeps."""
+    weight, norm = tiled(torch.empty((N, K), dtype=BF16)), torch.empty(N, dtype=BF16)
+    for rows in (8, 9, 16):
+        x = torch.empty((rows, K), dtype=BF16)
+        into, sums = ops.adds_into_stream(rows, weight, norm), ops.ring_takes_few(x, weight, True) == 2
+        assert into or sums or K % 8, (rows, N, K)
+        assert into == (not sums or N > 2048) or K % 8, (rows, N, K)
+    assert ops.adds_into_stream(16, ops.LinearWeight(weight.rows), norm) == (K % 8 == 0)
