@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import itertools
 from typing import Dict, Iterable, Optional, Tuple
 
 import torch
@@ -1098,8 +1099,8 @@ def choose_tile_rows(N: int) -> int:
 class LinearWeight:
     """A projection's weight as the products want it: ``rows`` [N, K] as the model file has it, and for
     bfloat16 weights ``tiled``, the copy that products with few rows of x (decoding) stream from.  The
-    copy doubles the weight's memory; it is left out when ``decode_weight_copy`` is off or when the
-    card has no room for it, and products with few rows then read ``rows``."""
+    copy doubles the weight's memory (see ``prepare_stacked`` for weights that are also rows of a larger one); it is left out when
+    ``decode_weight_copy`` is off or when the card has no room for it, and products with few rows then read ``rows``."""
 
     __slots__ = ("rows", "tiled", "order", "tile_rows")
 
@@ -1149,6 +1150,22 @@ def prepare_linear(weight: torch.Tensor, order: Optional[torch.Tensor] = None, t
             log.warn("kernels", f"no room for the decode copy of a {tuple(weight.shape)} weight "
                                 f"({free / 2**30:.1f} GiB free): decoding reads the plain rows")
     return LinearWeight(weight, tiled, order if tiled is not None else None, tile_rows if tiled is not None else 16)
+
+
+def prepare_stacked(weights) -> Tuple[Optional[LinearWeight], list]:
+    """(``weights`` [N_i, K] one below the other as one weight, each of them as a weight of its own), over the same rows.
+
+    A part that would by itself have tiles as high as the whole's, and whose rows whole tiles of it hold, shares the whole's tiled copy (up to 2,048 rows in
+    all, as a rule, every part).  The others have copies of their own, and the whole's is then one more, which it gets while a quarter of the card is free:
+    copies of other weights may still have to be made.  The whole is None where it has no copy and a part has one."""
+    rows = torch.cat(list(weights))
+    ends = list(itertools.accumulate(w.shape[0] for w in weights))
+    spans, height = list(zip([0] + ends, ends)), choose_tile_rows(rows.shape[0])
+    shared = [choose_tile_rows(b - a) == height and a % height == 0 and (b % height == 0 or b == ends[-1]) for a, b in spans]
+    free, total = torch.cuda.mem_get_info(rows.device)
+    whole = prepare_linear(rows) if all(shared) or free >= total // 4 else LinearWeight(rows)
+    parts = [whole.part(a, b) if s and whole.tiled is not None else prepare_linear(rows[a:b]) for s, (a, b) in zip(shared, spans)]
+    return (None if whole.tiled is None and any(p.tiled is not None for p in parts) else whole), parts
 
 
 class ScaledRows:

@@ -142,9 +142,9 @@ class LatentAttention(Mixer):
         self.w_few = None
         if w_q.is_cuda and not (self.q_rank or self.output_gate) and down.dtype == w_q.dtype == torch.bfloat16 and self.hidden_size % 8 == 0:
             # queries and latent as one product, for steps of few rows (its rows are the two weights' own)
-            self.w_few = ops.prepare_linear(torch.cat([w_q, down]))
-            w_q, down = self.w_few.rows[:w_q.shape[0]], self.w_few.rows[w_q.shape[0]:]
-        self.w_down, self.w_uq = ops.prepare_linear(down), ops.prepare_linear(w_q)
+            self.w_few, (self.w_uq, self.w_down) = ops.prepare_stacked([w_q, down])
+        else:
+            self.w_down, self.w_uq = ops.prepare_linear(down), ops.prepare_linear(w_q)
         if self.sinks:
             self.sink_scores = tensors[f"{n}.sink"].float().contiguous()        # scores are float whatever the file holds
         self.w_o = ops.prepare_linear(tensors[f"{n}.o"])

@@ -332,6 +332,34 @@ def test_norm_over_a_products_first_columns(T, N, K, rank, N2, scaled, norm_dtyp
         ops.linear_normed(xd, down, g.to(DEV), rank + 1, 1e-5)
 
 
+@pytest.mark.parametrize("heads,share", [(8, "both"), (16, "neither"), (40, "queries")])
+def test_joined_queries_and_latent_share_their_copy_or_give_way(heads, share, monkeypatch):
+    """768 + 128, 1,536 + 640 and 3,840 + 640 rows: one copy for all three weights, or further ones while the card has much room."""
+    from inferflux_amd.parts.latent_attention import LatentAttention
+    from inferflux_amd.parts.plan import PartSpec
+
+    def loaded():
+        a = LatentAttention("a", 256, heads, 64, 32, 64, None, 96 if share == "both" else 608, 0.1, 1e-5, PartSpec("none"))
+        a.load({n: rnd(90 + i, *s.shape, scale=0.1).bfloat16().to(DEV) for i, (n, s) in enumerate(a.param_specs().items())})
+        return a
+    a, x = loaded(), rnd(95, 12, 256).bfloat16().to(DEV)
+    where = lambda w: w.tiled.untyped_storage().data_ptr()
+    assert (where(a.w_uq) == where(a.w_few), where(a.w_down) == where(a.w_few)) == {"both": (True, True), "neither": (False, False), "queries": (True, False)}[share]
+    assert torch.equal(torch.cat([a.w_uq.rows, a.w_down.rows]), a.w_few.rows)
+    want = x.double() @ a.w_few.rows.double().T
+    for w, cols in ((a.w_few, slice(0, None)), (a.w_uq, slice(0, heads * 96)), (a.w_down, slice(heads * 96, None))):
+        alone = ops.prepare_linear(w.rows.clone())
+        assert w.tile_rows == alone.tile_rows and torch.equal(w.tiled, alone.tiled)          # (the copy that it would have by itself)
+        assert rel_err(ops.linear(x, w).cpu(), want[:, cols].cpu()) < 4e-3
+    total = torch.cuda.mem_get_info()[1]
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (total // 4 - 1, total))
+    a = loaded()
+    assert (a.w_few is not None) == (share == "both") and a.w_uq.tiled is not None and a.w_down.tiled is not None
+    monkeypatch.setattr(ops, "decode_weight_copy", False)
+    a = loaded()
+    assert a.w_few.tiled is None and a.w_uq.tiled is None and a.w_down.tiled is None
+
+
 def test_rows_leave_their_splits_to_the_reader():
     q, kc, vc, table, want = _paged_case("bfloat16", 300, None, 48, 48, 4)
     rows, pos = torch.tensor([0, 17, 64, 299]), torch.tensor([0, 17, 64, 299], dtype=torch.int32, device=DEV)
