@@ -558,8 +558,8 @@ __global__ __launch_bounds__(1024) void gemm_f32_groups_kernel(const float* __re
 // at K = 896 was measured at 5.6 us for 16 x 16 outputs, 7.5 for 32 x 16 and 10.3 for 32 x 32 with the slices side by side; the
 // tile kernel, which walks K in one go, takes 31 us for up to 256 tiles of 64 x 64 and 0.083 us a tile beyond that (but not
 // less than 44), with direct loads 12 us and 16 for each 256 tiles.  Before these kernels (one thread summing an output, tiles of 64 x 64, scalar loads) a product took 83 us at
-// 1 row and 102 at 475 of 896 x 896 (now 4.3 and 20), 449 and 559 of 896 x 4,864 (14.5 and 97), 90 and 266 of 9,728 x 896 (10.2
-// and 105), 410 at one row of 151,936 x 896 (97: 5.6 TB/s); 2,048 rows of 22,016 x 2,048 run at 103 TFLOP/s.  Errors against 64
+// 1 row and 102 at 475 of 896 x 896 (now, in a graph, 2.8 and 14.4), 449 and 559 of 896 x 4,864 (8.5 and 54), 90 and 266 of 9,728 x 896 (10.0
+// and 87), 410 at one row of 151,936 x 896 (103: 5.3 TB/s); 2,048 rows of 22,016 x 2,048 run at 121 TFLOP/s.  Errors against 64
 // bits fell to a third (5.4e-7 to 2.0e-7 at K = 896, 1.9e-6 to 6.6e-7 at 11,008): shorter chains.
 template <typename TA, typename TO, bool VEC>
 static void launch(const TA* A, const float* W, const float* bias, TO* C, int M, int N, int K, Gated gated, hipStream_t s) {
@@ -601,8 +601,10 @@ static void launch(const TA* A, const float* W, const float* bias, TO* C, int M,
   else if (direct && K <= 1 << 22)
     hipLaunchKernelGGL((gemm_f32_walk_kernel<TO, 2, 2>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, (const float*)A, W, bias, C, M, N, K, gated);
   else
-    hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K, gated);
+    // (float rows beyond 4M k-values, whose tiles no buffer's offsets reach, go with those that do not lie on 16 bytes)
+    hipLaunchKernelGGL((gemm_f32_tiles_kernel<TA, TO, 2, 2, VEC && !direct>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, W, bias, C, M, N, K, gated);
 #undef FEW
+#undef GROUPS_
 #undef NARROW
 }
 
