@@ -386,11 +386,10 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
         # Two query tiles per wave (128 rows per workgroup) read every key and value from LDS half as often.
         tiled = ctx.h_q_len >= TILE_MIN
         qt, splits, chunk = 1, 1, 0
+        two = beside = False
         if tiled.any():
             qt, splits, chunk = choose_tiling(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, lambda t: ops.attention_tile_rows(d, t),
                                               tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not keep_first and not block)
-        two = beside = False
-        if tiled.any():
             row_req = np.nonzero(~tiled & (ctx.h_q_len > 0))[0]
             two, beside = choose_groups(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, ctx.h_kv_len[row_req], int(ctx.h_q_len[row_req].sum()) * n_kv,
                                         window, splits, not keep_first)
