@@ -21,8 +21,9 @@
 // columns of v into LDS (the next stage's are asked for before the walk and land in registers meanwhile), a few lanes per
 // (token, vector) form the unit norms, a thread per token beta and the decay; everybody walks the stage's tokens and
 // leaves o in LDS, from where it goes to ``o_raw`` [T, H dv] (float).  A second kernel, a wave per (token, head), norms and
-// gates o.  The order of a token's operations does not depend on how the request was cut into steps, so results are
-// bit-equal across cuttings.
+// gates o.  The order of a token's operations does not depend on how a request's portions were cut, so its results are the same bits in
+// every cutting into portions.  Tokens that come one to a step differ by their sums' order: in 32 bits their layout gives a thread of the walk more channels
+// (differences of 1e-6); in bfloat16 they have a kernel of their own (delta_step_kernel), which does not round the convolution's output either.
 #include "common.h"
 #include "lane_sums.h"
 
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(256) void delta_finish_kernel(DeltaArgs a) {
 // results and the gates meet in LDS, and every load goes out before any is used, without branches between them, so that what meets there is waited for
 // while S is on its way.  Everything between the rows and the output is float.  Bound by its launch, a trip to memory and the arithmetic behind it, for
 // many requests by S.  16 heads of 64 x 128, four taps, us in launches for the convolution, the walk and the norm / in one, at 1, 16, 32, 64
-// requests: 13.0 / 5.2, 24.0 / 7.6, 37.8 / 10.1, 70.4 / 19.7 (67 MB of S at 64).  (In 32 bits a token's bits are the same alone and among others of its request: the walk's.)
+// requests: 13.0 / 5.2, 24.0 / 7.6, 37.8 / 10.1, 70.4 / 19.7 (67 MB of S at 64).  (32-bit steps stay with the walk.)
 struct StepConv {
   const void* w;          // [2 G d + H dv][TAPS]
   int w_dtype;

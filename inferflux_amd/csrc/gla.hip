@@ -745,10 +745,11 @@ static int launch_gla(const GlaArgs& a, int T_rows, int R, int n_chunks, const i
     }
   }
   // A thread holds 1, 2 or 4 columns of S as its registers allow (4 for runs of 16 channels, 2 for 32): what it reads of a
-  // token's q, k and decays from LDS then serves several columns.  Two where possible (steps of single tokens, which are bound
-  // by reading and writing S: 23 against 33 us for 64 requests of 16 heads x 64 x 128; chunks side by side: 86 + 64 against
-  // 95 + 67 us for 2,048 rows), more only where a head's columns would not fit a workgroup otherwise.  The first d threads also
-  // load, so a head of few values still gets a thread per key channel.
+  // token's q, k and decays from LDS then serves several columns.  Two where possible, more only where a head's columns would not fit a
+  // workgroup otherwise.  us by one column / two: single tokens of 1, 16 and 64 requests in 32 bits, 16 heads of 64 x 128, 4.9, 8.2, 23.7 / 5.6, 9.0,
+  // 23.4, in bfloat16 where gla_step_kernel does not take them, 4 heads of 128 x 256, 15.0, 17.1, 25.3 / 12.5, 15.1, 23.1; chunks that the
+  // matrix cores do not take, 2,048 rows of 16 heads of 96 x 128, 493 / 382, but of 64 x 96 140 / 178; a prompt of 2,048 rows in 32 bits, one chain,
+  // is longer by two: 16 heads of 64 x 128 1,639 / 2,732.  The first d threads also load, so a head of few values still gets a thread per key channel.
   IFX_REQUIRE(a.z, "gla_scan: the decays' second product is formed in steps of single tokens only (bfloat16, heads that gla_step_takes)");
   constexpr int MAX_COLS = DP <= 16 ? 4 : (DP <= 32 ? 2 : 1);
   const auto threads_for = [&](int cols) { return ((max((a.dv + cols - 1) / cols * a.parts, a.d) + WAVE - 1) / WAVE) * WAVE; };

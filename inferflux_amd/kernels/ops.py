@@ -1575,12 +1575,13 @@ RING_DEEP_STEPS = 48          # steps of 128 k-values from which a slice's own t
 
 @functools.lru_cache(maxsize=4096)
 def ring_plan(M: int, N: int, K: int, tile_rows: int, one_slice: bool, row_tiles: int = 0, slices: int = 0) -> Tuple[int, int]:
-    """(row tiles to a workgroup, steps of 128 k-values to a slice): about one workgroup to each of the 256 compute units.  Weights that
-    are cut into slices of K take two row tiles where K is short (896 x 4,864 at 64 rows 7.3 us, 8.0 with eight) and, where it is
-    deep, four up to 32 rows and eight beyond, whose x is read half as often (3,584 x 18,944 30.1 :
-    28.3, but at 17 rows 24.1 : 25.3).  Of up to 128 tiles of 16 rows (or pairs of 8, which the kernel joins) K is cut into four, or more where that leaves compute units
-    without a workgroup; a workgroup takes one tile, two where K is deep or there are 96 tiles and 17 rows (us by one, two and four tiles: 1,024 x 4,224 at 16 rows 4.3, 4.9,
-    6.3, 2,048 x 4,096 at 32 6.8, 6.3, 6.8, 1,536 x 8,960 at 16 9.0, 7.5, 8.4, at 64 13.0, 10.3, and 10.1 with twice the partial sums to read)."""
+    """(row tiles to a workgroup, steps of 128 k-values to a slice): about one workgroup to each of the 256 compute units.
+
+    Weights that are cut into slices of K: of up to 128 tiles of 16 rows (or pairs of 8, which the kernel joins: up to 2,048 rows) K is cut into four, or more where that leaves compute
+    units without a workgroup; a workgroup takes one tile, two where K is deep or there are 96 tiles and 17 rows (us by one, two and four tiles: 1,024 x 4,224 at 16 rows 4.3, 4.9,
+    6.3, 2,048 x 4,096 at 32 6.8, 6.3, 6.8, 1,536 x 8,960 at 16 9.0, 7.5, 8.4, at 64 13.0, 10.3, and 10.1 with twice the partial sums to read).  Of more tiles a workgroup
+    takes two where K is short (us by one, two, four and eight: 2,560 x 2,048 at 17 rows 6.3, 5.2, 5.7, 6.8, at 64 8.5, 7.1, 7.4, 7.8) and, where it is deep,
+    four up to 32 rows and eight beyond, whose x is read half as often (3,584 x 18,944 at 17 rows 40.4, 25.2, 25.8, 26.8, at 64 52.9, 39.4, 32.6, 29.5)."""
     steps = -(-K // 128)
     if not one_slice and row_tiles <= 0 and slices <= 0 and -(-N // (16 if tile_rows == 8 else tile_rows)) <= 128:
         n_tiles, deep = -(-N // (16 if tile_rows == 8 else tile_rows)), steps >= RING_DEEP_STEPS
@@ -2171,7 +2172,8 @@ def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
 # ----------------------------------------------------------------------------------------
 DELTA_THREAD_CHANNELS = (4, 8, 16, 32, 64)  # key channels of a column of S a thread may hold
 DELTA_MAX_PADDED_DIM, DELTA_MAX_COLS, DELTA_THREADS = 256, 128, 256
-DELTA_DECODE_MAX_CHANNELS = 8               # ... at most this many in steps of single tokens (64 decoded rows at 16 heads of 64 x 128: 62.8 us with 8, 70.2 with 16)
+# ... at most this many in steps of single tokens that ``delta_step`` does not take (64 decoded rows, us with 4, 8 and 16: 16 heads of 64 x 128 in 32 bits 84.9, 51.0,
+DELTA_DECODE_MAX_CHANNELS = 8               # 58.5, 4 heads of 128 x 256 in bfloat16 110.7, 71.2, 79.6)
 
 
 def delta_padded_dim(d: int) -> int:
@@ -2614,7 +2616,8 @@ def time_mix_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
 # ----------------------------------------------------------------------------------------
 MEMORY_THREAD_CHANNELS = (4, 8, 16, 32)     # key channels of a column of S a thread may hold
 MEMORY_MAX_PADDED_DIM, MEMORY_THREADS = 512, 256
-MEMORY_DECODE_MAX_CHANNELS = 8              # ... at most this many in steps of single tokens (64 rows at 16 heads of 64 x 128: 25.6 us with 8, 27.2 with 16, 32.4 with 4)
+# ... at most this many in steps of single tokens whose heads are too large or too small for the kernel that takes a head whole (64 rows at 4 heads of 256 x 256: 69.0 us
+MEMORY_DECODE_MAX_CHANNELS = 8              # with 4, 47.4 with 8, 48.1 with 16)
 
 
 def matrix_memory_layout(d: int, dv: int, single_tokens: bool = False) -> Tuple[int, int, int]:
