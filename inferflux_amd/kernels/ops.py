@@ -1327,7 +1327,10 @@ def adds_into_stream(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
     but 2,560 x 9,728 22.3, 21.0, 23.5 : 22.8, 21.8, 22.4, 3,584 x 18,944 38.4, 41.8, 47.4 : 40.6, 41.3, 42.0, and at 8 rows all but one slower)."""
     if not _into_stream_takes(n_rows, weight, norm_weight):
         return False
-    return weight.rows.shape[0] > RING_FEW_STREAM_MAX_N or not _few_in_slices(n_rows, weight)
+    if n_rows < RING_FEW_MIN_ROWS or weight.tiled is None:
+        return True
+    N, K = weight.rows.shape
+    return N > RING_FEW_STREAM_MAX_N or not _few_in_slices(n_rows, N, K, weight.tile_rows)
 
 
 def _into_stream_takes(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
@@ -1629,11 +1632,10 @@ RING_FEW_MIN_SLICED_K = 4096
 RING_FEW_STREAM_MAX_N = 2048         # (see ``adds_into_stream``)
 
 
-def _few_in_slices(n_rows: int, weight: LinearWeight) -> bool:
-    """Whether ``n_rows`` rows times ``weight`` go to ``ring_gemm`` in slices of K where their reader adds the slices (see ``ring_takes_few``)."""
-    N, K = weight.rows.shape
-    return (RING_FEW_MIN_ROWS <= n_rows <= 16 and weight.tiled is not None and weight.rows.dtype == torch.bfloat16 and -(-N // weight.tile_rows) <= COMPUTE_UNITS
-            and RING_FEW_MIN_SLICED_K <= K < 1 << 20 and K % 8 == 0 and _small_m_kernel(n_rows, N, K, True) == "skinny")
+def _few_in_slices(n_rows: int, N: int, K: int, tile_rows: int) -> bool:
+    """Whether so many rows times a weight that would go to the product whose waves split K go to ``ring_gemm`` in slices of K instead, where their reader adds
+    the slices (see ``ring_takes_few``; ``adds_into_stream`` asks for every product of a step, so this is a few comparisons)."""
+    return RING_FEW_MIN_ROWS <= n_rows <= 16 and -(-N // tile_rows) <= COMPUTE_UNITS and RING_FEW_MIN_SLICED_K <= K < 1 << 20
 
 
 def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
@@ -1651,7 +1653,7 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
     (M, K), N = x.shape, weight.rows.shape[0]
     if not RING_FEW_MIN_ROWS <= M <= 16 or K % 8 or K != weight.rows.shape[1] or _small_m_kernel(M, N, K, True) != "skinny":
         return 0
-    if keep_slices and _few_in_slices(M, weight):
+    if keep_slices and _few_in_slices(M, N, K, weight.tile_rows):
         return 2
     tiles = -(-N // weight.tile_rows)
     return 1 if 2048 < N and tiles <= 3 * COMPUTE_UNITS and K <= RING_FEW_MIN_SLICED_K else 0
@@ -1659,6 +1661,8 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
 
 def leaves_few_rows_in_sums(x, weight) -> bool:
     """Whether ``linear`` with ``keep_slices`` leaves these up to 16 rows times ``weight`` as partial sums in float."""
+    if x.shape[0] < 8:              # (neither of the two kernels that cut K takes fewer)
+        return False
     N, K = weight.rows.shape
     return ring_takes_few(x, weight, True) == 2 or (weight.tiled is not None and N < WIDE_FEW_ROWS_MIN_N and _small_m_kernel(x.shape[0], N, K, True) == "wide")
 
