@@ -388,11 +388,12 @@ def paged_attention(q: torch.Tensor, cache, ctx, window: Optional[int], scale: f
         qt, splits, chunk = 1, 1, 0
         two = beside = False
         if tiled.any():
-            qt, splits, chunk = choose_tiling(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, lambda t: ops.attention_tile_rows(d, t),
+            # (Python's numbers: a step that is run launch by launch waits for this, and numpy's take three times as long one by one)
+            rows, keys = ctx.h_q_len[tiled].tolist(), ctx.h_kv_len[tiled].tolist()
+            qt, splits, chunk = choose_tiling(rows, keys, nH, lambda t: ops.attention_tile_rows(d, t),
                                               tall_direct=d == ops.DIRECT_TILE_HEAD_DIM and not keep_first and not block)
-            row_req = np.nonzero(~tiled & (ctx.h_q_len > 0))[0]
-            two, beside = choose_groups(ctx.h_q_len[tiled], ctx.h_kv_len[tiled], nH, ctx.h_kv_len[row_req], int(ctx.h_q_len[row_req].sum()) * n_kv,
-                                        window, splits, not keep_first)
+            others = [(n, k) for n, k in zip(ctx.h_q_len.tolist(), ctx.h_kv_len.tolist()) if 0 < n < TILE_MIN] if len(rows) < tiled.size else []
+            two, beside = choose_groups(rows, keys, nH, [k for _, k in others], sum(n for n, _ in others) * n_kv, window, splits, not keep_first)
             if two:
                 qt, splits, chunk = 1, 1, 0
         tile_rows = ops.attention_tile_rows(d, qt)
