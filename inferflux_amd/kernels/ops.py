@@ -1318,16 +1318,18 @@ def takes_scaled_rows(n_rows: int, weight) -> bool:
             and _small_m_kernel(n_rows, N, K, weight.tiled is not None) in ("skinny", "wide"))
 
 
-def adds_into_stream(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
+def adds_into_stream(n_rows: int, weight, norm_weight: torch.Tensor, single_tokens: bool = True) -> bool:
     """Whether a product of this shape is best added to the stream by ``linear_into_stream``, which takes it then.
 
     Where 9 to 16 rows times a deep weight of up to 2,048 rows go to the ring in slices of K, they and the norm that adds the slices are faster (us of down and the
     product behind it, into the stream : slices and norm, at 9, 12 and 16 rows: 896 x 4,864 12.0, 13.1, 14.1 : 11.1,
     11.6, 11.8, 1,024 x 4,224 12.1, 13.1, 13.9 : 11.4, 11.5, 11.8, 1,536 x 8,960 17.3, 18.1, 19.3 : 15.6, 16.0, 16.0, 2,048 x 11,008 33.5, 34.8, 34.4 : 30.6, 30.9, 30.4;
-    but 2,560 x 9,728 22.3, 21.0, 23.5 : 22.8, 21.8, 22.4, 3,584 x 18,944 38.4, 41.8, 47.4 : 40.6, 41.3, 42.0, and at 8 rows all but one slower)."""
+    but 2,560 x 9,728 22.3, 21.0, 23.5 : 22.8, 21.8, 22.4, 3,584 x 18,944 38.4, 41.8, 47.4 : 40.6, 41.3, 42.0, and at 8 rows all but one slower).  So in steps of single tokens, which
+    graphs replay (ms for 48 tokens of 16 requests at the 0.5B, 1.5B and 3B shapes 42.0, 68.9, 102.7 : 39.7, 65.3, 97.6); a prompt's step is run launch by launch and waits for the
+    host, to whom the norm and the sums are a launch and an allocation more a layer (12 tokens 1.48, 1.72, 2.20 : 1.70, 2.00, 2.53)."""
     if not _into_stream_takes(n_rows, weight, norm_weight):
         return False
-    if n_rows < RING_FEW_MIN_ROWS or weight.tiled is None:
+    if n_rows < RING_FEW_MIN_ROWS or weight.tiled is None or not single_tokens:
         return True
     N, K = weight.rows.shape
     return N > RING_FEW_STREAM_MAX_N or not _few_in_slices(n_rows, N, K, weight.tile_rows)

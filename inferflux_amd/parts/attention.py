@@ -209,7 +209,7 @@ class PagedAttention(Mixer):
         return not self.position.needs_apply and ops.takes_scaled_rows(n_rows, self.w_qkv)
 
     def _project_out(self, out, sink):
-        if sink is not None and ops.adds_into_stream(out.shape[0], self.w_o, sink.norm_weight):
+        if sink is not None and ops.adds_into_stream(out.shape[0], self.w_o, sink.norm_weight, sink.single_tokens):
             return ops.linear_into_stream(out, self.w_o, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(out, self.w_o, keep_slices=sink is not None)   # an RMS norm's kernel adds partial sums itself
 

@@ -138,12 +138,14 @@ class MixerBinding:
 class StreamSink:
     """Where a mixer or feed-forward may add its result itself: the float32 stream, and the weight and eps
     of the RMS norm that reads the stream next.  ``mult`` is the factor on what is added (a model's factor on every
-    sub-block's output; 1 otherwise).  Without a stream and a norm (both None) nothing may be added, but the reader takes a
+    sub-block's output; 1 otherwise).  ``single_tokens``: every request of the step brings one row, as in steps that captured graphs
+    replay (see ``ops.adds_into_stream``).  Without a stream and a norm (both None) nothing may be added, but the reader takes a
     product left as partial sums (``SliceSums``) and adds them up itself."""
     stream: Optional[torch.Tensor]
     norm_weight: Optional[torch.Tensor]
     eps: float
     mult: float = 1.0
+    single_tokens: bool = True
 
 
 class Mixer(Part):

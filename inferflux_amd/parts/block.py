@@ -58,11 +58,11 @@ def normed_for(norm, reader, residual, pending, ctx):
     return norm.forward(residual, pending, ctx.act_dtype)
 
 
-def _sink(part, residual, norm, mult=1.0):
+def _sink(part, residual, norm, ctx, mult=1.0):
     if norm is None or not getattr(part, "adds_to_stream", False):
         return None
     params = norm.rms_params()
-    return StreamSink(residual, *params, mult) if params is not None else None
+    return StreamSink(residual, *params, mult, ctx.n_tokens == ctx.n_requests) if params is not None else None
 
 
 @register_part("block", "prenorm")
@@ -92,12 +92,12 @@ class PreNormBlock(Block):
         return ScaledDelta(delta, self.residual_scale)
 
     def _mixer(self, h, ctx, binding, residual, following):
-        sink = _sink(self.mixer, residual, self.norm_post if self.ffn is not None else following, self.residual_scale)
+        sink = _sink(self.mixer, residual, self.norm_post if self.ffn is not None else following, ctx, self.residual_scale)
         out = self.mixer.forward(h, ctx, binding, sink=sink) if sink is not None else self.mixer.forward(h, ctx, binding)
         return self._scaled(out)
 
     def _ffn(self, h, ctx, residual, following):
-        sink = _sink(self.ffn, residual, following, self.residual_scale)
+        sink = _sink(self.ffn, residual, following, ctx, self.residual_scale)
         return self._scaled(self.ffn.forward(h, ctx, sink=sink) if sink is not None else self.ffn.forward(h, ctx))
 
     def forward(self, residual, pending, ctx, binding: MixerBinding, following=None):
@@ -159,7 +159,7 @@ class ParallelBlock(Block):
     def forward(self, residual, pending, ctx, binding: MixerBinding, following=None):
         t = ctx.timer
         params = following.rms_params() if following is not None else None
-        sink = StreamSink(residual, *params) if params is not None else _PARTIAL_SUMS_WELCOME
+        sink = StreamSink(residual, *params, single_tokens=ctx.n_tokens == ctx.n_requests) if params is not None else _PARTIAL_SUMS_WELCOME
         if t is not None:
             t.enter("norm")
         h = normed_for(self.norm_in, self._readers, residual, pending, ctx)

@@ -80,7 +80,7 @@ class SwiGLU(FeedForward):
         a = ops.linear_swiglu(h, self.w_gate_up, self.act, self.limit)
         if ctx.timer is not None:
             ctx.timer.mark("ffn.gate_up")
-        if sink is not None and ops.adds_into_stream(a.shape[0], self.w_down, sink.norm_weight):
+        if sink is not None and ops.adds_into_stream(a.shape[0], self.w_down, sink.norm_weight, sink.single_tokens):
             return ops.linear_into_stream(a, self.w_down, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(a, self.w_down, keep_slices=sink is not None)   # an RMS norm's kernel adds partial sums itself
 
@@ -118,6 +118,6 @@ class DenseFFN(FeedForward):
         a = ops.linear_act(h, self.w_up, self.act)
         if ctx.timer is not None:
             ctx.timer.mark("ffn.up")
-        if sink is not None and ops.adds_into_stream(a.shape[0], self.w_down, sink.norm_weight):
+        if sink is not None and ops.adds_into_stream(a.shape[0], self.w_down, sink.norm_weight, sink.single_tokens):
             return ops.linear_into_stream(a, self.w_down, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(a, self.w_down, keep_slices=sink is not None)

@@ -208,7 +208,7 @@ class LatentAttention(Mixer):
                          gate=(y, y.shape[1] - self.gate_rows) if self.output_gate else None)    # [T, heads, vdim]
         v = v.view(T, nh * self.v_dim)
         v = v if v.dtype == dtype else v.to(dtype)
-        if sink is not None and ops.adds_into_stream(T, self.w_o, sink.norm_weight):
+        if sink is not None and ops.adds_into_stream(T, self.w_o, sink.norm_weight, sink.single_tokens):
             return ops.linear_into_stream(v, self.w_o, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(v, self.w_o, keep_slices=True)
 

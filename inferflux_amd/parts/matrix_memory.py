@@ -105,6 +105,6 @@ class MatrixMemory(Mixer):
                               ctx.state_slots, ctx.row_req, dtype, single_tokens=ctx.n_tokens == ctx.n_requests, chunks=chunks)
         if t is not None:
             t.mark("mixer.scan")
-        if sink is not None and ops.adds_into_stream(y.shape[0], self.w_o, sink.norm_weight):
+        if sink is not None and ops.adds_into_stream(y.shape[0], self.w_o, sink.norm_weight, sink.single_tokens):
             return ops.linear_into_stream(y, self.w_o, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(y, self.w_o, keep_slices=sink is not None)

@@ -115,6 +115,6 @@ class SelectiveSSM(Mixer):
                                ctx.q_start, ctx.q_len, ctx.state_slots, chunks)
         if t is not None:
             t.mark("mixer.scan")
-        if sink is not None and ops.adds_into_stream(y.shape[0], self.w_o, sink.norm_weight):
+        if sink is not None and ops.adds_into_stream(y.shape[0], self.w_o, sink.norm_weight, sink.single_tokens):
             return ops.linear_into_stream(y, self.w_o, sink.stream, sink.norm_weight, sink.eps, sink.mult)
         return ops.linear(y, self.w_o, keep_slices=sink is not None)

@@ -1119,3 +1119,30 @@ def test_a_shrinking_batch_replays_few_layouts(dtype, sharp_folders):
     assert graphed.manager.free_pages() == eager.manager.free_pages() == [40, 40]
     # the scratch page lies beyond every pool: no block table ever names it
     assert graphed.storage.scratch_pages == [40, 40] and graphed.storage.binding(0).cache.k.shape[0] == 41
+
+
+def test_9_to_16_rows_of_deep_weights_in_prompts_and_in_decoding(tmp_path, monkeypatch):
+    """A down projection of 4,096 k-values: its slices are left to the norm in steps of nine single tokens, eager and captured, and it adds into the
+    stream in a prompt of nine, whose launches the host is the one to wait for; either against the plain model."""
+    from inferflux_amd.config import config_from_dict
+    from inferflux_amd.kernels import ops
+    from inferflux_amd.weights import write_random_model
+    cfg = dict(TINY["A"], intermediate_size=4096)
+    write_random_model(str(tmp_path), config_from_dict(cfg), seed=31, dtype=torch.bfloat16)
+    added, sliced = [], []              # rows of the products of 4,096 k-values by either way
+    into, ring = ops.linear_into_stream, ops.ring_gemm
+    monkeypatch.setattr(ops, "linear_into_stream", lambda x, w, *a: (added.append(x.shape[0]) if w.shape[1] == 4096 else None, into(x, w, *a))[1])
+    monkeypatch.setattr(ops, "ring_gemm", lambda x, w, *a, **k: (sliced.append(x.shape[0]) if w.shape[1] == 4096 else None, ring(x, w, *a, **k))[1])
+    runner = load_runner(str(tmp_path), torch.bfloat16, num_pages=64, max_requests=16)
+    seqs = [seeded_ids(700 + i, 12, cfg["vocab_size"]) for i in range(9)]
+    first = []
+    for i, ids in enumerate(seqs):
+        runner.add_request(i)
+        first.append(runner.step([StepEntry(i, ids[:9], [8])]).float().cpu()[0])
+    assert set(added) == {9} and not sliced
+    added.clear()
+    got = [runner.step([StepEntry(i, [ids[9 + k]], [0]) for i, ids in enumerate(seqs)]).float().cpu().clone() for k in range(3)]
+    assert sliced and min(sliced) >= 9 and not added and runner.graph_replays >= 1      # (batches are filled up)
+    for i, ids in enumerate(seqs):
+        want = plain_logits(str(tmp_path), ids)
+        assert rel_err(torch.stack([first[i]] + [g[i] for g in got]), want[8:12]) < tol("bfloat16", "A"), i
