@@ -596,11 +596,14 @@ def normed_columns_take(n_rows: int, weight, rank: int) -> bool:
 def linear_normed(x, weight: LinearWeight, column_scale: torch.Tensor, rank: int, eps: float):
     """x [M <= 16, K] (a tensor or ``ScaledRows``) times ``weight`` [N, K] transposed, times ``column_scale`` [N], as bfloat16 [M, N], and its first
     ``rank`` columns as ``ScaledRows``: the rows of an RMS norm over them (whose weight the scale's first ``rank`` numbers are) up to the factor."""
-    if not linear_normed_takes(x, weight, rank):
+    N, K = weight.shape
+    if (not isinstance(weight, LinearWeight) or weight.order is not None or weight.tiled is None or x.shape[0] > 16 or N % 8 or K % 8 or not 0 < rank <= N
+            or rank % weight.tile_rows):
         raise KernelError(f"linear_normed: not for {x.shape[0]} rows times a {tuple(weight.rows.shape)} weight and a norm over {rank} columns")
     x, scale = _scale_args(x)
-    _check(x, "x", (None, weight.rows.shape[1]), torch.bfloat16)
-    (M, K), N = x.shape, weight.rows.shape[0]
+    M = x.shape[0]
+    _check(x, "x", (M, K), torch.bfloat16)
+    _check(weight.rows, "weight", (N, K), torch.bfloat16)
     _check(column_scale, "column_scale", (N,))
     y = empty((M, N), torch.bfloat16, x)
     pieces = empty((-(-N // weight.tile_rows), 16), torch.float32, x)
@@ -1649,6 +1652,8 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
         slices, a row tile for a compute unit at most and 4,096 k-values or more: 2,048 x 8,448 12.9, 14.4 : 9.0, 8.7     1,024 x 4,224 7.2, 8.6 : 4.2, 4.3
             2,048 x 5,632 9.7, 10.9 : 8.1, 8.2     1,536 x 8,960 12.3, 13.7 : 7.5, 7.6     3,584 x 18,944 26.2, 32.8 : 24.5, 24.2, but 2,048 x 2,048 5.4, 5.8 :
             4.5, 4.5 and a sum for the reader to form."""
+    if x.shape[0] < RING_FEW_MIN_ROWS:              # (most steps that ask)
+        return 0
     if not isinstance(weight, LinearWeight) or isinstance(x, ScaledRows) or weight.tiled is None or weight.rows.dtype != torch.bfloat16 \
             or x.dtype != torch.bfloat16 or not x.is_contiguous() or x.data_ptr() % 16:
         return 0
@@ -1783,7 +1788,7 @@ def linear(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, kee
         if plan and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and weight.is_contiguous():
             return _by_plan(x, weight, plan, keep_slices)
     if kind == "skinny":
-        ring = ring_takes_few(x, LinearWeight(weight, tiled, order, tile_rows), keep_slices and out_dtype == torch.bfloat16)
+        ring = M >= RING_FEW_MIN_ROWS and ring_takes_few(x, LinearWeight(weight, tiled, order, tile_rows), keep_slices and out_dtype == torch.bfloat16)
         if ring:
             return ring_gemm(x, LinearWeight(weight, tiled, order, tile_rows), out_dtype, slices=0 if ring == 2 else 1, keep_slices=True)
         return skinny_gemm(x, weight, out_dtype, tiled=tiled, order=order, tile_rows=tile_rows)

@@ -183,9 +183,10 @@ class LatentAttention(Mixer):
                 and not ops.leaves_few_rows_in_sums(h, self.w_down)):
             y = ops.linear(h, self.w_few)
             q, latent = y[:, :heads_w], y[:, heads_w:]
-        elif (self.few_scale is not None and h.dtype == cache.k.dtype and ops.linear_normed_takes(h, self.w_down, rank)
+        elif (self.few_scale is not None and ctx.n_tokens == ctx.n_requests and h.dtype == cache.k.dtype and ops.linear_normed_takes(h, self.w_down, rank)
                 and ops.normed_columns_take(T, self.w_uq, rank)
                 and (self.shared_latent or ops.latent_query_takes(T, h.dtype, self.dim, self.rot_dim, self.kv_rank))):
+            # (single tokens, which graphs replay: a prompt of few tokens waits for the host, and what is cut out of y costs it more than the launch)
             y, cq = ops.linear_normed(h, self.w_down, self.few_scale, rank, self.eps)
             q, latent = ops.linear(cq, self.w_uq), y[:, rank:rank + self.kv_rank + self.rot_dim]
         else:

@@ -21,8 +21,8 @@ def tiled(rows):
     return ops.LinearWeight(rows, torch.empty(0, dtype=rows.dtype), None, ops.choose_tile_rows(rows.shape[0]))
 
 
-def route(monkeypatch, hidden, rows, q_rank, gate):
-    """("joined" | "normed" | "apart", whether partial sums are taken) of a step of ``rows`` plain rows."""
+def route(monkeypatch, hidden, rows, q_rank, gate, requests):
+    """("joined" | "normed" | "apart", whether partial sums are taken) of a step of ``rows`` plain rows of ``requests`` requests."""
     a = LatentAttention("a", hidden, 8, 64, 32, 64, q_rank, 96, 0.1, 1e-5, PartSpec("none"), output_gate=gate)
     zeros = lambda *shape: torch.zeros(shape, dtype=BF16)
     a.load({n: zeros(*s.shape) for n, s in a.param_specs().items()})
@@ -41,7 +41,7 @@ def route(monkeypatch, hidden, rows, q_rank, gate):
     monkeypatch.setattr(ops, "linear", linear)
     monkeypatch.setattr(ops, "linear_normed", normed)
     cache = types.SimpleNamespace(group=0, k=zeros(1, 1, 16, 128))
-    ctx = types.SimpleNamespace(timer=None, write_slots=lambda group: None)
+    ctx = types.SimpleNamespace(timer=None, write_slots=lambda group: None, n_tokens=rows, n_requests=requests)
     with pytest.raises(Asked) as asked:
         a.forward(zeros(rows, hidden), ctx, types.SimpleNamespace(cache=cache, writes_cache=True))
     return asked.value.args
@@ -53,10 +53,10 @@ def route(monkeypatch, hidden, rows, q_rank, gate):
 def test_down_products_whose_sums_stayed_in_float_still_do(monkeypatch, hidden, q_rank, gate, rows):
     """9 to 16 plain rows times a deep down projection go to the ring in slices of K, whose float sums the latent's norm, the rotation and the
     output gate's sigmoid read: neither of the joined products, which write bfloat16, may take them away."""
-    way, sums = route(monkeypatch, hidden, rows, q_rank, gate)
     deep = rows >= 9 and hidden >= 4096
-    assert sums == deep
-    assert way == ("apart" if deep else "normed" if q_rank else "joined")
+    assert route(monkeypatch, hidden, rows, q_rank, gate, rows) == ("apart" if deep else "normed" if q_rank else "joined", deep)
+    if rows > 1:         # a prompt
+        assert route(monkeypatch, hidden, rows, q_rank, gate, 1) == ("apart" if deep or q_rank else "joined", deep)
 
 
 @pytest.mark.parametrize("N,K", [(8, 4096), (2048, 4096), (2048, 4088), (2048, 4104), (2052, 4096), (896, 4864), (8, 1 << 20), (16, (1 << 20) - 8), (64, 4100)])
