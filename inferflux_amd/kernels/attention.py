@@ -45,7 +45,8 @@ TILE_MAX_SPLITS = 16
 TILE_ORDER_MIN_ITEMS = 64       # launches of more workgroups than this get them in tile_order
 TILE_GROUPS_MAX = 256       # at most this many workgroups of 64-row tiles, one for each compute unit: two groups of waves to a workgroup,
 TILE_GROUPS_KEYS = 1024     # while no workgroup walks more keys than this
-TILE_GROUPS_KEYS_BESIDE = 1536      # ... or than this with the step's other rows in the same launch (see choose_groups)
+TILE_GROUPS_KEYS_BESIDE = 1536      # ... or than this with the step's other rows in the same launch (see choose_groups),
+TILE_GROUPS_FEW, TILE_GROUPS_KEYS_FEW = 48, 1152      # of fewer workgroups than these no more than so many keys
 ROW_CHUNK = 64      # keys per split of the row kernel: doubled while the launch keeps ROW_MIN_WAVES (ROW_MIN_WAVES_128
 ROW_MIN_WAVES_128 = 1000   # for the step from 64 to 128) waves or more: a split costs a fixed start-up, so longer splits
 ROW_MIN_WAVES = 1536       # pay when there are waves enough; and until a row has at most ROW_MAX_SPLITS splits.  The merge
@@ -141,10 +142,13 @@ def choose_groups(tiled_rows, tiled_keys, n_heads: int, row_keys, pairs: int, wi
     The other rows beside them cost little while they end no later than the tiles, against 10 to 13 us of their own launches: a row's walk takes some
     4.5 us and 11 for 1,000 keys, a tile's 5 and 19.5.  us with launches of their own / beside, 16 heads of 128 on 2: 500 rows and 23 rows of up to 299 keys
     28.7 / 15.6, 20 of up to 992 30.5 / 18.6, 512 after 1,500 and 20 of 981 58 / 44, 128 rows and 6 of 369 17.5 / 9.7, but 4 of 1,900 18.0 / 25.6; more
-    workgroups than compute units, 28 heads on 4, 500 rows and 23 of 283 31.9 / 17.6; 2 prompts of 512, 16 heads, and 4 rows of 1,933 25.6 / 31.6."""
+    workgroups than compute units, 28 heads on 4, 500 rows and 23 of 283 31.9 / 17.6; 2 prompts of 512, 16 heads, and 4 rows of 1,933 25.6 / 31.6.
+    Few tiles with long walks are better cut into splits, which many workgroups share, whatever rows are beside them: us in splits and with launches of their own /
+    beside, 12 workgroups of 128 and 1,193 keys 25.2 / 28.1, 16 and 1,463 27.2 / 32.9, 28 and 1,518 28.5 / 34.1, 36 and 1,413 31.5 / 33.4, but 12 and 1,142 27.2 / 26.8,
+    48 and 1,317 32.0 / 31.7, 80 and 1,500 42.4 / 34.9, 196 and 1,512 44.0 / 36.1."""
     blocks = sum(-(-int(n) // 64) for n in tiled_rows) * n_heads
     walk = int(max(tiled_keys)) if window is None else min(int(max(tiled_keys)), window + 64)
-    if blocks > TILE_GROUPS_MAX or walk > TILE_GROUPS_KEYS_BESIDE:
+    if blocks > TILE_GROUPS_MAX or walk > (TILE_GROUPS_KEYS_BESIDE if blocks >= TILE_GROUPS_FEW else TILE_GROUPS_KEYS_FEW):
         return False, False
     if pairs and beside_fits and pairs <= TILE_GROUPS_MAX:
         row_walk = int(max(row_keys)) if window is None else min(int(max(row_keys)), window)

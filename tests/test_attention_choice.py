@@ -288,3 +288,10 @@ def test_two_groups_of_waves_and_rows_beside_the_tiles_where_both_were_measured(
     for rows, keys, heads, row_keys, pairs, window, splits, want in cases:
         assert choose_groups(rows, keys, heads, row_keys, pairs, window, splits) == want, (rows, keys, heads, row_keys, pairs, window)
         assert not choose_groups(rows, keys, heads, row_keys, pairs, window, splits, beside_fits=False)[1]
+
+
+def test_few_tiles_with_long_walks_keep_their_splits_whatever_is_beside_them():
+    for heads, rows, keys, want in ((16, 25, 1152, (True, True)), (16, 25, 1153, (False, False)), (28, 31, 1518, (False, False)), (12, 156, 1413, (False, False)),
+                                    (12, 200, 1536, (True, True)), (16, 130, 1500, (True, True)), (16, 130, 1537, (False, False))):
+        assert choose_groups([rows], [keys], heads, [11], 2, None, 3) == want, (heads, rows, keys)
+    assert choose_groups([25], [3000], 16, [11], 2, 1024, 3) == (True, True)           # (a window of 1,024: 1,088 keys)
