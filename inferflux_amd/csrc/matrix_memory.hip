@@ -182,6 +182,9 @@ __global__ __launch_bounds__(256) void memory_finish_kernel(MemoryArgs a) {
 // is the first such threads' own.  q, k, v and the gates are formed once and meet in LDS; every load goes out before any is used, without branches
 // between them, so that what meets there is waited for while S is on its way.  16 heads of 64 x 128, us with 16 channels of one column to a thread / 4
 // columns / 8 columns, at 1, 16, 24, 32, 48 requests: 5.0 / 4.9, 7.3 / 7.3, 11.0 / 8.8, 12.0 / 9.7, 16.8 / 13.6, and at 64 22.3 / 18.1 / 16.9 (67 MB of S).
+// A small head's columns are short waits one after the other, and two to a thread end sooner: us by four / two, 16 x 32 of 8 (request, head) pairs 4.7 / 4.3, of 16 x 128 and
+// 160 5.4 / 5.1, 32 x 128 and 96 5.6 / 5.1, 32 x 32 and 896 (by eight) 6.9 / 5.5, 64 x 64 and 16 5.3 / 4.7, 128 x 32 and 160 6.0 / 5.3, but 64 x 128 and 64 5.4 / 5.6, and 656 12.9 / 16.5.
+#define STEP_SMALL_HEAD 4096     // numbers of S up to which a thread takes two columns
 #define STEP_MANY_HEADS 768      // (request, head) pairs beyond which eight columns, in four waves, are the better choice
 template <typename TI, typename TO, int V, int COLS>
 __global__ __launch_bounds__(1024) void memory_step_kernel(MemoryArgs a) {
@@ -629,7 +632,8 @@ extern "C" int ifx_matrix_memory(const void* rows, int dtype, int ld, int q_col,
   const int dpad = ch * ks, runs = dpad > 4 * WAVE ? 2 : 1, lanes = dpad / 4 / runs;
   const auto threads_of = [&](int cols_) { return (lanes * ((dv + cols_ - 1) / cols_) + WAVE - 1) / WAVE * WAVE; };
   const bool four = runs > 1 || (threads_of(4) <= 1024 && (long long)H * R <= STEP_MANY_HEADS) || threads_of(8) > 1024;
-  const int step_threads = threads_of(four ? 4 : 8);
+  const bool two = runs == 1 && dpad * dv <= STEP_SMALL_HEAD;
+  const int step_threads = threads_of(two ? 2 : four ? 4 : 8);
   if (T <= R && lanes >= 4 && lanes <= WAVE && step_threads <= 1024) {
     a.KS = lanes;
     const size_t step_lds = (size_t)(2 * dpad + dv + 1) * sizeof(float);
@@ -637,6 +641,7 @@ extern "C" int ifx_matrix_memory(const void* rows, int dtype, int ld, int q_col,
 #define STEP(TI, TO)                                                                                                             \
   do {                                                                                                                           \
     if (runs > 1) hipLaunchKernelGGL((memory_step_kernel<TI, TO, 2, 4>), step_grid, dim3(step_threads), step_lds, s, a);         \
+    else if (two) hipLaunchKernelGGL((memory_step_kernel<TI, TO, 1, 2>), step_grid, dim3(step_threads), step_lds, s, a);         \
     else if (four) hipLaunchKernelGGL((memory_step_kernel<TI, TO, 1, 4>), step_grid, dim3(step_threads), step_lds, s, a);        \
     else hipLaunchKernelGGL((memory_step_kernel<TI, TO, 1, 8>), step_grid, dim3(step_threads), step_lds, s, a);                  \
   } while (0)

@@ -422,6 +422,13 @@ def test_single_tokens_of_the_memory_against_the_walk(dtype, H, d, dv):
     assert rel_err(states[0], states[1]) < 2e-6
 
 
+@pytest.mark.parametrize("H,d,dv", [(3, 64, 64), (3, 64, 65), (2, 16, 256), (2, 9, 257), (1, 256, 16), (1, 256, 17), (5, 32, 7)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float32 to bfloat16"])
+def test_single_tokens_of_small_heads_of_the_memory_against_the_walk(dtype, H, d, dv):
+    """As above, on both sides of the heads whose threads take two columns (4,096 numbers of S)."""
+    test_single_tokens_of_the_memory_against_the_walk(dtype, H, d, dv)
+
+
 @pytest.mark.parametrize("R,H,d,dv", [(769, 1, 16, 1), (385, 2, 10, 63), (193, 4, 64, 128), (769, 1, 64, 130), (193, 4, 256, 128), (193, 4, 256, 129), (385, 2, 8, 40)])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float32 to bfloat16"])
 def test_single_tokens_of_many_heads_of_the_memory_against_the_walk(dtype, R, H, d, dv):
