@@ -263,12 +263,20 @@ __global__ __launch_bounds__(256) void headwise_kernel(HeadwiseArgs a) {
 // The same for steps of few rows: a thread owns one output element of one (row, head) and reads its weight row in
 // 16-byte pieces, all asked for at once (a wave's rows are one contiguous run of memory); no LDS, no barrier.  The sum
 // runs over k in the tiled kernel's order, so both give the same bits.
-__device__ __forceinline__ void hw_load8(const bf16_t* p, float* v) {
-  typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-  const bf16x8 t = *(const bf16x8*)p;
+// The row of x, the same for all threads, is read through the constant address space: scalar loads, which no vector load waits for.  Where workgroups beside these write
+// (latent_query_kernel) the compiler read it by vector loads otherwise, each of which waited for itself and for the weights asked for before it.
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 hw_bf16x8;
+#define HW_CONSTANT __attribute__((address_space(4)))
+__device__ __forceinline__ void hw_widen(hw_bf16x8 t, float* v) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = (float)t[i];
 }
+__device__ __forceinline__ void hw_load8(const HW_CONSTANT bf16_t* p, float* v) { hw_widen(*(const HW_CONSTANT hw_bf16x8*)p, v); }
+__device__ __forceinline__ void hw_load8(const HW_CONSTANT float* p, float* v) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = p[i];
+}
+__device__ __forceinline__ void hw_load8(const bf16_t* p, float* v) { hw_widen(*(const hw_bf16x8*)p, v); }
 __device__ __forceinline__ void hw_load8(const float* p, float* v) {
   const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
   v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
@@ -281,11 +289,12 @@ __device__ __forceinline__ void headwise_row(const HeadwiseArgs& a, int t, int h
   T* out = (T*)a.out + ((size_t)t * a.H + h) * out_head;
   if (n < a.N) {
     const T* w = (const T*)a.w + ((size_t)h * a.N + n) * a.K;
+    const HW_CONSTANT T* xc = (const HW_CONSTANT T*)xt;
     float acc = 0.f;
 #pragma unroll 4
     for (int k = 0; k < a.K; k += 8) {
       float xv[8], wv[8];
-      hw_load8(xt + k, xv);
+      hw_load8(xc + k, xv);
       hw_load8(w + k, wv);
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc = fmaf(xv[i], wv[i], acc);
@@ -310,7 +319,8 @@ __global__ __launch_bounds__(256) void headwise_rows_kernel(HeadwiseArgs a) {
 }
 
 // The queries' side of a step and the cache's, which do not need each other: workgroups (row, head) for the product, and one a row
-// behind them for ``finish_row``.  Bound by the launch and a chain of two trips: one row of 16 heads 4.0 us, apart 4.6 and 4.6.
+// behind them for ``finish_row``.  Bound by the launch and a chain of two trips, or W_uk: us in one launch / two, 4 rows of 32 heads of 96 x 512 5.2 / 4.2 + 3.6, 8 rows
+// 6.7 / 6.2 + 3.7, of 96 x 96 4.0 / 3.7 + 3.3, 8 rows of 64 heads of 128 x 512 13.7 / 13.3 + 4.1.
 template <int LF_EACH>
 __global__ __launch_bounds__(256) void latent_query_kernel(HeadwiseArgs a, FinishArgs<bf16_t, bf16_t> f) {
   __shared__ float red[32];
@@ -371,7 +381,7 @@ extern "C" int ifx_headwise(const void* x, const void* w, void* out, int dtype, 
   IFX_REQUIRE(!tail_only || tail > 0, "headwise: tail_only without a tail");
   a.tile0 = tail_only ? (N + HW_TN - 1) / HW_TN : 0;
   hipStream_t s = (hipStream_t)stream;
-  if (!tail_only && T <= HW_ROWS_MAX_T && K % 8 == 0 && x_row % 8 == 0 && x_head % 8 == 0) {
+  if (!tail_only && T <= HW_ROWS_MAX_T && K % 8 == 0 && x_row % 8 == 0 && x_head % 8 == 0 && (uintptr_t)x % 4 == 0) {      // (scalar loads: on 4 bytes)
     const dim3 grid(T, H, (N + tail + 255) / 256);
     if (dtype == DT_F32) hipLaunchKernelGGL(headwise_rows_kernel<float>, grid, dim3(256), 0, s, a);
     else if (dtype == DT_BF16) hipLaunchKernelGGL(headwise_rows_kernel<bf16_t>, grid, dim3(256), 0, s, a);

@@ -249,6 +249,16 @@ def test_headwise_product_on_the_matrix_cores(T, H, K, N, tail, rot):
     assert torch.equal(got[..., N:], few[..., N:])
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_rows_of_heads_that_do_not_lie_on_4_bytes(dtype):
+    """The bits of the same rows where they start on 16 bytes (in bfloat16 two bytes behind them, where the kernel of few rows does not read)."""
+    dt = DT[dtype]
+    flat, w = rnd(47, 1 + 5 * 3 * 24).to(dt).to(DEV), rnd(48, 3, 40, 24).to(dt).to(DEV)
+    x = flat[1:].view(5, 72)
+    assert x.data_ptr() % 16 != 0
+    assert torch.equal(ops.headwise(x, w, 3, 24), ops.headwise(x.clone(), w, 3, 24))
+
+
 def split_rows(seed, T, H, splits, D, sinks=False):
     """Partial results of attention's splits as the row kernel leaves them, and what they join to in 64 bits.  Splits that saw no key hold anything."""
     o, m, l = rnd(seed, T, H, splits, D), rnd(seed + 1, T, H, splits, scale=6.0), rnd(seed + 2, T, H, splits).abs() + 0.1
