@@ -588,14 +588,9 @@ def linear_normed_takes(x, weight, rank: int) -> bool:
 
 
 def normed_columns_take(n_rows: int, weight, rank: int) -> bool:
-    """Whether ``linear`` is best given ``linear_normed``'s ``ScaledRows`` of ``n_rows`` rows with this weight, which it takes then: not from 9 rows on where it would send
-    normed rows to the ring (us from the mixer's input to the queries, apart / joined: 12 and 16 rows, 4,096 x 384 16.3, 16.4 / 17.6, 19.4, 4,096 x 1,536 18.2, 18.9 /
-    19.1, 21.0, 8,192 x 768 20.0, 21.3 / 23.8, 26.9; 9 rows, 8,192 x 384 17.7 / 20.9, but 3,584 x 1,536 17.9 / 16.5)."""
-    if not isinstance(weight, LinearWeight) or weight.rows.dtype != torch.bfloat16 or n_rows > 16 or rank % 8 or weight.rows.shape[1] != rank:
-        return False
-    N = weight.rows.shape[0]
-    return (_small_m_kernel(n_rows, N, rank, weight.tiled is not None) == "skinny"
-            and not (n_rows >= RING_FEW_MIN_ROWS and weight.tiled is not None and _few_in_one_slice(N, rank, weight.tile_rows)))
+    """Whether ``linear`` takes ``linear_normed``'s ``ScaledRows`` of ``n_rows`` rows with this weight."""
+    return (isinstance(weight, LinearWeight) and weight.rows.dtype == torch.bfloat16 and n_rows <= 16 and rank % 8 == 0 and weight.rows.shape[1] == rank
+            and _small_m_kernel(n_rows, weight.rows.shape[0], rank, weight.tiled is not None) == "skinny")
 
 
 def linear_normed(x, weight: LinearWeight, column_scale: torch.Tensor, rank: int, eps: float):
@@ -1648,11 +1643,6 @@ def _few_in_slices(n_rows: int, N: int, K: int, tile_rows: int) -> bool:
     return RING_FEW_MIN_ROWS <= n_rows <= 16 and -(-N // tile_rows) <= COMPUTE_UNITS and RING_FEW_MIN_SLICED_K <= K < 1 << 20
 
 
-def _few_in_one_slice(N: int, K: int, tile_rows: int) -> bool:
-    """Whether 9 to 16 rows times such a weight go to ``ring_gemm`` in one slice of K, unless they go in several (see ``ring_takes_few``)."""
-    return 2048 < N and -(-N // tile_rows) <= 3 * COMPUTE_UNITS and K <= RING_FEW_MIN_SLICED_K
-
-
 def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
     """Whether 9 to 16 rows that would go to the product whose waves each read x from the L2 go to ``ring_gemm``, whose workgroups read it
     once: 1 in one slice of K, 2 in slices whose sum the caller takes, 0 not (us at 9 and 16 rows, that product : this one)
@@ -1672,7 +1662,8 @@ def ring_takes_few(x, weight, keep_slices: bool = False) -> int:
         return 0
     if keep_slices and _few_in_slices(M, N, K, weight.tile_rows):
         return 2
-    return 1 if _few_in_one_slice(N, K, weight.tile_rows) else 0
+    tiles = -(-N // weight.tile_rows)
+    return 1 if 2048 < N and tiles <= 3 * COMPUTE_UNITS and K <= RING_FEW_MIN_SLICED_K else 0
 
 
 def leaves_few_rows_in_sums(x, weight) -> bool:

@@ -70,14 +70,3 @@ def test_what_is_not_added_into_the_stream_leaves_its_sums_in_float(N, K):
         assert into or sums or K % 8, (rows, N, K)
         assert into == (not sums or N > 2048) or K % 8, (rows, N, K)
     assert ops.adds_into_stream(16, ops.LinearWeight(weight.rows), norm) == (K % 8 == 0)
-
-
-def test_norm_without_a_launch_gives_way_to_the_ring():
-    """From 9 rows on, where the ring takes the product behind the norm, whose rows it wants normed: 2,050 to 12,288 rows of up to 4,096 k-values."""
-    for N, K, ring in ((2048, 384, False), (2056, 384, True), (4096, 1536, True), (12288, 768, True), (12304, 768, False), (4096, 4104, False)):
-        weight = tiled(torch.empty((N, K), dtype=BF16))
-        for rows in (1, 8, 9, 16):
-            takes = ops.ring_takes_few(torch.empty((rows, K), dtype=BF16), weight)
-            assert takes == (1 if ring and rows >= 9 else 0)
-            assert ops.normed_columns_take(rows, weight, K) == (takes == 0), (N, K, rows)
-        assert ops.normed_columns_take(16, ops.LinearWeight(weight.rows), K)            # (no copy: the ring takes none)
