@@ -254,6 +254,7 @@ __global__ __launch_bounds__(WHOLE ? 512 : GLA_MAX_THREADS(DP)) void gla_kernel(
 // LOW: the decays' second product is formed here, too, by as many neighbouring lanes to a channel as there are, from weights that are asked for first: of
 // rank 128 6.4 us in two launches / 6.2, 9.2 / 7.7, 15.6 / 10.0, 19.5 / 13.8, 24.4 / 18.8.
 #define STEP_THREADS 512
+#define LOGIT_MAX 1.329228e36f   // 2^120
 #define LOW_AHEAD 2              // runs of 8 that a lane has on their way at once
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 gla_bf16x8;
 template <typename T, typename TO, int STEP_COLS, bool LOW>
@@ -326,6 +327,8 @@ __global__ __launch_bounds__(STEP_THREADS) __attribute__((amdgpu_waves_per_eu(ST
 #pragma unroll
           for (int e = 0; e < 8; ++e) z = fmaf((float)l[e], (float)w[e], z);
         }
+        // (an infinite sum would reach the neighbours' channels as 0 times it: 2^120 decays as it does, and sixty-four of them are finite)
+        z = z > LOGIT_MAX ? LOGIT_MAX : z < -LOGIT_MAX ? -LOGIT_MAX : z;
         z = column_sum(z, shares);
       } else {
         z = first ? z0 : z_t[(unsigned)min(c, d - 1)];

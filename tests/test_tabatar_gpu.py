@@ -306,6 +306,25 @@ def test_single_tokens_of_linear_attention_form_the_decays_product(R, H, d, dv, 
                      q_start.to(DEV), 2 * q_len.to(DEV), slots)
 
 
+@pytest.mark.parametrize("H,d,dv,rank", [(2, 64, 128, 128), (1, 32, 48, 64), (3, 10, 63, 24), (1, 256, 64, 16)])
+def test_an_infinite_logit_is_its_own_channels_affair(H, d, dv, rank):
+    """A channel whose product overflows decays at once or not at all, and the others as they do: the same as from the float logits."""
+    R = 3
+    rows, cols, _, bias, w = _gla_inputs(6, R, H, d, dv, torch.bfloat16)
+    low, w2 = rnd(33, R, rank).bfloat16().to(DEV), rnd(34, H * d, rank, scale=rank ** -0.5).bfloat16().to(DEV)
+    low[:, 1] = 1.0
+    w2[::7, 1], w2[3::7, 1] = -torch.inf, torch.inf
+    q_start, q_len = _step_arrays([1] * R)
+    outs = []
+    for z in ((low, w2), (low[:, None].double() * w2.double()).sum(-1).float()):
+        state = torch.zeros((R, ops.gla_state_floats(H, d, dv)), device=DEV)
+        for turn in range(2):
+            out = ops.gla_scan(rows.to(DEV), cols, z, bias.to(DEV), 16.0, d ** -0.5, w.to(DEV), 1e-5, H, d, dv, state, 0, q_start.to(DEV), q_len.to(DEV),
+                               torch.arange(R, dtype=torch.int32, device=DEV))
+        outs.append(torch.cat([out.cpu().double().flatten(), state.cpu().double().flatten()]))
+    assert torch.isfinite(outs[1]).all() and rel_err(outs[0], outs[1]) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("R,H,d,dv", [(4, 2, 16, 1), (4, 3, 10, 63), (4, 4, 64, 128), (4, 2, 24, 130), (4, 1, 64, 128), (4, 1, 64, 129), (4, 1, 64, 256), (4, 1, 64, 257),
                                       (4, 1, 256, 64), (4, 1, 256, 65), (4, 1, 100, 40), (768, 1, 16, 24), (257, 3, 10, 63), (200, 4, 64, 128)])
