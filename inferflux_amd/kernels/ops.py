@@ -578,8 +578,8 @@ def latent_query(q: torch.Tensor, latent: torch.Tensor, weight: torch.Tensor, n_
 def linear_normed_takes(x, weight, rank: int) -> bool:
     """Whether ``linear_normed`` takes ``x`` and this weight, a norm over the first ``rank`` columns of whose product follows: a weight whose tiles end where
     those columns do (weights of 2,049 to 3,584 rows have tiles of 10 to 14, which divide few ranks: there the norm keeps its launch), and rows that
-    ``linear`` would not send to the ring in slices, whose sums reach the norm in float (928 x 4,096 to the heads' queries at 9 and 16 rows 17.2, 17.1 us,
-    joined 15.0, 17.0, but a cached latent's error against 64 bits is 1.65e-3 so and 2.35e-3 through bfloat16)."""
+    ``linear`` would not send to the ring in slices, whose sums reach the norm in float (928 x 4,096 to the heads' queries at 9 and 16 rows 17.0, 17.1 us,
+    joined 14.0, 16.0, but a cached latent's error against 64 bits is 1.65e-3 so and 2.35e-3 through bfloat16)."""
     if not isinstance(weight, LinearWeight) or weight.order is not None or weight.tiled is None or x.dtype != torch.bfloat16:
         return False
     N, K = weight.rows.shape
