@@ -1339,13 +1339,12 @@ def adds_into_stream(n_rows: int, weight, norm_weight: torch.Tensor, single_toke
 
 
 def _into_stream_takes(n_rows: int, weight, norm_weight: torch.Tensor) -> bool:
-    if not isinstance(weight, LinearWeight) or weight.order is not None:
+    # (without a norm's weight: a reader that takes partial sums but keeps the addition to itself)
+    if n_rows > 16 or norm_weight is None or not isinstance(weight, LinearWeight) or weight.order is not None:
         return False
-    N, K = weight.rows.shape
-    if norm_weight is None:           # (a reader that takes partial sums but keeps the addition to itself)
-        return False
-    return (weight.rows.dtype == torch.bfloat16 and n_rows <= 16 and N % 4 == 0
-            and _small_m_kernel(n_rows, N, K, weight.tiled is not None) == "skinny")
+    rows = weight.rows
+    N, K = rows.shape
+    return N % 4 == 0 and rows.dtype == torch.bfloat16 and _small_m_kernel(n_rows, N, K, weight.tiled is not None) == "skinny"
 
 
 def linear_into_stream(x: torch.Tensor, weight: LinearWeight, stream: torch.Tensor, norm_weight: torch.Tensor,
